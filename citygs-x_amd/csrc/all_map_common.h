@@ -1,6 +1,7 @@
 // The per-Gaussian geometry channels of the blend ("all_map": camera-space normal, 1, plane distance): what the
-// all_map kernels and the preprocess kernel (when it writes the blend kernels' operand records) share, so that
-// both form the same bits from the same inputs.
+// all_map kernels and the preprocess kernels (which also form the channels, for the blend kernels' operand records and
+// for a caller whose all_map belongs to their own inputs, and take their gradient) share, so that both form the same
+// bits from the same inputs.
 #pragma once
 
 #include "gs_common.h"
@@ -62,6 +63,57 @@ __device__ __forceinline__ void all_map_channels(const AllMapGeom& g, float* o) 
   o[2] = g.loc[2];
   o[3] = 1.0f;
   o[4] = fabsf((g.loc[0] * g.pc[0] + g.loc[1] * g.pc[1]) + g.loc[2] * g.pc[2]);
+}
+
+// Backward of the channels: gradients with respect to the centre and to the (unnormalised) rotation, from those of
+// channels 0, 1, 2 and 4 (channel 3 is constant).
+__device__ __forceinline__ void all_map_gradient(const AllMapGeom& g, const float* V, float g0, float g1, float g2,
+                                                 float g4, float* dmean, float* dq) {
+  const float sdot = (g.loc[0] * g.pc[0] + g.loc[1] * g.pc[1]) + g.loc[2] * g.pc[2];
+  const float gs_ = g4 * (sdot > 0.0f ? 1.0f : (sdot < 0.0f ? -1.0f : 0.0f));  // d|s| = sign(s)
+  const float gl[3] = {g0 + gs_ * g.pc[0], g1 + gs_ * g.pc[1], g2 + gs_ * g.pc[2]};
+  const float gp[3] = {gs_ * g.loc[0], gs_ * g.loc[1], gs_ * g.loc[2]};
+  float gn[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    gn[a] = g.sgn * ((gl[0] * V[4 * a] + gl[1] * V[4 * a + 1]) + gl[2] * V[4 * a + 2]);
+    dmean[a] = (gp[0] * V[4 * a] + gp[1] * V[4 * a + 1]) + gp[2] * V[4 * a + 2];
+  }
+  // the chosen column of R as a function of (r,i,j,k) and two_s = 2/(q.q)
+  const float r = g.q[0], i = g.q[1], j = g.q[2], k = g.q[3], ts = g.two_s;
+  float gq[4], gts;
+  if (g.axis == 0) {
+    gq[0] = ts * (k * gn[1] - j * gn[2]);
+    gq[1] = ts * (j * gn[1] + k * gn[2]);
+    gq[2] = ts * ((-2.0f * j * gn[0] + i * gn[1]) - r * gn[2]);
+    gq[3] = ts * ((-2.0f * k * gn[0] + r * gn[1]) + i * gn[2]);
+    gts = (-(j * j + k * k) * gn[0] + (i * j + k * r) * gn[1]) + (i * k - j * r) * gn[2];
+  } else if (g.axis == 1) {
+    gq[0] = ts * (-k * gn[0] + i * gn[2]);
+    gq[1] = ts * ((j * gn[0] - 2.0f * i * gn[1]) + r * gn[2]);
+    gq[2] = ts * (i * gn[0] + k * gn[2]);
+    gq[3] = ts * ((-r * gn[0] - 2.0f * k * gn[1]) + j * gn[2]);
+    gts = ((i * j - k * r) * gn[0] - (i * i + k * k) * gn[1]) + (j * k + i * r) * gn[2];
+  } else {
+    gq[0] = ts * (j * gn[0] - i * gn[1]);
+    gq[1] = ts * ((k * gn[0] - r * gn[1]) - 2.0f * i * gn[2]);
+    gq[2] = ts * ((r * gn[0] + k * gn[1]) - 2.0f * j * gn[2]);
+    gq[3] = ts * (i * gn[0] + j * gn[1]);
+    gts = ((i * k + j * r) * gn[0] + (j * k - i * r) * gn[1]) - (i * i + j * j) * gn[2];
+  }
+  const float w = -(ts * ts) * gts;  // d two_s / dq = -two_s^2 q
+#pragma unroll
+  for (int a = 0; a < 4; a++) gq[a] += w * g.q[a];
+  // backward of q / max(|q|, eps)
+  if (g.len > 1e-12f) {
+    const float dot = ((g.q[0] * gq[0] + g.q[1] * gq[1]) + g.q[2] * gq[2]) + g.q[3] * gq[3];
+#pragma unroll
+    for (int a = 0; a < 4; a++) dq[a] = (gq[a] - g.q[a] * dot) / g.len;
+  } else {
+    const float den = fmaxf(g.len, 1e-12f);
+#pragma unroll
+    for (int a = 0; a < 4; a++) dq[a] = gq[a] / den;
+  }
 }
 
 }  // namespace gs

@@ -280,17 +280,18 @@ int gs_visible_filter(int P, int M, int width, int height, const float* means3D,
   return check_launch("visible_filter", (hipStream_t)stream, debug != 0);
 }
 
-int gs_preprocess_forward(float* means2D, float* depths, int* radii, float* cov3D, float* conic_opacity, float* rgb,
-                          uint8_t* clamped, uint32_t* tiles_touched, int P, int D, int M, int width, int height,
-                          const float* means3D, const float* scales, const float* rotations, const float* shs,
-                          const float* opacities, float scale_modifier, const float* viewmatrix,
-                          const float* projmatrix, const float* cam_pos, float tan_fovx, float tan_fovy,
-                          int prefiltered, int debug, float* dcolor_ddir, float* blend_records,
-                          gs_stream_t stream) {
+int gs_preprocess_channels_forward(float* means2D, float* depths, int* radii, float* cov3D, float* conic_opacity, float* rgb,
+                                   uint8_t* clamped, uint32_t* tiles_touched, int P, int D, int M, int width, int height,
+                                   const float* means3D, const float* scales, const float* rotations, const float* shs,
+                                   const float* opacities, float scale_modifier, const float* viewmatrix,
+                                   const float* projmatrix, const float* cam_pos, float tan_fovx, float tan_fovy,
+                                   int prefiltered, int debug, float* dcolor_ddir, float* blend_records,
+                                   float* all_map, gs_stream_t stream) {
   (void)prefiltered;
   GS_REQUIRE(P >= 0 && width > 0 && height > 0, "gs_preprocess_forward: bad sizes");
   GS_REQUIRE(((uintptr_t)blend_records & 15u) == 0u, "gs_preprocess_forward: blend_records must be 16-byte aligned");
-  GS_REQUIRE(blend_records == nullptr || cam_pos != nullptr, "gs_preprocess_forward: blend_records needs cam_pos");
+  GS_REQUIRE((blend_records == nullptr && all_map == nullptr) || cam_pos != nullptr,
+             "gs_preprocess_forward: blend_records and all_map need cam_pos");
   if (P == 0) return 0;
   GS_REQUIRE(means2D && depths && radii && conic_opacity && rgb && clamped, "gs_preprocess_forward: null output");
   GS_REQUIRE(means3D && scales && rotations && opacities && viewmatrix && projmatrix,
@@ -309,6 +310,7 @@ int gs_preprocess_forward(float* means2D, float* depths, int* radii, float* cov3
   a.rgb = rgb; a.clamped = clamped; a.tiles_touched = tiles_touched;
   a.dcolor_ddir = sh_mode ? dcolor_ddir : nullptr;
   a.blend_records = blend_records;
+  a.all_map = all_map;
   {
     StageScope _t("preprocess_fwd", (hipStream_t)stream);
     launch_preprocess_fwd(a, (hipStream_t)stream);
@@ -316,13 +318,27 @@ int gs_preprocess_forward(float* means2D, float* depths, int* radii, float* cov3
   return check_launch("preprocess_forward", (hipStream_t)stream, debug != 0);
 }
 
-int gs_preprocess_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
-                           int width, int height, const float* means3D, const float* scales, const float* rotations,
-                           const float* shs, float scale_modifier, const float* viewmatrix, const float* projmatrix,
-                           const float* campos, float tan_fovx, float tan_fovy, const float* dL_dmean2D,
-                           int mean2D_stride, const float* dL_dconic_opacity, const float* dL_dcolor,
-                           float* dL_dmean3D, float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
-                           float* dL_dopacity, int debug, const float* dcolor_ddir, gs_stream_t stream) {
+int gs_preprocess_forward(float* means2D, float* depths, int* radii, float* cov3D, float* conic_opacity, float* rgb,
+                          uint8_t* clamped, uint32_t* tiles_touched, int P, int D, int M, int width, int height,
+                          const float* means3D, const float* scales, const float* rotations, const float* shs,
+                          const float* opacities, float scale_modifier, const float* viewmatrix,
+                          const float* projmatrix, const float* cam_pos, float tan_fovx, float tan_fovy,
+                          int prefiltered, int debug, float* dcolor_ddir, float* blend_records,
+                          gs_stream_t stream) {
+  return gs_preprocess_channels_forward(means2D, depths, radii, cov3D, conic_opacity, rgb, clamped, tiles_touched, P, D,
+                                        M, width, height, means3D, scales, rotations, shs, opacities, scale_modifier,
+                                        viewmatrix, projmatrix, cam_pos, tan_fovx, tan_fovy, prefiltered, debug,
+                                        dcolor_ddir, blend_records, nullptr, stream);
+}
+
+int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
+                                    int width, int height, const float* means3D, const float* scales, const float* rotations,
+                                    const float* shs, float scale_modifier, const float* viewmatrix, const float* projmatrix,
+                                    const float* campos, float tan_fovx, float tan_fovy, const float* dL_dmean2D,
+                                    int mean2D_stride, const float* dL_dconic_opacity, const float* dL_dcolor,
+                                    float* dL_dmean3D, float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
+                                    float* dL_dopacity, int debug, const float* dcolor_ddir, const float* dL_dall_map,
+                                    gs_stream_t stream) {
   GS_REQUIRE(P >= 0 && width > 0 && height > 0, "gs_preprocess_backward: bad sizes");
   if (P == 0) return 0;
   GS_REQUIRE(radii && means3D && viewmatrix && projmatrix && dL_dmean2D && dL_dconic_opacity && dL_dmean3D,
@@ -334,6 +350,8 @@ int gs_preprocess_backward(const int* radii, const float* cov3D, const uint8_t* 
   const bool sh_mode = (shs != nullptr || dcolor_ddir != nullptr) && M > 0 && dL_dsh != nullptr;
   GS_REQUIRE(!sh_mode || (campos && clamped && dL_dcolor && D >= 0 && D <= 3 && M >= (D + 1) * (D + 1) && M <= 16),
              "gs_preprocess_backward: SH mode needs campos, clamped, dL_dcolor and (D+1)^2 <= M <= 16");
+  GS_REQUIRE(dL_dall_map == nullptr || (scales && rotations && campos),
+             "gs_preprocess_backward: dL_dall_map needs scales, rotations and campos");
   PreprocessBwdArgs a;
   a.P = P; a.D = D; a.M = sh_mode ? M : 0; a.W = width; a.H = height;
   a.means3D = means3D; a.radii = radii; a.shs = sh_mode ? shs : nullptr; a.clamped = clamped;
@@ -344,12 +362,26 @@ int gs_preprocess_backward(const int* radii, const float* cov3D, const uint8_t* 
   a.dL_dmean2D = dL_dmean2D; a.mean2D_stride = mean2D_stride; a.dL_dconic_opacity = dL_dconic_opacity;
   a.dL_dcolor = dL_dcolor;
   a.dL_dmean3D = dL_dmean3D; a.dL_dcov3D = dL_dcov3D; a.dL_dsh = sh_mode ? dL_dsh : nullptr;
+  a.dL_dall_map = dL_dall_map;
   a.dL_dscale = dL_dscale; a.dL_drot = dL_drot; a.dL_dopacity = dL_dopacity;
   {
     StageScope _t("preprocess_bwd", (hipStream_t)stream);
     launch_preprocess_bwd(a, (hipStream_t)stream);
   }
   return check_launch("preprocess_backward", (hipStream_t)stream, debug != 0);
+}
+
+int gs_preprocess_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
+                           int width, int height, const float* means3D, const float* scales, const float* rotations,
+                           const float* shs, float scale_modifier, const float* viewmatrix, const float* projmatrix,
+                           const float* campos, float tan_fovx, float tan_fovy, const float* dL_dmean2D,
+                           int mean2D_stride, const float* dL_dconic_opacity, const float* dL_dcolor,
+                           float* dL_dmean3D, float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
+                           float* dL_dopacity, int debug, const float* dcolor_ddir, gs_stream_t stream) {
+  return gs_preprocess_channels_backward(radii, cov3D, clamped, P, D, M, width, height, means3D, scales, rotations, shs,
+                                         scale_modifier, viewmatrix, projmatrix, campos, tan_fovx, tan_fovy, dL_dmean2D,
+                                         mean2D_stride, dL_dconic_opacity, dL_dcolor, dL_dmean3D, dL_dcov3D, dL_dscale,
+                                         dL_drot, dL_dsh, dL_dopacity, debug, dcolor_ddir, nullptr, stream);
 }
 
 // Host-visible words through which the scan hands the instance count to the waiting host thread.  Pinned

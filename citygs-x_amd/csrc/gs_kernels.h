@@ -26,6 +26,7 @@ struct PreprocessFwdArgs {
   // Gaussians, complete: the geometry channels are formed from means3D, scales, rotations, viewmatrix and campos
   // as launch_all_map_fwd forms them
   float* blend_records = nullptr;
+  float* all_map = nullptr;  // optional (P,5): the geometry channels of all Gaussians, as launch_all_map_fwd gives them
 };
 
 struct PreprocessBwdArgs {
@@ -44,6 +45,7 @@ struct PreprocessBwdArgs {
   const float* dL_dcolor;          // (P,3), SH mode only
   float *dL_dmean3D, *dL_dcov3D /*optional*/, *dL_dsh /*optional*/, *dL_dscale, *dL_drot, *dL_dopacity /*optional*/;
   const float* dcolor_ddir = nullptr;  // optional: what the forward kernel left (PreprocessFwdArgs::dcolor_ddir)
+  const float* dL_dall_map = nullptr;  // optional (P,5): gradient of the channels (PreprocessFwdArgs::all_map)
 };
 
 // Brackets a stage with an event pair on its stream while stage timing is enabled (gs_stage_timing_enable; the

@@ -7,6 +7,8 @@
 // for the rounding policy).  One thread per Gaussian; every output element is
 // written by the kernel (zeros for culled Gaussians), so callers may hand in
 // uninitialised buffers.
+#include <type_traits>
+
 #include "all_map_common.h"
 #include "gs_common.h"
 #include "gs_kernels.h"
@@ -245,6 +247,18 @@ __device__ __forceinline__ void sh_basis_and_direction_derivative(int D, float x
 #undef SHV
 }
 
+// What the colours' derivative with respect to the view direction contributes to the gradient of the mean, through the
+// normalisation of d0 = mean - camera (cuda_rasterizer/auxiliary.h:161-171).
+__device__ __forceinline__ void sh_gradient_of_mean(const float* d0, const float* dRdx, const float* dRdy,
+                                                    const float* dRdz, const float* gr, float* gm) {
+  const float s2 = dot3(d0, d0);
+  const float gdir[3] = {dot3(dRdx, gr), dot3(dRdy, gr), dot3(dRdz, gr)};
+  const float inv32 = 1.0f / sqrtf(s2 * s2 * s2);
+  gm[0] = ((s2 - d0[0] * d0[0]) * gdir[0] - d0[1] * d0[0] * gdir[1] - d0[2] * d0[0] * gdir[2]) * inv32;
+  gm[1] = (-d0[0] * d0[1] * gdir[0] + (s2 - d0[1] * d0[1]) * gdir[1] - d0[2] * d0[1] * gdir[2]) * inv32;
+  gm[2] = (-d0[0] * d0[2] * gdir[0] - d0[1] * d0[2] * gdir[1] + (s2 - d0[2] * d0[2]) * gdir[2]) * inv32;
+}
+
 // The same evaluation, one coefficient at a time: B[k] is everything of term k but the coefficient (the products
 // in sh_channel associate from the left, so term k = B[k] * c[k] is the same rounding), and sh_accumulate<K> is
 // the step of the running sum that takes in coefficient K.  Coefficients of degrees above `deg` are left out.
@@ -343,13 +357,14 @@ __device__ __forceinline__ void wave_rows_load(const float4* __restrict__ g4, ui
   wave_sync_lds();
 }
 
-// stores the first `rows` rows, streaming: SH coefficient gradients exist only when the coefficients are leaf
+// stores the first `rows` of the STAGED rows in LDS, streaming: SH coefficient gradients exist only when the coefficients are leaf
 // parameters, and then the optimizer is their next reader; the position, scale and rotation gradients can feed
 // the caller's backward pass at once and are stored normally
+template <int STAGED>
 __device__ __forceinline__ void wave_rows_store(float4* __restrict__ g4, int rows, const float4* lds, int lane) {
   wave_sync_lds();
 #pragma unroll
-  for (int j = 0; j < 12; j++) {
+  for (int j = 0; j < STAGED * 12 / GS_WAVE; j++) {
     const int idx = j * GS_WAVE + lane;
     const int row = idx / 12;
     if (row < rows) store_streaming(g4 + idx, lds[row * SH_ROW4 + (idx - row * 12)]);
@@ -361,9 +376,12 @@ __device__ __forceinline__ void wave_rows_store(float4* __restrict__ g4, int row
 // RECORDS: also write the blend kernels' operand record of every surviving Gaussian, (x, y, conic.x, conic.y)
 // (conic.w, opacity, r, g) (b, map0, map1, map2) (map3, map4, depth, 0), the geometry channels formed here by the
 // all_map kernel's own operations on the same inputs; a wave's 64 records leave through LDS as contiguous lines.
-// (six waves per SIMD; five with the records: six would spill there, and a kernel that spills starts its waves slowly)
-template <bool DERIV, bool RECORDS>
-__global__ void __launch_bounds__(GS_BLOCK_1D) __attribute__((amdgpu_waves_per_eu(RECORDS ? 5 : 6)))
+// MAP: also write the geometry channels of all Gaussians, culled ones included, as the (P,5) tensor the all_map kernel
+// would write (same operations, same bits).
+// (six waves per SIMD; five with the records, or with channels and derivative: six would spill there, and a kernel that
+// spills starts its waves slowly)
+template <bool DERIV, bool RECORDS, bool MAP>
+__global__ void __launch_bounds__(GS_BLOCK_1D) __attribute__((amdgpu_waves_per_eu(RECORDS || (DERIV && MAP) ? 5 : 6)))
 preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, const float* __restrict__ scales,
                       float mod, const float* __restrict__ rots, const float* __restrict__ opac,
                       const float* __restrict__ shs, const float* __restrict__ Vg, const float* __restrict__ PMg,
@@ -371,11 +389,13 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
                       uint32_t gx, uint32_t gy, int* __restrict__ radii, float2* __restrict__ means2D,
                       float* __restrict__ depths, float* __restrict__ cov3D, float4* __restrict__ conic_opacity,
                       float* __restrict__ rgb, uint8_t* __restrict__ clamped, uint32_t* __restrict__ tiles_touched,
-                      float* __restrict__ dcolor_ddir, float* __restrict__ blend_records) {
+                      float* __restrict__ dcolor_ddir, float* __restrict__ blend_records,
+                      float* __restrict__ all_map) {
   __shared__ float4 s_sh[GS_BLOCK_1D / GS_WAVE][GS_WAVE * SH_THIRD4];
   // RECORDS: what the record takes of the geometry, parked per lane while the colour is evaluated (held in
   // registers it would make the kernel spill; fetched again at the end it would keep every wave waiting for loads)
-  __shared__ float s_keep[RECORDS ? GS_BLOCK_1D / GS_WAVE : 1][RECORDS ? 12 * GS_WAVE : 1];
+  // (the geometry channels first: with MAP they leave for the caller's tensor from here)
+  __shared__ float s_keep[RECORDS || MAP ? GS_BLOCK_1D / GS_WAVE : 1][(RECORDS ? 12 : MAP ? 5 : 1) * GS_WAVE];
   const int slot = blockIdx.x * GS_BLOCK_1D + threadIdx.x;
   const bool live = slot < P;
   const int i = live ? slot : P - 1;  // lanes past the end keep step with a copy of the last Gaussian and store nothing
@@ -402,21 +422,37 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     conic_opacity[i] = ok ? make_float4(g.conic[0], g.conic[1], g.conic[2], opac[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
     if (tiles_touched) tiles_touched[i] = ok ? (g.rect.x1 - g.rect.x0) * (g.rect.y1 - g.rect.y0) : 0u;
   }
-  if (RECORDS && ok) {  // (culled Gaussians have no record)
+  if (MAP || (RECORDS && ok)) {  // (culled Gaussians have channels, but no record)
     float chan[5];
     AllMapGeom ag;
     all_map_geom(mean, sc, q4, cam.V, cam.campos, ag);
     all_map_channels(ag, chan);
     float* keep = s_keep[threadIdx.x / GS_WAVE] + (threadIdx.x & (GS_WAVE - 1));
-    keep[0 * GS_WAVE] = g.px;
-    keep[1 * GS_WAVE] = g.py;
-    keep[2 * GS_WAVE] = g.conic[0];
-    keep[3 * GS_WAVE] = g.conic[1];
-    keep[4 * GS_WAVE] = g.conic[2];
-    keep[5 * GS_WAVE] = opac[i];
-    keep[6 * GS_WAVE] = g.depth;
 #pragma unroll
-    for (int k = 0; k < 5; k++) keep[(7 + k) * GS_WAVE] = chan[k];
+    for (int k = 0; k < 5; k++) keep[k * GS_WAVE] = chan[k];
+    if (RECORDS && ok) {
+      keep[5 * GS_WAVE] = g.px;
+      keep[6 * GS_WAVE] = g.py;
+      keep[7 * GS_WAVE] = g.conic[0];
+      keep[8 * GS_WAVE] = g.conic[1];
+      keep[9 * GS_WAVE] = g.conic[2];
+      keep[10 * GS_WAVE] = opac[i];
+      keep[11 * GS_WAVE] = g.depth;
+    }
+  }
+  if (MAP) {
+    // the wave's 64 rows of 5 floats leave as five runs of consecutive floats
+    const int lane = threadIdx.x & (GS_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GS_WAVE);
+    const size_t wave_first = (size_t)blockIdx.x * GS_BLOCK_1D + (size_t)wave * GS_WAVE;
+    const size_t rows_left = (size_t)P > wave_first ? (size_t)P - wave_first : 0;
+    float* out = all_map + 5 * wave_first;
+    wave_sync_lds();
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+      const int e = j * GS_WAVE + lane, row = e / 5;
+      if ((size_t)e < 5 * rows_left) out[e] = s_keep[wave][(e - 5 * row) * GS_WAVE + row];
+    }
   }
 
   float col[3] = {0.f, 0.f, 0.f};
@@ -518,10 +554,10 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       float4* mine = s_sh[wave];
       wave_sync_lds();  // (everyone has read what the buffer last held)
       const float* keep = s_keep[wave] + lane;
-      mine[0 * WORD_STRIDE + lane] = make_float4(keep[0 * GS_WAVE], keep[1 * GS_WAVE], keep[2 * GS_WAVE], keep[3 * GS_WAVE]);
-      mine[1 * WORD_STRIDE + lane] = make_float4(keep[4 * GS_WAVE], keep[5 * GS_WAVE], col[0], col[1]);
-      mine[2 * WORD_STRIDE + lane] = make_float4(col[2], keep[7 * GS_WAVE], keep[8 * GS_WAVE], keep[9 * GS_WAVE]);
-      mine[3 * WORD_STRIDE + lane] = make_float4(keep[10 * GS_WAVE], keep[11 * GS_WAVE], keep[6 * GS_WAVE], 0.f);
+      mine[0 * WORD_STRIDE + lane] = make_float4(keep[5 * GS_WAVE], keep[6 * GS_WAVE], keep[7 * GS_WAVE], keep[8 * GS_WAVE]);
+      mine[1 * WORD_STRIDE + lane] = make_float4(keep[9 * GS_WAVE], keep[10 * GS_WAVE], col[0], col[1]);
+      mine[2 * WORD_STRIDE + lane] = make_float4(col[2], keep[0 * GS_WAVE], keep[1 * GS_WAVE], keep[2 * GS_WAVE]);
+      mine[3 * WORD_STRIDE + lane] = make_float4(keep[3 * GS_WAVE], keep[4 * GS_WAVE], keep[11 * GS_WAVE], 0.f);
       wave_sync_lds();
       float4* out = reinterpret_cast<float4*>(blend_records) +
                     4 * ((size_t)blockIdx.x * GS_BLOCK_1D + (size_t)wave * GS_WAVE);  // the wave's first record
@@ -589,7 +625,12 @@ mark_visible_kernel(int P, const float* __restrict__ means, const float* __restr
 // gradient stays in registers.  dL_dconic_opacity is packed [x, y, w, opacity].
 // SAVED: the forward kernel's derivative of the colours with respect to the view direction is given, and the
 // coefficient rows are not read.
-template <bool SAVED>
+// MAP: the gradient of the geometry channels (all_map, formed from the same means, scales and rotations) is given as
+// well; its part is added to the gradients of means and rotations here, where those inputs are at hand.  As a kernel of
+// its own plus the two accumulations it reads them again and moves 56 + 84 more bytes per Gaussian: 18 + 15 us at 1 M
+// Gaussians and 168 + 140 us at 10 M, against 6 and 45 us in here.
+// The kernel is bound by HBM (10 M Gaussians, 3 M of them visible: 3.8 GB in 680 us).
+template <bool SAVED, bool MAP>
 __global__ void __launch_bounds__(GS_BLOCK_1D)
 preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, const int* __restrict__ radii,
                       const float* __restrict__ shs, const uint8_t* __restrict__ clamped,
@@ -600,8 +641,11 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
                       const float4* __restrict__ dL_dconic_opacity, const float* __restrict__ dL_dcolor,
                       float* __restrict__ dL_dmean3D, float* __restrict__ dL_dcov3D_out, float* __restrict__ dL_dsh,
                       float* __restrict__ dL_dscale, float* __restrict__ dL_drot, float* __restrict__ dL_dopacity,
-                      const float* __restrict__ dcolor_ddir) {
-  __shared__ float4 s_rows[GS_BLOCK_1D / GS_WAVE][SH_WAVE_ROWS4];
+                      const float* __restrict__ dcolor_ddir, const float* __restrict__ dL_dall_map) {
+  // (SAVED stages sixteen rows at a time: all rows of a wave would take 53 KB and leave three waves per SIMD, which cost
+  // 10 us of 87 at 1 M Gaussians and 85 of 765 at 10 M)
+  constexpr int STORE_ROWS = SAVED ? GS_WAVE / 4 : GS_WAVE;
+  __shared__ float4 s_rows[GS_BLOCK_1D / GS_WAVE][STORE_ROWS * SH_ROW4];
   const int lane = threadIdx.x & (GS_WAVE - 1), wave = threadIdx.x / GS_WAVE;
   const int raw_i = blockIdx.x * GS_BLOCK_1D + threadIdx.x;
   const bool in_range = raw_i < P;
@@ -614,7 +658,58 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   float gc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const bool live = in_range && radii[i] > 0;
   const size_t wave_first = (size_t)blockIdx.x * GS_BLOCK_1D + (size_t)wave * GS_WAVE;
-  float4* my_row = s_rows[wave] + lane * SH_ROW4;
+  float4* my_row = s_rows[wave] + (lane & (STORE_ROWS - 1)) * SH_ROW4;
+  float map_g[4] = {0.f, 0.f, 0.f, 0.f};
+  if (MAP) {
+    const float* go = dL_dall_map + 5 * (size_t)i;
+    map_g[0] = go[0]; map_g[1] = go[1]; map_g[2] = go[2]; map_g[3] = go[4];
+  }
+  const long long left = (long long)P - (long long)wave_first;
+  const int rows = left <= 0 ? 0 : left < GS_WAVE ? (int)left : GS_WAVE;
+  // SAVED: the colour part comes first, so that what it keeps in registers (the row of coefficient gradients is the
+  // outer product of basis and colour gradient) is gone before the geometry part starts.
+  float sh_gm[3] = {0.f, 0.f, 0.f};  // what it adds to the gradient of the mean
+  if (SAVED && sh_mode) {
+    float basis[16], gr[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 16; k++) basis[k] = 0.f;
+    if (live) {
+      const float d0[3] = {means[3 * (size_t)i] - camg[0], means[3 * (size_t)i + 1] - camg[1],
+                           means[3 * (size_t)i + 2] - camg[2]};
+#pragma unroll
+      for (int ch = 0; ch < 3; ch++) gr[ch] = dL_dcolor[3 * (size_t)i + ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
+      const float* dd = dcolor_ddir + 9 * (size_t)i;
+      const float dRdx[3] = {dd[0], dd[1], dd[2]}, dRdy[3] = {dd[3], dd[4], dd[5]}, dRdz[3] = {dd[6], dd[7], dd[8]};
+      sh_gradient_of_mean(d0, dRdx, dRdy, dRdz, gr, sh_gm);
+      const float len = sqrtf(dot3(d0, d0));
+      float none[3];
+      sh_basis_and_direction_derivative<false>(D, d0[0] / len, d0[1] / len, d0[2] / len, nullptr, basis, none, none,
+                                               none);
+    }
+    if (M == 16) {
+      float4* out = reinterpret_cast<float4*>(dL_dsh) + wave_first * 12;
+#pragma unroll 1
+      for (int q = 0; q < GS_WAVE / STORE_ROWS; q++) {
+        wave_sync_lds();  // (the sixteen rows before these have left)
+        if (lane / STORE_ROWS == q) {
+#pragma unroll
+          for (int j = 0; j < 12; j++)
+            my_row[j] = make_float4(basis[(4 * j) / 3] * gr[(4 * j) % 3], basis[(4 * j + 1) / 3] * gr[(4 * j + 1) % 3],
+                                    basis[(4 * j + 2) / 3] * gr[(4 * j + 2) % 3],
+                                    basis[(4 * j + 3) / 3] * gr[(4 * j + 3) % 3]);
+        }
+        wave_rows_store<STORE_ROWS>(out + q * STORE_ROWS * 12, rows - q * STORE_ROWS, s_rows[wave], lane);
+      }
+    } else if (in_range) {
+      float* gsh = dL_dsh + (size_t)i * M * 3;
+      for (int k = 0; k < M; k++) {
+        const float bk = k < 16 ? basis[k] : 0.f;
+        gsh[3 * k] = bk * gr[0];
+        gsh[3 * k + 1] = bk * gr[1];
+        gsh[3 * k + 2] = bk * gr[2];
+      }
+    }
+  }
   // (the coefficients are only needed for the colours' derivative with respect to the view direction; a caller
   // that kept the forward pass's nine numbers per Gaussian saves this kernel the 192-byte rows)
   if (sh_staged && !SAVED) {
@@ -702,47 +797,35 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     gm[1] += (PM[4] * m_w - PM[7] * mul1) * g2x + (PM[5] * m_w - PM[7] * mul2) * g2y;
     gm[2] += (PM[8] * m_w - PM[11] * mul1) * g2x + (PM[9] * m_w - PM[11] * mul2) * g2y;
 
-    if (sh_mode) {
+    if (SAVED) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) gm[k] += sh_gm[k];
+    } else if (sh_mode) {
       const float* sh = shs + (size_t)i * M * 3;
       float* gsh = dL_dsh + (size_t)i * M * 3;
       // the Gaussian's coefficients, in registers; 16-coefficient rows (192 bytes) move as twelve 16-byte words
       float shv[48];
-      if (!SAVED) {
-        if (M == 16) {
+      if (M == 16) {
 #pragma unroll
-          for (int j = 0; j < 12; j++) {
-            const float4 v = my_row[j];
-            shv[4 * j] = v.x;
-            shv[4 * j + 1] = v.y;
-            shv[4 * j + 2] = v.z;
-            shv[4 * j + 3] = v.w;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 48; e++) shv[e] = e < 3 * M ? sh[e] : 0.f;
+        for (int j = 0; j < 12; j++) {
+          const float4 v = my_row[j];
+          shv[4 * j] = v.x;
+          shv[4 * j + 1] = v.y;
+          shv[4 * j + 2] = v.z;
+          shv[4 * j + 3] = v.w;
         }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 48; e++) shv[e] = e < 3 * M ? sh[e] : 0.f;
       }
       const float d0[3] = {mean[0] - cam.campos[0], mean[1] - cam.campos[1], mean[2] - cam.campos[2]};
-      const float s2 = dot3(d0, d0);
-      const float len = sqrtf(s2);
-      const float x = d0[0] / len, y = d0[1] / len, z = d0[2] / len;
+      const float len = sqrtf(dot3(d0, d0));
       float gr[3];
 #pragma unroll
       for (int ch = 0; ch < 3; ch++) gr[ch] = dL_dcolor[3 * (size_t)i + ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
       float basis[16];
       float dRdx[3], dRdy[3], dRdz[3];
-      if (SAVED) {
-        sh_basis_and_direction_derivative<false>(D, x, y, z, nullptr, basis, dRdx, dRdy, dRdz);
-        const float* dd = dcolor_ddir + 9 * (size_t)i;
-#pragma unroll
-        for (int ch = 0; ch < 3; ch++) {
-          dRdx[ch] = dd[ch];
-          dRdy[ch] = dd[3 + ch];
-          dRdz[ch] = dd[6 + ch];
-        }
-      } else {
-        sh_basis_and_direction_derivative<true>(D, x, y, z, shv, basis, dRdx, dRdy, dRdz);
-      }
+      sh_basis_and_direction_derivative<true>(D, d0[0] / len, d0[1] / len, d0[2] / len, shv, basis, dRdx, dRdy, dRdz);
       if (M == 16) {
 #pragma unroll
         for (int j = 0; j < 12; j++)
@@ -756,11 +839,9 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
           gsh[3 * k + 2] = bk * gr[2];
         }
       }
-      const float gdir[3] = {dot3(dRdx, gr), dot3(dRdy, gr), dot3(dRdz, gr)};
-      const float inv32 = 1.0f / sqrtf(s2 * s2 * s2);
-      gm[0] += ((s2 - d0[0] * d0[0]) * gdir[0] - d0[1] * d0[0] * gdir[1] - d0[2] * d0[0] * gdir[2]) * inv32;
-      gm[1] += (-d0[0] * d0[1] * gdir[0] + (s2 - d0[1] * d0[1]) * gdir[1] - d0[2] * d0[1] * gdir[2]) * inv32;
-      gm[2] += (-d0[0] * d0[2] * gdir[0] - d0[1] * d0[2] * gdir[1] + (s2 - d0[2] * d0[2]) * gdir[2]) * inv32;
+      sh_gradient_of_mean(d0, dRdx, dRdy, dRdz, gr, sh_gm);
+#pragma unroll
+      for (int k = 0; k < 3; k++) gm[k] += sh_gm[k];
     }
 
     if (scales) {
@@ -803,22 +884,39 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
                2 * y * (dMt.m[1][2] + dMt.m[2][1])) -
               4 * z * (dMt.m[1][1] + dMt.m[0][0]);
     }
-  } else if (sh_mode && in_range) {
-    float* gsh = dL_dsh + (size_t)i * M * 3;
+  } else if (!SAVED && sh_mode && in_range) {
     if (M == 16) {
 #pragma unroll
       for (int j = 0; j < 12; j++) my_row[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     } else {
+      float* gsh = dL_dsh + (size_t)i * M * 3;
       for (int k = 0; k < 3 * M; k++) gsh[k] = 0.f;
     }
   }
-  if (sh_staged) {
-    const long long left = (long long)P - (long long)wave_first;
-    if (left > 0)
-      wave_rows_store(reinterpret_cast<float4*>(dL_dsh) + wave_first * 12, left < GS_WAVE ? (int)left : GS_WAVE,
-                      s_rows[wave], lane);
-  }
+  if (sh_staged && !SAVED)
+    wave_rows_store<STORE_ROWS>(reinterpret_cast<float4*>(dL_dsh) + wave_first * 12, rows, s_rows[wave], lane);
   if (!in_range) return;
+  if (MAP) {
+    const float g0 = map_g[0], g1 = map_g[1], g2 = map_g[2], g4 = map_g[3];
+    // (zero for a Gaussian no pixel blended, culled ones first of all)
+    if (!(g0 == 0.f && g1 == 0.f && g2 == 0.f && g4 == 0.f)) {
+      float V[16], campos[3];
+#pragma unroll
+      for (int k = 0; k < 16; k++) V[k] = Vg[k];
+#pragma unroll
+      for (int k = 0; k < 3; k++) campos[k] = camg[k];
+      const float mean[3] = {means[3 * (size_t)i], means[3 * (size_t)i + 1], means[3 * (size_t)i + 2]};
+      const float sc[3] = {scales[3 * (size_t)i], scales[3 * (size_t)i + 1], scales[3 * (size_t)i + 2]};
+      AllMapGeom ag;
+      all_map_geom(mean, sc, reinterpret_cast<const float4*>(rots)[i], V, campos, ag);
+      float dmean[3], dq[4];
+      all_map_gradient(ag, V, g0, g1, g2, g4, dmean, dq);
+#pragma unroll
+      for (int k = 0; k < 3; k++) gm[k] += dmean[k];
+#pragma unroll
+      for (int k = 0; k < 4; k++) gq[k] += dq[k];
+    }
+  }
   dL_dmean3D[3 * (size_t)i] = gm[0];
   dL_dmean3D[3 * (size_t)i + 1] = gm[1];
   dL_dmean3D[3 * (size_t)i + 2] = gm[2];
@@ -846,15 +944,23 @@ int launch_preprocess_fwd(const PreprocessFwdArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, a.P, a.D, a.M, a.means3D, a.scales,
                        a.scale_modifier, a.rotations, a.opacities, a.shs, a.viewmatrix, a.projmatrix, a.campos, a.W,
                        a.H, a.tanx, a.tany, fx, fy, gx, gy, a.radii, (float2*)a.means2D, a.depths, a.cov3D,
-                       (float4*)a.conic_opacity, a.rgb, a.clamped, a.tiles_touched, a.dcolor_ddir, a.blend_records);
+                       (float4*)a.conic_opacity, a.rgb, a.clamped, a.tiles_touched, a.dcolor_ddir, a.blend_records,
+                       a.all_map);
   };
   const bool deriv = a.dcolor_ddir != nullptr && a.shs != nullptr && a.M > 0;
+  auto choose = [&](auto deriv_tag, auto records_tag) {
+    constexpr bool DERIV = decltype(deriv_tag)::value, RECORDS = decltype(records_tag)::value;
+    if (a.all_map != nullptr) go(preprocess_fwd_kernel<DERIV, RECORDS, true>);
+    else go(preprocess_fwd_kernel<DERIV, RECORDS, false>);
+  };
+  using yes = std::true_type;
+  using no = std::false_type;
   if (a.blend_records != nullptr) {
-    if (deriv) go(preprocess_fwd_kernel<true, true>);
-    else go(preprocess_fwd_kernel<false, true>);
+    if (deriv) choose(yes{}, yes{});
+    else choose(no{}, yes{});
   } else {
-    if (deriv) go(preprocess_fwd_kernel<true, false>);
-    else go(preprocess_fwd_kernel<false, false>);
+    if (deriv) choose(yes{}, no{});
+    else choose(no{}, no{});
   }
   return 0;
 }
@@ -889,10 +995,15 @@ int launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t stream) {
                        a.clamped, a.scales, a.rotations, a.scale_modifier, a.cov3D, a.viewmatrix, a.projmatrix,
                        a.campos, h_x, h_y, a.tanx, a.tany, a.dL_dmean2D, a.mean2D_stride,
                        (const float4*)a.dL_dconic_opacity, a.dL_dcolor, a.dL_dmean3D, a.dL_dcov3D, a.dL_dsh,
-                       a.dL_dscale, a.dL_drot, a.dL_dopacity, a.dcolor_ddir);
+                       a.dL_dscale, a.dL_drot, a.dL_dopacity, a.dcolor_ddir, a.dL_dall_map);
   };
-  if (a.dcolor_ddir != nullptr) go(preprocess_bwd_kernel<true>);
-  else go(preprocess_bwd_kernel<false>);
+  if (a.dL_dall_map != nullptr) {
+    if (a.dcolor_ddir != nullptr) go(preprocess_bwd_kernel<true, true>);
+    else go(preprocess_bwd_kernel<false, true>);
+  } else {
+    if (a.dcolor_ddir != nullptr) go(preprocess_bwd_kernel<true, false>);
+    else go(preprocess_bwd_kernel<false, false>);
+  }
   return 0;
 }
 

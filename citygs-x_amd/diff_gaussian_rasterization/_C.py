@@ -86,7 +86,7 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacity, scale_modifier
 
 def preprocess_gaussians_ex(means3D, scales, rotations, sh, opacity, scale_modifier, viewmatrix, projmatrix, tan_fovx,
                             tan_fovy, image_height, image_width, degree, campos, prefiltered, debug, args,
-                            want_direction_derivative=False, want_cov3D=True, blend_records=None):
+                            want_direction_derivative=False, want_cov3D=True, blend_records=None, all_map=None):
     """preprocess_gaussians plus what the reference's tuple has no slot for: returns (tuple, dcolor_ddir).  With
     want_direction_derivative (and SH colours) dcolor_ddir is the (P,3,3) derivative of every surviving Gaussian's
     colour with respect to the unit view direction; handed to preprocess_gaussians_backward it replaces the
@@ -95,7 +95,8 @@ def preprocess_gaussians_ex(means3D, scales, rotations, sh, opacity, scale_modif
     covariances again from scales and rotations (the same bits), and neither pass moves the 24 bytes per Gaussian.
     blend_records: an optional (P,16) float32 tensor that receives the blend kernels' operand records of the
     surviving Gaussians, geometry channels included (those build_all_map gives for the same means3D, scales,
-    rotations, viewmatrix and campos); see render_gaussians_ex."""
+    rotations, viewmatrix and campos); see render_gaussians_ex.
+    all_map: an optional (P,5) float32 tensor that receives what build_all_map gives for the same inputs."""
     if means3D.ndimension() != 2 or means3D.size(1) != 3:
         raise RuntimeError("means3D must have dimensions (num_points, 3)")
     means3D = _f32c(means3D, "means3D")
@@ -120,21 +121,23 @@ def preprocess_gaussians_ex(means3D, scales, rotations, sh, opacity, scale_modif
     shc = _f32c(sh, "sh") if sh_mode else None
     ddir = torch.empty(P, 3, 3, **f32) if (sh_mode and want_direction_derivative) else None
     with torch.cuda.device(dev):
-        _n.check(_lib.gs_preprocess_forward(
+        _n.check(_lib.gs_preprocess_channels_forward(
             _ptr(means2D), _ptr(depths), _ptr(radii), _ptr(cov3D), _ptr(conic_opacity), _ptr(rgb), _ptr(clamped), None,
             P, int(degree), M, int(image_width), int(image_height), _ptr(means3D), _ptr(scales), _ptr(rotations),
             _ptr(shc), _ptr(opacity), float(scale_modifier), _ptr(vm), _ptr(pm), _ptr(cp), float(tan_fovx),
             float(tan_fovy), int(bool(prefiltered)), int(bool(debug)), _ptr(ddir), _ptr(blend_records),
-            _stream(dev)),
+            _ptr(all_map), _stream(dev)),
             "preprocess_gaussians")
     return (0, means2D, depths, radii, cov3D, conic_opacity, rgb, clamped), ddir
 
 
 def preprocess_gaussians_backward(radii, cov3D, clamped, means3D, scales, rotations, sh, scale_modifier, viewmatrix,
                                   projmatrix, tan_fovx, tan_fovy, image_height, image_width, degree, campos,
-                                  dL_dmeans2D, dL_dconic_opacity, dL_dcolors, R, debug, args, dcolor_ddir=None):
+                                  dL_dmeans2D, dL_dconic_opacity, dL_dcolors, R, debug, args, dcolor_ddir=None,
+                                  dL_dall_map=None):
     """rasterize_points.cu:146-234.  dL_dmeans2D may be (P,2) or (P,3).  dcolor_ddir: what
-    preprocess_gaussians_ex returned for the same inputs, or None."""
+    preprocess_gaussians_ex returned for the same inputs, or None.  dL_dall_map: None, or the gradient of the
+    channels that call wrote; build_all_map_backward's results are then part of the gradients returned."""
     means3D = _f32c(means3D, "means3D")
     dev = means3D.device
     P = means3D.shape[0]
@@ -158,14 +161,15 @@ def preprocess_gaussians_backward(radii, cov3D, clamped, means3D, scales, rotati
     vm, pm, cp = _f32c(viewmatrix, "viewmatrix"), _f32c(projmatrix, "projmatrix"), _f32c(campos, "campos")
     shc = _f32c(sh, "sh") if sh_mode else None
     with torch.cuda.device(dev):
-        _n.check(_lib.gs_preprocess_backward(
+        _n.check(_lib.gs_preprocess_channels_backward(
             _ptr(radii.contiguous()), _ptr(cov3D.contiguous() if cov3D is not None else None),
             _ptr(clamped.contiguous()), P, int(degree), M,
             int(image_width), int(image_height), _ptr(means3D), _ptr(scales), _ptr(rotations), _ptr(shc),
             float(scale_modifier), _ptr(vm), _ptr(pm), _ptr(cp), float(tan_fovx), float(tan_fovy), _ptr(g2),
             int(g2.shape[1]), _ptr(gco), _ptr(gcol), _ptr(dL_dmeans3D), None, _ptr(dL_dscales), _ptr(dL_drotations),
             _ptr(dL_dsh) if sh_mode else None, _ptr(dL_dopacity), int(bool(debug)),
-            _ptr(dcolor_ddir) if (sh_mode and dcolor_ddir is not None) else None, _stream(dev)),
+            _ptr(dcolor_ddir) if (sh_mode and dcolor_ddir is not None) else None,
+            _ptr(_f32c(dL_dall_map, "dL_dall_map") if dL_dall_map is not None else None), _stream(dev)),
             "preprocess_gaussians_backward")
     return dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity
 

@@ -52,11 +52,18 @@ class GaussianRasterizationSettings(NamedTuple):
 # tensors and camera preprocess_gaussians had; otherwise the library packs.  Nothing a caller sees changes: same
 # tensors, same values.
 
-class _BlendRecords:
-    __slots__ = ("records", "refs", "versions", "sources", "source_versions", "all_map_ref", "all_map_version")
+# In the same way preprocess_gaussians forms the channels tensor itself, as one more output of its autograd node, once
+# a caller builds all_map through build_all_map(..., blend_records_of=means2D): that call then hands out this tensor
+# instead of launching a kernel, and the channels' gradient arrives in the backward kernel of the node, which has
+# means and rotations in registers, instead of in one of its own whose results autograd would add up.
 
-    def __init__(self, records, parts, sources):
-        self.records = records
+class _BlendRecords:
+    __slots__ = ("records", "refs", "versions", "sources", "source_versions", "all_map", "all_map_ref",
+                 "all_map_version")
+
+    def __init__(self, records, all_map, parts, sources):
+        self.records = records  # (None: only the channels were formed)
+        self.all_map = all_map  # the node's channels output, until build_all_map hands it out
         self.refs = [weakref.ref(t) for t in parts]
         self.versions = [t._version for t in parts]
         # means3D, scales, rotations, viewmatrix, campos as preprocess_gaussians had them
@@ -68,7 +75,21 @@ class _BlendRecords:
     def same_sources(self, sources):
         return all(ref() is t and t._version == v for ref, v, t in zip(self.sources, self.source_versions, sources))
 
+    def take_all_map(self, sources):
+        """The channels preprocess_gaussians formed, if they are those of `sources` and carry the gradient the caller's
+        mode asks for; once (two callers must not share a tensor either may modify)."""
+        all_map = self.all_map
+        if all_map is None or not self.same_sources(sources):
+            return None
+        needs_grad = torch.is_grad_enabled() and (sources[0].requires_grad or sources[2].requires_grad)
+        if needs_grad and not all_map.requires_grad:
+            return None
+        self.all_map = None
+        return all_map if needs_grad or not all_map.requires_grad else all_map.detach()
+
     def usable(self, parts, all_maps, render_geo):
+        if self.records is None:
+            return False
         for ref, version, t in zip(self.refs, self.versions, parts):
             if ref() is not t or t._version != version:
                 return False
@@ -104,12 +125,15 @@ class _PreprocessGaussians(torch.autograd.Function):
         P = means3D.shape[0]
         records = (torch.empty(P, 16, dtype=torch.float32, device=means3D.device)
                    if P > 0 and _records_wanted(rs, P, means3D.device) else None)
+        all_map = (torch.empty(P, 5, dtype=torch.float32, device=means3D.device)
+                   if P > 0 and rs.render_geo and _linked_all_map_seen[0] else None)
         (num_rendered, means2D, depths, radii, cov3D, conic_opacity, rgb, clamped), ddir = _C.preprocess_gaussians_ex(
             means3D, scales, rotations, sh, opacities, rs.scale_modifier, rs.viewmatrix, rs.projmatrix, rs.tanfovx,
             rs.tanfovy, rs.image_height, rs.image_width, rs.sh_degree, rs.campos, rs.prefiltered, rs.debug, cuda_args,
-            want_direction_derivative=any(ctx.needs_input_grad[:5]), want_cov3D=False, blend_records=records)
+            want_direction_derivative=any(ctx.needs_input_grad[:5]), want_cov3D=False, blend_records=records,
+            all_map=all_map)
         _pending_blend[0] = ((records, (means3D, scales, rotations, rs.viewmatrix, rs.campos))
-                             if records is not None else None)
+                             if records is not None or all_map is not None else None)
         # (cov3D is None: the backward kernel forms the covariances again from scales and rotations, which it reads
         # anyway, instead of both passes moving 24 bytes per Gaussian)
         ctx.raster_settings = rs
@@ -121,12 +145,17 @@ class _PreprocessGaussians(torch.autograd.Function):
         ctx.mark_non_differentiable(radii, depths)
         # no zero tensors for the outputs nobody differentiates (radii, depths): backward fills in what it needs
         ctx.set_materialize_grads(False)
-        return means2D, rgb, conic_opacity, radii, depths
+        return means2D, rgb, conic_opacity, radii, depths, all_map
 
     @staticmethod
-    def backward(ctx, grad_means2D, grad_rgb, grad_conic_opacity, grad_radii, grad_depths):
+    def backward(ctx, grad_means2D, grad_rgb, grad_conic_opacity, grad_radii, grad_depths, grad_all_map):
         rs = ctx.raster_settings
         means3D, scales, rotations, sh, radii, cov3D, clamped = ctx.saved_tensors[:7]
+        if grad_means2D is None and grad_rgb is None and grad_conic_opacity is None and grad_all_map is not None:
+            # (only the channels were differentiated)
+            dL_dmeans3D, dL_drotations = _C.build_all_map_backward(means3D, scales, rotations, rs.viewmatrix, rs.campos,
+                                                                   grad_all_map)
+            return dL_dmeans3D, None, dL_drotations, None, None, None, None
         ddir = ctx.saved_tensors[7] if ctx.has_ddir else None
         P = means3D.shape[0]
         if grad_means2D is None:
@@ -138,7 +167,8 @@ class _PreprocessGaussians(torch.autograd.Function):
         dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity = _C.preprocess_gaussians_backward(
             radii, cov3D, clamped, means3D, scales, rotations, sh, rs.scale_modifier, rs.viewmatrix, rs.projmatrix,
             rs.tanfovx, rs.tanfovy, rs.image_height, rs.image_width, rs.sh_degree, rs.campos, grad_means2D,
-            grad_conic_opacity, grad_rgb, ctx.num_rendered, rs.debug, ctx.cuda_args, dcolor_ddir=ddir)
+            grad_conic_opacity, grad_rgb, ctx.num_rendered, rs.debug, ctx.cuda_args, dcolor_ddir=ddir,
+            dL_dall_map=grad_all_map)
         if dL_dsh.shape != sh.shape:
             dL_dsh = torch.zeros_like(sh)
         return dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity, None, None
@@ -146,11 +176,11 @@ class _PreprocessGaussians(torch.autograd.Function):
 
 def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_settings, cuda_args):
     _pending_blend[0] = None
-    means2D, rgb, conic_opacity, radii, depths = _PreprocessGaussians.apply(means3D, scales, rotations, sh, opacities,
-                                                                            raster_settings, cuda_args)
+    means2D, rgb, conic_opacity, radii, depths, all_map = _PreprocessGaussians.apply(
+        means3D, scales, rotations, sh, opacities, raster_settings, cuda_args)
     pending, _pending_blend[0] = _pending_blend[0], None
     if pending is not None:
-        means2D._gs_blend = _BlendRecords(pending[0], (means2D, conic_opacity, rgb, depths), pending[1])
+        means2D._gs_blend = _BlendRecords(pending[0], all_map, (means2D, conic_opacity, rgb, depths), pending[1])
     return means2D, rgb, conic_opacity, radii, depths
 
 
@@ -201,9 +231,10 @@ class _RenderGaussians(torch.autograd.Function):
         blend = getattr(means2D, "_gs_blend", None)
         records = (blend.records if blend is not None and blend.usable((means2D, conic_opacity, rgb, depths), all_maps,
                                                                        rs.render_geo) else None)
-        if blend is not None and records is None and rs.render_geo:
-            # records were written and cannot be used: the caller does not (or no longer) build all_map through
-            # build_all_map(..., blend_records_of=means2D); stop writing them until it does
+        if (blend is not None and records is None and rs.render_geo
+                and (blend.records is not None or blend.all_map is not None)):
+            # records or channels were written and cannot be used: the caller does not (or no longer) build all_map
+            # through build_all_map(..., blend_records_of=means2D); stop writing them until it does
             _linked_all_map_seen[0] = False
         ((num_rendered, color, n_render, n_consider, n_contrib, out_observe, out_all_map, out_plane_depth, geomBuffer,
           binningBuffer, imgBuffer), info) = _C.render_gaussians_ex(
@@ -278,14 +309,19 @@ def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_
     blend_records_of (optional): the means2D tensor preprocess_gaussians returned for the same parameter tensors
     and camera (the settings' viewmatrix and campos tensors).  preprocess_gaussians then writes the blend kernels'
     operand records with these very channels in them (from the next view on), and render_gaussians, given these
-    very tensors, skips the pass that packs them.  The returned tensor is the same either way."""
-    all_map = _BuildAllMap.apply(means3D, scales, rotations, viewmatrix, campos)
-    if blend_records_of is not None:
-        _linked_all_map_seen[0] = True
-        blend = getattr(blend_records_of, "_gs_blend", None)
-        if blend is not None and blend.same_sources((means3D, scales, rotations, viewmatrix, campos)):
-            blend.all_map_ref = weakref.ref(all_map)
-            blend.all_map_version = all_map._version
+    very tensors, skips the pass that packs them; it also forms this tensor, whose gradient its own backward pass then
+    takes.  The returned values and the gradients are the same either way."""
+    sources = (means3D, scales, rotations, viewmatrix, campos)
+    if blend_records_of is None:
+        return _BuildAllMap.apply(*sources)
+    _linked_all_map_seen[0] = True
+    blend = getattr(blend_records_of, "_gs_blend", None)
+    all_map = blend.take_all_map(sources) if blend is not None else None
+    if all_map is None:
+        all_map = _BuildAllMap.apply(*sources)
+    if blend is not None and blend.same_sources(sources):
+        blend.all_map_ref = weakref.ref(all_map)
+        blend.all_map_version = all_map._version
     return all_map
 
 

@@ -32,6 +32,10 @@ _SIGNATURES = {
                                    _vp]),
     "gs_preprocess_backward": (_i, [_vp] * 3 + [_i] * 5 + [_vp] * 4 + [_f] + [_vp] * 3 + [_f, _f] + [_vp, _i] +
                                [_vp] * 8 + [_i, _vp, _vp]),
+    "gs_preprocess_channels_forward": (_i, [_vp] * 8 + [_i] * 5 + [_vp] * 5 + [_f] + [_vp] * 3 + [_f, _f, _i, _i] +
+                                       [_vp] * 4),
+    "gs_preprocess_channels_backward": (_i, [_vp] * 3 + [_i] * 5 + [_vp] * 4 + [_f] + [_vp] * 3 + [_f, _f] +
+                                        [_vp, _i] + [_vp] * 8 + [_i] + [_vp] * 3),
     "gs_render_forward": (_i, [RESIZE_FN, _vp, RESIZE_FN, _vp, RESIZE_FN, _vp, _i, _vp, _i, _i, _f, _f, _f, _f] +
                           [_vp] * 17 + [_i, _i, C.POINTER(_i), C.POINTER(_f), _vp, _vp, _vp]),
     "gs_render_backward_workspace_bytes": (_sz, [_i]),

@@ -89,6 +89,17 @@ int gs_preprocess_forward(float* means2D, float* depths, int* radii, float* cov3
                           int prefiltered, int debug, float* dcolor_ddir, float* blend_records,
                           gs_stream_t stream);
 
+/* gs_preprocess_forward that also writes the five geometry channels of every Gaussian, culled ones included: all_map
+ * (P,5) receives what gs_all_map_forward gives for the same means3D, scales, rotations, viewmatrix and cam_pos, bit
+ * for bit (NULL: gs_preprocess_forward itself). */
+int gs_preprocess_channels_forward(float* means2D, float* depths, int* radii, float* cov3D, float* conic_opacity,
+                                   float* rgb, uint8_t* clamped, uint32_t* tiles_touched, int P, int D, int M,
+                                   int width, int height, const float* means3D, const float* scales,
+                                   const float* rotations, const float* shs, const float* opacities,
+                                   float scale_modifier, const float* viewmatrix, const float* projmatrix,
+                                   const float* cam_pos, float tan_fovx, float tan_fovy, int prefiltered, int debug,
+                                   float* dcolor_ddir, float* blend_records, float* all_map, gs_stream_t stream);
+
 /* Replaces Rasterizer::preprocessBackward (CR/rasterizer.h:86-111,
  * CR/rasterizer_impl.cu:427-489) together with the tensor repacking of
  * PreprocessGaussiansBackwardCUDA (DGR/rasterize_points.cu:181-194):
@@ -110,6 +121,19 @@ int gs_preprocess_backward(const int* radii, const float* cov3D, const uint8_t* 
                            const float* dL_dconic_opacity, const float* dL_dcolor, float* dL_dmean3D,
                            float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh, float* dL_dopacity,
                            int debug, const float* dcolor_ddir, gs_stream_t stream);
+
+/* gs_preprocess_backward that also takes the gradient of the geometry channels gs_preprocess_channels_forward wrote
+ * (P,5): dL_dmean3D and dL_drot then hold the sum of what gs_preprocess_backward and gs_all_map_backward give (NULL:
+ * gs_preprocess_backward itself).  A Gaussian whose channels' gradient is zero gets nothing added. */
+int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
+                                    int width, int height, const float* means3D, const float* scales,
+                                    const float* rotations, const float* shs, float scale_modifier,
+                                    const float* viewmatrix, const float* projmatrix, const float* campos,
+                                    float tan_fovx, float tan_fovy, const float* dL_dmean2D, int mean2D_stride,
+                                    const float* dL_dconic_opacity, const float* dL_dcolor, float* dL_dmean3D,
+                                    float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
+                                    float* dL_dopacity, int debug, const float* dcolor_ddir,
+                                    const float* dL_dall_map, gs_stream_t stream);
 
 /* No counterpart in the reference: per-call options of gs_render_forward (NULL = all defaults).  A field below
  * zero keeps its default; struct_bytes is sizeof(gs_render_options) as the caller compiled it.
