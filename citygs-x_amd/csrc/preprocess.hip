@@ -170,7 +170,6 @@ __device__ __forceinline__ float sh_channel(int deg, float x, float y, float z, 
 // completely; a lane then reads or writes its own row in LDS.  Rows are padded to 13 x 16 bytes, which keeps
 // both access patterns free of bank conflicts.
 constexpr int SH_ROW4 = 13;
-constexpr int SH_WAVE_ROWS4 = GS_WAVE * SH_ROW4;
 
 __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -4,27 +4,31 @@
 // over pixels.
 //
 // Workgroup = one 16x16 tile = four 64-lane waves; a wave owns an 8x8 quadrant
-// and each of its 16-lane rows a 4x4 pixel block.  Gaussians are staged in LDS
-// 128 at a time, in back-to-front order, and worked on 64 at a time:
-//   * a wave ballots, for each of its rows, which of the 64 Gaussians can touch
-//     the row's block (the forward kernel's own answer, 16 bits per instance,
-//     when the caller hands them on; otherwise the inflated alpha >= 1/255
-//     ellipse is tested against the block again) and lie in front of the
-//     row's deepest contributor, and compacts their slot numbers into a byte
-//     list per row; the four rows then walk their own lists concurrently
-//     (entry n of each in pass n), so one pass of the loop handles up to four
-//     Gaussians;
-//   * the 16 partial sums of a Gaussian (mean2D x/y, |mean2D| x/y, conic
-//     x/y/w, opacity, colour 3, map 5) are reduced over the row's 16 lanes by
-//     a transposing DPP reduction (15 additions instead of 64) that leaves
-//     component q in lane q; rows of the wave that are at the same Gaussian
-//     are merged, and the sums go into the wave's own 16x64 accumulator in
-//     LDS with a plain read-add-write (no atomics: an LDS float atomic costs
-//     about three cycles per active lane here, and the kernel was bound by
-//     them);
-//   * then the four waves' accumulators are added in wave order and every
-//     (tile, Gaussian) instance's 16 sums are stored as one 64-byte record, at
-//     the instance's index in emission order (the order key emission wrote
+// and each of its 16-lane rows a 4x4 pixel block, a quad of lanes four pixels
+// of an image row.
+//   * The tile's list is scanned back to front, 256 entries at a time, and the
+//     entries that touch a block in front of its deepest contributor (the
+//     forward kernel's own answer, 16 bits per instance, when the caller hands
+//     them on; otherwise the inflated alpha >= 1/255 ellipse is tested again)
+//     are compacted into a ring; the others' records are zero.
+//   * 128 of them at a time are staged in LDS and worked on 64 at a time: a
+//     wave compacts, for each of its rows, the slots that touch the row's
+//     block into a byte list, and the four rows walk their own lists
+//     concurrently, four entries per pass.
+//   * A pass has two halves.  In the first, lane = pixel: the recurrence over
+//     the four entries, which leaves w = alpha T and q = G dL/dalpha per
+//     (entry, pixel).  In the second, lane e of a quad works for entry e: the
+//     4x4 blocks of w and q are transposed inside the quads, the sums over
+//     pixels of q and its moments are plain additions over registers, those of
+//     w times the eight upstream channels are matrix instructions (so is the
+//     dot product of an entry's channels with a pixel's upstream gradients in
+//     the first half), and two halving steps add up the quads of a row.
+//   * The sixteen sums of an entry go into the wave's own accumulator in LDS,
+//     row after row, with a plain read-add-write (no atomics: an LDS float
+//     atomic costs about three cycles per active lane here).
+//   * After 64 slots the four waves' accumulators are added in wave order and
+//     every (tile, Gaussian) instance's sums are stored as one 64-byte record,
+//     at the instance's index in emission order (the order key emission wrote
 //     them: all instances of a Gaussian are consecutive there).  No global
 //     atomics either.
 // A second kernel then sums, for every Gaussian, its consecutive records and
@@ -32,16 +36,27 @@
 // fixed order, so the gradients are the same bits from run to run.  (The
 // reference issues 16 global float atomics per pixel and Gaussian,
 // cuda_rasterizer/backward.cu:510-563.)
+//
+// What bounds it: vector issue (busy share 0.8 at 1 M Gaussians, 1152x864: some 90
+// vector instructions per entry of a row; 125 when every pass took one entry
+// and reduced its sixteen sums over the sixteen lanes of the row).  Before and
+// after: 256 -> 229 us there, 757 -> 537 us for 4 M Gaussians from the air,
+// 1117 -> 904 us for 10 M at street level, 129 -> 110 us for 300 k without
+// geometry channels.  The matrix cores take what contracts an operand that all
+// entries or all pixels share; the recurrence itself is a serial chain per
+// pixel.
+//
 // The per-pixel arithmetic follows the CPU statement's operation for operation
-// (transmittance, reciprocal, weights, the derivative of the exponent), with
-// three exceptions: the order in which pixels are summed; the factors that are
-// constant per Gaussian (W/2, H/2, the opacity and -1/2 of the geometric
-// gradients), which multiply the sums instead of every term; and the blend of
-// everything behind a Gaussian, which the reference
-// keeps per channel and this kernel keeps as its dot product with the upstream
-// gradients (one recurrence instead of eight: see `behind_dot`).  Gradients
-// therefore agree with a CPU evaluation to rounding (rel. L2 of the order of
-// 1e-7 on the test scenes), not bit for bit.
+// in everything that decides what counts (the exponent, alpha, the tests) and
+// in the transmittance, with these exceptions after that: the order in which
+// pixels are summed (fixed for thin Gaussians, see `exact`); the factors that
+// are constant per Gaussian (W/2, H/2, the opacity, the conic and -1/2 of the
+// geometric gradients), which multiply the sums instead of every term; and the
+// blend of everything behind a Gaussian, background included, which the
+// reference keeps per channel and this kernel keeps as its dot product with the
+// upstream gradients (one recurrence instead of eight: see `behind_dot`).
+// Gradients therefore agree with a CPU evaluation to rounding (rel. L2 of the
+// order of 1e-7 on the test scenes), not bit for bit.
 #include <type_traits>
 
 #include "gs_common.h"
@@ -53,10 +68,117 @@ namespace gs {
 namespace {
 
 constexpr int BATCH = GS_TILE_PIX / 2;  // Gaussians staged in LDS per round
+constexpr int RUN = GS_WAVE;        // consecutive positions of a tile's list that stay together (see the order of the sums)
+constexpr float THIN = 0.8f;        // squared correlation b * b / (a * c) from which a Gaussian counts as thin
 constexpr int SUB = GS_WAVE;        // Gaussians whose sums are in the accumulators at a time: one ballot's worth
-constexpr int NV = 16;
+constexpr int PENDING = 512;        // ring of list positions that wait to be staged: at most BATCH - 1 + GS_TILE_PIX of them
+constexpr int GROUP = 4;            // entries of a list handled per pass of the walk, one per lane of a quad
 constexpr int WAVES = GS_TILE_PIX / GS_WAVE;
 static_assert(SUB * 4 == GS_TILE_PIX, "a thread hands over a quarter of one record of the sub-batch");
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// The value lane E of a quad (four neighbouring lanes) holds, in all four lanes.
+template <int E>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), E * 0x55, 0xF, 0xF, true));
+}
+
+// Transposes the 4x4 blocks of a and b inside every quad: register e of lane p becomes register p of lane e.  A DPP
+// operand written by the preceding VALU instruction needs two idle issue slots first, a matrix instruction one.
+__device__ __forceinline__ void quad_transpose2(float (&a)[4], float (&b)[4]) {
+  const uint64_t bit0 = 0xAAAAAAAAAAAAAAAAull, bit1 = 0xCCCCCCCCCCCCCCCCull;
+  float c[4], d[4];
+  asm volatile(
+      "s_nop 1\n\t"
+      "s_mov_b64 vcc, %16\n\t"
+      "v_cndmask_b32_dpp %1, %8, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %10, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %12, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %14, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %0, %9, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %2, %11, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %4, %13, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %15, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      : "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3]), "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "s"(bit0)
+      : "vcc", "scc");
+  asm volatile(
+      "s_nop 1\n\t"
+      "s_mov_b64 vcc, %16\n\t"
+      "v_cndmask_b32_dpp %2, %8, %10, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %9, %11, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %12, %14, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %13, %15, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %0, %10, %8, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %1, %11, %9, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %4, %14, %12, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %15, %13, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
+      : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "s"(bit1)
+      : "vcc", "scc");
+}
+
+// Sums sixteen values over the four quads of every 16-lane row and leaves values 4 q .. 4 q + 3 in quad q, in v[0..3]
+// (v is overwritten).  Two halving steps, two instructions per value kept: the bank mask of a DPP addition selects the
+// quads that take its result.  The matrix results among the inputs need up to seven idle slots first.  LAST = false:
+// v[12..15] are not given, and quad 3 ends up with no meaningful sums.
+template <bool LAST>
+__device__ __forceinline__ void quads_reduce16(float (&v)[16]) {
+  if (LAST)
+    asm volatile(
+        "s_nop 7\n\t"
+        "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %4, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %5, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %7, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+        : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
+  else
+    asm volatile(
+        "s_nop 7\n\t"
+        "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+        : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]));
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %1, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %2, %2, %2 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %3, %3, %3 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %4, %4 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %1, %5, %5 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %2, %6, %6 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %3, %7, %7 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])
+      : "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+}
 
 // HITS: the forward blend left, per sorted instance, which 4x4 blocks of the tile the Gaussian can touch; without
 // it the same test is made again here.
@@ -77,25 +199,30 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                              ? packed_records : nullptr;
   constexpr bool render_geo = RENDER_GEO;
   __shared__ uint32_t s_emis[BATCH];
-  __shared__ float4 s_xyf[BATCH];  // centre x, y; the power floor; unused
-  __shared__ float4 s_co[BATCH];
-  __shared__ float4 s_cp[HITS ? 1 : BATCH];
-  __shared__ uint16_t s_hits[HITS ? BATCH : 1];
+  __shared__ int s_pend[PENDING];
+  __shared__ uint16_t s_pend_hits[PENDING];
+  __shared__ int s_found[2][WAVES];
+  // (slot BATCH: what an entry behind the end of a list refers to, a Gaussian whose floor no exponent reaches)
+  __shared__ float4 s_xyf[BATCH + 1];  // centre x, y; the power floor; the position in the tile's list, as bits
+  __shared__ float4 s_co[BATCH + 1];
+  __shared__ uint16_t s_hits[BATCH];
   // colour, then the five geometry channels: eight floats per Gaussian, read as two 16-byte words
-  __shared__ float4 s_chan[BATCH][RENDER_GEO ? 2 : 1];
-  // one accumulator per wave; +1: the 16 components of one Gaussian fall in 16 different banks
-  __shared__ float s_acc[WAVES][NV][SUB + 1];
-  // the four rows' lists of every wave: the slots of the sub-batch that can touch the row's block and are not
-  // behind its deepest contributor, one byte each, in walking order; bytes behind a list's end are 0
-  __shared__ __attribute__((aligned(16))) uint32_t s_idx[GS_TILE_PIX / GS_WAVE][4][SUB / 4];
-  __shared__ int s_max[GS_TILE_PIX / GS_WAVE];
-  __shared__ int s_bad[GS_TILE_PIX / GS_WAVE];
+  __shared__ float4 s_chan[BATCH + 1][RENDER_GEO ? 2 : 1];
+  // one accumulator per wave: word 4 slot + (part ^ (slot / 4 & 3)) holds sums 4 part .. 4 part + 3 of a slot, so that
+  // neither the walk's accesses (a part of consecutive slots) nor the hand-over's pile up on a few banks
+  __shared__ float4 s_acc[WAVES][4 * SUB];
+  // the four rows' lists of every wave: the slots of the batch that can touch the row's block and are not
+  // behind its deepest contributor, one byte each, in walking order; bytes behind a list's end are BATCH
+  __shared__ __attribute__((aligned(16))) uint32_t s_idx[GS_TILE_PIX / GS_WAVE][4][2 * SUB / 4];
+  __shared__ int4 s_row_last[WAVES];  // the deepest contributor of every row
 
   const int tid = threadIdx.x;
   const RowThread rt = row_thread(blockIdx.x, blockIdx.y);
-  const int lane = rt.lane, wave = rt.wave, row = rt.row, l16 = rt.l16;
+  const int lane = rt.lane, wave = rt.wave, row = rt.row;
   const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
-  const uint32_t px = rt.px, py = rt.py;
+  // (a quad of lanes holds one column of the row's 4x4 block: see the order of the sums below)
+  const uint32_t px = (uint32_t)rt.qx0 + (uint32_t)(row & 1) * 4u + (uint32_t)(rt.l16 >> 2);
+  const uint32_t py = (uint32_t)rt.qy0 + (uint32_t)(row >> 1) * 4u + (uint32_t)(rt.l16 & 3);
   const bool inside = px < (uint32_t)W && py < (uint32_t)H;
   const size_t pid = (size_t)W * py + px;
   const size_t HW = (size_t)H * W;
@@ -122,13 +249,15 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   int row_last = last_contributor;
 #pragma unroll
   for (int d = 8; d >= 1; d >>= 1) row_last = max(row_last, __shfl_xor(row_last, d, GS_WAVE));
-  int row_last_of[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) row_last_of[r] = __builtin_amdgcn_readlane(row_last, 16 * r);
-  const int wave_last = max(max(row_last_of[0], row_last_of[1]), max(row_last_of[2], row_last_of[3]));
-  if (lane == 0) s_max[wave] = wave_last;
+  if ((lane & 15) == 0) reinterpret_cast<int*>(&s_row_last[wave])[row] = row_last;
   __syncthreads();
-  const int tile_last = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+  int tile_last = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; w++) {
+    const int4 r = s_row_last[w];
+    tile_last = max(tile_last, max(max(r.x, r.y), max(r.z, r.w)));
+  }
+  tile_last = __builtin_amdgcn_readfirstlane(tile_last);
   // Every instance record of the tile is written exactly once: the ones behind the deepest contributor
   // get zeros here, the others are written at the end of their batch.
   for (int p = tile_last + tid; p < total; p += GS_TILE_PIX) {
@@ -158,40 +287,119 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   float bg_dot = 0.f;
 #pragma unroll
   for (int ch = 0; ch < GS_N_RGB; ch++) bg_dot += bg[ch] * gpix[ch];
-
-  const float bg_term = T_final * bg_dot;
   // dL/dalpha of a Gaussian needs sum_ch (c_ch - b_ch) g_ch, with b the blend of everything behind it and g the
   // upstream gradients of the eight channels.  The reference keeps b per channel (accum_rec,
   // cuda_rasterizer/backward.cu:463-472: b <- alpha c + (1 - alpha) b at every step); the sum is linear in b, so
   // here the pixel keeps the one number B = sum_ch b_ch g_ch instead, which obeys the same recurrence with
   // S = sum_ch c_ch g_ch in place of c: the term is S - B, and B <- alpha S + (1 - alpha) B.  Same value, eight
   // multiply-adds per step instead of forty operations; it is rounded differently (an error of the order of
-  // eps |c| |g| per term where the per-channel form has eps |c - b| |g|), well inside the stated tolerance.
-  float behind_dot = 0.f;
+  // eps |c| |g| per term where the per-channel form has eps |c - b| |g|), well inside the stated tolerance.  The
+  // background is what lies behind the last Gaussian: B starts as its dot product, which is the reference's separate
+  // term -T_final / (1 - alpha) sum_ch bg_ch g_ch (cuda_rasterizer/backward.cu:505-508).
+  float behind_dot = bg_dot;
 
-  // Positions are 0-based indices into the tile's list; the walk starts at the tile's deepest contributor.
-  // Slot j of batch i holds position start - (i*BATCH + j).
-  const int start = tile_last - 1;
-  const int rounds = (start + 1 + BATCH - 1) / BATCH;
+  // The pixels' upstream gradients as the matrix instructions that sum over pixels take them: register p of lane i of
+  // a quad holds channel i (and 4 + i) of the quad's pixel p.
+  float grad_t[RENDER_GEO ? 2 : 1][4];
+  {
+    const float chan[8] = {gpix[0], gpix[1], gpix[2], gmap[0], gmap[1], gmap[2], gmap[3], gmap[4]};
+#pragma unroll
+    for (int h = 0; h < (RENDER_GEO ? 2 : 1); h++) {
+      float t[4] = {chan[4 * h], chan[4 * h + 1], chan[4 * h + 2], chan[4 * h + 3]}, unused[4] = {0.f, 0.f, 0.f, 0.f};
+      quad_transpose2(t, unused);
+#pragma unroll
+      for (int p = 0; p < 4; p++) grad_t[h][p] = t[p];
+    }
+  }
 
   // thread tid hands over components 4*part .. 4*part+3 of the sub-batch's slot tid / 4 and clears them
   const int my_slot = tid >> 2, my_part = tid & 3;
+  const int my_word = 4 * my_slot + (my_part ^ ((my_slot >> 2) & 3));
 #pragma unroll
-  for (int w = 0; w < WAVES; w++) {
+  for (int w = 0; w < WAVES; w++) s_acc[w][my_word] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (tid == 0) {
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+    s_xyf[BATCH] = make_float4(0.f, 0.f, __builtin_inff(), 0.f);
+    s_co[BATCH] = z;
 #pragma unroll
-    for (int e = 0; e < 4; e++) s_acc[w][4 * my_part + e][my_slot] = 0.f;
+    for (int h = 0; h < (RENDER_GEO ? 2 : 1); h++) s_chan[BATCH][h] = z;
   }
+  const uint32_t quad_shift = 8u * (uint32_t)(lane & 3), quad = (uint32_t)(rt.l16 >> 2);
+  const float block_y0 = (float)(py & ~3u);  // the first of the four pixels of a quad
 
-  for (int i = 0; i < rounds; i++) {
-    const int first_pos = start - i * BATCH;  // position in slot 0
-    const int count = first_pos + 1 < BATCH ? first_pos + 1 : BATCH;
-    // (the barrier that ends the previous batch's last sub-batch has let every wave finish with the staged data)
-    // (a lane for which a Gaussian does not count takes part with alpha = 0, which is exact as long as the
-    // Gaussian's colour and geometry channels are finite; a batch holding a non-finite one is walked by the
-    // variant of the loop that leaves such a lane's recurrence state alone instead)
-    bool finite = true;
+  // Positions are 0-based indices into the tile's list; the walk goes down from the tile's deepest contributor.  A Gaussian
+  // that touches no row's block in front of the row's deepest contributor is not staged: its record is zero.  (Of a
+  // list of thousands of small Gaussians most touch nothing: a street-level tile of 17 000 entries stages 4 500.  Walked
+  // entry by entry it took 1.1 ms, longer than all other tiles of that view together.)
+  auto hits_at = [&](int pos) { return pos >= 0 ? (uint32_t)block_hits[range.x + (uint32_t)pos] : 0u; };
+  auto hits_by_test = [&](int pos) {
+    if (pos < 0) return 0u;
+    const uint32_t g = point_list[range.x + (uint32_t)pos];
+    const float2 xy = means2D[g];
+    const float4 co = conic_opacity[g];
+    const float tile_x0 = (float)(blockIdx.x * GS_TILE_X), tile_y0 = (float)(blockIdx.y * GS_TILE_Y);
+    float pfl, mark_limit;
+    const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
+    uint32_t found = 0u;
+#pragma unroll
+    for (int k = 0; k < WAVES; k++) {
+      bool hit[4];
+      ellipse_hits_quadrant(xy, co, cp.x, cp.y, cp.z, tile_x0 + 8.f * (float)(k & 1), tile_y0 + 8.f * (float)(k >> 1),
+                            hit);
+#pragma unroll
+      for (int r = 0; r < 4; r++) found |= hit[r] ? 1u << (4 * k + r) : 0u;
+    }
+    return found;
+  };
+  int unscanned = tile_last;  // positions below this one have not been looked at
+  uint32_t head = 0u, tail = 0u, parity = 0u;
+  uint32_t carried[4] = {0u, 0u, 0u, 0u}, carried_run = 0xFFFFFFFFu;  // see `exact` below
+  uint32_t hits_next = HITS ? hits_at(unscanned - 1 - tid) : 0u;  // (fetched one step ahead)
+  for (;;) {
+    while (tail - head < (uint32_t)BATCH && unscanned > 0) {
+      const int pos = unscanned - 1 - tid;
+      uint32_t hits = HITS ? hits_next : hits_by_test(pos);
+      unscanned = max(unscanned - GS_TILE_PIX, 0);
+      if (HITS) hits_next = hits_at(unscanned - 1 - tid);
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) {
+        const int4 last = s_row_last[w];
+        hits &= ~((pos >= last.x ? 1u << (4 * w) : 0u) | (pos >= last.y ? 2u << (4 * w) : 0u) |
+                  (pos >= last.z ? 4u << (4 * w) : 0u) | (pos >= last.w ? 8u << (4 * w) : 0u));
+      }
+      const bool take = pos >= 0 && hits != 0u;
+      const uint64_t take_m = gs_ballot(take);
+      if (lane == 0) s_found[parity][wave] = (int)__popcll(take_m);
+      if (pos >= 0 && !take) {
+        float4* rec = instance_grads + 4 * (size_t)emission_sorted[range.x + (uint32_t)pos];
+        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+        rec[0] = z; rec[1] = z; rec[2] = z; rec[3] = z;
+      }
+      __syncthreads();
+      uint32_t before = tail;
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) {
+        const uint32_t n = (uint32_t)s_found[parity][w];
+        before += w < wave ? n : 0u;
+        tail += n;
+      }
+      if (take) {
+        const uint32_t at = (before + __builtin_amdgcn_mbcnt_hi((uint32_t)(take_m >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)take_m, 0u))) &
+                            (PENDING - 1);
+        s_pend[at] = pos;
+        s_pend_hits[at] = (uint16_t)hits;
+      }
+      parity ^= 1u;  // (the counts are rewritten two barriers later)
+    }
+    const int count = (int)min((uint32_t)BATCH, tail - head);
+    if (count == 0) break;
+    __syncthreads();
+    // (the barrier that ended the previous batch's last sub-batch has let every wave finish with the staged data)
     if (tid < count) {
-      const uint32_t k_sorted = range.x + (uint32_t)(first_pos - tid);
+      const uint32_t at = (head + (uint32_t)tid) & (PENDING - 1);
+      const int pos = s_pend[at];
+      const uint32_t k_sorted = range.x + (uint32_t)pos;
       const uint32_t g = point_list[k_sorted];
       // A Gaussian's operands: one 64-byte record where the forward call packed them (a single line of memory,
       // every byte of it used), else gathered from the four arrays.  (Each route loads and then stages by itself:
@@ -201,23 +409,12 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         s_emis[tid] = emission_sorted[k_sorted];
         s_co[tid] = co;
         float pfl, mark_limit;
-        const float4 cp = block_test_params(co, xy, (float)(blockIdx.x * GS_TILE_X), (float)(blockIdx.y * GS_TILE_Y),
-                                            pfl, mark_limit);
-        if (HITS) s_hits[tid] = block_hits[k_sorted];
-        else s_cp[tid] = cp;
-        s_xyf[tid] = make_float4(xy.x, xy.y, pfl, 0.f);
-        float mag = fmaxf(fmaxf(fabsf(c0), fabsf(c1)), fabsf(c2));
-        bool fin = c0 == c0 && c1 == c1 && c2 == c2;
-        if (render_geo) {
-#pragma unroll
-          for (int ch = 0; ch < GS_N_MAP; ch++) {
-            mag = fmaxf(mag, fabsf(m[ch]));
-            fin = fin && m[ch] == m[ch];
-          }
-          s_chan[tid][RENDER_GEO ? 1 : 0] = make_float4(m[1], m[2], m[3], m[4]);
-        }
+        (void)block_test_params(co, xy, (float)(blockIdx.x * GS_TILE_X), (float)(blockIdx.y * GS_TILE_Y), pfl,
+                                mark_limit);
+        s_hits[tid] = s_pend_hits[at];
+        s_xyf[tid] = make_float4(xy.x, xy.y, pfl, __int_as_float(pos));
+        if (render_geo) s_chan[tid][RENDER_GEO ? 1 : 0] = make_float4(m[1], m[2], m[3], m[4]);
         s_chan[tid][0] = make_float4(c0, c1, c2, m[0]);
-        return fin && mag < __builtin_inff();
       };
       if (packed != nullptr) {
         const float4* rec = packed + 4 * (size_t)g;
@@ -227,7 +424,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           const float4 r3 = rec[3];
           m[3] = r3.x, m[4] = r3.y;
         }
-        finite = stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
+        stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
       } else {
         const float2 xy = means2D[g];
         const float4 co = conic_opacity[g];
@@ -237,219 +434,242 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
 #pragma unroll
           for (int ch = 0; ch < GS_N_MAP; ch++) m[ch] = all_map[5 * (size_t)g + ch];
         }
-        finite = stage(xy, co, c0, c1, c2, m);
+        stage(xy, co, c0, c1, c2, m);
       }
     }
-    {
-      const uint64_t bad_m = gs_ballot(!finite);
-      if (lane == 0) s_bad[wave] = bad_m != 0ull;
-    }
+    head += (uint32_t)count;
     __syncthreads();
-    const bool select_state = (s_bad[0] | s_bad[1] | s_bad[2] | s_bad[3]) != 0;
 
     for (int base = 0; base < count; base += SUB) {
       // Per-row lists: lane = slot of the sub-batch; the lanes whose Gaussian counts for row r append their slot
       // numbers to the row's list, in lane order (a lane's place is the number of set bits below its own).
-      uint32_t len0, len1, len2, len3;  // the lists' lengths (wave-uniform)
+      uint32_t passes;  // wave-uniform, like all that follows here: the longest of the four lists
+      bool exact, thin;
       {
-        static_assert(sizeof(s_idx[0]) == 4 * GS_WAVE, "a wave clears its own lists, one word per lane");
-        (&s_idx[wave][0][0])[lane] = 0u;
+        uint32_t* const words = &s_idx[wave][0][0];
+        static_assert(sizeof(s_idx[0]) == 8 * GS_WAVE, "a wave clears its own lists, two words per lane");
+        *reinterpret_cast<uint2*>(words + 2 * lane) = make_uint2((uint32_t)BATCH * 0x01010101u, (uint32_t)BATCH * 0x01010101u);
         const int jj = base + lane;
-        const bool valid = jj < count;
-        const uint64_t valid_m = gs_ballot(valid);  // (masks of single comparisons, combined in scalar registers)
-        float2 mu = make_float2(0.f, 0.f);
-        float4 cq = make_float4(0.f, 0.f, 0.f, 0.f), cp = cq;
-        uint32_t nibble = 0u;
-        if (HITS) {
-          nibble = (uint32_t)s_hits[valid ? jj : 0] >> (4 * wave);
-        } else {
-          const float4 xyf = s_xyf[valid ? jj : 0];
-          mu = make_float2(xyf.x, xyf.y);
-          cq = s_co[valid ? jj : 0];
-          cp = s_cp[valid ? jj : 0];
-        }
+        const int js = jj < count ? jj : BATCH;
+        const uint32_t nibble = jj < count ? (uint32_t)s_hits[jj] >> (4 * wave) & 15u : 0u;
         uint64_t hit_m[4];
-        bool hits[4] = {false, false, false, false};
-        if (!HITS) ellipse_hits_quadrant(mu, cq, cp.x, cp.y, cp.z, rt.qx0, rt.qy0, hits);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const bool touches = HITS ? ((nibble >> r) & 1u) != 0u : hits[r];
-          hit_m[r] = valid_m & gs_ballot((first_pos - jj) < row_last_of[r]) & gs_ballot(touches);
-        }
-        auto list_row = [&](auto row_tag) {
-          constexpr int r = decltype(row_tag)::value;
-          const uint64_t b = hit_m[r];
-          const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
-          if (__builtin_amdgcn_inverse_ballot_w64(b)) reinterpret_cast<uint8_t*>(&s_idx[wave][r][0])[below] = (uint8_t)lane;
-          return (uint32_t)__builtin_amdgcn_readfirstlane((int)__popcll(b));
+        for (int r = 0; r < 4; r++) hit_m[r] = gs_ballot(((nibble >> r) & 1u) != 0u);
+        auto list_row = [&](int r, uint64_t b, uint32_t from) {
+          const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, from));
+          if (__builtin_amdgcn_inverse_ballot_w64(b)) reinterpret_cast<uint8_t*>(&s_idx[wave][r][0])[below] = (uint8_t)jj;
+          return from + (uint32_t)__popcll(b);
         };
-        len0 = list_row(std::integral_constant<int, 0>{});
-        len1 = list_row(std::integral_constant<int, 1>{});
-        len2 = list_row(std::integral_constant<int, 2>{});
-        len3 = list_row(std::integral_constant<int, 3>{});
+        // The gradient of a thin Gaussian's covariance is a small difference of its three conic sums: a change in how
+        // they are rounded comes back multiplied by a c / (a c - b b), squared for scale and rotation.  Where a wave has
+        // such a Gaussian its conic sums are taken in a fixed order (`thin`: the sixteen pixels of a row as a tree; and
+        // `exact`, if three or four rows touch it: the rows by their places in the lists of a run of 64 positions, rows
+        // at the same place merged first), whatever else is staged or skipped.  Below THIN the factor is at most 25.
+        const float4 cq = s_co[js];
+        const bool is_thin = !(cq.y * cq.y < THIN * cq.x * cq.z);
+        thin = gs_ballot(is_thin && nibble != 0u) != 0ull;
+        exact = gs_ballot(is_thin && ((0xE880u >> nibble) & 1u) != 0u) != 0ull;
+        const uint32_t run = (uint32_t)(tile_last - 1 - __float_as_int(s_xyf[js].w)) / RUN;
+        const int last_lane = (count - base < SUB ? count - base : SUB) - 1;
+        const uint32_t first_run = (uint32_t)__builtin_amdgcn_readlane((int)run, 0);
+        const uint32_t last_run = (uint32_t)__builtin_amdgcn_readlane((int)run, last_lane);
+        if (!exact) {
+          const uint32_t l0 = list_row(0, hit_m[0], 0u), l1 = list_row(1, hit_m[1], 0u);
+          const uint32_t l2 = list_row(2, hit_m[2], 0u), l3 = list_row(3, hit_m[3], 0u);
+          passes = max(max(l0, l1), max(l2, l3));
+        } else {
+          // (a run that began in an earlier sub-batch has `carried` entries per row there)
+          const uint32_t least = min(min(carried[0], carried[1]), min(carried[2], carried[3]));
+          uint64_t todo = last_lane == SUB - 1 ? ~0ull : (1ull << (last_lane + 1)) - 1ull;
+          passes = 0u;
+          while (todo != 0ull) {
+            const uint32_t this_run = (uint32_t)__builtin_amdgcn_readlane((int)run, (int)__builtin_ctzll(todo));
+            const uint64_t run_m = todo & gs_ballot(run == this_run);
+            todo &= ~run_m;
+            uint32_t end = passes;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const uint32_t from = passes + (this_run == carried_run ? carried[r] - least : 0u);
+              end = max(end, list_row(r, hit_m[r] & run_m, from));
+            }
+            passes = end;
+          }
+        }
+        passes = (uint32_t)__builtin_amdgcn_readfirstlane((int)passes);
+        const uint64_t last_m = gs_ballot(run == last_run);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          carried[r] = (first_run == last_run && last_run == carried_run ? carried[r] : 0u) + (uint32_t)__popcll(hit_m[r] & last_m);
+        carried_run = last_run;
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const uint32_t my_len = row == 0 ? len0 : (row == 1 ? len1 : (row == 2 ? len2 : len3));
-      const uint32_t passes = max(max(len0, len1), max(len2, len3));  // wave-uniform
-      // The passes in which two rows of the wave are at the same Gaussian (their sums are merged before they go
-      // to the accumulator) are known as soon as the lists are: bit n of meet_m = entry n of two lists is the
-      // same slot.  Lane n looks at entry n of the four lists.
-      uint64_t meet_m;
-      {
-        const uint8_t* lists = reinterpret_cast<const uint8_t*>(&s_idx[wave][0][0]);
-        const uint32_t e0 = lists[lane], e1 = lists[SUB + lane], e2 = lists[2 * SUB + lane], e3 = lists[3 * SUB + lane];
-        const bool v0 = (uint32_t)lane < len0, v1 = (uint32_t)lane < len1, v2 = (uint32_t)lane < len2,
-                   v3 = (uint32_t)lane < len3;
-        meet_m = gs_ballot((v0 && v1 && e0 == e1) || (v0 && v2 && e0 == e2) || (v0 && v3 && e0 == e3) ||
-                           (v1 && v2 && e1 == e2) || (v1 && v3 && e1 == e3) || (v2 && v3 && e2 == e3));
-      }
-
-      // SELECT: a lane for which the Gaussian does not count takes the Gaussian's colour and geometry channels
-      // as 0 (its step then still only rotates the recurrence state: alpha = 0 with a finite colour), so that a
-      // non-finite channel only reaches the pixels that blended it in the forward pass, as in the reference
-      // (cuda_rasterizer/backward.cu:463-472).  Same bits for finite inputs.
-      auto walk = [&, my_len, passes, meet_m](auto select_tag) {
-        constexpr bool SELECT = decltype(select_tag)::value;
-        uint32_t word = 0u;  // four entries of the list
-        for (uint32_t n = 0; n < passes; n++) {
-          if ((n & 3u) == 0u) word = s_idx[wave][row][n >> 2];
-          const bool has = n < my_len;
-          const uint64_t has_m = gs_ballot(has);
-          // (slot 0 behind the end of the list: its data are this sub-batch's)
-          const int ja = (int)__builtin_amdgcn_ubfe(word, (n & 3u) * 8u, 8u);  // slot of the accumulators
-          const int j = base + ja;                                             // slot of the batch
-          const int pos = first_pos - j;
-          // Straight-line from here on: every lane evaluates its row's Gaussian, and a lane for which the
-          // Gaussian does not count (behind the pixel's last contributor, outside the power window, alpha
-          // below 1/255) takes part with alpha = 0, G = 0.  Such a step leaves T unchanged (T * 1/(1-0)),
-          // contributes zeros to every sum and leaves the recurrence state as it is
-          // (fma(0, c, 1 * accum) == accum), so results are those of skipping it.
-          // Same tests as the forward pass, on the same bits.
-          const float4 xy = s_xyf[j];
-          const float4 co = s_co[j];
-          const float dx = xy.x - pfx, dy = xy.y - pfy;
-          const float power = -0.5f * (co.x * dx * dx + co.z * dy * dy) - co.y * dx * dy;
-          // never true for pixels outside the image (last_contributor = 0)
-          const float floor_j = xy.z;
-          // (lane masks of single comparisons, combined in scalar registers: no short-circuit branches in the loop)
-          const uint64_t in_m = has_m & gs_ballot(pos < last_contributor) & gs_ballot(!(power > 0.0f)) &
-                                gs_ballot(!(power < floor_j));
-          if (in_m == 0ull) continue;  // wave-uniform
+      for (uint32_t n = 0; n < passes; n += GROUP) {
+        // Four entries of every row's list.  Lane e of each of the row's quads fetches entry e.
+        const uint32_t word = s_idx[wave][row][n / GROUP];
+        const uint32_t j_own = __builtin_amdgcn_ubfe(word, quad_shift, 8u);
+        const float4 xyf = s_xyf[j_own];
+        const float4 co = s_co[j_own];
+        // S = sum_ch c_ch g_ch of every (entry, pixel): a contraction over the channels, of the entries' colours and the
+        // pixels' upstream gradients.  Register e of lane p of a quad receives entry e at pixel p (one fused
+        // multiply-add per channel, in channel order: the bits of the same chain of vector instructions).
+        f32x4 S = {0.f, 0.f, 0.f, 0.f};
+        {
+          const float4 c4 = s_chan[j_own][0];
+          S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.x, gpix[0], S, 0, 0, 0);
+          S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.y, gpix[1], S, 0, 0, 0);
+          S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.z, gpix[2], S, 0, 0, 0);
+          if (render_geo) {
+            const float4 m4 = s_chan[j_own][RENDER_GEO ? 1 : 0];
+            S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.w, gmap[0], S, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f32_4x4x1f32(m4.x, gmap[1], S, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f32_4x4x1f32(m4.y, gmap[2], S, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f32_4x4x1f32(m4.z, gmap[3], S, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f32_4x4x1f32(m4.w, gmap[4], S, 0, 0, 0);
+          }
+        }
+        // The recurrence, entry after entry, lane = pixel.  Straight-line: every lane evaluates its row's Gaussian, and
+        // a lane for which it does not count (behind the pixel's last contributor, outside the power window, alpha
+        // below 1/255) takes part with alpha = 0, G = 0: T and what lies behind stay as they are, w and q are 0.
+        // Same tests as the forward pass, on the same bits.
+        float w[GROUP], q[GROUP];
+        auto step = [&](auto e_tag) {
+          constexpr int e = decltype(e_tag)::value;
+          const float dx = quad_lane<e>(xyf.x) - pfx, dy = quad_lane<e>(xyf.y) - pfy;
+          const float power = -0.5f * (quad_lane<e>(co.x) * dx * dx + quad_lane<e>(co.z) * dy * dy) -
+                              quad_lane<e>(co.y) * dx * dy;
+          const float floor_e = quad_lane<e>(xyf.z);
+          const int pos_e = __float_as_int(quad_lane<e>(xyf.w));
           const float G_raw = gs_expf_core(power);
-          const float alpha_raw = fminf(0.99f, co.w * G_raw);
-          const uint64_t active_m = in_m & gs_ballot(!(alpha_raw < 1.0f / 255.0f));
-          if (active_m == 0ull) continue;  // wave-uniform
+          const float alpha_raw = fminf(0.99f, quad_lane<e>(co.w) * G_raw);
+          // (lane masks of single comparisons, combined in scalar registers)
+          const uint64_t active_m = gs_ballot(pos_e < last_contributor) & gs_ballot(!(power > 0.0f)) &
+                                    gs_ballot(!(power < floor_e)) & gs_ballot(!(alpha_raw < 1.0f / 255.0f));
           const bool active = __builtin_amdgcn_inverse_ballot_w64(active_m);
           const float alpha = active ? alpha_raw : 0.f;
-          const float G = active ? G_raw : 0.f;
-
-          float v[NV];
           // The transmittance follows the CPU statement's operation sequence exactly (IEEE reciprocal):
           // upstream gradients of the geometry channels can be many orders of magnitude larger than the
           // result (plane depth divides by a blended normal that may be nearly perpendicular to the ray), so
-          // T, which multiplies them, decides how far a gradient can drift.  What follows dL/dalpha is
-          // products only.
-          const float rcp1ma = gs_rcp_normal(1.f - alpha);  // alpha <= 0.99: the bits of 1.f / (1.f - alpha)
-          T = T * rcp1ma;
-          const float w = alpha * T;
+          // T, which multiplies them, decides how far a gradient can drift.
           const float oma = 1.f - alpha;
-          float colour_dot = 0.0f;  // S
-          {
-            const float4 c4 = s_chan[j][0];
-            const float c[4] = {c4.x, c4.y, c4.z, c4.w};
+          const float rcp1ma = gs_rcp_normal(oma);  // alpha <= 0.99: the bits of 1.f / (1.f - alpha)
+          T = T * rcp1ma;
+          w[e] = alpha * T;
+          // (S may be NaN or infinite where the Gaussian does not count: a non-finite channel only reaches the pixels
+          // that blended it in the forward pass, as in the reference, cuda_rasterizer/backward.cu:463-472)
+          const float ahead = S[e] - behind_dot;
+          const float behind_next = __builtin_fmaf(alpha, S[e], oma * behind_dot);
+          behind_dot = active ? behind_next : behind_dot;
+          const float g_dalpha = G_raw * (ahead * T);
+          q[e] = active ? g_dalpha : 0.f;
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        // The sums over pixels.  From here on lane e of a quad works for entry e, register p is the quad's pixel p (four
+        // pixels of one image row).  The per-Gaussian factors of the geometric gradients stay out of the sums: with
+        // q = G dL/dalpha, u = conic (dx, dy), a pixel's terms are dL/dmean = -opacity q u,
+        // dL/dconic = -opacity/2 q (dx dx, dx dy, dy dy) and dL/dopacity = q
+        // (cuda_rasterizer/backward.cu:520-541); sum q u is formed from sum q (dx, dy) by the thread that hands the
+        // record over, sum q |u| here.  (The factors W/2 and H/2 from pixel to normalised coordinates are applied once
+        // per Gaussian by the reduction kernel.)
+        quad_transpose2(w, q);
+        f32x4 c_lo = {0.f, 0.f, 0.f, 0.f}, c_hi = {0.f, 0.f, 0.f, 0.f};  // sum_p w g: registers = channels
 #pragma unroll
-            for (int ch = 0; ch < GS_N_RGB; ch++) {
-              colour_dot = __builtin_fmaf((!SELECT || active) ? c[ch] : 0.f, gpix[ch], colour_dot);
-              v[8 + ch] = w * gpix[ch];
-            }
-            if (render_geo) {
-              const float4 m4 = s_chan[j][RENDER_GEO ? 1 : 0];
-              const float m[GS_N_MAP] = {c4.w, m4.x, m4.y, m4.z, m4.w};
-#pragma unroll
-              for (int ch = 0; ch < GS_N_MAP; ch++) {
-                colour_dot = __builtin_fmaf((!SELECT || active) ? m[ch] : 0.f, gmap[ch], colour_dot);
-                v[11 + ch] = w * gmap[ch];
-              }
-            } else {
-#pragma unroll
-              for (int ch = 0; ch < GS_N_MAP; ch++) v[11 + ch] = 0.f;
-            }
-          }
-          float dL_dalpha = colour_dot - behind_dot;
-          behind_dot = __builtin_fmaf(alpha, colour_dot, oma * behind_dot);  // (alpha = 0: unchanged)
-          dL_dalpha = __builtin_fmaf(dL_dalpha, T, -(bg_term * rcp1ma));
-          dL_dalpha = active ? dL_dalpha : 0.f;
-          // The per-Gaussian factors of the geometric gradients stay out of the pixel sums: with
-          // q = G dL/dalpha, u = conic (dx, dy), a pixel's terms are dL/dmean = -opacity q u,
-          // dL/dconic = -opacity/2 q (dx dx, dx dy, dy dy) and dL/dopacity = q
-          // (cuda_rasterizer/backward.cu:520-541), so the row sums q u, q (dx dx, dx dy, dy dy) and q, and the
-          // thread that hands a record over multiplies by -opacity, |opacity| (the sums of absolute values,
-          // formed inside the row reduction) and -opacity/2.  (The factors W/2 and H/2 from pixel to normalised
-          // coordinates are applied once per Gaussian by the reduction kernel.)
-          const float q = G * dL_dalpha;
-          const float ux = __builtin_fmaf(co.y, dy, co.x * dx), uy = __builtin_fmaf(co.y, dx, co.z * dy);
-          v[0] = q * ux;
-          v[1] = q * uy;
-          const float qx = q * dx;
-          v[4] = qx * dx;
-          v[5] = qx * dy;
-          v[6] = (q * dy) * dy;
-          v[7] = q;
-          // lane q of the row now receives the row's total of component q
-          float tot = row_transpose_reduce16_abs23(v);
-          // Rows of this wave that are at the same Gaussian in this pass are merged, and the lowest of them
-          // adds the sum to the wave's own accumulator with a plain read-add-write: rows that write hold
-          // different Gaussians, so their addresses differ.  (An LDS float atomic takes about three cycles per
-          // active lane on this hardware, thirteen times the read-add-write.)
-          bool writes = has;
-          if ((meet_m >> n) & 1ull) {  // wave-uniform, uncommon
-            const int key = has ? ja : -1 - row;
-            const int k0 = __builtin_amdgcn_readlane(key, 0), k1 = __builtin_amdgcn_readlane(key, 16);
-            const int k2 = __builtin_amdgcn_readlane(key, 32), k3 = __builtin_amdgcn_readlane(key, 48);
-            constexpr uint64_t R0 = 0xFFFFull, R1 = R0 << 16, R2 = R0 << 32, R3 = R0 << 48;
-            const uint64_t eq16 = (k0 == k1 ? R0 | R1 : 0ull) | (k2 == k3 ? R2 | R3 : 0ull);
-            const uint64_t eq32 = (k0 == k2 ? R0 | R2 : 0ull) | (k1 == k3 ? R1 | R3 : 0ull);
-            const uint64_t eq48 = (k0 == k3 ? R0 | R3 : 0ull) | (k1 == k2 ? R1 | R2 : 0ull);
-            const uint64_t follower = (k1 == k0 ? R1 : 0ull) | ((k2 == k0 || k2 == k1) ? R2 : 0ull) |
-                                      ((k3 == k0 || k3 == k1 || k3 == k2) ? R3 : 0ull);
-            const float t16 = __shfl_xor(tot, 16, GS_WAVE), t32 = __shfl_xor(tot, 32, GS_WAVE);
-            const float t48 = __shfl_xor(tot, 48, GS_WAVE);
-            tot += __builtin_amdgcn_inverse_ballot_w64(eq16) ? t16 : 0.f;
-            tot += __builtin_amdgcn_inverse_ballot_w64(eq32) ? t32 : 0.f;
-            tot += __builtin_amdgcn_inverse_ballot_w64(eq48) ? t48 : 0.f;
-            writes = has && !__builtin_amdgcn_inverse_ballot_w64(follower);
-          }
-          if (writes && tot != 0.f) s_acc[wave][l16][ja] += tot;
+        for (int p = 0; p < 4; p++) {
+          c_lo = __builtin_amdgcn_mfma_f32_4x4x1f32(grad_t[0][p], w[p], c_lo, 0, 0, 0);
+          if (render_geo) c_hi = __builtin_amdgcn_mfma_f32_4x4x1f32(grad_t[RENDER_GEO ? 1 : 0][p], w[p], c_hi, 0, 0, 0);
         }
-      };
-      if (select_state) walk(std::true_type{});
-      else walk(std::false_type{});
+        const float dx = xyf.x - pfx, a_dx = co.x * dx, b_dx = co.y * dx;
+        float dy[4], q_dy[4], ax = 0.f, ay = 0.f;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+          dy[p] = xyf.y - (block_y0 + (float)p);
+          q_dy[p] = q[p] * dy[p];
+          const float ux = __builtin_fmaf(co.y, dy[p], a_dx), uy = __builtin_fmaf(co.z, dy[p], b_dx);
+          ax = __builtin_fmaf(fabsf(q[p]), fabsf(ux), ax);
+          ay = __builtin_fmaf(fabsf(q[p]), fabsf(uy), ay);
+        }
+        auto sum4 = [](const float (&t)[4]) { return (t[0] + t[2]) + (t[1] + t[3]); };
+        const float q0 = sum4(q), qy = sum4(q_dy);
+        float qx = q0 * dx, xx = qx * dx, xy = qy * dx;
+        float yy = __builtin_fmaf(q_dy[3], dy[3], __builtin_fmaf(q_dy[2], dy[2], __builtin_fmaf(q_dy[1], dy[1], q_dy[0] * dy[0])));
+        if (thin) {  // (every product rounded by itself, sums as a tree over y, then x)
+          float t0[4], t1[4], t2[4], t3[4];
+#pragma unroll
+          for (int p = 0; p < 4; p++) {
+            t0[p] = q[p] * dx;
+            t1[p] = t0[p] * dx;
+            t2[p] = t0[p] * dy[p];
+            t3[p] = q_dy[p] * dy[p];
+          }
+          qx = sum4(t0); xx = sum4(t1); xy = sum4(t2); yy = sum4(t3);
+        }
+        float v[16] = {qx, qy, ax, ay, xx, xy, yy, q0, c_lo[0], c_lo[1], c_lo[2], c_lo[3],
+                       c_hi[0], c_hi[1], c_hi[2], c_hi[3]};
+        quads_reduce16<RENDER_GEO>(v);
+        // Quad k of a row now holds components 4 k .. 4 k + 3 of its entry e.  They go into the wave's own accumulator with
+        // a plain read-add-write (the LDS accesses of a wave complete in order), one row after the other, since two rows
+        // may be at the same Gaussian.  An LDS float atomic takes about three cycles per active lane.
+        const uint32_t a_slot = j_own - (uint32_t)base;
+        float4* const acc = &s_acc[wave][4u * (a_slot & (SUB - 1)) + (quad ^ ((a_slot >> 2) & 3u))];
+        uint64_t write_m = gs_ballot(j_own < (uint32_t)BATCH);
+        if (exact) {
+          const float own[4] = {v[0], v[1], v[2], v[3]};
+#pragma unroll
+          for (int d = 1; d < 4; d++) {
+            // (entries behind the ends of two lists are the same too: their sums are zero and go nowhere)
+            const bool same = (uint32_t)__shfl_xor((int)j_own, 16 * d, GS_WAVE) == j_own;
+            float t[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) t[k] = __shfl_xor(own[k], 16 * d, GS_WAVE);
+            if (same) {
+#pragma unroll
+              for (int k = 0; k < 4; k++) v[k] += t[k];
+            }
+            write_m &= ~gs_ballot(same && (row ^ d) < row);
+          }
+        }
+        // (exact: entry after entry; otherwise row after row)
+        uint64_t turn_m = exact ? 0x1111111111111111ull : 0xFFFFull;
+        const int turn_shift = exact ? 1 : 16;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if (__builtin_amdgcn_inverse_ballot_w64(write_m & turn_m)) {
+            float4 a = *acc;
+            a.x += v[0]; a.y += v[1]; a.z += v[2]; a.w += v[3];
+            *acc = a;
+          }
+          turn_m <<= turn_shift;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+      }
       __syncthreads();
       // a thread stores a quarter of a record: the four waves' sums of four components, added in wave order;
       // it leaves zeros behind for the next sub-batch
       {
-        float c[4];
+        float4 c = s_acc[0][my_word];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          c[e] = s_acc[0][4 * my_part + e][my_slot];
-          s_acc[0][4 * my_part + e][my_slot] = 0.f;
-#pragma unroll
-          for (int w = 1; w < WAVES; w++) {
-            c[e] += s_acc[w][4 * my_part + e][my_slot];
-            s_acc[w][4 * my_part + e][my_slot] = 0.f;
-          }
+        for (int w = 1; w < WAVES; w++) {
+          const float4 o = s_acc[w][my_word];
+          c.x += o.x; c.y += o.y; c.z += o.z; c.w += o.w;
         }
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) s_acc[w][my_word] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (base + my_slot < count) {
-          const float opacity = s_co[base + my_slot].w;
+          const float4 co = s_co[base + my_slot];
           if (my_part == 0) {  // mean2D x, y and their sums of absolute values
-            c[0] *= -opacity; c[1] *= -opacity; c[2] *= fabsf(opacity); c[3] *= fabsf(opacity);
+            c = make_float4(-co.w * (co.x * c.x + co.y * c.y), -co.w * (co.y * c.x + co.z * c.y), c.z * fabsf(co.w),
+                            c.w * fabsf(co.w));
           } else if (my_part == 1) {  // conic x, y, w; the fourth component is the opacity gradient itself
-            const float h = -0.5f * opacity;
-            c[0] *= h; c[1] *= h; c[2] *= h;
+            const float h = -0.5f * co.w;
+            c.x *= h; c.y *= h; c.z *= h;
           }
-          instance_grads[4 * (size_t)s_emis[base + my_slot] + my_part] = make_float4(c[0], c[1], c[2], c[3]);
+          instance_grads[4 * (size_t)s_emis[base + my_slot] + my_part] = c;
         }
       }
       __syncthreads();
