@@ -1,0 +1,63 @@
+"""Backward blend at the list lengths where its steps change: four entries per pass, sub-batches of 64 slots, staged
+batches of 128, scans of 256 positions, runs of 64; with and without thin Gaussians (whose sums keep a fixed order), on
+an image whose last tiles are cut off, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def H():
+    import gpu_harness
+    return gpu_harness
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 127, 128, 129, 256, 257, 700])
+@pytest.mark.parametrize("thin,geo", [(False, True), (True, True), (True, False)])
+def test_list_lengths(H, orc, n, thin, geo):
+    gen = torch.Generator().manual_seed(n)
+    r = lambda *s: torch.rand(*s, generator=gen)
+    W, Hh, tan = 41, 27, 0.5
+    means2D = (r(n, 2) * torch.tensor([W + 8.0, Hh + 8.0]) - 4.0).numpy()
+    s1 = torch.exp(r(n) * 2.5)
+    s2 = s1 * torch.where(r(n) < 0.5, 0.05, 0.6) if thin else s1 * (0.4 + 0.6 * r(n))
+    s2 = torch.clamp(s2, min=0.55)
+    ang = r(n) * 3.14159
+    c, s = torch.cos(ang), torch.sin(ang)
+    i1, i2 = 1 / s1 ** 2, 1 / s2 ** 2
+    opac = r(n) * (0.9 if n < 100 else 0.08) + 0.01
+    co = torch.stack([c * c * i1 + s * s * i2, c * s * (i1 - i2), s * s * i1 + c * c * i2, opac], 1).float().numpy()
+    radii = torch.ceil(3 * s1).int().numpy()
+    depths = (r(n) * 10 + 1).numpy()
+    rgb = r(n, 3).numpy()
+    am = torch.randn(n, 5, generator=gen)
+    am[:, 2] = am[:, 2].abs() + 2.0  # faces the camera: the plane depth stays well conditioned
+    am[:, 3] = 1.0
+    am = am.numpy()
+    gx, gy = H.grid(W, Hh)
+    cl = np.ones(gx * gy, bool)
+    bg = np.array([0.3, 0.6, 0.1], np.float32)
+    b = orc.bin_and_sort(radii, means2D, depths, cl, W, Hh)
+    f = orc.render_fwd(b["ranges"], b["point_list"], means2D, rgb, am, co, cl, bg, W, Hh, tan, tan, render_geo=geo)
+    gpix, gmap, gdep = (torch.randn(k, Hh, W, generator=gen).numpy() for k in (3, 5, 1))
+    ref = orc.render_bwd(b["ranges"], b["point_list"], means2D, co, rgb, am, f["out_all_map"], f["final_T"],
+                         f["n_contrib"], cl, bg, gpix, gmap, gdep, W, Hh, tan, tan, render_geo=geo)
+
+    def run():
+        return H.render_bwd(n, W, Hh, tan, tan, H.dev(bg), H.as_u32(b["ranges"]), H.as_u32(b["point_list"]),
+                            H.dev(means2D), H.dev(co), H.dev(rgb), H.dev(am), H.dev(f["out_all_map"]),
+                            H.dev(f["final_T"]), H.as_u32(f["n_contrib"]), H.dev(cl), H.dev(gpix), H.dev(gmap),
+                            H.dev(gdep), H.as_u32(b["emission_sorted"]), H.as_u32(b["point_offsets"]), render_geo=geo)
+
+    got, again = run(), run()
+    # 24-bit sums of at most 700 x 256 terms in another order: about sqrt(terms) * 2^-24 of the sum of magnitudes,
+    # which is some ten times the sum itself
+    for k, want in (("dL_dmeans2D", ref["dL_dmeans2D"][:, :2]), ("dL_dmeans2D_abs", ref["dL_dmeans2D_abs"]),
+                    ("dL_dconic_opacity", ref["dL_dconic_opacity"]), ("dL_dcolors", ref["dL_dcolors"]),
+                    ("dL_dall_map", ref["dL_dall_map"])):
+        if k == "dL_dall_map" and not geo:
+            continue
+        assert torch.equal(got[k], again[k]), k
+        assert H.rel_l2(got[k].cpu().numpy(), want) <= 1e-4, (k, H.rel_l2(got[k].cpu().numpy(), want))
