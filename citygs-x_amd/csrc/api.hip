@@ -115,7 +115,7 @@ inline void tile_grid(int W, int H, int& gx, int& gy) {
 }
 
 struct ImageLayout {
-  size_t accum_alpha, n_contrib, n_contrib2loss, ranges, bucket_table, total;
+  size_t accum_alpha, n_contrib, n_contrib2loss, ranges, bucket_table, tile_order, total;
 };
 ImageLayout image_layout(int W, int H) {
   ImageLayout L;
@@ -130,6 +130,7 @@ ImageLayout image_layout(int W, int H) {
   L.ranges = take((size_t)gx * gy * 8);
   // workgroup-by-tile counts of the counting sort by tile (nothing when the grid is too large for it)
   L.bucket_table = take(gx * gy <= bucket_max_tiles() ? bucket_table_bytes(gx * gy) : 0);
+  L.tile_order = take(gx * gy <= bucket_max_tiles() ? (size_t)gx * gy * 4 : 0);  // see launch_tile_sort
   L.total = off + 256;
   return L;
 }
@@ -145,7 +146,9 @@ GeometryLayout geometry_layout(int P) {
   L.tiles_touched = take(n * 4);
   L.point_offsets = take(n * 4);
   L.scan_temp = take(scan_temp_bytes((int64_t)n));
-  L.packed_valid = take(4);  // one word: whether the forward call packed operand records (binning buffer)
+  // two words: whether the forward call packed operand records (binning buffer), and whether it left an order of the
+  // tiles (image buffer)
+  L.packed_valid = take(8);
   L.total = off + 256;
   return L;
 }
@@ -540,6 +543,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   uint32_t* n_contrib_px = (uint32_t*)(ibase + IL.n_contrib);
   uint32_t* n_contrib2loss_px = (uint32_t*)(ibase + IL.n_contrib2loss);
   uint32_t* ranges = (uint32_t*)(ibase + IL.ranges);
+  uint32_t* tile_order = (uint32_t*)(ibase + IL.tile_order);
 
   // Two ways to the sorted per-tile lists.  The default buckets the instances by tile (counting sort) and sorts
   // every tile's list on its own; it needs the tile histogram to fit in LDS.  Otherwise: emit (tile | depth) keys,
@@ -577,6 +581,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     StageScope _t("tile_count", stream);
     // also clears the tile ranges (cudaMemset of CR/rasterizer_impl.cu:687), which nothing reads before
     // identify_tile_ranges fills them
+    launch_fill_u32(2, 0u, packed_valid, stream);
     launch_tile_count(P, width, height, radii, means2D, compute_locally, tiles_touched, stream, ranges,
                       (int64_t)2 * T, out_observe);
   }
@@ -626,19 +631,15 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   };
   // Packs the library's own records into the arrays just carved.  With the caller's records, or none, the word
   // beside them must say "none" (a backward call that is not handed the caller's records again then gathers the
-  // operands from the arrays): the counting kernels of the per-tile route have cleared it on their way.
+  // operands from the arrays): the counting step has cleared it.
   auto pack_records = [&](const Arrays& A) -> int {
-    if (caller_records != nullptr || !use_packed) {
-      if (bucketed) return 0;
-      launch_fill_u32(1, 0u, packed_valid, stream);
-      return check_launch("pack_operands", stream, dbg);
-    }
+    if (caller_records != nullptr || !use_packed) return 0;
     StageScope _t("pack_operands", stream);
     launch_pack_blend_operands(P, radii, means2D, conic_opacity, rgb, render_geo ? all_map : nullptr, depths,
                                A.packed, packed_valid, stream);
     return check_launch("pack_operands", stream, dbg);
   };
-  auto blend = [&](const Arrays& A, bool ahead_of_host) -> int {
+  auto blend = [&](const Arrays& A, bool ordered, bool ahead_of_host) -> int {
     RenderFwdArgs a;
     a.P = P; a.W = width; a.H = height;
     a.fx = focal_x; a.fy = focal_y; a.cx = cx; a.cy = cy;
@@ -653,6 +654,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     a.fits_word = ahead_of_host ? bucket_fits_word(bucket_table, T) : nullptr;
     a.block_hits = A.block_hits;
     a.packed = use_packed ? (caller_records != nullptr ? caller_records : A.packed) : nullptr;
+    a.tile_order = ordered ? tile_order : nullptr;
     {
       StageScope _t("render_fwd", stream);
       launch_render_fwd(a, stream);
@@ -673,7 +675,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
       StageScope _t("tile_sort", stream);
       if (launch_tile_sort(T, longest_for_launch, radix_tiles, sort_limit, (uint32_t)limits.block, ranges,
                            bucket_table, A.keys_other, A.radix_scratch, A.capacity, A.keys, A.emission,
-                           A.point_list, ahead_of_host, stream))
+                           A.point_list, tile_order, packed_valid + 1, ahead_of_host, stream))
         return 1;
     }
     return check_launch("tile_sort", stream, dbg);
@@ -687,7 +689,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     if (timer.begin(elapsed_ms != nullptr, stream)) return 1;
     if (pack_records(A)) return 1;
     if (lists_by_tile(A, cap_longest, 0xFFFFFFFFu, true)) return 1;
-    if (blend(A, true)) return 1;
+    if (blend(A, cap_longest > 0, true)) return 1;
   }
 
   // The host needs the instance count: it sizes the binning buffer (unless that was done ahead), and the caller
@@ -782,7 +784,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     if (check_launch("identify_tile_ranges", stream, dbg)) return 1;
   }
 
-  if (blend(A, false)) return 1;
+  if (blend(A, bucketed && longest > 0, false)) return 1;
   if (timer.end(stream, elapsed_ms)) return 1;
   // (debug mode and the timer have waited for the stream: a sort that gave up in this call is known by now)
   if ((dbg || elapsed_ms != nullptr) && pending_fault("gs_render_forward")) return 1;
@@ -831,6 +833,14 @@ int gs_render_backward(int P, int R, const float* background, int width, int hei
   a.fx = width / (2.0f * tan_fovx);
   a.bg = background;
   a.ranges = (const uint32_t*)(ibase + IL.ranges);
+  {
+    int gx, gy;
+    tile_grid(width, height, gx, gy);
+    if (gx * gy <= bucket_max_tiles()) {
+      a.tile_order = (const uint32_t*)(ibase + IL.tile_order);
+      a.tile_order_valid = (const uint32_t*)(gbase + GL.packed_valid) + 1;
+    }
+  }
   a.point_list = (const uint32_t*)(bbase + BL.point_list);
   a.means2D = means2D; a.conic_opacity = conic_opacity; a.rgb = rgb; a.all_map = all_maps;
   a.all_map_pixels = all_map_pixels;

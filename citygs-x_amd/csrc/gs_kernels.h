@@ -106,7 +106,8 @@ size_t bucket_table_bytes(int T);
 // (word 2: larger kernel's << 16 | smaller kernel's).  block_limit (0 = the maximum): the records the radix sort
 // holds in one block, see launch_tile_sort.
 // cap_instances / cap_longest: what kernels launched ahead of the host's decision were sized for; the ranges kernel
-// leaves 1 in bucket_fits_word(table) if the view has at most that many instances and no longer list, else 0
+// leaves 1 in bucket_fits_word(table) if the view has at most that many instances and no longer list, else 0.
+// clear_word: two words the ranges kernel clears
 int launch_bucket_count(int P, int W, int H, const int* radii, const float* means2D, const uint8_t* compute_locally,
                         uint32_t* tiles_touched, void* table, uint32_t* ranges, uint32_t small_limit,
                         uint32_t block_limit, uint32_t* host_words, int* zero_per_gaussian, uint32_t cap_instances,
@@ -123,8 +124,8 @@ int launch_bucket_scatter(int P, int W, int H, const float* means2D, const float
 // scratch: 24 bytes per instance, used for lists of more than block_limit records
 int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t small_limit, uint32_t block_limit,
                      const uint32_t* ranges, const void* table, const void* records, void* scratch, int64_t capacity,
-                     uint64_t* keys, uint32_t* emission, uint32_t* point_list, bool ahead_of_host,
-                     hipStream_t stream);
+                     uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
+                     uint32_t* tile_order_valid, bool ahead_of_host, hipStream_t stream);
 int tile_radix_mid_records();    // records one workgroup of the radix sort's smaller kernel holds (4096)
 int tile_radix_block_records();  // ... and of its larger kernel (16384): longer lists are sorted in blocks
 int launch_tile_radix_sort(int T, bool mid, bool lng, const uint32_t* ranges, const uint32_t* tile_lists,
@@ -241,6 +242,7 @@ struct RenderFwdArgs {
   // optional (P,4) 16-byte words: pack_blend_operands' records; the kernel then fetches a Gaussian's operands as
   // one 64-byte line instead of gathering them from means2D, conic_opacity, rgb, all_map (and depths)
   const float* packed = nullptr;
+  const uint32_t* tile_order = nullptr;  // optional (T): the order in which the tiles are taken (launch_tile_sort)
 };
 int launch_render_fwd(const RenderFwdArgs& a, hipStream_t stream);
 
@@ -264,6 +266,9 @@ struct RenderBwdArgs {
   const float* packed = nullptr;         // optional (P,4) 16-byte words: see RenderFwdArgs::packed
   // optional device word beside `packed`: non-zero if the forward call did pack the records (it decides per view)
   const uint32_t* packed_valid = nullptr;
+  // optional (T): the order in which the tiles are taken, if the device word beside it is not zero
+  const uint32_t* tile_order = nullptr;
+  const uint32_t* tile_order_valid = nullptr;
   // outputs, fully written by the per-Gaussian reduction
   float* dL_dmean2D;         // (P,2)
   float* dL_dmean2D_abs;     // (P,3)

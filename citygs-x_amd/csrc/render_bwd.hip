@@ -193,7 +193,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                   const float* __restrict__ dL_dout_all_map, const float* __restrict__ dL_dout_plane_depth,
                   const uint32_t* __restrict__ emission_sorted, float4* __restrict__ instance_grads,
                   const uint16_t* __restrict__ block_hits, const float4* __restrict__ packed_records,
-                  const uint32_t* __restrict__ packed_valid) {
+                  const uint32_t* __restrict__ packed_valid, const uint32_t* __restrict__ tile_order,
+                  const uint32_t* __restrict__ tile_order_valid, uint32_t tiles_x) {
   // (whether the forward call packed the records is its decision per view: a word beside them says)
   const float4* packed = (packed_records != nullptr && (packed_valid == nullptr || *packed_valid != 0u))
                              ? packed_records : nullptr;
@@ -217,9 +218,14 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   __shared__ int4 s_row_last[WAVES];  // the deepest contributor of every row
 
   const int tid = threadIdx.x;
-  const RowThread rt = row_thread(blockIdx.x, blockIdx.y);
+  uint32_t tile = blockIdx.x;
+  if (tile_order != nullptr) {
+    const uint32_t ordered = tile_order[blockIdx.x];
+    tile = *tile_order_valid != 0u ? ordered : tile;
+  }
+  const uint32_t tile_y = tile / tiles_x, tile_x = tile - tile_y * tiles_x;
+  const RowThread rt = row_thread(tile_x, tile_y);
   const int lane = rt.lane, wave = rt.wave, row = rt.row;
-  const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
   // (a quad of lanes holds one column of the row's 4x4 block: see the order of the sums below)
   const uint32_t px = (uint32_t)rt.qx0 + (uint32_t)(row & 1) * 4u + (uint32_t)(rt.l16 >> 2);
   const uint32_t py = (uint32_t)rt.qy0 + (uint32_t)(row >> 1) * 4u + (uint32_t)(rt.l16 & 3);
@@ -337,7 +343,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     const uint32_t g = point_list[range.x + (uint32_t)pos];
     const float2 xy = means2D[g];
     const float4 co = conic_opacity[g];
-    const float tile_x0 = (float)(blockIdx.x * GS_TILE_X), tile_y0 = (float)(blockIdx.y * GS_TILE_Y);
+    const float tile_x0 = (float)(tile_x * GS_TILE_X), tile_y0 = (float)(tile_y * GS_TILE_Y);
     float pfl, mark_limit;
     const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
     uint32_t found = 0u;
@@ -409,7 +415,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         s_emis[tid] = emission_sorted[k_sorted];
         s_co[tid] = co;
         float pfl, mark_limit;
-        (void)block_test_params(co, xy, (float)(blockIdx.x * GS_TILE_X), (float)(blockIdx.y * GS_TILE_Y), pfl,
+        (void)block_test_params(co, xy, (float)(tile_x * GS_TILE_X), (float)(tile_y * GS_TILE_Y), pfl,
                                 mark_limit);
         s_hits[tid] = s_pend_hits[at];
         s_xyf[tid] = make_float4(xy.x, xy.y, pfl, __int_as_float(pos));
@@ -790,13 +796,13 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
 }  // namespace
 
 int launch_render_bwd(const RenderBwdArgs& a, hipStream_t stream) {
-  const dim3 grid((a.W + GS_TILE_X - 1) / GS_TILE_X, (a.H + GS_TILE_Y - 1) / GS_TILE_Y, 1);
+  const uint32_t gx = (a.W + GS_TILE_X - 1) / GS_TILE_X, gy = (a.H + GS_TILE_Y - 1) / GS_TILE_Y;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges, a.point_list, a.W, a.H,
+    hipLaunchKernelGGL(kernel, dim3(gx * gy), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges, a.point_list, a.W, a.H,
                        a.fx, a.fy, a.bg, (const float2*)a.means2D, (const float4*)a.conic_opacity, a.rgb, a.all_map,
                        a.all_map_pixels, a.final_T, a.n_contrib_px, a.compute_locally, a.dL_dpix, a.dL_dout_all_map,
                        a.dL_dout_plane_depth, a.emission_sorted, (float4*)a.instance_grads, a.block_hits,
-                       (const float4*)a.packed, a.packed_valid);
+                       (const float4*)a.packed, a.packed_valid, a.tile_order, a.tile_order_valid, gx);
   };
   if (a.render_geo) {
     if (a.block_hits) go(render_bwd_kernel<true, true>);

@@ -70,7 +70,8 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                   float* __restrict__ out_plane_depth, int* __restrict__ n_render, int* __restrict__ n_consider,
                   int* __restrict__ n_contrib_tile, const float* __restrict__ depths,
                   float* __restrict__ out_max_weight_depth, const uint32_t* __restrict__ fits_word,
-                  uint16_t* __restrict__ block_hits, const float4* __restrict__ packed) {
+                  uint16_t* __restrict__ block_hits, const float4* __restrict__ packed,
+                  const uint32_t* __restrict__ tile_order, uint32_t tiles_x) {
   constexpr bool render_geo = RENDER_GEO;
   // launched ahead of the host's decision on how the per-tile lists are built: nothing to do if they were not
   if (fits_word != nullptr && *fits_word == 0u) return;
@@ -97,9 +98,10 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   __shared__ int s_red[2][GS_TILE_PIX / GS_WAVE];
 
   const int tid = threadIdx.x;
-  const RowThread rt = row_thread(blockIdx.x, blockIdx.y);
+  const uint32_t tile = tile_order != nullptr ? tile_order[blockIdx.x] : blockIdx.x;
+  const uint32_t tile_y = tile / tiles_x, tile_x = tile - tile_y * tiles_x;
+  const RowThread rt = row_thread(tile_x, tile_y);
   const int lane = rt.lane, wave = rt.wave, row = rt.row;
-  const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
   const uint2 range = ranges[tile];
   if (tid == 0) n_render[tile] = (int)(range.y - range.x);
   const uint32_t px = rt.px, py = rt.py;
@@ -140,6 +142,8 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   float Mp[GS_N_MAP] = {0.f, 0.f, 0.f, 0.f, 0.f};
   float best_w = 0.f, best_depth = 0.f;
 
+  // (the Gaussian of a thread's slot is fetched one batch ahead: the operands' address is known when a batch starts)
+  uint32_t g_next = tid < todo ? point_list[range.x + (uint32_t)tid] : 0u;
   for (int i = 0; i < rounds; i++, todo -= BATCH) {
     const uint64_t alive_mask = alive;
     if (lane == 0) s_done[wave] = alive_mask == 0ull;
@@ -152,8 +156,9 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     // the variant of the loop that selects instead (below).
     bool finite = true;
     const int ts = not_hoisted(tid);
+    const uint32_t g = g_next;
+    if (ts + BATCH < todo) g_next = point_list[range.x + (uint32_t)(i + 1) * BATCH + ts];
     if (ts < count) {
-      const uint32_t g = point_list[range.x + (uint32_t)i * BATCH + ts];
       // A Gaussian's operands: one 64-byte record where the caller had them packed (a single line of memory,
       // every byte of it used), else gathered from the five arrays.  (Each route loads and then stages by itself:
       // with the loaded values merged across the two routes the compiler splits the gathers into single words.)
@@ -163,7 +168,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // rounding per operation: the mark limit's margin covers both, and the blend tests the exponent itself
         // again)
         float pfl, mark_limit;
-        s_cull[ts] = block_test_params(co, xy, (float)(blockIdx.x * GS_TILE_X), (float)(blockIdx.y * GS_TILE_Y), pfl,
+        s_cull[ts] = block_test_params(co, xy, (float)(tile_x * GS_TILE_X), (float)(tile_y * GS_TILE_Y), pfl,
                                        mark_limit);
         s_geo0[ts] = make_float4(xy.x, xy.y, co.x, co.y);
         s_geo1[ts] = make_float4(co.z, mark_limit, co.w, pfl);
@@ -450,13 +455,13 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
 
 template <bool GEO, bool MAXD>
 static void launch_render_fwd_variant(const RenderFwdArgs& a, hipStream_t stream) {
-  const dim3 grid((a.W + GS_TILE_X - 1) / GS_TILE_X, (a.H + GS_TILE_Y - 1) / GS_TILE_Y, 1);
-  hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD>), grid, dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges,
+  const uint32_t gx = (a.W + GS_TILE_X - 1) / GS_TILE_X, gy = (a.H + GS_TILE_Y - 1) / GS_TILE_Y;
+  hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD>), dim3(gx * gy), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges,
                      a.point_list, a.W, a.H, a.fx, a.fy, a.cx, a.cy, (const float2*)a.means2D, a.rgb, a.all_map,
                      (const float4*)a.conic_opacity, a.compute_locally, a.bg, a.final_T, a.n_contrib_px,
                      a.n_contrib2loss_px, a.out_color, a.out_observe, a.out_all_map, a.out_plane_depth, a.n_render,
                      a.n_consider, a.n_contrib_tile, a.depths, a.out_max_weight_depth, a.fits_word, a.block_hits,
-                     (const float4*)a.packed);
+                     (const float4*)a.packed, a.tile_order, gx);
 }
 
 int launch_render_fwd(const RenderFwdArgs& a, hipStream_t stream) {

@@ -271,7 +271,7 @@ bucket_ranges_kernel(uint32_t T, uint32_t small_limit, uint32_t mid_limit, uint3
     }
     tile_lists[T] = carry_class;
     tile_lists[T + 1u] = carry_split;
-    if (clear_word != nullptr) *clear_word = 0u;  // (a word the caller wants cleared on the way: saves a launch)
+    if (clear_word != nullptr) clear_word[0] = clear_word[1] = 0u;  // (two words the caller wants cleared: saves a launch)
     // more instances than 32-bit positions can address: the host must not go on with the wrapped count
     const uint32_t reported = all > (double)GS_MAX_INSTANCES ? GS_TOO_MANY_INSTANCES : carry;
     // Kernels launched ahead of the host's decision (buffers sized from the caller's expectation) look at this
@@ -780,6 +780,35 @@ __device__ __forceinline__ void register_sort_tile(uint32_t t, uint32_t start, u
   }
 }
 
+// The order in which the blend kernels take the tiles: by falling length of the lists, in steps of half a power of two.  A
+// tile's workgroup works for as long as its list is, and workgroups start in the order of their numbers: taken row by
+// row, a street-level view (10 M Gaussians, 1920x1080, lists up to 28 000 entries along the horizon, half way down
+// the image) ends with a few long tiles on an idle chip (backward blend 904 -> 716 us, forward 610 -> 564; views from
+// the air, whose lists differ less, take the same time either way).  The place inside a class is whatever the LDS counter
+// hands out (about ascending): no result depends on it.
+__device__ __forceinline__ void order_tiles(uint32_t T, const uint32_t* __restrict__ ranges, uint32_t* __restrict__ order,
+                                            uint32_t* __restrict__ order_valid, uint32_t* s_count) {
+  constexpr int CLASSES = 64;
+  auto class_of = [&](uint32_t t) {  // 0 = the longest lists
+    const uint32_t n = ranges[2 * t + 1] - ranges[2 * t];
+    if (n == 0) return CLASSES - 1;
+    const int msb = 31 - __clz((int)n);
+    return CLASSES - 2 - (2 * msb + (msb > 0 ? (int)((n >> (msb - 1)) & 1u) : 0));
+  };
+  if (threadIdx.x < CLASSES) s_count[threadIdx.x] = 0u;
+  __syncthreads();
+  for (uint32_t t = threadIdx.x; t < T; t += blockDim.x) atomicAdd(&s_count[class_of(t)], 1u);
+  __syncthreads();
+  if (threadIdx.x < CLASSES) {  // (one wave)
+    const uint32_t c = s_count[threadIdx.x];
+    s_count[threadIdx.x] = wave_inclusive_scan_u32(c, (int)threadIdx.x) - c;
+  }
+  __syncthreads();
+  for (uint32_t t = threadIdx.x; t < T; t += blockDim.x) order[atomicAdd(&s_count[class_of(t)], 1u)] = t;
+  if (threadIdx.x == 0) *order_valid = 1u;
+}
+
+// Workgroup 0 orders the tiles for the blend kernels, workgroup t + 1 sorts tile t.
 // Dynamic LDS: 8 bytes per record of the longest list the kernel takes, rounded up to a power of two (at least
 // 256 records).  Lists of more than max_n records are left to the radix sort's kernels.
 #define GS_SORT_CASE(EE, WW) register_sort_tile<EE, WW>(t, start, n, records, keys, emission, point_list, s_exchange)
@@ -787,10 +816,15 @@ __global__ void __launch_bounds__(512)
 tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord* __restrict__ records,
                            uint64_t* __restrict__ keys, uint32_t* __restrict__ emission,
                            uint32_t* __restrict__ point_list, uint32_t max_n,
-                           const uint32_t* __restrict__ fits_word) {
+                           const uint32_t* __restrict__ fits_word, uint32_t* __restrict__ order,
+                           uint32_t* __restrict__ order_valid) {
   extern __shared__ uint64_t s_exchange[];
   if (fits_word != nullptr && *fits_word == 0u) return;  // launched ahead of the host's decision: see the scatter
-  const uint32_t t = blockIdx.x;
+  if (blockIdx.x == 0) {
+    order_tiles(gridDim.x - 1, ranges, order, order_valid, reinterpret_cast<uint32_t*>(s_exchange));
+    return;
+  }
+  const uint32_t t = blockIdx.x - 1;
   const uint32_t start = ranges[2 * t];
   const uint32_t n = ranges[2 * t + 1] - start;
   if (n == 0 || n > (uint32_t)TILE_SORT_SMALL || n > max_n) return;
@@ -910,19 +944,21 @@ int launch_bucket_scatter(int P, int W, int H, const float* means2D, const float
 // `radix_tiles` what the ranges kernel reported (number of lists for the radix sort's larger kernel << 16 | number
 // for its smaller one; a caller that does not know passes 0xFFFFFFFF): the kernels that have nothing to do are
 // not launched.  small_limit (at most TILE_SORT_SMALL) and block_limit as given to launch_bucket_count; `scratch`
-// holds 24 bytes for each of the `capacity` instances the binning arrays are laid out for.
+// holds 24 bytes for each of the `capacity` instances the binning arrays are laid out for.  tile_order (T words) and
+// the word that says it is there: see order_tiles (neither is written where there is no list at all).
 int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t small_limit, uint32_t block_limit,
                      const uint32_t* ranges, const void* table, const void* records, void* scratch, int64_t capacity,
-                     uint64_t* keys, uint32_t* emission, uint32_t* point_list, bool ahead_of_host,
-                     hipStream_t stream) {
+                     uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
+                     uint32_t* tile_order_valid, bool ahead_of_host, hipStream_t stream) {
   if (T <= 0 || longest == 0) return 0;
   const uint32_t* fits = ahead_of_host ? bucket_fits_word(table, T) : nullptr;
   if (small_limit == 0 || small_limit > (uint32_t)TILE_SORT_SMALL) small_limit = TILE_SORT_SMALL;
   const uint32_t whole = longest < small_limit ? longest : small_limit;  // the longest list sorted in registers
   uint32_t m = 256;
   while (m < whole) m <<= 1;
-  hipLaunchKernelGGL(tile_sort_registers_kernel, dim3(T), dim3(512), (size_t)m * sizeof(uint64_t), stream, ranges,
-                     (const TileRecord*)records, keys, emission, point_list, small_limit, fits);
+  hipLaunchKernelGGL(tile_sort_registers_kernel, dim3(T + 1), dim3(512), (size_t)m * sizeof(uint64_t), stream, ranges,
+                     (const TileRecord*)records, keys, emission, point_list, small_limit, fits, tile_order,
+                     tile_order_valid);
   if (longest > small_limit) {
     const uint32_t* tile_lists = (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 1) * (size_t)T;
     // scratch: `capacity` 16-byte records for the lists that are split first, then as many 8-byte words
