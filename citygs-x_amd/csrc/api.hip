@@ -961,6 +961,76 @@ int gs_adam_step(int count, float* const* params, const float* const* grads, flo
   return check_launch("adam_step", (hipStream_t)stream, false);
 }
 
+size_t gs_visible_rows_workspace_bytes(int64_t A) { return visible_rows_workspace_words(A) * sizeof(uint32_t); }
+
+int gs_visible_rows_count(int64_t A, const uint8_t* mask, void* workspace, size_t workspace_bytes,
+                          int64_t* num_visible, gs_stream_t stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  GS_REQUIRE(num_visible, "gs_visible_rows_count: null num_visible");
+  *num_visible = 0;
+  GS_REQUIRE(A >= 0 && A < 0x7FFFFFFFll, "gs_visible_rows_count: bad row count");
+  if (A == 0) return 0;
+  GS_REQUIRE(mask, "gs_visible_rows_count: null mask");
+  GS_REQUIRE(workspace && ((uintptr_t)workspace & 3) == 0 && workspace_bytes >= gs_visible_rows_workspace_bytes(A),
+             "gs_visible_rows_count: workspace missing, misaligned or too small");
+  uint32_t* total_slot = acquire_total_slot();
+  {
+    StageScope _t("visible_count", stream);
+    launch_visible_count(A, mask, (uint32_t*)workspace, total_slot, stream);
+  }
+  if (check_launch("visible_count", stream, false)) return 1;
+  uint32_t total = 0;
+  if (total_slot != nullptr) {
+    if (wait_for_total(total_slot, stream, &total)) return 1;
+  } else {
+    GS_HIP_TRY(hipMemcpyAsync(&total, visible_rows_total((const uint32_t*)workspace, A), sizeof(uint32_t),
+                              hipMemcpyDeviceToHost, stream));
+    GS_HIP_TRY(hipStreamSynchronize(stream));
+  }
+  *num_visible = (int64_t)total;
+  return 0;
+}
+
+int gs_visible_rows_gather(int64_t A, int k, int64_t N, const uint8_t* mask, const void* workspace,
+                           size_t workspace_bytes, const float* anchor, const float* feat, const float* offsets,
+                           const float* scaling, float* anchor_out, float* feat_out, float* offsets_out,
+                           float* scaling_out, uint32_t* rank, int64_t* index, gs_stream_t stream) {
+  GS_REQUIRE(A >= 0 && A < 0x7FFFFFFFll && N >= 0 && N <= A, "gs_visible_rows_gather: bad row count");
+  GS_REQUIRE(k > 0 && k <= 256, "gs_visible_rows_gather: n_offsets must be between 1 and 256");
+  if (A == 0) return 0;
+  GS_REQUIRE(mask && rank, "gs_visible_rows_gather: null mask or rank");
+  GS_REQUIRE(N == 0 || (anchor && feat && offsets && scaling && anchor_out && feat_out && offsets_out && scaling_out),
+             "gs_visible_rows_gather: null pointer");
+  GS_REQUIRE(((uintptr_t)feat & 15) == 0 && ((uintptr_t)feat_out & 15) == 0,
+             "gs_visible_rows_gather: feat and feat_out must be 16-byte aligned");
+  GS_REQUIRE(workspace && workspace_bytes >= gs_visible_rows_workspace_bytes(A),
+             "gs_visible_rows_gather: workspace missing or too small");
+  {
+    StageScope _t("visible_gather", (hipStream_t)stream);
+    launch_visible_gather(A, k, N, mask, (const uint32_t*)workspace, anchor, feat, offsets, scaling, anchor_out,
+                          feat_out, offsets_out, scaling_out, rank, index, (hipStream_t)stream);
+  }
+  return check_launch("visible_gather", (hipStream_t)stream, false);
+}
+
+int gs_visible_rows_spread(int64_t A, int k, const uint32_t* rank, const float* g_anchor, const float* g_feat,
+                           const float* g_offsets, const float* g_scaling, float* d_anchor, float* d_feat,
+                           float* d_offsets, float* d_scaling, gs_stream_t stream) {
+  GS_REQUIRE(A >= 0 && A < 0x7FFFFFFFll, "gs_visible_rows_spread: bad row count");
+  GS_REQUIRE(k > 0 && k <= 256, "gs_visible_rows_spread: n_offsets must be between 1 and 256");
+  if (A == 0) return 0;
+  GS_REQUIRE(rank, "gs_visible_rows_spread: null rank");
+  GS_REQUIRE((((uintptr_t)g_feat | (uintptr_t)d_anchor | (uintptr_t)d_feat | (uintptr_t)d_offsets |
+               (uintptr_t)d_scaling) & 15) == 0,
+             "gs_visible_rows_spread: g_feat and the outputs must be 16-byte aligned");
+  {
+    StageScope _t("visible_spread", (hipStream_t)stream);
+    launch_visible_spread(A, k, rank, g_anchor, g_feat, g_offsets, g_scaling, d_anchor, d_feat, d_offsets, d_scaling,
+                          (hipStream_t)stream);
+  }
+  return check_launch("visible_spread", (hipStream_t)stream, false);
+}
+
 int gs_neural_supported(int n_offsets) { return neural_supported(n_offsets) ? 1 : 0; }
 
 namespace {

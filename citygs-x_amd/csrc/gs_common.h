@@ -50,6 +50,38 @@ __device__ __forceinline__ int f2i_sat(float v) {
   return r;
 }
 
+// Inclusive prefix of v across the wave.
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+  const int lane = threadIdx.x & (GS_WAVE - 1);
+#pragma unroll
+  for (int d = 1; d < GS_WAVE; d <<= 1) {
+    const uint32_t o = __shfl_up(v, d, GS_WAVE);
+    if (lane >= d) v += o;
+  }
+  return v;
+}
+
+// Exclusive prefix of v across the block plus the block total.
+template <int THREADS>
+__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_wave /*THREADS/64 + 1*/,
+                                                         uint32_t& total) {
+  constexpr int NW = THREADS / GS_WAVE;
+  const int lane = threadIdx.x & (GS_WAVE - 1), wave = threadIdx.x / GS_WAVE;
+  const uint32_t inc = wave_inclusive_scan(v);
+  if (lane == GS_WAVE - 1) s_wave[wave] = inc;
+  __syncthreads();
+  uint32_t base = 0, tot = 0;
+#pragma unroll
+  for (int w = 0; w < NW; w++) {
+    const uint32_t s = s_wave[w];
+    if (w < wave) base += s;
+    tot += s;
+  }
+  __syncthreads();
+  total = tot;
+  return base + inc - v;
+}
+
 // Workgroups go to the eight XCDs in turn (workgroup b of a launch runs on XCD b % 8), and each XCD has its own L2.
 // This renumbers them so that the workgroups of one XCD hold consecutive indices (XCD 0 the first eighth, and so
 // on, each in launch order): work items that are neighbours in memory then share an L2.  A bijection on [0, n).

@@ -182,6 +182,18 @@ int launch_neural_backward(int64_t N, int k, const float* anchor, const float* f
                            const float* g_rot, float* d_anchor, float* d_feat, float* d_offsets, float* d_scaling,
                            float* const* d_params, float* slot_grads, float* partials, hipStream_t stream);
 size_t neural_slot_grad_floats(int k, int64_t N);
+// ---- rows of the anchors a view shows (workspace: visible_rows_workspace_words) ----
+size_t visible_rows_workspace_words(int64_t A);
+const uint32_t* visible_rows_total(const uint32_t* workspace, int64_t A);  // device word: number of set entries
+void launch_visible_count(int64_t A, const uint8_t* mask, uint32_t* workspace, uint32_t* total_out,
+                          hipStream_t stream);
+void launch_visible_gather(int64_t A, int k, int64_t N, const uint8_t* mask, const uint32_t* workspace,
+                           const float* anchor, const float* feat, const float* offsets, const float* scaling,
+                           float* anchor_out, float* feat_out, float* offsets_out, float* scaling_out,
+                           uint32_t* rank, int64_t* index, hipStream_t stream);
+void launch_visible_spread(int64_t A, int k, const uint32_t* rank, const float* g_anchor, const float* g_feat,
+                           const float* g_offsets, const float* g_scaling, float* d_anchor, float* d_feat,
+                           float* d_offsets, float* d_scaling, hipStream_t stream);
 int launch_all_map_fwd(int P, const float* means, const float* scales, const float* rots, const float* V,
                        const float* campos, float* out, hipStream_t stream);
 int launch_all_map_bwd(int P, const float* means, const float* scales, const float* rots, const float* V,

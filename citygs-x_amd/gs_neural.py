@@ -133,6 +133,74 @@ def neural_gaussians(anchor, feat, offsets, scaling, camera_center, mlp_opacity,
                                   *mlp_opacity, *mlp_color, *mlp_cov)
 
 
+class _VisibleRows(torch.autograd.Function):
+    """The rows of anchor, feat, offsets and scaling that a bool mask selects (gaussian_renderer/__init__.py:794-798)
+    and their numbers: what nonzero() and four index_select()s give."""
+
+    @staticmethod
+    def forward(ctx, mask, anchor, feat, offsets, scaling, want_index):
+        A, k = offsets.shape[:2]
+        dev = anchor.device
+        stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        nb = _n.lib.gs_visible_rows_workspace_bytes(A)
+        ws = torch.empty(nb // 4, dtype=torch.int32, device=dev)
+        N = C.c_int64(0)
+        _n.check(_n.lib.gs_visible_rows_count(A, _p(mask), _p(ws), nb, C.byref(N), stream), "visible rows")
+        N = N.value
+        out = [torch.empty(N, *t.shape[1:], device=dev) for t in (anchor, feat, offsets, scaling)]
+        rank = torch.empty(A, dtype=torch.int32, device=dev)
+        index = torch.empty(N, dtype=torch.int64, device=dev) if want_index else None
+        _n.check(_n.lib.gs_visible_rows_gather(A, k, N, _p(mask), _p(ws), nb, _p(anchor), _p(feat), _p(offsets),
+                                               _p(scaling), *[_p(t) for t in out], _p(rank), _p(index), stream),
+                 "visible rows")
+        ctx.save_for_backward(rank)
+        ctx.k = k
+        ctx.set_materialize_grads(False)
+        # rows of an array without a gradient carry none either
+        ctx.mark_non_differentiable(*[t for t, need in zip(out, ctx.needs_input_grad[1:5]) if not need],
+                                    *([index] if want_index else []))
+        return (*out, index)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        rank, = ctx.saved_tensors
+        A, k, dev = rank.shape[0], ctx.k, rank.device
+        grads = [g if need else None for g, need in zip(grads[:4], ctx.needs_input_grad[1:5])]
+        shapes = ((A, 3), (A, 32), (A, k, 3), (A, 6))
+        if torch.is_grad_enabled():  # a graph of the backward pass is asked for
+            idx = (rank >= 0).nonzero(as_tuple=True)[0]
+            return (None, *[None if g is None else torch.zeros(s, device=dev).index_add(0, idx, g)
+                            for g, s in zip(grads, shapes)], None)
+        grads = [None if g is None else g.contiguous() for g in grads]
+        if grads[1] is not None and grads[1].data_ptr() % 16:
+            grads[1] = grads[1].clone()
+        d = [None if g is None else torch.empty(s, device=dev) for g, s in zip(grads, shapes)]
+        stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        _n.check(_n.lib.gs_visible_rows_spread(A, k, _p(rank), *[_p(t) for t in grads], *[_p(t) for t in d], stream),
+                 "visible rows backward")
+        return (None, *d, None)
+
+
+def _visible_rows(mask, anchor, feat, offsets, scaling, want_index):
+    """anchor[mask], feat[mask], offsets[mask], scaling[mask] and, if wanted, mask.nonzero(): one pass over the arrays
+    where they are the dense float32 arrays of a model on the current device with 16-byte rows of features, torch's
+    gathers for everything else (other types, strides, devices and mask shapes, n_offsets without a kernel, a stream
+    under capture, functorch transforms)."""
+    t4 = (anchor, feat, offsets, scaling)
+    if (mask.dtype is torch.bool and mask.is_cuda and mask.dim() == 1 and mask.is_contiguous()
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is torch.float32
+                    and t.device == mask.device and t.is_contiguous() and t.shape[0] == mask.shape[0] for t in t4)
+            and anchor.shape[1:] == (3,) and feat.shape[1:] == (32,) and scaling.shape[1:] == (6,)
+            and offsets.dim() == 3 and offsets.shape[2] == 3 and _n.lib.gs_neural_supported(offsets.shape[1])
+            and feat.data_ptr() % 16 == 0 and mask.shape[0] > 0
+            and mask.device.index == torch.cuda.current_device()
+            and not torch.cuda.is_current_stream_capturing()):
+        return _VisibleRows.apply(mask, anchor, feat, offsets, scaling, want_index)
+    # one nonzero() (one host synchronisation) serves the four gathers; x[visible_mask] would run it four times
+    idx = mask.nonzero(as_tuple=True)[0]
+    return (*[t.index_select(0, idx) for t in t4], idx)
+
+
 def _linear_pair(seq):
     """(W1, b1, W2, b2) of a Sequential(Linear, ReLU, Linear[, activation]) (scene/gaussian_model.py:131-149)."""
     return seq[0].weight, seq[0].bias, seq[2].weight, seq[2].bias
@@ -159,10 +227,8 @@ def generate_neural_gaussians(viewpoint_camera, pc, visible_mask=None, is_traini
             opacity_scale = torch.where(pc.transition_mask, pc._prog_ratio.reshape(-1),
                                         torch.ones_like(pc._prog_ratio.reshape(-1)))
     else:
-        # one nonzero() (one host synchronisation) serves the four gathers; x[visible_mask] would run it four times
-        idx = visible_mask.nonzero(as_tuple=True)[0]
-        anchor, feat = pc.get_anchor.index_select(0, idx), pc.get_anchor_feat.index_select(0, idx)
-        offsets, scaling = pc._offset.index_select(0, idx), pc.get_scaling.index_select(0, idx)
+        anchor, feat, offsets, scaling, idx = _visible_rows(
+            visible_mask, pc.get_anchor, pc.get_anchor_feat, pc._offset, pc.get_scaling, pc.add_level or progressive)
         if pc.add_level:
             level = pc.get_level.reshape(-1).index_select(0, idx).float()
         if progressive:

@@ -47,6 +47,10 @@ _SIGNATURES = {
     "gs_training_stats": (_i, [_i64, _i, _i64, _i64, _vp, _vp, _vp, _vp, _i] + [_vp] * 6 + [_sz, _vp]),
     "gs_max_radii_update": (_i, [_i64, _vp, _vp, _vp, _vp]),
     "gs_adam_step": (_i, [_i] + [_vp] * 7 + [C.c_double, C.c_double, C.c_double, _f, _vp]),
+    "gs_visible_rows_workspace_bytes": (_sz, [_i64]),
+    "gs_visible_rows_count": (_i, [_i64, _vp, _vp, _sz, _vp, _vp]),
+    "gs_visible_rows_gather": (_i, [_i64, _i, _i64, _vp, _vp, _sz] + [_vp] * 11),
+    "gs_visible_rows_spread": (_i, [_i64, _i] + [_vp] * 10),
     "gs_neural_supported": (_i, [_i]),
     "gs_neural_workspace_bytes": (_sz, [_i64, _i]),
     "gs_neural_opacity_forward": (_i, [_i64, _i] + [_vp] * 6 + [_i] + [_vp] * 5 + [_sz, _vp, _vp]),

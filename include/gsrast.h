@@ -275,6 +275,25 @@ int gs_all_map_backward(int P, const float* means3D, const float* scales, const 
                         const float* viewmatrix, const float* campos, const float* dL_dall_map,
                         float* dL_dmeans3D, float* dL_drotations, gs_stream_t stream);
 
+/* The rows of the four anchor arrays that visible_mask selects (gaussian_renderer/__init__.py:794-798): anchor (A,3),
+ * feat (A,32), offsets (A,n_offsets,3), scaling (A,6), mask (A bytes, non-zero = selected), 1 <= n_offsets <= 256.
+ * gs_visible_rows_count waits for the number of selected rows N; gs_visible_rows_gather, with the same workspace
+ * (gs_visible_rows_workspace_bytes(A)), writes them in order into the *_out arrays (N rows), rank (u32, A: the row's
+ * place among them, 0xFFFFFFFF if it is not selected) and, unless NULL, index (int64, N: the selected rows' numbers).
+ * gs_visible_rows_spread is the gather's gradient: row i of every d_* array (A rows, each may be NULL) becomes row
+ * rank[i] of its g_* array (N rows), or zeros; every element is written. */
+size_t gs_visible_rows_workspace_bytes(int64_t num_anchors);
+int gs_visible_rows_count(int64_t num_anchors, const uint8_t* mask, void* workspace, size_t workspace_bytes,
+                          int64_t* num_visible, gs_stream_t stream);
+int gs_visible_rows_gather(int64_t num_anchors, int n_offsets, int64_t num_visible, const uint8_t* mask,
+                           const void* workspace, size_t workspace_bytes, const float* anchor, const float* feat,
+                           const float* offsets, const float* scaling, float* anchor_out, float* feat_out,
+                           float* offsets_out, float* scaling_out, uint32_t* rank, int64_t* index,
+                           gs_stream_t stream);
+int gs_visible_rows_spread(int64_t num_anchors, int n_offsets, const uint32_t* rank, const float* g_anchor,
+                           const float* g_feat, const float* g_offsets, const float* g_scaling, float* d_anchor,
+                           float* d_feat, float* d_offsets, float* d_scaling, gs_stream_t stream);
+
 /* Replaces the body of generate_neural_gaussians (gaussian_renderer/__init__.py:789-899) in the reference's
  * default configuration (arguments/__init__.py:94-124: feat_dim 32, no feature bank, no appearance embedding, no
  * distance or level inputs, dist2level 'round'; the options further down add to it), on the anchors already
