@@ -4,9 +4,9 @@
 //
 // Bound by memory.  As nonzero() and four index_select()s the forward part was nine launches and 97 us at 500 k
 // anchors of 10 offsets (35 % visible), and the backward part (a fill and an index_add per array, whose atomic adds
-// fetch every line they touch) eight launches and 117 us; here 4 + 3 + 27 and 41 us (142 MB written).  A workgroup owns 256 consecutive rows, so that both
-// sides of the forward copy run through memory in order, and the backward kernel writes every element of the full
-// arrays once, the gradient's row or zero.
+// fetch every line they touch) eight launches and 117 us; here 4 + 3 + 27 and 41 us (142 MB written).  A workgroup
+// owns 256 consecutive rows, so that both sides of the forward copy run through memory in order, and the backward
+// kernel writes every element of the full arrays once, the gradient's row or zero.
 #include "gs_common.h"
 #include "gs_kernels.h"
 

@@ -1,7 +1,8 @@
 """Drop-in for the reference's compiled extension module
 (submodule_cityx/diff-gaussian-rasterization/ext.cpp:16-35): same function
-names, argument order and return tuples, implemented on libgsrast.so through
-ctypes.  torch is used for device memory and the current stream only.
+names, argument order and return tuples, implemented on libgsrast.so, through
+csrc/torch_ops.cpp where a training view passes on every iteration and ctypes
+elsewhere.  torch is used for device memory and the current stream only.
 """
 import ctypes as C
 import os
@@ -101,33 +102,15 @@ def preprocess_gaussians_ex(means3D, scales, rotations, sh, opacity, scale_modif
         raise RuntimeError("means3D must have dimensions (num_points, 3)")
     means3D = _f32c(means3D, "means3D")
     dev = means3D.device
-    P = means3D.shape[0]
-    f32 = dict(dtype=torch.float32, device=dev)
-    if P == 0:
+    if means3D.shape[0] == 0:
+        f32 = dict(dtype=torch.float32, device=dev)
         return ((0, torch.zeros(0, 2, **f32), torch.zeros(0, **f32), torch.zeros(0, dtype=torch.int32, device=dev),
                  torch.zeros(0, 6, **f32), torch.zeros(0, 4, **f32), torch.zeros(0, 3, **f32),
                  torch.zeros(0, 3, dtype=torch.bool, device=dev)), None)
-    means2D = torch.empty(P, 2, **f32)
-    depths = torch.empty(P, **f32)
-    radii = torch.empty(P, dtype=torch.int32, device=dev)
-    cov3D = torch.empty(P, 6, **f32) if want_cov3D else None
-    conic_opacity = torch.empty(P, 4, **f32)
-    rgb = torch.empty(P, 3, **f32)
-    clamped = torch.empty(P, 3, dtype=torch.bool, device=dev)
-    scales, rotations, opacity = _f32c(scales, "scales"), _f32c(rotations, "rotations"), _f32c(opacity, "opacity")
-    vm, pm, cp = _f32c(viewmatrix, "viewmatrix"), _f32c(projmatrix, "projmatrix"), _f32c(campos, "campos")
-    sh_mode = sh is not None and sh.dim() == 3 and sh.shape[0] == P
-    M = sh.shape[1] if sh_mode else 0
-    shc = _f32c(sh, "sh") if sh_mode else None
-    ddir = torch.empty(P, 3, 3, **f32) if (sh_mode and want_direction_derivative) else None
-    with torch.cuda.device(dev):
-        _n.check(_lib.gs_preprocess_channels_forward(
-            _ptr(means2D), _ptr(depths), _ptr(radii), _ptr(cov3D), _ptr(conic_opacity), _ptr(rgb), _ptr(clamped), None,
-            P, int(degree), M, int(image_width), int(image_height), _ptr(means3D), _ptr(scales), _ptr(rotations),
-            _ptr(shc), _ptr(opacity), float(scale_modifier), _ptr(vm), _ptr(pm), _ptr(cp), float(tan_fovx),
-            float(tan_fovy), int(bool(prefiltered)), int(bool(debug)), _ptr(ddir), _ptr(blend_records),
-            _ptr(all_map), _stream(dev)),
-            "preprocess_gaussians")
+    means2D, depths, radii, cov3D, conic_opacity, rgb, clamped, ddir = _n.ops.preprocess_forward(
+        means3D, scales, rotations, sh, opacity, float(scale_modifier), viewmatrix, projmatrix, campos, float(tan_fovx),
+        float(tan_fovy), int(image_height), int(image_width), int(degree), bool(prefiltered), bool(debug),
+        want_direction_derivative, want_cov3D, blend_records, all_map, _n.stream_handle(dev))
     return (0, means2D, depths, radii, cov3D, conic_opacity, rgb, clamped), ddir
 
 
@@ -140,58 +123,16 @@ def preprocess_gaussians_backward(radii, cov3D, clamped, means3D, scales, rotati
     channels that call wrote; build_all_map_backward's results are then part of the gradients returned."""
     means3D = _f32c(means3D, "means3D")
     dev = means3D.device
-    P = means3D.shape[0]
-    f32 = dict(dtype=torch.float32, device=dev)
-    sh_mode = sh is not None and sh.dim() == 3 and sh.shape[0] == P
-    M = sh.shape[1] if sh_mode else 0
-    dL_dsh = torch.empty(P, M, 3, **f32) if sh_mode else torch.zeros(P, 3, **f32)
-    if P == 0:
+    if means3D.shape[0] == 0:
+        f32 = dict(dtype=torch.float32, device=dev)
+        sh_mode = sh is not None and sh.dim() == 3 and sh.shape[0] == 0
+        dL_dsh = torch.empty(0, sh.shape[1], 3, **f32) if sh_mode else torch.zeros(0, 3, **f32)
         return (torch.zeros(0, 3, **f32), torch.zeros(0, 3, **f32), torch.zeros(0, 4, **f32), dL_dsh,
                 torch.zeros(0, 1, **f32))
-    dL_dmeans3D = torch.empty(P, 3, **f32)
-    dL_dscales = torch.empty(P, 3, **f32)
-    dL_drotations = torch.empty(P, 4, **f32)
-    dL_dopacity = torch.empty(P, 1, **f32)
-    g2 = _f32c(dL_dmeans2D, "dL_dmeans2D")
-    gco = _f32c(dL_dconic_opacity, "dL_dconic_opacity")
-    gcol = _f32c(dL_dcolors, "dL_dcolors") if (sh_mode and dL_dcolors is not None) else None
-    if sh_mode and gcol is None:
-        gcol = torch.zeros(P, 3, **f32)
-    scales, rotations = _f32c(scales, "scales"), _f32c(rotations, "rotations")
-    vm, pm, cp = _f32c(viewmatrix, "viewmatrix"), _f32c(projmatrix, "projmatrix"), _f32c(campos, "campos")
-    shc = _f32c(sh, "sh") if sh_mode else None
-    with torch.cuda.device(dev):
-        _n.check(_lib.gs_preprocess_channels_backward(
-            _ptr(radii.contiguous()), _ptr(cov3D.contiguous() if cov3D is not None else None),
-            _ptr(clamped.contiguous()), P, int(degree), M,
-            int(image_width), int(image_height), _ptr(means3D), _ptr(scales), _ptr(rotations), _ptr(shc),
-            float(scale_modifier), _ptr(vm), _ptr(pm), _ptr(cp), float(tan_fovx), float(tan_fovy), _ptr(g2),
-            int(g2.shape[1]), _ptr(gco), _ptr(gcol), _ptr(dL_dmeans3D), None, _ptr(dL_dscales), _ptr(dL_drotations),
-            _ptr(dL_dsh) if sh_mode else None, _ptr(dL_dopacity), int(bool(debug)),
-            _ptr(dcolor_ddir) if (sh_mode and dcolor_ddir is not None) else None,
-            _ptr(_f32c(dL_dall_map, "dL_dall_map") if dL_dall_map is not None else None), _stream(dev)),
-            "preprocess_gaussians_backward")
-    return dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity
-
-
-class _GrowBuffer:
-    """Byte tensor grown on demand by the native side (resizeFunctional,
-    rasterize_points.cu:31-37)."""
-
-    def __init__(self, device):
-        self.device = device
-        self.tensor = torch.empty(0, dtype=torch.uint8, device=device)
-        self.callback = _n.RESIZE_FN(self._resize)
-
-    def _resize(self, nbytes, _user):
-        if self.tensor.numel() < nbytes:
-            self.tensor = torch.empty(int(nbytes), dtype=torch.uint8, device=self.device)
-        return self.tensor.data_ptr()
-
-    def release(self):
-        # drop the callback so this object does not keep the tensor alive through a reference cycle
-        self.callback = None
-        return self.tensor
+    return _n.ops.preprocess_backward(
+        radii, cov3D, clamped, means3D, scales, rotations, sh, float(scale_modifier), viewmatrix, projmatrix,
+        float(tan_fovx), float(tan_fovy), int(image_height), int(image_width), int(degree), campos, dL_dmeans2D,
+        dL_dconic_opacity, dL_dcolors, bool(debug), dcolor_ddir, dL_dall_map, _n.stream_handle(dev))
 
 
 def render_gaussians(background, image_height, image_width, means2D, depths, radii, conic_opacity, rgb,
@@ -269,74 +210,36 @@ def render_gaussians_ex(background, image_height, image_width, means2D, depths, 
     packed); the same tensor goes to render_gaussians_backward."""
     means2D = _f32c(means2D, "means2D")
     dev = means2D.device
-    P = means2D.shape[0]
     H, W = int(image_height), int(image_width)
-    f32 = dict(dtype=torch.float32, device=dev)
-    i32 = dict(dtype=torch.int32, device=dev)
-    tiles = ((H + BLOCK_Y - 1) // BLOCK_Y) * ((W + BLOCK_X - 1) // BLOCK_X)
-    geo = bool(render_geo)
-    if P == 0:
+    if means2D.shape[0] == 0:
+        f32 = dict(dtype=torch.float32, device=dev)
+        i32 = dict(dtype=torch.int32, device=dev)
+        tiles = ((H + BLOCK_Y - 1) // BLOCK_Y) * ((W + BLOCK_X - 1) // BLOCK_X)
         empty = torch.empty(0, dtype=torch.uint8, device=dev)
         return ((0, torch.zeros(NUM_CHANNELS, H, W, **f32), torch.zeros(tiles, **i32), torch.zeros(tiles, **i32),
                  torch.zeros(tiles, **i32), torch.zeros(0, **i32), torch.zeros(NUM_ALL_MAP, H, W, **f32),
                  torch.zeros(1, H, W, **f32), empty, empty.clone(), empty.clone()),
                 {"longest_list": 0, "binning_capacity": 0, "launched_ahead": False})
-    out_color = torch.empty(NUM_CHANNELS, H, W, **f32)
-    out_observe = torch.empty(P, **i32)  # cleared by the call itself
-    out_all_map = torch.empty(NUM_ALL_MAP, H, W, **f32) if geo else torch.zeros(NUM_ALL_MAP, H, W, **f32)
-    out_plane_depth = torch.empty(1, H, W, **f32) if geo else torch.zeros(1, H, W, **f32)
-    n_render = torch.empty(tiles, **i32)
-    n_consider = torch.empty(tiles, **i32)
-    n_contrib = torch.empty(tiles, **i32)
-    geom, binning, img = _GrowBuffer(dev), _GrowBuffer(dev), _GrowBuffer(dev)
-    bg = _f32c(background, "background")
-    depths, conic_opacity, rgb = _f32c(depths, "depths"), _f32c(conic_opacity, "conic_opacity"), _f32c(rgb, "rgb")
-    radii = radii.contiguous()
-    if radii.dtype != torch.int32:
-        raise TypeError("radii must be int32")
-    cl = compute_locally.contiguous()
-    if cl.dtype != torch.bool or cl.numel() != tiles:
-        raise RuntimeError(f"compute_locally must be a bool tensor with {tiles} elements")
-    am = _f32c(all_map, "all_map") if geo else None
     want_mwd = isinstance(args, dict) and bool(args.get("max_weight_depth"))
     # (small_limit, block_records) for this call only: how the per-tile lists are built (a test hook)
     limits = args.get("tile_sort_limits") if isinstance(args, dict) else None
-    options = None
-    if blend_records is not None and (blend_records.shape != (P, 16) or blend_records.dtype != torch.float32
-                                      or not blend_records.is_contiguous() or blend_records.device != dev):
-        raise RuntimeError("blend_records must be a contiguous (P, 16) float32 tensor on the same device")
-    if limits is not None or expected_instances > 0 or blend_records is not None:
-        options = _n.RenderOptions(*(limits if limits is not None else (-1, -1)),
-                                   expected_instances=expected_instances,
-                                   expected_longest_list=expected_longest_list,
-                                   blend_records=blend_records.data_ptr() if blend_records is not None else None)
-    result = _n.RenderResult()
-    mwd = torch.empty(1, H, W, **f32) if want_mwd else None
+    small_limit, block_records = limits if limits is not None else (-1, -1)
     # fp32 arithmetic, as `H / (2.0f * tan_fovy)` at rasterize_points.cu:328-329
     focal_y = np.float32(H) / (np.float32(2.0) * np.float32(tan_fovy))
     focal_x = np.float32(W) / (np.float32(2.0) * np.float32(tan_fovx))
-    num_rendered = C.c_int(0)
-    elapsed = C.c_float(0.0)
-    timing = _want_timing(args)
-    with torch.cuda.device(dev):
-        _n.check(_lib.gs_render_forward(
-            geom.callback, None, binning.callback, None, img.callback, None, P, _ptr(bg), W, H, float(focal_x),
-            float(focal_y), float(W * 0.5), float(H * 0.5), _ptr(viewmatrix), _ptr(campos), _ptr(am), _ptr(means2D),
-            _ptr(depths), _ptr(radii), _ptr(conic_opacity), _ptr(rgb), _ptr(cl), _ptr(out_color), _ptr(n_render),
-            _ptr(n_consider), _ptr(n_contrib), _ptr(out_observe), _ptr(out_all_map), _ptr(out_plane_depth), _ptr(mwd),
-            int(geo),
-            int(bool(debug)), C.byref(num_rendered), C.byref(elapsed) if timing else None,
-            C.byref(options) if options is not None else None, C.byref(result), _stream(dev)),
-            "render_gaussians")
-    _record_time(args, "forward_render_time", elapsed.value)
+    (num_rendered, out_color, n_render, n_consider, n_contrib, out_observe, out_all_map, out_plane_depth, geom, binning,
+     img, longest_list, binning_capacity, launched_ahead, elapsed, mwd) = _n.ops.render_forward(
+        background, H, W, means2D, depths, radii, conic_opacity, rgb, compute_locally, float(focal_x), float(focal_y),
+        all_map if render_geo else None, bool(render_geo), bool(debug), want_mwd, _want_timing(args), int(small_limit),
+        int(block_records), int(expected_instances), int(expected_longest_list), blend_records, _n.stream_handle(dev))
+    _record_time(args, "forward_render_time", elapsed)
     if want_mwd:
         args.setdefault("stats_collector", {})["max_weight_depth"] = mwd
     if _want_tile_log(args):
         _write_tile_log(args, H, W, n_render, n_consider, n_contrib)
-    info = {"longest_list": int(result.longest_list), "binning_capacity": int(result.binning_capacity),
-            "launched_ahead": bool(result.launched_ahead)}
-    return ((num_rendered.value, out_color, n_render, n_consider, n_contrib, out_observe, out_all_map,
-             out_plane_depth, geom.release(), binning.release(), img.release()), info)
+    info = {"longest_list": longest_list, "binning_capacity": binning_capacity, "launched_ahead": launched_ahead}
+    return ((num_rendered, out_color, n_render, n_consider, n_contrib, out_observe, out_all_map, out_plane_depth, geom,
+             binning, img), info)
 
 
 def render_gaussians_backward(background, tan_fovx, tan_fovy, all_map_pixels, all_maps, R, geomBuffer, binningBuffer,
@@ -349,41 +252,17 @@ def render_gaussians_backward(background, tan_fovx, tan_fovy, all_map_pixels, al
     was given, if any."""
     means2D = _f32c(means2D, "means2D")
     dev = means2D.device
-    P = means2D.shape[0]
-    H, W = dL_dout_color.shape[1], dL_dout_color.shape[2]
-    f32 = dict(dtype=torch.float32, device=dev)
-    geo = bool(render_geo)
-    # every element is written by the native reduction, so no zero fill is needed
-    dL_dmeans2D = torch.empty(P, 2, **f32)
-    dL_dmeans2D_abs = torch.empty(P, 3, **f32)
-    dL_dconic_opacity = torch.empty(P, 4, **f32)
-    dL_dcolors = torch.empty(P, NUM_CHANNELS, **f32)
-    dL_dall_map = torch.empty(P, NUM_ALL_MAP, **f32)
-    if P != 0:
-        ws_bytes = _lib.gs_render_backward_workspace_bytes(int(R))
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        bg = _f32c(background, "background")
-        gpix = _f32c(dL_dout_color, "dL_dout_color")
-        gmap = _f32c(dL_dout_all_map, "dL_dout_all_map") if geo else None
-        gdep = _f32c(dL_dout_plane_depth, "dL_dout_plane_depth") if geo else None
-        amp = _f32c(all_map_pixels, "all_map_pixels") if geo else None
-        am = _f32c(all_maps, "all_maps") if geo else None
-        co, col = _f32c(conic_opacity, "conic_opacity"), _f32c(rgb, "rgb")
-        elapsed = C.c_float(0.0)
-        timing = _want_timing(args)
-        with torch.cuda.device(dev):
-            _n.check(_lib.gs_render_backward(
-                P, int(R), _ptr(bg), W, H, float(tan_fovx), float(tan_fovy), _ptr(geomBuffer), _ptr(binningBuffer),
-                _ptr(imageBuffer), _ptr(compute_locally.contiguous()), _ptr(gpix), _ptr(gmap), _ptr(gdep),
-                _ptr(dL_dmeans2D), _ptr(dL_dmeans2D_abs), _ptr(dL_dconic_opacity), _ptr(dL_dcolors), _ptr(dL_dall_map),
-                _ptr(means2D), _ptr(co), _ptr(col), _ptr(am), _ptr(amp), int(geo), int(bool(debug)), _ptr(workspace),
-                ws_bytes, C.byref(elapsed) if timing else None, int(binning_capacity), _ptr(blend_records),
-                _stream(dev)),
-                "render_gaussians_backward")
-        _record_time(args, "backward_render_time", elapsed.value)
-    else:
+    if means2D.shape[0] == 0:
         _record_time(args, "backward_render_time", 0.0)
-    return dL_dmeans2D, dL_dmeans2D_abs, dL_dconic_opacity, dL_dcolors, dL_dall_map
+        return tuple(torch.empty(0, n, dtype=torch.float32, device=dev) for n in (2, 3, 4, NUM_CHANNELS, NUM_ALL_MAP))
+    geo = bool(render_geo)
+    *grads, elapsed = _n.ops.render_backward(
+        background, float(tan_fovx), float(tan_fovy), all_map_pixels if geo else None, all_maps if geo else None, int(R),
+        geomBuffer, binningBuffer, imageBuffer, compute_locally, dL_dout_color, dL_dout_all_map if geo else None,
+        dL_dout_plane_depth if geo else None, means2D, conic_opacity, rgb, geo, bool(debug), _want_timing(args),
+        int(binning_capacity), blend_records, _n.stream_handle(dev))
+    _record_time(args, "backward_render_time", elapsed)
+    return tuple(grads)
 
 
 def rasterize_aussians_filter(means3D, scales, rotations, scale_modifier, cov3D_precomp, viewmatrix, projmatrix,

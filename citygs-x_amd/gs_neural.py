@@ -4,37 +4,9 @@ in libgsrast.so.  The fused operator is the reference's default model configurat
 feat_dim 32, inputs [feature, view direction]; the operator also takes the optional distance and level inputs of the
 three MLPs (add_opacity_dist, add_color_dist, add_cov_dist, add_level) and the per-anchor opacity factor of dist2level
 'progressive'; the drop-in function also serves the appearance embedding and the feature bank, which reduce to it."""
-import ctypes as C
-
 import torch
 
 import gsrast_native as _n
-
-
-def _p(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
-
-
-def _f32(t, name, shape):
-    if t.dtype != torch.float32:
-        raise TypeError(f"{name} must be float32, got {t.dtype}")
-    if not t.is_cuda:
-        raise RuntimeError(f"{name} must be a GPU tensor: there is no CPU path")
-    if tuple(t.shape) != tuple(shape):
-        raise RuntimeError(f"{name} must have shape {tuple(shape)}, got {tuple(t.shape)}")
-    return t.contiguous()
-
-
-def _table(tensors):
-    arr = (C.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
-    return arr
-
-
-def _param_shapes(k, input_flags=0):
-    shapes = []
-    for m, out in enumerate((k, 3 * k, 7 * k)):
-        shapes += [(32, 35 + ((input_flags >> m) & 1) + ((input_flags >> 3) & 1)), (32,), (out, 32), (out,)]
-    return shapes
 
 
 class _NeuralGaussians(torch.autograd.Function):
@@ -42,81 +14,29 @@ class _NeuralGaussians(torch.autograd.Function):
     def forward(ctx, anchor, feat, offsets, scaling, campos, opacity_scale, level, input_flags, *params):
         if len(params) != 12:
             raise RuntimeError("expected W1, b1, W2, b2 of the opacity, color and cov MLPs (12 tensors)")
-        N = anchor.shape[0]
         if offsets.dim() != 3:
             raise RuntimeError("offsets must be (anchors, n_offsets, 3)")
         k = offsets.shape[1]
         if not _n.lib.gs_neural_supported(k):
             raise NotImplementedError(f"n_offsets = {k} is not among the values the kernels are built for")
-        anchor, feat = _f32(anchor, "anchor", (N, 3)), _f32(feat, "feat", (N, 32))
-        offsets, scaling = _f32(offsets, "offsets", (N, k, 3)), _f32(scaling, "scaling", (N, 6))
-        campos = _f32(campos, "camera_center", (3,))
-        if opacity_scale is not None:
-            opacity_scale = _f32(opacity_scale.detach(), "opacity_scale", (N,))
-        if input_flags & 8:
-            if level is None:
-                raise RuntimeError("input_flags asks for the level input")
-            level = _f32(level.detach().reshape(-1), "level", (N,))
-        else:
-            level = None
-        params = [_f32(p, f"MLP parameter {i}", s)
-                  for i, (p, s) in enumerate(zip(params, _param_shapes(k, input_flags)))]
-        dev = anchor.device
-        stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        neural_opacity = torch.empty(N * k, 1, dtype=torch.float32, device=dev)
-        # with a factor on the opacity the backward pass needs the MLP's own output as well
-        opacity_tanh = torch.empty(N * k, dtype=torch.float32, device=dev) if opacity_scale is not None else None
-        mask = torch.empty(N * k, dtype=torch.bool, device=dev)
-        first = torch.empty(max(N, 1), dtype=torch.int32, device=dev)
-        ws_bytes = _n.lib.gs_neural_workspace_bytes(N, k)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        table = _table(params)
-        S = C.c_int64(0)
-        _n.check(_n.lib.gs_neural_opacity_forward(N, k, _p(anchor), _p(feat), _p(campos), table,
-                                                  _p(opacity_scale), _p(level), input_flags,
-                                                  _p(neural_opacity), _p(opacity_tanh), _p(mask), _p(first), _p(ws), ws_bytes,
-                                                  C.byref(S), stream),
-                 "generate_neural_gaussians")
-        S = S.value
-        xyz, color = torch.empty(S, 3, device=dev), torch.empty(S, 3, device=dev)
-        opacity, scal = torch.empty(S, 1, device=dev), torch.empty(S, 3, device=dev)
-        rot, aux = torch.empty(S, 4, device=dev), torch.empty(S, 4, device=dev)
-        _n.check(_n.lib.gs_neural_gaussians_forward(N, k, S, _p(anchor), _p(feat), _p(offsets), _p(scaling),
-                                                    _p(campos), _p(level), _p(neural_opacity), _p(first), _p(ws),
-                                                    ws_bytes,
-                                                    _p(xyz), _p(color), _p(opacity), _p(scal), _p(rot), _p(aux),
-                                                    stream), "generate_neural_gaussians")
-        ctx.save_for_backward(anchor, feat, offsets, scaling, campos, neural_opacity, first, color, rot, aux, *params)
-        ctx.sizes = (N, k, S)
-        ctx.opacity_scale = opacity_scale  # carries no gradient (a buffer of the model)
-        ctx.level, ctx.input_flags, ctx.opacity_tanh = level, input_flags, opacity_tanh
+        out, saved, params, ctx.opacity_scale, ctx.level, ctx.opacity_tanh = _n.ops.neural_forward(
+            anchor, feat, offsets, scaling, campos, opacity_scale, level, input_flags, params,
+            _n.stream_handle(anchor.device))
+        # (opacity_scale carries no gradient: a buffer of the model)
+        ctx.save_for_backward(*saved, *params)
+        ctx.input_flags = input_flags
+        neural_opacity, mask = out[5:]
         ctx.mark_non_differentiable(neural_opacity, mask)
         ctx.set_materialize_grads(False)
-        return xyz, color, opacity, scal, rot, neural_opacity, mask
+        return out
 
     @staticmethod
     def backward(ctx, g_xyz, g_color, g_opacity, g_scal, g_rot, _g_nop, _g_mask):
-        anchor, feat, offsets, scaling, campos, neural_opacity, first, color, rot, aux, *params = ctx.saved_tensors
-        N, k, S = ctx.sizes
-        dev = anchor.device
-        ups = []
-        for g, c in ((g_xyz, 3), (g_color, 3), (g_opacity, 1), (g_scal, 3), (g_rot, 4)):
-            ups.append(torch.zeros(S, c, device=dev) if g is None else _f32(g, "upstream gradient", (S, c)))
-        d_anchor, d_feat = torch.empty_like(anchor), torch.empty_like(feat)
-        d_offsets, d_scaling = torch.empty_like(offsets), torch.empty_like(scaling)
-        d_params = [torch.empty_like(p) for p in params]
-        ws_bytes = _n.lib.gs_neural_backward_workspace_bytes(N, k)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        _n.check(_n.lib.gs_neural_backward(N, k, S, _p(anchor), _p(feat), _p(offsets), _p(scaling), _p(campos),
-                                           _table(params),
-                                           _p(ctx.opacity_scale), _p(ctx.level), ctx.input_flags,
-                                           _p(neural_opacity), _p(ctx.opacity_tanh), _p(first), _p(color), _p(rot),
-                                           _p(aux),
-                                           *[_p(u) for u in ups], _p(d_anchor), _p(d_feat), _p(d_offsets),
-                                           _p(d_scaling), _table(d_params), _p(ws), ws_bytes, stream),
-                 "generate_neural_gaussians backward")
-        return (d_anchor, d_feat, d_offsets, d_scaling, None, None, None, None, *d_params)
+        saved = ctx.saved_tensors
+        d_inputs = _n.ops.neural_backward(*saved[:10], saved[10:], ctx.opacity_scale, ctx.level, ctx.input_flags,
+                                          ctx.opacity_tanh, (g_xyz, g_color, g_opacity, g_scal, g_rot),
+                                          _n.stream_handle(saved[0].device))
+        return (*d_inputs[:4], None, None, None, None, *d_inputs[4:])
 
 
 def neural_gaussians(anchor, feat, offsets, scaling, camera_center, mlp_opacity, mlp_color, mlp_cov,
@@ -139,22 +59,10 @@ class _VisibleRows(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, mask, anchor, feat, offsets, scaling, want_index):
-        A, k = offsets.shape[:2]
-        dev = anchor.device
-        stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        nb = _n.lib.gs_visible_rows_workspace_bytes(A)
-        ws = torch.empty(nb // 4, dtype=torch.int32, device=dev)
-        N = C.c_int64(0)
-        _n.check(_n.lib.gs_visible_rows_count(A, _p(mask), _p(ws), nb, C.byref(N), stream), "visible rows")
-        N = N.value
-        out = [torch.empty(N, *t.shape[1:], device=dev) for t in (anchor, feat, offsets, scaling)]
-        rank = torch.empty(A, dtype=torch.int32, device=dev)
-        index = torch.empty(N, dtype=torch.int64, device=dev) if want_index else None
-        _n.check(_n.lib.gs_visible_rows_gather(A, k, N, _p(mask), _p(ws), nb, _p(anchor), _p(feat), _p(offsets),
-                                               _p(scaling), *[_p(t) for t in out], _p(rank), _p(index), stream),
-                 "visible rows")
+        *out, index, rank = _n.ops.visible_rows(mask, anchor, feat, offsets, scaling, want_index,
+                                                _n.stream_handle(anchor.device))
         ctx.save_for_backward(rank)
-        ctx.k = k
+        ctx.k = offsets.shape[1]
         ctx.set_materialize_grads(False)
         # rows of an array without a gradient carry none either
         ctx.mark_non_differentiable(*[t for t, need in zip(out, ctx.needs_input_grad[1:5]) if not need],
@@ -164,28 +72,20 @@ class _VisibleRows(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         rank, = ctx.saved_tensors
-        A, k, dev = rank.shape[0], ctx.k, rank.device
         grads = [g if need else None for g, need in zip(grads[:4], ctx.needs_input_grad[1:5])]
-        shapes = ((A, 3), (A, 32), (A, k, 3), (A, 6))
         if torch.is_grad_enabled():  # a graph of the backward pass is asked for
+            A = rank.shape[0]
             idx = (rank >= 0).nonzero(as_tuple=True)[0]
-            return (None, *[None if g is None else torch.zeros(s, device=dev).index_add(0, idx, g)
-                            for g, s in zip(grads, shapes)], None)
-        grads = [None if g is None else g.contiguous() for g in grads]
-        if grads[1] is not None and grads[1].data_ptr() % 16:
-            grads[1] = grads[1].clone()
-        d = [None if g is None else torch.empty(s, device=dev) for g, s in zip(grads, shapes)]
-        stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        _n.check(_n.lib.gs_visible_rows_spread(A, k, _p(rank), *[_p(t) for t in grads], *[_p(t) for t in d], stream),
-                 "visible rows backward")
-        return (None, *d, None)
+            return (None, *[None if g is None else
+                            torch.zeros(A, *g.shape[1:], device=g.device).index_add(0, idx, g) for g in grads], None)
+        return (None, *_n.ops.visible_rows_backward(rank, ctx.k, grads, _n.stream_handle(rank.device)), None)
 
 
 def _visible_rows(mask, anchor, feat, offsets, scaling, want_index):
     """anchor[mask], feat[mask], offsets[mask], scaling[mask] and, if wanted, mask.nonzero(): one pass over the arrays
     where they are the dense float32 arrays of a model on the current device with 16-byte rows of features, torch's
     gathers for everything else (other types, strides, devices and mask shapes, n_offsets without a kernel, a stream
-    under capture, functorch transforms)."""
+    under capture)."""
     t4 = (anchor, feat, offsets, scaling)
     if (mask.dtype is torch.bool and mask.is_cuda and mask.dim() == 1 and mask.is_contiguous()
             and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is torch.float32

@@ -5,7 +5,11 @@ resolved, importing this module raises, and every entry point raises
 RuntimeError with the library's message on a non-zero status.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libgsrast.so")
@@ -16,6 +20,28 @@ if not os.path.exists(LIB_PATH):
         "or __graft_entry__.build()); there is no CPU fallback")
 
 lib = C.CDLL(LIB_PATH)
+
+# the torch side of the hot entry points (csrc/torch_ops.cpp), linked against the library above
+OPS_PATH = os.path.join(_HERE, "lib", "gsrast_ops.so")
+
+
+def _load_ops():
+    if not os.path.exists(OPS_PATH):
+        raise ImportError(f"{OPS_PATH} not found: build it first (make -C {os.path.join(_HERE, 'csrc')})")
+    loader = importlib.machinery.ExtensionFileLoader("gsrast_ops", OPS_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("gsrast_ops", loader))
+    loader.exec_module(module)
+    return module
+
+
+ops = _load_ops()
+
+
+def stream_handle(device):
+    """The device's current stream as the number the entry points of `ops` take (0 for the CPU: those entry points
+    refuse its tensors)."""
+    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
+
 
 RESIZE_FN = C.CFUNCTYPE(C.c_void_p, C.c_size_t, C.c_void_p)
 
