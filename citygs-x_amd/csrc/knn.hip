@@ -170,30 +170,87 @@ __global__ void __launch_bounds__(GS_BLOCK_1D) curve_key_kernel(int P, const flo
   idx[i] = (uint32_t)i;
 }
 
-__global__ void __launch_bounds__(GS_BLOCK_1D) gather_points_kernel(int P, const float* __restrict__ pts,
-                                                                    const uint32_t* __restrict__ idx,
-                                                                    float4* __restrict__ sorted_pts) {
-  const int i = blockIdx.x * GS_BLOCK_1D + threadIdx.x;
-  if (i >= P) return;
-  const size_t g = idx[i];
-  sorted_pts[i] = make_float4(pts[3 * g], pts[3 * g + 1], pts[3 * g + 2], 0.f);
+// A value moved round its row of sixteen lanes: lane i reads lane (i + 16 - N) % 16 of the row.
+template <int N>
+__device__ __forceinline__ float row_ror(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, true));
 }
 
-// simple-knn/simple_knn.cu:78-117: one workgroup per run of 1024 sorted points.
-__global__ void __launch_bounds__(MM_THREADS) box_minmax_kernel(int P, const float4* __restrict__ sorted_pts,
-                                                                float* __restrict__ boxes) {
-  __shared__ float s[6][MM_THREADS / GS_WAVE];
+__device__ __forceinline__ float row_max(float v) {
+  v = fmaxf(v, row_ror<8>(v));
+  v = fmaxf(v, row_ror<4>(v));
+  v = fmaxf(v, row_ror<2>(v));
+  return fmaxf(v, row_ror<1>(v));
+}
+
+__device__ __forceinline__ float row_min(float v) {
+  v = fminf(v, row_ror<8>(v));
+  v = fminf(v, row_ror<4>(v));
+  v = fminf(v, row_ror<2>(v));
+  return fminf(v, row_ror<1>(v));
+}
+
+// The points in curve order, and the bounding boxes of every run of KNN_BOX of them (simple-knn/simple_knn.cu:78-117),
+// of every run of KNN_LEAF (one wave each) and of every run of KNN_TWIG (a row of sixteen lanes each): a workgroup
+// per box, a thread per point.  Leaves and twigs are additions to the reference's boxes, which prune work without
+// changing which neighbours are found.  (A gather, a box and a leaf kernel before: 32 us at
+// 1 M points; now 20.)
+__global__ void __launch_bounds__(KNN_BOX) gather_boxes_kernel(int P, const float* __restrict__ pts,
+                                                               const uint32_t* __restrict__ idx,
+                                                               float4* __restrict__ sorted_pts,
+                                                               float* __restrict__ boxes, float* __restrict__ leaves,
+                                                               float* __restrict__ twigs) {
+  static_assert(KNN_LEAF == GS_WAVE && KNN_TWIG == 16, "a leaf is a wave, a twig a row of 16 lanes");
+  constexpr int LEAVES = KNN_BOX / KNN_LEAF;
+  static_assert(LEAVES == 16, "a box is combined from its leaves by one row of lanes");
+  __shared__ float s[6][LEAVES];
+  const int i = blockIdx.x * KNN_BOX + threadIdx.x;
+  const int lane = threadIdx.x & (GS_WAVE - 1), wave = threadIdx.x / GS_WAVE;
   float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-  const int start = blockIdx.x * KNN_BOX;
-  for (int t = threadIdx.x; t < KNN_BOX; t += MM_THREADS) {
-    const int i = start + t;
-    if (i < P) {
-      const float4 p = sorted_pts[i];
-      v[0] = fminf(v[0], p.x); v[1] = fminf(v[1], p.y); v[2] = fminf(v[2], p.z);
-      v[3] = fmaxf(v[3], p.x); v[4] = fmaxf(v[4], p.y); v[5] = fmaxf(v[5], p.z);
+  if (i < P) {
+    const size_t g = idx[i];
+    const float4 p = make_float4(pts[3 * g], pts[3 * g + 1], pts[3 * g + 2], 0.f);
+    sorted_pts[i] = p;
+    // (a NaN coordinate leaves the box as it is: minima and maxima pass it over)
+    v[0] = fminf(v[0], p.x); v[1] = fminf(v[1], p.y); v[2] = fminf(v[2], p.z);
+    v[3] = fmaxf(v[3], p.x); v[4] = fmaxf(v[4], p.y); v[5] = fmaxf(v[5], p.z);
+  }
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    v[c] = row_min(v[c]);
+    v[3 + c] = row_max(v[3 + c]);
+  }
+  if ((lane & (KNN_TWIG - 1)) == 0 && i < P) {
+#pragma unroll
+    for (int c = 0; c < 6; c++) twigs[6 * (size_t)(i / KNN_TWIG) + c] = v[c];
+  }
+#pragma unroll
+  for (int d = KNN_TWIG; d < GS_WAVE; d <<= 1) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      v[c] = fminf(v[c], __shfl_xor(v[c], d, GS_WAVE));
+      v[3 + c] = fmaxf(v[3 + c], __shfl_xor(v[3 + c], d, GS_WAVE));
     }
   }
-  reduce6(v, s, boxes + 6 * blockIdx.x);
+  if (lane == 0) {
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+      if (i < P) leaves[6 * (size_t)(i / KNN_LEAF) + c] = v[c];
+      s[c][wave] = v[c];
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const float mn = row_min(s[c][lane & (LEAVES - 1)]), mx = row_max(s[3 + c][lane & (LEAVES - 1)]);
+      if (lane == 0) {
+        boxes[6 * blockIdx.x + c] = mn;
+        boxes[6 * blockIdx.x + 3 + c] = mx;
+      }
+    }
+  }
 }
 
 // Bounding box of every run of KNN_GROUP consecutive boxes: lets the search discard that many boxes with
@@ -218,41 +275,6 @@ __global__ void __launch_bounds__(GS_WAVE) box_group_kernel(int nboxes, const fl
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int c = 0; c < 6; c++) groups[6 * blockIdx.x + c] = v[c];
-  }
-}
-
-// Bounding box of every run of KNN_LEAF consecutive sorted points (one wave each) and, inside it, of every run
-// of KNN_TWIG points (a 16-lane row each): the two finest levels of the search.  Like the groups, additions that
-// prune work without changing which neighbours are found.
-__global__ void __launch_bounds__(GS_BLOCK_1D) leaf_minmax_kernel(int P, const float4* __restrict__ sorted_pts,
-                                                                  float* __restrict__ leaves,
-                                                                  float* __restrict__ twigs) {
-  static_assert(KNN_LEAF == GS_WAVE && KNN_TWIG == 16, "a leaf is a wave, a twig a row of 16 lanes");
-  const int i = blockIdx.x * GS_BLOCK_1D + threadIdx.x;
-  float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-  if (i < P) {
-    const float4 p = sorted_pts[i];
-    v[0] = v[3] = p.x; v[1] = v[4] = p.y; v[2] = v[5] = p.z;
-  }
-#pragma unroll
-  for (int d = 1; d < GS_WAVE; d <<= 1) {
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      v[c] = fminf(v[c], __shfl_xor(v[c], d, GS_WAVE));
-      v[3 + c] = fmaxf(v[3 + c], __shfl_xor(v[3 + c], d, GS_WAVE));
-    }
-    if (d == KNN_TWIG / 2) {
-      const int twig = i / KNN_TWIG;
-      if ((threadIdx.x & (KNN_TWIG - 1)) == 0 && twig * KNN_TWIG < P) {
-#pragma unroll
-        for (int c = 0; c < 6; c++) twigs[6 * (size_t)twig + c] = v[c];
-      }
-    }
-  }
-  const int leaf = i / KNN_LEAF;
-  if ((threadIdx.x & (GS_WAVE - 1)) == 0 && leaf * KNN_LEAF < P) {
-#pragma unroll
-    for (int c = 0; c < 6; c++) leaves[6 * (size_t)leaf + c] = v[c];
   }
 }
 
@@ -303,13 +325,10 @@ __device__ __forceinline__ float point_box_dist2(const float4& p, const NodeBox&
 }
 
 // Keeps the three smallest of {knn[0..2], dist(ref, p)} in ascending order (simple_knn.cu:131-145 inserts by
-// compare-and-swap; minimum and medians leave the same three values).  A NaN distance (a point with a NaN
-// coordinate) is never inserted, as with the reference's `knn[j] > dist`: the minimum with FLT_MAX turns it into a
-// value that changes nothing.
-__device__ __forceinline__ void update3(const float4& ref, const float4& p, float* knn, bool skip = false) {
-  const float dx = p.x - ref.x, dy = p.y - ref.y, dz = p.z - ref.z;
-  float dist = fminf((dx * dx + dy * dy) + dz * dz, FLT_MAX);
-  dist = skip ? FLT_MAX : dist;
+// compare-and-swap; minimum and medians leave the same three values).  A distance that is infinite or larger than
+// FLT_MAX changes nothing.
+__device__ __forceinline__ void update3(const float dx, const float dy, const float dz, float* knn) {
+  const float dist = (dx * dx + dy * dy) + dz * dz;
   const float n0 = fminf(knn[0], dist);
   const float n1 = __builtin_amdgcn_fmed3f(knn[0], knn[1], dist);
   const float n2 = __builtin_amdgcn_fmed3f(knn[1], knn[2], dist);
@@ -318,27 +337,45 @@ __device__ __forceinline__ void update3(const float4& ref, const float4& p, floa
   knn[2] = n2;
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int d = GS_WAVE / 2; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, GS_WAVE));
-  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+// Every lane meets the points that the sixteen lanes of its row hold (from the FIRST-th one round; 1 leaves out the
+// lane's own).  The rotation is an operand modifier of the subtractions, so a distance costs eleven vector
+// instructions and no memory access.
+template <int FIRST, int LAST = KNN_TWIG>
+__device__ __forceinline__ void meet_row(const float4& p, const float4& c, float* knn) {
+  if constexpr (FIRST < LAST) {
+    update3(row_ror<FIRST>(c.x) - p.x, row_ror<FIRST>(c.y) - p.y, row_ror<FIRST>(c.z) - p.z, knn);
+    meet_row<FIRST + 1, LAST>(p, c, knn);
+  }
+}
+template <>
+__device__ __forceinline__ void meet_row<0, KNN_TWIG>(const float4& p, const float4& c, float* knn) {
+  update3(c.x - p.x, c.y - p.y, c.z - p.z, knn);
+  meet_row<1, KNN_TWIG>(p, c, knn);
 }
 
 // simple-knn/simple_knn.cu:147-183.  The reference gives every point a thread that seeds a rejection radius from
 // the point's neighbours in sorted order and then walks all boxes, skipping those farther away than that radius or
 // than the third-best distance so far (simple_knn.cu:161-171).  Here a wave owns a leaf, 64 consecutive points
-// along the curve, and walks the tree for all of them at once:
-//   * every point first meets the points of its own leaf and of the two leaves next to it along the curve, which
-//     gives it a third-best distance to start from;
-//   * 64 nodes of a level (groups of boxes, boxes, 16-point twigs) are tested in one step, a lane each, against
-//     the leaf's bounding box and the largest third-best distance of the wave; a box or twig that passes is then
-//     tested by every lane for its own point and its own third-best distance, the reference's test, and opened
-//     if any lane needs it (the first test alone would open everything between the two ends of a leaf whose
-//     points lie in two places, where the curve leaves the occupied part of the grid and comes back elsewhere);
-//   * the points of the twigs that are opened go to LDS 64 at a time and every lane measures its distance to each.
+// along the curve, and each of its four rows of sixteen lanes a twig of it:
+//   * every point first meets the points of its own twig and of the SEED twigs on either side of it along the curve,
+//     which gives it a third-best distance to start from;
+//   * 64 nodes of a level (groups of boxes, boxes, twigs) are tested in one step, a lane each: groups and boxes
+//     against the leaf's bounding box and the largest third-best distance of the wave, the twigs of a box against
+//     each row's own bounding box and largest third-best distance; a box or twig that passes is then tested by every
+//     lane for its own point and its own third-best distance, the reference's test, and opened by the rows (a box:
+//     by the wave) that have a lane which needs it (the first test alone would open everything between the two ends
+//     of a leaf whose points lie in two places, where the curve leaves the occupied part of the grid and comes back
+//     elsewhere);
+//   * every row then walks its own list of twigs, its sixteen lanes holding the sixteen points, the next twig's
+//     points on their way meanwhile.
 // A lane then also sees points that its own test would have skipped; only true distances are ever inserted, and
 // nothing nearer than a point's third-best distance is ever skipped, so the three distances are those of a
 // brute-force search whatever the order.
+// Bound by vector issue.  With the whole leaf as the unit that opens twigs (64 points against every point of the
+// three leaves around it and of the twigs any of them needs, over LDS) the search took 335 us for 1 M points of an
+// SfM-like cloud; with the row as the unit 298 us.
+constexpr int SEED = 2;
+
 __global__ void __launch_bounds__(GS_BLOCK_1D) box_mean_dist_kernel(int P, const float4* __restrict__ sorted_pts,
                                                                     const uint32_t* __restrict__ idx,
                                                                     const float* __restrict__ boxes, int nboxes,
@@ -346,100 +383,114 @@ __global__ void __launch_bounds__(GS_BLOCK_1D) box_mean_dist_kernel(int P, const
                                                                     const float* __restrict__ leaves,
                                                                     const float* __restrict__ twigs,
                                                                     float* __restrict__ out) {
-  constexpr int TWIGS_PER_BOX = KNN_BOX / KNN_TWIG, TWIGS_PER_LEAF = KNN_LEAF / KNN_TWIG;
-  constexpr int TWIGS_PER_STEP = GS_WAVE / KNN_TWIG;
+  constexpr int TWIGS_PER_BOX = KNN_BOX / KNN_TWIG, ROWS = KNN_LEAF / KNN_TWIG;
   static_assert(TWIGS_PER_BOX == GS_WAVE && KNN_GROUP == GS_WAVE, "a lane tests one node of a level");
-  __shared__ float4 s_pts[GS_BLOCK_1D / GS_WAVE][GS_WAVE];
-  const int lane = threadIdx.x & (GS_WAVE - 1);
+  const int lane = threadIdx.x & (GS_WAVE - 1), row = lane / KNN_TWIG, in_row = lane % KNN_TWIG;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GS_WAVE);
   const int own = blockIdx.x * (GS_BLOCK_1D / GS_WAVE) + wave;  // this wave's leaf
   if (own * KNN_LEAF >= P) return;                              // (whole waves only: no workgroup barrier below)
   const int k = own * KNN_LEAF + lane;
-  const int n_own = min(KNN_LEAF, P - own * KNN_LEAF);
-  // lanes past the last point keep step with a copy of it and store nothing
-  const float4 p = sorted_pts[min(k, P - 1)];
+  const int ntwigs = (P + KNN_TWIG - 1) / KNN_TWIG;
+  const float4 nowhere = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f);
+  // the row's lanes fetch the points of twig t; a lane without a point (t < 0: no twig) holds one that is infinitely
+  // far away, and so does one whose point has a NaN coordinate (a NaN distance is never inserted, as with the
+  // reference's `knn[j] > dist`)
+  auto points_of = [&](int t) {
+    const int at = t * KNN_TWIG + in_row;
+    return t >= 0 && at < P ? sorted_pts[at] : nowhere;
+  };
+  auto without_nan = [&](float4 c) {
+    return c.x == c.x && c.y == c.y && c.z == c.z ? c : nowhere;
+  };
+  const float4 p = k < P ? sorted_pts[k] : nowhere;
   // a point with a non-finite coordinate has no finite distance to anything: its result never changes
-  const bool searching = k < P && fabsf(p.x) < __builtin_inff() && fabsf(p.y) < __builtin_inff() &&
+  const bool searching = fabsf(p.x) < __builtin_inff() && fabsf(p.y) < __builtin_inff() &&
                          fabsf(p.z) < __builtin_inff();
   float best[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
-  float4* mine = s_pts[wave];
-  auto wave_sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
 
-  // The leaf itself and the leaves before and after it along the curve come first, unconditionally: they hold
-  // most of the neighbours, and the third-best distance they leave is the bound for everything that follows
-  // (the reference seeds its rejection radius from a point's neighbours in sorted order too,
-  // simple_knn.cu:153-160).
-  const int nleaves = (P + KNN_LEAF - 1) / KNN_LEAF;
+  // The row's own twig and those before and after it along the curve come first, unconditionally: they hold most of
+  // the neighbours, and the third-best distance they leave is the bound for everything that follows (the reference
+  // seeds its rejection radius from a point's neighbours in sorted order too, simple_knn.cu:153-160).
+  {
+    const int t = own * ROWS + row;
+    float4 seed[2 * SEED];
 #pragma unroll
-  for (int side = -1; side <= 1; side++) {
-    const int other = own + side;
-    if (other < 0 || other >= nleaves) continue;  // wave-uniform
-    const int at = other * KNN_LEAF + lane;
-    // a slot without a point holds one that is infinitely far away
-    mine[lane] = side == 0 ? p
-                 : at < P  ? sorted_pts[at]
-                           : make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f);
-    wave_sync();
-    const int n = side == 0 ? n_own : KNN_LEAF;
-    for (int i = 0; i < n; i++) update3(p, mine[i], best, side == 0 && i == lane);  // (not its own neighbour)
-    wave_sync();
+    for (int s = 0; s < 2 * SEED; s++) {
+      const int other = t + (s < SEED ? s - SEED : s - SEED + 1);
+      seed[s] = points_of(other < ntwigs ? other : -1);
+    }
+    meet_row<1>(p, without_nan(p), best);
+#pragma unroll 1
+    for (int s = 0; s < 2 * SEED; s++) meet_row<0>(p, without_nan(seed[s]), best);
   }
 
   float q[6];  // the leaf's bounding box
 #pragma unroll
   for (int c = 0; c < 6; c++) q[c] = leaves[6 * (size_t)own + c];
+  NodeBox row_box[ROWS];  // the twigs'
+#pragma unroll
+  for (int r = 0; r < ROWS; r++) row_box[r] = load_box(twigs + 6 * (size_t)(own * ROWS + r), own * ROWS + r < ntwigs);
   // (a margin of a few units in the last place: the node test and the point distances round differently)
   constexpr float MARGIN = 1.0f + 0x1p-20f;
-  float reach = wave_max(searching ? best[2] : 0.f) * MARGIN;
+  float row_reach[ROWS], reach;  // wave-uniform
+  auto update_reach = [&] {
+    const float m = row_max(searching ? best[2] : 0.f) * MARGIN;
+    reach = 0.f;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+      row_reach[r] = __builtin_bit_cast(
+          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), r * KNN_TWIG));
+      reach = fmaxf(reach, row_reach[r]);
+    }
+  };
+  update_reach();
 
   const int own_box = own / (KNN_BOX / KNN_LEAF);
-  // does any lane need a node, by the reference's test (simple_knn.cu:161-171) for its own point?
-  auto needed = [&](const NodeBox& n) {
-    const float d = point_box_dist2(p, n);
-    return (gs_ballot(searching) & gs_ballot(!(d > best[2]))) != 0ull;
-  };
+  const uint64_t searching_m = gs_ballot(searching);
+  // which lanes need a node, by the reference's test (simple_knn.cu:161-171) for their own points?
+  auto needing = [&](const NodeBox& n) { return searching_m & gs_ballot(!(point_box_dist2(p, n) > best[2])); };
   auto open_box = [&](int b) {
     const int t = b * TWIGS_PER_BOX + lane;
-    const NodeBox mine_t = load_box(twigs + 6 * (size_t)t, (size_t)t * KNN_TWIG < (size_t)P);
-    uint64_t near = gs_ballot(!(boxes_dist2(q, mine_t) > reach));
-    // (the twigs of the three leaves met at the start are not met again)
-    const int met = (own - 1) * TWIGS_PER_LEAF - b * TWIGS_PER_BOX;
-    const int met_lo = max(met, 0), met_hi = min(met + 3 * TWIGS_PER_LEAF, TWIGS_PER_BOX);
-    if (met_lo < met_hi) near &= ~(((1ull << (met_hi - met_lo)) - 1ull) << met_lo);
-    uint64_t todo = 0ull;
-    while (near != 0ull) {
-      const int c = (int)__builtin_ctzll(near);
-      near &= near - 1ull;
-      if (needed(box_of_lane(mine_t, c))) todo |= 1ull << c;
-    }
-    while (todo != 0ull) {
-      int tw[TWIGS_PER_STEP], n = 0;
+    const NodeBox mine_t = load_box(twigs + 6 * (size_t)t, t < ntwigs);
+    uint64_t near[ROWS], any = 0ull;
 #pragma unroll
-      for (int e = 0; e < TWIGS_PER_STEP; e++) {
-        tw[e] = -1;
-        if (todo != 0ull) {
-          tw[e] = (int)__builtin_ctzll(todo);
-          todo &= todo - 1ull;
-          n++;
-        }
-      }
-      const int part = lane / KNN_TWIG;
-      const int sel = part == 0 ? tw[0] : part == 1 ? tw[1] : part == 2 ? tw[2] : tw[3];
-      const size_t at = ((size_t)b * TWIGS_PER_BOX + (size_t)max(sel, 0)) * KNN_TWIG + (size_t)(lane % KNN_TWIG);
-      // a slot without a point holds one that is infinitely far away
-      float4 cand = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f);
-      if (sel >= 0 && at < (size_t)P) cand = sorted_pts[at];
-      mine[lane] = cand;
-      wave_sync();
-      const int m = n * KNN_TWIG;
-      for (int i = 0; i < m; i++) update3(p, mine[i], best);
-      wave_sync();
+    for (int r = 0; r < ROWS; r++) {
+      const float qr[6] = {row_box[r].lo[0], row_box[r].lo[1], row_box[r].lo[2],
+                           row_box[r].hi[0], row_box[r].hi[1], row_box[r].hi[2]};
+      near[r] = gs_ballot(!(boxes_dist2(qr, mine_t) > row_reach[r]));
+      // (the twigs met at the start are not met again)
+      const int met = own * ROWS + r - SEED - b * TWIGS_PER_BOX;
+      const int met_lo = max(met, 0), met_hi = min(met + 2 * SEED + 1, TWIGS_PER_BOX);
+      if (met_lo < met_hi) near[r] &= ~(((1ull << (met_hi - met_lo)) - 1ull) << met_lo);
+      any |= near[r];
     }
-    reach = wave_max(searching ? best[2] : 0.f) * MARGIN;
+    if (any == 0ull) return;
+    const uint64_t row_near = row == 0 ? near[0] : row == 1 ? near[1] : row == 2 ? near[2] : near[3];
+    // the row's list, one bit per twig of the box
+    uint64_t todo = 0ull;
+    while (any != 0ull) {
+      const int c = (int)__builtin_ctzll(any);
+      any &= any - 1ull;
+      const uint64_t need = needing(box_of_lane(mine_t, c));
+      const bool row_needs = ((uint32_t)(need >> (row * KNN_TWIG)) & 0xFFFFu) != 0u;
+      todo |= row_needs ? 1ull << c : 0ull;
+    }
+    todo &= row_near;
+    auto next = [&] {
+      const int c = todo != 0ull ? b * TWIGS_PER_BOX + (int)__builtin_ctzll(todo) : -1;
+      todo &= todo - 1ull;
+      return points_of(c);
+    };
+    uint64_t left = gs_ballot(todo != 0ull);
+    float4 ahead = nowhere;
+    if (left != 0ull) ahead = next();
+    while (left != 0ull) {
+      const float4 c = without_nan(ahead);
+      left = gs_ballot(todo != 0ull);
+      if (left != 0ull) ahead = next();
+      meet_row<0>(p, c, best);
+    }
+    update_reach();
   };
 
   open_box(own_box);
@@ -457,10 +508,11 @@ __global__ void __launch_bounds__(GS_BLOCK_1D) box_mean_dist_kernel(int P, const
       while (bm != 0ull) {
         const int c = (int)__builtin_ctzll(bm);
         bm &= bm - 1ull;
-        if (needed(box_of_lane(mine_b, c))) open_box(gi * KNN_GROUP + c);
+        if (needing(box_of_lane(mine_b, c)) != 0ull) open_box(gi * KNN_GROUP + c);
       }
     }
   }
+  if (!searching) best[0] = best[1] = best[2] = FLT_MAX;  // (what NaN differences left there)
   if (k < P) out[idx[k]] = ((best[0] + best[1]) + best[2]) / 3.0f;
 }
 
@@ -506,14 +558,9 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
   }
   const uint32_t* idx_sorted = sort_result_in_b(end_bit) ? idx_b : idx_a;
   {
-    StageScope _t("knn_gather", stream);
-    hipLaunchKernelGGL(gather_points_kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, P, points, idx_sorted,
-                       sorted_pts);
-  }
-  {
     StageScope _t("knn_boxes", stream);
-    hipLaunchKernelGGL(box_minmax_kernel, dim3(nboxes), dim3(MM_THREADS), 0, stream, P, sorted_pts, boxes);
-    hipLaunchKernelGGL(leaf_minmax_kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, P, sorted_pts, leaves, twigs);
+    hipLaunchKernelGGL(gather_boxes_kernel, dim3(nboxes), dim3(KNN_BOX), 0, stream, P, points, idx_sorted, sorted_pts,
+                       boxes, leaves, twigs);
     hipLaunchKernelGGL(box_group_kernel, dim3((nboxes + KNN_GROUP - 1) / KNN_GROUP), dim3(GS_WAVE), 0, stream, nboxes,
                        boxes, groups);
   }

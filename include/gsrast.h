@@ -503,7 +503,7 @@ int gs_selftest_reductions(const float* in, float* out_wave, float* out_rows, gs
  * tile_count, bucket_scatter, tile_sort, or on the radix route inclusive_sum,
  * duplicate_with_keys, sort_pairs, identify_tile_ranges; pack_operands; render_fwd,
  * render_bwd, preprocess_bwd; knn_dist2 and its phases knn_minmax, knn_keys,
- * knn_sort, knn_gather, knn_boxes, knn_box_mean_dist)
+ * knn_sort, knn_boxes, knn_box_mean_dist)
  * is bracketed by an event pair on its stream.  Nothing is synchronised until
  * gs_stage_timing_collect, which waits for the recorded events and writes one
  * line per stage, "name total_ms launches", into report (host buffer), then
