@@ -82,6 +82,31 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
   return base + inc - v;
 }
 
+// counts[0 .. n) -> exclusive prefixes in place by one workgroup of 1024 threads; returns the total, in every thread.
+__device__ __forceinline__ uint32_t exclusive_prefix_in_place(uint32_t n, uint32_t* __restrict__ counts,
+                                                              uint32_t* s_wave /*1024/64*/) {
+  constexpr int ITEMS = 4;
+  uint32_t carry = 0;
+  for (uint32_t start = 0; start < n; start += 1024 * ITEMS) {
+    const uint32_t first = start + threadIdx.x * ITEMS;
+    uint32_t v[ITEMS], sum = 0;
+#pragma unroll
+    for (int q = 0; q < ITEMS; q++) {
+      v[q] = first + q < n ? counts[first + q] : 0u;
+      sum += v[q];
+    }
+    uint32_t total;
+    uint32_t run = carry + block_exclusive_scan<1024>(sum, s_wave, total);
+#pragma unroll
+    for (int q = 0; q < ITEMS; q++) {
+      if (first + q < n) counts[first + q] = run;
+      run += v[q];
+    }
+    carry += total;
+  }
+  return carry;
+}
+
 // Workgroups go to the eight XCDs in turn (workgroup b of a launch runs on XCD b % 8), and each XCD has its own L2.
 // This renumbers them so that the workgroups of one XCD hold consecutive indices (XCD 0 the first eighth, and so
 // on, each in launch order): work items that are neighbours in memory then share an L2.  A bijection on [0, n).

@@ -34,26 +34,8 @@ visible_count_kernel(uint32_t A, uint32_t chunks, const uint8_t* __restrict__ ma
 // One workgroup turns the counts into exclusive prefixes in place and hands the total to the host.
 __global__ void __launch_bounds__(1024)
 visible_spine_kernel(uint32_t chunks, uint32_t* __restrict__ counts, uint32_t* total_out) {
-  constexpr int ITEMS = 4;
   __shared__ uint32_t s_wave[1024 / GS_WAVE];
-  uint32_t carry = 0;
-  for (uint32_t start = 0; start < chunks; start += 1024 * ITEMS) {
-    const uint32_t first = start + threadIdx.x * ITEMS;
-    uint32_t v[ITEMS], sum = 0;
-#pragma unroll
-    for (int q = 0; q < ITEMS; q++) {
-      v[q] = first + q < chunks ? counts[first + q] : 0u;
-      sum += v[q];
-    }
-    uint32_t total;
-    uint32_t run = carry + block_exclusive_scan<1024>(sum, s_wave, total);
-#pragma unroll
-    for (int q = 0; q < ITEMS; q++) {
-      if (first + q < chunks) counts[first + q] = run;
-      run += v[q];
-    }
-    carry += total;
-  }
+  const uint32_t carry = exclusive_prefix_in_place(chunks, counts, s_wave);
   if (threadIdx.x == 0) {
     counts[chunks] = carry;
     // the host may be polling this word (host-visible memory)

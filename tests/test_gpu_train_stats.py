@@ -99,3 +99,22 @@ def test_update_max_radii_matches_torch_statement():
     got = gs_densify.update_max_radii(m.to(DEV), radii.to(DEV), vis.to(DEV)).cpu()
     assert torch.equal(got, want)
     assert torch.equal(got[~vis], m[~vis])
+
+
+@pytest.mark.parametrize("A,k,p", [(1, 1, (1.0, 1.0, 1.0)), (255, 10, (1.0, 0.5, 0.9)), (257, 256, (0.9, 0.6, 0.9)),
+                                   (700, 255, (1.0, 0.97, 0.6)), (300, 257, (0.7, 0.6, 0.9)), (1025, 3, (0.4, 0.0, 1.0)),
+                                   (3000, 7, (0.5, 0.6, 0.9))])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_training_stats_chunk_edges(orc, A, k, p, offset):
+    """Anchors, candidates and rounds that end inside and at the edge of a chunk, the offset counts on either side of
+    the last one that chunks take, and masks that start at any byte.  Sums of k terms in the oracle's order."""
+    import gs_densify
+    vis, sel, flt, grad, opacity, acc = _case(A, k, A + k, *p)
+    ref = orc.training_stats(acc[0].numpy(), acc[1].numpy(), acc[2].numpy(), acc[3].numpy(), k, grad.numpy(),
+                             opacity.numpy(), flt.numpy(), sel.numpy(), vis.numpy())
+    shifted = lambda m: torch.cat([torch.ones(offset, dtype=torch.bool), m]).to(DEV)[offset:]
+    d = [t.to(DEV) for t in acc]
+    gs_densify.training_statis(d[0], d[1], d[2], d[3], k, grad.to(DEV), opacity.to(DEV), shifted(flt), shifted(sel),
+                               shifted(vis))
+    for got, want in zip(d, ref):
+        assert np.abs(got.cpu().numpy().ravel() - want).max() <= 1e-6 * max(1.0, np.abs(want).max())
