@@ -373,10 +373,11 @@ __device__ __forceinline__ void meet_row<0, KNN_TWIG>(const float4& p, const flo
 // brute-force search whatever the order.
 // Bound by vector issue.  With the whole leaf as the unit that opens twigs (64 points against every point of the
 // three leaves around it and of the twigs any of them needs, over LDS) the search took 335 us for 1 M points of an
-// SfM-like cloud; with the row as the unit 298 us.
+// SfM-like cloud; with the row as the unit 298 us, and 281 us with a workgroup per wave, whose place is taken as soon
+// as that wave ends (a leaf among sparse points takes ten times as long as the median).
 constexpr int SEED = 2;
 
-__global__ void __launch_bounds__(GS_BLOCK_1D) box_mean_dist_kernel(int P, const float4* __restrict__ sorted_pts,
+__global__ void __launch_bounds__(GS_WAVE) box_mean_dist_kernel(int P, const float4* __restrict__ sorted_pts,
                                                                     const uint32_t* __restrict__ idx,
                                                                     const float* __restrict__ boxes, int nboxes,
                                                                     const float* __restrict__ groups,
@@ -385,10 +386,8 @@ __global__ void __launch_bounds__(GS_BLOCK_1D) box_mean_dist_kernel(int P, const
                                                                     float* __restrict__ out) {
   constexpr int TWIGS_PER_BOX = KNN_BOX / KNN_TWIG, ROWS = KNN_LEAF / KNN_TWIG;
   static_assert(TWIGS_PER_BOX == GS_WAVE && KNN_GROUP == GS_WAVE, "a lane tests one node of a level");
-  const int lane = threadIdx.x & (GS_WAVE - 1), row = lane / KNN_TWIG, in_row = lane % KNN_TWIG;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GS_WAVE);
-  const int own = blockIdx.x * (GS_BLOCK_1D / GS_WAVE) + wave;  // this wave's leaf
-  if (own * KNN_LEAF >= P) return;                              // (whole waves only: no workgroup barrier below)
+  const int lane = threadIdx.x, row = lane / KNN_TWIG, in_row = lane % KNN_TWIG;
+  const int own = blockIdx.x;  // this wave's leaf
   const int k = own * KNN_LEAF + lane;
   const int ntwigs = (P + KNN_TWIG - 1) / KNN_TWIG;
   const float4 nowhere = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f);
@@ -566,7 +565,7 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
   }
   {
     StageScope _t("knn_box_mean_dist", stream);
-    hipLaunchKernelGGL(box_mean_dist_kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, P, sorted_pts, idx_sorted,
+    hipLaunchKernelGGL(box_mean_dist_kernel, dim3((P + KNN_LEAF - 1) / KNN_LEAF), dim3(GS_WAVE), 0, stream, P, sorted_pts, idx_sorted,
                        boxes, nboxes, groups, leaves, twigs, mean_dist2);
   }
   return 0;
