@@ -224,7 +224,10 @@ inline bool sort_result_in_b(int end_bit) { return (sort_num_passes(end_bit) & 1
 int launch_sort_pairs_u64(int64_t n, uint64_t* keys_a, uint64_t* keys_b, uint32_t* vals_a, uint32_t* vals_b,
                           int end_bit, void* temp, hipStream_t stream);
 int launch_sort_pairs_u32(int64_t n, uint32_t* keys_a, uint32_t* keys_b, uint32_t* vals_a, uint32_t* vals_b,
-                          int end_bit, void* temp, hipStream_t stream);
+                          int end_bit, void* temp, hipStream_t stream, bool counted = false);
+// counted: the caller's own kernels have done the sort's first two steps: cleared the first sort_clear_words words of
+// the workspace, then counted, in its first words, how often every value of every digit occurs ([pass][digit])
+int64_t sort_clear_words(int64_t n, int end_bit);
 
 // ---- tile render ----
 struct RenderFwdArgs {

@@ -27,9 +27,12 @@ constexpr int KNN_LEAF = 64;   // points per leaf box inside a box (one leaf tes
 constexpr int KNN_TWIG = 16;   // points per twig box inside a leaf (the finest level)
 constexpr int MM_BLOCKS = 512;
 constexpr int MM_THREADS = 256;
+constexpr int KEY_THREADS = 512;
+constexpr int KEY_BLOCKS = 256;  // at most: a workgroup adds its digit counts to the sort's once
+constexpr int KEY_BITS = 32;     // 4 passes (even): the sorted pairs come back where they were
 
 struct KnnLayout {
-  size_t partial, minmax, codes_a, codes_b, idx_a, idx_b, sorted_pts, boxes, groups, leaves, twigs, sort_temp, total;
+  size_t partial, codes_a, codes_b, idx_a, idx_b, sorted_pts, boxes, groups, leaves, twigs, sort_temp, total;
 };
 
 KnnLayout knn_layout(int P) {
@@ -43,7 +46,6 @@ KnnLayout knn_layout(int P) {
   const size_t n = (size_t)(P > 0 ? P : 1);
   const size_t nb = (n + KNN_BOX - 1) / KNN_BOX;
   L.partial = take(sizeof(float) * 6 * MM_BLOCKS);
-  L.minmax = take(sizeof(float) * 6);
   L.codes_a = take(sizeof(uint32_t) * n);
   L.codes_b = take(sizeof(uint32_t) * n);
   L.idx_a = take(sizeof(uint32_t) * n);
@@ -58,8 +60,9 @@ KnnLayout knn_layout(int P) {
   return L;
 }
 
-__device__ __forceinline__ void reduce6(float* v, float (*s)[MM_THREADS / GS_WAVE], float* out) {
-  // v[0..2] min, v[3..5] max
+// v[0..2] min, v[3..5] max over the workgroup; thread 0 leaves them in out (LDS or memory)
+template <int THREADS>
+__device__ __forceinline__ void reduce6(float* v, float (*s)[THREADS / GS_WAVE], float* out) {
 #pragma unroll
   for (int d = GS_WAVE / 2; d >= 1; d >>= 1) {
 #pragma unroll
@@ -78,7 +81,7 @@ __device__ __forceinline__ void reduce6(float* v, float (*s)[MM_THREADS / GS_WAV
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       float mn = s[k][0], mx = s[3 + k][0];
-      for (int w = 1; w < MM_THREADS / GS_WAVE; w++) {
+      for (int w = 1; w < THREADS / GS_WAVE; w++) {
         mn = fminf(mn, s[k][w]);
         mx = fmaxf(mx, s[3 + k][w]);
       }
@@ -89,9 +92,12 @@ __device__ __forceinline__ void reduce6(float* v, float (*s)[MM_THREADS / GS_WAV
 }
 
 // (The reference reduces from 0, simple-knn/simple_knn.cu:191, which makes its grid include the origin; the keys
-// here are only a means of ordering, so the grid is the points' own bounding box.)
+// here are only a means of ordering, so the grid is the points' own bounding box.)  Clears the sort's words on the way.
 __global__ void __launch_bounds__(MM_THREADS) minmax_partial_kernel(int P, const float* __restrict__ pts,
-                                                                     float* __restrict__ partial) {
+                                                                     float* __restrict__ partial, int64_t clear_words,
+                                                                     uint32_t* __restrict__ clear) {
+  for (int64_t i = (int64_t)blockIdx.x * MM_THREADS + threadIdx.x; i < clear_words; i += MM_BLOCKS * MM_THREADS)
+    clear[i] = 0u;
   __shared__ float s[6][MM_THREADS / GS_WAVE];
   float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
   for (int i = blockIdx.x * MM_THREADS + threadIdx.x; i < P; i += MM_BLOCKS * MM_THREADS) {
@@ -102,21 +108,7 @@ __global__ void __launch_bounds__(MM_THREADS) minmax_partial_kernel(int P, const
       v[3 + k] = fmaxf(v[3 + k], c);
     }
   }
-  reduce6(v, s, partial + 6 * blockIdx.x);
-}
-
-__global__ void __launch_bounds__(MM_THREADS) minmax_final_kernel(const float* __restrict__ partial,
-                                                                   float* __restrict__ minmax) {
-  __shared__ float s[6][MM_THREADS / GS_WAVE];
-  float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-  for (int b = threadIdx.x; b < MM_BLOCKS; b += MM_THREADS) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      v[k] = fminf(v[k], partial[6 * b + k]);
-      v[3 + k] = fmaxf(v[3 + k], partial[6 * b + 3 + k]);
-    }
-  }
-  reduce6(v, s, minmax);
+  reduce6<MM_THREADS>(v, s, partial + 6 * blockIdx.x);
 }
 
 __device__ __forceinline__ uint32_t spread10(uint32_t x) {  // every bit of a 10-bit number to every third place
@@ -155,19 +147,56 @@ __device__ __forceinline__ uint32_t hilbert30(uint32_t x, uint32_t y, uint32_t z
   return (spread10(X[0] ^ t) << 2) | (spread10(X[1] ^ t) << 1) | spread10(X[2] ^ t);
 }
 
-__global__ void __launch_bounds__(GS_BLOCK_1D) curve_key_kernel(int P, const float* __restrict__ pts,
-                                                                const float* __restrict__ minmax,
-                                                                uint32_t* __restrict__ codes, uint32_t* __restrict__ idx) {
-  const int i = blockIdx.x * GS_BLOCK_1D + threadIdx.x;
-  if (i >= P) return;
-  // cubic cells: the longest side of the bounding box takes the 1024 steps
-  const float side = fmaxf(fmaxf(minmax[3] - minmax[0], minmax[4] - minmax[1]), minmax[5] - minmax[2]);
-  uint32_t c[3];
+// Every point's key, and the digit counts of the sort that follows.  17 us at 1 M points (20 with twice the workgroups);
+// as kernels of their own the keys took 9, the rest of the bounding box 4 and the counts, which read the keys again, 15.
+__global__ void __launch_bounds__(KEY_THREADS) curve_key_kernel(int P, const float* __restrict__ pts,
+                                                                const float* __restrict__ partial,
+                                                                uint32_t* __restrict__ codes, uint32_t* __restrict__ idx,
+                                                                uint32_t* __restrict__ hist) {
+  constexpr int RADIX = 1 << SORT_DIGIT_BITS, PASSES = (KEY_BITS + SORT_DIGIT_BITS - 1) / SORT_DIGIT_BITS;
+  // the last digit has few values, which would make a wave's counts queue for the same words: sixteen counts each
+  constexpr int LAST_COPIES = 16;
+  static_assert((1 << (KEY_BITS - (PASSES - 1) * SORT_DIGIT_BITS)) * LAST_COPIES == RADIX, "fills the last row");
+  static_assert(KEY_THREADS == RADIX && MM_BLOCKS == KEY_THREADS, "a thread per digit value and per partial box");
+  __shared__ uint32_t s_hist[PASSES][RADIX];
+  __shared__ float s[6][KEY_THREADS / GS_WAVE];
+  __shared__ float s_box[6];
 #pragma unroll
-  for (int k = 0; k < 3; k++)
-    c[k] = min(f2u_sat(((pts[3 * (size_t)i + k] - minmax[k]) / side) * (float)((1 << 10) - 1)), (1u << 10) - 1u);
-  codes[i] = hilbert30(c[0], c[1], c[2]);
-  idx[i] = (uint32_t)i;
+  for (int p = 0; p < PASSES; p++) s_hist[p][threadIdx.x] = 0u;
+  {
+    float v[6];
+#pragma unroll
+    for (int c = 0; c < 6; c++) v[c] = partial[6 * threadIdx.x + c];
+    reduce6<KEY_THREADS>(v, s, s_box);
+  }
+  __syncthreads();
+  const float lo[3] = {s_box[0], s_box[1], s_box[2]};
+  // cubic cells: the longest side of the bounding box takes the 1024 steps
+  const float side = fmaxf(fmaxf(s_box[3] - lo[0], s_box[4] - lo[1]), s_box[5] - lo[2]);
+  for (int64_t i = (int64_t)blockIdx.x * KEY_THREADS + threadIdx.x; i < P; i += (int64_t)gridDim.x * KEY_THREADS) {
+    uint32_t c[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      c[k] = min(f2u_sat(((pts[3 * i + k] - lo[k]) / side) * (float)((1 << 10) - 1)), (1u << 10) - 1u);
+    const uint32_t key = hilbert30(c[0], c[1], c[2]);
+    codes[i] = key;
+    idx[i] = (uint32_t)i;
+#pragma unroll
+    for (int p = 0; p < PASSES - 1; p++) atomicAdd(&s_hist[p][(key >> (SORT_DIGIT_BITS * p)) & (RADIX - 1)], 1u);
+    atomicAdd(&s_hist[PASSES - 1][(key >> (SORT_DIGIT_BITS * (PASSES - 1))) * LAST_COPIES + threadIdx.x % LAST_COPIES],
+              1u);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < PASSES - 1; p++) {
+    const uint32_t n = s_hist[p][threadIdx.x];
+    if (n != 0u) atomicAdd(&hist[p * RADIX + threadIdx.x], n);
+  }
+  if (threadIdx.x < RADIX / LAST_COPIES) {
+    uint32_t n = 0u;
+    for (int q = 0; q < LAST_COPIES; q++) n += s_hist[PASSES - 1][threadIdx.x * LAST_COPIES + q];
+    if (n != 0u) atomicAdd(&hist[(PASSES - 1) * RADIX + threadIdx.x], n);
+  }
 }
 
 // A value moved round its row of sixteen lanes: lane i reads lane (i + 16 - N) % 16 of the row.
@@ -256,8 +285,13 @@ __global__ void __launch_bounds__(KNN_BOX) gather_boxes_kernel(int P, const floa
 // Bounding box of every run of KNN_GROUP consecutive boxes: lets the search discard that many boxes with
 // one test.  (Not in the reference, which tests every box for every point; the result is the same set of
 // three nearest neighbours, because a group's box bounds its members' boxes from below.)
+// Also hands a sort that gave up waiting on to the host (fault_word), as launch_sort_fault_report does.
 __global__ void __launch_bounds__(GS_WAVE) box_group_kernel(int nboxes, const float* __restrict__ boxes,
-                                                            float* __restrict__ groups) {
+                                                            float* __restrict__ groups,
+                                                            const uint32_t* __restrict__ sort_error,
+                                                            uint32_t* __restrict__ fault_word) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && fault_word != nullptr && *sort_error != 0u)
+    __hip_atomic_store(fault_word, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   const int b = blockIdx.x * KNN_GROUP + threadIdx.x;
   float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
   if (threadIdx.x < KNN_GROUP && b < nboxes) {
@@ -525,7 +559,6 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
   const KnnLayout L = knn_layout(P);
   char* base = (char*)temp;
   float* partial = (float*)(base + L.partial);
-  float* minmax = (float*)(base + L.minmax);
   uint32_t* codes_a = (uint32_t*)(base + L.codes_a);
   uint32_t* codes_b = (uint32_t*)(base + L.codes_b);
   uint32_t* idx_a = (uint32_t*)(base + L.idx_a);
@@ -536,37 +569,36 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
   float* leaves = (float*)(base + L.leaves);
   float* twigs = (float*)(base + L.twigs);
   void* sort_temp = base + L.sort_temp;
-  const int blocks = (P + GS_BLOCK_1D - 1) / GS_BLOCK_1D;
   const int nboxes = (P + KNN_BOX - 1) / KNN_BOX;
 
   // (the per-phase scopes only record events while stage timing is enabled)
   {
     StageScope _t("knn_minmax", stream);
-    hipLaunchKernelGGL(minmax_partial_kernel, dim3(MM_BLOCKS), dim3(MM_THREADS), 0, stream, P, points, partial);
-    hipLaunchKernelGGL(minmax_final_kernel, dim3(1), dim3(MM_THREADS), 0, stream, partial, minmax);
+    hipLaunchKernelGGL(minmax_partial_kernel, dim3(MM_BLOCKS), dim3(MM_THREADS), 0, stream, P, points, partial,
+                       sort_clear_words(P, KEY_BITS), (uint32_t*)sort_temp);
   }
   {
     StageScope _t("knn_keys", stream);
-    hipLaunchKernelGGL(curve_key_kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, P, points, minmax, codes_a, idx_a);
+    const int key_blocks = (P + KEY_THREADS - 1) / KEY_THREADS;
+    hipLaunchKernelGGL(curve_key_kernel, dim3(key_blocks < KEY_BLOCKS ? key_blocks : KEY_BLOCKS), dim3(KEY_THREADS), 0,
+                       stream, P, points, partial, codes_a, idx_a, (uint32_t*)sort_temp);
   }
-  const int end_bit = 32;  // 4 passes (even): the sorted pairs come back in the (a) arrays
   {
     StageScope _t("knn_sort", stream);
-    if (launch_sort_pairs_u32(P, codes_a, codes_b, idx_a, idx_b, end_bit, sort_temp, stream)) return 1;
-    launch_sort_fault_report(sort_error_word(sort_temp), fault_word, stream);
+    if (launch_sort_pairs_u32(P, codes_a, codes_b, idx_a, idx_b, KEY_BITS, sort_temp, stream, true)) return 1;
   }
-  const uint32_t* idx_sorted = sort_result_in_b(end_bit) ? idx_b : idx_a;
+  const uint32_t* idx_sorted = sort_result_in_b(KEY_BITS) ? idx_b : idx_a;
   {
     StageScope _t("knn_boxes", stream);
     hipLaunchKernelGGL(gather_boxes_kernel, dim3(nboxes), dim3(KNN_BOX), 0, stream, P, points, idx_sorted, sorted_pts,
                        boxes, leaves, twigs);
     hipLaunchKernelGGL(box_group_kernel, dim3((nboxes + KNN_GROUP - 1) / KNN_GROUP), dim3(GS_WAVE), 0, stream, nboxes,
-                       boxes, groups);
+                       boxes, groups, sort_error_word(sort_temp), fault_word);
   }
   {
     StageScope _t("knn_box_mean_dist", stream);
-    hipLaunchKernelGGL(box_mean_dist_kernel, dim3((P + KNN_LEAF - 1) / KNN_LEAF), dim3(GS_WAVE), 0, stream, P, sorted_pts, idx_sorted,
-                       boxes, nboxes, groups, leaves, twigs, mean_dist2);
+    hipLaunchKernelGGL(box_mean_dist_kernel, dim3((P + KNN_LEAF - 1) / KNN_LEAF), dim3(GS_WAVE), 0, stream, P, sorted_pts,
+                       idx_sorted, boxes, nboxes, groups, leaves, twigs, mean_dist2);
   }
   return 0;
 }

@@ -410,7 +410,7 @@ SortLayout sort_layout(int64_t n) {
 
 template <typename K>
 int sort_pairs_impl(int64_t n, K* keys_a, K* keys_b, uint32_t* vals_a, uint32_t* vals_b, int end_bit, void* temp,
-                    hipStream_t stream) {
+                    hipStream_t stream, bool counted = false) {
   if (n <= 0) return 0;
   if (n > sort_max_pairs()) {
     set_error("radix sort: %lld pairs exceed the supported 2^30-2", (long long)n);
@@ -428,12 +428,14 @@ int sort_pairs_impl(int64_t n, K* keys_a, K* keys_b, uint32_t* vals_a, uint32_t*
   uint32_t* error_flag = tickets + MAX_PASSES;
   uint32_t* states = ctrl + L.ctrl_words;
   uint32_t* group_states = states + (size_t)passes * L.ntiles * RADIX;
-  const int64_t clear_words = (int64_t)(L.ctrl_words + (size_t)passes * (L.ntiles + L.ngroups) * RADIX);
-  hipLaunchKernelGGL(sort_clear_kernel, dim3((unsigned)((clear_words + 255) / 256)), dim3(256), 0, stream, clear_words,
-                     ctrl);
-  const int hist_blocks = (int)((n + SORT_THREADS * HIST_ITEMS - 1) / (SORT_THREADS * HIST_ITEMS));
-  hipLaunchKernelGGL(sort_histogram_kernel<K>, dim3(hist_blocks), dim3(SORT_THREADS), 0, stream, n, keys_a, passes,
-                     end_bit, hist);
+  if (!counted) {
+    const int64_t clear_words = sort_clear_words(n, end_bit);
+    hipLaunchKernelGGL(sort_clear_kernel, dim3((unsigned)((clear_words + 255) / 256)), dim3(256), 0, stream,
+                       clear_words, ctrl);
+    const int hist_blocks = (int)((n + SORT_THREADS * HIST_ITEMS - 1) / (SORT_THREADS * HIST_ITEMS));
+    hipLaunchKernelGGL(sort_histogram_kernel<K>, dim3(hist_blocks), dim3(SORT_THREADS), 0, stream, n, keys_a, passes,
+                       end_bit, hist);
+  }
   hipLaunchKernelGGL(sort_digit_bases_kernel, dim3(passes), dim3(RADIX), 0, stream, hist);
   K* kin = keys_a;
   K* kout = keys_b;
@@ -455,6 +457,11 @@ int sort_pairs_impl(int64_t n, K* keys_a, K* keys_b, uint32_t* vals_a, uint32_t*
 }  // namespace
 
 size_t sort_temp_bytes(int64_t n) { return sort_layout(n).total_bytes; }
+
+int64_t sort_clear_words(int64_t n, int end_bit) {
+  const SortLayout L = sort_layout(n);
+  return (int64_t)(L.ctrl_words + (size_t)sort_num_passes(end_bit) * (L.ntiles + L.ngroups) * RADIX);
+}
 
 // A look-back word carries a 30-bit count beside its two flag bits, and a count can be the whole input.
 int64_t sort_max_pairs() { return (int64_t)VALUE_MASK - 1; }
@@ -483,8 +490,8 @@ int launch_sort_pairs_u64(int64_t n, uint64_t* keys_a, uint64_t* keys_b, uint32_
 }
 
 int launch_sort_pairs_u32(int64_t n, uint32_t* keys_a, uint32_t* keys_b, uint32_t* vals_a, uint32_t* vals_b,
-                          int end_bit, void* temp, hipStream_t stream) {
-  return sort_pairs_impl<uint32_t>(n, keys_a, keys_b, vals_a, vals_b, end_bit, temp, stream);
+                          int end_bit, void* temp, hipStream_t stream, bool counted) {
+  return sort_pairs_impl<uint32_t>(n, keys_a, keys_b, vals_a, vals_b, end_bit, temp, stream, counted);
 }
 
 }  // namespace gs

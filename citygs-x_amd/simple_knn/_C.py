@@ -16,7 +16,7 @@ def distCUDA2(points):
     pts = points.contiguous()
     P = pts.shape[0]
     dev = pts.device
-    out = torch.zeros(P, dtype=torch.float32, device=dev)
+    out = torch.empty(P, dtype=torch.float32, device=dev)
     if P == 0:
         return out
     nbytes = _n.lib.gs_knn_workspace_bytes(P)
