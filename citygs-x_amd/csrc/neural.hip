@@ -405,9 +405,13 @@ neural_gaussians_kernel(int64_t N, int ntiles, const float* __restrict__ anchor,
 // become the 11 pre-activation gradients of its offset's output units (zero for unselected offsets), written
 // as one record per offset; the direct gradients of offsets, scaling and anchor (xyz = anchor + offset * scaling)
 // are finished here, the per-anchor sums running over an anchor's offsets in order.
+// Bound by memory: opacity, then the anchor's first rank, then everything else is a chain of three loads, so a wave
+// takes as many anchors as fill its lanes with offsets and is done, and the records leave through LDS as runs of
+// consecutive floats.  With a wave per tile of 32 anchors, which went through the chain once per group of six
+// (5 waves per SIMD at 175 k visible anchors, and stores 44 bytes apart), it took 65 us; now 42.
 template <int K>
 __global__ void __launch_bounds__(NG_THREADS)
-neural_offset_backward_kernel(int64_t N, int ntiles, const float* __restrict__ offsets,
+neural_offset_backward_kernel(int64_t N, const float* __restrict__ offsets,
                               const float* __restrict__ scaling, const float* __restrict__ neural_opacity,
                               const float* __restrict__ opacity_scale, const float* __restrict__ opacity_tanh,
                               const uint32_t* __restrict__ first, const float* __restrict__ color_out,
@@ -419,75 +423,78 @@ neural_offset_backward_kernel(int64_t N, int ntiles, const float* __restrict__ o
                               float* __restrict__ d_scaling) {
   using S = Shape<K>;
   __shared__ float sC[NG_WAVES][64 * 9];
+  __shared__ float sG[NG_WAVES][64 * NG_SLOT_GRADS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tile = blockIdx.x * NG_WAVES + wave;
-  if (tile >= ntiles) return;  // no workgroup barrier below
+  const int64_t anchor0 = ((int64_t)blockIdx.x * NG_WAVES + wave) * S::APG;  // the wave's first anchor
+  if (anchor0 >= N) return;  // no workgroup barrier below
   float* con_s = sC[wave];
-#pragma unroll 1
-  for (int g = 0; g < S::GROUPS; g++) {
-    const int idx = g * S::APG * K + lane;
-    const int ax = idx / K, j = idx % K;
-    const int64_t sa = (int64_t)tile * NG_ANCHORS + ax;
-    const bool ok = lane < S::APG * K && ax < NG_ANCHORS && sa < N;
-    const int64_t slot = sa * K + j;
-    const float t = ok ? neural_opacity[slot] : 0.0f;
-    const bool sel = t > 0.0f;
-    const unsigned long long bits = __ballot(sel);
-    float grad[NG_SLOT_GRADS] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    float con[9] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, dof[3] = {0.0f, 0.0f, 0.0f};
-    if (sel) {
-      const int64_t r = (int64_t)first[sa] + count_lanes(bits, lane - j, lane);
-      const float* sc = scaling + sa * 6;
-      // opacity = tanh(.) * scale (scale > 0 wherever an offset is selected): d/d pre = scale * (1 - tanh^2)
-      const float ps = opacity_scale != nullptr ? opacity_scale[sa] : 1.0f;
-      const float th = opacity_scale != nullptr ? opacity_tanh[slot] : t;
-      grad[0] = g_opacity[r] * ((1.0f - th * th) * ps);
-      const float4 ax4 = *(const float4*)(aux + r * 4);
-      const float sg[3] = {ax4.x, ax4.y, ax4.z};
+  float* rec_s = sG[wave];
+  const int ax = lane / K, j = lane % K;
+  const int64_t sa = anchor0 + ax;
+  const bool ok = ax < S::APG && sa < N;
+  const int64_t slot = sa * K + j;
+  const float t = ok ? neural_opacity[slot] : 0.0f;
+  const bool sel = t > 0.0f;
+  const unsigned long long bits = __ballot(sel);
+  float grad[NG_SLOT_GRADS] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  float con[9] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, dof[3] = {0.0f, 0.0f, 0.0f};
+  if (sel) {
+    const int64_t r = (int64_t)first[sa] + count_lanes(bits, lane - j, lane);
+    const float* sc = scaling + sa * 6;
+    // opacity = tanh(.) * scale (scale > 0 wherever an offset is selected): d/d pre = scale * (1 - tanh^2)
+    const float ps = opacity_scale != nullptr ? opacity_scale[sa] : 1.0f;
+    const float th = opacity_scale != nullptr ? opacity_tanh[slot] : t;
+    grad[0] = g_opacity[r] * ((1.0f - th * th) * ps);
+    const float4 ax4 = *(const float4*)(aux + r * 4);
+    const float sg[3] = {ax4.x, ax4.y, ax4.z};
 #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const float cs = color_out[r * 3 + c];
-        grad[1 + c] = g_color[r * 3 + c] * (cs * (1.0f - cs));
-        const float gx = g_xyz[r * 3 + c], gs = g_scal[r * 3 + c];
-        con[c] = gx;
-        dof[c] = gx * sc[c];
-        con[3 + c] = gx * offsets[slot * 3 + c];
-        con[6 + c] = gs * sg[c];
-        grad[4 + c] = gs * sc[3 + c] * (sg[c] * (1.0f - sg[c]));
-      }
-      const float len = ax4.w;
-      const float4 gr = *(const float4*)(g_rot + r * 4);
-      if (len > 1e-12f) {
-        const float4 qh = *(const float4*)(rot_out + r * 4);
-        const float dot = ((qh.x * gr.x + qh.y * gr.y) + qh.z * gr.z) + qh.w * gr.w;
-        grad[7] = (gr.x - qh.x * dot) / len; grad[8] = (gr.y - qh.y * dot) / len;
-        grad[9] = (gr.z - qh.z * dot) / len; grad[10] = (gr.w - qh.w * dot) / len;
-      } else {
-        grad[7] = gr.x / 1e-12f; grad[8] = gr.y / 1e-12f; grad[9] = gr.z / 1e-12f; grad[10] = gr.w / 1e-12f;
-      }
+    for (int c = 0; c < 3; c++) {
+      const float cs = color_out[r * 3 + c];
+      grad[1 + c] = g_color[r * 3 + c] * (cs * (1.0f - cs));
+      const float gx = g_xyz[r * 3 + c], gs = g_scal[r * 3 + c];
+      con[c] = gx;
+      dof[c] = gx * sc[c];
+      con[3 + c] = gx * offsets[slot * 3 + c];
+      con[6 + c] = gs * sg[c];
+      grad[4 + c] = gs * sc[3 + c] * (sg[c] * (1.0f - sg[c]));
     }
-    if (ok) {
-#pragma unroll
-      for (int c = 0; c < NG_SLOT_GRADS; c++) slot_grads[slot * NG_SLOT_GRADS + c] = grad[c];
-#pragma unroll
-      for (int c = 0; c < 3; c++) d_offsets[slot * 3 + c] = dof[c];
+    const float len = ax4.w;
+    const float4 gr = *(const float4*)(g_rot + r * 4);
+    if (len > 1e-12f) {
+      const float4 qh = *(const float4*)(rot_out + r * 4);
+      const float dot = ((qh.x * gr.x + qh.y * gr.y) + qh.z * gr.z) + qh.w * gr.w;
+      grad[7] = (gr.x - qh.x * dot) / len; grad[8] = (gr.y - qh.y * dot) / len;
+      grad[9] = (gr.z - qh.z * dot) / len; grad[10] = (gr.w - qh.w * dot) / len;
+    } else {
+      grad[7] = gr.x / 1e-12f; grad[8] = gr.y / 1e-12f; grad[9] = gr.z / 1e-12f; grad[10] = gr.w / 1e-12f;
     }
+  }
+  if (ok) {
 #pragma unroll
-    for (int c = 0; c < 9; c++) con_s[lane * 9 + c] = con[c];
-    wave_sync();
-    for (int item = lane; item < S::APG * 9; item += 64) {
-      const int ga = item / 9, comp = item % 9;
-      const int ax2 = g * S::APG + ga;
-      const int64_t sa2 = (int64_t)tile * NG_ANCHORS + ax2;
-      if (ax2 < NG_ANCHORS && sa2 < N) {
-        float sum = 0.0f;
+    for (int c = 0; c < 3; c++) d_offsets[slot * 3 + c] = dof[c];
+  }
 #pragma unroll
-        for (int jj = 0; jj < K; jj++) sum += con_s[(ga * K + jj) * 9 + comp];
-        if (comp < 3) d_anchor[sa2 * 3 + comp] = sum;
-        else d_scaling[sa2 * 6 + (comp - 3)] = sum;
-      }
+  for (int c = 0; c < NG_SLOT_GRADS; c++) rec_s[lane * NG_SLOT_GRADS + c] = grad[c];
+#pragma unroll
+  for (int c = 0; c < 9; c++) con_s[lane * 9 + c] = con[c];
+  wave_sync();
+  const int anchors = (int)(N - anchor0 < S::APG ? N - anchor0 : S::APG);
+  const int words = anchors * (K * NG_SLOT_GRADS);
+#pragma unroll
+  for (int c = 0; c < NG_SLOT_GRADS; c++) {
+    const int e = c * 64 + lane;
+    if (e < words) slot_grads[anchor0 * (K * NG_SLOT_GRADS) + e] = rec_s[e];
+  }
+  for (int item = lane; item < S::APG * 9; item += 64) {
+    const int ga = item / 9, comp = item % 9;
+    const int64_t sa2 = anchor0 + ga;
+    if (ga < anchors) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int jj = 0; jj < K; jj++) sum += con_s[(ga * K + jj) * 9 + comp];
+      if (comp < 3) d_anchor[sa2 * 3 + comp] = sum;
+      else d_scaling[sa2 * 6 + (comp - 3)] = sum;
     }
-    wave_sync();
   }
 }
 
@@ -876,9 +883,11 @@ struct Launcher {
                        float* d_anchor, float* d_feat, float* d_offsets, float* d_scaling, float* const* d_params,
                        float* slot_grads, float* partials, hipStream_t stream) {
     const int ntiles = (int)((N + NG_ANCHORS - 1) / NG_ANCHORS);
-    hipLaunchKernelGGL(neural_offset_backward_kernel<K>, dim3((ntiles + NG_WAVES - 1) / NG_WAVES), dim3(NG_THREADS), 0,
-                       stream, N, ntiles, offsets, scaling, neural_opacity, opacity_scale, opacity_tanh, first, color_out,
-                       rot_out, aux, g_xyz, g_color, g_opacity, g_scal, g_rot, slot_grads, d_anchor, d_offsets, d_scaling);
+    const int64_t offset_block = (int64_t)S::APG * NG_WAVES;  // anchors per workgroup
+    hipLaunchKernelGGL(neural_offset_backward_kernel<K>, dim3((unsigned)((N + offset_block - 1) / offset_block)),
+                       dim3(NG_THREADS), 0, stream, N, offsets, scaling, neural_opacity, opacity_scale, opacity_tanh,
+                       first, color_out, rot_out, aux, g_xyz, g_color, g_opacity, g_scal, g_rot, slot_grads, d_anchor,
+                       d_offsets, d_scaling);
     const int nblocks = backward_blocks(N);
     hipLaunchKernelGGL(neural_mlp_backward_kernel<K>, dim3(nblocks), dim3(64 * S::BWD_WAVES), 0, stream, N, ntiles,
                        anchor, feat, level, campos, packed, slot_grads, d_anchor, d_feat, partials);
