@@ -1,7 +1,7 @@
 // Mean squared distance to the three nearest neighbours of every point
 // (simple-knn/simple_knn.cu:185-221, distCUDA2): global bounding box, a 30-bit
-// key along a space-filling curve, stable sort by key, bounding boxes of runs
-// of 1024 sorted points, then an exact search that visits only boxes closer
+// key along a space-filling curve (27-bit for few points), stable sort by key,
+// bounding boxes of runs of 1024 sorted points, then an exact search that visits only boxes closer
 // than the current third-best distance.  The search is exhaustive within that
 // bound, so the three distances equal a brute-force search whatever the order
 // of the points and whatever the visiting order.  That leaves the curve free:
@@ -29,7 +29,16 @@ constexpr int MM_BLOCKS = 512;
 constexpr int MM_THREADS = 256;
 constexpr int KEY_THREADS = 512;
 constexpr int KEY_BLOCKS = 256;  // at most: a workgroup adds its digit counts to the sort's once
-constexpr int KEY_BITS = 32;     // 4 passes (even): the sorted pairs come back where they were
+constexpr int AXIS_BITS = 10;    // of the curve
+constexpr int KEY_BITS = 3 * AXIS_BITS;
+// Few points take the curve's first nine levels, which the sort orders in three passes instead of four; points of one
+// cell then keep their input order, which the boxes do not mind until a cell holds many.  32 k points of an SfM-like
+// cloud: 106-112 -> 94-100 us a call, 5 k 100 -> 90; in 64 tight clusters of a scene a hundred times their size, the
+// worst for coarse cells, 32 k: 113-161 -> 98-152 us (ten draws each, faster in all).  Above, such clusters lose: 65 k
+// 152 -> 201 us in one draw, 200 k 214 -> 260, 1 M 1186 -> 2204.  (Six levels and two passes: 20 k 84 us in the first
+// cloud, but 50 k 145 instead of 134 us in the second.)
+constexpr int KEY_SHORT_BITS = 27;
+constexpr int KEY_SHORT_MAX = 1 << 15;
 
 struct KnnLayout {
   size_t partial, codes_a, codes_b, idx_a, idx_b, sorted_pts, boxes, groups, leaves, twigs, sort_temp, total;
@@ -149,14 +158,15 @@ __device__ __forceinline__ uint32_t hilbert30(uint32_t x, uint32_t y, uint32_t z
 
 // Every point's key, and the digit counts of the sort that follows.  17 us at 1 M points (20 with twice the workgroups);
 // as kernels of their own the keys took 9, the rest of the bounding box 4 and the counts, which read the keys again, 15.
+template <int BITS>
 __global__ void __launch_bounds__(KEY_THREADS) curve_key_kernel(int P, const float* __restrict__ pts,
                                                                 const float* __restrict__ partial,
                                                                 uint32_t* __restrict__ codes, uint32_t* __restrict__ idx,
                                                                 uint32_t* __restrict__ hist) {
-  constexpr int RADIX = 1 << SORT_DIGIT_BITS, PASSES = (KEY_BITS + SORT_DIGIT_BITS - 1) / SORT_DIGIT_BITS;
-  // the last digit has few values, which would make a wave's counts queue for the same words: sixteen counts each
-  constexpr int LAST_COPIES = 16;
-  static_assert((1 << (KEY_BITS - (PASSES - 1) * SORT_DIGIT_BITS)) * LAST_COPIES == RADIX, "fills the last row");
+  constexpr int RADIX = 1 << SORT_DIGIT_BITS, PASSES = (BITS + SORT_DIGIT_BITS - 1) / SORT_DIGIT_BITS;
+  // where the last digit has few values, which would make a wave's counts queue for the same words, they have several
+  // counts each
+  constexpr int LAST_COPIES = RADIX >> (BITS - (PASSES - 1) * SORT_DIGIT_BITS);
   static_assert(KEY_THREADS == RADIX && MM_BLOCKS == KEY_THREADS, "a thread per digit value and per partial box");
   __shared__ uint32_t s_hist[PASSES][RADIX];
   __shared__ float s[6][KEY_THREADS / GS_WAVE];
@@ -177,8 +187,9 @@ __global__ void __launch_bounds__(KEY_THREADS) curve_key_kernel(int P, const flo
     uint32_t c[3];
 #pragma unroll
     for (int k = 0; k < 3; k++)
-      c[k] = min(f2u_sat(((pts[3 * i + k] - lo[k]) / side) * (float)((1 << 10) - 1)), (1u << 10) - 1u);
-    const uint32_t key = hilbert30(c[0], c[1], c[2]);
+      c[k] = min(f2u_sat(((pts[3 * i + k] - lo[k]) / side) * (float)((1 << AXIS_BITS) - 1)),
+                 (1u << AXIS_BITS) - 1u);
+    const uint32_t key = hilbert30(c[0], c[1], c[2]) >> (3 * AXIS_BITS - BITS);
     codes[i] = key;
     idx[i] = (uint32_t)i;
 #pragma unroll
@@ -570,24 +581,26 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
   float* twigs = (float*)(base + L.twigs);
   void* sort_temp = base + L.sort_temp;
   const int nboxes = (P + KNN_BOX - 1) / KNN_BOX;
+  const int key_bits = P <= KEY_SHORT_MAX ? KEY_SHORT_BITS : KEY_BITS;
+  const auto key_kernel = P <= KEY_SHORT_MAX ? curve_key_kernel<KEY_SHORT_BITS> : curve_key_kernel<KEY_BITS>;
 
   // (the per-phase scopes only record events while stage timing is enabled)
   {
     StageScope _t("knn_minmax", stream);
     hipLaunchKernelGGL(minmax_partial_kernel, dim3(MM_BLOCKS), dim3(MM_THREADS), 0, stream, P, points, partial,
-                       sort_clear_words(P, KEY_BITS), (uint32_t*)sort_temp);
+                       sort_clear_words(P, key_bits), (uint32_t*)sort_temp);
   }
   {
     StageScope _t("knn_keys", stream);
     const int key_blocks = (P + KEY_THREADS - 1) / KEY_THREADS;
-    hipLaunchKernelGGL(curve_key_kernel, dim3(key_blocks < KEY_BLOCKS ? key_blocks : KEY_BLOCKS), dim3(KEY_THREADS), 0,
+    hipLaunchKernelGGL(key_kernel, dim3(key_blocks < KEY_BLOCKS ? key_blocks : KEY_BLOCKS), dim3(KEY_THREADS), 0,
                        stream, P, points, partial, codes_a, idx_a, (uint32_t*)sort_temp);
   }
   {
     StageScope _t("knn_sort", stream);
-    if (launch_sort_pairs_u32(P, codes_a, codes_b, idx_a, idx_b, KEY_BITS, sort_temp, stream, true)) return 1;
+    if (launch_sort_pairs_u32(P, codes_a, codes_b, idx_a, idx_b, key_bits, sort_temp, stream, true)) return 1;
   }
-  const uint32_t* idx_sorted = sort_result_in_b(KEY_BITS) ? idx_b : idx_a;
+  const uint32_t* idx_sorted = sort_result_in_b(key_bits) ? idx_b : idx_a;
   {
     StageScope _t("knn_boxes", stream);
     hipLaunchKernelGGL(gather_boxes_kernel, dim3(nboxes), dim3(KNN_BOX), 0, stream, P, points, idx_sorted, sorted_pts,

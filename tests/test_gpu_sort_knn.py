@@ -85,6 +85,20 @@ def test_knn_dist2(H, orc, P, kind):
         np.testing.assert_allclose(got, _brute(pts), rtol=2e-4, atol=1e-9)
 
 
+@pytest.mark.parametrize("P", [32_768, 32_769])
+@pytest.mark.parametrize("outlier", [False, True])
+def test_knn_dist2_where_the_sort_key_changes(H, orc, P, outlier):
+    """Up to 2^15 points are ordered by a shorter key; with an outlier many points share a cell of either grid."""
+    import simple_knn._C as knn
+    rng = np.random.default_rng(P)
+    pts = rng.normal(0, 1, (P, 3)) + rng.integers(0, 8, (P, 1)) * 30.0
+    if outlier:
+        pts[P // 2] = (4000.0, -4000.0, 4000.0)
+    pts = pts.astype(np.float32)
+    got = knn.distCUDA2(torch.from_numpy(pts).to(H.DEV)).cpu().numpy()
+    assert np.array_equal(got, orc.knn_dist2(pts))
+
+
 def _brute_f32(pts):
     """The three smallest squared distances of every point in float32 with the kernel's association,
     ((dx*dx + dy*dy) + dz*dz), and their mean ((a + b) + c) / 3: what any exact search must return, bit for bit.
