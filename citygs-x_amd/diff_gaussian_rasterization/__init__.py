@@ -61,16 +61,19 @@ class _BlendRecords:
     __slots__ = ("records", "refs", "versions", "sources", "source_versions", "all_map", "all_map_ref",
                  "all_map_version")
 
-    def __init__(self, records, all_map, parts, sources):
-        self.records = records  # (None: only the channels were formed)
-        self.all_map = all_map  # the node's channels output, until build_all_map hands it out
-        self.refs = [weakref.ref(t) for t in parts]
-        self.versions = [t._version for t in parts]
-        # means3D, scales, rotations, viewmatrix, campos as preprocess_gaussians had them
-        self.sources = [weakref.ref(t) for t in sources]
-        self.source_versions = [t._version for t in sources]
+    def __init__(self):
+        self.records = None  # (None: only the channels were formed)
+        self.all_map = None  # the node's channels output, until build_all_map hands it out
         self.all_map_ref = None
         self.all_map_version = -1
+
+    def written_from(self, parts, sources):
+        """parts: the outputs the records repeat; sources: means3D, scales, rotations, viewmatrix, campos as
+        preprocess_gaussians had them."""
+        self.refs = [weakref.ref(t) for t in parts]
+        self.versions = [t._version for t in parts]
+        self.sources = [weakref.ref(t) for t in sources]
+        self.source_versions = [t._version for t in sources]
 
     def same_sources(self, sources):
         return all(ref() is t and t._version == v for ref, v, t in zip(self.sources, self.source_versions, sources))
@@ -100,7 +103,6 @@ class _BlendRecords:
 
 
 _linked_all_map_seen = [False]  # the caller builds all_map with blend_records_of=...: records are worth starting
-_pending_blend = [None]         # from _PreprocessGaussians.forward to the wrapper that tags its outputs
 
 
 def _records_wanted(rs, P, device):
@@ -118,7 +120,7 @@ def _records_wanted(rs, P, device):
 
 class _PreprocessGaussians(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, means3D, scales, rotations, sh, opacities, raster_settings, cuda_args):
+    def forward(ctx, means3D, scales, rotations, sh, opacities, raster_settings, cuda_args, blend):
         rs = raster_settings
         # (when a backward pass can follow, the forward kernel also leaves the colours' derivative with respect to
         # the view direction, nine numbers per Gaussian, which is all the backward kernel needs the coefficients for)
@@ -132,8 +134,7 @@ class _PreprocessGaussians(torch.autograd.Function):
             rs.tanfovy, rs.image_height, rs.image_width, rs.sh_degree, rs.campos, rs.prefiltered, rs.debug, cuda_args,
             want_direction_derivative=any(ctx.needs_input_grad[:5]), want_cov3D=False, blend_records=records,
             all_map=all_map)
-        _pending_blend[0] = ((records, (means3D, scales, rotations, rs.viewmatrix, rs.campos))
-                             if records is not None or all_map is not None else None)
+        blend.records = records
         # (cov3D is None: the backward kernel forms the covariances again from scales and rotations, which it reads
         # anyway, instead of both passes moving 24 bytes per Gaussian)
         ctx.raster_settings = rs
@@ -155,7 +156,7 @@ class _PreprocessGaussians(torch.autograd.Function):
             # (only the channels were differentiated)
             dL_dmeans3D, dL_drotations = _C.build_all_map_backward(means3D, scales, rotations, rs.viewmatrix, rs.campos,
                                                                    grad_all_map)
-            return dL_dmeans3D, None, dL_drotations, None, None, None, None
+            return dL_dmeans3D, None, dL_drotations, None, None, None, None, None
         ddir = ctx.saved_tensors[7] if ctx.has_ddir else None
         P = means3D.shape[0]
         if grad_means2D is None:
@@ -171,16 +172,17 @@ class _PreprocessGaussians(torch.autograd.Function):
             dL_dall_map=grad_all_map)
         if dL_dsh.shape != sh.shape:
             dL_dsh = torch.zeros_like(sh)
-        return dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity, None, None
+        return dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity, None, None, None
 
 
 def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_settings, cuda_args):
-    _pending_blend[0] = None
-    means2D, rgb, conic_opacity, radii, depths, all_map = _PreprocessGaussians.apply(
-        means3D, scales, rotations, sh, opacities, raster_settings, cuda_args)
-    pending, _pending_blend[0] = _pending_blend[0], None
-    if pending is not None:
-        means2D._gs_blend = _BlendRecords(pending[0], all_map, (means2D, conic_opacity, rgb, depths), pending[1])
+    blend = _BlendRecords()
+    means2D, rgb, conic_opacity, radii, depths, blend.all_map = _PreprocessGaussians.apply(
+        means3D, scales, rotations, sh, opacities, raster_settings, cuda_args, blend)
+    if blend.records is not None or blend.all_map is not None:
+        blend.written_from((means2D, conic_opacity, rgb, depths),
+                           (means3D, scales, rotations, raster_settings.viewmatrix, raster_settings.campos))
+        means2D._gs_blend = blend
     return means2D, rgb, conic_opacity, radii, depths
 
 
