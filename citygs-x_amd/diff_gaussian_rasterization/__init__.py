@@ -52,24 +52,27 @@ class GaussianRasterizationSettings(NamedTuple):
 # tensors and camera preprocess_gaussians had; otherwise the library packs.  Nothing a caller sees changes: same
 # tensors, same values.
 
-# In the same way preprocess_gaussians forms the channels tensor itself, as one more output of its autograd node, once
-# a caller builds all_map through build_all_map(..., blend_records_of=means2D): that call then hands out this tensor
-# instead of launching a kernel, and the channels' gradient arrives in the backward kernel of the node, which has
-# means and rotations in registers, instead of in one of its own whose results autograd would add up.
+# In the same way preprocess_gaussians forms the channels themselves once a caller builds all_map through
+# build_all_map(..., blend_records_of=means2D): that call then hands out what the preprocess kernel left instead of
+# launching one of its own.  The autograd graph is the same with and without: build_all_map's result belongs to a node
+# of its own, with its own saved tensors, so that a loss on the channels and a loss on the image can be differentiated
+# one after the other.  Where both nodes run in one backward pass the channels' node leaves its gradient to the
+# preprocess node (_ChannelGradients), whose kernel has means and rotations in registers.
 
 class _BlendRecords:
-    __slots__ = ("records", "refs", "versions", "sources", "source_versions", "all_map", "all_map_ref",
-                 "all_map_version")
+    """What one preprocess call leaves for build_all_map and render_gaussians, beside its outputs."""
+    __slots__ = ("records", "all_map", "gradients", "refs", "versions", "sources", "source_versions",
+                 "all_map_ref", "all_map_version")
 
     def __init__(self):
-        self.records = None  # (None: only the channels were formed)
-        self.all_map = None  # the node's channels output, until build_all_map hands it out
+        self.records = None    # the blend kernels' operand records
+        self.all_map = None    # the channels, until build_all_map hands them out
+        self.gradients = None  # the node's _ChannelGradients
         self.all_map_ref = None
         self.all_map_version = -1
 
     def written_from(self, parts, sources):
-        """parts: the outputs the records repeat; sources: means3D, scales, rotations, viewmatrix, campos as
-        preprocess_gaussians had them."""
+        """parts: the outputs the records repeat; sources: means3D, scales, rotations, viewmatrix, campos."""
         self.refs = [weakref.ref(t) for t in parts]
         self.versions = [t._version for t in parts]
         self.sources = [weakref.ref(t) for t in sources]
@@ -79,16 +82,12 @@ class _BlendRecords:
         return all(ref() is t and t._version == v for ref, v, t in zip(self.sources, self.source_versions, sources))
 
     def take_all_map(self, sources):
-        """The channels preprocess_gaussians formed, if they are those of `sources` and carry the gradient the caller's
-        mode asks for; once (two callers must not share a tensor either may modify)."""
-        all_map = self.all_map
-        if all_map is None or not self.same_sources(sources):
+        """The channels preprocess_gaussians formed, if they are those of `sources`; once (two callers must not
+        share a tensor either may modify)."""
+        if self.all_map is None or not self.same_sources(sources):
             return None
-        needs_grad = torch.is_grad_enabled() and (sources[0].requires_grad or sources[2].requires_grad)
-        if needs_grad and not all_map.requires_grad:
-            return None
-        self.all_map = None
-        return all_map if needs_grad or not all_map.requires_grad else all_map.detach()
+        all_map, self.all_map = self.all_map, None
+        return all_map
 
     def usable(self, parts, all_maps, render_geo):
         if self.records is None:
@@ -102,7 +101,41 @@ class _BlendRecords:
         return True
 
 
-_linked_all_map_seen = [False]  # the caller builds all_map with blend_records_of=...: records are worth starting
+class _ChannelGradients:
+    """Carries the gradient of the channels from their node to the preprocess node, which adds what it makes of it to
+    its own results, if the preprocess node is still to run in the same backward pass and passes its gradients of
+    means and rotations on to where the channels' node would have passed them.  Everything is kept per backward pass
+    (the autograd engine numbers them): a pass that failed half way leaves nothing for another one, and passes over a
+    retained graph do not meet."""
+    __slots__ = ("node", "handed", "done")
+
+    def __init__(self, node):
+        self.node = weakref.ref(node)
+        self.handed = {}  # pass: gradient
+        self.done = set()  # passes in which the preprocess node has run
+
+    def leave(self, channels_node, grad):
+        node = self.node()
+        if node is None or torch.is_grad_enabled():  # (a graph of the backward pass is asked for)
+            return False
+        this_pass = torch._C._current_graph_task_id()
+        if this_pass < 0 or this_pass in self.done or not torch._C._will_engine_execute_node(node):
+            return False
+        here, there = channels_node.next_functions, node.next_functions
+        if here[0] != there[0] or here[2] != there[2]:
+            return False
+        self.handed[this_pass] = grad
+        return True
+
+    def take(self):
+        this_pass = torch._C._current_graph_task_id()
+        self.done.add(this_pass)
+        return self.handed.pop(this_pass, None)
+
+
+# The caller builds all_map with blend_records_of=...: records and channels are worth writing.  Only the time depends
+# on it, never a result or the graph.
+_linked_all_map_seen = [False]
 
 
 def _records_wanted(rs, P, device):
@@ -134,7 +167,8 @@ class _PreprocessGaussians(torch.autograd.Function):
             rs.tanfovy, rs.image_height, rs.image_width, rs.sh_degree, rs.campos, rs.prefiltered, rs.debug, cuda_args,
             want_direction_derivative=any(ctx.needs_input_grad[:5]), want_cov3D=False, blend_records=records,
             all_map=all_map)
-        blend.records = records
+        blend.records, blend.all_map = records, all_map
+        ctx.channel_gradients = blend.gradients = _ChannelGradients(ctx) if all_map is not None else None
         # (cov3D is None: the backward kernel forms the covariances again from scales and rotations, which it reads
         # anyway, instead of both passes moving 24 bytes per Gaussian)
         ctx.raster_settings = rs
@@ -146,17 +180,13 @@ class _PreprocessGaussians(torch.autograd.Function):
         ctx.mark_non_differentiable(radii, depths)
         # no zero tensors for the outputs nobody differentiates (radii, depths): backward fills in what it needs
         ctx.set_materialize_grads(False)
-        return means2D, rgb, conic_opacity, radii, depths, all_map
+        return means2D, rgb, conic_opacity, radii, depths
 
     @staticmethod
-    def backward(ctx, grad_means2D, grad_rgb, grad_conic_opacity, grad_radii, grad_depths, grad_all_map):
+    def backward(ctx, grad_means2D, grad_rgb, grad_conic_opacity, grad_radii, grad_depths):
         rs = ctx.raster_settings
         means3D, scales, rotations, sh, radii, cov3D, clamped = ctx.saved_tensors[:7]
-        if grad_means2D is None and grad_rgb is None and grad_conic_opacity is None and grad_all_map is not None:
-            # (only the channels were differentiated)
-            dL_dmeans3D, dL_drotations = _C.build_all_map_backward(means3D, scales, rotations, rs.viewmatrix, rs.campos,
-                                                                   grad_all_map)
-            return dL_dmeans3D, None, dL_drotations, None, None, None, None, None
+        grad_all_map = ctx.channel_gradients.take() if ctx.channel_gradients is not None else None
         ddir = ctx.saved_tensors[7] if ctx.has_ddir else None
         P = means3D.shape[0]
         if grad_means2D is None:
@@ -177,7 +207,7 @@ class _PreprocessGaussians(torch.autograd.Function):
 
 def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_settings, cuda_args):
     blend = _BlendRecords()
-    means2D, rgb, conic_opacity, radii, depths, blend.all_map = _PreprocessGaussians.apply(
+    means2D, rgb, conic_opacity, radii, depths = _PreprocessGaussians.apply(
         means3D, scales, rotations, sh, opacities, raster_settings, cuda_args, blend)
     if blend.records is not None or blend.all_map is not None:
         blend.written_from((means2D, conic_opacity, rgb, depths),
@@ -292,16 +322,21 @@ def render_gaussians(means2D, means2D_abs, conic_opacity, rgb, all_map, depths, 
 
 class _BuildAllMap(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, means3D, scales, rotations, viewmatrix, campos):
-        ctx.save_for_backward(means3D, scales, rotations, viewmatrix, campos)
-        return _C.build_all_map(means3D, scales, rotations, viewmatrix, campos)
+    def forward(ctx, means3D, scales, rotations, viewmatrix, campos, blend):
+        sources = (means3D, scales, rotations, viewmatrix, campos)
+        ctx.save_for_backward(*sources)
+        all_map = blend.take_all_map(sources) if blend is not None else None
+        ctx.gradients = blend.gradients if all_map is not None else None
+        return all_map if all_map is not None else _C.build_all_map(*sources)
 
     @staticmethod
     def backward(ctx, grad_all_map):
         means3D, scales, rotations, viewmatrix, campos = ctx.saved_tensors
+        if ctx.gradients is not None and ctx.gradients.leave(ctx, grad_all_map):
+            return (None,) * 6
         dL_dmeans3D, dL_drotations = _C.build_all_map_backward(means3D, scales, rotations, viewmatrix, campos,
                                                                grad_all_map)
-        return dL_dmeans3D, None, dL_drotations, None, None
+        return dL_dmeans3D, None, dL_drotations, None, None, None
 
 
 def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_of=None):
@@ -311,16 +346,15 @@ def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_
     blend_records_of (optional): the means2D tensor preprocess_gaussians returned for the same parameter tensors
     and camera (the settings' viewmatrix and campos tensors).  preprocess_gaussians then writes the blend kernels'
     operand records with these very channels in them (from the next view on), and render_gaussians, given these
-    very tensors, skips the pass that packs them; it also forms this tensor, whose gradient its own backward pass then
-    takes.  The returned values and the gradients are the same either way."""
+    very tensors, skips the pass that packs them; it also forms this tensor's values and, where one backward pass runs
+    through both, takes its gradient.  The returned values, the gradients and the autograd graph are the same either
+    way."""
     sources = (means3D, scales, rotations, viewmatrix, campos)
     if blend_records_of is None:
-        return _BuildAllMap.apply(*sources)
+        return _BuildAllMap.apply(*sources, None)
     _linked_all_map_seen[0] = True
     blend = getattr(blend_records_of, "_gs_blend", None)
-    all_map = blend.take_all_map(sources) if blend is not None else None
-    if all_map is None:
-        all_map = _BuildAllMap.apply(*sources)
+    all_map = _BuildAllMap.apply(*sources, blend)
     if blend is not None and blend.same_sources(sources):
         blend.all_map_ref = weakref.ref(all_map)
         blend.all_map_version = all_map._version

@@ -1,9 +1,11 @@
-"""What preprocess_gaussians leaves for build_all_map(..., blend_records_of=means2D) and render_gaussians, on the CPU with
-torch statements in place of the kernels."""
+"""The autograd graph around build_all_map(..., blend_records_of=means2D), on the CPU with torch statements in place of
+the kernels: the channels have a node and saved tensors of their own whether or not preprocess_gaussians formed them,
+and their gradient goes through the preprocess node exactly where that node runs in the same backward pass."""
 import threading
 
 import pytest
 import torch
+from torch.utils.checkpoint import checkpoint
 
 P = 7
 
@@ -82,6 +84,150 @@ def view(t, rs, linked=True):
     am = dgr.build_all_map(t["m"], t["s"], t["q"], rs.viewmatrix, rs.campos,
                            blend_records_of=means2D if linked else None)
     return means2D, co, am
+
+
+def image_loss(means2D, co):
+    return (means2D * means2D).sum() + (co * co).sum()
+
+
+def channel_loss(am):
+    return (am * am).sum()
+
+
+def grads(t):
+    return [t[k].grad for k in sorted(t)]
+
+
+def same(a, b):
+    return all((x is None) == (y is None) and (x is None or torch.equal(x, y)) for x, y in zip(a, b))
+
+
+def reference(parts):
+    """The gradients of the chosen losses with the channels as an operator of their own."""
+    t = leaves()
+    means2D, co, am = view(t, settings(), linked=False)
+    loss = 0
+    if "image" in parts:
+        loss = loss + image_loss(means2D, co)
+    if "channels" in parts:
+        loss = loss + channel_loss(am)
+    loss.backward()
+    return grads(t)
+
+
+def test_one_backward_pass_uses_the_channels_of_the_preprocess_kernel(K):
+    want = reference("image channels".split())
+    rs = settings()
+    for n in range(3):
+        t = leaves()
+        K.calls.clear()
+        means2D, co, am = view(t, rs)
+        (image_loss(means2D, co) + channel_loss(am)).backward()
+        assert same(grads(t), want), n
+        if n > 0:  # (the first view learns that the channels are wanted)
+            assert K.calls == ["preprocess", "preprocess backward with channels"]
+
+
+@pytest.mark.parametrize("order", ["channels first", "image first"])
+def test_two_losses_differentiated_one_after_the_other(K, order):
+    want = reference("image channels".split())
+    rs = settings()
+    for n in range(3):
+        t = leaves()
+        means2D, co, am = view(t, rs)
+        losses = [channel_loss(am), image_loss(means2D, co)]
+        for loss in losses if order == "channels first" else losses[::-1]:
+            loss.backward()
+        assert same(grads(t), want), n
+
+
+@pytest.mark.parametrize("parts", ["image", "channels"])
+def test_one_of_the_two_losses(K, parts):
+    want = reference([parts])
+    rs = settings()
+    for n in range(2):
+        t = leaves()
+        means2D, co, am = view(t, rs)
+        (image_loss(means2D, co) if parts == "image" else channel_loss(am)).backward()
+        assert same(grads(t), want), n
+
+
+def test_retained_graph_failed_pass_and_hooks(K):
+    rs = settings()
+    view(leaves(), rs)
+    want = reference("image channels".split())
+    t = leaves()
+    means2D, co, am = view(t, rs)
+    loss = image_loss(means2D, co) + channel_loss(am)
+    seen = []
+    am.register_hook(lambda g: seen.append(g.clone()))
+    loss.backward(retain_graph=True)
+    assert same(grads(t), want)
+    # a pass that ends between the two nodes leaves nothing behind for the next one
+    stop = means2D.register_hook(lambda g: 1 / 0)
+    with pytest.raises(ZeroDivisionError):
+        loss.backward(retain_graph=True)
+    stop.remove()
+    for x in t.values():
+        x.grad = None
+    image_loss(means2D, co).backward(retain_graph=True)
+    assert same(grads(t), reference(["image"]))
+    for x in t.values():
+        x.grad = None
+    loss.backward()
+    assert same(grads(t), want)
+    assert all(torch.equal(g, 2 * am.detach()) for g in seen) and len(seen) >= 2
+
+
+def test_gradients_of_chosen_inputs(K):
+    rs = settings()
+    view(leaves(), rs)
+    for names in (["m"], ["q"], ["s"], ["o"], ["q", "o"], ["m", "s"]):
+        got = {}
+        for linked in (False, True):
+            t = leaves()
+            means2D, co, am = view(t, rs, linked)
+            loss = image_loss(means2D, co) + channel_loss(am)
+            got[linked] = torch.autograd.grad(loss, [t[k] for k in names] + [am])
+        assert same(got[False], got[True]), names
+    # an input that has become a leaf of its own between the two calls
+    t = leaves()
+    base = t["m"]
+    t["m"] = base * 1.0
+    means2D, rgb, co, radii, depths = __import__("diff_gaussian_rasterization").preprocess_gaussians(
+        t["m"], t["s"], t["q"], t["sh"], t["o"], rs, None)
+    t["m"].detach_().requires_grad_()
+    import diff_gaussian_rasterization as dgr
+    am = dgr.build_all_map(t["m"], t["s"], t["q"], rs.viewmatrix, rs.campos, blend_records_of=means2D)
+    (image_loss(means2D, co) + channel_loss(am)).backward()
+    a, _ = K.channels_gradient(t["m"].detach(), None, t["q"].detach(), 2 * am.detach())
+    assert torch.equal(t["m"].grad, a)
+    assert torch.equal(base.grad[:, :2], 8 * base.detach()[:, :2])
+
+
+def test_checkpointed_view(K):
+    want = reference("image channels".split())
+    rs = settings()
+    for n in range(3):
+        t = leaves()
+
+        def run(*args):
+            means2D, co, am = view(dict(zip(sorted(t), args)), rs)
+            return image_loss(means2D, co) + channel_loss(am)
+
+        checkpoint(run, *[t[k] for k in sorted(t)], use_reentrant=False).backward()
+        assert same(grads(t), want), n
+
+
+def test_linked_and_unlinked_views_in_turn(K):
+    want = reference("image channels".split())
+    rs = settings()
+    for n in range(6):
+        t = leaves()
+        means2D, co, am = view(t, rs, linked=n % 3 != 1)
+        saved = len(am.grad_fn.saved_tensors)
+        (image_loss(means2D, co) + channel_loss(am)).backward()
+        assert saved == 5 and same(grads(t), want), n
 
 
 def test_views_of_several_threads_do_not_meet(K, monkeypatch):
