@@ -18,6 +18,8 @@ from typing import NamedTuple
 import torch
 import torch.nn as nn
 
+import gsrast_native as _n
+
 from . import _C
 
 __all__ = ["GaussianRasterizationSettings", "GaussianRasterizer", "preprocess_gaussians", "render_gaussians",
@@ -61,13 +63,14 @@ class GaussianRasterizationSettings(NamedTuple):
 
 class _BlendRecords:
     """What one preprocess call leaves for build_all_map and render_gaussians, beside its outputs."""
-    __slots__ = ("records", "all_map", "gradients", "refs", "versions", "sources", "source_versions",
+    __slots__ = ("records", "all_map", "gradients", "stream", "refs", "versions", "sources", "source_versions",
                  "all_map_ref", "all_map_version")
 
     def __init__(self):
         self.records = None    # the blend kernels' operand records
         self.all_map = None    # the channels, until build_all_map hands them out
         self.gradients = None  # the node's _ChannelGradients
+        self.stream = 0        # what the kernel that writes the two was launched on
         self.all_map_ref = None
         self.all_map_version = -1
 
@@ -78,19 +81,23 @@ class _BlendRecords:
         self.sources = [weakref.ref(t) for t in sources]
         self.source_versions = [t._version for t in sources]
 
+    def on_this_stream(self, device):
+        """Both tensors were allocated for the stream that writes them, and only work on it is ordered behind that."""
+        return self.stream == _n.stream_handle(device)
+
     def same_sources(self, sources):
         return all(ref() is t and t._version == v for ref, v, t in zip(self.sources, self.source_versions, sources))
 
     def take_all_map(self, sources):
-        """The channels preprocess_gaussians formed, if they are those of `sources`; once (two callers must not
-        share a tensor either may modify)."""
-        if self.all_map is None or not self.same_sources(sources):
+        """The channels preprocess_gaussians formed, if they are those of `sources` and this stream's; once (two
+        callers must not share a tensor either may modify)."""
+        if self.all_map is None or not self.same_sources(sources) or not self.on_this_stream(sources[0].device):
             return None
         all_map, self.all_map = self.all_map, None
         return all_map
 
     def usable(self, parts, all_maps, render_geo):
-        if self.records is None:
+        if self.records is None or not self.on_this_stream(parts[0].device):
             return False
         for ref, version, t in zip(self.refs, self.versions, parts):
             if ref() is not t or t._version != version:
@@ -168,6 +175,8 @@ class _PreprocessGaussians(torch.autograd.Function):
             want_direction_derivative=any(ctx.needs_input_grad[:5]), want_cov3D=False, blend_records=records,
             all_map=all_map)
         blend.records, blend.all_map = records, all_map
+        if records is not None or all_map is not None:
+            blend.stream = _n.stream_handle(means3D.device)
         ctx.channel_gradients = blend.gradients = _ChannelGradients(ctx) if all_map is not None else None
         # (cov3D is None: the backward kernel forms the covariances again from scales and rotations, which it reads
         # anyway, instead of both passes moving 24 bytes per Gaussian)
@@ -348,7 +357,7 @@ def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_
     operand records with these very channels in them (from the next view on), and render_gaussians, given these
     very tensors, skips the pass that packs them; it also forms this tensor's values and, where one backward pass runs
     through both, takes its gradient.  The returned values, the gradients and the autograd graph are the same either
-    way."""
+    way.  Both are used on the stream preprocess_gaussians ran on only."""
     sources = (means3D, scales, rotations, viewmatrix, campos)
     if blend_records_of is None:
         return _BuildAllMap.apply(*sources, None)

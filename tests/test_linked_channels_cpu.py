@@ -230,6 +230,31 @@ def test_linked_and_unlinked_views_in_turn(K):
         assert saved == 5 and same(grads(t), want), n
 
 
+def test_another_stream_gets_channels_of_its_own(K, monkeypatch):
+    """What the preprocess kernel writes belongs to the stream that kernel runs on."""
+    import diff_gaussian_rasterization as dgr
+    rs = settings()
+    view(leaves(), rs)
+    current = [11]
+    monkeypatch.setattr(dgr._n, "stream_handle", lambda device: current[0])
+    t = leaves()
+    means2D, rgb, co, radii, depths = dgr.preprocess_gaussians(t["m"], t["s"], t["q"], t["sh"], t["o"], rs, None)
+    current[0] = 12
+    K.calls.clear()
+    am = dgr.build_all_map(t["m"], t["s"], t["q"], rs.viewmatrix, rs.campos, blend_records_of=means2D)
+    assert K.calls == ["channels"]
+    (image_loss(means2D, co) + channel_loss(am)).backward()
+    assert K.calls[1:] == ["channels backward", "preprocess backward"] or \
+        K.calls[1:] == ["preprocess backward", "channels backward"]
+    blend = means2D._gs_blend
+    blend.records = torch.zeros(P, 16)
+    parts = [r() for r in blend.refs]
+    assert not blend.usable([means2D] + parts[1:], am, True)
+    current[0] = 11
+    assert dgr.build_all_map(t["m"], t["s"], t["q"], rs.viewmatrix, rs.campos, blend_records_of=means2D) is not None
+    assert K.calls.count("channels") == 1  # (handed out on its own stream)
+
+
 def test_views_of_several_threads_do_not_meet(K, monkeypatch):
     """What a preprocess call leaves goes to its own outputs, whichever thread runs in between."""
     import diff_gaussian_rasterization as dgr
