@@ -51,6 +51,13 @@ T* ptr(const Tensor& t) {
 
 gs_stream_t stream_of(uintptr_t s) { return (gs_stream_t)s; }
 
+// A tensor that a kernel reads or writes as P rows where it lies: there is no copy that would put it right.
+void check_rows(const OptTensor& t, const char* name, const Tensor& like, at::IntArrayRef shape) {
+  TORCH_CHECK(!t.has_value() || (t->scalar_type() == at::kFloat && t->sizes() == shape && t->is_contiguous() &&
+                                 t->device() == like.device()),
+              name, " must be a contiguous ", shape, " float32 tensor on the same device");
+}
+
 struct Options {
   at::TensorOptions f32, i32, u8, b8, i64;
   explicit Options(const at::Device& d)
@@ -88,8 +95,10 @@ py::tuple preprocess_forward(const Tensor& means3D_, const Tensor& scales_, cons
                              float tan_fovy, int height, int width, int degree, bool prefiltered, bool debug,
                              bool want_ddir, bool want_cov3D, const OptTensor& blend_records,
                              const OptTensor& all_map, uintptr_t stream) {
+  const int64_t P = means3D_.size(0);
+  check_rows(blend_records, "blend_records", means3D_, {P, 16});
+  check_rows(all_map, "all_map", means3D_, {P, 5});
   const Tensor means3D = f32c(means3D_, "means3D");
-  const int64_t P = means3D.size(0);
   const Options o(means3D.device());
   const c10::DeviceGuard guard(means3D.device());
   const Tensor scales = f32c(scales_, "scales"), rotations = f32c(rotations_, "rotations"),
@@ -123,11 +132,15 @@ py::tuple preprocess_backward(const Tensor& radii, const OptTensor& cov3D_, cons
                               int degree, const Tensor& campos, const Tensor& dL_dmeans2D,
                               const Tensor& dL_dconic_opacity, const OptTensor& dL_dcolors, bool debug,
                               const OptTensor& dcolor_ddir, const OptTensor& dL_dall_map, uintptr_t stream) {
+  const int64_t P = means3D_.size(0);
+  const bool sh_mode = sh.has_value() && sh->dim() == 3 && sh->size(0) == P;
+  if (sh_mode) check_rows(dcolor_ddir, "dcolor_ddir", means3D_, {P, 3, 3});  // (not used otherwise)
+  TORCH_CHECK(!dL_dall_map.has_value() || (dL_dall_map->sizes() == at::IntArrayRef({P, 5}) &&
+                                           dL_dall_map->device() == means3D_.device()),
+              "dL_dall_map must have shape [", P, ", 5] and be on the same device");
   const Tensor means3D = f32c(means3D_, "means3D");
-  const int64_t P = means3D.size(0);
   const Options o(means3D.device());
   const c10::DeviceGuard guard(means3D.device());
-  const bool sh_mode = sh.has_value() && sh->dim() == 3 && sh->size(0) == P;
   const int64_t M = sh_mode ? sh->size(1) : 0;
   Tensor dL_dsh = sh_mode ? at::empty({P, M, 3}, o.f32) : at::zeros({P, 3}, o.f32);
   Tensor dmeans = at::empty({P, 3}, o.f32), dscales = at::empty({P, 3}, o.f32), drot = at::empty({P, 4}, o.f32),
@@ -174,11 +187,7 @@ py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& m
               tiles, " elements");
   TORCH_CHECK_TYPE(!geo || all_map.has_value(), "all_map must be a tensor where geometry channels are rendered");
   const Tensor am = geo ? f32c(*all_map, "all_map") : Tensor();
-  TORCH_CHECK(!blend_records.has_value() ||
-                  (blend_records->dim() == 2 && blend_records->size(0) == P && blend_records->size(1) == 16 &&
-                   blend_records->scalar_type() == at::kFloat && blend_records->is_contiguous() &&
-                   blend_records->device() == means2D.device()),
-              "blend_records must be a contiguous (P, 16) float32 tensor on the same device");
+  check_rows(blend_records, "blend_records", means2D, {P, 16});
   Tensor color = at::empty({CHANNELS, H, W}, o.f32), observe = at::empty({P}, o.i32);
   Tensor map = geo ? at::empty({MAP_CHANNELS, H, W}, o.f32) : at::zeros({MAP_CHANNELS, H, W}, o.f32);
   Tensor depth = geo ? at::empty({1, H, W}, o.f32) : at::zeros({1, H, W}, o.f32);
@@ -220,8 +229,9 @@ py::tuple render_backward(const Tensor& background, float tan_fovx, float tan_fo
                           const OptTensor& dL_dout_all_map, const OptTensor& dL_dout_plane_depth,
                           const Tensor& means2D_, const Tensor& conic_opacity, const Tensor& rgb, bool geo, bool debug,
                           bool timing, int64_t binning_capacity, const OptTensor& blend_records, uintptr_t stream) {
+  const int64_t P = means2D_.size(0);
+  check_rows(blend_records, "blend_records", means2D_, {P, 16});
   const Tensor means2D = f32c(means2D_, "means2D");
-  const int64_t P = means2D.size(0);
   const Options o(means2D.device());
   const c10::DeviceGuard guard(means2D.device());
   const int H = (int)dL_dout_color.size(1), W = (int)dL_dout_color.size(2);

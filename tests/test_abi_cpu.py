@@ -102,3 +102,45 @@ def test_python_modules_refuse_cpu_tensors():
         rast.preprocess_gaussians(z(4, 3), z(4, 3), z(4, 4), z(4, 3), z(4, 1), {})
     with pytest.raises(RuntimeError, match="no CPU path"):
         distCUDA2(z(10, 3))
+
+
+def test_tensors_the_kernels_use_in_place_are_checked():
+    """What preprocess and render read or write without a copy of their own is refused unless it has the rows the
+    kernels address; looked at before anything else, so the refusal is seen without a GPU."""
+    import pytest
+    import torch
+    import gsrast_native as gn
+    P = 6
+    z = torch.zeros
+    cam = (z(4, 4), z(4, 4))
+
+    def forward(records=None, all_map=None):
+        gn.ops.preprocess_forward(z(P, 3), z(P, 3), z(P, 4), None, z(P, 1), 1.0, *cam, z(3), 0.5, 0.5, 32, 32, 0, False,
+                                  False, False, False, records, all_map, 0)
+
+    def backward(ddir=None, gmap=None):
+        gn.ops.preprocess_backward(z(P, dtype=torch.int32), None, z(P, 3, dtype=torch.bool), z(P, 3), z(P, 3), z(P, 4),
+                                   z(P, 16, 3), 1.0, *cam, 0.5, 0.5, 32, 32, 0, z(3), z(P, 2), z(P, 4), None, False, ddir,
+                                   gmap, 0)
+
+    def render_backward(records):
+        u8 = z(16, dtype=torch.uint8)
+        gn.ops.render_backward(z(3), 0.5, 0.5, None, None, 0, u8, u8, u8, z(4, dtype=torch.bool), z(3, 32, 32), None,
+                               None, z(P, 2), z(P, 4), z(P, 3), False, False, False, 0, records, 0)
+
+    for call, name, shape in ((lambda t: forward(records=t), "blend_records", (P, 16)),
+                              (lambda t: forward(all_map=t), "all_map", (P, 5)),
+                              (lambda t: backward(ddir=t), "dcolor_ddir", (P, 3, 3)),
+                              (render_backward, "blend_records", (P, 16))):
+        short = z(P - 1, *shape[1:])
+        strided = z(*shape[:-1], 2 * shape[-1])[..., ::2]
+        for bad in (short, strided, z(*shape, dtype=torch.float64), z(*shape, device="meta"), z(P * 16)):
+            with pytest.raises(RuntimeError, match=f"{name} must be a contiguous"):
+                call(bad)
+        with pytest.raises(RuntimeError, match="no CPU path"):
+            call(z(*shape))
+    for bad in (z(P - 1, 5), z(P, 4), z(P, 5, device="meta")):
+        with pytest.raises(RuntimeError, match="dL_dall_map must have shape"):
+            backward(gmap=bad)
+    with pytest.raises(RuntimeError, match="no CPU path"):
+        backward(gmap=z(P, 10)[:, ::2])  # (made contiguous by the call)
