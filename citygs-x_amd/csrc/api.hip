@@ -1426,6 +1426,12 @@ int gs_selftest_reductions(const float* in, float* out_wave, float* out_rows, gs
   return check_launch("selftest_reductions", (hipStream_t)stream, true);
 }
 
+int gs_selftest_quads(const float* in, float* out, gs_stream_t stream) {
+  GS_REQUIRE(in && out, "gs_selftest_quads: null pointer");
+  launch_quad_selftest(in, out, (hipStream_t)stream);
+  return check_launch("selftest_quads", (hipStream_t)stream, true);
+}
+
 int gs_stage_timing_enable(int enable) {
   g_clock.enabled.store(enable != 0);
   return 0;

@@ -1,6 +1,6 @@
 // Pieces shared by the forward and backward tile kernels: the pixel layout of a
 // workgroup, the conservative test that culls Gaussians per 4x4 pixel block, and
-// the reductions of 16 values over a wave and over a 16-lane row.
+// the cross-lane steps of the backward kernel's sums over pixels.
 #pragma once
 
 #include "gs_common.h"
@@ -94,36 +94,6 @@ __device__ __forceinline__ void ellipse_hits_quadrant(float2 mu, float4 co, floa
   }
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_row_add(float v) {
-  const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false);
-  return v + __int_as_float(moved);
-}
-
-// Sums 16 per-lane values over the 64 lanes of a wave in 40 operations.
-//   level 1: v_permlane32_swap pairs value k with k+8: the low 32 lanes keep k, the high 32 lanes k+8;
-//   level 2: v_permlane16_swap pairs k with k+4: each 16-lane row keeps one value;
-//   level 3: four DPP adds (quad swaps, row rotations) finish the sum inside each row.
-// On return every lane of row r (lanes 16r..16r+15) of out[k] holds the total of value k + 4r.
-__device__ __forceinline__ void wave_reduce16(const float* v, float* out) {
-  float h[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]), __float_as_uint(v[k + 8]), false, false);
-    h[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[k]), __float_as_uint(h[k + 4]), false, false);
-    float s = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    s = dpp_row_add<0xB1>(s);   // quad_perm [1,0,3,2]
-    s = dpp_row_add<0x4E>(s);   // quad_perm [2,3,0,1]
-    s = dpp_row_add<0x124>(s);  // row_ror:4
-    s = dpp_row_add<0x128>(s);  // row_ror:8
-    out[k] = s;
-  }
-}
-
 // ---- 4x4-pixel rows -------------------------------------------------------
 // Inside a wave's 8x8 quadrant every 16-lane DPP row owns a 4x4 pixel block
 // (row r at x offset 4*(r&1), y offset 4*(r>>1); lane l16 of the row is pixel
@@ -152,41 +122,94 @@ __device__ __forceinline__ RowThread row_thread(uint32_t tile_x, uint32_t tile_y
   return t;
 }
 
-// Transposing reduction inside every 16-lane row: on entry each lane holds 16
-// values, on return lane l16 of a row holds the sum over the row's 16 lanes of
-// value number l16.  Four halving steps (distances 8, 4, 2, 1): at each step a
-// lane keeps half of its values and adds the partner lane's copy of them, so
-// 8 + 4 + 2 + 1 lane-pair sums replace 16 x 4.  Written as DPP additions whose
-// bank mask selects which lanes of a row take the result, two instructions per
-// kept value in the first two steps (33 VALU instructions in all); v[0..7] are
-// overwritten.  All 64 lanes must be active.
-__device__ __forceinline__ float row_transpose_reduce16(float* v) {
-  const uint64_t bit1_lanes = 0xCCCCCCCCCCCCCCCCull, bit0_lanes = 0xAAAAAAAAAAAAAAAAull;
-  // A DPP operand written by the preceding VALU instruction needs two idle issue slots first; the s_nop 1
-  // between the steps provide them, inside a step no instruction reads a register written less than two
-  // instructions earlier through DPP.
+// ---- quads ----------------------------------------------------------------
+// In the backward blend's second half a quad of lanes works for four entries and its registers for four pixels.
+
+// Transposes the 4x4 blocks of a and b inside every quad: register e of lane p becomes register p of lane e.  A DPP
+// operand written by the preceding VALU instruction needs two idle issue slots first, a matrix instruction one.
+__device__ __forceinline__ void quad_transpose2(float (&a)[4], float (&b)[4]) {
+  const uint64_t bit0 = 0xAAAAAAAAAAAAAAAAull, bit1 = 0xCCCCCCCCCCCCCCCCull;
+  float c[4], d[4];
   asm volatile(
       "s_nop 1\n\t"
-      // distance 8: lanes 0-7 of a row keep values 0-7, lanes 8-15 keep values 8-15
-      "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %4, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %5, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "v_add_f32_dpp %7, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "s_mov_b64 vcc, %16\n\t"
+      "v_cndmask_b32_dpp %1, %8, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %10, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %12, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %14, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %0, %9, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %2, %11, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %4, %13, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %15, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      : "=&v"(c[0]), "=&v"(c[1]), "=&v"(c[2]), "=&v"(c[3]), "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "s"(bit0)
+      : "vcc", "scc");
+  asm volatile(
       "s_nop 1\n\t"
-      // distance 4: lanes with bit 2 clear (banks 0, 2) keep registers 0-3 and add lane +4's copy,
-      // the others keep registers 4-7 and add lane -4's copy
+      "s_mov_b64 vcc, %16\n\t"
+      "v_cndmask_b32_dpp %2, %8, %10, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %9, %11, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %12, %14, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %13, %15, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %0, %10, %8, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %1, %11, %9, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %4, %14, %12, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %15, %13, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3])
+      : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "s"(bit1)
+      : "vcc", "scc");
+}
+
+// Sums sixteen values over the four quads of every 16-lane row and leaves values 4 q .. 4 q + 3 in quad q, in v[0..3]
+// (v is overwritten).  Two halving steps, two instructions per value kept: the bank mask of a DPP addition selects the
+// quads that take its result.  Results are written before the last operands are read, so no operand may share a result's
+// register, whatever its value.  The matrix results among the inputs need up to seven idle slots first.  LAST = false:
+// v[12..15] are not given, and quad 3 ends up with no meaningful sums.
+template <bool LAST>
+__device__ __forceinline__ void quads_reduce16(float (&v)[16]) {
+  if (LAST)
+    asm volatile(
+        "s_nop 7\n\t"
+        "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %4, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %5, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %6, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %7, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        : "+&v"(v[0]), "+&v"(v[1]), "+&v"(v[2]), "+&v"(v[3]), "+&v"(v[4]), "+&v"(v[5]), "+&v"(v[6]), "+&v"(v[7])
+        : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]));
+  else
+    asm volatile(
+        "s_nop 7\n\t"
+        "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %5, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %6, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %7, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32_dpp %0, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %1, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %2, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %3, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        : "+&v"(v[0]), "+&v"(v[1]), "+&v"(v[2]), "+&v"(v[3]), "+&v"(v[4]), "+&v"(v[5]), "+&v"(v[6]), "+&v"(v[7])
+        : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]));
+  asm volatile(
+      "s_nop 1\n\t"
       "v_add_f32_dpp %0, %0, %0 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
       "v_add_f32_dpp %1, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
       "v_add_f32_dpp %2, %2, %2 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
@@ -195,24 +218,8 @@ __device__ __forceinline__ float row_transpose_reduce16(float* v) {
       "v_add_f32_dpp %1, %5, %5 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
       "v_add_f32_dpp %2, %6, %6 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
       "v_add_f32_dpp %3, %7, %7 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
-      "s_nop 1\n\t"
-      // distance 2: + lane^2; lanes with bit 1 set keep registers 2, 3
-      "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %3, %3, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_e64 %0, %0, %2, %16\n\t"
-      "v_cndmask_b32_e64 %1, %1, %3, %16\n\t"
-      "s_nop 1\n\t"
-      // distance 1: + lane^1; lanes with bit 0 set keep register 1
-      "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_add_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "s_nop 0\n\t"
-      "v_cndmask_b32_e64 %0, %0, %1, %17\n\t"
-      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
-      : "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]), "v"(v[15]),
-        "s"(bit1_lanes), "s"(bit0_lanes));
-  return v[0];
+      : "+&v"(v[0]), "+&v"(v[1]), "+&v"(v[2]), "+&v"(v[3])
+      : "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
 }
 
 }  // namespace gs

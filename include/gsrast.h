@@ -490,12 +490,15 @@ int gs_render_tiles_backward(int P, int width, int height, float tan_fovx, float
                              float* instance_grads, float* dL_dmean2D, float* dL_dmean2D_abs,
                              float* dL_dconic_opacity, float* dL_dcolor, float* dL_dall_map, gs_stream_t stream);
 
-/* A test hook, not part of the path (no counterpart in the reference, nothing in the library calls it; it is
- * exported so that the test suite can check the inline-assembly reductions on their own): runs the two cross-lane
- * reductions of the blend kernels on one 64-lane wave.  in is (64,16) floats;
- * out_wave (16) receives the sums over all 64 lanes, out_rows (4,16) the sums
- * over each 16-lane row.  Synchronises the stream. */
+/* Test hooks, not part of the path (no counterpart in the reference, nothing in the library calls them; they are
+ * exported so that the test suite can check the inline assembly of the blend kernels on its own).  Both run one
+ * 64-lane wave on in, (64,16) floats, and synchronise the stream.
+ * gs_selftest_reductions: out_wave (16) receives the sums over all 64 lanes, out_rows (4,16) the sums over each
+ * 16-lane row, formed by the cross-lane steps of the backward blend.
+ * gs_selftest_quads: out (64,24) receives the results of those steps one by one (quad_selftest_kernel in
+ * csrc/selftest.hip lists them). */
 int gs_selftest_reductions(const float* in, float* out_wave, float* out_rows, gs_stream_t stream);
+int gs_selftest_quads(const float* in, float* out, gs_stream_t stream);
 
 /* Optional per-stage GPU timing, the role of the reference's MyTimerOnGPU
  * (CR/timers.cu:11-79; stage names at CR/rasterizer_impl.cu:385-752): while

@@ -157,6 +157,27 @@ def test_cross_lane_reductions(H):
     assert np.array_equal(orow.cpu().numpy(), x.reshape(4, 16, 16).sum(1))
 
 
+def test_quad_steps_of_the_backward_blend(H):
+    """Transposition inside quads, the halving sums over a row's quads (with and without the last four values, and with
+    operands of equal value) and the lane layout of the 4x4 outer product, each against what its comment states."""
+    rng = np.random.default_rng(1)
+    x = rng.integers(-50, 51, (64, 16)).astype(np.float32)
+    out = torch.zeros(64, 24, device=H.DEV)
+    H.gn.check(H.lib.gs_selftest_quads(H.ptr(H.dev(x)), H.ptr(out), H.stream()), "selftest")
+    got = out.cpu().numpy().reshape(4, 4, 4, 24)  # row, quad, lane of the quad
+    q = x.reshape(4, 4, 4, 16)
+    assert np.array_equal(got[..., 0:4], q[..., 0:4].transpose(0, 1, 3, 2))
+    assert np.array_equal(got[..., 4:8], q[..., 4:8].transpose(0, 1, 3, 2))
+
+    def over_quads(v):  # value 4 k + r of lane e, summed over the quads, in register r of quad k
+        return v.sum(1).reshape(4, 4, 4, 4).transpose(0, 2, 1, 3)
+
+    assert np.array_equal(got[..., 8:12], over_quads(q))
+    assert np.array_equal(got[:, :3, :, 12:16], over_quads(q)[:, :3])
+    assert np.array_equal(got[..., 16:20], over_quads(np.concatenate([q[..., :8], q[..., :8]], -1)))
+    assert np.array_equal(got[..., 20:24], q[..., 1][..., None] * q[..., 0][:, :, None, :])
+
+
 def test_a_sort_that_gave_up_fails_the_next_call(H):
     """The radix sort's bounded wait is never made to run out on the GPU; instead the error word it would leave in
     its workspace is written by hand, and the plumbing behind it is followed: gs_sort_status reports it, the check
