@@ -221,6 +221,17 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
       for (int p = 0; p < 4; p++) grad_t[h][p] = t[p];
     }
   }
+  // Does a pixel of the wave have an upstream gradient that is not finite?  It belongs to the Gaussians the pixel
+  // blended; the others' weight 0 would make a NaN of it in the sums.
+  bool odd = false;
+  {
+    float top = 0.f;  // (0 x is 0 for every finite x)
+#pragma unroll
+    for (int ch = 0; ch < GS_N_RGB; ch++) top += 0.f * gpix[ch];
+#pragma unroll
+    for (int ch = 0; ch < GS_N_MAP; ch++) top += 0.f * gmap[ch];
+    odd = gs_ballot(top != 0.f) != 0ull;
+  }
 
   // thread tid hands over components 4*part .. 4*part+3 of the sub-batch's slot tid / 4 and clears them
   const int my_slot = tid >> 2, my_part = tid & 3;
@@ -487,10 +498,30 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // per Gaussian by the reduction kernel.)
         quad_transpose2(w, q);
         f32x4 c_lo = {0.f, 0.f, 0.f, 0.f}, c_hi = {0.f, 0.f, 0.f, 0.f};  // sum_p w g: registers = channels
+        if (__builtin_expect(!odd, 1)) {
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
-          c_lo = __builtin_amdgcn_mfma_f32_4x4x1f32(grad_t[0][p], w[p], c_lo, 0, 0, 0);
-          if (render_geo) c_hi = __builtin_amdgcn_mfma_f32_4x4x1f32(grad_t[RENDER_GEO ? 1 : 0][p], w[p], c_hi, 0, 0, 0);
+          for (int p = 0; p < 4; p++) {
+            c_lo = __builtin_amdgcn_mfma_f32_4x4x1f32(grad_t[0][p], w[p], c_lo, 0, 0, 0);
+            if (render_geo) c_hi = __builtin_amdgcn_mfma_f32_4x4x1f32(grad_t[RENDER_GEO ? 1 : 0][p], w[p], c_hi, 0, 0, 0);
+          }
+        } else {
+          // the same chains of multiply-adds, of the pixels that blended the entry (whose weights are not zero)
+          auto channel = [&](auto ch_tag, const float (&g)[4], f32x4& c) {
+            constexpr int ch = decltype(ch_tag)::value;
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+              const float sum = __builtin_fmaf(quad_lane<ch>(g[p]), w[p], c[ch]);
+              c[ch] = w[p] != 0.f ? sum : c[ch];
+            }
+          };
+          auto channels = [&](const float (&g)[4], f32x4& c) {
+            channel(std::integral_constant<int, 0>{}, g, c);
+            channel(std::integral_constant<int, 1>{}, g, c);
+            channel(std::integral_constant<int, 2>{}, g, c);
+            channel(std::integral_constant<int, 3>{}, g, c);
+          };
+          channels(grad_t[0], c_lo);
+          if (render_geo) channels(grad_t[RENDER_GEO ? 1 : 0], c_hi);
         }
         const float dx = xyf.x - pfx, a_dx = co.x * dx, b_dx = co.y * dx;
         float dy[4], q_dy[4], ax = 0.f, ay = 0.f;
