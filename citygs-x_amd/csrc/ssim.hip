@@ -17,8 +17,9 @@
 //   dL/dx = conv(d_mu) + 2 x conv(d_xx) + y conv(d_xy) + g_l1 * mask * sign(x - y).
 // 20 bytes per pixel and channel forward (+12 for the derivative maps), 36 backward.
 // The block is as tall as wide because the horizontal pass also runs over the ten rows of halo: with 16 rows it was
-// half of the taps.  Three channels of 1152x864: 36.6 us forward and 27.5 backward with 32x16 blocks and six
-// divisions per pixel, 33.8 and 24.3 now.
+// half of the taps.  Three channels of 1152x864: 36.6 us forward and 27.5 backward with 32x16 blocks,
+// 37 and 25 now.  (Reciprocals and products instead of the divisions: 34 forward, and SSIM of an image with itself a unit
+// in the last place off 1 in two pixels of five.)
 #include "gs_common.h"
 #include "gs_kernels.h"
 
@@ -147,19 +148,18 @@ ssim_l1_fwd_kernel(int H, int W, const float* __restrict__ img1, const float* __
     const float mu1_sq = mu1 * mu1, mu2_sq = mu2 * mu2, mu12 = mu1 * mu2;
     const float s1 = st[2] - mu1_sq, s2 = st[3] - mu2_sq, s12 = st[4] - mu12;
     const float A1 = 2 * mu12 + C1, A2 = 2 * s12 + C2, B1 = (mu1_sq + mu2_sq) + C1, B2 = (s1 + s2) + C2;
-    // (two divisions instead of six, each of a dozen instructions: the products add a unit in the last place to values
-    // that the variances' cancellation has left some hundred units off)
-    const float r1 = 1.0f / B1, r2 = 1.0f / B2, r12 = r1 * r2;
-    const float S = (A1 * A2) * r12;
+    // (correctly rounded quotients, not products with reciprocals: where the images agree numerator and denominator are
+    // the same number and SSIM is 1)
+    const float S = (A1 * A2) / (B1 * B2);
     const float mk = mask ? (float)(mask[(size_t)y * W + x] != 0) : 1.0f;
     const size_t oidx = plane + (size_t)y * W + x;
     const float p = s_a[ty + o + SR][tx + SR], q = s_b[ty + o + SR][tx + SR];
     ssim_map[oidx] = S * mk;
     l1_map[oidx] = fabsf(p - q) * mk;
     if (d_mu != nullptr) {
-      d_mu[oidx] = mk * ((2 * mu2 * (A2 - A1)) * r12 - S * (2 * mu1 * r1) + S * (2 * mu1 * r2));
-      d_xx[oidx] = mk * (-S * r2);
-      d_xy[oidx] = mk * (2 * A1 * r12);
+      d_mu[oidx] = mk * ((2 * mu2 * (A2 - A1)) / (B1 * B2) - S * (2 * mu1 / B1) + S * (2 * mu1 / B2));
+      d_xx[oidx] = mk * (-S / B2);
+      d_xy[oidx] = mk * (2 * A1 / (B1 * B2));
     }
   }
 }

@@ -76,6 +76,15 @@ def test_training_resolution_against_torch_statements():
     assert torch.equal(gs_loss.pixelwise_ssim_with_mask(a, b, mask), ss.detach())
 
 
+@pytest.mark.parametrize("H,W,scale", [(130, 171, 1.0), (16, 33, 255.0), (5, 7, 1e-3)])
+def test_an_image_against_itself(H, W, scale):
+    """Numerator and denominator are the same numbers in every pixel: their quotient is 1, with nothing to round."""
+    from gs_loss import pixelwise_l1_ssim_with_mask
+    a = (_images(3, H, W, seed=H)[0] * scale).to(DEV)
+    l1, ss = pixelwise_l1_ssim_with_mask(a.clone().requires_grad_(True), a, None)
+    assert torch.equal(ss, torch.ones_like(a)) and torch.equal(l1, torch.zeros_like(a))
+
+
 def test_rejects_cpu_and_mismatched_inputs():
     import gs_loss
     with pytest.raises(RuntimeError):
