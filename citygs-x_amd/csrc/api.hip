@@ -1426,6 +1426,14 @@ int gs_selftest_reductions(const float* in, float* out_wave, float* out_rows, gs
   return check_launch("selftest_reductions", (hipStream_t)stream, true);
 }
 
+int gs_selftest_reciprocal(uint32_t first, uint32_t n, uint32_t* out, gs_stream_t stream) {
+  GS_REQUIRE(out, "gs_selftest_reciprocal: null pointer");
+  GS_REQUIRE(n <= 0x10000000u, "gs_selftest_reciprocal: at most 2^28 floats at a time");
+  if (n == 0) return 0;
+  launch_reciprocal_selftest(first, n, out, (hipStream_t)stream);
+  return check_launch("selftest_reciprocal", (hipStream_t)stream, true);
+}
+
 int gs_selftest_quads(const float* in, float* out, gs_stream_t stream) {
   GS_REQUIRE(in && out, "gs_selftest_quads: null pointer");
   launch_quad_selftest(in, out, (hipStream_t)stream);

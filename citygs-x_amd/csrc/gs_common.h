@@ -173,7 +173,9 @@ __device__ __forceinline__ float gs_expf_core(float x) {
 }
 
 // 1.0f / d for d in [2^-7, 1]: the hardware's approximation and one Newton step, which gives the correctly rounded
-// reciprocal of every float in that range (compared with the IEEE division one by one).
+// reciprocal of every float in that range.  (That rests on the approximation: correctly rounded itself it would always
+// be enough, a unit in the last place off for all but a few hundred of the floats.  gs_selftest_reciprocal compares all
+// 58720257 of them with the division.)
 __device__ __forceinline__ float gs_rcp_normal(float d) {
   const float r0 = __builtin_amdgcn_rcpf(d);
   return __builtin_fmaf(__builtin_fmaf(-d, r0, 1.0f), r0, r0);

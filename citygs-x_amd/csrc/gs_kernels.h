@@ -294,6 +294,7 @@ struct RenderBwdArgs {
 int launch_render_bwd(const RenderBwdArgs& a, hipStream_t stream);
 
 int launch_reduce_selftest(const float* in, float* out_wave, float* out_rows, hipStream_t stream);
+int launch_reciprocal_selftest(uint32_t first, uint32_t n, uint32_t* out, hipStream_t stream);
 int launch_quad_selftest(const float* in, float* out, hipStream_t stream);
 
 // ---- k-nearest-neighbour mean squared distance ----

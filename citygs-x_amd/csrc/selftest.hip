@@ -1,5 +1,5 @@
 // Device self-tests of what the blend kernels build on and no result of theirs shows on its own: the cross-lane steps
-// in inline assembly.
+// in inline assembly, and the reciprocal, whose rounding rests on the hardware's approximation.
 #include "gs_common.h"
 #include "gs_kernels.h"
 #include "render_common.h"
@@ -75,10 +75,28 @@ __global__ void __launch_bounds__(GS_WAVE) quad_selftest_kernel(const float* __r
   for (int k = 0; k < 4; k++) o[20 + k] = d[k];
 }
 
+// gs_rcp_normal against the division on the floats whose bits are first, first + 1, ...: out[0] counts those it
+// rounds differently, out[1] is the largest of them.
+__global__ void __launch_bounds__(GS_BLOCK_1D) reciprocal_selftest_kernel(uint32_t first, uint32_t n,
+                                                                          uint32_t* __restrict__ out) {
+  for (uint32_t i = blockIdx.x * GS_BLOCK_1D + threadIdx.x; i < n; i += gridDim.x * GS_BLOCK_1D) {
+    const float d = __uint_as_float(first + i);
+    if (__float_as_uint(gs_rcp_normal(d)) != __float_as_uint(1.0f / d)) {
+      atomicAdd(&out[0], 1u);
+      atomicMax(&out[1], first + i);
+    }
+  }
+}
+
 }  // namespace
 
 int launch_reduce_selftest(const float* in, float* out_wave, float* out_rows, hipStream_t stream) {
   hipLaunchKernelGGL(reduce_selftest_kernel, dim3(1), dim3(GS_WAVE), 0, stream, in, out_wave, out_rows);
+  return 0;
+}
+
+int launch_reciprocal_selftest(uint32_t first, uint32_t n, uint32_t* out, hipStream_t stream) {
+  hipLaunchKernelGGL(reciprocal_selftest_kernel, dim3(2048), dim3(GS_BLOCK_1D), 0, stream, first, n, out);
   return 0;
 }
 

@@ -491,14 +491,17 @@ int gs_render_tiles_backward(int P, int width, int height, float tan_fovx, float
                              float* dL_dconic_opacity, float* dL_dcolor, float* dL_dall_map, gs_stream_t stream);
 
 /* Test hooks, not part of the path (no counterpart in the reference, nothing in the library calls them; they are
- * exported so that the test suite can check the inline assembly of the blend kernels on its own).  Both run one
- * 64-lane wave on in, (64,16) floats, and synchronise the stream.
+ * exported so that the test suite can check what the blend kernels build on by itself).  They synchronise the stream;
+ * the first two run one 64-lane wave on in, (64,16) floats.
  * gs_selftest_reductions: out_wave (16) receives the sums over all 64 lanes, out_rows (4,16) the sums over each
  * 16-lane row, formed by the cross-lane steps of the backward blend.
  * gs_selftest_quads: out (64,24) receives the results of those steps one by one (quad_selftest_kernel in
- * csrc/selftest.hip lists them). */
+ * csrc/selftest.hip lists them).
+ * gs_selftest_reciprocal: the backward blend's reciprocal against the division on the n floats whose bits are first,
+ * first + 1, ...; out (two words, cleared by the caller): how many differ, and the bits of the largest that does. */
 int gs_selftest_reductions(const float* in, float* out_wave, float* out_rows, gs_stream_t stream);
 int gs_selftest_quads(const float* in, float* out, gs_stream_t stream);
+int gs_selftest_reciprocal(uint32_t first, uint32_t n, uint32_t* out, gs_stream_t stream);
 
 /* Optional per-stage GPU timing, the role of the reference's MyTimerOnGPU
  * (CR/timers.cu:11-79; stage names at CR/rasterizer_impl.cu:385-752): while

@@ -178,6 +178,14 @@ def test_quad_steps_of_the_backward_blend(H):
     assert np.array_equal(got[..., 20:24], q[..., 1][..., None] * q[..., 0][:, :, None, :])
 
 
+def test_reciprocal_of_the_backward_blend(H):
+    """The bits of the division for every float in [2^-7, 1], the range 1 - alpha lies in (alpha is at most 0.99)."""
+    first, last = (int(np.float32(v).view(np.uint32)) for v in (2.0 ** -7, 1.0))
+    out = torch.zeros(2, dtype=torch.int32, device=H.DEV)
+    H.gn.check(H.lib.gs_selftest_reciprocal(first, last - first + 1, H.ptr(out), H.stream()), "selftest")
+    assert out[0] == 0, (int(out[0]), hex(int(out[1])))
+
+
 def test_a_sort_that_gave_up_fails_the_next_call(H):
     """The radix sort's bounded wait is never made to run out on the GPU; instead the error word it would leave in
     its workspace is written by hand, and the plumbing behind it is followed: gs_sort_status reports it, the check
