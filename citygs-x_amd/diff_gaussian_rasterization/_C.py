@@ -12,7 +12,7 @@ import torch
 
 import gsrast_native as _n
 
-_lib = _n.lib
+_lib, _ops = _n.lib, _n.ops
 BLOCK_X, BLOCK_Y, ONE_DIM_BLOCK_SIZE = 16, 16, 256
 NUM_CHANNELS, NUM_ALL_MAP = 3, 5
 
@@ -107,7 +107,7 @@ def preprocess_gaussians_ex(means3D, scales, rotations, sh, opacity, scale_modif
         return ((0, torch.zeros(0, 2, **f32), torch.zeros(0, **f32), torch.zeros(0, dtype=torch.int32, device=dev),
                  torch.zeros(0, 6, **f32), torch.zeros(0, 4, **f32), torch.zeros(0, 3, **f32),
                  torch.zeros(0, 3, dtype=torch.bool, device=dev)), None)
-    means2D, depths, radii, cov3D, conic_opacity, rgb, clamped, ddir = _n.ops.preprocess_forward(
+    means2D, depths, radii, cov3D, conic_opacity, rgb, clamped, ddir = _ops.preprocess_forward(
         means3D, scales, rotations, sh, opacity, float(scale_modifier), viewmatrix, projmatrix, campos, float(tan_fovx),
         float(tan_fovy), int(image_height), int(image_width), int(degree), bool(prefiltered), bool(debug),
         want_direction_derivative, want_cov3D, blend_records, all_map, _n.stream_handle(dev))
@@ -129,7 +129,7 @@ def preprocess_gaussians_backward(radii, cov3D, clamped, means3D, scales, rotati
         dL_dsh = torch.empty(0, sh.shape[1], 3, **f32) if sh_mode else torch.zeros(0, 3, **f32)
         return (torch.zeros(0, 3, **f32), torch.zeros(0, 3, **f32), torch.zeros(0, 4, **f32), dL_dsh,
                 torch.zeros(0, 1, **f32))
-    return _n.ops.preprocess_backward(
+    return _ops.preprocess_backward(
         radii, cov3D, clamped, means3D, scales, rotations, sh, float(scale_modifier), viewmatrix, projmatrix,
         float(tan_fovx), float(tan_fovy), int(image_height), int(image_width), int(degree), campos, dL_dmeans2D,
         dL_dconic_opacity, dL_dcolors, bool(debug), dcolor_ddir, dL_dall_map, _n.stream_handle(dev))
@@ -228,7 +228,7 @@ def render_gaussians_ex(background, image_height, image_width, means2D, depths, 
     focal_y = np.float32(H) / (np.float32(2.0) * np.float32(tan_fovy))
     focal_x = np.float32(W) / (np.float32(2.0) * np.float32(tan_fovx))
     (num_rendered, out_color, n_render, n_consider, n_contrib, out_observe, out_all_map, out_plane_depth, geom, binning,
-     img, longest_list, binning_capacity, launched_ahead, elapsed, mwd) = _n.ops.render_forward(
+     img, longest_list, binning_capacity, launched_ahead, elapsed, mwd) = _ops.render_forward(
         background, H, W, means2D, depths, radii, conic_opacity, rgb, compute_locally, float(focal_x), float(focal_y),
         all_map if render_geo else None, bool(render_geo), bool(debug), want_mwd, _want_timing(args), int(small_limit),
         int(block_records), int(expected_instances), int(expected_longest_list), blend_records, _n.stream_handle(dev))
@@ -256,7 +256,7 @@ def render_gaussians_backward(background, tan_fovx, tan_fovy, all_map_pixels, al
         _record_time(args, "backward_render_time", 0.0)
         return tuple(torch.empty(0, n, dtype=torch.float32, device=dev) for n in (2, 3, 4, NUM_CHANNELS, NUM_ALL_MAP))
     geo = bool(render_geo)
-    *grads, elapsed = _n.ops.render_backward(
+    *grads, elapsed = _ops.render_backward(
         background, float(tan_fovx), float(tan_fovy), all_map_pixels if geo else None, all_maps if geo else None, int(R),
         geomBuffer, binningBuffer, imageBuffer, compute_locally, dL_dout_color, dL_dout_all_map if geo else None,
         dL_dout_plane_depth if geo else None, means2D, conic_opacity, rgb, geo, bool(debug), _want_timing(args),

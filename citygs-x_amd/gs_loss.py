@@ -6,12 +6,14 @@ import torch
 
 import gsrast_native as _n
 
+_ops = _n.ops
+
 
 class _L1SsimMaps(torch.autograd.Function):
     @staticmethod
     def forward(ctx, img1, img2, pixel_mask):
         need = ctx.needs_input_grad[0]
-        l1, ss, *saved = _n.ops.ssim_l1_forward(img1, img2, pixel_mask, need, _n.stream_handle(img1.device))
+        l1, ss, *saved = _ops.ssim_l1_forward(img1, img2, pixel_mask, need, _n.stream_handle(img1.device))
         if need:
             ctx.save_for_backward(*saved)
         ctx.set_materialize_grads(False)
@@ -22,7 +24,7 @@ class _L1SsimMaps(torch.autograd.Function):
         a, b, m, d_mu, d_xx, d_xy = ctx.saved_tensors
         if g_l1 is None and g_ssim is None:
             return torch.zeros_like(a), None, None
-        return (_n.ops.ssim_l1_backward(a, b, m, g_l1, g_ssim, d_mu, d_xx, d_xy, _n.stream_handle(a.device)), None,
+        return (_ops.ssim_l1_backward(a, b, m, g_l1, g_ssim, d_mu, d_xx, d_xy, _n.stream_handle(a.device)), None,
                 None)
 
 

@@ -8,6 +8,8 @@ import torch
 
 import gsrast_native as _n
 
+_ops = _n.ops
+
 
 class _NeuralGaussians(torch.autograd.Function):
     @staticmethod
@@ -19,7 +21,7 @@ class _NeuralGaussians(torch.autograd.Function):
         k = offsets.shape[1]
         if not _n.lib.gs_neural_supported(k):
             raise NotImplementedError(f"n_offsets = {k} is not among the values the kernels are built for")
-        out, saved, params, ctx.opacity_scale, ctx.level, ctx.opacity_tanh = _n.ops.neural_forward(
+        out, saved, params, ctx.opacity_scale, ctx.level, ctx.opacity_tanh = _ops.neural_forward(
             anchor, feat, offsets, scaling, campos, opacity_scale, level, input_flags, params,
             _n.stream_handle(anchor.device))
         # (opacity_scale carries no gradient: a buffer of the model)
@@ -33,7 +35,7 @@ class _NeuralGaussians(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_xyz, g_color, g_opacity, g_scal, g_rot, _g_nop, _g_mask):
         saved = ctx.saved_tensors
-        d_inputs = _n.ops.neural_backward(*saved[:10], saved[10:], ctx.opacity_scale, ctx.level, ctx.input_flags,
+        d_inputs = _ops.neural_backward(*saved[:10], saved[10:], ctx.opacity_scale, ctx.level, ctx.input_flags,
                                           ctx.opacity_tanh, (g_xyz, g_color, g_opacity, g_scal, g_rot),
                                           _n.stream_handle(saved[0].device))
         return (*d_inputs[:4], None, None, None, None, *d_inputs[4:])
@@ -59,7 +61,7 @@ class _VisibleRows(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, mask, anchor, feat, offsets, scaling, want_index):
-        *out, index, rank = _n.ops.visible_rows(mask, anchor, feat, offsets, scaling, want_index,
+        *out, index, rank = _ops.visible_rows(mask, anchor, feat, offsets, scaling, want_index,
                                                 _n.stream_handle(anchor.device))
         ctx.save_for_backward(rank)
         ctx.k = offsets.shape[1]
@@ -78,7 +80,7 @@ class _VisibleRows(torch.autograd.Function):
             idx = (rank >= 0).nonzero(as_tuple=True)[0]
             return (None, *[None if g is None else
                             torch.zeros(A, *g.shape[1:], device=g.device).index_add(0, idx, g) for g in grads], None)
-        return (None, *_n.ops.visible_rows_backward(rank, ctx.k, grads, _n.stream_handle(rank.device)), None)
+        return (None, *_ops.visible_rows_backward(rank, ctx.k, grads, _n.stream_handle(rank.device)), None)
 
 
 def _visible_rows(mask, anchor, feat, offsets, scaling, want_index):

@@ -3,13 +3,14 @@
 There is no fallback: if the library is missing or a symbol cannot be
 resolved, importing this module raises, and every entry point raises
 RuntimeError with the library's message on a non-zero status.
+
+The module itself needs neither torch nor the torch extension (any caller of the library can use its table); `ops` and
+`stream_handle`, what the operator modules call beside the table, load both when they are first asked for.
 """
 import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
-
-import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libgsrast.so")
@@ -34,13 +35,18 @@ def _load_ops():
     return module
 
 
-ops = _load_ops()
+def __getattr__(name):
+    if name not in ("ops", "stream_handle"):
+        raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+    import torch
 
+    def stream_handle(device):
+        """The device's current stream as the number the entry points of `ops` take (0 for the CPU: those entry points
+        refuse its tensors)."""
+        return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
 
-def stream_handle(device):
-    """The device's current stream as the number the entry points of `ops` take (0 for the CPU: those entry points
-    refuse its tensors)."""
-    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
+    globals().update(ops=_load_ops(), stream_handle=stream_handle)
+    return globals()[name]
 
 
 RESIZE_FN = C.CFUNCTYPE(C.c_void_p, C.c_size_t, C.c_void_p)

@@ -144,3 +144,27 @@ def test_tensors_the_kernels_use_in_place_are_checked():
             backward(gmap=bad)
     with pytest.raises(RuntimeError, match="no CPU path"):
         backward(gmap=z(P, 10)[:, ::2])  # (made contiguous by the call)
+
+
+def test_the_table_needs_neither_torch_nor_the_torch_extension():
+    """gsrast_native is what any caller of the C ABI can use: the library and its table of argument types."""
+    import subprocess
+    import sys
+    code = """
+import sys
+sys.modules["torch"] = None  # (import torch raises)
+sys.path.insert(0, %r)
+import gsrast_native as gn
+gn.OPS_PATH = "/nowhere/gsrast_ops.so"
+assert gn.lib.gs_higher_msb(8160) == 13 and len(gn.EXPORTED_SYMBOLS) > 25
+gn.RenderOptions(), gn.RenderResult()
+for name in ("ops", "stream_handle"):
+    try:
+        getattr(gn, name)
+    except ImportError:
+        continue
+    raise SystemExit(name)
+assert not hasattr(gn, "nothing_of_that_name")
+""" % os.path.join(ROOT, "citygs-x_amd")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.stdout, r.stderr)
