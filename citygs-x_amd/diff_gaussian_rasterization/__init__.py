@@ -145,6 +145,11 @@ class _ChannelGradients:
 _linked_all_map_seen = [False]
 
 
+def _have_versions(sources):
+    """Whether the link between the calls can be checked: tensors of inference mode have no version counter."""
+    return not (torch.is_inference_mode_enabled() or any(t.is_inference() for t in sources))
+
+
 def _records_wanted(rs, P, device):
     """Whether preprocess should write the records: the last view of this image size had enough instances per
     Gaussian for records to pay (written on the way they cost about a third of the library's packing pass, which
@@ -165,10 +170,11 @@ class _PreprocessGaussians(torch.autograd.Function):
         # (when a backward pass can follow, the forward kernel also leaves the colours' derivative with respect to
         # the view direction, nine numbers per Gaussian, which is all the backward kernel needs the coefficients for)
         P = means3D.shape[0]
+        linkable = P > 0 and _have_versions((means3D, scales, rotations, rs.viewmatrix, rs.campos))
         records = (torch.empty(P, 16, dtype=torch.float32, device=means3D.device)
-                   if P > 0 and _records_wanted(rs, P, means3D.device) else None)
+                   if linkable and _records_wanted(rs, P, means3D.device) else None)
         all_map = (torch.empty(P, 5, dtype=torch.float32, device=means3D.device)
-                   if P > 0 and rs.render_geo and _linked_all_map_seen[0] else None)
+                   if linkable and rs.render_geo and _linked_all_map_seen[0] else None)
         (num_rendered, means2D, depths, radii, cov3D, conic_opacity, rgb, clamped), ddir = _C.preprocess_gaussians_ex(
             means3D, scales, rotations, sh, opacities, rs.scale_modifier, rs.viewmatrix, rs.projmatrix, rs.tanfovx,
             rs.tanfovy, rs.image_height, rs.image_width, rs.sh_degree, rs.campos, rs.prefiltered, rs.debug, cuda_args,
@@ -364,7 +370,7 @@ def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_
     _linked_all_map_seen[0] = True
     blend = getattr(blend_records_of, "_gs_blend", None)
     all_map = _BuildAllMap.apply(*sources, blend)
-    if blend is not None and blend.same_sources(sources):
+    if blend is not None and blend.same_sources(sources) and not all_map.is_inference():
         blend.all_map_ref = weakref.ref(all_map)
         blend.all_map_version = all_map._version
     return all_map

@@ -293,3 +293,27 @@ def test_views_of_several_threads_do_not_meet(K, monkeypatch):
     for name in "ab":
         t, out = outs[name]
         assert out[0]._gs_blend.sources[0]() is t["m"], name
+
+
+def test_views_in_inference_mode(K):
+    """Tensors of inference mode have no version counter to check the link by: such a view is an unlinked one."""
+    import diff_gaussian_rasterization as dgr
+    rs = settings()
+    view(leaves(), rs)
+    dgr._expectations[(rs.image_height, rs.image_width, torch.device("cpu"))] = (100, 10)  # (records are worth writing)
+    try:
+        want = K.channels(*[leaves()[k].detach() for k in "msq"])
+        with torch.inference_mode():
+            means2D, co, am = view(leaves(), rs)
+            cold = {k: v.detach().clone() for k, v in leaves().items()}
+        assert torch.equal(am, want) and not hasattr(means2D, "_gs_blend")
+        with torch.no_grad():
+            assert torch.equal(view(cold, rs)[2], want)
+        t = leaves()
+        means2D = dgr.preprocess_gaussians(t["m"], t["s"], t["q"], t["sh"], t["o"], rs, None)[0]
+        with torch.inference_mode():
+            for _ in range(2):  # (handed out, then formed)
+                am = dgr.build_all_map(t["m"], t["s"], t["q"], rs.viewmatrix, rs.campos, blend_records_of=means2D)
+                assert torch.equal(am, want)
+    finally:
+        dgr._expectations.clear()
