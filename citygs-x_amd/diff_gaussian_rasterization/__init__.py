@@ -263,7 +263,8 @@ def _remember(key, instances, longest):
     _expectations.pop(key, None)  # (re-inserted at the end: the dict keeps insertion order)
     _expectations[key] = (instances, longest)
     while len(_expectations) > _MAX_EXPECTATIONS:
-        _expectations.pop(next(iter(_expectations)))
+        # (a copy to look at: another thread may be adding entries, or have removed this one)
+        _expectations.pop(list(_expectations)[0], None)
 
 
 class _RenderGaussians(torch.autograd.Function):

@@ -317,3 +317,28 @@ def test_views_in_inference_mode(K):
                 assert torch.equal(am, want)
     finally:
         dgr._expectations.clear()
+
+
+def test_expectations_remembered_by_several_threads():
+    """More image sizes than are kept, from four threads: entries come and go under each other's hands."""
+    import sys
+    import diff_gaussian_rasterization as dgr
+    failed = []
+
+    def work(i):
+        try:
+            for k in range(20000):
+                dgr._remember((i, k), 1, 1)
+        except Exception as e:
+            failed.append(repr(e))
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+        assert not failed and len(dgr._expectations) <= dgr._MAX_EXPECTATIONS
+    finally:
+        sys.setswitchinterval(interval)
+        dgr._expectations.clear()
