@@ -57,8 +57,8 @@ class GaussianRasterizationSettings(NamedTuple):
 # In the same way preprocess_gaussians forms the channels themselves once a caller builds all_map through
 # build_all_map(..., blend_records_of=means2D): that call then hands out what the preprocess kernel left instead of
 # launching one of its own.  The autograd graph is the same with and without: build_all_map's result belongs to a node
-# of its own, with its own saved tensors, so that a loss on the channels and a loss on the image can be differentiated
-# one after the other.  Where both nodes run in one backward pass the channels' node leaves its gradient to the
+# of its own, with its own saved tensors, so that a loss on the channels and one that does not go through them can be
+# differentiated one after the other.  Where both nodes run in one backward pass the channels' node leaves its gradient to the
 # preprocess node (_ChannelGradients), whose kernel has means and rotations in registers.
 
 class _BlendRecords:
@@ -364,7 +364,8 @@ def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_
     operand records with these very channels in them (from the next view on), and render_gaussians, given these
     very tensors, skips the pass that packs them; it also forms this tensor's values and, where one backward pass runs
     through both, takes its gradient.  The returned values, the gradients and the autograd graph are the same either
-    way.  Both are used on the stream preprocess_gaussians ran on only."""
+    way, except that through the link a Gaussian whose channels get a gradient of zero gets zero from them whatever its
+    parameters are (build_all_map's own kernel makes a NaN of it where they are not finite).  Both are used on the stream preprocess_gaussians ran on only."""
     sources = (means3D, scales, rotations, viewmatrix, campos)
     if blend_records_of is None:
         return _BuildAllMap.apply(*sources, None)
