@@ -46,11 +46,12 @@ BYTES_PER_GAUSSIAN = {
 # sort_pairs: the radix sort (5 passes of 9-bit digits over 44 key bits), timed on its own on keys of the same
 # distribution: only a view whose tile grid has more than 30000 tiles builds its lists with it.
 BYTES_PER_INSTANCE = {"sort_pairs": 128, "identify_tile_ranges": 20, "tile_sort": 32}
-# simple-knn (distCUDA2) per point: bounding box 24 B (12 read, twice: partial and final are one pass over the
-# points plus a small second one: the figure the reference's two reduction passes give), curve keys 16 B (12 in, 4 out), 32-bit radix sort with
-# index payload 68 B (4 B histogram read + 4 passes x (8 in + 8 out)), gather into sorted order 32 B (4 B index +
-# 12 B point in, 16 B out), box bounds 32 B (the 1024-point boxes and the 64-point leaves each read the 16 B points).
-BYTES_PER_POINT = {"knn_minmax": 24, "knn_keys": 16, "knn_sort": 68, "knn_boxes": 32}
+# simple-knn (distCUDA2) per point: bounding box 12 B read; curve keys 12 B in, 4 B key and 4 B index out (the kernel
+# counts the sort's digits as well); 32-bit radix sort with index payload, 8 B in and 8 B out per 9-bit digit (four
+# digits of a 30-bit key, three of the 27-bit key up to 2^15 points); gather into sorted order with the bounds of boxes,
+# leaves and twigs formed on the way, one pass: 4 B index and 12 B point in, 16 B out.
+BYTES_PER_POINT = {"knn_minmax": 12, "knn_keys": 20, "knn_sort": 64, "knn_boxes": 32}
+KNN_SHORT_SORT = (1 << 15, 48)  # up to this many points: bytes per point of the sort
 # The binning stage as a whole, in per-unit figures of the reference's algorithm on the same job:
 # per Gaussian tile count 16 + prefix sum 8 + key emission 20 B; per instance 12 B of key/value written, 152 B
 # for a radix sort with 8-bit digits over the 44 key bits, 8 B for the tile ranges.  The per-tile route here moves
@@ -579,7 +580,10 @@ def main():
         elif name in BYTES_PER_INSTANCE:
             nbytes = BYTES_PER_INSTANCE[name] * R
         elif name in BYTES_PER_POINT:
-            nbytes = BYTES_PER_POINT[name] * P
+            per_point = BYTES_PER_POINT[name]
+            if name == "knn_sort" and P <= KNN_SHORT_SORT[0]:
+                per_point = KNN_SHORT_SORT[1]
+            nbytes = per_point * P
         elif name == "duplicate_with_keys":
             nbytes = 20 * P + 12 * R
         elif name == "bucket_scatter":

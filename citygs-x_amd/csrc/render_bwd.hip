@@ -4,8 +4,8 @@
 // over pixels.
 //
 // Workgroup = one 16x16 tile = four 64-lane waves; a wave owns an 8x8 quadrant
-// and each of its 16-lane rows a 4x4 pixel block, a quad of lanes four pixels
-// of an image row.
+// and each of its 16-lane rows a 4x4 pixel block, a quad of lanes one of the
+// block's columns.
 //   * The tile's list is scanned back to front, 256 entries at a time, and the
 //     entries that touch a block in front of its deepest contributor (the
 //     forward kernel's own answer, 16 bits per instance, when the caller hands
@@ -386,6 +386,10 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // such a Gaussian its conic sums are taken in a fixed order (`thin`: the sixteen pixels of a row as a tree; and
         // `exact`, if three or four rows touch it: the rows by their places in the lists of a run of 64 positions, rows
         // at the same place merged first), whatever else is staged or skipped.  Below THIN the factor is at most 25.
+        // That is the order of a kernel that takes one entry per pass and reduces its sums over the row's lanes.  On 16
+        // scenes of 60 to 4000 Gaussians, a quarter of them thin, the covariance gradients of the thin ones are a relative
+        // 7.9e-6 from float64 in this order, 7.9e-6 in that kernel and 8.9e-6 with the order left to the lists (12 of the
+        // 16 worse); the conic gradients themselves are 2.1e-6 off in all three.
         const float4 cq = s_co[js];
         const bool is_thin = !(cq.y * cq.y < THIN * cq.x * cq.z);
         thin = gs_ballot(is_thin && nibble != 0u) != 0ull;
@@ -489,8 +493,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         step(std::integral_constant<int, 1>{});
         step(std::integral_constant<int, 2>{});
         step(std::integral_constant<int, 3>{});
-        // The sums over pixels.  From here on lane e of a quad works for entry e, register p is the quad's pixel p (four
-        // pixels of one image row).  The per-Gaussian factors of the geometric gradients stay out of the sums: with
+        // The sums over pixels.  From here on lane e of a quad works for entry e, register p is the quad's pixel p (the
+        // quad's four pixels are one column of the block: dx is the quad's, dy the register's).  The per-Gaussian factors of the geometric gradients stay out of the sums: with
         // q = G dL/dalpha, u = conic (dx, dy), a pixel's terms are dL/dmean = -opacity q u,
         // dL/dconic = -opacity/2 q (dx dx, dx dy, dy dy) and dL/dopacity = q
         // (cuda_rasterizer/backward.cu:520-541); sum q u is formed from sum q (dx, dy) by the thread that hands the

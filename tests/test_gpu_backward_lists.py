@@ -1,4 +1,5 @@
-"""Backward blend at the list lengths where its steps change: four entries per pass, sub-batches of 64 slots, staged
+"""Backward blend by itself (the entry point that is handed finished lists and neither hit words nor an order of the
+tiles; tests/test_gpu_backward_view.py has the whole view) at the list lengths where its steps change: four entries per pass, sub-batches of 64 slots, staged
 batches of 128, scans of 256 positions, runs of 64; with and without thin Gaussians (whose sums keep a fixed order), on
 an image whose last tiles are cut off, against the oracle."""
 import numpy as np
@@ -52,8 +53,8 @@ def test_list_lengths(H, orc, n, thin, geo):
                             H.dev(gdep), H.as_u32(b["emission_sorted"]), H.as_u32(b["point_offsets"]), render_geo=geo)
 
     got, again = run(), run()
-    # 24-bit sums of at most 700 x 256 terms in another order: about sqrt(terms) * 2^-24 of the sum of magnitudes,
-    # which is some ten times the sum itself
+    # 24-bit sums in another order: about sqrt(terms) * 2^-24 of the sum of magnitudes, which is some ten times the sum
+    # itself.  A Gaussian's terms are its pixels', at most 41 x 27 of them: sqrt(1107) * 2^-24 * 10 = 2e-5.
     for k, want in (("dL_dmeans2D", ref["dL_dmeans2D"][:, :2]), ("dL_dmeans2D_abs", ref["dL_dmeans2D_abs"]),
                     ("dL_dconic_opacity", ref["dL_dconic_opacity"]), ("dL_dcolors", ref["dL_dcolors"]),
                     ("dL_dall_map", ref["dL_dall_map"])):
