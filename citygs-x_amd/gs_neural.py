@@ -78,8 +78,8 @@ class _VisibleRows(torch.autograd.Function):
         if torch.is_grad_enabled():  # a graph of the backward pass is asked for
             A = rank.shape[0]
             idx = (rank >= 0).nonzero(as_tuple=True)[0]
-            return (None, *[None if g is None else
-                            torch.zeros(A, *g.shape[1:], device=g.device).index_add(0, idx, g) for g in grads], None)
+            return (None, *[None if g is None else g.new_zeros(A, *g.shape[1:]).index_add(0, idx, g) for g in grads],
+                    None)
         return (None, *_ops.visible_rows_backward(rank, ctx.k, grads, _n.stream_handle(rank.device)), None)
 
 
