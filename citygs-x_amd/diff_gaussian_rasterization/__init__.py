@@ -58,8 +58,8 @@ class GaussianRasterizationSettings(NamedTuple):
 # build_all_map(..., blend_records_of=means2D): that call then hands out what the preprocess kernel left instead of
 # launching one of its own.  The autograd graph is the same with and without: build_all_map's result belongs to a node
 # of its own, with its own saved tensors, so that a loss on the channels and one that does not go through them can be
-# differentiated one after the other.  Where both nodes run in one backward pass the channels' node leaves its gradient to the
-# preprocess node (_ChannelGradients), whose kernel has means and rotations in registers.
+# differentiated one after the other.  Where both nodes run in one backward pass the channels' node leaves its gradient
+# to the preprocess node (_ChannelGradients), whose kernel has means and rotations in registers.
 
 class _BlendRecords:
     """What one preprocess call leaves for build_all_map and render_gaussians, beside its outputs."""
@@ -365,7 +365,8 @@ def build_all_map(means3D, scales, rotations, viewmatrix, campos, blend_records_
     very tensors, skips the pass that packs them; it also forms this tensor's values and, where one backward pass runs
     through both, takes its gradient.  The returned values, the gradients and the autograd graph are the same either
     way, except that through the link a Gaussian whose channels get a gradient of zero gets zero from them whatever its
-    parameters are (build_all_map's own kernel makes a NaN of it where they are not finite).  Both are used on the stream preprocess_gaussians ran on only."""
+    parameters are (build_all_map's own kernel makes a NaN of it where they are not finite).  Both are used on the
+    stream preprocess_gaussians ran on only."""
     sources = (means3D, scales, rotations, viewmatrix, campos)
     if blend_records_of is None:
         return _BuildAllMap.apply(*sources, None)
