@@ -91,3 +91,31 @@ def test_fused_adam_tracks_torch_adam():
         c = FusedAdam([torch.zeros(3, requires_grad=True)], lr=1e-3)
         c.param_groups[0]["params"][0].grad = torch.ones(3)
         c.step()
+
+
+@pytest.mark.parametrize("sizes", [[1, 511, 512, 513, 5119], [0, 1024, 100_003]])
+def test_a_step_that_streams_past_the_caches_gives_the_same_bits(sizes):
+    # beside a tensor of 20 M elements the same tensors are stepped by the streaming variant of the kernel
+    from gs_optim import FusedAdam
+
+    def step(filler):
+        gen = torch.Generator().manual_seed(17)
+        store = [torch.randn(n + 1, generator=gen).to(DEV) for n in sizes]
+        # (the last one starts 4 bytes off a 16-byte boundary)
+        params = [torch.nn.Parameter(s[1:] if i == len(sizes) - 1 else s[:n])
+                  for i, (s, n) in enumerate(zip(store, sizes))]
+        grads = [torch.randn(n, generator=gen).to(DEV) for n in sizes]
+        big = [torch.nn.Parameter(torch.ones(filler, device=DEV))] if filler else []
+        opt = FusedAdam([{"params": [p], "lr": 1e-2} for p in params + big], lr=0.0, eps=1e-15)
+        for _ in range(2):
+            for p, g in zip(params, grads):
+                p.grad = g.clone()
+            for p in big:
+                p.grad = torch.full_like(p, 0.5)
+            opt.step()
+        if big:  # every element of the large tensor moved, and alike
+            assert float(big[0].detach().amin()) == float(big[0].detach().amax()) < 1.0
+        return [t for p in params for t in (p.detach(), opt.state[p]["exp_avg"], opt.state[p]["exp_avg_sq"])]
+
+    for a, b in zip(step(0), step(20_000_001)):
+        assert torch.equal(a, b)
