@@ -124,8 +124,9 @@ __device__ __forceinline__ uint32_t f2u_sat(float v) {
 }
 
 // Store for data that is written once and not read again on the GPU for a long while (gradients of leaf
-// parameters on their way to the optimizer): it goes out past the caches, so it does not evict what the next
-// kernel reads.
+// parameters on their way to the optimizer, what the forward pass leaves for the backward pass): it goes out past the
+// caches, so it does not evict what the next kernel reads.
+__device__ __forceinline__ void store_streaming(float* p, float v) { __builtin_nontemporal_store(v, p); }
 __device__ __forceinline__ void store_streaming(float4* p, const float4& v) {
   typedef float v4f __attribute__((ext_vector_type(4)));
   const v4f w = {v.x, v.y, v.z, v.w};

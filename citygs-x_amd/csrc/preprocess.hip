@@ -370,6 +370,21 @@ __device__ __forceinline__ void wave_rows_store(float4* __restrict__ g4, int row
   }
 }
 
+// The rows of N floats that the lanes of a wave hold leave through LDS as N runs of consecutive floats.
+template <int N>
+__device__ __forceinline__ void wave_rows_turn_store(float* __restrict__ out, int rows, const float* own, float* lds,
+                                                     int lane) {
+  wave_sync_lds();  // (everyone has read what the buffer last held)
+#pragma unroll
+  for (int k = 0; k < N; k++) lds[N * lane + k] = own[k];
+  wave_sync_lds();
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const int e = j * GS_WAVE + lane;
+    if (e < N * rows) out[e] = lds[e];
+  }
+}
+
 // DERIV: also leave, per surviving Gaussian, the derivative of its colour with respect to the view direction
 // (nine numbers), which is all the backward kernel needs the coefficients for.
 // RECORDS: also write the blend kernels' operand record of every surviving Gaussian, (x, y, conic.x, conic.y)
@@ -377,6 +392,9 @@ __device__ __forceinline__ void wave_rows_store(float4* __restrict__ g4, int row
 // all_map kernel's own operations on the same inputs; a wave's 64 records leave through LDS as contiguous lines.
 // MAP: also write the geometry channels of all Gaussians, culled ones included, as the (P,5) tensor the all_map kernel
 // would write (same operations, same bits).
+// What only the backward pass reads (derivative, channels and, where the records are written, the conics) is stored past
+// the caches: 10 M Gaussians 463 us against 495, 1 M 75 against 78, and the counting kernel that follows finds more of its
+// input cached (53 us against 60).  Streaming loads of the coefficients lose (1 M 92 us): a row's thirds share lines.
 // (six waves per SIMD; five with the records, or with channels and derivative: six would spill there, and a kernel that
 // spills starts its waves slowly)
 template <bool DERIV, bool RECORDS, bool MAP>
@@ -418,7 +436,9 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     radii[i] = ok ? g.radius : 0;
     depths[i] = ok ? g.depth : 0.f;
     means2D[i] = ok ? make_float2(g.px, g.py) : make_float2(0.f, 0.f);
-    conic_opacity[i] = ok ? make_float4(g.conic[0], g.conic[1], g.conic[2], opac[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 co = ok ? make_float4(g.conic[0], g.conic[1], g.conic[2], opac[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (RECORDS) store_streaming(conic_opacity + i, co);  // (the blend kernels read the records instead)
+    else conic_opacity[i] = co;
     if (tiles_touched) tiles_touched[i] = ok ? (g.rect.x1 - g.rect.x0) * (g.rect.y1 - g.rect.y0) : 0u;
   }
   if (MAP || (RECORDS && ok)) {  // (culled Gaussians have channels, but no record)
@@ -450,7 +470,7 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
 #pragma unroll
     for (int j = 0; j < 5; j++) {
       const int e = j * GS_WAVE + lane, row = e / 5;
-      if ((size_t)e < 5 * rows_left) out[e] = s_keep[wave][(e - 5 * row) * GS_WAVE + row];
+      if ((size_t)e < 5 * rows_left) store_streaming(out + e, s_keep[wave][(e - 5 * row) * GS_WAVE + row]);
     }
   }
 
@@ -506,7 +526,7 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
 #pragma unroll
         for (int j = 0; j < 9; j++) {
           const size_t e = (size_t)j * GS_WAVE + (size_t)lane;
-          if (e < 9 * rows_left) out[e] = lds[e];
+          if (e < 9 * rows_left) store_streaming(out + e, lds[e]);
         }
       }
     } else if (ok) {
@@ -628,7 +648,10 @@ mark_visible_kernel(int P, const float* __restrict__ means, const float* __restr
 // well; its part is added to the gradients of means and rotations here, where those inputs are at hand.  As a kernel of
 // its own plus the two accumulations it reads them again and moves 56 + 84 more bytes per Gaussian: 18 + 15 us at 1 M
 // Gaussians and 168 + 140 us at 10 M, against 6 and 45 us in here.
-// The kernel is bound by HBM (10 M Gaussians, 3 M of them visible: 3.8 GB in 680 us).
+// The kernel is bound by HBM.  All loads of a Gaussian go out together and the 12-byte rows leave through LDS: 10 M
+// Gaussians, a quarter of them visible, 639 us (3.6 GB) against 677 with each load where its value is used and each lane
+// storing its own rows; 4 M 276 against 291, 1 M 73 against 77.  (Fetching the rows through LDS as well costs what it
+// gains, with and without non-temporal loads.)
 template <bool SAVED, bool MAP>
 __global__ void __launch_bounds__(GS_BLOCK_1D)
 preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, const int* __restrict__ radii,
@@ -663,6 +686,29 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     const float* go = dL_dall_map + 5 * (size_t)i;
     map_g[0] = go[0]; map_g[1] = go[1]; map_g[2] = go[2]; map_g[3] = go[4];
   }
+  // (zero for a Gaussian no pixel blended, culled ones first of all)
+  const bool map_live = MAP && !(map_g[0] == 0.f && map_g[1] == 0.f && map_g[2] == 0.f && map_g[3] == 0.f);
+  // Everything the two parts below take of a Gaussian is asked for at once: one latency for all of it, and a line that
+  // several loads share is still there.
+  float mean[3] = {0.f, 0.f, 0.f}, sc[3] = {0.f, 0.f, 0.f}, gcol[3] = {0.f, 0.f, 0.f}, dd[9];
+  float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (live || map_live) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) mean[k] = means[3 * (size_t)i + k];
+    if (scales) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) sc[k] = scales[3 * (size_t)i + k];
+      q4 = reinterpret_cast<const float4*>(rots)[i];
+    }
+  }
+  if (live && sh_mode) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) gcol[k] = dL_dcolor[3 * (size_t)i + k];
+    if (SAVED) {
+#pragma unroll
+      for (int k = 0; k < 9; k++) dd[k] = dcolor_ddir[9 * (size_t)i + k];
+    }
+  }
   const long long left = (long long)P - (long long)wave_first;
   const int rows = left <= 0 ? 0 : left < GS_WAVE ? (int)left : GS_WAVE;
   // SAVED: the colour part comes first, so that what it keeps in registers (the row of coefficient gradients is the
@@ -673,11 +719,9 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
 #pragma unroll
     for (int k = 0; k < 16; k++) basis[k] = 0.f;
     if (live) {
-      const float d0[3] = {means[3 * (size_t)i] - camg[0], means[3 * (size_t)i + 1] - camg[1],
-                           means[3 * (size_t)i + 2] - camg[2]};
+      const float d0[3] = {mean[0] - camg[0], mean[1] - camg[1], mean[2] - camg[2]};
 #pragma unroll
-      for (int ch = 0; ch < 3; ch++) gr[ch] = dL_dcolor[3 * (size_t)i + ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
-      const float* dd = dcolor_ddir + 9 * (size_t)i;
+      for (int ch = 0; ch < 3; ch++) gr[ch] = gcol[ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
       const float dRdx[3] = {dd[0], dd[1], dd[2]}, dRdy[3] = {dd[3], dd[4], dd[5]}, dRdz[3] = {dd[6], dd[7], dd[8]};
       sh_gradient_of_mean(d0, dRdx, dRdy, dRdz, gr, sh_gm);
       const float len = sqrtf(dot3(d0, d0));
@@ -719,7 +763,6 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   if (live) {
     CamParams cam;
     load_cam(Vg, PMg, camg, cam);
-    const float mean[3] = {means[3 * (size_t)i], means[3 * (size_t)i + 1], means[3 * (size_t)i + 2]};
     float c6[6];
     if (cov3D != nullptr) {
       const float2* c6v = reinterpret_cast<const float2*>(cov3D + 6 * (size_t)i);
@@ -727,8 +770,6 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       c6[0] = a.x; c6[1] = a.y; c6[2] = b.x; c6[3] = b.y; c6[4] = c.x; c6[5] = c.y;
     } else {
       // the forward pass's own operations on the same inputs: the same bits it would have stored
-      const float sc[3] = {scales[3 * (size_t)i], scales[3 * (size_t)i + 1], scales[3 * (size_t)i + 2]};
-      const float4 q4 = reinterpret_cast<const float4*>(rots)[i];
       const float q[4] = {q4.x, q4.y, q4.z, q4.w};
       M3 unused_m, unused_r;
       cov3d_from_scale_rot(sc, mod, q, c6, &unused_m, &unused_r);
@@ -821,7 +862,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       const float len = sqrtf(dot3(d0, d0));
       float gr[3];
 #pragma unroll
-      for (int ch = 0; ch < 3; ch++) gr[ch] = dL_dcolor[3 * (size_t)i + ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
+      for (int ch = 0; ch < 3; ch++) gr[ch] = gcol[ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
       float basis[16];
       float dRdx[3], dRdy[3], dRdz[3];
       sh_basis_and_direction_derivative<true>(D, d0[0] / len, d0[1] / len, d0[2] / len, shv, basis, dRdx, dRdy, dRdz);
@@ -844,8 +885,6 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     }
 
     if (scales) {
-      const float sc[3] = {scales[3 * (size_t)i], scales[3 * (size_t)i + 1], scales[3 * (size_t)i + 2]};
-      const float4 q4 = reinterpret_cast<const float4*>(rots)[i];
       const float q[4] = {q4.x, q4.y, q4.z, q4.w};
       M3 Mm, R;
       float tmp6[6];
@@ -894,20 +933,16 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   }
   if (sh_staged && !SAVED)
     wave_rows_store<STORE_ROWS>(reinterpret_cast<float4*>(dL_dsh) + wave_first * 12, rows, s_rows[wave], lane);
-  if (!in_range) return;
   if (MAP) {
     const float g0 = map_g[0], g1 = map_g[1], g2 = map_g[2], g4 = map_g[3];
-    // (zero for a Gaussian no pixel blended, culled ones first of all)
-    if (!(g0 == 0.f && g1 == 0.f && g2 == 0.f && g4 == 0.f)) {
+    if (map_live) {
       float V[16], campos[3];
 #pragma unroll
       for (int k = 0; k < 16; k++) V[k] = Vg[k];
 #pragma unroll
       for (int k = 0; k < 3; k++) campos[k] = camg[k];
-      const float mean[3] = {means[3 * (size_t)i], means[3 * (size_t)i + 1], means[3 * (size_t)i + 2]};
-      const float sc[3] = {scales[3 * (size_t)i], scales[3 * (size_t)i + 1], scales[3 * (size_t)i + 2]};
       AllMapGeom ag;
-      all_map_geom(mean, sc, reinterpret_cast<const float4*>(rots)[i], V, campos, ag);
+      all_map_geom(mean, sc, q4, V, campos, ag);
       float dmean[3], dq[4];
       all_map_gradient(ag, V, g0, g1, g2, g4, dmean, dq);
 #pragma unroll
@@ -916,14 +951,10 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       for (int k = 0; k < 4; k++) gq[k] += dq[k];
     }
   }
-  dL_dmean3D[3 * (size_t)i] = gm[0];
-  dL_dmean3D[3 * (size_t)i + 1] = gm[1];
-  dL_dmean3D[3 * (size_t)i + 2] = gm[2];
-  if (dL_dscale) {
-    dL_dscale[3 * (size_t)i] = gs_[0];
-    dL_dscale[3 * (size_t)i + 1] = gs_[1];
-    dL_dscale[3 * (size_t)i + 2] = gs_[2];
-  }
+  float* const lds = reinterpret_cast<float*>(s_rows[wave]);
+  wave_rows_turn_store<3>(dL_dmean3D + 3 * wave_first, rows, gm, lds, lane);
+  if (dL_dscale) wave_rows_turn_store<3>(dL_dscale + 3 * wave_first, rows, gs_, lds, lane);
+  if (!in_range) return;
   if (dL_drot) reinterpret_cast<float4*>(dL_drot)[i] = make_float4(gq[0], gq[1], gq[2], gq[3]);
   if (dL_dcov3D_out) {
 #pragma unroll
