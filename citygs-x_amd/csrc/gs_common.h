@@ -155,21 +155,33 @@ __device__ __forceinline__ float gs_expf(float x) {
   return __builtin_ldexpf(p, (int)n);
 }
 
-// Same routine without the range checks, for callers that guarantee -87 <= x <= 0
-// (or NaN, which propagates); returns the same bits as gs_expf there.
-__device__ __forceinline__ float gs_expf_core(float x) {
-  float n = __builtin_rintf(x * 1.44269504088896341f);
-  float r = __builtin_fmaf(n, -0.693145751953125f, x);
-  r = __builtin_fmaf(n, -1.42860682030941723212e-6f, r);
-  float p = 1.9875691500e-4f;
-  p = __builtin_fmaf(p, r, 1.3981999507e-3f);
-  p = __builtin_fmaf(p, r, 8.3334519073e-3f);
-  p = __builtin_fmaf(p, r, 4.1665795894e-2f);
-  p = __builtin_fmaf(p, r, 1.6666665459e-1f);
-  p = __builtin_fmaf(p, r, 5.0000001201e-1f);
-  float r2 = r * r;
+// -2 times the exponent of a Gaussian at offset (dx, dy) from its centre (cuda_rasterizer/forward.cu:366), of the conic
+// (A, 2 B, C): the operations of the exponent in its order, every intermediate result -2 times (or twice) the
+// exponent's own.  Scaling by a power of two is exact, so this is the same number as long as nothing overflows, and what
+// overflows lies outside the window either way.
+__device__ __forceinline__ float gauss_form(const float a, const float b2, const float c, const float dx, const float dy) {
+  return (a * dx * dx + c * dy * dy) + b2 * dx * dy;
+}
+
+// An exponent below -87 is no exponent: gs_expf is 0 there.
+#define GS_FORM_MAX 174.0f
+
+// -2 gs_expf(-0.5f * u) for 0 <= u <= GS_FORM_MAX (or NaN, which propagates), the same bits but for the factor: every
+// step works on -2, 4, -8, ... times what the step there works on, with the constants scaled by the same powers of two,
+// which is exact.
+__device__ __forceinline__ float gs_neg2_exp_of_form(float u) {
+  const float n = __builtin_rintf(u * (-0.5f * 1.44269504088896341f));
+  float r = __builtin_fmaf(n, 2.0f * 0.693145751953125f, u);
+  r = __builtin_fmaf(n, 2.0f * 1.42860682030941723212e-6f, r);
+  float p = 1.9875691500e-4f / 64;
+  p = __builtin_fmaf(p, r, -1.3981999507e-3f / 32);
+  p = __builtin_fmaf(p, r, 8.3334519073e-3f / 16);
+  p = __builtin_fmaf(p, r, -4.1665795894e-2f / 8);
+  p = __builtin_fmaf(p, r, 1.6666665459e-1f / 4);
+  p = __builtin_fmaf(p, r, -5.0000001201e-1f / 2);
+  const float r2 = r * r;
   p = __builtin_fmaf(p, r2, r);
-  p = p + 1.0f;
+  p = p - 2.0f;
   return __builtin_ldexpf(p, (int)n);
 }
 

@@ -107,9 +107,9 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   __shared__ int s_pend[PENDING];
   __shared__ uint16_t s_pend_hits[PENDING];
   __shared__ int s_found[2][WAVES];
-  // (slot BATCH: what an entry behind the end of a list refers to, a Gaussian whose floor no exponent reaches)
-  __shared__ float4 s_xyf[BATCH + 1];  // centre x, y; the power floor; the position in the tile's list, as bits
-  __shared__ float4 s_co[BATCH + 1];
+  // (slot BATCH: what an entry behind the end of a list refers to, a Gaussian of opacity 0)
+  __shared__ float4 s_xyp[BATCH + 1];  // centre x, y; the position in the tile's list, as bits; unused
+  __shared__ float4 s_co[BATCH + 1];   // the conic as (A, 2 B, C), and -1/2 of the opacity
   __shared__ uint16_t s_hits[BATCH];
   // colour, then the five geometry channels: eight floats per Gaussian, read as two 16-byte words
   __shared__ float4 s_chan[BATCH + 1][RENDER_GEO ? 2 : 1];
@@ -240,7 +240,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   for (int w = 0; w < WAVES; w++) s_acc[w][my_word] = make_float4(0.f, 0.f, 0.f, 0.f);
   if (tid == 0) {
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    s_xyf[BATCH] = make_float4(0.f, 0.f, __builtin_inff(), 0.f);
+    s_xyp[BATCH] = z;
     s_co[BATCH] = z;
 #pragma unroll
     for (int h = 0; h < (RENDER_GEO ? 2 : 1); h++) s_chan[BATCH][h] = z;
@@ -261,16 +261,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     const float tile_x0 = (float)(tile_x * GS_TILE_X), tile_y0 = (float)(tile_y * GS_TILE_Y);
     float pfl, mark_limit;
     const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
-    uint32_t found = 0u;
-#pragma unroll
-    for (int k = 0; k < WAVES; k++) {
-      bool hit[4];
-      ellipse_hits_quadrant(xy, co, cp.x, cp.y, cp.z, tile_x0 + 8.f * (float)(k & 1), tile_y0 + 8.f * (float)(k >> 1),
-                            hit);
-#pragma unroll
-      for (int r = 0; r < 4; r++) found |= hit[r] ? 1u << (4 * k + r) : 0u;
-    }
-    return found;
+    return ellipse_hits_tile(xy, co, cp.x, cp.y, cp.z, tile_x0, tile_y0);
   };
   int unscanned = tile_last;  // positions below this one have not been looked at
   uint32_t head = 0u, tail = 0u, parity = 0u;
@@ -328,12 +319,9 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
       auto stage = [&](const float2 xy, const float4 co, const float c0, const float c1, const float c2,
                        const float (&m)[GS_N_MAP]) {
         s_emis[tid] = emission_sorted[k_sorted];
-        s_co[tid] = co;
-        float pfl, mark_limit;
-        (void)block_test_params(co, xy, (float)(tile_x * GS_TILE_X), (float)(tile_y * GS_TILE_Y), pfl,
-                                mark_limit);
+        s_co[tid] = make_float4(co.x, 2.0f * co.y, co.z, -0.5f * co.w);
         s_hits[tid] = s_pend_hits[at];
-        s_xyf[tid] = make_float4(xy.x, xy.y, pfl, __int_as_float(pos));
+        s_xyp[tid] = make_float4(xy.x, xy.y, __int_as_float(pos), 0.f);
         if (render_geo) s_chan[tid][RENDER_GEO ? 1 : 0] = make_float4(m[1], m[2], m[3], m[4]);
         s_chan[tid][0] = make_float4(c0, c1, c2, m[0]);
       };
@@ -391,10 +379,11 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // 7.9e-6 from float64 in this order, 7.9e-6 in that kernel and 8.9e-6 with the order left to the lists (12 of the
         // 16 worse); the conic gradients themselves are 2.1e-6 off in all three.
         const float4 cq = s_co[js];
-        const bool is_thin = !(cq.y * cq.y < THIN * cq.x * cq.z);
+        const float cq_b = 0.5f * cq.y;
+        const bool is_thin = !(cq_b * cq_b < THIN * cq.x * cq.z);
         thin = gs_ballot(is_thin && nibble != 0u) != 0ull;
         exact = gs_ballot(is_thin && ((0xE880u >> nibble) & 1u) != 0u) != 0ull;
-        const uint32_t run = (uint32_t)(tile_last - 1 - __float_as_int(s_xyf[js].w)) / RUN;
+        const uint32_t run = (uint32_t)(tile_last - 1 - __float_as_int(s_xyp[js].z)) / RUN;
         const int last_lane = (count - base < SUB ? count - base : SUB) - 1;
         const uint32_t first_run = (uint32_t)__builtin_amdgcn_readlane((int)run, 0);
         const uint32_t last_run = (uint32_t)__builtin_amdgcn_readlane((int)run, last_lane);
@@ -434,7 +423,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // Four entries of every row's list.  Lane e of each of the row's quads fetches entry e.
         const uint32_t word = s_idx[wave][row][n / GROUP];
         const uint32_t j_own = __builtin_amdgcn_ubfe(word, quad_shift, 8u);
-        const float4 xyf = s_xyf[j_own];
+        const float4 xyp = s_xyp[j_own];
         const float4 co = s_co[j_own];
         // S = sum_ch c_ch g_ch of every (entry, pixel): a contraction over the channels, of the entries' colours and the
         // pixels' upstream gradients.  Register e of lane p of a quad receives entry e at pixel p (one fused
@@ -461,16 +450,14 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         float w[GROUP], q[GROUP];
         auto step = [&](auto e_tag) {
           constexpr int e = decltype(e_tag)::value;
-          const float dx = quad_lane<e>(xyf.x) - pfx, dy = quad_lane<e>(xyf.y) - pfy;
-          const float power = -0.5f * (quad_lane<e>(co.x) * dx * dx + quad_lane<e>(co.z) * dy * dy) -
-                              quad_lane<e>(co.y) * dx * dy;
-          const float floor_e = quad_lane<e>(xyf.z);
-          const int pos_e = __float_as_int(quad_lane<e>(xyf.w));
-          const float G_raw = gs_expf_core(power);
+          const float dx = quad_lane<e>(xyp.x) - pfx, dy = quad_lane<e>(xyp.y) - pfy;
+          const float form = gauss_form(quad_lane<e>(co.x), quad_lane<e>(co.y), quad_lane<e>(co.z), dx, dy);
+          const int pos_e = __float_as_int(quad_lane<e>(xyp.z));
+          const float G_raw = gs_neg2_exp_of_form(form);  // -2 times the Gaussian's value
           const float alpha_raw = fminf(0.99f, quad_lane<e>(co.w) * G_raw);
           // (lane masks of single comparisons, combined in scalar registers)
-          const uint64_t active_m = gs_ballot(pos_e < last_contributor) & gs_ballot(!(power > 0.0f)) &
-                                    gs_ballot(!(power < floor_e)) & gs_ballot(!(alpha_raw < 1.0f / 255.0f));
+          const uint64_t active_m = gs_ballot(pos_e < last_contributor) & gs_ballot(!(form < 0.0f)) &
+                                    gs_ballot(!(form > GS_FORM_MAX)) & gs_ballot(!(alpha_raw < 1.0f / 255.0f));
           const bool active = __builtin_amdgcn_inverse_ballot_w64(active_m);
           const float alpha = active ? alpha_raw : 0.f;
           // The transmittance follows the CPU statement's operation sequence exactly (IEEE reciprocal):
@@ -493,6 +480,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         step(std::integral_constant<int, 1>{});
         step(std::integral_constant<int, 2>{});
         step(std::integral_constant<int, 3>{});
+        // (q is -2 times what it stands for below, as G is: the thread that hands the record over takes the factor out)
         // The sums over pixels.  From here on lane e of a quad works for entry e, register p is the quad's pixel p (the
         // quad's four pixels are one column of the block: dx is the quad's, dy the register's).  The per-Gaussian factors of the geometric gradients stay out of the sums: with
         // q = G dL/dalpha, u = conic (dx, dy), a pixel's terms are dL/dmean = -opacity q u,
@@ -527,13 +515,13 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           channels(grad_t[0], c_lo);
           if (render_geo) channels(grad_t[RENDER_GEO ? 1 : 0], c_hi);
         }
-        const float dx = xyf.x - pfx, a_dx = co.x * dx, b_dx = co.y * dx;
+        const float dx = xyp.x - pfx, b = 0.5f * co.y, a_dx = co.x * dx, b_dx = b * dx;
         float dy[4], q_dy[4], ax = 0.f, ay = 0.f;
 #pragma unroll
         for (int p = 0; p < 4; p++) {
-          dy[p] = xyf.y - (block_y0 + (float)p);
+          dy[p] = xyp.y - (block_y0 + (float)p);
           q_dy[p] = q[p] * dy[p];
-          const float ux = __builtin_fmaf(co.y, dy[p], a_dx), uy = __builtin_fmaf(co.z, dy[p], b_dx);
+          const float ux = __builtin_fmaf(b, dy[p], a_dx), uy = __builtin_fmaf(co.z, dy[p], b_dx);
           ax = __builtin_fmaf(fabsf(q[p]), fabsf(ux), ax);
           ay = __builtin_fmaf(fabsf(q[p]), fabsf(uy), ay);
         }
@@ -555,6 +543,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         float v[16] = {qx, qy, ax, ay, xx, xy, yy, q0, c_lo[0], c_lo[1], c_lo[2], c_lo[3],
                        c_hi[0], c_hi[1], c_hi[2], c_hi[3]};
         quads_reduce16<RENDER_GEO>(v);
+        float sum[4] = {v[0], v[1], v[2], v[3]};
+        asm("" : "+v"(sum[0]), "+v"(sum[1]), "+v"(sum[2]), "+v"(sum[3]));  // (four registers, not a part of sixteen)
         // Quad k of a row now holds components 4 k .. 4 k + 3 of its entry e.  They go into the wave's own accumulator with
         // a plain read-add-write (the LDS accesses of a wave complete in order), one row after the other, since two rows
         // may be at the same Gaussian.  An LDS float atomic takes about three cycles per active lane.
@@ -562,7 +552,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         float4* const acc = &s_acc[wave][4u * (a_slot & (SUB - 1)) + (quad ^ ((a_slot >> 2) & 3u))];
         uint64_t write_m = gs_ballot(j_own < (uint32_t)BATCH);
         if (exact) {
-          const float own[4] = {v[0], v[1], v[2], v[3]};
+          const float own[4] = {sum[0], sum[1], sum[2], sum[3]};
 #pragma unroll
           for (int d = 1; d < 4; d++) {
             // (entries behind the ends of two lists are the same too: their sums are zero and go nowhere)
@@ -572,7 +562,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
             for (int k = 0; k < 4; k++) t[k] = __shfl_xor(own[k], 16 * d, GS_WAVE);
             if (same) {
 #pragma unroll
-              for (int k = 0; k < 4; k++) v[k] += t[k];
+              for (int k = 0; k < 4; k++) sum[k] += t[k];
             }
             write_m &= ~gs_ballot(same && (row ^ d) < row);
           }
@@ -584,7 +574,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         for (int e = 0; e < 4; e++) {
           if (__builtin_amdgcn_inverse_ballot_w64(write_m & turn_m)) {
             float4 a = *acc;
-            a.x += v[0]; a.y += v[1]; a.z += v[2]; a.w += v[3];
+            a.x += sum[0]; a.y += sum[1]; a.z += sum[2]; a.w += sum[3];
             *acc = a;
           }
           turn_m <<= turn_shift;
@@ -606,13 +596,16 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
 #pragma unroll
         for (int w = 0; w < WAVES; w++) s_acc[w][my_word] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (base + my_slot < count) {
+          // (the sums are those of -2 q)
           const float4 co = s_co[base + my_slot];
+          const float b = 0.5f * co.y;
           if (my_part == 0) {  // mean2D x, y and their sums of absolute values
-            c = make_float4(-co.w * (co.x * c.x + co.y * c.y), -co.w * (co.y * c.x + co.z * c.y), c.z * fabsf(co.w),
+            c = make_float4(-co.w * (co.x * c.x + b * c.y), -co.w * (b * c.x + co.z * c.y), c.z * fabsf(co.w),
                             c.w * fabsf(co.w));
           } else if (my_part == 1) {  // conic x, y, w; the fourth component is the opacity gradient itself
             const float h = -0.5f * co.w;
             c.x *= h; c.y *= h; c.z *= h;
+            c.w *= -0.5f;
           }
           instance_grads[4 * (size_t)s_emis[base + my_slot] + my_part] = c;
         }

@@ -56,42 +56,52 @@ __device__ __forceinline__ float4 block_test_params(float4 co, float2 xy, float 
   return make_float4(cp.x, cp.y, never ? -1.0f : (untrusted ? cp.z : mark_limit), 0.f);
 }
 
-// The four 4x4 pixel blocks of an 8x8 quadrant at (qx0, qy0), block r at x offset 4 (r & 1), y offset 4 (r >> 1):
-// hit[r] = can any point of block r have q <= limit?  q is convex, so over a block it is smallest either at the
-// centre (inside the block: 0) or on one of the two block edges that face the centre; along an edge it is a
-// parabola whose minimiser is clamped to the edge.  A block is treated as a continuous rectangle, which can only
-// add hits.  What the two columns and the two rows of blocks have in common is computed once; the parabolas are
-// evaluated in Horner form with fused multiply-adds.  inv_a, inv_c and limit: block_test_params.  NaNs count as
-// hits.
-__device__ __forceinline__ void ellipse_hits_quadrant(float2 mu, float4 co, float inv_a, float inv_c, float limit,
-                                                      float qx0, float qy0, bool (&hit)[4]) {
+// The sixteen 4x4 pixel blocks of the tile at (tile_x0, tile_y0): bit 4 k + r of the result is block r of quadrant k
+// (quadrant k at offset 8 (k & 1), 8 (k >> 1), block r in it at 4 (r & 1), 4 (r >> 1)): can any point of the block have
+// q <= limit?  q is convex, so over a block it is smallest either at the centre (inside the block: 0) or on one of the two
+// block edges that face the centre; along an edge it is a parabola whose minimiser is clamped to the edge.  A block is
+// treated as a continuous rectangle, which can only add hits.  What the four columns and the four rows of blocks have in
+// common is computed once; the parabolas are evaluated in Horner form with fused multiply-adds.  inv_a, inv_c and limit:
+// block_test_params.  NaNs count as hits.
+__device__ __forceinline__ uint32_t ellipse_hits_tile(float2 mu, float4 co, float inv_a, float inv_c, float limit,
+                                                      float tile_x0, float tile_y0) {
   const float two_b = 2.0f * co.y;
-  float lox[2], hix[2], dxc[2], t1[2], a1[2], b1[2];  // per column of blocks
-  float loy[2], hiy[2], dyc[2], t2[2], a2[2], b2[2];  // per row of blocks
+  uint32_t hits = 0u;  // (columns 2 h and 2 h + 1 of row d: bits 8 h + 2 d and the next)
+#pragma unroll 1
+  for (int h = 1; h >= 0; h--) {  // (loops: unrolled they take registers that the blend kernels do not have)
+    float lox[2], t1[2], a1[2], b1[2];
 #pragma unroll
-  for (int c = 0; c < 2; c++) {
-    lox[c] = (qx0 + (float)(4 * c)) - mu.x;
-    hix[c] = lox[c] + 3.0f;
-    dxc[c] = fminf(fmaxf(0.f, lox[c]), hix[c]);  // offset of the nearest column of the block
-    t1[c] = -co.y * dxc[c] * inv_c;              // where q is smallest along that column
-    a1[c] = co.x * dxc[c] * dxc[c];
-    b1[c] = two_b * dxc[c];
-    loy[c] = (qy0 + (float)(4 * c)) - mu.y;
-    hiy[c] = loy[c] + 3.0f;
-    dyc[c] = fminf(fmaxf(0.f, loy[c]), hiy[c]);  // offset of the nearest row of the block
-    t2[c] = -co.y * dyc[c] * inv_a;              // where q is smallest along that row
-    a2[c] = co.z * dyc[c] * dyc[c];
-    b2[c] = two_b * dyc[c];
-  }
+    for (int c = 0; c < 2; c++) {
+      lox[c] = (tile_x0 + (float)(8 * h + 4 * c)) - mu.x;
+      const float dxc = __builtin_amdgcn_fmed3f(0.f, lox[c], lox[c] + 3.0f);  // offset of the block's nearest column
+      t1[c] = -co.y * dxc * inv_c;                                            // where q is smallest along that column
+      a1[c] = co.x * dxc * dxc;
+      b1[c] = two_b * dxc;
+    }
+#pragma unroll 1
+    for (int d = 3; d >= 0; d--) {
+      const float loy = (tile_y0 + (float)(4 * d)) - mu.y;
+      const float hiy = loy + 3.0f;
+      const float dyc = __builtin_amdgcn_fmed3f(0.f, loy, hiy);  // offset of the block's nearest row
+      const float t2 = -co.y * dyc * inv_a;                      // where q is smallest along that row
+      const float a2 = co.z * dyc * dyc;
+      const float b2 = two_b * dyc;
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int c = r & 1, d = r >> 1;
-    const float dy1 = fminf(fmaxf(t1[c], loy[d]), hiy[d]);  // best point of the column x = dxc
-    const float q1 = __builtin_fmaf(__builtin_fmaf(co.z, dy1, b1[c]), dy1, a1[c]);
-    const float dx2 = fminf(fmaxf(t2[d], lox[c]), hix[c]);  // best point of the row y = dyc
-    const float q2 = __builtin_fmaf(__builtin_fmaf(co.x, dx2, b2[d]), dx2, a2[d]);
-    hit[r] = !(fminf(q1, q2) > limit);
+      for (int c = 1; c >= 0; c--) {
+        const float dy1 = __builtin_amdgcn_fmed3f(t1[c], loy, hiy);  // best point of the column x = dxc
+        const float q1 = __builtin_fmaf(__builtin_fmaf(co.z, dy1, b1[c]), dy1, a1[c]);
+        const float dx2 = __builtin_amdgcn_fmed3f(t2, lox[c], lox[c] + 3.0f);  // best point of the row y = dyc
+        const float q2 = __builtin_fmaf(__builtin_fmaf(co.x, dx2, b2), dx2, a2);
+        // (a hit is shifted in at bit 0, as the carry of hits + hits)
+        asm("v_cmp_ngt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"
+            : "+v"(hits)
+            : "v"(fminf(q1, q2)), "v"(limit)
+            : "vcc");
+      }
+    }
   }
+  // row d of columns 2 h, 2 h + 1 are blocks 2 (d & 1), 2 (d & 1) + 1 of quadrant 2 (d >> 1) + h
+  return (hits & 0xF00Fu) | ((hits & 0x00F0u) << 4) | ((hits & 0x0F00u) >> 4);
 }
 
 // ---- 4x4-pixel rows -------------------------------------------------------
