@@ -11,10 +11,11 @@
 //     forward kernel's own answer, 16 bits per instance, when the caller hands
 //     them on; otherwise the inflated alpha >= 1/255 ellipse is tested again)
 //     are compacted into a ring; the others' records are zero.
-//   * 128 of them at a time are staged in LDS and worked on 64 at a time: a
-//     wave compacts, for each of its rows, the slots that touch the row's
-//     block into a byte list, and the four rows walk their own lists
-//     concurrently, four entries per pass.
+//   * Out of a window of up to 256 waiting Gaussians every wave picks those
+//     that touch its own quadrant, stages up to SLOTS of them in LDS, compacts
+//     for each of its rows the slots that touch the row's block into a byte
+//     list, and the four rows walk their own lists concurrently, four entries
+//     per pass.  The window ends where a wave has no slot left.
 //   * A pass has two halves.  In the first, lane = pixel: the recurrence over
 //     the four entries, which leaves w = alpha T and q = G dL/dalpha per
 //     (entry, pixel).  In the second, lane e of a quad works for entry e: the
@@ -26,7 +27,8 @@
 //   * The sixteen sums of an entry go into the wave's own accumulator in LDS,
 //     row after row, with a plain read-add-write (no atomics: an LDS float
 //     atomic costs about three cycles per active lane here).
-//   * After 64 slots the four waves' accumulators are added in wave order and
+//   * After the window the accumulators of the waves that have staged a
+//     Gaussian are added in wave order and
 //     every (tile, Gaussian) instance's sums are stored as one 64-byte record,
 //     at the instance's index in emission order (the order key emission wrote
 //     them: all instances of a Gaussian are consecutive there).  No global
@@ -37,19 +39,26 @@
 // reference issues 16 global float atomics per pixel and Gaussian,
 // cuda_rasterizer/backward.cu:510-563.)
 //
-// What bounds it: vector issue (busy share 0.8 at 1 M Gaussians, 1152x864: some 90
-// vector instructions per entry of a row; 125 when every pass took one entry
-// and reduced its sixteen sums over the sixteen lanes of the row).  Before and
-// after: 256 -> 229 us there, 757 -> 537 us for 4 M Gaussians from the air,
-// 1117 -> 904 us for 10 M at street level, 129 -> 110 us for 300 k without
-// geometry channels.  The matrix cores take what contracts an operand that all
+// What bounds it: the vector ALU, which the matrix instructions share (a
+// 4x4x1 one takes the time of five additions).  A pass costs some 770 cycles of
+// it and 16 matrix instructions, about 17 of them a wave at 1 M Gaussians,
+// 1152x864; the steps between the walks a fifth of the whole.  With the staging
+// shared by the four waves (batches of 128, 64 of them walked at a time) there
+// were 13 barriers per 256 entries, three or four now, lists four times shorter
+// and 12 % more passes.  Before and after: 208 -> 197 us there, 491 -> 464 us for
+// 4 M Gaussians from the air, 567 -> 549 us for 10 M at street level, 104 -> 96 us
+// for 300 k without geometry channels.  Four workgroups a CU with 64 slots, or
+// five with 48: 464 and 522 us at 4 M with geometry channels, whose 95 registers
+// would spill with five; without them 56 slots and five (96 us against 106).  The
+// accumulators' reads a pass ahead of their use gain nothing.
+// The matrix cores take what contracts an operand that all
 // entries or all pixels share; the recurrence itself is a serial chain per
 // pixel.
 //
 // The per-pixel arithmetic follows the CPU statement's operation for operation
 // in everything that decides what counts (the exponent, alpha, the tests) and
 // in the transmittance, with these exceptions after that: the order in which
-// pixels are summed (fixed for thin Gaussians, see `exact`); the factors that
+// pixels are summed (fixed for thin Gaussians, see `aligned`); the factors that
 // are constant per Gaussian (W/2, H/2, the opacity, the conic and -1/2 of the
 // geometric gradients), which multiply the sums instead of every term; and the
 // blend of everything behind a Gaussian, background included, which the
@@ -67,14 +76,13 @@ namespace gs {
 
 namespace {
 
-constexpr int BATCH = GS_TILE_PIX / 2;  // Gaussians staged in LDS per round
+constexpr int WINDOW = GS_TILE_PIX;  // waiting Gaussians that are looked at together
+constexpr int PENDING = 512;         // ring of list positions that wait: at most WINDOW - 1 + GS_TILE_PIX of them
 constexpr int RUN = GS_WAVE;        // consecutive positions of a tile's list that stay together (see the order of the sums)
 constexpr float THIN = 0.8f;        // squared correlation b * b / (a * c) from which a Gaussian counts as thin
-constexpr int SUB = GS_WAVE;        // Gaussians whose sums are in the accumulators at a time: one ballot's worth
-constexpr int PENDING = 512;        // ring of list positions that wait to be staged: at most BATCH - 1 + GS_TILE_PIX of them
 constexpr int GROUP = 4;            // entries of a list handled per pass of the walk, one per lane of a quad
 constexpr int WAVES = GS_TILE_PIX / GS_WAVE;
-static_assert(SUB * 4 == GS_TILE_PIX, "a thread hands over a quarter of one record of the sub-batch");
+constexpr uint32_t NO_SLOT = 255u;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -87,7 +95,7 @@ __device__ __forceinline__ float quad_lane(float v) {
 // HITS: the forward blend left, per sorted instance, which 4x4 blocks of the tile the Gaussian can touch; without
 // it the same test is made again here.
 template <bool RENDER_GEO, bool HITS>
-__global__ void __launch_bounds__(GS_TILE_PIX) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ void __launch_bounds__(GS_TILE_PIX) __attribute__((amdgpu_waves_per_eu(RENDER_GEO ? 4 : 5)))
 render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__ point_list, int W, int H, float fx,
                   float fy, const float* __restrict__ bg, const float2* __restrict__ means2D,
                   const float4* __restrict__ conic_opacity, const float* __restrict__ rgb,
@@ -103,22 +111,31 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   const float4* packed = (packed_records != nullptr && (packed_valid == nullptr || *packed_valid != 0u))
                              ? packed_records : nullptr;
   constexpr bool render_geo = RENDER_GEO;
-  __shared__ uint32_t s_emis[BATCH];
+  // The Gaussians a wave can stage at a time: as many as the LDS holds with four or five workgroups.
+  constexpr int SLOTS = RENDER_GEO ? 64 : 56;
+  constexpr int LIST_BYTES = SLOTS + RUN;  // a row's list: its entries, and what keeps the places of a run that began earlier
+  static_assert(SLOTS <= GS_WAVE && SLOTS % GROUP == 0 && LIST_BYTES % GROUP == 0, "a lane per slot, whole words of lists");
+  static_assert(LIST_BYTES <= 2 * GS_WAVE, "a wave clears its four lists in two rounds");
+  // What a wave has staged.  (Slot SLOTS: what an entry behind the end of a list refers to, a Gaussian of opacity 0.)
+  __shared__ float4 s_xyp[WAVES][SLOTS + 1];  // centre x, y; as bits: the position in the list; 1 thin, 2 exact
+  __shared__ float4 s_co[WAVES][SLOTS + 1];   // the conic as (A, 2 B, C), and -1/2 of the opacity
+  // colour, then the five geometry channels: eight floats per Gaussian, read as two 16-byte words
+  __shared__ float4 s_chan[WAVES][SLOTS + 1][RENDER_GEO ? 2 : 1];
+  // accumulators: word 4 slot + (part ^ (slot / 4 & 3)) holds sums 4 part .. 4 part + 3 of a slot, so that
+  // neither the walk's accesses (a part of consecutive slots) nor the hand-over's pile up on a few banks
+  __shared__ float4 s_acc[WAVES][4 * SLOTS];
+  // the four rows' lists of every wave: the slots that can touch the row's block and are not
+  // behind its deepest contributor, one byte each, in walking order; bytes behind a list's end are SLOTS
+  __shared__ uint32_t s_idx[WAVES][4][LIST_BYTES / 4];
+  // the Gaussians that wait to be staged: position in the list, blocks touched
   __shared__ int s_pend[PENDING];
   __shared__ uint16_t s_pend_hits[PENDING];
   __shared__ int s_found[2][WAVES];
-  // (slot BATCH: what an entry behind the end of a list refers to, a Gaussian of opacity 0)
-  __shared__ float4 s_xyp[BATCH + 1];  // centre x, y; the position in the tile's list, as bits; unused
-  __shared__ float4 s_co[BATCH + 1];   // the conic as (A, 2 B, C), and -1/2 of the opacity
-  __shared__ uint16_t s_hits[BATCH];
-  // colour, then the five geometry channels: eight floats per Gaussian, read as two 16-byte words
-  __shared__ float4 s_chan[BATCH + 1][RENDER_GEO ? 2 : 1];
-  // one accumulator per wave: word 4 slot + (part ^ (slot / 4 & 3)) holds sums 4 part .. 4 part + 3 of a slot, so that
-  // neither the walk's accesses (a part of consecutive slots) nor the hand-over's pile up on a few banks
-  __shared__ float4 s_acc[WAVES][4 * SUB];
-  // the four rows' lists of every wave: the slots of the batch that can touch the row's block and are not
-  // behind its deepest contributor, one byte each, in walking order; bytes behind a list's end are BATCH
-  __shared__ __attribute__((aligned(16))) uint32_t s_idx[GS_TILE_PIX / GS_WAVE][4][2 * SUB / 4];
+  // which slot each wave has given a Gaussian of the window (byte w of a word: wave w's, or NO_SLOT); a wave's own slots:
+  // place in the window, rows touched << 8; how much of the window the wave has slots for
+  __shared__ uint32_t s_place[WINDOW];
+  __shared__ uint16_t s_own[WAVES][SLOTS];
+  __shared__ int s_limit[WAVES];
   __shared__ int4 s_row_last[WAVES];  // the deepest contributor of every row
 
   const int tid = threadIdx.x;
@@ -233,25 +250,20 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     odd = gs_ballot(top != 0.f) != 0ull;
   }
 
-  // thread tid hands over components 4*part .. 4*part+3 of the sub-batch's slot tid / 4 and clears them
-  const int my_slot = tid >> 2, my_part = tid & 3;
-  const int my_word = 4 * my_slot + (my_part ^ ((my_slot >> 2) & 3));
-#pragma unroll
-  for (int w = 0; w < WAVES; w++) s_acc[w][my_word] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (tid == 0) {
+  if (lane == 0) {
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-    s_xyp[BATCH] = z;
-    s_co[BATCH] = z;
+    s_xyp[wave][SLOTS] = z;
+    s_co[wave][SLOTS] = z;
 #pragma unroll
-    for (int h = 0; h < (RENDER_GEO ? 2 : 1); h++) s_chan[BATCH][h] = z;
+    for (int h = 0; h < (RENDER_GEO ? 2 : 1); h++) s_chan[wave][SLOTS][h] = z;
   }
   const uint32_t quad_shift = 8u * (uint32_t)(lane & 3), quad = (uint32_t)(rt.l16 >> 2);
   const float block_y0 = (float)(py & ~3u);  // the first of the four pixels of a quad
 
-  // Positions are 0-based indices into the tile's list; the walk goes down from the tile's deepest contributor.  A Gaussian
-  // that touches no row's block in front of the row's deepest contributor is not staged: its record is zero.  (Of a
-  // list of thousands of small Gaussians most touch nothing: a street-level tile of 17 000 entries stages 4 500.  Walked
-  // entry by entry it took 1.1 ms, longer than all other tiles of that view together.)
+  // Positions are 0-based indices into the tile's list; the walk goes down from the tile's deepest contributor.  Every wave
+  // picks, out of a window of positions, the Gaussians that touch one of its rows in front of the row's deepest contributor,
+  // a quarter of the list where Gaussians are small, stages those and walks them; the window ends where a wave has no slot
+  // left.  A position that no wave has taken has a record of zeros.
   auto hits_at = [&](int pos) { return pos >= 0 ? (uint32_t)block_hits[range.x + (uint32_t)pos] : 0u; };
   auto hits_by_test = [&](int pos) {
     if (pos < 0) return 0u;
@@ -263,12 +275,17 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
     return ellipse_hits_tile(xy, co, cp.x, cp.y, cp.z, tile_x0, tile_y0);
   };
+  auto sync_wave = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
   int unscanned = tile_last;  // positions below this one have not been looked at
   uint32_t head = 0u, tail = 0u, parity = 0u;
-  uint32_t carried[4] = {0u, 0u, 0u, 0u}, carried_run = 0xFFFFFFFFu;  // see `exact` below
   uint32_t hits_next = HITS ? hits_at(unscanned - 1 - tid) : 0u;  // (fetched one step ahead)
+  uint32_t carried[4] = {0u, 0u, 0u, 0u}, carried_run = 0xFFFFFFFFu;  // see `aligned` below
   for (;;) {
-    while (tail - head < (uint32_t)BATCH && unscanned > 0) {
+    while (tail - head < (uint32_t)WINDOW && unscanned > 0) {
       const int pos = unscanned - 1 - tid;
       uint32_t hits = HITS ? hits_next : hits_by_test(pos);
       unscanned = max(unscanned - GS_TILE_PIX, 0);
@@ -304,97 +321,121 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
       }
       parity ^= 1u;  // (the counts are rewritten two barriers later)
     }
-    const int count = (int)min((uint32_t)BATCH, tail - head);
-    if (count == 0) break;
+    const int waiting = (int)min((uint32_t)WINDOW, tail - head);
+    if (waiting == 0) break;
     __syncthreads();
-    // (the barrier that ended the previous batch's last sub-batch has let every wave finish with the staged data)
-    if (tid < count) {
-      const uint32_t at = (head + (uint32_t)tid) & (PENDING - 1);
-      const int pos = s_pend[at];
-      const uint32_t k_sorted = range.x + (uint32_t)pos;
-      const uint32_t g = point_list[k_sorted];
-      // A Gaussian's operands: one 64-byte record where the forward call packed them (a single line of memory,
-      // every byte of it used), else gathered from the four arrays.  (Each route loads and then stages by itself:
-      // with the loaded values merged across the two routes the compiler splits the gathers into single words.)
-      auto stage = [&](const float2 xy, const float4 co, const float c0, const float c1, const float c2,
-                       const float (&m)[GS_N_MAP]) {
-        s_emis[tid] = emission_sorted[k_sorted];
-        s_co[tid] = make_float4(co.x, 2.0f * co.y, co.z, -0.5f * co.w);
-        s_hits[tid] = s_pend_hits[at];
-        s_xyp[tid] = make_float4(xy.x, xy.y, __int_as_float(pos), 0.f);
-        if (render_geo) s_chan[tid][RENDER_GEO ? 1 : 0] = make_float4(m[1], m[2], m[3], m[4]);
-        s_chan[tid][0] = make_float4(c0, c1, c2, m[0]);
-      };
-      if (packed != nullptr) {
-        const float4* rec = packed + 4 * (size_t)g;
-        const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
-        float m[GS_N_MAP] = {r2.y, r2.z, r2.w, 0.f, 0.f};
-        if (render_geo) {
-          const float4 r3 = rec[3];
-          m[3] = r3.x, m[4] = r3.y;
-        }
-        stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
-      } else {
-        const float2 xy = means2D[g];
-        const float4 co = conic_opacity[g];
-        const float c0 = rgb[3 * (size_t)g], c1 = rgb[3 * (size_t)g + 1], c2 = rgb[3 * (size_t)g + 2];
-        float m[GS_N_MAP] = {0.f, 0.f, 0.f, 0.f, 0.f};
-        if (render_geo) {
+    // the wave's slots in the window
+    uint32_t found = 0u;
+    {
+      int limit = waiting;
 #pragma unroll
-          for (int ch = 0; ch < GS_N_MAP; ch++) m[ch] = all_map[5 * (size_t)g + ch];
-        }
-        stage(xy, co, c0, c1, c2, m);
+      for (int k = 0; k < WINDOW / GS_WAVE; k++) {
+        const int at = k * GS_WAVE + lane;
+        const uint32_t rows = at < waiting ? (uint32_t)s_pend_hits[(head + (uint32_t)at) & (PENDING - 1)] >> (4 * wave) & 15u : 0u;
+        const uint64_t take_m = gs_ballot(rows != 0u);
+        const uint32_t slot = __builtin_amdgcn_mbcnt_hi((uint32_t)(take_m >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)take_m, found));
+        reinterpret_cast<uint8_t*>(s_place)[4 * at + wave] = (uint8_t)(rows != 0u ? slot : NO_SLOT);
+        if (rows != 0u && slot < (uint32_t)SLOTS) s_own[wave][slot] = (uint16_t)((uint32_t)at | rows << 8);
+        const uint64_t over_m = gs_ballot(rows != 0u && slot == (uint32_t)SLOTS);
+        if (over_m != 0ull) limit = k * GS_WAVE + (int)__builtin_ctzll(over_m);
+        found += (uint32_t)__popcll(take_m);
       }
+      if (lane == 0) s_limit[wave] = limit;
+      found = min(found, (uint32_t)SLOTS);
     }
-    head += (uint32_t)count;
     __syncthreads();
+    int length = waiting;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) length = min(length, s_limit[w]);
+    length = __builtin_amdgcn_readfirstlane(length);
+    // lane = slot
+    const uint32_t own = (uint32_t)lane < found ? (uint32_t)s_own[wave][lane] : (uint32_t)WINDOW;
+    const bool have = (uint32_t)lane < found && (int)(own & 255u) < length;
+    const int count = (int)__popcll(gs_ballot(have));
+    if (count != 0) {
+      const int pos = s_pend[(head + (own & 255u)) & (PENDING - 1)];
+      const uint32_t nibble = have ? own >> 8 : 0u;
+      bool is_thin = false;
+      if (have) {
+        const uint32_t g = point_list[range.x + (uint32_t)pos];
+        // A Gaussian's operands: one 64-byte record where the forward call packed them (a single line of memory,
+        // every byte of it used), else gathered from the four arrays.  (Each route loads and then stages by itself:
+        // with the loaded values merged across the two routes the compiler splits the gathers into single words.)
+        auto stage = [&](const float2 xy, const float4 co, const float c0, const float c1, const float c2,
+                         const float (&m)[GS_N_MAP]) {
+          s_co[wave][lane] = make_float4(co.x, 2.0f * co.y, co.z, -0.5f * co.w);
+          is_thin = !(co.y * co.y < THIN * co.x * co.z);
+          s_xyp[wave][lane] =
+              make_float4(xy.x, xy.y, __int_as_float(pos),
+                          __int_as_float(!is_thin ? 0 : ((0xE880u >> nibble) & 1u) != 0u ? 2 : 1));
+          if (render_geo) s_chan[wave][lane][RENDER_GEO ? 1 : 0] = make_float4(m[1], m[2], m[3], m[4]);
+          s_chan[wave][lane][0] = make_float4(c0, c1, c2, m[0]);
+        };
+        if (packed != nullptr) {
+          const float4* rec = packed + 4 * (size_t)g;
+          const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+          float m[GS_N_MAP] = {r2.y, r2.z, r2.w, 0.f, 0.f};
+          if (render_geo) {
+            const float4 r3 = rec[3];
+            m[3] = r3.x, m[4] = r3.y;
+          }
+          stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
+        } else {
+          const float2 xy = means2D[g];
+          const float4 co = conic_opacity[g];
+          const float c0 = rgb[3 * (size_t)g], c1 = rgb[3 * (size_t)g + 1], c2 = rgb[3 * (size_t)g + 2];
+          float m[GS_N_MAP] = {0.f, 0.f, 0.f, 0.f, 0.f};
+          if (render_geo) {
+#pragma unroll
+            for (int ch = 0; ch < GS_N_MAP; ch++) m[ch] = all_map[5 * (size_t)g + ch];
+          }
+          stage(xy, co, c0, c1, c2, m);
+        }
+      }
+      // (every wave has read the accumulators of the window before: the barrier at the end of the loop)
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (k * GS_WAVE + lane < 4 * SLOTS) s_acc[wave][k * GS_WAVE + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
 
-    for (int base = 0; base < count; base += SUB) {
-      // Per-row lists: lane = slot of the sub-batch; the lanes whose Gaussian counts for row r append their slot
+      // Per-row lists: the lanes whose Gaussian counts for row r append their slot
       // numbers to the row's list, in lane order (a lane's place is the number of set bits below its own).
       uint32_t passes;  // wave-uniform, like all that follows here: the longest of the four lists
-      bool exact, thin;
+      bool aligned;
       {
         uint32_t* const words = &s_idx[wave][0][0];
-        static_assert(sizeof(s_idx[0]) == 8 * GS_WAVE, "a wave clears its own lists, two words per lane");
-        *reinterpret_cast<uint2*>(words + 2 * lane) = make_uint2((uint32_t)BATCH * 0x01010101u, (uint32_t)BATCH * 0x01010101u);
-        const int jj = base + lane;
-        const int js = jj < count ? jj : BATCH;
-        const uint32_t nibble = jj < count ? (uint32_t)s_hits[jj] >> (4 * wave) & 15u : 0u;
+        words[lane] = (uint32_t)SLOTS * 0x01010101u;
+        if (GS_WAVE + lane < LIST_BYTES) words[GS_WAVE + lane] = (uint32_t)SLOTS * 0x01010101u;
         uint64_t hit_m[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) hit_m[r] = gs_ballot(((nibble >> r) & 1u) != 0u);
         auto list_row = [&](int r, uint64_t b, uint32_t from) {
           const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, from));
-          if (__builtin_amdgcn_inverse_ballot_w64(b)) reinterpret_cast<uint8_t*>(&s_idx[wave][r][0])[below] = (uint8_t)jj;
+          if (__builtin_amdgcn_inverse_ballot_w64(b)) reinterpret_cast<uint8_t*>(&s_idx[wave][r][0])[below] = (uint8_t)lane;
           return from + (uint32_t)__popcll(b);
         };
         // The gradient of a thin Gaussian's covariance is a small difference of its three conic sums: a change in how
         // they are rounded comes back multiplied by a c / (a c - b b), squared for scale and rotation.  Where a wave has
         // such a Gaussian its conic sums are taken in a fixed order (`thin`: the sixteen pixels of a row as a tree; and
         // `exact`, if three or four rows touch it: the rows by their places in the lists of a run of 64 positions, rows
-        // at the same place merged first), whatever else is staged or skipped.  Below THIN the factor is at most 25.
+        // at the same place merged first), whatever else is staged or skipped: its lists keep the places (`aligned`),
+        // and the passes that hold it take the sums in that order.  Below THIN the factor is at most 25.
         // That is the order of a kernel that takes one entry per pass and reduces its sums over the row's lanes.  On 16
         // scenes of 60 to 4000 Gaussians, a quarter of them thin, the covariance gradients of the thin ones are a relative
         // 7.9e-6 from float64 in this order, 7.9e-6 in that kernel and 8.9e-6 with the order left to the lists (12 of the
         // 16 worse); the conic gradients themselves are 2.1e-6 off in all three.
-        const float4 cq = s_co[js];
-        const float cq_b = 0.5f * cq.y;
-        const bool is_thin = !(cq_b * cq_b < THIN * cq.x * cq.z);
-        thin = gs_ballot(is_thin && nibble != 0u) != 0ull;
-        exact = gs_ballot(is_thin && ((0xE880u >> nibble) & 1u) != 0u) != 0ull;
-        const uint32_t run = (uint32_t)(tile_last - 1 - __float_as_int(s_xyp[js].z)) / RUN;
-        const int last_lane = (count - base < SUB ? count - base : SUB) - 1;
+        aligned = gs_ballot(is_thin && ((0xE880u >> nibble) & 1u) != 0u) != 0ull;
+        const uint32_t run = (uint32_t)(tile_last - 1 - pos) / RUN;
         const uint32_t first_run = (uint32_t)__builtin_amdgcn_readlane((int)run, 0);
-        const uint32_t last_run = (uint32_t)__builtin_amdgcn_readlane((int)run, last_lane);
-        if (!exact) {
+        const uint32_t last_run = (uint32_t)__builtin_amdgcn_readlane((int)run, count - 1);
+        if (!aligned) {
           const uint32_t l0 = list_row(0, hit_m[0], 0u), l1 = list_row(1, hit_m[1], 0u);
           const uint32_t l2 = list_row(2, hit_m[2], 0u), l3 = list_row(3, hit_m[3], 0u);
           passes = max(max(l0, l1), max(l2, l3));
         } else {
-          // (a run that began in an earlier sub-batch has `carried` entries per row there)
+          // (a run that began in an earlier window has `carried` entries per row there)
           const uint32_t least = min(min(carried[0], carried[1]), min(carried[2], carried[3]));
-          uint64_t todo = last_lane == SUB - 1 ? ~0ull : (1ull << (last_lane + 1)) - 1ull;
+          uint64_t todo = gs_ballot(have);
           passes = 0u;
           while (todo != 0ull) {
             const uint32_t this_run = (uint32_t)__builtin_amdgcn_readlane((int)run, (int)__builtin_ctzll(todo));
@@ -410,32 +451,32 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           }
         }
         passes = (uint32_t)__builtin_amdgcn_readfirstlane((int)passes);
-        const uint64_t last_m = gs_ballot(run == last_run);
+        const uint64_t last_m = gs_ballot(have && run == last_run);
 #pragma unroll
         for (int r = 0; r < 4; r++)
           carried[r] = (first_run == last_run && last_run == carried_run ? carried[r] : 0u) + (uint32_t)__popcll(hit_m[r] & last_m);
         carried_run = last_run;
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      sync_wave();
       for (uint32_t n = 0; n < passes; n += GROUP) {
         // Four entries of every row's list.  Lane e of each of the row's quads fetches entry e.
         const uint32_t word = s_idx[wave][row][n / GROUP];
         const uint32_t j_own = __builtin_amdgcn_ubfe(word, quad_shift, 8u);
-        const float4 xyp = s_xyp[j_own];
-        const float4 co = s_co[j_own];
+        const float4 xyp = s_xyp[wave][j_own];
+        const float4 co = s_co[wave][j_own];
+        const bool thin = gs_ballot(__float_as_int(xyp.w) > 0) != 0ull;
+        const bool exact = gs_ballot(__float_as_int(xyp.w) > 1) != 0ull;
         // S = sum_ch c_ch g_ch of every (entry, pixel): a contraction over the channels, of the entries' colours and the
         // pixels' upstream gradients.  Register e of lane p of a quad receives entry e at pixel p (one fused
         // multiply-add per channel, in channel order: the bits of the same chain of vector instructions).
         f32x4 S = {0.f, 0.f, 0.f, 0.f};
         {
-          const float4 c4 = s_chan[j_own][0];
+          const float4 c4 = s_chan[wave][j_own][0];
           S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.x, gpix[0], S, 0, 0, 0);
           S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.y, gpix[1], S, 0, 0, 0);
           S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.z, gpix[2], S, 0, 0, 0);
           if (render_geo) {
-            const float4 m4 = s_chan[j_own][RENDER_GEO ? 1 : 0];
+            const float4 m4 = s_chan[wave][j_own][RENDER_GEO ? 1 : 0];
             S = __builtin_amdgcn_mfma_f32_4x4x1f32(c4.w, gmap[0], S, 0, 0, 0);
             S = __builtin_amdgcn_mfma_f32_4x4x1f32(m4.x, gmap[1], S, 0, 0, 0);
             S = __builtin_amdgcn_mfma_f32_4x4x1f32(m4.y, gmap[2], S, 0, 0, 0);
@@ -548,9 +589,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // Quad k of a row now holds components 4 k .. 4 k + 3 of its entry e.  They go into the wave's own accumulator with
         // a plain read-add-write (the LDS accesses of a wave complete in order), one row after the other, since two rows
         // may be at the same Gaussian.  An LDS float atomic takes about three cycles per active lane.
-        const uint32_t a_slot = j_own - (uint32_t)base;
-        float4* const acc = &s_acc[wave][4u * (a_slot & (SUB - 1)) + (quad ^ ((a_slot >> 2) & 3u))];
-        uint64_t write_m = gs_ballot(j_own < (uint32_t)BATCH);
+        float4* const acc = &s_acc[wave][4u * j_own + (quad ^ ((j_own >> 2) & 3u))];
+        uint64_t write_m = gs_ballot(j_own < (uint32_t)SLOTS);
         if (exact) {
           const float own[4] = {sum[0], sum[1], sum[2], sum[3]};
 #pragma unroll
@@ -578,40 +618,44 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
             *acc = a;
           }
           turn_m <<= turn_shift;
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          sync_wave();
         }
       }
-      __syncthreads();
-      // a thread stores a quarter of a record: the four waves' sums of four components, added in wave order;
-      // it leaves zeros behind for the next sub-batch
-      {
-        float4 c = s_acc[0][my_word];
-#pragma unroll
-        for (int w = 1; w < WAVES; w++) {
-          const float4 o = s_acc[w][my_word];
-          c.x += o.x; c.y += o.y; c.z += o.z; c.w += o.w;
-        }
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) s_acc[w][my_word] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (base + my_slot < count) {
-          // (the sums are those of -2 q)
-          const float4 co = s_co[base + my_slot];
-          const float b = 0.5f * co.y;
-          if (my_part == 0) {  // mean2D x, y and their sums of absolute values
-            c = make_float4(-co.w * (co.x * c.x + b * c.y), -co.w * (b * c.x + co.z * c.y), c.z * fabsf(co.w),
-                            c.w * fabsf(co.w));
-          } else if (my_part == 1) {  // conic x, y, w; the fourth component is the opacity gradient itself
-            const float h = -0.5f * co.w;
-            c.x *= h; c.y *= h; c.z *= h;
-            c.w *= -0.5f;
-          }
-          instance_grads[4 * (size_t)s_emis[base + my_slot] + my_part] = c;
-        }
-      }
-      __syncthreads();
     }
+    __syncthreads();
+    // A thread stores a quarter of a record: the sums of four components of the waves that have the Gaussian, added in
+    // wave order.
+    const int part = tid & 3;
+    for (int at = tid >> 2; at < length; at += GS_TILE_PIX / 4) {
+      const uint32_t emission = emission_sorted[range.x + (uint32_t)s_pend[(head + (uint32_t)at) & (PENDING - 1)]];
+      const uint32_t places = s_place[at];
+      float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (places != 0xFFFFFFFFu) {
+        uint32_t staged = 0u;  // where the Gaussian is
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+          const uint32_t slot = places >> (8 * w) & 255u;
+          if (slot != NO_SLOT) {
+            const float4 o = s_acc[w][4u * slot + ((uint32_t)part ^ ((slot >> 2) & 3u))];
+            c.x += o.x; c.y += o.y; c.z += o.z; c.w += o.w;
+            staged = (uint32_t)(w * (SLOTS + 1)) + slot;
+          }
+        }
+        // (the sums are those of -2 q)
+        const float4 co = (&s_co[0][0])[staged];
+        const float b = 0.5f * co.y;
+        if (part == 0) {  // mean2D x, y and their sums of absolute values
+          c = make_float4(-co.w * (co.x * c.x + b * c.y), -co.w * (b * c.x + co.z * c.y), c.z * fabsf(co.w),
+                          c.w * fabsf(co.w));
+        } else if (part == 1) {  // conic x, y, w; the fourth component is the opacity gradient itself
+          const float h = -0.5f * co.w;
+          c.x *= h; c.y *= h; c.z *= h;
+          c.w *= -0.5f;
+        }
+      }
+      instance_grads[4 * (size_t)emission + part] = c;
+    }
+    head += (uint32_t)length;
   }
 }
 

@@ -62,3 +62,43 @@ def test_list_lengths(H, orc, n, thin, geo):
             continue
         assert torch.equal(got[k], again[k]), k
         assert H.rel_l2(got[k].cpu().numpy(), want) <= 1e-4, (k, H.rel_l2(got[k].cpu().numpy(), want))
+
+
+@pytest.mark.parametrize("n", [55, 56, 57, 63, 64, 65, 112, 113, 255, 256, 257, 321])
+@pytest.mark.parametrize("geo", [True, False])
+def test_every_wave_needs_every_slot(H, orc, n, geo):
+    # Gaussians that cover the whole image: every wave stages every entry, so the windows end at the waves' slots (56 or
+    # 64), and a run of 64 positions spans two of them
+    gen = torch.Generator().manual_seed(1000 + n)
+    r = lambda *s: torch.rand(*s, generator=gen)
+    W, Hh, tan = 33, 17, 0.5
+    means2D = (r(n, 2) * torch.tensor([float(W), float(Hh)])).numpy()
+    s1 = 40.0 + 20.0 * r(n)
+    s2 = s1 * torch.where(r(n) < 0.3, 0.3, 0.8)  # (correlations up to 0.83: some count as thin)
+    ang = r(n) * 3.14159
+    c, s = torch.cos(ang), torch.sin(ang)
+    i1, i2 = 1 / s1 ** 2, 1 / s2 ** 2
+    co = torch.stack([c * c * i1 + s * s * i2, c * s * (i1 - i2), s * s * i1 + c * c * i2, 0.01 + 0.01 * r(n)],
+                     1).float().numpy()
+    radii, depths, rgb = torch.ceil(3 * s1).int().numpy(), (r(n) * 10 + 1).numpy(), r(n, 3).numpy()
+    am = torch.randn(n, 5, generator=gen)
+    am[:, 2] = am[:, 2].abs() + 2.0
+    am = am.numpy()
+    gx, gy = H.grid(W, Hh)
+    cl = np.ones(gx * gy, bool)
+    bg = np.array([0.3, 0.6, 0.1], np.float32)
+    b = orc.bin_and_sort(radii, means2D, depths, cl, W, Hh)
+    f = orc.render_fwd(b["ranges"], b["point_list"], means2D, rgb, am, co, cl, bg, W, Hh, tan, tan, render_geo=geo)
+    gpix, gmap, gdep = (torch.randn(k, Hh, W, generator=gen).numpy() for k in (3, 5, 1))
+    ref = orc.render_bwd(b["ranges"], b["point_list"], means2D, co, rgb, am, f["out_all_map"], f["final_T"],
+                         f["n_contrib"], cl, bg, gpix, gmap, gdep, W, Hh, tan, tan, render_geo=geo)
+    got = H.render_bwd(n, W, Hh, tan, tan, H.dev(bg), H.as_u32(b["ranges"]), H.as_u32(b["point_list"]), H.dev(means2D),
+                       H.dev(co), H.dev(rgb), H.dev(am), H.dev(f["out_all_map"]), H.dev(f["final_T"]),
+                       H.as_u32(f["n_contrib"]), H.dev(cl), H.dev(gpix), H.dev(gmap), H.dev(gdep),
+                       H.as_u32(b["emission_sorted"]), H.as_u32(b["point_offsets"]), render_geo=geo)
+    # the bound of the test above (561 pixels here)
+    for k, want in (("dL_dmeans2D", ref["dL_dmeans2D"][:, :2]), ("dL_dmeans2D_abs", ref["dL_dmeans2D_abs"]),
+                    ("dL_dconic_opacity", ref["dL_dconic_opacity"]), ("dL_dcolors", ref["dL_dcolors"]),
+                    ("dL_dall_map", ref["dL_dall_map"])):
+        if k != "dL_dall_map" or geo:
+            assert H.rel_l2(got[k].cpu().numpy(), want) <= 1e-4, (k, H.rel_l2(got[k].cpu().numpy(), want))
