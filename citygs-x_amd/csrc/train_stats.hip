@@ -57,7 +57,7 @@ train_stats_kernel(IDX slots, int k, IDX Vk, IDX M, const uint8_t* __restrict__ 
 
 constexpr int STATS_ROWS = 256;         // anchors per workgroup, one thread each for the visibility mask
 constexpr int STATS_SEL_CHUNK = 1024;   // candidates per prefix of the selection mask
-constexpr int STATS_ITEMS = 8;          // candidates per thread and round
+constexpr int STATS_ITEMS = 4;          // candidates per thread and round
 constexpr int STATS_ROUND = GS_BLOCK_1D * STATS_ITEMS;
 constexpr int STATS_MAX_OFFSETS = 256;
 static_assert(STATS_ROWS == GS_BLOCK_1D && STATS_SEL_CHUNK == 16 * GS_WAVE, "a wave counts 1024 entries, 16 a lane");
@@ -114,7 +114,9 @@ train_stats_spine_kernel(uint32_t vis_chunks, uint32_t sel_chunks, uint32_t* vis
 // all of a thread's loads in flight at once.  The anchor's opacities are added from LDS in candidate order.
 // Bound by memory, most of it the lines of the two slot accumulators.  With the ranks written out by two scans and
 // one slot per thread, each waiting for six loads one after the other, the call took 139 us at 1 M anchors of 10
-// offsets (40 % visible, 60 % of those selected), 70 us now.
+// offsets (40 % visible, 60 % of those selected), 59 us now (33 with 5 offsets).  Eight candidates a thread, whose
+// registers leave five waves a SIMD, take 70 (42), six 68 (39), five 63 (36), three and two the same as four.  (The
+// accumulators asked for with the masks, before it is known which slots are hit: 60.)
 __global__ void __launch_bounds__(GS_BLOCK_1D)
 train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, uint32_t M,
                          const uint8_t* __restrict__ visible, const uint32_t* __restrict__ vis_prefix,
@@ -157,7 +159,7 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
   if (set) s_row[place] = row0 + tid;
   __syncthreads();
 
-  const uint32_t rows_per_round = STATS_ROUND / k;  // (at least 8)
+  const uint32_t rows_per_round = STATS_ROUND / k;  // (at least 4)
   for (uint32_t r0 = 0; r0 < rows; r0 += rows_per_round) {
     const uint32_t nr = min(rows_per_round, rows - r0), n = nr * k;
     const uint64_t c0 = ((uint64_t)vis0 + r0) * k;  // the round's first candidate
