@@ -269,7 +269,16 @@ int gs_visible_filter(int P, int M, int width, int height, const float* means3D,
                       const float* viewmatrix, const float* projmatrix, float tan_fovx, float tan_fovy,
                       int prefiltered, int* radii, int debug, gs_stream_t stream) {
   (void)M;
+  return gs_visible_filter_rows(P, 3, width, height, means3D, scales, scale_modifier, rotations, cov3D_precomp, viewmatrix,
+                                projmatrix, tan_fovx, tan_fovy, prefiltered, radii, debug, stream);
+}
+
+int gs_visible_filter_rows(int P, int scale_stride, int width, int height, const float* means3D, const float* scales,
+                           float scale_modifier, const float* rotations, const float* cov3D_precomp,
+                           const float* viewmatrix, const float* projmatrix, float tan_fovx, float tan_fovy,
+                           int prefiltered, int* radii, int debug, gs_stream_t stream) {
   (void)prefiltered;
+  GS_REQUIRE(scale_stride >= 3, "gs_visible_filter: rows of scales shorter than three");
   GS_REQUIRE(P >= 0 && width > 0 && height > 0, "gs_visible_filter: bad sizes");
   if (P == 0) return 0;
   GS_REQUIRE(means3D && viewmatrix && projmatrix && radii, "gs_visible_filter: null pointer");
@@ -277,7 +286,7 @@ int gs_visible_filter(int P, int M, int width, int height, const float* means3D,
              "gs_visible_filter: need scales+rotations or a precomputed 3D covariance");
   {
     StageScope _t("visible_filter", (hipStream_t)stream);
-    launch_visible_filter(P, means3D, scales, scale_modifier, rotations, cov3D_precomp, viewmatrix, projmatrix, width,
+    launch_visible_filter(P, means3D, scales, scale_stride, scale_modifier, rotations, cov3D_precomp, viewmatrix, projmatrix, width,
                         height, tan_fovx, tan_fovy, radii, (hipStream_t)stream);
   }
   return check_launch("visible_filter", (hipStream_t)stream, debug != 0);

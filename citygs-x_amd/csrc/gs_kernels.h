@@ -63,7 +63,7 @@ struct StageScope {
 
 int launch_preprocess_fwd(const PreprocessFwdArgs& a, hipStream_t stream);
 int launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t stream);
-int launch_visible_filter(int P, const float* means, const float* scales, float mod, const float* rots,
+int launch_visible_filter(int P, const float* means, const float* scales, int scale_stride, float mod, const float* rots,
                           const float* cov_pre, const float* V, const float* PM, int W, int H, float tanx,
                           float tany, int* radii, hipStream_t stream);
 int launch_mark_visible(int P, const float* means, const float* V, uint8_t* present, hipStream_t stream);

@@ -598,7 +598,7 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
 
 // cuda_rasterizer/forward.cu:545-620.
 __global__ void __launch_bounds__(GS_BLOCK_1D)
-visible_filter_kernel(int P, const float* __restrict__ means, const float* __restrict__ scales, float mod,
+visible_filter_kernel(int P, const float* __restrict__ means, const float* __restrict__ scales, int scale_stride, float mod,
                       const float* __restrict__ rots, const float* __restrict__ cov_pre,
                       const float* __restrict__ Vg, const float* __restrict__ PMg, int W, int H, float tanx,
                       float tany, float fx, float fy, uint32_t gx, uint32_t gy, int* __restrict__ radii) {
@@ -609,7 +609,8 @@ visible_filter_kernel(int P, const float* __restrict__ means, const float* __res
   const float mean[3] = {means[3 * (size_t)i], means[3 * (size_t)i + 1], means[3 * (size_t)i + 2]};
   float sc[3] = {0.f, 0.f, 0.f}, q[4] = {0.f, 0.f, 0.f, 0.f};
   if (!cov_pre) {
-    sc[0] = scales[3 * (size_t)i]; sc[1] = scales[3 * (size_t)i + 1]; sc[2] = scales[3 * (size_t)i + 2];
+    const float* s = scales + (size_t)scale_stride * i;
+    sc[0] = s[0]; sc[1] = s[1]; sc[2] = s[2];
     q[0] = rots[4 * (size_t)i]; q[1] = rots[4 * (size_t)i + 1]; q[2] = rots[4 * (size_t)i + 2];
     q[3] = rots[4 * (size_t)i + 3];
   }
@@ -995,7 +996,7 @@ int launch_preprocess_fwd(const PreprocessFwdArgs& a, hipStream_t stream) {
   return 0;
 }
 
-int launch_visible_filter(int P, const float* means, const float* scales, float mod, const float* rots,
+int launch_visible_filter(int P, const float* means, const float* scales, int scale_stride, float mod, const float* rots,
                           const float* cov_pre, const float* V, const float* PM, int W, int H, float tanx,
                           float tany, int* radii, hipStream_t stream) {
   if (P <= 0) return 0;
@@ -1003,7 +1004,7 @@ int launch_visible_filter(int P, const float* means, const float* scales, float 
   const float fy = H / (2.0f * tany);
   const float fx = W / (2.0f * tanx);
   const int blocks = (P + GS_BLOCK_1D - 1) / GS_BLOCK_1D;
-  hipLaunchKernelGGL(visible_filter_kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, P, means, scales, mod, rots,
+  hipLaunchKernelGGL(visible_filter_kernel, dim3(blocks), dim3(GS_BLOCK_1D), 0, stream, P, means, scales, scale_stride, mod, rots,
                      cov_pre, V, PM, W, H, tanx, tany, fx, fy, gx, gy, radii);
   return 0;
 }

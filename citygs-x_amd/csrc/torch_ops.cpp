@@ -167,9 +167,42 @@ py::tuple preprocess_backward(const Tensor& radii, const OptTensor& cov3D_, cons
   return py::make_tuple(dmeans, dscales, drot, dL_dsh, dopacity);
 }
 
+// What the caller passes for "not given": None or an empty tensor, of whatever type.
+OptTensor given(const OptTensor& t) { return t.has_value() && t->numel() != 0 ? t : OptTensor(); }
+
+// Radii only.  Scales may be the first columns of wider rows, as the anchor model holds them: they are read where they lie.
+Tensor visible_filter(const Tensor& means3D_, const OptTensor& scales_, const OptTensor& rotations_,
+                      float scale_modifier, const OptTensor& cov3D_, const Tensor& viewmatrix, const Tensor& projmatrix,
+                      float tan_fovx, float tan_fovy, int height, int width, bool prefiltered, bool debug,
+                      uintptr_t stream) {
+  const at::AutoDispatchBelowADInplaceOrView no_grad;  // (a copy made here is no part of a graph)
+  const Tensor means3D = f32c(means3D_, "means3D");
+  const int64_t P = means3D.size(0);
+  const Options o(means3D.device());
+  const c10::DeviceGuard guard(means3D.device());
+  Tensor radii = at::empty({P}, o.i32);
+  if (P == 0) return radii;
+  OptTensor scales = given(scales_);
+  int64_t stride = 3;
+  if (scales.has_value()) {
+    const Tensor& s = *scales;
+    const bool in_place = s.scalar_type() == at::kFloat && s.is_cuda() && s.dim() == 2 && s.size(0) == P && s.size(1) == 3 &&
+                          s.stride(1) == 1 && s.stride(0) >= 3 && s.stride(0) <= 1024;
+    if (in_place) stride = s.stride(0);
+    else scales = f32c(s, "scales");
+  }
+  const Tensor rot = f32c(given(rotations_), "rotations"), cov = f32c(given(cov3D_), "cov3D_precomp");
+  const Tensor vm = f32c(viewmatrix, "viewmatrix"), pm = f32c(projmatrix, "projmatrix");
+  check(gs_visible_filter_rows((int)P, (int)stride, width, height, ptr(means3D), scales ? ptr(*scales) : nullptr,
+                               scale_modifier, ptr(rot), ptr(cov), ptr(vm), ptr(pm), tan_fovx, tan_fovy, prefiltered,
+                               ptr<int>(radii), debug, stream_of(stream)),
+        "rasterize_aussians_filter");
+  return radii;
+}
+
 py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& means2D_, const Tensor& depths_,
                          const Tensor& radii_, const Tensor& conic_opacity, const Tensor& rgb, const Tensor& locally,
-                         float focal_x, float focal_y, const OptTensor& all_map, bool geo, bool debug,
+                         float tan_fovx, float tan_fovy, const OptTensor& all_map, bool geo, bool debug,
                          bool want_max_weight_depth, bool timing, int small_limit, int block_records,
                          int64_t expected_instances, int expected_longest_list, const OptTensor& blend_records,
                          uintptr_t stream) {
@@ -204,6 +237,8 @@ py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& m
   options.blend_records = blend_records.has_value() ? ptr(*blend_records) : nullptr;
   gs_render_result result = {};
   result.struct_bytes = sizeof(result);
+  // fp32 arithmetic, as `H / (2.0f * tan_fovy)` at rasterize_points.cu:328-329
+  const float focal_x = (float)W / (2.0f * tan_fovx), focal_y = (float)H / (2.0f * tan_fovy);
   int num_rendered = 0, status;
   float elapsed = 0.f;
   {
@@ -465,6 +500,7 @@ py::tuple visible_rows_backward(const Tensor& rank, int64_t k, const std::vector
 PYBIND11_MODULE(gsrast_ops, m) {
   m.def("preprocess_forward", &preprocess_forward);
   m.def("preprocess_backward", &preprocess_backward);
+  m.def("visible_filter", &visible_filter);
   m.def("render_forward", &render_forward);
   m.def("render_backward", &render_backward);
   m.def("ssim_l1_forward", &ssim_l1_forward);

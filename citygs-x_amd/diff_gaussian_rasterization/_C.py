@@ -224,12 +224,9 @@ def render_gaussians_ex(background, image_height, image_width, means2D, depths, 
     # (small_limit, block_records) for this call only: how the per-tile lists are built (a test hook)
     limits = args.get("tile_sort_limits") if isinstance(args, dict) else None
     small_limit, block_records = limits if limits is not None else (-1, -1)
-    # fp32 arithmetic, as `H / (2.0f * tan_fovy)` at rasterize_points.cu:328-329
-    focal_y = np.float32(H) / (np.float32(2.0) * np.float32(tan_fovy))
-    focal_x = np.float32(W) / (np.float32(2.0) * np.float32(tan_fovx))
     (num_rendered, out_color, n_render, n_consider, n_contrib, out_observe, out_all_map, out_plane_depth, geom, binning,
      img, longest_list, binning_capacity, launched_ahead, elapsed, mwd) = _ops.render_forward(
-        background, H, W, means2D, depths, radii, conic_opacity, rgb, compute_locally, float(focal_x), float(focal_y),
+        background, H, W, means2D, depths, radii, conic_opacity, rgb, compute_locally, float(tan_fovx), float(tan_fovy),
         all_map if render_geo else None, bool(render_geo), bool(debug), want_mwd, _want_timing(args), int(small_limit),
         int(block_records), int(expected_instances), int(expected_longest_list), blend_records, _n.stream_handle(dev))
     _record_time(args, "forward_render_time", elapsed)
@@ -270,21 +267,9 @@ def rasterize_aussians_filter(means3D, scales, rotations, scale_modifier, cov3D_
     """rasterize_points.cu:865-930 (the misspelt name is the reference's)."""
     if means3D.ndimension() != 2 or means3D.size(1) != 3:
         raise RuntimeError("means3D must have dimensions (num_points, 3)")
-    means3D = _f32c(means3D, "means3D")
-    dev = means3D.device
-    P = means3D.shape[0]
-    radii = torch.empty(P, dtype=torch.int32, device=dev)
-    if P != 0:
-        sc = _f32c(scales, "scales") if scales is not None and scales.numel() else None
-        rot = _f32c(rotations, "rotations") if rotations is not None and rotations.numel() else None
-        cov = _f32c(cov3D_precomp, "cov3D_precomp") if cov3D_precomp is not None and cov3D_precomp.numel() else None
-        vm, pm = _f32c(viewmatrix, "viewmatrix"), _f32c(projmatrix, "projmatrix")
-        with torch.cuda.device(dev):
-            _n.check(_lib.gs_visible_filter(P, 0, int(image_width), int(image_height), _ptr(means3D), _ptr(sc),
-                                            float(scale_modifier), _ptr(rot), _ptr(cov), _ptr(vm), _ptr(pm),
-                                            float(tan_fovx), float(tan_fovy), int(bool(prefiltered)), _ptr(radii),
-                                            int(bool(debug)), _stream(dev)), "rasterize_aussians_filter")
-    return radii
+    return _ops.visible_filter(means3D, scales, rotations, float(scale_modifier), cov3D_precomp, viewmatrix, projmatrix,
+                               float(tan_fovx), float(tan_fovy), int(image_height), int(image_width), bool(prefiltered),
+                               bool(debug), _n.stream_handle(means3D.device))
 
 
 def build_all_map(means3D, scales, rotations, viewmatrix, campos):

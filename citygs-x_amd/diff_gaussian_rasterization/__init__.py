@@ -200,9 +200,9 @@ class _PreprocessGaussians(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_means2D, grad_rgb, grad_conic_opacity, grad_radii, grad_depths):
         rs = ctx.raster_settings
-        means3D, scales, rotations, sh, radii, cov3D, clamped = ctx.saved_tensors[:7]
+        means3D, scales, rotations, sh, radii, cov3D, clamped, *ddir = ctx.saved_tensors
         grad_all_map = ctx.channel_gradients.take() if ctx.channel_gradients is not None else None
-        ddir = ctx.saved_tensors[7] if ctx.has_ddir else None
+        ddir = ddir[0] if ctx.has_ddir else None
         P = means3D.shape[0]
         if grad_means2D is None:
             grad_means2D = means3D.new_zeros(P, 2)
@@ -397,16 +397,9 @@ class GaussianRasterizer(nn.Module):
 
     def visible_filter(self, means3D, scales=None, rotations=None, cov3D_precomp=None):
         rs = self.raster_settings
-        if scales is None:
-            scales = torch.Tensor([])
-        if rotations is None:
-            rotations = torch.Tensor([])
-        if cov3D_precomp is None:
-            cov3D_precomp = torch.Tensor([])
-        with torch.no_grad():
-            return _C.rasterize_aussians_filter(means3D, scales, rotations, rs.scale_modifier, cov3D_precomp,
-                                                rs.viewmatrix, rs.projmatrix, rs.tanfovx, rs.tanfovy, rs.image_height,
-                                                rs.image_width, rs.prefiltered, rs.debug)
+        return _C.rasterize_aussians_filter(means3D, scales, rotations, rs.scale_modifier, cov3D_precomp, rs.viewmatrix,
+                                            rs.projmatrix, rs.tanfovx, rs.tanfovy, rs.image_height, rs.image_width,
+                                            rs.prefiltered, rs.debug)
 
     def render_gaussians(self, means2D, means2D_abs, conic_opacity, rgb, all_map, depths, radii, compute_locally,
                          extended_compute_locally, cuda_args=None):

@@ -105,7 +105,8 @@ def _visible_rows(mask, anchor, feat, offsets, scaling, want_index):
 
 def _linear_pair(seq):
     """(W1, b1, W2, b2) of a Sequential(Linear, ReLU, Linear[, activation]) (scene/gaussian_model.py:131-149)."""
-    return seq[0].weight, seq[0].bias, seq[2].weight, seq[2].bias
+    first, second = seq[0], seq[2]
+    return first.weight, first.bias, second.weight, second.bias
 
 
 def generate_neural_gaussians(viewpoint_camera, pc, visible_mask=None, is_training=False, ape_code=-1):

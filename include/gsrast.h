@@ -56,6 +56,13 @@ int gs_visible_filter(int P, int M, int width, int height, const float* means3D,
                       const float* viewmatrix, const float* projmatrix, float tan_fovx, float tan_fovy,
                       int prefiltered, int* radii, int debug, gs_stream_t stream);
 
+/* The same with scales read from rows of scale_stride floats (>= 3), of which the
+ * first three are the scales; gs_visible_filter has rows of three. */
+int gs_visible_filter_rows(int P, int scale_stride, int width, int height, const float* means3D, const float* scales,
+                           float scale_modifier, const float* rotations, const float* cov3D_precomp,
+                           const float* viewmatrix, const float* projmatrix, float tan_fovx, float tan_fovy,
+                           int prefiltered, int* radii, int debug, gs_stream_t stream);
+
 /* Replaces Rasterizer::preprocessForward (CR/rasterizer.h:61-84,
  * CR/rasterizer_impl.cu:336-425).  Shapes: means2D (P,2), depths (P), radii
  * (P) int32, cov3D (P,6), conic_opacity (P,4), rgb (P,3), clamped (P,3) bytes.

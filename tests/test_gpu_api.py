@@ -694,3 +694,32 @@ def test_per_tile_debug_log_is_written_like_the_reference(tmp_path):
                                 "num_rendered: %d," % (len(busy), 256 * len(busy), nr.sum()))
     run(21)
     assert len(path.read_text().splitlines()) == 2 * (len(busy) + 1)  # appended, like the reference
+
+
+@pytest.mark.parametrize("P", [1, 255, 256, 257, 3001])
+def test_visible_filter_reads_scales_in_wider_rows(P):
+    # the anchor model hands over the first three columns of its (P, 6) scaling; other layouts are copied first
+    import gs_scenes
+    from diff_gaussian_rasterization import GaussianRasterizationSettings, GaussianRasterizer
+    g, cams = gs_scenes.make_scene(0, P=P)
+    cam = cams[0]
+    rs = GaussianRasterizationSettings(
+        image_height=cam.image_height, image_width=cam.image_width, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy,
+        bg=torch.zeros(3, device="cuda"), scale_modifier=1.0, viewmatrix=cam.world_view_transform.cuda(),
+        projmatrix=cam.full_proj_transform.cuda(), sh_degree=3, campos=cam.camera_center.cuda(), prefiltered=False,
+        render_geo=True, debug=False)
+    rast = GaussianRasterizer(rs)
+    means, scales, rot = (g[k].cuda() for k in ("means3D", "scales", "rotations"))
+    want = rast.visible_filter(means, scales, rot)
+    wide = torch.full((P, 6), 1e9, device="cuda")
+    wide[:, :3] = scales
+    shifted = torch.full((P, 7), 1e9, device="cuda")
+    shifted[:, 2:5] = scales
+    for s in (wide[:, :3], shifted[:, 2:5], scales.t().contiguous().t(),
+              scales.repeat_interleave(2, 0)[::2], wide.requires_grad_()[:, :3]):
+        got = rast.visible_filter(means, s, rot)
+        assert torch.equal(got, want) and not got.requires_grad
+    with pytest.raises(TypeError):
+        rast.visible_filter(means, wide[:, :3].double(), rot)
+    with pytest.raises(RuntimeError):
+        rast.visible_filter(means, scales.cpu(), rot)
