@@ -40,8 +40,23 @@ constexpr int KEY_BITS = 3 * AXIS_BITS;
 constexpr int KEY_SHORT_BITS = 27;
 constexpr int KEY_SHORT_MAX = 1 << 15;
 
+// The search takes the leaves by falling size where there are more of them than waves that run at a time (32 a CU): one
+// among sparse points takes ten times as long as the median, and if it starts with the last ones the chip idles
+// until it ends.  1 M points of an SfM-like cloud: all waves had started after 123 us, half of them had ended after 94,
+// nine in ten after 161 and the last after 251.
+constexpr int ORDER_THREADS = 1024;
+constexpr int ORDER_MIN_LEAVES = 8192;
+constexpr int ORDER_BINS = 512;  // of a leaf's longest side: the exponent and one bit of the fraction
+constexpr uint32_t NO_LEAF = 0xFFFFFFFFu;
+
+// The leaves are ordered in `segments` parts, leaf l in part l % segments: none where they are too few to order.
+int order_segments(int P) {
+  const int leaves = (P + KNN_LEAF - 1) / KNN_LEAF;
+  return leaves > ORDER_MIN_LEAVES ? (leaves + ORDER_THREADS - 1) / ORDER_THREADS : 0;
+}
+
 struct KnnLayout {
-  size_t partial, codes_a, codes_b, idx_a, idx_b, sorted_pts, boxes, groups, leaves, twigs, sort_temp, total;
+  size_t partial, codes_a, codes_b, idx_a, idx_b, sorted_pts, boxes, groups, leaves, twigs, order, sort_temp, total;
 };
 
 KnnLayout knn_layout(int P) {
@@ -64,6 +79,7 @@ KnnLayout knn_layout(int P) {
   L.leaves = take(sizeof(float) * 6 * ((n + KNN_LEAF - 1) / KNN_LEAF));
   L.twigs = take(sizeof(float) * 6 * ((n + KNN_TWIG - 1) / KNN_TWIG));
   L.groups = take(sizeof(float) * 6 * ((nb + KNN_GROUP - 1) / KNN_GROUP));
+  L.order = take(sizeof(uint32_t) * ORDER_THREADS * (size_t)order_segments(P));
   L.sort_temp = take(sort_temp_bytes((int64_t)n));
   L.total = off;
   return L;
@@ -296,31 +312,89 @@ __global__ void __launch_bounds__(KNN_BOX) gather_boxes_kernel(int P, const floa
 // Bounding box of every run of KNN_GROUP consecutive boxes: lets the search discard that many boxes with
 // one test.  (Not in the reference, which tests every box for every point; the result is the same set of
 // three nearest neighbours, because a group's box bounds its members' boxes from below.)
-// Also hands a sort that gave up waiting on to the host (fault_word), as launch_sort_fault_report does.
-__global__ void __launch_bounds__(GS_WAVE) box_group_kernel(int nboxes, const float* __restrict__ boxes,
-                                                            float* __restrict__ groups,
-                                                            const uint32_t* __restrict__ sort_error,
-                                                            uint32_t* __restrict__ fault_word) {
-  if (blockIdx.x == 0 && threadIdx.x == 0 && fault_word != nullptr && *sort_error != 0u)
+// Also hands a sort that gave up waiting on to the host (fault_word), as launch_sort_fault_report does, and orders the
+// leaves for the search (order != nullptr): workgroup s those of part s, a thread each, by a counting sort over bins of
+// their longest sides, largest first, leaves of one bin in their old order; entry i * segments + s is the i-th of them,
+// so that the parts' largest come first together and neighbours along the curve stay neighbours.
+__global__ void __launch_bounds__(ORDER_THREADS)
+box_group_kernel(int nboxes, const float* __restrict__ boxes, float* __restrict__ groups, int nleaves,
+                 const float* __restrict__ leaves, uint32_t* __restrict__ order, const uint32_t* __restrict__ sort_error,
+                 uint32_t* __restrict__ fault_word) {
+  constexpr int WAVES = ORDER_THREADS / GS_WAVE;
+  __shared__ uint32_t s_count[WAVES][ORDER_BINS];
+  __shared__ uint32_t s_scan[ORDER_BINS / GS_WAVE];
+  const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
+  if (blockIdx.x == 0 && tid == 0 && fault_word != nullptr && *sort_error != 0u)
     __hip_atomic_store(fault_word, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  const int b = blockIdx.x * KNN_GROUP + threadIdx.x;
-  float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-  if (threadIdx.x < KNN_GROUP && b < nboxes) {
+  const int group = blockIdx.x * WAVES + wave;
+  if (group < (nboxes + KNN_GROUP - 1) / KNN_GROUP) {
+    static_assert(KNN_GROUP == GS_WAVE, "a lane per box of the group");
+    const int b = group * KNN_GROUP + lane;
+    float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
+    if (b < nboxes) {
 #pragma unroll
-    for (int c = 0; c < 6; c++) v[c] = boxes[6 * b + c];
-  }
+      for (int c = 0; c < 6; c++) v[c] = boxes[6 * b + c];
+    }
 #pragma unroll
-  for (int d = GS_WAVE / 2; d >= 1; d >>= 1) {
+    for (int d = GS_WAVE / 2; d >= 1; d >>= 1) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      v[c] = fminf(v[c], __shfl_xor(v[c], d, GS_WAVE));
-      v[3 + c] = fmaxf(v[3 + c], __shfl_xor(v[3 + c], d, GS_WAVE));
+      for (int c = 0; c < 3; c++) {
+        v[c] = fminf(v[c], __shfl_xor(v[c], d, GS_WAVE));
+        v[3 + c] = fmaxf(v[3 + c], __shfl_xor(v[3 + c], d, GS_WAVE));
+      }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int c = 0; c < 6; c++) groups[6 * group + c] = v[c];
     }
   }
-  if (threadIdx.x == 0) {
+  if (order == nullptr) return;
+  const int leaf = (int)blockIdx.x + (int)gridDim.x * tid;
+  uint32_t bin = ORDER_BINS - 1;  // (a leaf that does not exist comes last, behind those of side 0)
+  if (leaf < nleaves) {
+    float side = 0.f;
 #pragma unroll
-    for (int c = 0; c < 6; c++) groups[6 * blockIdx.x + c] = v[c];
+    for (int c = 0; c < 3; c++) side = fmaxf(side, leaves[6 * (size_t)leaf + 3 + c] - leaves[6 * (size_t)leaf + c]);
+    const uint32_t size = __builtin_bit_cast(uint32_t, side) >> 22;  // (never negative: below 512)
+    bin = size < ORDER_BINS - 2 ? ORDER_BINS - 2 - size : 0u;
   }
+  for (int e = tid; e < WAVES * ORDER_BINS; e += ORDER_THREADS) (&s_count[0][0])[e] = 0u;
+  __syncthreads();
+  // a wave's leaves of the same bin: how many, and this one's place among them
+  uint32_t place = 0u;
+  for (uint64_t rest = ~0ull; rest != 0ull;) {
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)bin, (int)__builtin_ctzll(rest));
+    const uint64_t same = gs_ballot(bin == b);
+    if (bin == b) place = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+    if (lane == 0) s_count[wave][b] = (uint32_t)__popcll(same);
+    rest &= ~same;
+  }
+  __syncthreads();
+  uint32_t total = 0u, inc = 0u;
+  if (tid < ORDER_BINS) {
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) total += s_count[w][tid];
+    inc = total;
+#pragma unroll
+    for (int d = 1; d < GS_WAVE; d <<= 1) {
+      const uint32_t o = __shfl_up(inc, d, GS_WAVE);
+      if (lane >= d) inc += o;
+    }
+    if (lane == GS_WAVE - 1) s_scan[wave] = inc;
+  }
+  __syncthreads();
+  if (tid < ORDER_BINS) {
+    uint32_t run = inc - total;
+    for (int w = 0; w < wave; w++) run += s_scan[w];
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+      const uint32_t n = s_count[w][tid];
+      s_count[w][tid] = run;
+      run += n;
+    }
+  }
+  __syncthreads();
+  order[(size_t)(s_count[wave][bin] + place) * gridDim.x + blockIdx.x] = leaf < nleaves ? (uint32_t)leaf : NO_LEAF;
 }
 
 // A node's bounding box: lo = minimum corner, hi = maximum corner.  An absent node is an inverted box, infinitely far
@@ -369,11 +443,10 @@ __device__ __forceinline__ float point_box_dist2(const float4& p, const NodeBox&
   return (gap[0] * gap[0] + gap[1] * gap[1]) + gap[2] * gap[2];
 }
 
-// Keeps the three smallest of {knn[0..2], dist(ref, p)} in ascending order (simple_knn.cu:131-145 inserts by
+// Keeps the three smallest of {knn[0..2], dist} in ascending order (simple_knn.cu:131-145 inserts by
 // compare-and-swap; minimum and medians leave the same three values).  A distance that is infinite or larger than
 // FLT_MAX changes nothing.
-__device__ __forceinline__ void update3(const float dx, const float dy, const float dz, float* knn) {
-  const float dist = (dx * dx + dy * dy) + dz * dz;
+__device__ __forceinline__ void update3(const float dist, float* knn) {
   const float n0 = fminf(knn[0], dist);
   const float n1 = __builtin_amdgcn_fmed3f(knn[0], knn[1], dist);
   const float n2 = __builtin_amdgcn_fmed3f(knn[1], knn[2], dist);
@@ -382,20 +455,44 @@ __device__ __forceinline__ void update3(const float dx, const float dy, const fl
   knn[2] = n2;
 }
 
+// The squared distance to the point that the lane N places back in the row holds.  The rotation is an operand modifier of
+// the subtractions: no instructions of its own and no memory access.
+template <int N>
+__device__ __forceinline__ float row_dist2(const float4& p, const float4& c) {
+  float dx, dy, dz;
+  if constexpr (N == 0) {
+    dx = c.x - p.x, dy = c.y - p.y, dz = c.z - p.z;
+  } else {
+    dx = row_ror<N>(c.x) - p.x, dy = row_ror<N>(c.y) - p.y, dz = row_ror<N>(c.z) - p.z;
+  }
+  return (dx * dx + dy * dy) + dz * dz;
+}
+
 // Every lane meets the points that the sixteen lanes of its row hold (from the FIRST-th one round; 1 leaves out the
-// lane's own).  The rotation is an operand modifier of the subtractions, so a distance costs eleven vector
-// instructions and no memory access.
+// lane's own).
 template <int FIRST, int LAST = KNN_TWIG>
 __device__ __forceinline__ void meet_row(const float4& p, const float4& c, float* knn) {
   if constexpr (FIRST < LAST) {
-    update3(row_ror<FIRST>(c.x) - p.x, row_ror<FIRST>(c.y) - p.y, row_ror<FIRST>(c.z) - p.z, knn);
+    update3(row_dist2<FIRST>(p, c), knn);
     meet_row<FIRST + 1, LAST>(p, c, knn);
   }
 }
-template <>
-__device__ __forceinline__ void meet_row<0, KNN_TWIG>(const float4& p, const float4& c, float* knn) {
-  update3(c.x - p.x, c.y - p.y, c.z - p.z, knn);
-  meet_row<1, KNN_TWIG>(p, c, knn);
+
+// The same, four points at a time, for twigs that few lanes gain from: where none of the four is nearer than the third
+// best of any lane there is nothing to keep (1 M points: 209 -> 191 us).
+template <int FIRST = 0>
+__device__ __forceinline__ void meet_row_of_few(const float4& p, const float4& c, float* knn) {
+  if constexpr (FIRST < KNN_TWIG) {
+    const float d0 = row_dist2<FIRST>(p, c), d1 = row_dist2<FIRST + 1>(p, c), d2 = row_dist2<FIRST + 2>(p, c),
+                d3 = row_dist2<FIRST + 3>(p, c);
+    if (gs_ballot(fminf(fminf(fminf(d0, d1), d2), d3) < knn[2]) != 0ull) {
+      update3(d0, knn);
+      update3(d1, knn);
+      update3(d2, knn);
+      update3(d3, knn);
+    }
+    meet_row_of_few<FIRST + 4>(p, c, knn);
+  }
 }
 
 // simple-knn/simple_knn.cu:147-183.  The reference gives every point a thread that seeds a rejection radius from
@@ -418,8 +515,9 @@ __device__ __forceinline__ void meet_row<0, KNN_TWIG>(const float4& p, const flo
 // brute-force search whatever the order.
 // Bound by vector issue.  With the whole leaf as the unit that opens twigs (64 points against every point of the
 // three leaves around it and of the twigs any of them needs, over LDS) the search took 335 us for 1 M points of an
-// SfM-like cloud; with the row as the unit 298 us, and 281 us with a workgroup per wave, whose place is taken as soon
-// as that wave ends (a leaf among sparse points takes ten times as long as the median).
+// SfM-like cloud; with the row as the unit 298 us, 265 us with a workgroup per wave, whose place is taken as soon
+// as that wave ends (a leaf among sparse points takes ten times as long as the median), and 209 us with the leaves in
+// falling order of their size (4 M points, the whole call: 1150 -> 1060 us; 600 k: 282 -> 246).
 constexpr int SEED = 2;
 
 __global__ void __launch_bounds__(GS_WAVE) box_mean_dist_kernel(int P, const float4* __restrict__ sorted_pts,
@@ -428,11 +526,14 @@ __global__ void __launch_bounds__(GS_WAVE) box_mean_dist_kernel(int P, const flo
                                                                     const float* __restrict__ groups,
                                                                     const float* __restrict__ leaves,
                                                                     const float* __restrict__ twigs,
+                                                                    const uint32_t* __restrict__ order,
                                                                     float* __restrict__ out) {
   constexpr int TWIGS_PER_BOX = KNN_BOX / KNN_TWIG, ROWS = KNN_LEAF / KNN_TWIG;
   static_assert(TWIGS_PER_BOX == GS_WAVE && KNN_GROUP == GS_WAVE, "a lane tests one node of a level");
   const int lane = threadIdx.x, row = lane / KNN_TWIG, in_row = lane % KNN_TWIG;
-  const int own = blockIdx.x;  // this wave's leaf
+  const uint32_t taken = order != nullptr ? order[blockIdx.x] : blockIdx.x;
+  if (taken == NO_LEAF) return;
+  const int own = (int)taken;  // this wave's leaf
   const int k = own * KNN_LEAF + lane;
   const int ntwigs = (P + KNN_TWIG - 1) / KNN_TWIG;
   const float4 nowhere = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.f);
@@ -532,7 +633,7 @@ __global__ void __launch_bounds__(GS_WAVE) box_mean_dist_kernel(int P, const flo
       const float4 c = without_nan(ahead);
       left = gs_ballot(todo != 0ull);
       if (left != 0ull) ahead = next();
-      meet_row<0>(p, c, best);
+      meet_row_of_few(p, c, best);
     }
     update_reach();
   };
@@ -579,6 +680,8 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
   float* groups = (float*)(base + L.groups);
   float* leaves = (float*)(base + L.leaves);
   float* twigs = (float*)(base + L.twigs);
+  const int segments = order_segments(P);
+  uint32_t* order = segments > 0 ? (uint32_t*)(base + L.order) : nullptr;
   void* sort_temp = base + L.sort_temp;
   const int nboxes = (P + KNN_BOX - 1) / KNN_BOX;
   const int key_bits = P <= KEY_SHORT_MAX ? KEY_SHORT_BITS : KEY_BITS;
@@ -605,13 +708,17 @@ int launch_knn_dist2(int P, const float* points, float* mean_dist2, void* temp, 
     StageScope _t("knn_boxes", stream);
     hipLaunchKernelGGL(gather_boxes_kernel, dim3(nboxes), dim3(KNN_BOX), 0, stream, P, points, idx_sorted, sorted_pts,
                        boxes, leaves, twigs);
-    hipLaunchKernelGGL(box_group_kernel, dim3((nboxes + KNN_GROUP - 1) / KNN_GROUP), dim3(GS_WAVE), 0, stream, nboxes,
-                       boxes, groups, sort_error_word(sort_temp), fault_word);
+    // (a wave per group of boxes, of which the parts to order have plenty: a group is 1024 leaves, a part has 16 waves)
+    const int group_blocks = ((nboxes + KNN_GROUP - 1) / KNN_GROUP + ORDER_THREADS / GS_WAVE - 1) / (ORDER_THREADS / GS_WAVE);
+    hipLaunchKernelGGL(box_group_kernel, dim3(segments > 0 ? segments : group_blocks), dim3(ORDER_THREADS), 0, stream,
+                       nboxes, boxes, groups, (P + KNN_LEAF - 1) / KNN_LEAF, leaves, order, sort_error_word(sort_temp),
+                       fault_word);
   }
   {
     StageScope _t("knn_box_mean_dist", stream);
-    hipLaunchKernelGGL(box_mean_dist_kernel, dim3((P + KNN_LEAF - 1) / KNN_LEAF), dim3(GS_WAVE), 0, stream, P, sorted_pts,
-                       idx_sorted, boxes, nboxes, groups, leaves, twigs, mean_dist2);
+    hipLaunchKernelGGL(box_mean_dist_kernel, dim3(segments > 0 ? segments * ORDER_THREADS : (P + KNN_LEAF - 1) / KNN_LEAF),
+                       dim3(GS_WAVE), 0, stream, P, sorted_pts, idx_sorted, boxes, nboxes, groups, leaves, twigs, order,
+                       mean_dist2);
   }
   return 0;
 }

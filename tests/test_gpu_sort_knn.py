@@ -116,6 +116,22 @@ def _brute_f32(pts):
     return out
 
 
+@pytest.mark.parametrize("P", [524_288, 524_289, 589_825])
+def test_knn_dist2_where_the_leaves_are_ordered(H, orc, P):
+    """Beyond 8192 leaves of 64 points the search takes them by size: dense clusters, a thin plane and sparse points (with
+    coincident ones, whose leaves have no size), the last leaf and the last part of the order not full."""
+    import simple_knn._C as knn
+    rng = np.random.default_rng(P)
+    pts = rng.uniform(-100, 100, (P, 3))
+    kind = rng.integers(0, 4, P)
+    pts[kind == 0] = rng.normal(0, 0.5, (int((kind == 0).sum()), 3)) + rng.integers(-3, 3, (int((kind == 0).sum()), 3)) * 30
+    pts[kind == 1, 2] *= 1e-4
+    pts[:200] = pts[0]
+    pts = pts.astype(np.float32)
+    got = knn.distCUDA2(torch.from_numpy(pts).to(H.DEV)).cpu().numpy()
+    assert np.array_equal(got, orc.knn_dist2(pts))
+
+
 @pytest.mark.parametrize("case", ["one", "two", "three", "four", "63", "64", "65", "129", "identical", "duplicates",
                                   "line", "plane", "nan_and_inf", "far_outliers", "two_clusters", "2500"])
 def test_knn_edge_cases_match_a_float32_brute_force(H, orc, case):
