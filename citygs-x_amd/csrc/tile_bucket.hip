@@ -574,91 +574,115 @@ bucket_scatter_staged_kernel(int P, int per_block, int nblocks, uint32_t gx, uin
 //
 // The key is one 32-bit word: (depth bits - smallest depth bits of the list) >> shift in the high bits, the
 // record's place in the unsorted segment in the low log2(64 E W) bits; shift is what it takes to fit the list's
-// range of depth bits (0 when it fits as it is).  A step then costs three vector instructions per key (one move,
-// one comparison, one select) where a 64-bit key cost five.  Keys whose depths agree in the bits kept end up next
+// range of depth bits (0 when it fits as it is).  A step then costs two vector instructions per key (a cross-lane
+// move and a median with 0 or all ones, or a minimum and a maximum that each read across lanes).  With all runs of a
+// stage sorted upwards nothing depends on a run's direction any more but the complements at the start of the stage, and
+// with the steps inside a wave unrolled the chains of a lane's registers overlap; with a compare, a scalar mask and a
+// select per step, and the directions in masks, the kernel took 27.9 us at 1 M Gaussians, 1152 x 864 and 29.0 us at 4 M,
+// now 22.0 and 22.8; 13.2 and 11.4 us at 300 k, 1237 x 822.  Keys whose depths agree in the bits kept end up next
 // to each other in the order of their places; the last step (emit_list_entry) puts every such run into its true
 // order, by all depth bits and then the emission index, exactly as it does for runs of equal depth bits.  Depths
 // inside a tile are spread over the view's range, so with the 21 to 24 bits kept runs are as rare as before.
 
-// Which element of a pair (a, b) each lane keeps is decided in scalar registers: keep_min is the lane mask of the
-// elements that keep the smaller one, less the lane mask of a < b; a lane keeps a where the two agree.
-__device__ __forceinline__ uint32_t keep_pair(uint32_t a, uint32_t b, uint64_t keep_min) {
-  const uint64_t less = __builtin_amdgcn_ballot_w64(a < b);
-  return __builtin_amdgcn_inverse_ballot_w64(~(less ^ keep_min)) ? a : b;
+// A pair's smaller key where `keep` is 0, its larger one where it is all ones: the median of the three.  (The idle slots
+// are for a cross-lane instruction that reads the result next: the compiler does not look into these statements for what
+// such an instruction has to wait for.)
+__device__ __forceinline__ uint32_t keep_pair(uint32_t a, uint32_t b, uint32_t keep) {
+  uint32_t r;
+  asm("v_med3_u32 %0, %1, %2, %3\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b), "v"(keep));
+  return r;
 }
 
-// Lanes whose bit J of the lane number is clear: the lower element of every pair at distance J.
+// One step of the network with the partner in lane ^ J: the lanes whose bit J is clear keep the smaller key, the others
+// the larger (upper: all ones there).  A variable-distance __shfl_xor is a ds_bpermute, whose latency every one of the
+// sort's dependent steps would wait for.  All 64 lanes must be active.
+//   J = 1, 2: a DPP move inside the quad and a median;
+//   J = 4, 8: a minimum and a maximum whose DPP operands come from the other side, each for the quads of a row that take
+//     its result (a DPP operand written by the preceding vector instruction needs two idle issue slots);
+//   J = 16, 32: v_permlane16_swap / v_permlane32_swap exchange the odd rows (the upper half) of their first operand with
+//     the even rows (the lower half) of the second: from two copies of x they leave the lower element of every pair in
+//     all lanes of the first result and the upper element in the second.
 template <int J>
-__device__ __forceinline__ constexpr uint64_t lower_lanes() {
-  uint64_t m = 0;
-  for (int l = 0; l < 64; l++)
-    if ((l & J) == 0) m |= 1ull << l;
-  return m;
-}
-
-// x of lane (lane ^ J), J = 1, 2, 4 or 8, by DPP moves inside a 16-lane row (xor 4 = reverse the quads' lanes,
-// then mirror the half rows).  Every lane has a source, so nothing is kept of the old value (with bound_ctrl set
-// the destination needs no initialisation).  A variable-distance __shfl_xor is a ds_bpermute, whose latency
-// every one of the sort's dependent steps would wait for.  All 64 lanes must be active.
-template <int J>
-__device__ __forceinline__ uint32_t xor_lane(uint32_t x) {
-  static_assert(J == 1 || J == 2 || J == 4 || J == 8, "distance inside a 16-lane row");
+__device__ __forceinline__ uint32_t lane_step(uint32_t x, uint32_t upper) {
+  static_assert(J == 1 || J == 2 || J == 4 || J == 8 || J == 16 || J == 32, "a distance inside the wave");
+  uint32_t r;
   if constexpr (J == 1) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
+    asm("s_nop 1\n\t"
+        "v_mov_b32_dpp %0, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_med3_u32 %0, %1, %0, %2"
+        : "=&v"(r)
+        : "v"(x), "v"(upper));
   } else if constexpr (J == 2) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, true);  // quad_perm [2,3,0,1]
+    asm("s_nop 1\n\t"
+        "v_mov_b32_dpp %0, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_med3_u32 %0, %1, %0, %2"
+        : "=&v"(r)
+        : "v"(x), "v"(upper));
   } else if constexpr (J == 4) {
-    const int t = __builtin_amdgcn_update_dpp(0, (int)x, 0x1B, 0xF, 0xF, true);     // quad_perm [3,2,1,0]: lane ^ 3
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, t, 0x141, 0xF, 0xF, true);      // row_half_mirror: lane ^ 7
+    asm("s_nop 1\n\t"
+        "v_min_u32_dpp %0, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_max_u32_dpp %0, %1, %1 row_shr:4 row_mask:0xf bank_mask:0xa"
+        : "=&v"(r)
+        : "v"(x));
+  } else if constexpr (J == 8) {
+    asm("s_nop 1\n\t"
+        "v_min_u32_dpp %0, %1, %1 row_shl:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_max_u32_dpp %0, %1, %1 row_shr:8 row_mask:0xf bank_mask:0xc"
+        : "=&v"(r)
+        : "v"(x));
+  } else if constexpr (J == 16) {
+    const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    r = keep_pair(p[0], p[1], upper);
   } else {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, true);  // row_ror:8
+    const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    r = keep_pair(p[0], p[1], upper);
   }
+  return r;
 }
 
-// One step of the network with the partner in lane ^ J.  ascending[r]: lane mask of the elements of register r
-// that lie in an ascending run of this stage.
-template <int E, int J>
-__device__ __forceinline__ void lane_step(uint32_t (&v)[E], const uint64_t (&ascending)[E]) {
-  constexpr uint64_t lower = lower_lanes<J>();
+// The steps at distances J, J / 2 .. 1 of every register: the registers' chains of steps are independent of each other.
+template <int J, int E>
+__device__ __forceinline__ void lane_steps(uint32_t (&v)[E], const uint32_t (&upper)[6]) {
+#pragma unroll
+  for (int r = 0; r < E; r++) v[r] = lane_step<J>(v[r], upper[__builtin_ctz(J)]);
+  if constexpr (J > 1) lane_steps<J / 2>(v, upper);
+}
+
+// Element i = (row << 6 | lane) is sorted upwards in the stage of runs of k where (i & k) == 0, which is a property of the
+// lane below k = 64 and of the register (and wave) from there on.  Every step sorts upwards: the keys of the runs that a
+// stage sorts downwards are complemented before it.  flipped: all ones where a key is held complemented.
+template <int E>
+__device__ __forceinline__ void turn_runs(uint32_t (&v)[E], uint32_t (&flipped)[E], uint32_t row0, uint32_t lane, uint32_t k) {
 #pragma unroll
   for (int r = 0; r < E; r++) {
-    const uint64_t keep_min = ~(lower ^ ascending[r]);  // the lower element of an ascending pair, the upper of a descending
-    if constexpr (J < 16) {
-      v[r] = keep_pair(v[r], xor_lane<J>(v[r]), keep_min);
-    } else {
-      // v_permlane16_swap / v_permlane32_swap exchange the odd rows (the upper half) of their first operand with
-      // the even rows (the lower half) of the second: from two copies of x they leave the lower element of every
-      // pair in all lanes of the first result and the upper element in the second, so both lanes of a pair
-      // compare the same two values and each keeps its own.
-      if constexpr (J == 16) {
-        const auto p = __builtin_amdgcn_permlane16_swap(v[r], v[r], false, false);
-        v[r] = keep_pair(p[0], p[1], keep_min);
-      } else {
-        const auto p = __builtin_amdgcn_permlane32_swap(v[r], v[r], false, false);
-        v[r] = keep_pair(p[0], p[1], keep_min);
-      }
-    }
+    const uint32_t flip = ((((row0 + (uint32_t)r) << 6) | lane) & k) != 0u ? ~0u : 0u;
+    v[r] ^= flipped[r] ^ flip;
+    flipped[r] = flip;
   }
+}
+
+// The stages of runs of K .. 32: all their pairs lie in one register.
+template <int K, int E>
+__device__ __forceinline__ void lane_stages(uint32_t (&v)[E], uint32_t (&flipped)[E], uint32_t row0, uint32_t lane,
+                                            const uint32_t (&upper)[6]) {
+  turn_runs(v, flipped, row0, lane, K);
+  lane_steps<K / 2>(v, upper);
+  if constexpr (K < 32) lane_stages<2 * K>(v, flipped, row0, lane, upper);
 }
 
 template <int E, int W>
 __device__ __forceinline__ void register_sort(uint32_t (&v)[E], uint32_t wave, uint32_t lane, uint32_t* s_x) {
   constexpr uint32_t M = 64u * E * W;
   const uint32_t row0 = wave * E;
-  for (uint32_t k = 2; k <= M; k <<= 1) {
-    // the direction of this stage's runs: element i = (row << 6 | lane) ascends where (i & k) == 0, which is a
-    // property of the lane below k = 64 and of the register (and wave) from there on
-    uint64_t ascending[E];
-    {
-      const uint64_t by_lane = __builtin_amdgcn_ballot_w64((lane & k) == 0u);
+  uint32_t upper[6];
 #pragma unroll
-      for (int r = 0; r < E; r++) {
-        const uint64_t m = k < 64u ? by_lane : ((((row0 + (uint32_t)r) << 6) & k) == 0u ? ~0ull : 0ull);
-        // (wave-uniform: kept in scalar registers)
-        ascending[r] = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(m >> 32)) << 32) |
-                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)m);
-      }
-    }
+  for (int b = 0; b < 6; b++) upper[b] = (lane >> b & 1u) != 0u ? ~0u : 0u;
+  uint32_t flipped[E];
+#pragma unroll
+  for (int r = 0; r < E; r++) flipped[r] = 0u;
+  lane_stages<2>(v, flipped, row0, lane, upper);
+  for (uint32_t k = 64; k <= M; k <<= 1) {
+    turn_runs(v, flipped, row0, lane, k);
     for (uint32_t j = k >> 1; j >= 64; j >>= 1) {
       if (j < 64u * E) {
         const uint32_t jr = j >> 6;
@@ -668,12 +692,9 @@ __device__ __forceinline__ void register_sort(uint32_t (&v)[E], uint32_t wave, u
 #pragma unroll
           for (int r = 0; r < E; r++) {
             if (r & b) continue;
-            // (both registers of a pair lie in the same run)
             const uint32_t x = v[r], y = v[r | b];
-            const uint64_t less = __builtin_amdgcn_ballot_w64(x < y);
-            const bool x_first = __builtin_amdgcn_inverse_ballot_w64(~(less ^ ascending[r]));
-            v[r] = x_first ? x : y;
-            v[r | b] = x_first ? y : x;
+            v[r] = x < y ? x : y;
+            v[r | b] = x < y ? y : x;
           }
         }
       } else {
@@ -683,21 +704,12 @@ __device__ __forceinline__ void register_sort(uint32_t (&v)[E], uint32_t wave, u
 #pragma unroll
         for (int r = 0; r < E; r++) s_x[((wave * E + r) << 6) | lane] = v[r];
         __syncthreads();
-        const bool lower = (wave & jw) == 0;
+        const uint32_t keep = (wave & jw) == 0 ? 0u : ~0u;
 #pragma unroll
-        for (int r = 0; r < E; r++) {
-          const uint32_t other = s_x[(((wave ^ jw) * E + r) << 6) | lane];
-          v[r] = keep_pair(v[r], other, lower ? ascending[r] : ~ascending[r]);
-        }
+        for (int r = 0; r < E; r++) v[r] = keep_pair(v[r], s_x[(((wave ^ jw) * E + r) << 6) | lane], keep);
       }
     }
-    // the steps with the partner in another lane: distances min(k / 2, 32) down to 1
-    if (k >= 64) lane_step<E, 32>(v, ascending);
-    if (k >= 32) lane_step<E, 16>(v, ascending);
-    if (k >= 16) lane_step<E, 8>(v, ascending);
-    if (k >= 8) lane_step<E, 4>(v, ascending);
-    if (k >= 4) lane_step<E, 2>(v, ascending);
-    lane_step<E, 1>(v, ascending);
+    lane_steps<32>(v, upper);
   }
 }
 

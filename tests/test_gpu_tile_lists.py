@@ -331,3 +331,37 @@ def test_depths_that_agree_in_their_leading_bits(orc, H, P):
     keys = binB[b0 + off[1].value: b0 + off[1].value + 8 * R].view(torch.int64)
     assert np.array_equal(H.np_u64(keys), want["keys"])
     assert np.array_equal(H.np_u32(point_list), want["point_list"])
+
+
+@pytest.mark.parametrize("order", ["random", "falling", "equal"])
+@pytest.mark.parametrize("P", [1, 2, 63, 64, 65, 255, 256, 257, 511, 512, 513, 1024, 1025, 1537, 2047, 2048])
+def test_list_lengths_at_the_edges_of_the_register_sort(orc, H, P, order):
+    """One tile whose list holds exactly P entries: every number of registers per lane and of waves that the register
+    sort has, filled exactly, one entry short and one over; depths at random, falling, and all equal."""
+    import gsrast_native as gn
+    from diff_gaussian_rasterization import _C
+    gen = torch.Generator().manual_seed(P)
+    W = Hh = 16
+    means2D = torch.rand(P, 2, generator=gen) * 16.0
+    radii = torch.full((P,), 100, dtype=torch.int32)
+    depths = {"random": lambda: torch.rand(P, generator=gen) * 50.0 + 0.25,
+              "falling": lambda: torch.linspace(60.0, 0.5, P),
+              "equal": lambda: torch.full((P,), 3.0)}[order]()
+    cl = torch.ones(1, 1, dtype=torch.bool)
+    n = lambda t: t.detach().cpu().numpy()
+    want = orc.bin_and_sort(n(radii), n(means2D), n(depths), cl.numpy().reshape(-1), W, Hh)
+    assert int(want["point_list"].shape[0]) == P
+    co = torch.tensor([0.02, 0.0, 0.02, 0.3]).repeat(P, 1).to(DEV)
+    eye = torch.eye(4, device=DEV)
+    out = _C.render_gaussians(torch.zeros(3, device=DEV), Hh, W, means2D.to(DEV), depths.to(DEV), radii.to(DEV), co,
+                              torch.zeros(P, 3, device=DEV), cl.to(DEV), eye, torch.zeros(3, device=DEV), 1.0, 1.0,
+                              torch.zeros(P, 5, device=DEV), False, False, {"stats_collector": {}})
+    R, binB = out[0], out[9]
+    assert R == P
+    off = [C.c_size_t() for _ in range(5)]
+    gn.check(gn.lib.gs_binning_state_layout(R, W, Hh, *[C.byref(x) for x in off]), "layout")
+    b0 = (binB.data_ptr() + 255) // 256 * 256 - binB.data_ptr()
+    point_list = binB[b0 + off[0].value: b0 + off[0].value + 4 * R].view(torch.int32)
+    keys = binB[b0 + off[1].value: b0 + off[1].value + 8 * R].view(torch.int64)
+    assert np.array_equal(H.np_u64(keys), want["keys"])
+    assert np.array_equal(H.np_u32(point_list), want["point_list"])
