@@ -867,16 +867,21 @@ const uint32_t* bucket_fits_word(const void* table, int T) {
   return (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 2 + BK_MAX_BLOCKS;
 }
 
+// The longest list that the radix sort's smaller kernel takes (what one of its workgroups holds); longer ones go to the
+// larger kernel.
+static uint32_t radix_mid_limit(uint32_t small_limit, uint32_t block_limit) {
+  uint32_t limit = (uint32_t)tile_radix_mid_records();
+  if (block_limit != 0 && block_limit < limit) limit = block_limit;
+  return limit < small_limit ? small_limit : limit;
+}
+
 int launch_bucket_count(int P, int W, int H, const int* radii, const float* means2D, const uint8_t* compute_locally,
                         uint32_t* tiles_touched, void* table, uint32_t* ranges, uint32_t small_limit,
                         uint32_t block_limit, uint32_t* host_words, int* zero_per_gaussian, uint32_t cap_instances,
                         uint32_t cap_longest, uint32_t* clear_word, hipStream_t stream) {
   if (P <= 0) return 0;
   if (small_limit == 0 || small_limit > (uint32_t)TILE_SORT_SMALL) small_limit = TILE_SORT_SMALL;
-  // the lists one workgroup of the radix sort's smaller kernel holds; longer ones go to the larger kernel
-  uint32_t mid_limit = (uint32_t)tile_radix_mid_records();
-  if (block_limit != 0 && block_limit < mid_limit) mid_limit = block_limit;
-  if (mid_limit < small_limit) mid_limit = small_limit;
+  const uint32_t mid_limit = radix_mid_limit(small_limit, block_limit);
   // ... and the lists the larger kernel holds; longer ones are split first
   uint32_t split_limit = (uint32_t)tile_radix_block_records();
   if (block_limit != 0 && block_limit < split_limit) split_limit = block_limit;
@@ -972,10 +977,12 @@ int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t sma
                      (const TileRecord*)records, keys, emission, point_list, small_limit, fits, tile_order,
                      tile_order_valid);
   if (longest > small_limit) {
+    // (a launch with nothing to do takes 4.6 us of the device: a view whose longest list is bounded does without)
+    const bool lng = (radix_tiles >> 16) != 0u && longest > radix_mid_limit(small_limit, block_limit);
     const uint32_t* tile_lists = (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 1) * (size_t)T;
     // scratch: `capacity` 16-byte records for the lists that are split first, then as many 8-byte words
     uint64_t* pong = (uint64_t*)((char*)scratch + (size_t)capacity * 16);
-    if (launch_tile_radix_sort(T, (radix_tiles & 0xFFFFu) != 0u, (radix_tiles >> 16) != 0u, ranges, tile_lists,
+    if (launch_tile_radix_sort(T, (radix_tiles & 0xFFFFu) != 0u, lng, ranges, tile_lists,
                                tile_lists + T, block_limit, records, scratch, keys, pong, keys, emission, point_list,
                                fits, stream))
       return 1;

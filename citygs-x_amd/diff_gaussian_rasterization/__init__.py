@@ -252,11 +252,12 @@ def _expectation(key):
     if longest <= 0:
         return 0, 0  # a view without per-tile lists (a tile grid too large for them): nothing to gain
     # whole variants of the register sort (256 ... 2048 records per list), so that a slightly longer list still
-    # fits; beyond them any length (0): the radix sort's kernels are launched as well
+    # fits, then what the smaller of the radix sort's kernels holds (4096); beyond it any length (0): the larger one
+    # is launched as well
     cap = 256
     while cap < longest * _MARGIN:
         cap *= 2
-    return int(instances * _MARGIN) + 65536, (cap if cap <= 2048 else 0)
+    return int(instances * _MARGIN) + 65536, (cap if cap <= 4096 else 0)
 
 
 def _remember(key, instances, longest):

@@ -365,3 +365,36 @@ def test_list_lengths_at_the_edges_of_the_register_sort(orc, H, P, order):
     keys = binB[b0 + off[1].value: b0 + off[1].value + 8 * R].view(torch.int64)
     assert np.array_equal(H.np_u64(keys), want["keys"])
     assert np.array_equal(H.np_u32(point_list), want["point_list"])
+
+
+@pytest.mark.parametrize("longest,bound,ahead", [(2048, 4096, True), (2049, 4096, True), (4096, 4096, True),
+                                                 (4097, 4096, False), (4097, 4097, True), (4097, 0, True)])
+def test_launching_ahead_with_a_bound_on_the_longest_list(orc, H, longest, bound, ahead):
+    """A view launched ahead with a bound that the radix sort's smaller kernel covers does without the larger one; where
+    a list is longer than the bound after all, the lists are built again.  One tile, whose list is the longest."""
+    import gsrast_native as gn
+    from diff_gaussian_rasterization import _C
+    gen = torch.Generator().manual_seed(longest)
+    W = Hh = 16
+    means2D = torch.rand(longest, 2, generator=gen) * 16.0
+    radii = torch.full((longest,), 100, dtype=torch.int32)
+    depths = torch.rand(longest, generator=gen) * 50.0 + 0.25
+    cl = torch.ones(1, 1, dtype=torch.bool)
+    n = lambda t: t.detach().cpu().numpy()
+    want = orc.bin_and_sort(n(radii), n(means2D), n(depths), cl.numpy().reshape(-1), W, Hh)
+    co = torch.tensor([0.02, 0.0, 0.02, 0.3]).repeat(longest, 1).to(DEV)
+    eye = torch.eye(4, device=DEV)
+    out, info = _C.render_gaussians_ex(torch.zeros(3, device=DEV), Hh, W, means2D.to(DEV), depths.to(DEV), radii.to(DEV),
+                                       co, torch.zeros(longest, 3, device=DEV), cl.to(DEV), eye,
+                                       torch.zeros(3, device=DEV), 1.0, 1.0, torch.zeros(longest, 5, device=DEV), False,
+                                       False, {"stats_collector": {}}, expected_instances=longest + 500,
+                                       expected_longest_list=bound)
+    R, binB = out[0], out[9]
+    assert R == longest and info["launched_ahead"] == ahead and info["longest_list"] == longest
+    off = [C.c_size_t() for _ in range(5)]
+    gn.check(gn.lib.gs_binning_state_layout(info["binning_capacity"], W, Hh, *[C.byref(x) for x in off]), "layout")
+    b0 = (binB.data_ptr() + 255) // 256 * 256 - binB.data_ptr()
+    point_list = binB[b0 + off[0].value: b0 + off[0].value + 4 * R].view(torch.int32)
+    keys = binB[b0 + off[1].value: b0 + off[1].value + 8 * R].view(torch.int64)
+    assert np.array_equal(H.np_u64(keys), want["keys"])
+    assert np.array_equal(H.np_u32(point_list), want["point_list"])
