@@ -127,10 +127,21 @@ __device__ __forceinline__ uint32_t f2u_sat(float v) {
 // parameters on their way to the optimizer, what the forward pass leaves for the backward pass): it goes out past the
 // caches, so it does not evict what the next kernel reads.
 __device__ __forceinline__ void store_streaming(float* p, float v) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ void store_streaming(float2* p, const float2& v) {
+  typedef float v2f __attribute__((ext_vector_type(2)));
+  const v2f w = {v.x, v.y};
+  __builtin_nontemporal_store(w, reinterpret_cast<v2f*>(p));
+}
 __device__ __forceinline__ void store_streaming(float4* p, const float4& v) {
   typedef float v4f __attribute__((ext_vector_type(4)));
   const v4f w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<v4f*>(p));
+}
+// Load of data that is not read again.
+__device__ __forceinline__ float4 load_streaming(const float4* p) {
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  const v4f w = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p));
+  return make_float4(w.x, w.y, w.z, w.w);
 }
 
 // exp() of the blending loops: n = rint(x*log2e), r = x - n*ln2 (two-constant

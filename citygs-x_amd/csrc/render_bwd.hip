@@ -659,9 +659,40 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   }
 }
 
+// The rows of N floats that the lanes of a wave hold leave through LDS, past the caches, as N runs of consecutive floats.
+template <int N>
+__device__ __forceinline__ void stream_rows(float* __restrict__ out, int rows, const float (&own)[N], float* lds, int lane) {
+  auto sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  sync();  // (everyone has read what the buffer last held)
+#pragma unroll
+  for (int k = 0; k < N; k++) lds[N * lane + k] = own[k];
+  sync();
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const int e = j * GS_WAVE + lane;
+    if (e < N * rows) store_streaming(out + e, lds[e]);
+  }
+}
+
+// Where reduce_instances_kernel streams: from this many Gaussians on, whose results outgrow what the caches keep for
+// the next kernel.  This kernel and the preprocess backward kernel at 1152 x 864, stored plainly and streamed: 0.6 M
+// 68.3 and 71.2 us, 1 M 102.3 and 104.7, 1.5 M 145.6 and 143.3, 2 M 201.6 and 183.9, 3 M 293.7 and 268.6 (2.5 M without
+// geometry channels 132.4 and 127.0).
+constexpr int REDUCE_STREAM_GAUSSIANS = 1'500'000;
+
 // Sums the instance records of every Gaussian (consecutive in emission order) into the gradient
 // tensors.  Record layout: [mean2D.x, mean2D.y, |mean2D|.x, |mean2D|.y, conic.x, conic.y, conic.w,
 // opacity, rgb(3), map(5)].  Every output element is written.
+// Bound by memory (64 bytes per instance in, 68 or 48 per Gaussian out).  STREAM: the records are read and the results
+// stored past the caches.  Where the results are more than the caches hold anyway, the preprocess backward kernel that
+// follows otherwise runs beside the write-back of the lines they left dirty: 4 M Gaussians, 1152 x 864, 79.3 + 277 us ->
+// 79.5 + 248 (this kernel + that one), 10 M, 1920 x 1080, 175 + 633 -> 175 + 595.  That wants whole lines per store, so
+// the rows of 3 and 5 floats are turned in LDS (stored from the lanes that hold them, 80.5 and 180).
+template <bool STREAM>
 __global__ void __launch_bounds__(GS_BLOCK_1D)
 reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const float4* __restrict__ instance_grads,
                         float ddelx_dx, float ddely_dy, int render_geo, float2* __restrict__ dL_dmean2D, float* __restrict__ dL_dmean2D_abs,
@@ -729,7 +760,11 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const uint32_t idx = (uint32_t)(j * GS_WAVE + lane), r = c + (idx >> 2);
-        v[j] = r < run_end ? instance_grads[4 * (size_t)r + (idx & 3u)] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4* part = instance_grads + 4 * (size_t)r + (idx & 3u);
+        if constexpr (STREAM)
+          v[j] = r < run_end ? load_streaming(part) : make_float4(0.f, 0.f, 0.f, 0.f);
+        else
+          v[j] = r < run_end ? *part : make_float4(0.f, 0.f, 0.f, 0.f);
       }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
@@ -748,6 +783,24 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+  }
+  if constexpr (STREAM) {
+    const int first = i - lane, rows = P - first < GS_WAVE ? P - first : GS_WAVE;
+    if (rows <= 0) return;
+    if (live) {
+      store_streaming(dL_dmean2D + i, make_float2(a0.x * ddelx_dx, a0.y * ddely_dy));
+      store_streaming(dL_dconic_opacity + i, a1);
+    }
+    float* const lds = reinterpret_cast<float*>(s_rec[threadIdx.x / GS_WAVE]);
+    const float abs_row[3] = {a0.z * ddelx_dx, a0.w * ddely_dy, 0.f}, colour_row[3] = {a2.x, a2.y, a2.z};
+    stream_rows(dL_dmean2D_abs + 3 * (size_t)first, rows, abs_row, lds, lane);
+    stream_rows(dL_dcolors + 3 * (size_t)first, rows, colour_row, lds, lane);
+    if (dL_dall_map) {
+      const float map_row[5] = {render_geo ? a2.w : 0.f, render_geo ? a3.x : 0.f, render_geo ? a3.y : 0.f,
+                                render_geo ? a3.z : 0.f, render_geo ? a3.w : 0.f};
+      stream_rows(dL_dall_map + 5 * (size_t)first, rows, map_row, lds, lane);
+    }
+    return;
   }
   if (!live) return;
   // records hold the mean2D sums per pixel unit: d(pixel offset)/d(normalised coordinate) = W/2, H/2
@@ -787,11 +840,14 @@ int launch_render_bwd(const RenderBwdArgs& a, hipStream_t stream) {
     if (a.block_hits) go(render_bwd_kernel<false, true>);
     else go(render_bwd_kernel<false, false>);
   }
-  hipLaunchKernelGGL(reduce_instances_kernel, dim3((a.P + GS_BLOCK_1D - 1) / GS_BLOCK_1D), dim3(GS_BLOCK_1D), 0,
-                     stream, a.P, a.point_offsets, (const float4*)a.instance_grads, (float)(0.5 * a.W),
-                     (float)(0.5 * a.H), a.render_geo,
-                     (float2*)a.dL_dmean2D, a.dL_dmean2D_abs, (float4*)a.dL_dconic_opacity, a.dL_dcolors,
-                     a.dL_dall_map);
+  auto reduce = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((a.P + GS_BLOCK_1D - 1) / GS_BLOCK_1D), dim3(GS_BLOCK_1D), 0, stream, a.P,
+                       a.point_offsets, (const float4*)a.instance_grads, (float)(0.5 * a.W), (float)(0.5 * a.H),
+                       a.render_geo, (float2*)a.dL_dmean2D, a.dL_dmean2D_abs, (float4*)a.dL_dconic_opacity,
+                       a.dL_dcolors, a.dL_dall_map);
+  };
+  if (a.P >= REDUCE_STREAM_GAUSSIANS) reduce(reduce_instances_kernel<true>);
+  else reduce(reduce_instances_kernel<false>);
   return 0;
 }
 

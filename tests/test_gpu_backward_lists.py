@@ -102,3 +102,52 @@ def test_every_wave_needs_every_slot(H, orc, n, geo):
                     ("dL_dall_map", ref["dL_dall_map"])):
         if k != "dL_dall_map" or geo:
             assert H.rel_l2(got[k].cpu().numpy(), want) <= 1e-4, (k, H.rel_l2(got[k].cpu().numpy(), want))
+
+
+@pytest.mark.parametrize("P", [1_499_999, 1_500_000, 1_500_001, 1_500_063])
+@pytest.mark.parametrize("geo", [True, False])
+def test_results_of_a_large_view_are_streamed(H, orc, P, geo):
+    """From 1.5 M Gaussians on the sums over a Gaussian's instances leave past the caches and turned through LDS, the last
+    wave partly filled.  A small view's Gaussians, half of them at the start and half at the end of a large view that has
+    nothing between them: the same bits, and zeros for everybody else."""
+    n, half = 300, 150
+    gen = torch.Generator().manual_seed(3)
+    r = lambda *s: torch.rand(*s, generator=gen)
+    W, Hh, tan = 41, 27, 0.5
+    means2D = (r(n, 2) * torch.tensor([W + 8.0, Hh + 8.0]) - 4.0).numpy()
+    s1 = torch.exp(r(n) * 2.5)
+    i1 = 1 / s1 ** 2
+    co = torch.stack([i1, torch.zeros(n), i1, r(n) * 0.1 + 0.01], 1).float().numpy()
+    radii = torch.ceil(3 * s1).int().numpy()
+    depths, rgb = (r(n) * 10 + 1).numpy(), r(n, 3).numpy()
+    am = torch.randn(n, 5, generator=gen)
+    am[:, 2] = am[:, 2].abs() + 2.0
+    am[:, 3] = 1.0
+    am = am.numpy()
+    gx, gy = H.grid(W, Hh)
+    cl = np.ones(gx * gy, bool)
+    bg = np.array([0.3, 0.6, 0.1], np.float32)
+    b = orc.bin_and_sort(radii, means2D, depths, cl, W, Hh)
+    f = orc.render_fwd(b["ranges"], b["point_list"], means2D, rgb, am, co, cl, bg, W, Hh, tan, tan, render_geo=geo)
+    gpix, gmap, gdep = (torch.randn(k, Hh, W, generator=gen).numpy() for k in (3, 5, 1))
+
+    def run(count, place, point_offsets):
+        def spread(a):
+            out = np.zeros((count,) + a.shape[1:], a.dtype)
+            out[place] = a
+            return H.dev(out)
+        point_list = place.astype(np.uint32)[b["point_list"].astype(np.int64)]
+        return H.render_bwd(count, W, Hh, tan, tan, H.dev(bg), H.as_u32(b["ranges"]), H.as_u32(point_list),
+                            spread(means2D), spread(co), spread(rgb), spread(am), H.dev(f["out_all_map"]),
+                            H.dev(f["final_T"]), H.as_u32(f["n_contrib"]), H.dev(cl), H.dev(gpix), H.dev(gmap),
+                            H.dev(gdep), H.as_u32(b["emission_sorted"]), H.as_u32(point_offsets), render_geo=geo)
+
+    offsets = np.asarray(b["point_offsets"])
+    small = run(n, np.arange(n), offsets)
+    place = np.concatenate([np.arange(half), np.arange(P - (n - half), P)])
+    large = run(P, place, np.concatenate([offsets[:half], np.full(P - n, offsets[half - 1], offsets.dtype), offsets[half:]]))
+    index = torch.from_numpy(place).cuda()
+    for k in ("dL_dmeans2D", "dL_dmeans2D_abs", "dL_dconic_opacity", "dL_dcolors", "dL_dall_map"):
+        assert large[k].shape[0] == P
+        assert torch.equal(large[k][index], small[k]), k
+        assert not large[k][half:P - (n - half)].any(), k
