@@ -56,6 +56,22 @@ __device__ __forceinline__ float4 block_test_params(float4 co, float2 xy, float 
   return make_float4(cp.x, cp.y, never ? -1.0f : (untrusted ? cp.z : mark_limit), 0.f);
 }
 
+// bits <- 4 bits + 2 [a does not exceed limit_a] + [b does not exceed limit_b], NaNs not exceeding: each answer is shifted
+// in at bit 0, as the carry of bits + bits.  A vector instruction that reads a lane mask needs two issue slots between it
+// and the vector instruction that wrote the mask, and the compiler does not look into the statement to put them there: the
+// other comparison, the other addition and one idle slot are in between.
+__device__ __forceinline__ void shift_in_two(uint32_t& bits, float a, float limit_a, float b, float limit_b) {
+  uint64_t mask;
+  asm("v_cmp_ngt_f32 %1, %2, %3\n\t"
+      "v_cmp_ngt_f32 vcc, %4, %5\n\t"
+      "s_nop 0\n\t"
+      "v_addc_co_u32 %0, %1, %0, %0, %1\n\t"
+      "v_addc_co_u32 %0, vcc, %0, %0, vcc"
+      : "+v"(bits), "=&s"(mask)
+      : "v"(a), "v"(limit_a), "v"(b), "v"(limit_b)
+      : "vcc");
+}
+
 // The sixteen 4x4 pixel blocks of the tile at (tile_x0, tile_y0): bit 4 k + r of the result is block r of quadrant k
 // (quadrant k at offset 8 (k & 1), 8 (k >> 1), block r in it at 4 (r & 1), 4 (r >> 1)): can any point of the block have
 // q <= limit?  q is convex, so over a block it is smallest either at the centre (inside the block: 0) or on one of the two
@@ -86,18 +102,16 @@ __device__ __forceinline__ uint32_t ellipse_hits_tile(float2 mu, float4 co, floa
       const float t2 = -co.y * dyc * inv_a;                      // where q is smallest along that row
       const float a2 = co.z * dyc * dyc;
       const float b2 = two_b * dyc;
+      float nearest[2];
 #pragma unroll
-      for (int c = 1; c >= 0; c--) {
+      for (int c = 0; c < 2; c++) {
         const float dy1 = __builtin_amdgcn_fmed3f(t1[c], loy, hiy);  // best point of the column x = dxc
         const float q1 = __builtin_fmaf(__builtin_fmaf(co.z, dy1, b1[c]), dy1, a1[c]);
         const float dx2 = __builtin_amdgcn_fmed3f(t2, lox[c], lox[c] + 3.0f);  // best point of the row y = dyc
         const float q2 = __builtin_fmaf(__builtin_fmaf(co.x, dx2, b2), dx2, a2);
-        // (a hit is shifted in at bit 0, as the carry of hits + hits)
-        asm("v_cmp_ngt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"
-            : "+v"(hits)
-            : "v"(fminf(q1, q2)), "v"(limit)
-            : "vcc");
+        nearest[c] = fminf(q1, q2);
       }
+      shift_in_two(hits, nearest[1], limit, nearest[0], limit);
     }
   }
   // row d of columns 2 h, 2 h + 1 are blocks 2 (d & 1), 2 (d & 1) + 1 of quadrant 2 (d >> 1) + h

@@ -282,17 +282,19 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         for (int q = (int)words - 1; q >= 0; q--) {
           const uint32_t word = s_idx[wave][row][(base >> 2) + (uint32_t)q];  // (zero, slot 0, behind the list's end)
 #pragma unroll
-          for (int u = 3; u >= 0; u--) {
-            const int j = (int)__builtin_amdgcn_ubfe(word, 8u * u, 8u);
-            const float4 g0 = s_geo0[j];
-            const float2 g1 = *reinterpret_cast<const float2*>(&s_geo1[j]);  // C and the mark limit
-            const float dx = g0.x - pfx, dy = g0.y - pfy;
-            const float form = __builtin_fmaf(g1.x * dy, dy, __builtin_fmaf(g0.z, dx, g0.w * dy) * dx);
+          for (int u = 3; u >= 0; u -= 2) {
+            float form[2], limit[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+              const int j = (int)__builtin_amdgcn_ubfe(word, 8u * (u - k), 8u);
+              const float4 g0 = s_geo0[j];
+              const float2 g1 = *reinterpret_cast<const float2*>(&s_geo1[j]);  // C and the mark limit
+              const float dx = g0.x - pfx, dy = g0.y - pfy;
+              form[k] = __builtin_fmaf(g1.x * dy, dy, __builtin_fmaf(g0.z, dx, g0.w * dy) * dx);
+              limit[k] = g1.y;
+            }
             // marked unless the form exceeds the limit (so a NaN marks, as the blend's own tests let it through)
-            asm("v_cmp_ngt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"
-                : "+v"(marks)
-                : "v"(form), "v"(g1.y)
-                : "vcc");
+            shift_in_two(marks, form[0], limit[0], form[1], limit[1]);
           }
         }
         {
