@@ -167,11 +167,12 @@ __device__ __forceinline__ float gs_expf(float x) {
 }
 
 // -2 times the exponent of a Gaussian at offset (dx, dy) from its centre (cuda_rasterizer/forward.cu:366), of the conic
-// (A, 2 B, C): the operations of the exponent in its order, every intermediate result -2 times (or twice) the
-// exponent's own.  Scaling by a power of two is exact, so this is the same number as long as nothing overflows, and what
-// overflows lies outside the window either way.
-__device__ __forceinline__ float gauss_form(const float a, const float b2, const float c, const float dx, const float dy) {
-  return (a * dx * dx + c * dy * dy) + b2 * dx * dy;
+// (A, B, C): the operations of the exponent in its order.  Scaling by a power of two is exact, so this is the same number,
+// or an infinity where only the scaled one overflows, outside the window as the number itself is.  (The product with B is
+// doubled inside the last addition: doubled before, it can overflow to the infinity that turns a sum of squares which
+// overflows too into a NaN, and a NaN blends.)
+__device__ __forceinline__ float gauss_form(const float a, const float b, const float c, const float dx, const float dy) {
+  return __builtin_fmaf(b * dx * dy, 2.0f, a * dx * dx + c * dy * dy);
 }
 
 // An exponent below -87 is no exponent: gs_expf is 0 there.

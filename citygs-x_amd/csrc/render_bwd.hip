@@ -118,7 +118,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   static_assert(LIST_BYTES <= 2 * GS_WAVE, "a wave clears its four lists in two rounds");
   // What a wave has staged.  (Slot SLOTS: what an entry behind the end of a list refers to, a Gaussian of opacity 0.)
   __shared__ float4 s_xyp[WAVES][SLOTS + 1];  // centre x, y; as bits: the position in the list; 1 thin, 2 exact
-  __shared__ float4 s_co[WAVES][SLOTS + 1];   // the conic as (A, 2 B, C), and -1/2 of the opacity
+  __shared__ float4 s_co[WAVES][SLOTS + 1];   // the conic, and -1/2 of the opacity
   // colour, then the five geometry channels: eight floats per Gaussian, read as two 16-byte words
   __shared__ float4 s_chan[WAVES][SLOTS + 1][RENDER_GEO ? 2 : 1];
   // accumulators: word 4 slot + (part ^ (slot / 4 & 3)) holds sums 4 part .. 4 part + 3 of a slot, so that
@@ -364,7 +364,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // with the loaded values merged across the two routes the compiler splits the gathers into single words.)
         auto stage = [&](const float2 xy, const float4 co, const float c0, const float c1, const float c2,
                          const float (&m)[GS_N_MAP]) {
-          s_co[wave][lane] = make_float4(co.x, 2.0f * co.y, co.z, -0.5f * co.w);
+          s_co[wave][lane] = make_float4(co.x, co.y, co.z, -0.5f * co.w);
           is_thin = !(co.y * co.y < THIN * co.x * co.z);
           s_xyp[wave][lane] =
               make_float4(xy.x, xy.y, __int_as_float(pos),
@@ -556,13 +556,13 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           channels(grad_t[0], c_lo);
           if (render_geo) channels(grad_t[RENDER_GEO ? 1 : 0], c_hi);
         }
-        const float dx = xyp.x - pfx, b = 0.5f * co.y, a_dx = co.x * dx, b_dx = b * dx;
+        const float dx = xyp.x - pfx, a_dx = co.x * dx, b_dx = co.y * dx;
         float dy[4], q_dy[4], ax = 0.f, ay = 0.f;
 #pragma unroll
         for (int p = 0; p < 4; p++) {
           dy[p] = xyp.y - (block_y0 + (float)p);
           q_dy[p] = q[p] * dy[p];
-          const float ux = __builtin_fmaf(b, dy[p], a_dx), uy = __builtin_fmaf(co.z, dy[p], b_dx);
+          const float ux = __builtin_fmaf(co.y, dy[p], a_dx), uy = __builtin_fmaf(co.z, dy[p], b_dx);
           ax = __builtin_fmaf(fabsf(q[p]), fabsf(ux), ax);
           ay = __builtin_fmaf(fabsf(q[p]), fabsf(uy), ay);
         }
@@ -643,9 +643,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         }
         // (the sums are those of -2 q)
         const float4 co = (&s_co[0][0])[staged];
-        const float b = 0.5f * co.y;
         if (part == 0) {  // mean2D x, y and their sums of absolute values
-          c = make_float4(-co.w * (co.x * c.x + b * c.y), -co.w * (b * c.x + co.z * c.y), c.z * fabsf(co.w),
+          c = make_float4(-co.w * (co.x * c.x + co.y * c.y), -co.w * (co.y * c.x + co.z * c.y), c.z * fabsf(co.w),
                           c.w * fabsf(co.w));
         } else if (part == 1) {  // conic x, y, w; the fourth component is the opacity gradient itself
           const float h = -0.5f * co.w;

@@ -76,7 +76,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   // launched ahead of the host's decision on how the per-tile lists are built: nothing to do if they were not
   if (fits_word != nullptr && *fits_word == 0u) return;
   __shared__ float s_depth[MAX_DEPTH ? BATCH : 1];
-  // a slot's geometry, (x, y, A, 2 B) and (C, mark limit, -opacity / 2, unused), and its channels, (r, g, b, map0)
+  // a slot's geometry, (x, y, A, B) and (C / 4, mark limit, C, -opacity / 2), and its channels, (r, g, b, map0)
   // and (map1 .. map4), in four arrays of 16-byte elements: one address per slot serves them all, and lanes
   // that read different slots spread over all the banks
   __shared__ float4 s_geo0[BATCH];
@@ -167,8 +167,8 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         asm volatile("" : "+s"(ox), "+s"(oy));  // (as in not_hoisted)
         const float tile_x0 = (float)ox, tile_y0 = (float)oy;
         const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
-        s_geo0[ts] = make_float4(xy.x, xy.y, co.x, 2.0f * co.y);
-        s_geo1[ts] = make_float4(co.z, mark_limit, -0.5f * co.w, 0.f);
+        s_geo0[ts] = make_float4(xy.x, xy.y, co.x, co.y);
+        s_geo1[ts] = make_float4(0.25f * co.z, mark_limit, co.z, -0.5f * co.w);
         float mag = fmaxf(fmaxf(fabsf(c0), fabsf(c1)), fabsf(c2));
         bool fin = c0 == c0 && c1 == c1 && c2 == c2;
         if (render_geo) {
@@ -276,6 +276,10 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
       const uint8_t* const my_list = reinterpret_cast<const uint8_t*>(&s_idx[wave][row][0]);
       for (uint32_t base = 0; base < passes; base += CHUNK) {
         uint32_t marks = 0u;
+        // (the marking step works on 2 dy and C / 4, so that the conic's B serves it and the blend as it is)
+        float pfy_m2 = pfy;
+        asm volatile("" : "+v"(pfy_m2));  // (as in not_hoisted)
+        pfy_m2 *= -2.0f;
         const uint32_t words = min((uint32_t)CHUNK / 4u, (passes - base + 3u) / 4u);
         // (last entry first: a mark is shifted in at bit 0, as the carry of marks + marks, so entry e of the chunk
         // ends at bit e)
@@ -288,9 +292,9 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
             for (int k = 0; k < 2; k++) {
               const int j = (int)__builtin_amdgcn_ubfe(word, 8u * (u - k), 8u);
               const float4 g0 = s_geo0[j];
-              const float2 g1 = *reinterpret_cast<const float2*>(&s_geo1[j]);  // C and the mark limit
-              const float dx = g0.x - pfx, dy = g0.y - pfy;
-              form[k] = __builtin_fmaf(g1.x * dy, dy, __builtin_fmaf(g0.z, dx, g0.w * dy) * dx);
+              const float2 g1 = *reinterpret_cast<const float2*>(&s_geo1[j]);  // C / 4 and the mark limit
+              const float dx = g0.x - pfx, dy2 = __builtin_fmaf(g0.y, 2.0f, pfy_m2);
+              form[k] = __builtin_fmaf(g1.x * dy2, dy2, __builtin_fmaf(g0.z, dx, g0.w * dy2) * dx);
               limit[k] = g1.y;
             }
             // marked unless the form exceeds the limit (so a NaN marks, as the blend's own tests let it through)
@@ -312,7 +316,8 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           const uint32_t j = slot_next;
           marks &= marks - 1u;
           slot_next = my_list[base + ((uint32_t)__builtin_ctz(marks | 0x80000000u))];
-          const float4 g0 = s_geo0[j], g1 = s_geo1[j];
+          const float4 g0 = s_geo0[j];
+          const float2 g1 = *(reinterpret_cast<const float2*>(&s_geo1[j]) + 1);  // C and -opacity / 2
           float c[GS_N_RGB + GS_N_MAP] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
           {
             const float4 c0 = s_col0[j];
@@ -326,7 +331,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           if (MAX_DEPTH) depth_j = s_depth[j];
 
           const float form = gauss_form(g0.z, g0.w, g1.x, g0.x - pfx, g0.y - pfy);
-          const float alpha = fminf(0.99f, g1.z * gs_neg2_exp_of_form(form));
+          const float alpha = fminf(0.99f, g1.y * gs_neg2_exp_of_form(form));
           // the lanes whose entry counts: they have one in this pass, the exponent lies in the window and alpha reaches
           // 1/255 (a NaN passes: the reference blends it too).  Lane masks of single comparisons, combined in scalar
           // registers.

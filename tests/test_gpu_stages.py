@@ -443,6 +443,50 @@ def test_long_thin_splats_far_from_their_centre(H, orc, seed, reach):
     assert np.array_equal(got["color"].cpu().numpy(), ref["color"])
 
 
+@pytest.mark.parametrize("geo", [True, False])
+def test_an_exponent_whose_terms_overflow(H, orc, geo):
+    """A conic so large that the squares of the exponent overflow, and its product term where that is doubled but not as it
+    is: the exponent is minus infinity there and the Gaussian blends nowhere.  In front of it and behind it are others."""
+    gen = torch.Generator().manual_seed(1)
+    W = Hh = 9
+    P = 6
+    means2D = (torch.rand(P, 2, generator=gen) * 9.0).numpy()
+    co = np.tile(np.array([0.05, 0.01, 0.05, 0.4], np.float32), (P, 1))
+    for k in (1, 4):
+        means2D[k] = (0.25, 0.5)
+        co[k] = (1e37, -4e36, 1e37, 0.5)
+    dx, dy = np.float32(0.25) - np.arange(9, dtype=np.float32), np.float32(0.5) - np.arange(9, dtype=np.float32)
+    with np.errstate(over="ignore"):
+        term = np.float32(-4e36) * dx[None, :] * dy[:, None]
+        squares = np.float32(1e37) * dx[None, :] * dx[None, :] + np.float32(1e37) * dy[:, None] * dy[:, None]
+        assert np.isfinite(term).all() and (np.isinf(squares) & (2 * term == -np.inf)).sum() > 5
+    rgb, am = torch.rand(P, 3, generator=gen).numpy(), torch.randn(P, 5, generator=gen).numpy()
+    am[:, 2] = np.abs(am[:, 2]) + 2.0
+    radii, depths = np.full(P, 50, np.int32), np.arange(1, P + 1).astype(np.float32)
+    cl, bg, tan = np.ones(1, bool), np.array([0.3, 0.6, 0.1], np.float32), 0.5
+    b = orc.bin_and_sort(radii, means2D, depths, cl, W, Hh)
+    f = orc.render_fwd(b["ranges"], b["point_list"], means2D, rgb, am, co, cl, bg, W, Hh, tan, tan, render_geo=geo)
+    got = H.render_fwd(P, W, Hh, tan, tan, H.as_u32(b["ranges"]), H.as_u32(b["point_list"]), H.dev(means2D), H.dev(rgb),
+                       H.dev(am), H.dev(co), H.dev(cl), H.dev(bg), render_geo=geo)
+    assert f["out_observe"][1] == f["out_observe"][4] == 0 and f["n_contrib"].max() == P
+    for k in ("n_contrib", "n_contrib2loss"):
+        assert np.array_equal(H.np_u32(got[k]), f[k]), k
+    for k in ("out_observe", "final_T", "color"):
+        assert np.array_equal(got[k].cpu().numpy(), f[k]), k
+    gpix, gmap, gdep = (torch.randn(k, Hh, W, generator=gen).numpy() for k in (3, 5, 1))
+    ref = orc.render_bwd(b["ranges"], b["point_list"], means2D, co, rgb, am, f["out_all_map"], f["final_T"],
+                         f["n_contrib"], cl, bg, gpix, gmap, gdep, W, Hh, tan, tan, render_geo=geo)
+    back = H.render_bwd(P, W, Hh, tan, tan, H.dev(bg), H.as_u32(b["ranges"]), H.as_u32(b["point_list"]), H.dev(means2D),
+                        H.dev(co), H.dev(rgb), H.dev(am), H.dev(f["out_all_map"]), H.dev(f["final_T"]),
+                        H.as_u32(f["n_contrib"]), H.dev(cl), H.dev(gpix), H.dev(gmap), H.dev(gdep),
+                        H.as_u32(b["emission_sorted"]), H.as_u32(b["point_offsets"]), render_geo=geo)
+    for k, want in (("dL_dmeans2D", ref["dL_dmeans2D"][:, :2]), ("dL_dconic_opacity", ref["dL_dconic_opacity"]),
+                    ("dL_dcolors", ref["dL_dcolors"])):
+        a = back[k].cpu().numpy()
+        assert not a[[1, 4]].any(), k
+        assert H.rel_l2(a, want) <= GRAD_TOL, (k, H.rel_l2(a, want))
+
+
 def test_needles_through_the_whole_forward_pass(H, orc):
     """Needle-shaped Gaussians (one axis 10^3 to 10^5 times the others, tens to hundreds of metres long) around
     and in front of the camera: after projection their conics have one eigenvalue at the dilation limit and one
