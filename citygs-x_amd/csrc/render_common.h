@@ -40,7 +40,7 @@ __device__ __forceinline__ float4 cull_params(float4 co, float& power_floor) {
 // with it).  Both limits are q_max plus a margin for rounding: the block test, the pixel mark and the blend itself
 // evaluate q by different operation sequences at different points, each within a few units in the last place of
 // the LARGEST term, which for a long thin Gaussian far from its centre is much larger than q itself.  Every such
-// term is at most S = A X^2 + 2 |B| X Y + C Y^2 with X, Y the largest offsets of a pixel of the tile from the
+// term is at most S = |A| X^2 + 2 |B| X Y + |C| Y^2 with X, Y the largest offsets of a pixel of the tile from the
 // centre; the margin is 2e-6 S (about 32 units in the last place of S), on top of the 0.02 from tau + 0.01.  The
 // block limit is negative when the opacity alone rules every pixel out and +infinity when the conic cannot be
 // trusted.  The same numbers in the forward and the backward kernel, so both build the same lists.
@@ -49,7 +49,7 @@ __device__ __forceinline__ float4 block_test_params(float4 co, float2 xy, float 
   const float4 cp = cull_params(co, power_floor);
   const float far_x = fmaxf(fabsf(xy.x - tile_x0), fabsf(xy.x - (tile_x0 + (float)(GS_TILE_X - 1))));
   const float far_y = fmaxf(fabsf(xy.y - tile_y0), fabsf(xy.y - (tile_y0 + (float)(GS_TILE_Y - 1))));
-  const float spread = co.x * far_x * far_x + 2.0f * fabsf(co.y) * far_x * far_y + co.z * far_y * far_y;
+  const float spread = fabsf(co.x) * far_x * far_x + 2.0f * fabsf(co.y) * far_x * far_y + fabsf(co.z) * far_y * far_y;
   // (q_max = 2 (tau + 0.01) is -2 power_floor wherever the conic is trusted)
   mark_limit = __builtin_fmaf(2e-6f, spread, -2.0f * power_floor);
   const bool never = cp.z < 0.f, untrusted = cp.z == __builtin_inff();

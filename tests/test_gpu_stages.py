@@ -443,6 +443,37 @@ def test_long_thin_splats_far_from_their_centre(H, orc, seed, reach):
     assert np.array_equal(got["color"].cpu().numpy(), ref["color"])
 
 
+@pytest.mark.parametrize("seed,terms", [(0, 1e5), (1, 1e6), (2, 1e7)])
+def test_indefinite_conics_far_from_their_centre(H, orc, seed, terms):
+    """Conics whose squares have opposite signs (from a covariance that is not positive definite) and cancel in the image,
+    a million pixels from the centre: each term of the exponent is about `terms`, their sum is decided by rounding, and the
+    marking step must not drop an entry that the blend counts."""
+    gen = torch.Generator().manual_seed(40 + seed)
+    P, W, Hh, far = 400, 64, 48, 1e6
+    gx, gy = H.grid(W, Hh)
+    r = lambda *s: torch.rand(*s, generator=gen, dtype=torch.float64)
+    through = r(P, 2) * torch.tensor([float(W), float(Hh)])
+    ang = (0.15 + 0.7 * r(P)) * (math.pi / 2) + (math.pi / 2) * torch.randint(0, 4, (P,), generator=gen)
+    ux, uy = torch.cos(ang), torch.sin(ang)
+    means2D = torch.stack([through[:, 0] + far * ux, through[:, 1] + far * uy], 1).float().numpy()
+    s = torch.where(r(P) < 0.5, -1.0, 1.0) * terms / far ** 2
+    co = torch.stack([s * uy * uy, torch.zeros(P), -s * ux * ux, r(P) * 0.3 + 0.05], 1).float().numpy()
+    radii = np.full(P, 1 << 21, np.int32)            # every splat is listed in every tile
+    rgb, am = r(P, 3).float().numpy(), torch.randn(P, 5, generator=gen).numpy()
+    depths = (r(P) * 50 + 0.3).float().numpy()
+    cl, bg = np.ones(gx * gy, bool), np.zeros(3, np.float32)
+    bins = orc.bin_and_sort(radii, means2D, depths, cl, W, Hh)
+    ref = orc.render_fwd(bins["ranges"], bins["point_list"], means2D, rgb, am, co, cl, bg, W, Hh, 0.8, 0.6,
+                         render_geo=True)
+    got = H.render_fwd(P, W, Hh, 0.8, 0.6, H.as_u32(bins["ranges"]), H.as_u32(bins["point_list"]), H.dev(means2D),
+                       H.dev(rgb), H.dev(am), H.dev(co), H.dev(cl), H.dev(bg), render_geo=True)
+    assert ref["n_contrib2loss"].sum() > 100
+    for k in ("n_contrib", "n_contrib2loss"):
+        assert np.array_equal(H.np_u32(got[k]), ref[k]), (k, int((H.np_u32(got[k]) != ref[k]).sum()))
+    for k in ("out_observe", "final_T", "color"):
+        assert np.array_equal(got[k].cpu().numpy(), ref[k]), k
+
+
 @pytest.mark.parametrize("geo", [True, False])
 def test_an_exponent_whose_terms_overflow(H, orc, geo):
     """A conic so large that the squares of the exponent overflow, and its product term where that is doubled but not as it
