@@ -233,7 +233,8 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_setti
 
 # ------------------------------------------------------------------- render --
 
-# What the last view of a given image size needed, (instances, longest list) keyed by (height, width, device): the
+# What the last view of a given image size needed, (instances, longest list, whether any view of the size had a list
+# beyond _LONG_LIST) keyed by (height, width, device): the
 # next view of that size is launched without waiting for its instance count, on buffers sized for these figures plus
 # a margin (a training loop renders thousands of similar views; the number of Gaussians changes at every
 # densification, so it is not part of the key).  Only the time depends on it, never a result; a stale or missing
@@ -242,27 +243,29 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_setti
 _expectations = {}
 _MARGIN = 1.25
 _MAX_EXPECTATIONS = 16
+_LONG_LIST = 4096  # what the smaller of the radix sort's kernels holds
 
 
 def _expectation(key):
     seen = _expectations.get(key)
     if seen is None:
         return 0, 0
-    instances, longest = seen
+    instances, longest, *long = seen
     if longest <= 0:
         return 0, 0  # a view without per-tile lists (a tile grid too large for them): nothing to gain
     # whole variants of the register sort (256 ... 2048 records per list), so that a slightly longer list still
-    # fits, then what the smaller of the radix sort's kernels holds (4096); beyond it any length (0): the larger one
-    # is launched as well
+    # fits, then what the smaller of the radix sort's kernels holds; beyond it any length (0): the larger one
+    # is launched as well.  So it is for lists beyond the register sort wherever a view of this size has had a longer one:
+    # cameras on both sides of that length would miss the bound at every other view, for the 4.6 us of an empty launch.
     cap = 256
     while cap < longest * _MARGIN:
         cap *= 2
-    return int(instances * _MARGIN) + 65536, (cap if cap <= 4096 else 0)
+    return int(instances * _MARGIN) + 65536, (0 if cap > _LONG_LIST or (cap == _LONG_LIST and any(long)) else cap)
 
 
 def _remember(key, instances, longest):
-    _expectations.pop(key, None)  # (re-inserted at the end: the dict keeps insertion order)
-    _expectations[key] = (instances, longest)
+    seen = _expectations.pop(key, ())  # (re-inserted at the end: the dict keeps insertion order)
+    _expectations[key] = (instances, longest, longest > _LONG_LIST or any(seen[2:]))
     while len(_expectations) > _MAX_EXPECTATIONS:
         # (a copy to look at: another thread may be adding entries, or have removed this one)
         _expectations.pop(list(_expectations)[0], None)

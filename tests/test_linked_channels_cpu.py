@@ -342,3 +342,24 @@ def test_expectations_remembered_by_several_threads():
     finally:
         sys.setswitchinterval(interval)
         dgr._expectations.clear()
+
+
+def test_expectations_of_cameras_on_both_sides_of_a_long_list():
+    # (instances, longest list) of the views of one size, and the bound on the longest list that the next one is launched
+    # with: 0 is any length
+    import diff_gaussian_rasterization as dgr
+    saved = dict(dgr._expectations)
+    dgr._expectations.clear()
+    try:
+        bounds = []
+        for longest in (100, 1638, 1639, 3276, 4500, 3000, 4500, 3276, 1639, 1638, 100, 3000):
+            dgr._remember("size", 1000, longest)
+            bounds.append(dgr._expectation("size")[1])
+        assert bounds == [256, 2048, 4096, 4096, 0, 0, 0, 0, 0, 2048, 256, 0]
+        dgr._remember("another size", 1000, 3000)
+        assert dgr._expectation("another size") == (int(1000 * dgr._MARGIN) + 65536, 4096)
+        dgr._expectations["size"] = (1000, 3000)  # (an entry without the third figure)
+        assert dgr._expectation("size")[1] == 4096
+    finally:
+        dgr._expectations.clear()
+        dgr._expectations.update(saved)
