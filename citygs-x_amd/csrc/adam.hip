@@ -29,6 +29,9 @@ constexpr int ADAM_CHUNK = ADAM_THREADS * ADAM_VEC;  // elements per workgroup
 // if nothing else runs between them: 17.7 M elements 72 us cached and 79 streamed in a loop of steps, 23.6 M 112 and 106.
 // (With 640 MB written between the steps streaming is the faster at every size: 17.7 M 85 against 106 us, 1.2 M 11 against 13.)
 constexpr long long ADAM_STREAM_ELEMENTS = 20'000'000;
+// A launch's threads are counted in 32 bits (2^25 workgroups), and the tensors of one step may fill the memory with more:
+// a launch takes at most this many workgroups (537 M elements, 2.4 ms), and a tensor that does not fit goes on in the next.
+constexpr int ADAM_MAX_CHUNKS = 1 << 20;
 
 struct AdamTable {
   float* p[ADAM_MAX_TENSORS];
@@ -120,7 +123,53 @@ adam_kernel(const AdamTable t, float b1, float omb1, float b2, float omb2, float
   }
 }
 
+// The next launch of a step over `count` tensors: slice i is the elements first[i] .. first[i] + n[i] - 1 of tensor
+// index[i] and begins at workgroup first_chunk[i].  (tensor, element) is where the launch begins and is moved on; no slice
+// is left when all tensors are done.
+struct AdamSlices {
+  int count, chunks;
+  int index[ADAM_MAX_TENSORS], first_chunk[ADAM_MAX_TENSORS];
+  long long first[ADAM_MAX_TENSORS], n[ADAM_MAX_TENSORS];
+};
+
+AdamSlices adam_next_launch(int count, const long long* sizes, int& tensor, long long& element) {
+  AdamSlices s;
+  s.count = s.chunks = 0;
+  while (tensor < count && s.count < ADAM_MAX_TENSORS && s.chunks < ADAM_MAX_CHUNKS) {
+    const long long left = sizes[tensor] - element, room = (long long)(ADAM_MAX_CHUNKS - s.chunks) * ADAM_CHUNK;
+    const long long n = left < room ? left : room;
+    if (n > 0) {
+      s.index[s.count] = tensor;
+      s.first_chunk[s.count] = s.chunks;
+      s.first[s.count] = element;
+      s.n[s.count++] = n;
+      s.chunks += (int)((n + ADAM_CHUNK - 1) / ADAM_CHUNK);
+      element += n;
+    }
+    if (n == left || left <= 0) {
+      tensor++;
+      element = 0;
+    }
+  }
+  return s;
+}
+
 }  // namespace
+
+long long adam_plan(int count, const long long* sizes, long long* out, long long capacity) {
+  long long rows = 0;
+  int tensor = 0;
+  long long element = 0;
+  for (int launch = 0;; launch++) {
+    const AdamSlices s = adam_next_launch(count, sizes, tensor, element);
+    if (s.count == 0) return rows;
+    for (int i = 0; i < s.count; i++, rows++) {
+      if (rows >= capacity) continue;
+      const long long row[5] = {launch, s.index[i], s.first[i], s.n[i], (long long)s.chunks * ADAM_THREADS};
+      for (int k = 0; k < 5; k++) out[5 * rows + k] = row[k];
+    }
+  }
+}
 
 int launch_adam(int count, float* const* params, const float* const* grads, float* const* exp_avg,
                 float* const* exp_avg_sq, const long long* sizes, const double* lrs, const int* steps, double beta1,
@@ -128,30 +177,29 @@ int launch_adam(int count, float* const* params, const float* const* grads, floa
   long long elements = 0;
   for (int i = 0; i < count; i++) elements += sizes[i] > 0 ? sizes[i] : 0;
   const auto kernel = elements > ADAM_STREAM_ELEMENTS ? adam_kernel<true> : adam_kernel<false>;
-  int done = 0;
-  while (done < count) {
+  int tensor = 0;
+  long long element = 0;
+  for (;;) {
+    const AdamSlices s = adam_next_launch(count, sizes, tensor, element);
+    if (s.count == 0) break;
     AdamTable t;
-    int k = 0, chunks = 0;
-    for (; done < count && k < ADAM_MAX_TENSORS; done++) {
-      if (sizes[done] <= 0) continue;
-      t.p[k] = params[done];
-      t.g[k] = grads[done];
-      t.m[k] = exp_avg[done];
-      t.v[k] = exp_avg_sq[done];
-      t.n[k] = sizes[done];
+    for (int k = 0; k < s.count; k++) {
+      const int i = s.index[k];
+      t.p[k] = params[i] + s.first[k];
+      t.g[k] = grads[i] + s.first[k];
+      t.m[k] = exp_avg[i] + s.first[k];
+      t.v[k] = exp_avg_sq[i] + s.first[k];
+      t.n[k] = s.n[k];
       // bias corrections in double, like the Python floats of the reference optimizer
-      const double bc1 = 1.0 - pow(beta1, (double)steps[done]);
-      const double bc2 = 1.0 - pow(beta2, (double)steps[done]);
-      t.neg_step_size[k] = (float)(-(lrs[done] / bc1));
+      const double bc1 = 1.0 - pow(beta1, (double)steps[i]);
+      const double bc2 = 1.0 - pow(beta2, (double)steps[i]);
+      t.neg_step_size[k] = (float)(-(lrs[i] / bc1));
       t.bc2_sqrt[k] = (float)sqrt(bc2);
-      t.first_chunk[k] = chunks;
-      chunks += (int)((sizes[done] + ADAM_CHUNK - 1) / ADAM_CHUNK);
-      k++;
+      t.first_chunk[k] = s.first_chunk[k];
     }
-    if (k == 0) break;
-    t.first_chunk[k] = chunks;
-    t.count = k;
-    hipLaunchKernelGGL(kernel, dim3(chunks), dim3(ADAM_THREADS), 0, stream, t, (float)beta1,
+    t.first_chunk[s.count] = s.chunks;
+    t.count = s.count;
+    hipLaunchKernelGGL(kernel, dim3(s.chunks), dim3(ADAM_THREADS), 0, stream, t, (float)beta1,
                        (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), (float)eps, grad_scale);
   }
   return 0;

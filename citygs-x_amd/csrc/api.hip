@@ -1443,6 +1443,10 @@ int gs_selftest_reciprocal(uint32_t first, uint32_t n, uint32_t* out, gs_stream_
   return check_launch("selftest_reciprocal", (hipStream_t)stream, true);
 }
 
+long long gs_selftest_adam_plan(int count, const long long* sizes, long long* out, long long capacity) {
+  return adam_plan(count, sizes, out, capacity);
+}
+
 int gs_selftest_quads(const float* in, float* out, gs_stream_t stream) {
   GS_REQUIRE(in && out, "gs_selftest_quads: null pointer");
   launch_quad_selftest(in, out, (hipStream_t)stream);

@@ -153,6 +153,7 @@ int launch_train_stats(long long A, int k, long long Vk, long long M, const uint
                        float* denom, void* temp, hipStream_t stream);
 int launch_max_radii(long long n, const int* radii, const uint8_t* visible, float* max_radii, hipStream_t stream);
 constexpr int ADAM_MAX_TENSORS = 24;  // tensors per launch (more are split over several launches)
+long long adam_plan(int count, const long long* sizes, long long* out, long long capacity);
 int launch_adam(int count, float* const* params, const float* const* grads, float* const* exp_avg,
                 float* const* exp_avg_sq, const long long* sizes, const double* lrs, const int* steps, double beta1,
                 double beta2, double eps, float grad_scale, hipStream_t stream);

@@ -114,6 +114,7 @@ _SIGNATURES = {
     "gs_selftest_reductions": (_i, [_vp, _vp, _vp, _vp]),
     "gs_selftest_quads": (_i, [_vp, _vp, _vp]),
     "gs_selftest_reciprocal": (_i, [C.c_uint32, C.c_uint32, _vp, _vp]),
+    "gs_selftest_adam_plan": (C.c_longlong, [_i, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong), C.c_longlong]),
     "gs_stage_timing_enable": (_i, [_i]),
     "gs_stage_timing_collect": (_i, [C.c_char_p, _sz]),
     "gs_image_state_layout": (_i, [_i, _i] + [_psz] * 5),

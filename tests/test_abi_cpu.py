@@ -168,3 +168,26 @@ assert not hasattr(gn, "nothing_of_that_name")
 """ % os.path.join(ROOT, "citygs-x_amd")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.stdout, r.stderr)
+
+
+def test_adam_steps_of_any_size_fit_their_launches():
+    """A launch has fewer than 2^32 threads; 2^34 elements of four arrays fit the card's memory."""
+    import gsrast_native as gn
+    for sizes in ([], [0, -1], [1], [511, 512, 513, 0, 5], [2 ** 34 + 77], [2 ** 33, 2 ** 33, 0, 3],
+                  [2 ** 29], [2 ** 29 + 1, 7], [2 ** 29 - 512, 512, 1], [2 ** 29 - 511, 512], [100] * 70, [2 ** 28] * 40):
+        n = len(sizes)
+        out = (C.c_longlong * 2000)()
+        rows = gn.lib.gs_selftest_adam_plan(n, (C.c_longlong * max(n, 1))(*sizes), out, 400)
+        assert rows <= 400
+        table = np.array(out[:5 * rows], np.int64).reshape(rows, 5)
+        done = [0] * n
+        for launch, tensor, first, elements, threads in table:
+            assert first == done[tensor] and first % 4 == 0 and elements > 0  # (16-byte accesses stay aligned)
+            done[tensor] += int(elements)
+            assert 0 < threads < 2 ** 32
+        assert done == [max(k, 0) for k in sizes]
+        for launch in set(table[:, 0].tolist()):
+            mine = table[table[:, 0] == launch]
+            # 128 threads per 512 elements of a slice; a launch follows when the one before it is full
+            assert (mine[:, 4] == 128 * ((mine[:, 3] + 511) // 512).sum()).all()
+        assert (np.diff(table[:, 0]) >= 0).all() and (np.diff(table[:, 0]) <= 1).all()

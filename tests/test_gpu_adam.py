@@ -19,7 +19,7 @@ def _rel(a, b):
 def test_adam_c_abi_matches_oracle(orc):
     import gsrast_native as gn
     gen = torch.Generator().manual_seed(3)
-    # sizes around the 4096-element workgroup chunk, a misaligned view, an empty tensor, 30 tensors (> one launch)
+    # sizes around eight 512-element workgroup chunks, a misaligned view, an empty tensor, 30 tensors (> one launch)
     sizes = [1, 3, 4095, 4096, 4097, 100_003, 0, 1_000_000] + [17 + 13 * i for i in range(22)]
     store = [torch.randn(n + 1, generator=gen).to(DEV) for n in sizes]
     before5 = float(store[5][0])
@@ -119,3 +119,26 @@ def test_a_step_that_streams_past_the_caches_gives_the_same_bits(sizes):
 
     for a, b in zip(step(0), step(20_000_001)):
         assert torch.equal(a, b)
+
+
+def test_a_step_of_several_launches():
+    # 2^29 elements fill a launch: a tensor that goes on in the next one, and one behind it
+    import gsrast_native as gn
+    sizes = [2 ** 29 + 1000, 513]
+    t = [[torch.full((n,), x, device=DEV) for n in sizes] for x in (1.0, 0.5, 0.25, 0.125)]
+    t[1][0][2 ** 29 - 3:2 ** 29 + 3] = 2.0
+    small = [[a[2 ** 29 - 8:].clone() if i == 0 else a.clone() for i, a in enumerate(k)] for k in t]
+
+    def step(arrays):
+        n = [a.numel() for a in arrays[0]]
+        vp, two = C.c_void_p * 2, C.c_double * 2
+        gn.check(gn.lib.gs_adam_step(2, *[vp(*[a.data_ptr() for a in k]) for k in arrays], (C.c_longlong * 2)(*n),
+                                     two(1e-2, 1e-3), (C.c_int * 2)(3, 4), 0.9, 0.999, 1e-15, 1.0,
+                                     C.c_void_p(torch.cuda.current_stream().cuda_stream)), "gs_adam_step")
+
+    step(t)
+    step(small)
+    for k in (0, 2, 3):
+        assert torch.equal(t[k][0][2 ** 29 - 8:], small[k][0]) and torch.equal(t[k][1], small[k][1])
+        head = t[k][0][:2 ** 29 - 8]
+        assert float(head.amin()) == float(head.amax()) == float(small[k][0][0])
