@@ -193,10 +193,14 @@ Tensor visible_filter(const Tensor& means3D_, const OptTensor& scales_, const Op
   }
   const Tensor rot = f32c(given(rotations_), "rotations"), cov = f32c(given(cov3D_), "cov3D_precomp");
   const Tensor vm = f32c(viewmatrix, "viewmatrix"), pm = f32c(projmatrix, "projmatrix");
-  check(gs_visible_filter_rows((int)P, (int)stride, width, height, ptr(means3D), scales ? ptr(*scales) : nullptr,
-                               scale_modifier, ptr(rot), ptr(cov), ptr(vm), ptr(pm), tan_fovx, tan_fovy, prefiltered,
-                               ptr<int>(radii), debug, stream_of(stream)),
-        "rasterize_aussians_filter");
+  int status;
+  {
+    py::gil_scoped_release nogil;  // (with debug the call waits for the kernel)
+    status = gs_visible_filter_rows((int)P, (int)stride, width, height, ptr(means3D), scales ? ptr(*scales) : nullptr,
+                                    scale_modifier, ptr(rot), ptr(cov), ptr(vm), ptr(pm), tan_fovx, tan_fovy, prefiltered,
+                                    ptr<int>(radii), debug, stream_of(stream));
+  }
+  check(status, "rasterize_aussians_filter");
   return radii;
 }
 

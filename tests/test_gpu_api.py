@@ -723,3 +723,44 @@ def test_visible_filter_reads_scales_in_wider_rows(P):
         rast.visible_filter(means, wide[:, :3].double(), rot)
     with pytest.raises(RuntimeError):
         rast.visible_filter(means, scales.cpu(), rot)
+
+
+def test_visible_filter_that_waits_lets_other_threads_run():
+    # with debug the call waits for everything before it on the stream: some 0.2 s of products here
+    import threading
+    import time
+
+    import gs_scenes
+    from diff_gaussian_rasterization import GaussianRasterizationSettings, GaussianRasterizer
+    g, cams = gs_scenes.make_scene(0, P=300)
+    cam = cams[0]
+    rs = GaussianRasterizationSettings(
+        image_height=cam.image_height, image_width=cam.image_width, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy,
+        bg=torch.zeros(3, device="cuda"), scale_modifier=1.0, viewmatrix=cam.world_view_transform.cuda(),
+        projmatrix=cam.full_proj_transform.cuda(), sh_degree=3, campos=cam.camera_center.cuda(), prefiltered=False,
+        render_geo=True, debug=True)
+    rast = GaussianRasterizer(rs)
+    means, scales, rot = (g[k].cuda() for k in ("means3D", "scales", "rotations"))
+    rast.visible_filter(means, scales, rot)
+    a = torch.randn(8192, 8192, device="cuda")
+    torch.mm(a, a)
+    torch.cuda.synchronize()
+    took = []
+
+    def call():
+        for _ in range(20):
+            torch.mm(a, a)
+        start = time.perf_counter()
+        rast.visible_filter(means, scales, rot)
+        took.append(time.perf_counter() - start)
+
+    worker = threading.Thread(target=call)
+    worker.start()
+    longest, last = 0.0, time.perf_counter()
+    while worker.is_alive():
+        time.sleep(1e-3)
+        now = time.perf_counter()
+        longest, last = max(longest, now - last), now
+    worker.join()
+    assert took and took[0] > 0.05  # (it did wait)
+    assert longest < 0.5 * took[0], (longest, took[0])
