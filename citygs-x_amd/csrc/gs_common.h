@@ -144,8 +144,9 @@ __device__ __forceinline__ float4 load_streaming(const float4* p) {
   return make_float4(w.x, w.y, w.z, w.w);
 }
 
-// exp() of the blending loops: n = rint(x*log2e), r = x - n*ln2 (two-constant
-// split), degree-6 polynomial, scale by 2^n.  Only IEEE operations and explicit
+// exp() of the blending loops: n = rint(x*log2e), r = x - n*ln2 (ln2 split into two
+// constants, after Cody and Waite), the polynomial of expf in S. L. Moshier's Cephes
+// library, scale by 2^n.  Only IEEE operations and explicit
 // FMAs, so a CPU evaluates the same bits.  x < -87 -> 0, x > 88 -> +inf.
 __device__ __forceinline__ float gs_expf(float x) {
   if (!(x == x)) return x;

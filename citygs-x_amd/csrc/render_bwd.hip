@@ -39,17 +39,22 @@
 // reference issues 16 global float atomics per pixel and Gaussian,
 // cuda_rasterizer/backward.cu:510-563.)
 //
-// What bounds it: the vector ALU, which the matrix instructions share (a
-// 4x4x1 one takes the time of five additions).  A pass costs some 770 cycles of
-// it and 16 matrix instructions, about 17 of them a wave at 1 M Gaussians,
-// 1152x864; the steps between the walks a fifth of the whole.  With the staging
-// shared by the four waves (batches of 128, 64 of them walked at a time) there
-// were 13 barriers per 256 entries, three or four now, lists four times shorter
-// and 12 % more passes.  Before and after: 208 -> 197 us there, 491 -> 464 us for
-// 4 M Gaussians from the air, 567 -> 549 us for 10 M at street level, 104 -> 96 us
-// for 300 k without geometry channels.  Four workgroups a CU with 64 slots, or
-// five with 48: 464 and 522 us at 4 M with geometry channels, whose 95 registers
-// would spill with five; without them 56 slots and five (96 us against 106).  The
+// What bounds it: the vector ALU (about 0.7 busy), which the matrix instructions
+// share (a 4x4x1 one takes the time of four additions), and the latency of the
+// LDS reads at the head of a pass (list word, slot, operands, one after the
+// other), which four waves a SIMD do not hide altogether.  A pass has some 300
+// vector instructions of two or four cycles each and 16 matrix instructions, about
+// 17 passes a wave at 1 M Gaussians, 1152x864; the steps between the walks a fifth
+// of the whole.  With the staging shared by the four waves (batches of 128, 64 of
+// them walked at a time) there were 13 barriers per 256 entries; a window has three
+// and a scan of 256 positions one, so that it is four where Gaussians are small and
+// a wave has slots for all of its own, and 13 to 16 where every Gaussian covers
+// the tile and 256 entries take four or five windows.  Lists are four times
+// shorter, passes 12 % more.  Before and after: 208 -> 197 us there, 491 -> 464 us
+// for 4 M Gaussians from the air, 567 -> 549 us for 10 M at street level, 104 -> 96
+// us for 300 k without geometry channels.  Four workgroups a CU with 64 slots, or
+// five with 48: 464 and 522 us at 4 M with geometry channels, whose 118 registers
+// do not fit five; without them 56 slots and five (96 us against 106).  The
 // accumulators' reads a pass ahead of their use gain nothing.
 // The matrix cores take what contracts an operand that all
 // entries or all pixels share; the recurrence itself is a serial chain per
@@ -271,8 +276,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     const float2 xy = means2D[g];
     const float4 co = conic_opacity[g];
     const float tile_x0 = (float)(tile_x * GS_TILE_X), tile_y0 = (float)(tile_y * GS_TILE_Y);
-    float pfl, mark_limit;
-    const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
+    const float4 cp = block_test_params(co, xy, tile_x0, tile_y0);
     return ellipse_hits_tile(xy, co, cp.x, cp.y, cp.z, tile_x0, tile_y0);
   };
   auto sync_wave = [] {
@@ -393,7 +397,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
           stage(xy, co, c0, c1, c2, m);
         }
       }
-      // (every wave has read the accumulators of the window before: the barrier at the end of the loop)
+      // (every wave has read the accumulators of the window before: the barriers above)
 #pragma unroll
       for (int k = 0; k < 4; k++)
         if (k * GS_WAVE + lane < 4 * SLOTS) s_acc[wave][k * GS_WAVE + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -523,7 +527,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         step(std::integral_constant<int, 3>{});
         // (q is -2 times what it stands for below, as G is: the thread that hands the record over takes the factor out)
         // The sums over pixels.  From here on lane e of a quad works for entry e, register p is the quad's pixel p (the
-        // quad's four pixels are one column of the block: dx is the quad's, dy the register's).  The per-Gaussian factors of the geometric gradients stay out of the sums: with
+        // quad's four pixels are one column of the block: dx is the quad's, dy the register's).  The per-Gaussian factors
+        // of the geometric gradients stay out of the sums: with
         // q = G dL/dalpha, u = conic (dx, dy), a pixel's terms are dL/dmean = -opacity q u,
         // dL/dconic = -opacity/2 q (dx dx, dx dy, dy dy) and dL/dopacity = q
         // (cuda_rasterizer/backward.cu:520-541); sum q u is formed from sum q (dx, dy) by the thread that hands the

@@ -10,50 +10,46 @@ namespace gs {
 // Which Gaussians can pass the blend tests of cuda_rasterizer/forward.cu:381-393 (power <= 0 and
 // opacity * exp(power) >= 1/255) somewhere in a block of pixels.  With conic (A, B, C) and
 // tau = ln(255 * opacity), alpha >= 1/255 needs q(d) = A dx^2 + 2 B dx dy + C dy^2 <= 2 tau.
-// cull_params returns (1/A, 1/C, q_max, 0) with q_max = 2 (tau + 0.01).  q_max is +infinity when the conic
-// cannot be trusted (every block then counts as hit) and negative when the opacity alone rules every pixel out.
-// power_floor receives the exponent below which alpha < 1/255 is certain (never below -87, where gs_expf
-// returns 0 anyway): pixels with power < power_floor can skip the exponential.  Culling with these only skips
-// work, it never changes a result.
-__device__ __forceinline__ float4 cull_params(float4 co, float& power_floor) {
+// cull_params returns (1/A, 1/C, q_max, q_pixel) with q_max = q_pixel = 2 (tau + 0.01).  q_max is +infinity when the conic
+// cannot be trusted (every block then counts as hit) and negative when the opacity alone rules every pixel out; q_pixel
+// does not depend on the conic and is never above 174, beyond which gs_expf returns 0 anyway.  Culling with these only
+// skips work, it never changes a result.
+__device__ __forceinline__ float4 cull_params(float4 co) {
   const float inf = __builtin_inff();
   const float o = co.w;
-  power_floor = -87.0f;
-  if (o < 0.0039f) return make_float4(0.f, 0.f, -1.0f, 0.f);
-  float4 cp = make_float4(0.f, 0.f, inf, 0.f);
+  if (o < 0.0039f) return make_float4(0.f, 0.f, -1.0f, GS_FORM_MAX);
+  float4 cp = make_float4(0.f, 0.f, inf, GS_FORM_MAX);
   if (o < 1.0e30f) {
     const float tau = __logf(255.0f * o) + 0.01f;
     if (tau == tau) {
-      power_floor = fmaxf(-tau, -87.0f);
+      cp.w = fminf(2.0f * tau, GS_FORM_MAX);
       const float det = co.x * co.z - co.y * co.y;
       // (the hardware reciprocal: 1/A and 1/C only place the point of a block edge where q is evaluated, and q
       // there exceeds the edge's minimum by the square of the placement error)
       const float ia = __builtin_amdgcn_rcpf(co.x), ic = __builtin_amdgcn_rcpf(co.z);
-      if (det > 0.0f && co.x > 0.0f && co.z > 0.0f && ia < inf && ic < inf) cp = make_float4(ia, ic, 2.0f * tau, 0.f);
+      if (det > 0.0f && co.x > 0.0f && co.z > 0.0f && ia < inf && ic < inf) cp = make_float4(ia, ic, 2.0f * tau, cp.w);
     }
   }
   return cp;
 }
 
-// What the block tests of a tile's kernels need of a Gaussian centred at xy: (1/A, 1/C, limit on q, 0), and, in
-// mark_limit, the limit on q for a single pixel of the tile (the forward blend marks the pixels an entry can reach
-// with it).  Both limits are q_max plus a margin for rounding: the block test, the pixel mark and the blend itself
+// What the block tests of a tile's kernels need of a Gaussian centred at xy: (1/A, 1/C, limit on q for a block, limit on
+// q for a single pixel of the tile; the forward blend marks the pixels an entry can reach with the latter).  Both limits
+// are those of cull_params plus a margin for rounding: the block test, the pixel mark and the blend itself
 // evaluate q by different operation sequences at different points, each within a few units in the last place of
 // the LARGEST term, which for a long thin Gaussian far from its centre is much larger than q itself.  Every such
 // term is at most S = |A| X^2 + 2 |B| X Y + |C| Y^2 with X, Y the largest offsets of a pixel of the tile from the
 // centre; the margin is 2e-6 S (about 32 units in the last place of S), on top of the 0.02 from tau + 0.01.  The
 // block limit is negative when the opacity alone rules every pixel out and +infinity when the conic cannot be
 // trusted.  The same numbers in the forward and the backward kernel, so both build the same lists.
-__device__ __forceinline__ float4 block_test_params(float4 co, float2 xy, float tile_x0, float tile_y0,
-                                                    float& power_floor, float& mark_limit) {
-  const float4 cp = cull_params(co, power_floor);
+__device__ __forceinline__ float4 block_test_params(float4 co, float2 xy, float tile_x0, float tile_y0) {
+  const float4 cp = cull_params(co);
   const float far_x = fmaxf(fabsf(xy.x - tile_x0), fabsf(xy.x - (tile_x0 + (float)(GS_TILE_X - 1))));
   const float far_y = fmaxf(fabsf(xy.y - tile_y0), fabsf(xy.y - (tile_y0 + (float)(GS_TILE_Y - 1))));
   const float spread = fabsf(co.x) * far_x * far_x + 2.0f * fabsf(co.y) * far_x * far_y + fabsf(co.z) * far_y * far_y;
-  // (q_max = 2 (tau + 0.01) is -2 power_floor wherever the conic is trusted)
-  mark_limit = __builtin_fmaf(2e-6f, spread, -2.0f * power_floor);
+  const float pixel_limit = __builtin_fmaf(2e-6f, spread, cp.w);
   const bool never = cp.z < 0.f, untrusted = cp.z == __builtin_inff();
-  return make_float4(cp.x, cp.y, never ? -1.0f : (untrusted ? cp.z : mark_limit), 0.f);
+  return make_float4(cp.x, cp.y, never ? -1.0f : (untrusted ? cp.z : pixel_limit), pixel_limit);
 }
 
 // bits <- 4 bits + 2 [a does not exceed limit_a] + [b does not exceed limit_b], NaNs not exceeding: each answer is shifted

@@ -4,9 +4,9 @@
 //
 // One 256-thread workgroup per 16x16 tile; each 64-lane wave owns an 8x8
 // quadrant and each 16-lane row of a wave a 4x4 pixel block.  The tile's
-// depth-sorted Gaussians are staged through LDS in batches of 256 (index,
-// centre, conic+opacity, colour, the five geometry channels, the culling
-// parameters and the exponent below which alpha < 1/255 is certain).
+// depth-sorted Gaussians are staged through LDS in batches of 256 (centre,
+// conic, opacity, the limit of the marks, colour, the five geometry channels
+// and the blocks touched).
 // The thread that stages a Gaussian tests which of the tile's sixteen 4x4 blocks its alpha >= 1/255 ellipse (slightly
 // inflated) can reach; the sixteen bits are also left for the backward pass.  Per batch a wave compacts, for each of
 // its four rows, the slot numbers of those that reach the row's block into a byte list in LDS (a lane's
@@ -24,7 +24,7 @@
 // kernel that spills to scratch memory starts its waves much more slowly, so
 // index arithmetic is kept from being hoisted across the blend loop.
 // What bounds it: the vector ALU (about 0.8 busy; additions, multiplications, fused multiply-adds, moves and bitwise
-// operations of vector registers take two cycles a wave here, everything else four) and the LDS pipe (0.55).  So a blend
+// operations of vector registers take two cycles a wave here, everything else four) and the LDS pipe (0.5).  So a blend
 // works on -2 times the exponent (one constant less a pass), its tests are lane masks combined in scalar registers, and
 // what a pass counts it counts under the mask: 57 vector instructions a pass where there were 71, and a block test per
 // staged Gaussian where every wave made its own.  1 M Gaussians, 1152x864: 98 -> 94 us, 4 M from the air 279 -> 262, 20 M
@@ -32,8 +32,8 @@
 //
 // The per-pixel arithmetic keeps a fixed operation order, so contributor
 // counts and images match a CPU evaluation bit for bit; exp() is gs_expf.
-// out_observe increments are counted per lane in LDS, two 16-bit counts a
-// word, and added once per (tile, Gaussian).
+// out_observe increments are counted per lane in LDS, a word per slot, and
+// added once per (tile, Gaussian).
 #include <type_traits>
 
 #include "gs_common.h"
@@ -162,13 +162,12 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         // (the marking step evaluates the quadratic form with fused operations, the blend the exponent with one
         // rounding per operation: the mark limit's margin covers both, and the blend tests the exponent itself
         // again)
-        float pfl, mark_limit;
         uint32_t ox = tile_x * GS_TILE_X, oy = tile_y * GS_TILE_Y;
         asm volatile("" : "+s"(ox), "+s"(oy));  // (as in not_hoisted)
         const float tile_x0 = (float)ox, tile_y0 = (float)oy;
-        const float4 cp = block_test_params(co, xy, tile_x0, tile_y0, pfl, mark_limit);
+        const float4 cp = block_test_params(co, xy, tile_x0, tile_y0);
         s_geo0[ts] = make_float4(xy.x, xy.y, co.x, co.y);
-        s_geo1[ts] = make_float4(0.25f * co.z, mark_limit, co.z, -0.5f * co.w);
+        s_geo1[ts] = make_float4(0.25f * co.z, cp.w, co.z, -0.5f * co.w);
         float mag = fmaxf(fmaxf(fabsf(c0), fabsf(c1)), fabsf(c2));
         bool fin = c0 == c0 && c1 == c1 && c2 == c2;
         if (render_geo) {

@@ -84,8 +84,9 @@ inline uint32_t float_bits(float v) {
 }
 
 // exp for the alpha-blending loops (CR/forward.cu:390, CR/backward.cu:484).
-// n = rint(x*log2e); r = x - n*ln2 (two-constant split); degree-6 polynomial
-// in r; scale by 2^n through the exponent field.  Below -87 the result is 0,
+// n = rint(x*log2e); r = x - n*ln2 (ln2 split into two constants, after Cody and
+// Waite); the polynomial of expf in S. L. Moshier's Cephes library; scale by 2^n
+// through the exponent field.  Below -87 the result is 0,
 // above 88 it is +inf, so no subnormal is ever produced.
 inline float orc_expf(float x) {
   if (!(x == x)) return x;
