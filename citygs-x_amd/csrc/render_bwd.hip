@@ -40,9 +40,9 @@
 // cuda_rasterizer/backward.cu:510-563.)
 //
 // What bounds it: the vector ALU (about 0.7 busy), which the matrix instructions
-// share (a 4x4x1 one takes the time of four additions), and the latency of the
-// LDS reads at the head of a pass (list word, slot, operands, one after the
-// other), which four waves a SIMD do not hide altogether.  A pass has some 300
+// share (a 4x4x1 one takes the time of four additions), and latency that four
+// waves a SIMD do not hide (the head of a pass is a chain of LDS reads: list word
+// and slot, operands).  A pass has some 300
 // vector instructions of two or four cycles each and 16 matrix instructions, about
 // 17 passes a wave at 1 M Gaussians, 1152x864; the steps between the walks a fifth
 // of the whole.  With the staging shared by the four waves (batches of 128, 64 of
