@@ -1444,6 +1444,7 @@ int gs_selftest_reciprocal(uint32_t first, uint32_t n, uint32_t* out, gs_stream_
 }
 
 long long gs_selftest_adam_plan(int count, const long long* sizes, long long* out, long long capacity) {
+  if ((count > 0 && sizes == nullptr) || (capacity > 0 && out == nullptr)) return -1;
   return adam_plan(count, sizes, out, capacity);
 }
 

@@ -507,8 +507,8 @@ int gs_render_tiles_backward(int P, int width, int height, float tan_fovx, float
  * gs_selftest_reciprocal: the backward blend's reciprocal against the division on the n floats whose bits are first,
  * first + 1, ...; out (two words, cleared by the caller): how many differ, and the bits of the largest that does.
  * gs_selftest_adam_plan: how gs_adam_step shares tensors of these sizes out among its launches (host only, nothing is
- * launched): the number of slices; the first `capacity` of them in out, five numbers each: launch, tensor, first element,
- * elements, threads of the launch. */
+ * launched): the number of slices (-1: a null pointer); the first `capacity` of them in out, five numbers each: launch,
+ * tensor, first element, elements, threads of the launch. */
 int gs_selftest_reductions(const float* in, float* out_wave, float* out_rows, gs_stream_t stream);
 int gs_selftest_quads(const float* in, float* out, gs_stream_t stream);
 int gs_selftest_reciprocal(uint32_t first, uint32_t n, uint32_t* out, gs_stream_t stream);

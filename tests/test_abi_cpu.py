@@ -191,3 +191,6 @@ def test_adam_steps_of_any_size_fit_their_launches():
             # 128 threads per 512 elements of a slice; a launch follows when the one before it is full
             assert (mine[:, 4] == 128 * ((mine[:, 3] + 511) // 512).sum()).all()
         assert (np.diff(table[:, 0]) >= 0).all() and (np.diff(table[:, 0]) <= 1).all()
+    one = (C.c_longlong * 1)(7)
+    assert gn.lib.gs_selftest_adam_plan(1, None, one, 0) == -1 and gn.lib.gs_selftest_adam_plan(1, one, None, 1) == -1
+    assert gn.lib.gs_selftest_adam_plan(1, one, None, 0) == 1
