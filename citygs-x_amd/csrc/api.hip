@@ -174,7 +174,7 @@ BinningLayout binning_layout(int64_t R, int64_t packed_gaussians = 0) {
   L.emission_other = take(n * 4);
   L.emission = take(n * 4);
   L.sort_temp = take(sort_temp_bytes((int64_t)n));
-  L.block_hits = take(n * 2);  // what the forward blend leaves for the backward blend, per sorted instance
+  L.block_hits = take(n * 4);  // what the forward blend leaves for the backward blend, a word per sorted instance
   L.radix_scratch = take(n * 24);  // per-tile radix sort: lists beyond one block, split (16 B) and in blocks (8 B)
   // the blend kernels' operands, one 64-byte record per Gaussian, if the forward call packs them (last, so that
   // no other offset depends on whether it does)
@@ -617,7 +617,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     uint64_t *keys, *keys_other;
     void *sort_temp, *radix_scratch;
     int64_t capacity;
-    uint16_t* block_hits;
+    uint32_t* block_hits;
     float* packed;
   };
   auto carve = [&](int64_t n, Arrays& A) -> int {
@@ -632,7 +632,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     A.emission = (uint32_t*)(bbase + BL.emission);
     A.emission_other = (uint32_t*)(bbase + BL.emission_other);
     A.sort_temp = bbase + BL.sort_temp;
-    A.block_hits = (uint16_t*)(bbase + BL.block_hits);
+    A.block_hits = (uint32_t*)(bbase + BL.block_hits);
     A.radix_scratch = bbase + BL.radix_scratch;
     A.packed = (float*)(bbase + BL.packed);
     A.capacity = n > 0 ? n : 1;
@@ -648,7 +648,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
                                A.packed, packed_valid, stream);
     return check_launch("pack_operands", stream, dbg);
   };
-  auto blend = [&](const Arrays& A, bool ordered, bool ahead_of_host) -> int {
+  auto blend = [&](const Arrays& A, bool ordered, uint32_t longest_for_launch, bool ahead_of_host) -> int {
     RenderFwdArgs a;
     a.P = P; a.W = width; a.H = height;
     a.fx = focal_x; a.fy = focal_y; a.cx = cx; a.cy = cy;
@@ -664,6 +664,8 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     a.block_hits = A.block_hits;
     a.packed = use_packed ? (caller_records != nullptr ? caller_records : A.packed) : nullptr;
     a.tile_order = ordered ? tile_order : nullptr;
+    a.tile_order_word = ordered ? packed_valid + 1 : nullptr;
+    a.longest = longest_for_launch;
     {
       StageScope _t("render_fwd", stream);
       launch_render_fwd(a, stream);
@@ -684,7 +686,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
       StageScope _t("tile_sort", stream);
       if (launch_tile_sort(T, longest_for_launch, radix_tiles, sort_limit, (uint32_t)limits.block, ranges,
                            bucket_table, A.keys_other, A.radix_scratch, A.capacity, A.keys, A.emission,
-                           A.point_list, tile_order, packed_valid + 1, ahead_of_host, stream))
+                           A.point_list, tile_order, packed_valid + 1, n_consider, n_contrib, ahead_of_host, stream))
         return 1;
     }
     return check_launch("tile_sort", stream, dbg);
@@ -698,7 +700,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     if (timer.begin(elapsed_ms != nullptr, stream)) return 1;
     if (pack_records(A)) return 1;
     if (lists_by_tile(A, cap_longest, 0xFFFFFFFFu, true)) return 1;
-    if (blend(A, cap_longest > 0, true)) return 1;
+    if (blend(A, cap_longest > 0, cap_longest, true)) return 1;
   }
 
   // The host needs the instance count: it sizes the binning buffer (unless that was done ahead), and the caller
@@ -793,7 +795,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     if (check_launch("identify_tile_ranges", stream, dbg)) return 1;
   }
 
-  if (blend(A, bucketed && longest > 0, false)) return 1;
+  if (blend(A, bucketed && longest > 0, longest, false)) return 1;
   if (timer.end(stream, elapsed_ms)) return 1;
   // (debug mode and the timer have waited for the stream: a sort that gave up in this call is known by now)
   if ((dbg || elapsed_ms != nullptr) && pending_fault("gs_render_forward")) return 1;
@@ -830,7 +832,7 @@ int gs_render_backward(int P, int R, const float* background, int width, int hei
   const char* ibase = align_ptr(img_buffer, 256);
   RenderBwdArgs a;
   a.emission_sorted = (const uint32_t*)(bbase + BL.emission);
-  a.block_hits = (const uint16_t*)(bbase + BL.block_hits);
+  a.block_hits = (const uint32_t*)(bbase + BL.block_hits);
   a.point_offsets = (const uint32_t*)(gbase + GL.point_offsets);
   // (records of the arrays the forward call was given: the caller's own, or what the forward call packed)
   GS_REQUIRE(((uintptr_t)blend_records & 15u) == 0u, "gs_render_backward: blend_records must be 16-byte aligned");

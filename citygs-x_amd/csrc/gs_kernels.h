@@ -125,7 +125,7 @@ int launch_bucket_scatter(int P, int W, int H, const float* means2D, const float
 int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t small_limit, uint32_t block_limit,
                      const uint32_t* ranges, const void* table, const void* records, void* scratch, int64_t capacity,
                      uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
-                     uint32_t* tile_order_valid, bool ahead_of_host, hipStream_t stream);
+                     uint32_t* tile_order_word, int* n_consider, int* n_contrib, bool ahead_of_host, hipStream_t stream);
 int tile_radix_mid_records();    // records one workgroup of the radix sort's smaller kernel holds (4096)
 int tile_radix_block_records();  // ... and of its larger kernel (16384): longer lists are sorted in blocks
 int launch_tile_radix_sort(int T, bool mid, bool lng, const uint32_t* ranges, const uint32_t* tile_lists,
@@ -231,6 +231,12 @@ int launch_sort_pairs_u32(int64_t n, uint32_t* keys_a, uint32_t* keys_b, uint32_
 int64_t sort_clear_words(int64_t n, int end_bit);
 
 // ---- tile render ----
+// A list from which on a tile is blended by four workgroups (render_fwd.hip); a power of two or one and a half of one, since
+// the tiles are ordered by classes of these lengths.  A whole training view, us, with 2048, 3072, 4096, 6144 and without: 4 M
+// Gaussians from the air 1492, 1469, 1481, 1518, 1560; at street level, 10 M, 2848, 2842, 2820, 2813, 2937; rendering 20 M
+// from 600 m 2264, 2260, 2258, 2282, 2545.  Shorter lists pay for the instructions without ending a view.
+constexpr uint32_t GS_LONG_TILE = 3072;
+
 struct RenderFwdArgs {
   int P, W, H;
   float fx, fy, cx, cy;
@@ -251,14 +257,18 @@ struct RenderFwdArgs {
   // optional device word: the kernel was launched before the host knew whether the per-tile lists would be
   // built by the kernels queued ahead of it; it does nothing if the word is 0
   const uint32_t* fits_word = nullptr;
-  // optional (R): per sorted instance, which of the tile's sixteen 4x4 pixel blocks the Gaussian can touch (bit
-  // 4 * wave + row), as found by the kernel's own list building; the backward blend reads it instead of testing
-  // again
-  uint16_t* block_hits = nullptr;
+  // optional (R): per sorted instance, which of the tile's sixteen 4x4 pixel blocks the Gaussian can touch (hits_to_bytes
+  // of bit 4 * quadrant + block), as found by the kernel's own list building; the backward blend reads it instead of
+  // testing again
+  uint32_t* block_hits = nullptr;
   // optional (P,4) 16-byte words: pack_blend_operands' records; the kernel then fetches a Gaussian's operands as
   // one 64-byte line instead of gathering them from means2D, conic_opacity, rgb, all_map (and depths)
   const float* packed = nullptr;
   const uint32_t* tile_order = nullptr;  // optional (T): the order in which the tiles are taken (launch_tile_sort)
+  // the word launch_tile_sort leaves beside it (1 + the number of tiles with more than GS_LONG_TILE entries), and a bound
+  // on the longest list
+  const uint32_t* tile_order_word = nullptr;
+  uint32_t longest = 0;
 };
 int launch_render_fwd(const RenderFwdArgs& a, hipStream_t stream);
 
@@ -278,7 +288,7 @@ struct RenderBwdArgs {
   const uint32_t* emission_sorted;
   const uint32_t* point_offsets;
   float* instance_grads;  // (R,16) scratch, fully written by the blend kernel
-  const uint16_t* block_hits = nullptr;  // optional (R): left by the forward blend (RenderFwdArgs::block_hits)
+  const uint32_t* block_hits = nullptr;  // optional (R): left by the forward blend (RenderFwdArgs::block_hits)
   const float* packed = nullptr;         // optional (P,4) 16-byte words: see RenderFwdArgs::packed
   // optional device word beside `packed`: non-zero if the forward call did pack the records (it decides per view)
   const uint32_t* packed_valid = nullptr;

@@ -8,7 +8,7 @@
 // block's columns.
 //   * The tile's list is scanned back to front, 256 entries at a time, and the
 //     entries that touch a block in front of its deepest contributor (the
-//     forward kernel's own answer, 16 bits per instance, when the caller hands
+//     forward kernel's own answer, a word per instance, when the caller hands
 //     them on; otherwise the inflated alpha >= 1/255 ellipse is tested again)
 //     are compacted into a ring; the others' records are zero.
 //   * Out of a window of up to 256 waiting Gaussians every wave picks those
@@ -109,7 +109,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                   const uint8_t* __restrict__ compute_locally, const float* __restrict__ dL_dpix,
                   const float* __restrict__ dL_dout_all_map, const float* __restrict__ dL_dout_plane_depth,
                   const uint32_t* __restrict__ emission_sorted, float4* __restrict__ instance_grads,
-                  const uint16_t* __restrict__ block_hits, const float4* __restrict__ packed_records,
+                  const uint32_t* __restrict__ block_hits, const float4* __restrict__ packed_records,
                   const uint32_t* __restrict__ packed_valid, const uint32_t* __restrict__ tile_order,
                   const uint32_t* __restrict__ tile_order_valid, uint32_t tiles_x) {
   // (whether the forward call packed the records is its decision per view: a word beside them says)
@@ -269,7 +269,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   // picks, out of a window of positions, the Gaussians that touch one of its rows in front of the row's deepest contributor,
   // a quarter of the list where Gaussians are small, stages those and walks them; the window ends where a wave has no slot
   // left.  A position that no wave has taken has a record of zeros.
-  auto hits_at = [&](int pos) { return pos >= 0 ? (uint32_t)block_hits[range.x + (uint32_t)pos] : 0u; };
+  auto hits_at = [&](int pos) { return pos >= 0 ? hits_from_bytes(block_hits[range.x + (uint32_t)pos]) : 0u; };
   auto hits_by_test = [&](int pos) {
     if (pos < 0) return 0u;
     const uint32_t g = point_list[range.x + (uint32_t)pos];

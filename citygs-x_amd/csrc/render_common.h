@@ -68,6 +68,46 @@ __device__ __forceinline__ void shift_in_two(uint32_t& bits, float a, float limi
       : "vcc");
 }
 
+// What the block tests of two neighbouring columns of 4x4 blocks have in common (x0: the left one's first pixel).
+struct BlockColumns {
+  float lox[2], t1[2], a1[2], b1[2];
+};
+
+__device__ __forceinline__ BlockColumns block_columns(float2 mu, float4 co, float inv_c, float x0) {
+  const float two_b = 2.0f * co.y;
+  BlockColumns b;
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    b.lox[c] = (x0 + (float)(4 * c)) - mu.x;
+    const float dxc = __builtin_amdgcn_fmed3f(0.f, b.lox[c], b.lox[c] + 3.0f);  // offset of the block's nearest column
+    b.t1[c] = -co.y * dxc * inv_c;                                              // where q is smallest along that column
+    b.a1[c] = co.x * dxc * dxc;
+    b.b1[c] = two_b * dxc;
+  }
+  return b;
+}
+
+// hits <- 4 hits + 2 [right block] + [left block] of the two columns' row of blocks whose first pixel is at y0.
+__device__ __forceinline__ void test_block_pair(uint32_t& hits, const BlockColumns& b, float2 mu, float4 co, float inv_a,
+                                                float limit, float y0) {
+  const float loy = y0 - mu.y;
+  const float hiy = loy + 3.0f;
+  const float dyc = __builtin_amdgcn_fmed3f(0.f, loy, hiy);  // offset of the block's nearest row
+  const float t2 = -co.y * dyc * inv_a;                      // where q is smallest along that row
+  const float a2 = co.z * dyc * dyc;
+  const float b2 = 2.0f * co.y * dyc;
+  float nearest[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    const float dy1 = __builtin_amdgcn_fmed3f(b.t1[c], loy, hiy);  // best point of the column x = dxc
+    const float q1 = __builtin_fmaf(__builtin_fmaf(co.z, dy1, b.b1[c]), dy1, b.a1[c]);
+    const float dx2 = __builtin_amdgcn_fmed3f(t2, b.lox[c], b.lox[c] + 3.0f);  // best point of the row y = dyc
+    const float q2 = __builtin_fmaf(__builtin_fmaf(co.x, dx2, b2), dx2, a2);
+    nearest[c] = fminf(q1, q2);
+  }
+  shift_in_two(hits, nearest[1], limit, nearest[0], limit);
+}
+
 // The sixteen 4x4 pixel blocks of the tile at (tile_x0, tile_y0): bit 4 k + r of the result is block r of quadrant k
 // (quadrant k at offset 8 (k & 1), 8 (k >> 1), block r in it at 4 (r & 1), 4 (r >> 1)): can any point of the block have
 // q <= limit?  q is convex, so over a block it is smallest either at the centre (inside the block: 0) or on one of the two
@@ -77,41 +117,36 @@ __device__ __forceinline__ void shift_in_two(uint32_t& bits, float a, float limi
 // block_test_params.  NaNs count as hits.
 __device__ __forceinline__ uint32_t ellipse_hits_tile(float2 mu, float4 co, float inv_a, float inv_c, float limit,
                                                       float tile_x0, float tile_y0) {
-  const float two_b = 2.0f * co.y;
   uint32_t hits = 0u;  // (columns 2 h and 2 h + 1 of row d: bits 8 h + 2 d and the next)
 #pragma unroll 1
   for (int h = 1; h >= 0; h--) {  // (loops: unrolled they take registers that the blend kernels do not have)
-    float lox[2], t1[2], a1[2], b1[2];
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      lox[c] = (tile_x0 + (float)(8 * h + 4 * c)) - mu.x;
-      const float dxc = __builtin_amdgcn_fmed3f(0.f, lox[c], lox[c] + 3.0f);  // offset of the block's nearest column
-      t1[c] = -co.y * dxc * inv_c;                                            // where q is smallest along that column
-      a1[c] = co.x * dxc * dxc;
-      b1[c] = two_b * dxc;
-    }
+    const BlockColumns b = block_columns(mu, co, inv_c, tile_x0 + (float)(8 * h));
 #pragma unroll 1
-    for (int d = 3; d >= 0; d--) {
-      const float loy = (tile_y0 + (float)(4 * d)) - mu.y;
-      const float hiy = loy + 3.0f;
-      const float dyc = __builtin_amdgcn_fmed3f(0.f, loy, hiy);  // offset of the block's nearest row
-      const float t2 = -co.y * dyc * inv_a;                      // where q is smallest along that row
-      const float a2 = co.z * dyc * dyc;
-      const float b2 = two_b * dyc;
-      float nearest[2];
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const float dy1 = __builtin_amdgcn_fmed3f(t1[c], loy, hiy);  // best point of the column x = dxc
-        const float q1 = __builtin_fmaf(__builtin_fmaf(co.z, dy1, b1[c]), dy1, a1[c]);
-        const float dx2 = __builtin_amdgcn_fmed3f(t2, lox[c], lox[c] + 3.0f);  // best point of the row y = dyc
-        const float q2 = __builtin_fmaf(__builtin_fmaf(co.x, dx2, b2), dx2, a2);
-        nearest[c] = fminf(q1, q2);
-      }
-      shift_in_two(hits, nearest[1], limit, nearest[0], limit);
-    }
+    for (int d = 3; d >= 0; d--) test_block_pair(hits, b, mu, co, inv_a, limit, tile_y0 + (float)(4 * d));
   }
   // row d of columns 2 h, 2 h + 1 are blocks 2 (d & 1), 2 (d & 1) + 1 of quadrant 2 (d >> 1) + h
   return (hits & 0xF00Fu) | ((hits & 0x00F0u) << 4) | ((hits & 0x0F00u) >> 4);
+}
+
+// The same tests for the four blocks of the quadrant at (x0, y0): bits 4 k .. 4 k + 3 of ellipse_hits_tile (the offsets of
+// pixels are whole numbers, so they are the same whichever corner they are counted from).
+__device__ __forceinline__ uint32_t ellipse_hits_quadrant(float2 mu, float4 co, float inv_a, float inv_c, float limit,
+                                                          float x0, float y0) {
+  uint32_t hits = 0u;
+  const BlockColumns b = block_columns(mu, co, inv_c, x0);
+#pragma unroll
+  for (int d = 1; d >= 0; d--) test_block_pair(hits, b, mu, co, inv_a, limit, y0 + (float)(4 * d));
+  return hits;
+}
+
+// How the forward blend hands a Gaussian's sixteen hits to the backward blend: a word with byte k for quadrant k, whose
+// lower four bits are the quadrant's blocks (bytes, because the quadrants of a long tile are blended by workgroups of
+// their own).
+__device__ __forceinline__ uint32_t hits_to_bytes(uint32_t hits) {
+  return (hits & 0xFu) | ((hits & 0xF0u) << 4) | ((hits & 0xF00u) << 8) | ((hits & 0xF000u) << 12);
+}
+__device__ __forceinline__ uint32_t hits_from_bytes(uint32_t bytes) {
+  return (bytes & 0xFu) | ((bytes >> 4) & 0xF0u) | ((bytes >> 8) & 0xF00u) | ((bytes >> 12) & 0xF000u);
 }
 
 // ---- 4x4-pixel rows -------------------------------------------------------

@@ -30,6 +30,13 @@
 // staged Gaussian where every wave made its own.  1 M Gaussians, 1152x864: 98 -> 94 us, 4 M from the air 279 -> 262, 20 M
 // 660 -> 643, 300 k without geometry channels 59.5 -> 57.
 //
+// A tile's workgroup takes some 31 ns an entry whatever else the chip does: the chain of its waves' own instructions.  A
+// view whose lists differ much in length ended on a few such chains (4 M Gaussians from the air, lists up to 9600: 293 us,
+// in the last 150 of which less than a quarter of the chip had work; wave priorities change nothing).  Long tiles therefore
+// go to four workgroups, one per quadrant, whose waves have 16 pixels instead of 64 and four lanes for each
+// (blend_quadrant): 4.4 us per 256 entries instead of 8, for about 1.45 times the instructions of a tile.
+// 4 M, 1152x864: 263 -> 201 us; 20 M from 600 m, lists up to 69 000, of which 0.4 is walked: 648 -> 415.
+//
 // The per-pixel arithmetic keeps a fixed operation order, so contributor
 // counts and images match a CPU evaluation bit for bit; exp() is gs_expf.
 // out_observe increments are counted per lane in LDS, a word per slot, and
@@ -45,6 +52,9 @@ namespace gs {
 namespace {
 
 constexpr int BATCH = GS_TILE_PIX;
+// Tiles that four workgroups each may take, at most: the launch has three workgroups more for each of them, which do
+// nothing where a view has fewer.
+constexpr uint32_t LONG_TILES = 1024;
 constexpr int CHUNK = 32;  // entries of a list marked, then blended, at a time: one bit each in a register
 
 // The value itself, but opaque to the optimizer from here on: what is computed from it stays behind this point
@@ -55,10 +65,326 @@ __device__ __forceinline__ int not_hoisted(int x) {
   return x;
 }
 
+// The value that lane E of a quad (four neighbouring lanes) holds, in all four lanes.
+template <int E>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), E * 0x55, 0xF, 0xF, true));
+}
+template <int E>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, E * 0x55, 0xF, 0xF, true);
+}
+// v of the lane whose number differs in bit 0 (in bit 1).
+__device__ __forceinline__ uint32_t quad_xor1(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);
+}
+__device__ __forceinline__ uint32_t quad_xor2(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);
+}
+
+// What a workgroup has in LDS (see the kernel).
+template <bool RENDER_GEO>
+struct BlendLds {
+  float4 *geo0, *geo1, *col0, *col1;
+  uint32_t *obs, *idx;
+  uint16_t* hits;
+  int *done, *bad;
+};
+
+// One quadrant of a long tile by a workgroup of its own: a wave has one 4x4 block, a quad of its lanes one pixel.  The
+// four lanes of a pixel mark a quarter of a chunk each and blend the pixel's next four marked entries together: lane k has
+// the exponent and alpha of entry k, all four the transmittance in front of every entry (a chain of four products), and
+// lane k the sums of channels 2 k and 2 k + 1 (channel k where only the colour is rendered), in the order of the entries.
+// Every number is formed by the operations the other way has, in its order: the same bits.
+template <bool RENDER_GEO, bool PACKED>
+__device__ __forceinline__ void blend_quadrant(
+    const BlendLds<RENDER_GEO> lds, uint32_t tile, uint32_t quadrant, uint32_t tile_x, uint32_t tile_y, uint2 range,
+    const uint32_t* __restrict__ point_list, int W, int H, float fx, float fy, float cx, float cy,
+    const float2* __restrict__ means2D, const float* __restrict__ rgb, const float* __restrict__ all_map,
+    const float4* __restrict__ conic_opacity, bool computed_here, const float* __restrict__ bg,
+    float* __restrict__ final_T, uint32_t* __restrict__ n_contrib_px, uint32_t* __restrict__ n_contrib2loss_px,
+    float* __restrict__ out_color, int* __restrict__ out_observe, float* __restrict__ out_all_map,
+    float* __restrict__ out_plane_depth, int* __restrict__ n_render, int* __restrict__ n_consider,
+    int* __restrict__ n_contrib_tile, uint32_t* __restrict__ block_hits, const float4* __restrict__ packed) {
+  const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
+  const uint32_t k = (uint32_t)lane & 3u;
+  const uint32_t x0 = tile_x * GS_TILE_X + 8u * (quadrant & 1u), y0 = tile_y * GS_TILE_Y + 8u * (quadrant >> 1);
+  const uint32_t px = x0 + 4u * (uint32_t)(wave & 1) + ((uint32_t)lane >> 2 & 3u);
+  const uint32_t py = y0 + 4u * (uint32_t)(wave >> 1) + ((uint32_t)lane >> 4);
+  const bool inside = px < (uint32_t)W && py < (uint32_t)H;
+  const int total = (int)(range.y - range.x);
+  if (quadrant == 0u && tid == 0) n_render[tile] = total;
+  if (!computed_here) {  // (as in the other way)
+    const size_t HW = (size_t)H * W, pid = (size_t)W * py + px;
+    if (inside && k == 0u) {
+#pragma unroll
+      for (int ch = 0; ch < GS_N_RGB; ch++) out_color[ch * HW + pid] = 0.f;
+      if (RENDER_GEO) {
+#pragma unroll
+        for (int ch = 0; ch < GS_N_MAP; ch++) out_all_map[ch * HW + pid] = 0.f;
+        out_plane_depth[pid] = 0.f;
+      }
+    }
+    return;
+  }
+  const float pfx = (float)px, pfy = (float)py;
+  uint64_t alive = gs_ballot(inside);  // pixels that still blend, four bits each
+  constexpr int SUMS = RENDER_GEO ? 2 : 1;
+  float T = 1.0f, C[SUMS];
+  uint32_t last = 0, n2l = 0;  // of the entries this lane has blended
+#pragma unroll
+  for (int ch = 0; ch < SUMS; ch++) C[ch] = 0.f;
+  const char* const my_channels =
+      RENDER_GEO ? reinterpret_cast<const char*>(k < 2u ? lds.col0 : lds.col1) + 8u * (k & 1u)
+                 : reinterpret_cast<const char*>(lds.col0) + 4u * k;
+  uint8_t* const my_list = reinterpret_cast<uint8_t*>(lds.idx) + wave * BATCH;
+
+  // The operands of a thread's slot are fetched a batch ahead, their Gaussian two.
+  uint32_t g = tid < total ? point_list[range.x + (uint32_t)tid] : 0u;
+  uint32_t g_next = tid + BATCH < total ? point_list[range.x + (uint32_t)(tid + BATCH)] : 0u;
+  float4 r0, r1, r2;
+  auto fetch = [&](uint32_t gaussian) {
+    const float4* rec = packed + 4 * (size_t)gaussian;
+    r0 = rec[0], r1 = rec[1], r2 = rec[2];
+  };
+  r0 = r1 = r2 = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (PACKED && tid < total) fetch(g);
+  for (int base = 0;; base += BATCH) {
+    const int count = total - base < BATCH ? total - base : BATCH;
+    bool finite = true;
+    uint32_t hits = 0u;
+    const int ts = not_hoisted(tid);
+    if (ts < count) {
+      auto stage = [&](const float2 xy, const float4 co, const float c0, const float c1, const float c2,
+                       const float (&m)[GS_N_MAP]) {
+        const float4 cp = block_test_params(co, xy, (float)(tile_x * GS_TILE_X), (float)(tile_y * GS_TILE_Y));
+        lds.geo0[ts] = make_float4(xy.x, xy.y, co.x, co.y);
+        lds.geo1[ts] = make_float4(0.25f * co.z, cp.w, co.z, -0.5f * co.w);
+        float mag = fmaxf(fmaxf(fabsf(c0), fabsf(c1)), fabsf(c2));
+        bool fin = c0 == c0 && c1 == c1 && c2 == c2;
+        if (RENDER_GEO) {
+#pragma unroll
+          for (int ch = 0; ch < GS_N_MAP; ch++) {
+            mag = fmaxf(mag, fabsf(m[ch]));
+            fin = fin && m[ch] == m[ch];
+          }
+        }
+        lds.col0[ts] = make_float4(c0, c1, c2, m[0]);
+        if (RENDER_GEO) lds.col1[ts] = make_float4(m[1], m[2], m[3], m[4]);
+        hits = ellipse_hits_quadrant(xy, co, cp.x, cp.y, cp.z, (float)x0, (float)y0);
+        return fin && mag < __builtin_inff();
+      };
+      if constexpr (PACKED) {
+        // (the last two words are on the line that the others came with)
+        const float2 r3 = RENDER_GEO ? *reinterpret_cast<const float2*>(packed + 4 * (size_t)g + 3) : make_float2(0.f, 0.f);
+        const float m[GS_N_MAP] = {r2.y, r2.z, r2.w, r3.x, r3.y};
+        finite = stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
+      } else {
+        const float2 xy = means2D[g];
+        const float4 co = conic_opacity[g];
+        const float c0 = rgb[3 * (size_t)g], c1 = rgb[3 * (size_t)g + 1], c2 = rgb[3 * (size_t)g + 2];
+        float m[GS_N_MAP] = {0.f, 0.f, 0.f, 0.f, 0.f};
+        if (RENDER_GEO) {
+#pragma unroll
+          for (int ch = 0; ch < GS_N_MAP; ch++) m[ch] = all_map[5 * (size_t)g + ch];
+        }
+        finite = stage(xy, co, c0, c1, c2, m);
+      }
+      if (block_hits != nullptr)
+        reinterpret_cast<uint8_t*>(block_hits + range.x + (uint32_t)(base + ts))[quadrant] = (uint8_t)hits;
+    }
+    {
+      const uint64_t bad_m = gs_ballot(!finite);
+      if (lane == 0) lds.bad[wave] = bad_m != 0ull;
+    }
+    lds.obs[ts] = 0u;
+    lds.hits[ts] = (uint16_t)hits;
+    lds.idx[ts] = 0u;  // (a word of the four lists per thread; bytes behind a list's end are slot 0)
+    __syncthreads();
+    g = g_next;
+    if (PACKED && base + BATCH + tid < total) fetch(g);
+    {
+      const int tn = not_hoisted(tid) + base + 2 * BATCH;
+      g_next = tn < total ? point_list[range.x + (uint32_t)tn] : 0u;
+    }
+    const bool select_blend = (lds.bad[0] | lds.bad[1] | lds.bad[2] | lds.bad[3]) != 0;
+
+    if (alive != 0ull) {
+      uint32_t len = 0u;
+#pragma unroll
+      for (int q = 0; q < BATCH / GS_WAVE; q++) {
+        const int jj = q * GS_WAVE + (not_hoisted(tid) & (GS_WAVE - 1));
+        const uint64_t b = gs_ballot(((uint32_t)lds.hits[jj] >> wave & 1u) != 0u);
+        const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, len));
+        if (__builtin_amdgcn_inverse_ballot_w64(b)) my_list[at] = (uint8_t)jj;
+        len += (uint32_t)__popcll(b);
+      }
+      len = (uint32_t)__builtin_amdgcn_readfirstlane((int)len);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      auto walk = [&](auto select_tag) {
+        constexpr bool SELECT = decltype(select_tag)::value;
+        const float pfy_m2 = -2.0f * pfy;
+        for (uint32_t c0 = 0; c0 < len && alive != 0ull; c0 += CHUNK) {
+          // lane k of a pixel marks entries 8 k .. 8 k + 7 of the chunk, the last one first
+          uint32_t marks = 0u;
+          const uint2 words = *reinterpret_cast<const uint2*>(my_list + c0 + 8u * k);
+#pragma unroll
+          for (int u = 7; u >= 0; u -= 2) {
+            float form[2], limit[2];
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+              const int e = u - v;
+              const int j = (int)__builtin_amdgcn_ubfe(e >= 4 ? words.y : words.x, 8u * (e & 3), 8u);
+              const float4 g0 = lds.geo0[j];
+              const float2 g1 = *reinterpret_cast<const float2*>(&lds.geo1[j]);  // C / 4 and the mark limit
+              const float dx = g0.x - pfx, dy2 = __builtin_fmaf(g0.y, 2.0f, pfy_m2);
+              form[v] = __builtin_fmaf(g1.x * dy2, dy2, __builtin_fmaf(g0.z, dx, g0.w * dy2) * dx);
+              limit[v] = g1.y;
+            }
+            shift_in_two(marks, form[0], limit[0], form[1], limit[1]);
+          }
+          marks <<= 8u * k;
+          marks |= quad_xor1(marks);
+          marks |= quad_xor2(marks);
+          const uint32_t mine = len - c0;  // entries of the chunk that are in the list
+          marks = mine >= (uint32_t)CHUNK ? marks : (marks & ((1u << mine) - 1u));
+          marks = __builtin_amdgcn_inverse_ballot_w64(alive) ? marks : 0u;
+          // the pixel's next four entries: lane k's is the k-th mark that is left
+          auto take_four = [&](uint32_t& left) {
+            const uint32_t m1 = left & (left - 1u), m2 = m1 & (m1 - 1u), m3 = m2 & (m2 - 1u);
+            const uint32_t own = k == 0u ? left : (k == 1u ? m1 : (k == 2u ? m2 : m3));
+            left = m3 & (m3 - 1u);
+            return own;
+          };
+          uint32_t own_next = take_four(marks);
+          uint32_t slot_next = my_list[c0 + (uint32_t)__builtin_ctz(own_next | 0x80000000u)];
+          uint64_t marked = gs_ballot(own_next != 0u);
+          while (marked != 0ull) {
+            const uint32_t j = slot_next, at = j * 16u;
+            const uint64_t has = marked;
+            own_next = take_four(marks);
+            slot_next = my_list[c0 + (uint32_t)__builtin_ctz(own_next | 0x80000000u)];
+            const float4 g0 = lds.geo0[j];
+            const float2 g1 = *(reinterpret_cast<const float2*>(&lds.geo1[j]) + 1);  // C and -opacity / 2
+            float c[4][SUMS];
+            auto channels = [&](auto e_tag) {
+              constexpr int e = decltype(e_tag)::value;
+              const float* p = reinterpret_cast<const float*>(my_channels + quad_lane<e>(at));
+              if constexpr (RENDER_GEO) {
+                const float2 two = *reinterpret_cast<const float2*>(p);
+                c[e][0] = two.x, c[e][SUMS - 1] = two.y;
+              } else {
+                c[e][0] = *p;
+              }
+            };
+            channels(std::integral_constant<int, 0>{});
+            channels(std::integral_constant<int, 1>{});
+            channels(std::integral_constant<int, 2>{});
+            channels(std::integral_constant<int, 3>{});
+            const float form = gauss_form(g0.z, g0.w, g1.x, g0.x - pfx, g0.y - pfy);
+            float alpha = fminf(0.99f, g1.y * gs_neg2_exp_of_form(form));
+            uint64_t counts = has & gs_ballot(!(form < 0.0f)) & gs_ballot(!(form > GS_FORM_MAX)) &
+                              gs_ballot(!(alpha < 1.0f / 255.0f));
+            // (an entry that does not count is blended with alpha 0, which changes nothing)
+            alpha = __builtin_amdgcn_inverse_ballot_w64(counts) ? alpha : 0.f;
+            const float oma = 1 - alpha;
+            const float T1 = T * quad_lane<0>(oma), T2 = T1 * quad_lane<1>(oma), T3 = T2 * quad_lane<2>(oma);
+            float T4 = T3 * quad_lane<3>(oma);
+            const float before = k == 0u ? T : (k == 1u ? T1 : (k == 2u ? T2 : T3));
+            const uint64_t stops = gs_ballot(T4 < 0.0001f);  // (a pixel that has stopped before keeps a T above)
+            if (stops != 0ull) {
+              // the first entry that takes a pixel's transmittance below the limit is not blended, nor what is behind it
+              const bool over = before * oma < 0.0001f;
+              counts &= ~gs_ballot(over);
+              alpha = over ? 0.f : alpha;
+              T4 = !(T4 < 0.0001f) ? T4 : !(T3 < 0.0001f) ? T3 : !(T2 < 0.0001f) ? T2 : !(T1 < 0.0001f) ? T1 : T;
+              alive &= ~stops;
+              marks = __builtin_amdgcn_inverse_ballot_w64(stops) ? 0u : marks;
+              own_next = __builtin_amdgcn_inverse_ballot_w64(stops) ? 0u : own_next;
+            }
+            const float w[4] = {quad_lane<0>(alpha) * T, quad_lane<1>(alpha) * T1, quad_lane<2>(alpha) * T2,
+                                quad_lane<3>(alpha) * T3};
+            T = T4;
+            if (__builtin_amdgcn_inverse_ballot_w64(counts)) {
+              if (before > 0.5f) atomicAdd(&lds.obs[j], 1u);
+              last = (uint32_t)(base + 1) + j;
+              n2l++;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+#pragma unroll
+              for (int ch = 0; ch < SUMS; ch++) {
+                const float sum = __builtin_fmaf(c[e][ch], w[e], C[ch]);
+                C[ch] = (!SELECT || w[e] != 0.f) ? sum : C[ch];  // (a weight that counts is at least 1e-4 / 255)
+              }
+            }
+            marked = gs_ballot(own_next != 0u);
+          }
+        }
+      };
+      if (select_blend) walk(std::true_type{});
+      else walk(std::false_type{});
+    }
+    if (lane == 0) lds.done[wave] = alive == 0ull;
+    __syncthreads();
+    const int tf = not_hoisted(tid);
+    if (tf < count) {
+      const uint32_t seen = lds.obs[tf];
+      if (seen != 0u) atomicAdd(&out_observe[point_list[range.x + (uint32_t)(base + tf)]], (int)seen);
+    }
+    if (base + BATCH >= total || (lds.done[0] && lds.done[1] && lds.done[2] && lds.done[3])) break;
+  }
+
+  const size_t HW = (size_t)H * W, pid = (size_t)W * (uint32_t)pfy + (uint32_t)pfx;
+  // what the four lanes of a pixel have counted
+  last = max(last, quad_xor1(last));
+  last = max(last, quad_xor2(last));
+  n2l += quad_xor1(n2l);
+  n2l += quad_xor2(n2l);
+  if (inside && k == 0u) {
+    final_T[pid] = T;
+    n_contrib_px[pid] = last;
+    n_contrib2loss_px[pid] = n2l;
+  }
+  if constexpr (RENDER_GEO) {
+    // (lanes 0 .. 3: red and green; blue and channel 0; channels 1 and 2; channels 3 and 4)
+    const float m0 = quad_lane<1>(C[1]), m1 = quad_lane<2>(C[0]), m2 = quad_lane<2>(C[SUMS - 1]);
+    const float m4 = quad_lane<3>(C[SUMS - 1]);
+    if (inside) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const uint32_t ch = 2u * k + (uint32_t)h;
+        if (ch < GS_N_RGB) out_color[ch * HW + pid] = C[h] + T * bg[ch];
+        else out_all_map[(ch - GS_N_RGB) * HW + pid] = C[h];
+      }
+      if (k == 3u) {
+        const float rayx = (pfx - cx) / fx, rayy = (pfy - cy) / fy;
+        const float den_f = (m0 * rayx + m1 * rayy) + m2;
+        out_plane_depth[pid] = (float)((double)m4 / -((double)den_f + 1.0e-8));
+      }
+    }
+  } else {
+    if (inside && k < GS_N_RGB) out_color[k * HW + pid] = C[0] + T * bg[k];
+  }
+  // per-tile integer sums of the two per-pixel counters; the tile's four workgroups add up
+  int a = inside && k == 0u ? (int)last : 0, b = inside && k == 0u ? (int)n2l : 0;
+#pragma unroll
+  for (int d = GS_WAVE / 2; d >= 1; d >>= 1) {
+    a += __shfl_xor(a, d, GS_WAVE);
+    b += __shfl_xor(b, d, GS_WAVE);
+  }
+  if (lane == 0) {
+    atomicAdd(&n_consider[tile], a);
+    atomicAdd(&n_contrib_tile[tile], b);
+  }
+}
+
 // MAX_DEPTH adds one output with no counterpart in the reference: per pixel, the view-space depth of the Gaussian
 // that blends with the largest weight alpha * T (the front-most one among equals; 0 where nothing blends).  It
 // leaves every other output as it is.
-template <bool RENDER_GEO, bool MAX_DEPTH>
+template <bool RENDER_GEO, bool MAX_DEPTH, bool PACKED>
 __global__ void __launch_bounds__(GS_TILE_PIX) __attribute__((amdgpu_waves_per_eu(MAX_DEPTH ? 5 : 6)))
 render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__ point_list, int W, int H, float fx,
                   float fy, float cx, float cy, const float2* __restrict__ means2D, const float* __restrict__ rgb,
@@ -70,11 +396,18 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                   float* __restrict__ out_plane_depth, int* __restrict__ n_render, int* __restrict__ n_consider,
                   int* __restrict__ n_contrib_tile, const float* __restrict__ depths,
                   float* __restrict__ out_max_weight_depth, const uint32_t* __restrict__ fits_word,
-                  uint16_t* __restrict__ block_hits, const float4* __restrict__ packed,
-                  const uint32_t* __restrict__ tile_order, uint32_t tiles_x) {
+                  uint32_t* __restrict__ block_hits, const float4* __restrict__ packed,
+                  const uint32_t* __restrict__ tile_order, const uint32_t* __restrict__ order_word, uint32_t long_cap,
+                  uint32_t tiles, uint32_t tiles_x) {
   constexpr bool render_geo = RENDER_GEO;
+  // (asked for together: one memory latency instead of three)
+  uint32_t fits = 1u, long_tiles = 0u, tile = blockIdx.x;
+  if (fits_word != nullptr) fits = *fits_word;
+  if (!MAX_DEPTH && long_cap != 0u) long_tiles = *order_word - 1u;
+  if (tile_order != nullptr) tile = tile_order[tile < tiles ? tile : 0u];
+  asm volatile("" : "+s"(fits), "+s"(long_tiles), "+s"(tile));
   // launched ahead of the host's decision on how the per-tile lists are built: nothing to do if they were not
-  if (fits_word != nullptr && *fits_word == 0u) return;
+  if (fits == 0u) return;
   __shared__ float s_depth[MAX_DEPTH ? BATCH : 1];
   // a slot's geometry, (x, y, A, B) and (C / 4, mark limit, C, -opacity / 2), and its channels, (r, g, b, map0)
   // and (map1 .. map4), in four arrays of 16-byte elements: one address per slot serves them all, and lanes
@@ -94,7 +427,26 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   __shared__ int s_red[2][GS_TILE_PIX / GS_WAVE];
 
   const int tid = threadIdx.x;
-  const uint32_t tile = tile_order != nullptr ? tile_order[blockIdx.x] : blockIdx.x;
+  // The first tiles of the order, as many as are long (rounded up to whole groups of eight), take four workgroups each:
+  // the four of a tile on one XCD, whose L2 they share the records in.
+  if constexpr (!MAX_DEPTH) {
+    if (long_cap != 0u) {
+      const uint32_t split = min((long_tiles + 7u) & ~7u, long_cap);
+      if (blockIdx.x < 4u * split) {
+        const uint32_t quadrant = blockIdx.x / 8u & 3u;
+        tile = tile_order[blockIdx.x / 32u * 8u + blockIdx.x % 8u];
+        const uint32_t ty = tile / tiles_x;
+        const BlendLds<RENDER_GEO> lds = {s_geo0, s_geo1, s_col0, s_col1, s_obs, &s_idx[0][0][0], s_hits, s_done, s_bad};
+        blend_quadrant<RENDER_GEO, PACKED>(lds, tile, quadrant, tile - ty * tiles_x, ty, ranges[tile], point_list, W, H, fx,
+                                           fy, cx, cy, means2D, rgb, all_map, conic_opacity, compute_locally[tile] != 0, bg,
+                                           final_T, n_contrib_px, n_contrib2loss_px, out_color, out_observe, out_all_map,
+                                           out_plane_depth, n_render, n_consider, n_contrib_tile, block_hits, packed);
+        return;
+      }
+      if (blockIdx.x - 3u * split >= tiles) return;
+      if (split != 0u) tile = tile_order[blockIdx.x - 3u * split];
+    }
+  }
   const uint32_t tile_y = tile / tiles_x, tile_x = tile - tile_y * tiles_x;
   const RowThread rt = row_thread(tile_x, tile_y);
   const int lane = rt.lane, wave = rt.wave, row = rt.row;
@@ -183,7 +535,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         hits = ellipse_hits_tile(xy, co, cp.x, cp.y, cp.z, tile_x0, tile_y0);
         return fin && mag < __builtin_inff();
       };
-      if (packed != nullptr) {
+      if constexpr (PACKED) {
         const float4* rec = packed + 4 * (size_t)g;
         const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
         float m[GS_N_MAP] = {r2.y, r2.z, r2.w, 0.f, 0.f};
@@ -213,7 +565,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
     s_hits[ts] = (uint16_t)hits;
     // (for the backward pass; a row that has saturated lists nothing, and nothing behind a row's last contributor is
     // looked at there)
-    if (block_hits != nullptr && ts < count) block_hits[range.x + (uint32_t)i * BATCH + ts] = (uint16_t)hits;
+    if (block_hits != nullptr && ts < count) block_hits[range.x + (uint32_t)i * BATCH + ts] = hits_to_bytes(hits);
     static_assert(sizeof(s_idx) == 16 * GS_TILE_PIX, "four words of the lists per thread");
     *reinterpret_cast<uint4*>(&s_idx[0][0][0] + 4 * ts) = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
@@ -431,15 +783,25 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
 
 }  // namespace
 
-template <bool GEO, bool MAXD>
+template <bool GEO, bool MAXD, bool PACKED>
 static void launch_render_fwd_variant(const RenderFwdArgs& a, hipStream_t stream) {
   const uint32_t gx = (a.W + GS_TILE_X - 1) / GS_TILE_X, gy = (a.H + GS_TILE_Y - 1) / GS_TILE_Y;
-  hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD>), dim3(gx * gy), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges,
+  const uint32_t tiles = gx * gy;
+  uint32_t long_cap = 0;
+  if (!MAXD && a.tile_order != nullptr && a.tile_order_word != nullptr && a.longest > GS_LONG_TILE)
+    long_cap = (tiles < LONG_TILES ? tiles : LONG_TILES) & ~7u;
+  hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD, PACKED>), dim3(tiles + 3 * long_cap), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges,
                      a.point_list, a.W, a.H, a.fx, a.fy, a.cx, a.cy, (const float2*)a.means2D, a.rgb, a.all_map,
                      (const float4*)a.conic_opacity, a.compute_locally, a.bg, a.final_T, a.n_contrib_px,
                      a.n_contrib2loss_px, a.out_color, a.out_observe, a.out_all_map, a.out_plane_depth, a.n_render,
                      a.n_consider, a.n_contrib_tile, a.depths, a.out_max_weight_depth, a.fits_word, a.block_hits,
-                     (const float4*)a.packed, a.tile_order, gx);
+                     (const float4*)a.packed, a.tile_order, a.tile_order_word, long_cap, tiles, gx);
+}
+
+template <bool GEO, bool MAXD>
+static void launch_render_fwd_variant(const RenderFwdArgs& a, hipStream_t stream) {
+  if (a.packed != nullptr) launch_render_fwd_variant<GEO, MAXD, true>(a, stream);
+  else launch_render_fwd_variant<GEO, MAXD, false>(a, stream);
 }
 
 int launch_render_fwd(const RenderFwdArgs& a, hipStream_t stream) {

@@ -1,0 +1,125 @@
+"""Views whose tiles have long lists, which the forward blend gives to four workgroups each: lengths around the one where
+that begins and around whole batches, pixels that saturate early, late and never, cut-off tiles, tile masks, channels that
+are not finite, packed, caller-written and gathered operands, against the oracle, bit for bit; and the gradients that come
+out of the hit words such a tile leaves."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+LONG = 3072  # entries from which on a tile is long
+
+
+@pytest.fixture(scope="module")
+def H():
+    import gpu_harness
+    return gpu_harness
+
+
+def scene(n, everywhere, opacity, seed):
+    """n Gaussians around a 73 x 43 image (5 x 3 tiles); those up to `everywhere` are entered in every tile's list."""
+    gen = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.rand(*s, generator=gen)
+    W, Hh = 73, 43
+    s1 = torch.exp(r(n) * 2.5) * 0.8
+    s2 = torch.clamp(s1 * (0.2 + 0.8 * r(n)), min=0.5)
+    ang = r(n) * 3.14159
+    c, s = torch.cos(ang), torch.sin(ang)
+    i1, i2 = 1 / s1 ** 2, 1 / s2 ** 2
+    am = torch.randn(n, 5, generator=gen)
+    am[:, 2] = am[:, 2].abs() + 2.0
+    am[:, 3] = 1.0
+    radii = torch.ceil(3 * s1).int()
+    radii[:everywhere] = 200
+    return dict(W=W, H=Hh, tan=0.5, means2D=r(n, 2) * torch.tensor([W + 8.0, Hh + 8.0]) - 4.0,
+                co=torch.stack([c * c * i1 + s * s * i2, c * s * (i1 - i2), s * s * i1 + c * c * i2,
+                                r(n) * opacity + 0.003], 1).float(),
+                radii=radii, depths=r(n) * 10 + 1, rgb=r(n, 3), am=am, bg=torch.tensor([0.3, 0.6, 0.1]),
+                up=[torch.randn(k, Hh, W, generator=gen) for k in (3, 5, 1)])
+
+
+def same(a, b):
+    return np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
+
+
+def check(H, orc, v, cl, geo, ahead, records, gradients=True):
+    from diff_gaussian_rasterization import _C
+    n = {k: t.numpy() for k, t in v.items() if isinstance(t, torch.Tensor)}
+    W, Hh, tan, P, clf = v["W"], v["H"], v["tan"], v["co"].shape[0], cl.numpy().ravel()
+    b = orc.bin_and_sort(n["radii"], n["means2D"], n["depths"], clf, W, Hh)
+    f = orc.render_fwd(b["ranges"], b["point_list"], n["means2D"], n["rgb"], n["am"], n["co"], clf, n["bg"], W, Hh, tan,
+                       tan, render_geo=geo)
+    d = {k: t.to(DEV) for k, t in v.items() if isinstance(t, torch.Tensor)}
+    rec = None
+    if records:
+        rec = torch.cat([d["means2D"], d["co"], d["rgb"], d["am"], d["depths"][:, None], torch.zeros(P, 1, device=DEV)],
+                        1).contiguous()
+    args = {"stats_collector": {}}
+    out, info = _C.render_gaussians_ex(d["bg"], Hh, W, d["means2D"], d["depths"], d["radii"], d["co"], d["rgb"],
+                                       cl.to(DEV), torch.eye(4, device=DEV), torch.zeros(3, device=DEV), tan, tan, d["am"],
+                                       geo, False, args, expected_instances=16 * P if ahead else 0,
+                                       expected_longest_list=0, blend_records=rec)
+    assert info["launched_ahead"] == ahead
+    R, color, n_render, n_consider, n_contrib, obs, oam, opd, geom, binning, img = out
+    for k, got, want in (("color", color, f["color"]), ("n_render", n_render, f["n_render"]),
+                         ("n_consider", n_consider, f["n_consider"]), ("n_contrib", n_contrib, f["n_contrib_tile"]),
+                         ("observe", obs, f["out_observe"])):
+        assert same(got.cpu().numpy(), want), k
+    if geo:
+        assert same(oam.cpu().numpy(), f["out_all_map"])
+        assert same(opd.cpu().numpy(), f["out_plane_depth"])
+    if not gradients:
+        return b
+    got = _C.render_gaussians_backward(d["bg"], tan, tan, oam, d["am"], R, geom, binning, img, cl.to(DEV),
+                                       *[u.to(DEV) for u in v["up"]], d["means2D"], d["co"], d["rgb"], geo, False, args,
+                                       binning_capacity=info["binning_capacity"], blend_records=rec)
+    g = orc.render_bwd(b["ranges"], b["point_list"], n["means2D"], n["co"], n["rgb"], n["am"], f["out_all_map"],
+                       f["final_T"], f["n_contrib"], clf, n["bg"], *[u.numpy() for u in v["up"]], W, Hh, tan, tan,
+                       render_geo=geo)
+    # a Gaussian's sum has at most 73 x 43 terms, whose magnitudes add up to some ten times the sum: another order of them
+    # moves it by sqrt(3139) * 2^-24 * 10 = 3.3e-5
+    for k, a, w in zip(("dL_dmeans2D", "dL_dmeans2D_abs", "dL_dconic_opacity", "dL_dcolors", "dL_dall_map"), got,
+                       (g["dL_dmeans2D"][:, :2], g["dL_dmeans2D_abs"], g["dL_dconic_opacity"], g["dL_dcolors"],
+                        g["dL_dall_map"])):
+        if k != "dL_dall_map" or geo:
+            assert H.rel_l2(a.cpu().numpy(), w) <= 1e-4, k
+    return b
+
+
+@pytest.mark.parametrize("n", [LONG - 1, LONG, LONG + 1, 13 * 256 - 1, 13 * 256 + 1])
+@pytest.mark.parametrize("opacity", [0.9, 0.05, 0.01])
+def test_every_tile_at_a_length(H, orc, n, opacity):
+    # 15 tiles: eight are split, the other seven are not
+    v = scene(n, n, opacity, seed=n)
+    cl = torch.ones(3, 5, dtype=torch.bool)
+    for geo, ahead, records in ((True, False, False), (True, True, True), (False, True, False), (False, False, True)):
+        b = check(H, orc, v, cl, geo, ahead, records, gradients=opacity != 0.05)
+        assert (np.diff(b["ranges"].reshape(-1, 2).astype(np.int64)) == n).all()
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("geo", [False, True])
+def test_few_long_tiles(H, orc, masked, geo):
+    # the groups of eight are filled up with tiles below the limit, empty and masked ones among them
+    v = scene(9000, 0, 0.3, seed=5)
+    near = torch.rand(9000, generator=torch.Generator().manual_seed(1)) < 0.7
+    v["means2D"][near] = v["means2D"][near] * 0.2 + torch.tensor([2.0, 30.0])
+    v["means2D"][~near, 0] *= 0.6  # (the right-most tiles have short lists or none)
+    cl = torch.ones(3, 5, dtype=torch.bool)
+    if masked:
+        cl[1] = False
+    b = check(H, orc, v, cl, geo, ahead=False, records=True)
+    lengths = np.diff(b["ranges"].reshape(-1, 2).astype(np.int64)).ravel()
+    assert 0 < (lengths >= LONG).sum() < 8 and (lengths < LONG).any()
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_channels_that_are_not_finite(H, orc, value):
+    v = scene(LONG + 300, LONG + 300, 0.05, seed=9)
+    v["rgb"][100:110, 1] = value
+    v["am"][700:720, 4] = value
+    v["am"][2900:3300:7, 0] = value
+    cl = torch.ones(3, 5, dtype=torch.bool)
+    for geo, records in ((True, True), (False, True), (True, False)):
+        check(H, orc, v, cl, geo, False, records, gradients=False)
