@@ -422,10 +422,12 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   const float sc[3] = {scales[3 * (size_t)i], scales[3 * (size_t)i + 1], scales[3 * (size_t)i + 2]};
   const float4 q4 = reinterpret_cast<const float4*>(rots)[i];
   const float q[4] = {q4.x, q4.y, q4.z, q4.w};
+  float opacity = opac[i];  // (needed by surviving Gaussians only, but asked for with the rest: see below)
   float cov6[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   GeomOut g;
   bool in_front;
   const bool ok = geom_forward(mean, sc, mod, q, nullptr, cam, W, H, tanx, tany, fx, fy, gx, gy, cov6, in_front, g);
+  asm volatile("" : "+v"(opacity));  // (otherwise the compiler moves the load behind the cull: another latency per wave)
   if (live) {
     if (cov3D != nullptr) {  // (a caller that hands scales and rotations to the backward pass needs no copy)
       float2* c6v = reinterpret_cast<float2*>(cov3D + 6 * (size_t)i);  // 24-byte rows are 8-byte aligned
@@ -436,7 +438,7 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     radii[i] = ok ? g.radius : 0;
     depths[i] = ok ? g.depth : 0.f;
     means2D[i] = ok ? make_float2(g.px, g.py) : make_float2(0.f, 0.f);
-    const float4 co = ok ? make_float4(g.conic[0], g.conic[1], g.conic[2], opac[i]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 co = ok ? make_float4(g.conic[0], g.conic[1], g.conic[2], opacity) : make_float4(0.f, 0.f, 0.f, 0.f);
     if (RECORDS) store_streaming(conic_opacity + i, co);  // (the blend kernels read the records instead)
     else conic_opacity[i] = co;
     if (tiles_touched) tiles_touched[i] = ok ? (g.rect.x1 - g.rect.x0) * (g.rect.y1 - g.rect.y0) : 0u;
@@ -455,7 +457,7 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       keep[7 * GS_WAVE] = g.conic[0];
       keep[8 * GS_WAVE] = g.conic[1];
       keep[9 * GS_WAVE] = g.conic[2];
-      keep[10 * GS_WAVE] = opac[i];
+      keep[10 * GS_WAVE] = opacity;
       keep[11 * GS_WAVE] = g.depth;
     }
   }
@@ -587,13 +589,38 @@ preprocess_fwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       }
     }
   }
-  if (!live) return;
-  rgb[3 * (size_t)i] = col[0];
-  rgb[3 * (size_t)i + 1] = col[1];
-  rgb[3 * (size_t)i + 2] = col[2];
-  clamped[3 * (size_t)i] = clm[0];
-  clamped[3 * (size_t)i + 1] = clm[1];
-  clamped[3 * (size_t)i + 2] = clm[2];
+  {
+    // the wave's 64 rows of three colours and three flags leave through LDS as consecutive words (stored from the lanes
+    // that hold them, a word or a byte of every row at a time: 20 M Gaussians 881 us, 852 so)
+    const int lane = threadIdx.x & (GS_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GS_WAVE);
+    const int wave_first = (int)blockIdx.x * GS_BLOCK_1D + wave * GS_WAVE;
+    const int rows = P - wave_first < GS_WAVE ? P - wave_first : GS_WAVE;
+    float* const lds = reinterpret_cast<float*>(s_sh[wave]);
+    uint8_t* const flags = reinterpret_cast<uint8_t*>(lds + 3 * GS_WAVE);
+    wave_sync_lds();  // (everyone has read what the buffer last held)
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      lds[3 * lane + k] = col[k];
+      flags[3 * lane + k] = clm[k];
+    }
+    wave_sync_lds();
+    float* const out = rgb + 3 * (size_t)wave_first;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const int e = j * GS_WAVE + lane;
+      if (e >= 3 * rows) continue;
+      if (RECORDS) store_streaming(out + e, lds[e]);  // (the blend kernels read the records instead)
+      else out[e] = lds[e];
+    }
+    uint8_t* const cl = clamped + 3 * (size_t)wave_first;
+    if (rows == GS_WAVE && ((uintptr_t)clamped & 3u) == 0u) {
+      if (lane < 48) reinterpret_cast<uint32_t*>(cl)[lane] = reinterpret_cast<const uint32_t*>(flags)[lane];
+    } else if (live) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) cl[3 * lane + k] = clm[k];
+    }
+  }
 }
 
 // cuda_rasterizer/forward.cu:545-620.
@@ -676,7 +703,6 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   const bool sh_mode = (SAVED || shs != nullptr) && M > 0 && (dL_dsh != nullptr);
   const bool sh_staged = sh_mode && M == 16;  // coefficient rows and their gradients go through LDS
   const float4 gco = dL_dconic_opacity[i];
-  if (dL_dopacity && in_range) dL_dopacity[i] = gco.w;  // passthrough, rasterize_points.cu:191-194
   float gm[3] = {0.f, 0.f, 0.f}, gs_[3] = {0.f, 0.f, 0.f}, gq[4] = {0.f, 0.f, 0.f, 0.f};
   float gc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const bool live = in_range && radii[i] > 0;
@@ -690,8 +716,9 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   // (zero for a Gaussian no pixel blended, culled ones first of all)
   const bool map_live = MAP && !(map_g[0] == 0.f && map_g[1] == 0.f && map_g[2] == 0.f && map_g[3] == 0.f);
   // Everything the two parts below take of a Gaussian is asked for at once: one latency for all of it, and a line that
-  // several loads share is still there.
-  float mean[3] = {0.f, 0.f, 0.f}, sc[3] = {0.f, 0.f, 0.f}, gcol[3] = {0.f, 0.f, 0.f}, dd[9];
+  // several loads share is still there.  Nothing is stored before: a load behind a store waits for the store as well.
+  float mean[3] = {0.f, 0.f, 0.f}, sc[3] = {0.f, 0.f, 0.f}, gcol[3] = {0.f, 0.f, 0.f}, dd[9], g2x = 0.f, g2y = 0.f;
+  uint8_t was_clamped[3] = {0, 0, 0};
   float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
   if (live || map_live) {
 #pragma unroll
@@ -702,9 +729,15 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       q4 = reinterpret_cast<const float4*>(rots)[i];
     }
   }
+  if (live) {
+    g2x = dL_dmean2D[(size_t)mean2D_stride * i];
+    g2y = dL_dmean2D[(size_t)mean2D_stride * i + 1];
+  }
   if (live && sh_mode) {
 #pragma unroll
     for (int k = 0; k < 3; k++) gcol[k] = dL_dcolor[3 * (size_t)i + k];
+#pragma unroll
+    for (int k = 0; k < 3; k++) was_clamped[k] = clamped[3 * (size_t)i + k];
     if (SAVED) {
 #pragma unroll
       for (int k = 0; k < 9; k++) dd[k] = dcolor_ddir[9 * (size_t)i + k];
@@ -722,7 +755,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     if (live) {
       const float d0[3] = {mean[0] - camg[0], mean[1] - camg[1], mean[2] - camg[2]};
 #pragma unroll
-      for (int ch = 0; ch < 3; ch++) gr[ch] = gcol[ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
+      for (int ch = 0; ch < 3; ch++) gr[ch] = gcol[ch] * (was_clamped[ch] ? 0.f : 1.f);
       const float dRdx[3] = {dd[0], dd[1], dd[2]}, dRdy[3] = {dd[3], dd[4], dd[5]}, dRdz[3] = {dd[6], dd[7], dd[8]};
       sh_gradient_of_mean(d0, dRdx, dRdy, dRdz, gr, sh_gm);
       const float len = sqrtf(dot3(d0, d0));
@@ -833,7 +866,6 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     const float m_w = 1.0f / (mh[3] + 0.0000001f);
     const float mul1 = (((PM[0] * mean[0] + PM[4] * mean[1]) + PM[8] * mean[2]) + PM[12]) * m_w * m_w;
     const float mul2 = (((PM[1] * mean[0] + PM[5] * mean[1]) + PM[9] * mean[2]) + PM[13]) * m_w * m_w;
-    const float g2x = dL_dmean2D[(size_t)mean2D_stride * i], g2y = dL_dmean2D[(size_t)mean2D_stride * i + 1];
     gm[0] += (PM[0] * m_w - PM[3] * mul1) * g2x + (PM[1] * m_w - PM[3] * mul2) * g2y;
     gm[1] += (PM[4] * m_w - PM[7] * mul1) * g2x + (PM[5] * m_w - PM[7] * mul2) * g2y;
     gm[2] += (PM[8] * m_w - PM[11] * mul1) * g2x + (PM[9] * m_w - PM[11] * mul2) * g2y;
@@ -863,7 +895,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       const float len = sqrtf(dot3(d0, d0));
       float gr[3];
 #pragma unroll
-      for (int ch = 0; ch < 3; ch++) gr[ch] = gcol[ch] * (clamped[3 * (size_t)i + ch] ? 0.f : 1.f);
+      for (int ch = 0; ch < 3; ch++) gr[ch] = gcol[ch] * (was_clamped[ch] ? 0.f : 1.f);
       float basis[16];
       float dRdx[3], dRdy[3], dRdz[3];
       sh_basis_and_direction_derivative<true>(D, d0[0] / len, d0[1] / len, d0[2] / len, shv, basis, dRdx, dRdy, dRdz);
@@ -956,6 +988,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   wave_rows_turn_store<3>(dL_dmean3D + 3 * wave_first, rows, gm, lds, lane);
   if (dL_dscale) wave_rows_turn_store<3>(dL_dscale + 3 * wave_first, rows, gs_, lds, lane);
   if (!in_range) return;
+  if (dL_dopacity) dL_dopacity[i] = gco.w;  // passthrough, rasterize_points.cu:191-194
   if (dL_drot) reinterpret_cast<float4*>(dL_drot)[i] = make_float4(gq[0], gq[1], gq[2], gq[3]);
   if (dL_dcov3D_out) {
 #pragma unroll
