@@ -39,6 +39,15 @@ typedef __attribute__((address_space(3))) uint64_t lds_u64;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef __attribute__((address_space(3))) unsigned long long lds_mask;
 
+// The thread's number, opaque to the optimizer: what is computed from it is computed where it is used, not once for all
+// lists (some sixty registers of addresses, which the larger kernel has not and kept in scratch memory: its lists of 20 M
+// Gaussians from 600 m took 460 us, 422 so, those of 4 M 40 and 35).
+__device__ __forceinline__ int thread_here() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 __device__ __forceinline__ uint32_t tr_wave_inclusive_scan(uint32_t v, int lane) {
 #pragma unroll
   for (int d = 1; d < GS_WAVE; d <<= 1) {
@@ -79,8 +88,8 @@ struct TileRadixLds {
   lds_u32* key;        // [BLOCK], the same memory
   lds_u32* key_count;  // [WAVES][512], behind the masks of the one-word passes
   lds_u32* count;      // [WAVES][256]
-  lds_u32* total;      // [512]
-  lds_u32* first;      // [512]
+  lds_u32* total;      // [256]
+  lds_u32* first;      // [256]
   lds_u32* base;       // [4][256] blocked sort: where the next record of a digit goes in the segment, per pass
   lds_u32* scan;       // [16]
   lds_u32* bins;       // [257] partitioned sort: first place of every leading-digit bin in the list, then its length
@@ -90,14 +99,14 @@ struct TileRadixLds {
     key_count = (lds_u32*)p + WAVES * TR_KEY_DIGITS * 2;
     count = (lds_u32*)p + LEAD_BYTES / 4;
     total = count + WAVES * TR_DIGITS;
-    first = total + TR_KEY_DIGITS;
-    base = first + TR_KEY_DIGITS;
+    first = total + TR_DIGITS;
+    base = first + TR_DIGITS;
     scan = base + TR_PASSES * TR_DIGITS;
     bins = scan + 16;
   }
   static constexpr size_t bytes() {
     return LEAD_BYTES +
-           (size_t)(WAVES * TR_DIGITS + 2 * TR_KEY_DIGITS + TR_PASSES * TR_DIGITS + 16 + TR_DIGITS + 4) * 4;
+           (size_t)(WAVES * TR_DIGITS + 2 * TR_DIGITS + TR_PASSES * TR_DIGITS + 16 + TR_DIGITS + 4) * 4;
   }
   __device__ PassLds<lds_u64*> wide() const { return {rec, (lds_mask*)rec, count, total, first, scan}; }
   __device__ PassLds<lds_u32*> narrow() const { return {key, (lds_mask*)rec, key_count, total, first, scan}; }
@@ -112,7 +121,7 @@ __device__ __forceinline__ void radix_block_pass(const Rec (&rec)[ITEMS], uint32
   constexpr int THREADS = WAVES * GS_WAVE;
   constexpr int DIGITS = 1 << DIGIT_BITS;
   static_assert(THREADS >= DIGITS, "one thread per digit in the scan");
-  const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
+  const int tid = thread_here(), lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   lds_mask* s_mask = L.mask;
   for (int i = tid; i < WAVES * DIGITS; i += THREADS) {
     s_mask[i] = 0ull;
@@ -201,8 +210,10 @@ __device__ __forceinline__ void radix_block_pass(const Rec (&rec)[ITEMS], uint32
     for (int w = 0; w < DIGITS / GS_WAVE; w++)
       if (w < wave) before += L.scan[w];
     uint32_t run = before + inc - tot;
-    L.total[tid] = tot;
-    L.first[tid] = run;
+    if constexpr (DIGITS == TR_DIGITS) {  // (the passes that go through memory ask)
+      L.total[tid] = tot;
+      L.first[tid] = run;
+    }
 #pragma unroll
     for (int w = 0; w < WAVES; w++) {
       const uint32_t c = L.count[w * DIGITS + tid];
@@ -267,7 +278,7 @@ __device__ __forceinline__ void sort_resident(uint32_t tile, uint32_t start, uin
                                               const TileRadixLds<WAVES, ITEMS>& L) {
   constexpr int THREADS = WAVES * GS_WAVE;
   constexpr uint32_t PLACE_MASK = (1u << TR_PLACE_BITS) - 1u;
-  const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
+  const int tid = thread_here(), lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   const uint32_t E = (n + THREADS - 1) / THREADS;
   const uint32_t wave_first = (uint32_t)wave * GS_WAVE * E;
   uint32_t key[ITEMS];
@@ -386,7 +397,7 @@ __device__ __forceinline__ void sort_blocked(uint32_t tile, uint32_t start, uint
                                              uint32_t* __restrict__ point_list,
                                              const TileRadixLds<WAVES, ITEMS>& L) {
   constexpr int THREADS = WAVES * GS_WAVE;
-  const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
+  const int tid = thread_here(), lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   // (one workgroup has few loads in flight: every sweep over the list keeps SWEEP of them per thread going)
   constexpr int SWEEP = 8;
   uint32_t dmin = 0xFFFFFFFFu, dmax = 0u;
@@ -551,7 +562,7 @@ __device__ __forceinline__ void sort_partitioned(uint32_t tile, uint32_t start, 
                                                  uint32_t* point_list, const TileRadixLds<WAVES, ITEMS>& L) {
   constexpr int THREADS = WAVES * GS_WAVE;
   constexpr int SWEEP = 8;  // loads a thread keeps in flight in every sweep over the list
-  const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
+  const int tid = thread_here(), lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   uint32_t dmin = 0xFFFFFFFFu, dmax = 0u;
   for (uint32_t i0 = 0; i0 < n; i0 += THREADS * SWEEP) {
     uint32_t depth_bits[SWEEP];
@@ -655,7 +666,7 @@ __device__ __forceinline__ void sort_partitioned(uint32_t tile, uint32_t start, 
 // own order, a mix of both kinds, is kept: all long jobs first then sweep their lists at the same time, bound by
 // memory in that phase and idle in the next (3 % slower), and any order that starts some of them late is worse.
 template <int WAVES, int ITEMS>
-__global__ void __launch_bounds__(WAVES * GS_WAVE)
+__global__ void __launch_bounds__(WAVES * GS_WAVE) __attribute__((amdgpu_waves_per_eu(4)))
 tile_radix_sort_kernel(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ tile_list, int step,
                        const uint32_t* __restrict__ list_count, uint32_t count_shift, uint32_t block_limit,
                        const TileRecord* __restrict__ records, TileRecord* parted, uint64_t* ping, uint64_t* pong,
