@@ -17,9 +17,11 @@
 //   dL/dx = conv(d_mu) + 2 x conv(d_xx) + y conv(d_xy) + g_l1 * mask * sign(x - y).
 // 20 bytes per pixel and channel forward (+12 for the derivative maps), 36 backward.
 // The block is as tall as wide because the horizontal pass also runs over the ten rows of halo: with 16 rows it was
-// half of the taps.  Three channels of 1152x864: 36.6 us forward and 27.5 backward with 32x16 blocks,
-// 37 and 25 now.  (Reciprocals and products instead of the divisions: 34 forward, and SSIM of an image with itself a unit
-// in the last place off 1 in two pixels of five.)
+// half of the taps.  Three channels of 1152x864: 36.6 us forward and 27.5 backward with 32x16 blocks, 34.3 and 23.2 with
+// these, 30.7 and 21.1 with the window's weights in vector registers, the horizontal pass's LDS accesses as 16-byte words
+// and the sums of both output rows formed before the tests of the rows (78 registers to 47 forward).  (Reciprocals and
+// products instead of the divisions: 34 against 37 forward, and SSIM of an image with itself a unit in the last place off
+// 1 in two pixels of five.)
 #include "gs_common.h"
 #include "gs_kernels.h"
 
@@ -31,62 +33,93 @@ constexpr int SBX = 32, SBY = 32;   // block of output pixels
 constexpr int SR = 5;               // window radius
 constexpr int STX = SBX + 2 * SR;   // staged tile: 42 columns
 constexpr int STY = SBY + 2 * SR;   //              42 rows
-constexpr int SPITCH = STX + 1;     // odd row pitch
+constexpr int SPITCH = STX + 2;     // row pitch: whole 16-byte words, which the horizontal pass reads and writes
 constexpr int SS_THREADS = 512;
 constexpr int STAGE_ROUNDS = (STX * STY + SS_THREADS - 1) / SS_THREADS;
 constexpr int HG = 4;               // adjacent columns per thread of the horizontal pass
 constexpr int VG = 2;               // adjacent rows per thread of the vertical pass
 static_assert(STY * (SBX / HG) <= SS_THREADS, "one round of the horizontal pass");
+static_assert(HG == 4 && SPITCH % 4 == 0 && SBX - HG + ((HG + 2 * SR + 3) & ~3) <= SPITCH, "16-byte words, inside the row");
 static_assert((SBX * SBY) / VG == SS_THREADS, "one thread per pair of output rows");
 
 struct SsimWindow {
   float w[2 * SR + 1];
 };
 
+// The window's weights in vector registers, six of them since it is symmetric (make_window: the same bits on both
+// sides).  A multiply-add that takes one from a scalar register, where kernel arguments are, issues at half the rate.
+struct SsimTaps {
+  float w[SR + 1];
+  __device__ __forceinline__ explicit SsimTaps(const SsimWindow& win) {
+#pragma unroll
+    for (int i = 0; i <= SR; i++) {
+      w[i] = win.w[i];
+      asm volatile("" : "+v"(w[i]));
+    }
+  }
+  __device__ __forceinline__ float operator[](int t) const { return w[t <= SR ? t : 2 * SR - t]; }
+};
+
 // Horizontal pass: s_h[q][r][c] = sum_t w[t] * product_q(r, c + t) for the STY staged rows and the SBX output
-// columns; product(r, c, v) fills the NQ quantities at staged position (r, c).
-template <int NQ, typename F>
-__device__ __forceinline__ void horizontal_pass(const SsimWindow& win, float (*s_h)[STY][SBX], F&& product) {
+// columns; product(staged, v) forms the NQ quantities of a position from the NS staged values there.
+template <int NQ, int NS, typename F>
+__device__ __forceinline__ void horizontal_pass(const SsimWindow& win, const float (*s_in)[STY][SPITCH],
+                                                float (*s_h)[STY][SBX], F&& product) {
   const int item = threadIdx.x;
   if (item >= STY * (SBX / HG)) return;
+  const SsimTaps taps(win);
   const int r = item / (SBX / HG), c0 = (item - r * (SBX / HG)) * HG;
-  float v[HG + 2 * SR][NQ];
+  float acc[HG][NQ];
 #pragma unroll
-  for (int i = 0; i < HG + 2 * SR; i++) product(r, c0 + i, v[i]);
+  for (int g = 0; g < HG + 2 * SR; g += 4) {
+    float4 quad[NS];
 #pragma unroll
-  for (int o = 0; o < HG; o++) {
-    float acc[NQ];
+    for (int k = 0; k < NS; k++) quad[k] = *reinterpret_cast<const float4*>(&s_in[k][r][c0 + g]);
 #pragma unroll
-    for (int q = 0; q < NQ; q++) acc[q] = 0.f;
+    for (int j = 0; j < 4; j++) {
+      const int i = g + j;
+      if (i >= HG + 2 * SR) continue;
+      float staged[NS], v[NQ];
 #pragma unroll
-    for (int t = 0; t < 2 * SR + 1; t++) {
+      for (int k = 0; k < NS; k++) staged[k] = j == 0 ? quad[k].x : j == 1 ? quad[k].y : j == 2 ? quad[k].z : quad[k].w;
+      product(staged, v);
 #pragma unroll
-      for (int q = 0; q < NQ; q++) acc[q] = __builtin_fmaf(win.w[t], v[o + t][q], acc[q]);
+      for (int o = 0; o < HG; o++) {
+        const int t = i - o;
+        if (t < 0 || t > 2 * SR) continue;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) acc[o][q] = __builtin_fmaf(taps[t], v[q], t == 0 ? 0.f : acc[o][q]);
+      }
     }
-#pragma unroll
-    for (int q = 0; q < NQ; q++) s_h[q][r][c0 + o] = acc[q];
   }
+#pragma unroll
+  for (int q = 0; q < NQ; q++)
+    *reinterpret_cast<float4*>(&s_h[q][r][c0]) = make_float4(acc[0][q], acc[1][q], acc[2][q], acc[3][q]);
 }
 
 // Vertical pass for output rows ty and ty + 1 of column tx: out[o][q] = sum_t w[t] * s_h[q][ty + o + t][tx].
 template <int NQ>
 __device__ __forceinline__ void vertical_pass(const SsimWindow& win, const float (*s_h)[STY][SBX], int ty, int tx,
                                               float (*out)[NQ]) {
-  float v[VG + 2 * SR][NQ];
+  const SsimTaps taps(win);
 #pragma unroll
   for (int i = 0; i < VG + 2 * SR; i++) {
+    float v[NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; q++) v[i][q] = s_h[q][ty + i][tx];
+    for (int q = 0; q < NQ; q++) v[q] = s_h[q][ty + i][tx];
+#pragma unroll
+    for (int o = 0; o < VG; o++) {
+      const int t = i - o;
+      if (t < 0 || t > 2 * SR) continue;
+#pragma unroll
+      for (int q = 0; q < NQ; q++) out[o][q] = __builtin_fmaf(taps[t], v[q], t == 0 ? 0.f : out[o][q]);
+    }
   }
+  // (formed here: sunk behind the caller's test of the second row, that row's sums keep all the values they are made of)
 #pragma unroll
   for (int o = 0; o < VG; o++) {
 #pragma unroll
-    for (int q = 0; q < NQ; q++) out[o][q] = 0.f;
-#pragma unroll
-    for (int t = 0; t < 2 * SR + 1; t++) {
-#pragma unroll
-      for (int q = 0; q < NQ; q++) out[o][q] = __builtin_fmaf(win.w[t], v[o + t][q], out[o][q]);
-    }
+    for (int q = 0; q < NQ; q++) asm volatile("" : "+v"(out[o][q]));
   }
 }
 
@@ -95,9 +128,8 @@ ssim_l1_fwd_kernel(int H, int W, const float* __restrict__ img1, const float* __
                    const uint8_t* __restrict__ mask, SsimWindow win, float* __restrict__ l1_map,
                    float* __restrict__ ssim_map, float* __restrict__ d_mu, float* __restrict__ d_xx,
                    float* __restrict__ d_xy) {
-  __shared__ float s_a[STY][SPITCH];
-  __shared__ float s_b[STY][SPITCH];
-  __shared__ float s_h[5][STY][SBX];
+  __shared__ __attribute__((aligned(16))) float s_in[2][STY][SPITCH];
+  __shared__ __attribute__((aligned(16))) float s_h[5][STY][SBX];
   // Workgroups go to the eight XCDs in turn; dealt out this way an XCD holds a contiguous run of blocks, so the
   // halo that neighbouring blocks share is fetched into one second-level cache once, not into up to eight.
   const uint32_t blocks_xy = gridDim.x * gridDim.y;
@@ -122,14 +154,14 @@ ssim_l1_fwd_kernel(int H, int W, const float* __restrict__ img1, const float* __
       const int e = threadIdx.x + k * SS_THREADS;
       const int r = e / STX, c = e - r * STX;
       if (e < STX * STY) {
-        s_a[r][c] = va[k];
-        s_b[r][c] = vb[k];
+        s_in[0][r][c] = va[k];
+        s_in[1][r][c] = vb[k];
       }
     }
   }
   __syncthreads();
-  horizontal_pass<5>(win, s_h, [&](int r, int c, float* v) {
-    const float p = s_a[r][c], q = s_b[r][c];
+  horizontal_pass<5, 2>(win, s_in, s_h, [](const float* staged, float* v) {
+    const float p = staged[0], q = staged[1];
     v[0] = p; v[1] = q; v[2] = p * p; v[3] = q * q; v[4] = p * q;
   });
   __syncthreads();
@@ -153,7 +185,7 @@ ssim_l1_fwd_kernel(int H, int W, const float* __restrict__ img1, const float* __
     const float S = (A1 * A2) / (B1 * B2);
     const float mk = mask ? (float)(mask[(size_t)y * W + x] != 0) : 1.0f;
     const size_t oidx = plane + (size_t)y * W + x;
-    const float p = s_a[ty + o + SR][tx + SR], q = s_b[ty + o + SR][tx + SR];
+    const float p = s_in[0][ty + o + SR][tx + SR], q = s_in[1][ty + o + SR][tx + SR];
     ssim_map[oidx] = S * mk;
     l1_map[oidx] = fabsf(p - q) * mk;
     if (d_mu != nullptr) {
@@ -169,8 +201,8 @@ ssim_l1_bwd_kernel(int H, int W, const float* __restrict__ img1, const float* __
                    const uint8_t* __restrict__ mask, SsimWindow win, const float* __restrict__ g_l1,
                    const float* __restrict__ g_ssim, const float* __restrict__ d_mu,
                    const float* __restrict__ d_xx, const float* __restrict__ d_xy, float* __restrict__ dimg1) {
-  __shared__ float s_d[3][STY][SPITCH];
-  __shared__ float s_h[3][STY][SBX];
+  __shared__ __attribute__((aligned(16))) float s_d[3][STY][SPITCH];
+  __shared__ __attribute__((aligned(16))) float s_h[3][STY][SBX];
   // Workgroups go to the eight XCDs in turn; dealt out this way an XCD holds a contiguous run of blocks, so the
   // halo that neighbouring blocks share is fetched into one second-level cache once, not into up to eight.
   const uint32_t blocks_xy = gridDim.x * gridDim.y;
@@ -205,8 +237,8 @@ ssim_l1_bwd_kernel(int H, int W, const float* __restrict__ img1, const float* __
     }
   }
   __syncthreads();
-  horizontal_pass<3>(win, s_h, [&](int r, int c, float* v) {
-    v[0] = s_d[0][r][c]; v[1] = s_d[1][r][c]; v[2] = s_d[2][r][c];
+  horizontal_pass<3, 3>(win, s_d, s_h, [](const float* staged, float* v) {
+    v[0] = staged[0]; v[1] = staged[1]; v[2] = staged[2];
   });
   __syncthreads();
   const int tx = threadIdx.x % SBX, ty = (threadIdx.x / SBX) * VG;
