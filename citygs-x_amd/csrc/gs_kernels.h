@@ -97,7 +97,7 @@ int launch_duplicate_with_keys(int P, int W, int H, const float* means2D, const 
                                uint64_t* keys, uint32_t* values, uint32_t* emission /*optional*/,
                                hipStream_t stream);
 // ---- binning by tile: counting sort by tile + per-tile sorts (tile_bucket.hip, tile_radix.hip) ----
-constexpr int TILE_SORT_SMALL = 2048;  // longest list the register sort takes; longer ones go to the radix sort
+constexpr int TILE_SORT_SMALL = 4096;  // longest list the register sort takes; longer ones go to the radix sort
 int bucket_max_tiles();
 size_t bucket_table_bytes(int T);
 // tiles_touched per Gaussian, the workgroup-by-tile table, ranges (2 words per tile), the lists of tiles with more

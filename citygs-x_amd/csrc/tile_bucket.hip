@@ -7,7 +7,7 @@
 //   2. one workgroup per tile sorting its segment in registers by (depth bits, emission index): the emission index
 //      is unique, so the order does not depend on how the scatter happened to fill the segment, and it is the
 //      order a stable sort on the depth bits would leave.
-// No pass over all instances per digit, no look-back chain.  Lists of up to 2048 records are sorted in registers
+// No pass over all instances per digit, no look-back chain.  Lists of up to 4096 records are sorted in registers
 // by a bitonic network (below); longer ones by a radix sort on the depth bits that stays inside the CU
 // (tile_radix.hip).  The ranges kernel sorts the tiles into those classes.
 #include <atomic>
@@ -569,8 +569,8 @@ bucket_scatter_staged_kernel(int P, int per_block, int nblocks, uint32_t gx, uin
 }
 
 // 2. Per-tile sort, register variant: one workgroup of W waves per tile (4 for lists of up to 256 records, 8 up
-// to 2048).  A wave holds 64 E keys, key i = r * 64 + lane in register r of its lane, and the waves hold
-// consecutive runs of 64 E, so a list of up to 64 E W records is sorted with E = 1 .. 4.  In the bitonic network
+// to 4096).  A wave holds 64 E keys, key i = r * 64 + lane in register r of its lane, and the waves hold
+// consecutive runs of 64 E, so a list of up to 64 E W records is sorted with E = 1 .. 8.  In the bitonic network
 // a step pairs i with i ^ j:
 //   j < 64        the partner sits in another lane, same register: one cross-lane read, keep the smaller or larger;
 //   64 <= j < 64E the partner sits in another register of the same lane: no data moves at all;
@@ -578,7 +578,11 @@ bucket_scatter_staged_kernel(int P, int per_block, int nblocks, uint32_t gx, uin
 //                 4 waves, 6 with 8).
 // A tile takes as long as the instruction stream of one of its waves, and the kernel as long as its longest tiles:
 // a long list is spread over more waves rather than more registers per lane (eight waves with four records per
-// lane for 2048 records, not four with eight).
+// lane for 2048 records, not four with eight).  Lists of 2049 to 4096 records take eight, so that a view without longer
+// ones needs no further launch and the others have these lists under way beside the shorter: with a radix sort in a
+// launch of its own for them (tile_radix.hip, which is left with what a caller's options put between the limits) the two
+// kernels took 25.0 + 27.8 us for 20 M Gaussians from 600 m, 22.8 + 25.8 for 4 M from the air, 18.7 + 22.0 at street level
+// and, with hardly such a list, 22.6 + 4.7 for 1 M; this one takes 42.2, 44.4, 39.9 and 23.9.
 //
 // The key is one 32-bit word: (depth bits - smallest depth bits of the list) >> shift in the high bits, the
 // record's place in the unsorted segment in the low log2(64 E W) bits; shift is what it takes to fit the list's
@@ -729,8 +733,8 @@ __device__ __forceinline__ void register_sort_tile(uint32_t t, uint32_t start, u
                                                    uint64_t* __restrict__ keys, uint32_t* __restrict__ emission,
                                                    uint32_t* __restrict__ point_list, uint64_t* s_x) {
   constexpr uint32_t M = 64u * E * W;
-  constexpr int PLACE_BITS = M == 256 ? 8 : M == 512 ? 9 : M == 1024 ? 10 : 11;
-  static_assert(M == 1u << PLACE_BITS, "a list of 256 to 2048 places");
+  constexpr int PLACE_BITS = M == 256 ? 8 : M == 512 ? 9 : M == 1024 ? 10 : M == 2048 ? 11 : 12;
+  static_assert(M == 1u << PLACE_BITS, "a list of 256 to 4096 places");
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t* s_words = reinterpret_cast<uint32_t*>(s_x);
   uint32_t v[E];
@@ -793,7 +797,8 @@ __device__ __forceinline__ void register_sort_tile(uint32_t t, uint32_t start, u
   const uint64_t* sorted = s_x;
 #pragma unroll
   for (int r = 0; r < E; r++) {
-    const uint32_t i = ((wave * E + r) << 6) | lane;
+    uint32_t i = ((wave * E + r) << 6) | lane;
+    asm volatile("" : "+v"(i));  // (the lists' addresses are computed one entry at a time: of all eight at once they spill)
     if (i < n)
       emit_list_entry(t, start, n, i, gaussian[r], [&](uint32_t q) { return sorted[q]; }, keys, emission, point_list,
                       lo, shift);
@@ -840,7 +845,7 @@ __device__ __forceinline__ void order_tiles(uint32_t T, const uint32_t* __restri
 // Dynamic LDS: 8 bytes per record of the longest list the kernel takes, rounded up to a power of two (at least
 // 256 records).  Lists of more than max_n records are left to the radix sort's kernels.
 #define GS_SORT_CASE(EE, WW) register_sort_tile<EE, WW>(t, start, n, records, keys, emission, point_list, s_exchange)
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8)))
 tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord* __restrict__ records,
                            uint64_t* __restrict__ keys, uint32_t* __restrict__ emission,
                            uint32_t* __restrict__ point_list, uint32_t max_n,
@@ -862,7 +867,8 @@ tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord
     GS_SORT_CASE(1, 4);
   } else if (n <= 512) GS_SORT_CASE(1, 8);
   else if (n <= 1024) GS_SORT_CASE(2, 8);
-  else GS_SORT_CASE(4, 8);
+  else if (n <= 2048) GS_SORT_CASE(4, 8);
+  else GS_SORT_CASE(8, 8);
 }
 #undef GS_SORT_CASE
 
@@ -1003,7 +1009,9 @@ int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t sma
     const uint32_t* tile_lists = (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 1) * (size_t)T;
     // scratch: `capacity` 16-byte records for the lists that are split first, then as many 8-byte words
     uint64_t* pong = (uint64_t*)((char*)scratch + (size_t)capacity * 16);
-    if (launch_tile_radix_sort(T, (radix_tiles & 0xFFFFu) != 0u, lng, ranges, tile_lists,
+    // (the smaller kernel has lists only where the caller's options leave some between the two limits)
+    const bool mid = (radix_tiles & 0xFFFFu) != 0u && radix_mid_limit(small_limit, block_limit) > small_limit;
+    if (launch_tile_radix_sort(T, mid, lng, ranges, tile_lists,
                                tile_lists + T, block_limit, records, scratch, keys, pong, keys, emission, point_list,
                                fits, stream))
       return 1;

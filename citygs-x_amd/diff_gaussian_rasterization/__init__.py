@@ -243,7 +243,7 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_setti
 _expectations = {}
 _MARGIN = 1.25
 _MAX_EXPECTATIONS = 16
-_LONG_LIST = 4096  # what the smaller of the radix sort's kernels holds
+_LONG_LIST = 4096  # the longest list that is sorted in registers
 
 
 def _expectation(key):
@@ -253,10 +253,10 @@ def _expectation(key):
     instances, longest, *long = seen
     if longest <= 0:
         return 0, 0  # a view without per-tile lists (a tile grid too large for them): nothing to gain
-    # whole variants of the register sort (256 ... 2048 records per list), so that a slightly longer list still
-    # fits, then what the smaller of the radix sort's kernels holds; beyond it any length (0): the larger one
-    # is launched as well.  So it is for lists beyond the register sort wherever a view of this size has had a longer one:
-    # cameras on both sides of that length would miss the bound at every other view, for the 4.6 us of an empty launch.
+    # whole variants of the register sort (256 ... 4096 records per list), so that a slightly longer list still fits; beyond
+    # it any length (0): the radix sort is launched as well.  So it is for its longest lists wherever a view of this size
+    # has had a longer one: cameras on both sides of that length would miss the bound at every other view, for the 4.6 us
+    # of an empty launch.
     cap = 256
     while cap < longest * _MARGIN:
         cap *= 2

@@ -145,12 +145,12 @@ int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const 
 /* No counterpart in the reference: per-call options of gs_render_forward (NULL = all defaults).  A field below
  * zero keeps its default; struct_bytes is sizeof(gs_render_options) as the caller compiled it.
  * gs_render_forward builds the per-tile lists by bucketing the instances by tile (a counting sort) and sorting
- * each tile's list on its own: lists of up to 2048 records in registers, longer ones by a radix sort on the depth
+ * each tile's list on its own: lists of up to 4096 records in registers, longer ones by a radix sort on the depth
  * bits that one workgroup runs inside its CU (up to 16384 records at once; a longer list is first split by its
  * leading depth bits into parts that fit).  A tile grid of more than 30000 tiles takes the reference's own route instead: (tile | depth) keys
  * (rasterizer_impl.cu:74-117), one radix sort over all of them (:675-684), identifyTileRanges (:122-144).  All
  * give the same lists bit for bit.
- * tile_sort_small_limit lowers the list length that is sorted in registers (default and maximum 2048; 0 = the
+ * tile_sort_small_limit lowers the list length that is sorted in registers (default and maximum 4096; 0 = the
  * view takes the reference's route) and tile_sort_block_records the number of records the per-tile radix sort
  * holds at once (default and maximum 16384; 0 or below = default), so that small scenes can exercise every route.
  * The library keeps no such setting between calls. */
@@ -164,7 +164,7 @@ typedef struct gs_render_options {
    * instance count before it goes on: it sizes the binning buffer for expected_instances, launches the list
    * kernels and the blend right behind the counting kernels, and lets a device-side check turn them into no-ops
    * if the view has more instances than that or a list longer than expected_longest_list (0 = any length; a
-   * figure of at most 2048 spares the launch of the radix sort's kernels); in that case the lists are built
+   * figure of at most 4096 spares the launch of the radix sort's kernels); in that case the lists are built
    * again the ordinary way, so the result never depends on the expectation, only the time does. */
   int64_t expected_instances;
   /* The blend kernels' operand records of this view's Gaussians as gs_preprocess_forward wrote them (their
