@@ -96,16 +96,18 @@ struct BlendLds {
 // the exponent and alpha of entry k, all four the transmittance in front of every entry (a chain of four products), and
 // lane k the sums of channels 2 k and 2 k + 1 (channel k where only the colour is rendered), in the order of the entries.
 // Every number is formed by the operations the other way has, in its order: the same bits.
-template <bool RENDER_GEO, bool PACKED>
+// Of packed records only.  Operands gathered from their arrays come five lines of memory to an entry, and four workgroups
+// gather them four times: 10 M at street level whose records are not packed take 705 us unsplit, 810 split, and 860 with the
+// gathers a batch ahead like the records here; the sparser of two such views 253, 258 and 258.
+template <bool RENDER_GEO>
 __device__ __forceinline__ void blend_quadrant(
     const BlendLds<RENDER_GEO> lds, uint32_t tile, uint32_t quadrant, uint32_t tile_x, uint32_t tile_y, uint2 range,
-    const uint32_t* __restrict__ point_list, int W, int H, float fx, float fy, float cx, float cy,
-    const float2* __restrict__ means2D, const float* __restrict__ rgb, const float* __restrict__ all_map,
-    const float4* __restrict__ conic_opacity, bool computed_here, const float* __restrict__ bg,
-    float* __restrict__ final_T, uint32_t* __restrict__ n_contrib_px, uint32_t* __restrict__ n_contrib2loss_px,
-    float* __restrict__ out_color, int* __restrict__ out_observe, float* __restrict__ out_all_map,
-    float* __restrict__ out_plane_depth, int* __restrict__ n_render, int* __restrict__ n_consider,
-    int* __restrict__ n_contrib_tile, uint32_t* __restrict__ block_hits, const float4* __restrict__ packed) {
+    const uint32_t* __restrict__ point_list, int W, int H, float fx, float fy, float cx, float cy, bool computed_here,
+    const float* __restrict__ bg, float* __restrict__ final_T, uint32_t* __restrict__ n_contrib_px,
+    uint32_t* __restrict__ n_contrib2loss_px, float* __restrict__ out_color, int* __restrict__ out_observe,
+    float* __restrict__ out_all_map, float* __restrict__ out_plane_depth, int* __restrict__ n_render,
+    int* __restrict__ n_consider, int* __restrict__ n_contrib_tile, uint32_t* __restrict__ block_hits,
+    const float4* __restrict__ packed) {
   const int tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   const uint32_t k = (uint32_t)lane & 3u;
   const uint32_t x0 = tile_x * GS_TILE_X + 8u * (quadrant & 1u), y0 = tile_y * GS_TILE_Y + 8u * (quadrant >> 1);
@@ -148,7 +150,7 @@ __device__ __forceinline__ void blend_quadrant(
     r0 = rec[0], r1 = rec[1], r2 = rec[2];
   };
   r0 = r1 = r2 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (PACKED && tid < total) fetch(g);
+  if (tid < total) fetch(g);
   for (int base = 0;; base += BATCH) {
     const int count = total - base < BATCH ? total - base : BATCH;
     bool finite = true;
@@ -174,22 +176,10 @@ __device__ __forceinline__ void blend_quadrant(
         hits = ellipse_hits_quadrant(xy, co, cp.x, cp.y, cp.z, (float)x0, (float)y0);
         return fin && mag < __builtin_inff();
       };
-      if constexpr (PACKED) {
-        // (the last two words are on the line that the others came with)
-        const float2 r3 = RENDER_GEO ? *reinterpret_cast<const float2*>(packed + 4 * (size_t)g + 3) : make_float2(0.f, 0.f);
-        const float m[GS_N_MAP] = {r2.y, r2.z, r2.w, r3.x, r3.y};
-        finite = stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
-      } else {
-        const float2 xy = means2D[g];
-        const float4 co = conic_opacity[g];
-        const float c0 = rgb[3 * (size_t)g], c1 = rgb[3 * (size_t)g + 1], c2 = rgb[3 * (size_t)g + 2];
-        float m[GS_N_MAP] = {0.f, 0.f, 0.f, 0.f, 0.f};
-        if (RENDER_GEO) {
-#pragma unroll
-          for (int ch = 0; ch < GS_N_MAP; ch++) m[ch] = all_map[5 * (size_t)g + ch];
-        }
-        finite = stage(xy, co, c0, c1, c2, m);
-      }
+      // (the last two words are on the line that the others came with)
+      const float2 r3 = RENDER_GEO ? *reinterpret_cast<const float2*>(packed + 4 * (size_t)g + 3) : make_float2(0.f, 0.f);
+      const float m[GS_N_MAP] = {r2.y, r2.z, r2.w, r3.x, r3.y};
+      finite = stage(make_float2(r0.x, r0.y), make_float4(r0.z, r0.w, r1.x, r1.y), r1.z, r1.w, r2.x, m);
       if (block_hits != nullptr)
         reinterpret_cast<uint8_t*>(block_hits + range.x + (uint32_t)(base + ts))[quadrant] = (uint8_t)hits;
     }
@@ -202,7 +192,7 @@ __device__ __forceinline__ void blend_quadrant(
     lds.idx[ts] = 0u;  // (a word of the four lists per thread; bytes behind a list's end are slot 0)
     __syncthreads();
     g = g_next;
-    if (PACKED && base + BATCH + tid < total) fetch(g);
+    if (base + BATCH + tid < total) fetch(g);
     {
       const int tn = not_hoisted(tid) + base + 2 * BATCH;
       g_next = tn < total ? point_list[range.x + (uint32_t)tn] : 0u;
@@ -403,7 +393,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   // (asked for together: one memory latency instead of three)
   uint32_t fits = 1u, long_tiles = 0u, tile = blockIdx.x;
   if (fits_word != nullptr) fits = *fits_word;
-  if (!MAX_DEPTH && long_cap != 0u) long_tiles = *order_word - 1u;
+  if (PACKED && !MAX_DEPTH && long_cap != 0u) long_tiles = *order_word - 1u;
   if (tile_order != nullptr) tile = tile_order[tile < tiles ? tile : 0u];
   asm volatile("" : "+s"(fits), "+s"(long_tiles), "+s"(tile));
   // launched ahead of the host's decision on how the per-tile lists are built: nothing to do if they were not
@@ -429,7 +419,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   const int tid = threadIdx.x;
   // The first tiles of the order, as many as are long (rounded up to whole groups of eight), take four workgroups each:
   // the four of a tile on one XCD, whose L2 they share the records in.
-  if constexpr (!MAX_DEPTH) {
+  if constexpr (PACKED && !MAX_DEPTH) {
     if (long_cap != 0u) {
       const uint32_t split = min((long_tiles + 7u) & ~7u, long_cap);
       if (blockIdx.x < 4u * split) {
@@ -437,10 +427,10 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         tile = tile_order[blockIdx.x / 32u * 8u + blockIdx.x % 8u];
         const uint32_t ty = tile / tiles_x;
         const BlendLds<RENDER_GEO> lds = {s_geo0, s_geo1, s_col0, s_col1, s_obs, &s_idx[0][0][0], s_hits, s_done, s_bad};
-        blend_quadrant<RENDER_GEO, PACKED>(lds, tile, quadrant, tile - ty * tiles_x, ty, ranges[tile], point_list, W, H, fx,
-                                           fy, cx, cy, means2D, rgb, all_map, conic_opacity, compute_locally[tile] != 0, bg,
-                                           final_T, n_contrib_px, n_contrib2loss_px, out_color, out_observe, out_all_map,
-                                           out_plane_depth, n_render, n_consider, n_contrib_tile, block_hits, packed);
+        blend_quadrant<RENDER_GEO>(lds, tile, quadrant, tile - ty * tiles_x, ty, ranges[tile], point_list, W, H, fx, fy, cx,
+                                   cy, compute_locally[tile] != 0, bg, final_T, n_contrib_px, n_contrib2loss_px, out_color,
+                                   out_observe, out_all_map, out_plane_depth, n_render, n_consider, n_contrib_tile,
+                                   block_hits, packed);
         return;
       }
       if (blockIdx.x - 3u * split >= tiles) return;
@@ -788,7 +778,7 @@ static void launch_render_fwd_variant(const RenderFwdArgs& a, hipStream_t stream
   const uint32_t gx = (a.W + GS_TILE_X - 1) / GS_TILE_X, gy = (a.H + GS_TILE_Y - 1) / GS_TILE_Y;
   const uint32_t tiles = gx * gy;
   uint32_t long_cap = 0;
-  if (!MAXD && a.tile_order != nullptr && a.tile_order_word != nullptr && a.longest > GS_LONG_TILE)
+  if (PACKED && !MAXD && a.tile_order != nullptr && a.tile_order_word != nullptr && a.longest > GS_LONG_TILE)
     long_cap = (tiles < LONG_TILES ? tiles : LONG_TILES) & ~7u;
   hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD, PACKED>), dim3(tiles + 3 * long_cap), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges,
                      a.point_list, a.W, a.H, a.fx, a.fy, a.cx, a.cy, (const float2*)a.means2D, a.rgb, a.all_map,

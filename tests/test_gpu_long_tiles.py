@@ -43,7 +43,7 @@ def same(a, b):
     return np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
 
 
-def check(H, orc, v, cl, geo, ahead, records, gradients=True):
+def check(H, orc, v, cl, geo, ahead, records, gradients=True, gathered=False):
     from diff_gaussian_rasterization import _C
     n = {k: t.numpy() for k, t in v.items() if isinstance(t, torch.Tensor)}
     W, Hh, tan, P, clf = v["W"], v["H"], v["tan"], v["co"].shape[0], cl.numpy().ravel()
@@ -56,9 +56,11 @@ def check(H, orc, v, cl, geo, ahead, records, gradients=True):
         rec = torch.cat([d["means2D"], d["co"], d["rgb"], d["am"], d["depths"][:, None], torch.zeros(P, 1, device=DEV)],
                         1).contiguous()
     args = {"stats_collector": {}}
+    R = b["point_list"].shape[0]
+    assert gathered == (not records and R * 5 <= P * 4)  # (the library packs records itself above that)
     out, info = _C.render_gaussians_ex(d["bg"], Hh, W, d["means2D"], d["depths"], d["radii"], d["co"], d["rgb"],
                                        cl.to(DEV), torch.eye(4, device=DEV), torch.zeros(3, device=DEV), tan, tan, d["am"],
-                                       geo, False, args, expected_instances=16 * P if ahead else 0,
+                                       geo, False, args, expected_instances=R + R // 8 if ahead else 0,
                                        expected_longest_list=0, blend_records=rec)
     assert info["launched_ahead"] == ahead
     R, color, n_render, n_consider, n_contrib, obs, oam, opd, geom, binning, img = out
@@ -96,6 +98,16 @@ def test_every_tile_at_a_length(H, orc, n, opacity):
     for geo, ahead, records in ((True, False, False), (True, True, True), (False, True, False), (False, False, True)):
         b = check(H, orc, v, cl, geo, ahead, records, gradients=opacity != 0.05)
         assert (np.diff(b["ranges"].reshape(-1, 2).astype(np.int64)) == n).all()
+
+
+@pytest.mark.parametrize("n", [LONG - 1, LONG, 13 * 256 + 1])
+def test_operands_that_are_gathered(H, orc, n):
+    # (fewer instances than Gaussians: nobody packs records, and no tile is split)
+    v = scene(20 * n, n, 0.05, seed=n)
+    v["radii"][n:] = 0
+    cl = torch.ones(3, 5, dtype=torch.bool)
+    for geo, ahead in ((True, False), (True, True), (False, True)):
+        check(H, orc, v, cl, geo, ahead, records=False, gathered=True)
 
 
 @pytest.mark.parametrize("masked", [False, True])
