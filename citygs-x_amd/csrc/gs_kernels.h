@@ -265,7 +265,7 @@ struct RenderFwdArgs {
   // one 64-byte line instead of gathering them from means2D, conic_opacity, rgb, all_map (and depths)
   const float* packed = nullptr;
   const uint32_t* tile_order = nullptr;  // optional (T): the order in which the tiles are taken (launch_tile_sort)
-  // the word launch_tile_sort leaves beside it (1 + the number of tiles with more than GS_LONG_TILE entries), and a bound
+  // the word launch_tile_sort leaves beside it (1 + the number of tiles with GS_LONG_TILE entries or more), and a bound
   // on the longest list
   const uint32_t* tile_order_word = nullptr;
   uint32_t longest = 0;

@@ -374,7 +374,8 @@ __device__ __forceinline__ void blend_quadrant(
 // MAX_DEPTH adds one output with no counterpart in the reference: per pixel, the view-space depth of the Gaussian
 // that blends with the largest weight alpha * T (the front-most one among equals; 0 where nothing blends).  It
 // leaves every other output as it is.
-template <bool RENDER_GEO, bool MAX_DEPTH, bool PACKED>
+// LONG: the first tiles of the order are split as far as they are long; the operands are packed, the order is there.
+template <bool RENDER_GEO, bool MAX_DEPTH, bool LONG>
 __global__ void __launch_bounds__(GS_TILE_PIX) __attribute__((amdgpu_waves_per_eu(MAX_DEPTH ? 5 : 6)))
 render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__ point_list, int W, int H, float fx,
                   float fy, float cx, float cy, const float2* __restrict__ means2D, const float* __restrict__ rgb,
@@ -390,14 +391,20 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                   const uint32_t* __restrict__ tile_order, const uint32_t* __restrict__ order_word, uint32_t long_cap,
                   uint32_t tiles, uint32_t tiles_x) {
   constexpr bool render_geo = RENDER_GEO;
-  // (asked for together: one memory latency instead of three)
-  uint32_t fits = 1u, long_tiles = 0u, tile = blockIdx.x;
-  if (fits_word != nullptr) fits = *fits_word;
-  if (PACKED && !MAX_DEPTH && long_cap != 0u) long_tiles = *order_word - 1u;
-  if (tile_order != nullptr) tile = tile_order[tile < tiles ? tile : 0u];
-  asm volatile("" : "+s"(fits), "+s"(long_tiles), "+s"(tile));
   // launched ahead of the host's decision on how the per-tile lists are built: nothing to do if they were not
-  if (fits == 0u) return;
+  uint32_t tile, long_tiles = 0u;
+  if constexpr (LONG) {
+    // (asked for together: one memory latency instead of three)
+    uint32_t fits = 1u;
+    if (fits_word != nullptr) fits = *fits_word;
+    long_tiles = *order_word - 1u;
+    tile = tile_order[blockIdx.x < tiles ? blockIdx.x : 0u];
+    asm volatile("" : "+s"(fits), "+s"(long_tiles), "+s"(tile));
+    if (fits == 0u) return;
+  } else {
+    if (fits_word != nullptr && *fits_word == 0u) return;
+    tile = tile_order != nullptr ? tile_order[blockIdx.x] : blockIdx.x;
+  }
   __shared__ float s_depth[MAX_DEPTH ? BATCH : 1];
   // a slot's geometry, (x, y, A, B) and (C / 4, mark limit, C, -opacity / 2), and its channels, (r, g, b, map0)
   // and (map1 .. map4), in four arrays of 16-byte elements: one address per slot serves them all, and lanes
@@ -419,23 +426,21 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   const int tid = threadIdx.x;
   // The first tiles of the order, as many as are long (rounded up to whole groups of eight), take four workgroups each:
   // the four of a tile on one XCD, whose L2 they share the records in.
-  if constexpr (PACKED && !MAX_DEPTH) {
-    if (long_cap != 0u) {
-      const uint32_t split = min((long_tiles + 7u) & ~7u, long_cap);
-      if (blockIdx.x < 4u * split) {
-        const uint32_t quadrant = blockIdx.x / 8u & 3u;
-        tile = tile_order[blockIdx.x / 32u * 8u + blockIdx.x % 8u];
-        const uint32_t ty = tile / tiles_x;
-        const BlendLds<RENDER_GEO> lds = {s_geo0, s_geo1, s_col0, s_col1, s_obs, &s_idx[0][0][0], s_hits, s_done, s_bad};
-        blend_quadrant<RENDER_GEO>(lds, tile, quadrant, tile - ty * tiles_x, ty, ranges[tile], point_list, W, H, fx, fy, cx,
-                                   cy, compute_locally[tile] != 0, bg, final_T, n_contrib_px, n_contrib2loss_px, out_color,
-                                   out_observe, out_all_map, out_plane_depth, n_render, n_consider, n_contrib_tile,
-                                   block_hits, packed);
-        return;
-      }
-      if (blockIdx.x - 3u * split >= tiles) return;
-      if (split != 0u) tile = tile_order[blockIdx.x - 3u * split];
+  if constexpr (LONG) {
+    const uint32_t split = min((long_tiles + 7u) & ~7u, long_cap);
+    if (blockIdx.x < 4u * split) {
+      const uint32_t quadrant = blockIdx.x / 8u & 3u;
+      tile = tile_order[blockIdx.x / 32u * 8u + blockIdx.x % 8u];
+      const uint32_t ty = tile / tiles_x;
+      const BlendLds<RENDER_GEO> lds = {s_geo0, s_geo1, s_col0, s_col1, s_obs, &s_idx[0][0][0], s_hits, s_done, s_bad};
+      blend_quadrant<RENDER_GEO>(lds, tile, quadrant, tile - ty * tiles_x, ty, ranges[tile], point_list, W, H, fx, fy, cx,
+                                 cy, compute_locally[tile] != 0, bg, final_T, n_contrib_px, n_contrib2loss_px, out_color,
+                                 out_observe, out_all_map, out_plane_depth, n_render, n_consider, n_contrib_tile,
+                                 block_hits, packed);
+      return;
     }
+    if (blockIdx.x - 3u * split >= tiles) return;
+    if (split != 0u) tile = tile_order[blockIdx.x - 3u * split];
   }
   const uint32_t tile_y = tile / tiles_x, tile_x = tile - tile_y * tiles_x;
   const RowThread rt = row_thread(tile_x, tile_y);
@@ -525,7 +530,7 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         hits = ellipse_hits_tile(xy, co, cp.x, cp.y, cp.z, tile_x0, tile_y0);
         return fin && mag < __builtin_inff();
       };
-      if constexpr (PACKED) {
+      if (LONG || packed != nullptr) {
         const float4* rec = packed + 4 * (size_t)g;
         const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
         float m[GS_N_MAP] = {r2.y, r2.z, r2.w, 0.f, 0.f};
@@ -773,36 +778,37 @@ render_fwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
 
 }  // namespace
 
-template <bool GEO, bool MAXD, bool PACKED>
-static void launch_render_fwd_variant(const RenderFwdArgs& a, hipStream_t stream) {
+template <bool GEO, bool MAXD, bool LONG>
+static void launch_render_fwd_variant(const RenderFwdArgs& a, uint32_t long_cap, hipStream_t stream) {
   const uint32_t gx = (a.W + GS_TILE_X - 1) / GS_TILE_X, gy = (a.H + GS_TILE_Y - 1) / GS_TILE_Y;
-  const uint32_t tiles = gx * gy;
-  uint32_t long_cap = 0;
-  if (PACKED && !MAXD && a.tile_order != nullptr && a.tile_order_word != nullptr && a.longest > GS_LONG_TILE)
-    long_cap = (tiles < LONG_TILES ? tiles : LONG_TILES) & ~7u;
-  hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD, PACKED>), dim3(tiles + 3 * long_cap), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges,
-                     a.point_list, a.W, a.H, a.fx, a.fy, a.cx, a.cy, (const float2*)a.means2D, a.rgb, a.all_map,
-                     (const float4*)a.conic_opacity, a.compute_locally, a.bg, a.final_T, a.n_contrib_px,
+  hipLaunchKernelGGL((render_fwd_kernel<GEO, MAXD, LONG>), dim3(gx * gy + 3 * long_cap), dim3(GS_TILE_PIX), 0, stream,
+                     (const uint2*)a.ranges, a.point_list, a.W, a.H, a.fx, a.fy, a.cx, a.cy, (const float2*)a.means2D, a.rgb,
+                     a.all_map, (const float4*)a.conic_opacity, a.compute_locally, a.bg, a.final_T, a.n_contrib_px,
                      a.n_contrib2loss_px, a.out_color, a.out_observe, a.out_all_map, a.out_plane_depth, a.n_render,
                      a.n_consider, a.n_contrib_tile, a.depths, a.out_max_weight_depth, a.fits_word, a.block_hits,
-                     (const float4*)a.packed, a.tile_order, a.tile_order_word, long_cap, tiles, gx);
+                     (const float4*)a.packed, a.tile_order, a.tile_order_word, long_cap, gx * gy, gx);
 }
 
-template <bool GEO, bool MAXD>
-static void launch_render_fwd_variant(const RenderFwdArgs& a, hipStream_t stream) {
-  if (a.packed != nullptr) launch_render_fwd_variant<GEO, MAXD, true>(a, stream);
-  else launch_render_fwd_variant<GEO, MAXD, false>(a, stream);
+// A view that may have long tiles (as far as the bound on its longest list says) and whose operands are packed has a kernel
+// that splits them.  The others' is without: in one kernel the second way costs the first registers and its start three
+// loads.  1 M Gaussians, 1152x864: 94.8 us with it, 92.7 without, rendering alone 100.6 and 97.9; 300 k, colour only, 55.7 and
+// 54.5.
+template <bool GEO>
+static void launch_render_fwd_geo(const RenderFwdArgs& a, hipStream_t stream) {
+  const uint32_t tiles = (uint32_t)((a.W + GS_TILE_X - 1) / GS_TILE_X) * (uint32_t)((a.H + GS_TILE_Y - 1) / GS_TILE_Y);
+  const uint32_t long_cap = (tiles < LONG_TILES ? tiles : LONG_TILES) & ~7u;
+  if (a.out_max_weight_depth != nullptr)
+    launch_render_fwd_variant<GEO, true, false>(a, 0u, stream);
+  else if (a.packed != nullptr && a.tile_order != nullptr && a.tile_order_word != nullptr && a.longest >= GS_LONG_TILE &&
+           long_cap != 0u)
+    launch_render_fwd_variant<GEO, false, true>(a, long_cap, stream);
+  else
+    launch_render_fwd_variant<GEO, false, false>(a, 0u, stream);
 }
 
 int launch_render_fwd(const RenderFwdArgs& a, hipStream_t stream) {
-  const bool maxd = a.out_max_weight_depth != nullptr;
-  if (a.render_geo) {
-    if (maxd) launch_render_fwd_variant<true, true>(a, stream);
-    else launch_render_fwd_variant<true, false>(a, stream);
-  } else {
-    if (maxd) launch_render_fwd_variant<false, true>(a, stream);
-    else launch_render_fwd_variant<false, false>(a, stream);
-  }
+  if (a.render_geo) launch_render_fwd_geo<true>(a, stream);
+  else launch_render_fwd_geo<false>(a, stream);
   return 0;
 }
 

@@ -811,7 +811,7 @@ __device__ __forceinline__ void register_sort_tile(uint32_t t, uint32_t start, u
 // the image) ends with a few long tiles on an idle chip (backward blend 904 -> 716 us, forward 610 -> 564; views from
 // the air, whose lists differ less, take the same time either way).  The place inside a class is whatever the LDS counter
 // hands out (about ascending): no result depends on it.
-// order_word: 1 + the number of tiles with more than GS_LONG_TILE entries, which are the first of the order.  The two
+// order_word: 1 + the number of tiles with GS_LONG_TILE entries or more, which are the first of the order.  The two
 // per-tile sums that the forward blend's four workgroups of such a tile add up are cleared here.
 __device__ __forceinline__ void order_tiles(uint32_t T, const uint32_t* __restrict__ ranges, uint32_t* __restrict__ order,
                                             uint32_t* __restrict__ order_word, int* __restrict__ n_consider,

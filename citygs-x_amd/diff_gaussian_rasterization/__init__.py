@@ -244,6 +244,7 @@ _expectations = {}
 _MARGIN = 1.25
 _MAX_EXPECTATIONS = 16
 _LONG_LIST = 4096  # the longest list that is sorted in registers
+_LONG_TILE = 3072  # a list from which on the forward blend splits its tile
 
 
 def _expectation(key):
@@ -263,6 +264,16 @@ def _expectation(key):
     return int(instances * _MARGIN) + 65536, (0 if cap > _LONG_LIST or (cap == _LONG_LIST and any(long)) else cap)
 
 
+def _launch_bounds(key):
+    """The expectation as a view is launched with it: where the longest list, margin included, leaves no tile to split, the
+    bound says so (views that may have such tiles have a forward blend of their own, 2 us slower where there are none)."""
+    instances, bound = _expectation(key)
+    seen = _expectations.get(key)
+    if bound == _LONG_LIST and seen is not None and seen[1] * _MARGIN < _LONG_TILE:
+        bound = _LONG_TILE - 1
+    return instances, bound
+
+
 def _remember(key, instances, longest):
     seen = _expectations.pop(key, ())  # (re-inserted at the end: the dict keeps insertion order)
     _expectations[key] = (instances, longest, longest > _LONG_LIST or any(seen[2:]))
@@ -279,7 +290,7 @@ class _RenderGaussians(torch.autograd.Function):
         avoid = bool(cuda_args.get("avoid_pixel_all2all", False)) if cuda_args is not None else False
         mask = extended_compute_locally if avoid else compute_locally
         key = (rs.image_height, rs.image_width, means2D.device)
-        expected_instances, expected_longest = _expectation(key)
+        expected_instances, expected_longest = _launch_bounds(key)
         blend = getattr(means2D, "_gs_blend", None)
         records = (blend.records if blend is not None and blend.usable((means2D, conic_opacity, rgb, depths), all_maps,
                                                                        rs.render_geo) else None)

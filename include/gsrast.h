@@ -164,7 +164,8 @@ typedef struct gs_render_options {
    * instance count before it goes on: it sizes the binning buffer for expected_instances, launches the list
    * kernels and the blend right behind the counting kernels, and lets a device-side check turn them into no-ops
    * if the view has more instances than that or a list longer than expected_longest_list (0 = any length; a
-   * figure of at most 4096 spares the launch of the radix sort's kernels); in that case the lists are built
+   * figure of at most 4096 spares the launch of the radix sort's kernels, one below 3072 a blend kernel that is
+   * ready to split the tiles of longer lists); in that case the lists are built
    * again the ordinary way, so the result never depends on the expectation, only the time does. */
   int64_t expected_instances;
   /* The blend kernels' operand records of this view's Gaussians as gs_preprocess_forward wrote them (their

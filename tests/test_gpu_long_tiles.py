@@ -43,7 +43,7 @@ def same(a, b):
     return np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
 
 
-def check(H, orc, v, cl, geo, ahead, records, gradients=True, gathered=False):
+def check(H, orc, v, cl, geo, ahead, records, gradients=True, gathered=False, bound=0):
     from diff_gaussian_rasterization import _C
     n = {k: t.numpy() for k, t in v.items() if isinstance(t, torch.Tensor)}
     W, Hh, tan, P, clf = v["W"], v["H"], v["tan"], v["co"].shape[0], cl.numpy().ravel()
@@ -61,8 +61,8 @@ def check(H, orc, v, cl, geo, ahead, records, gradients=True, gathered=False):
     out, info = _C.render_gaussians_ex(d["bg"], Hh, W, d["means2D"], d["depths"], d["radii"], d["co"], d["rgb"],
                                        cl.to(DEV), torch.eye(4, device=DEV), torch.zeros(3, device=DEV), tan, tan, d["am"],
                                        geo, False, args, expected_instances=R + R // 8 if ahead else 0,
-                                       expected_longest_list=0, blend_records=rec)
-    assert info["launched_ahead"] == ahead
+                                       expected_longest_list=bound, blend_records=rec)
+    assert info["launched_ahead"] == (ahead and (bound == 0 or info["longest_list"] <= bound))
     R, color, n_render, n_consider, n_contrib, obs, oam, opd, geom, binning, img = out
     for k, got, want in (("color", color, f["color"]), ("n_render", n_render, f["n_render"]),
                          ("n_consider", n_consider, f["n_consider"]), ("n_contrib", n_contrib, f["n_contrib_tile"]),
@@ -92,12 +92,21 @@ def check(H, orc, v, cl, geo, ahead, records, gradients=True, gathered=False):
 @pytest.mark.parametrize("n", [LONG - 1, LONG, LONG + 1, 13 * 256 - 1, 13 * 256 + 1])
 @pytest.mark.parametrize("opacity", [0.9, 0.05, 0.01])
 def test_every_tile_at_a_length(H, orc, n, opacity):
-    # 15 tiles: eight are split, the other seven are not
+    # 15 tiles: of long ones eight are split, the other seven are not
     v = scene(n, n, opacity, seed=n)
     cl = torch.ones(3, 5, dtype=torch.bool)
     for geo, ahead, records in ((True, False, False), (True, True, True), (False, True, False), (False, False, True)):
         b = check(H, orc, v, cl, geo, ahead, records, gradients=opacity != 0.05)
         assert (np.diff(b["ranges"].reshape(-1, 2).astype(np.int64)) == n).all()
+
+
+@pytest.mark.parametrize("n,bound", [(LONG - 1, LONG - 1), (LONG - 1, LONG), (LONG - 1, 4096), (LONG, LONG - 1), (LONG, LONG)])
+def test_bounds_on_the_longest_list(H, orc, n, bound):
+    # launched ahead without the way for long tiles, with it but without such a tile, and without it where one turns up
+    v = scene(n, n, 0.05, seed=n)
+    cl = torch.ones(3, 5, dtype=torch.bool)
+    for geo in (True, False):
+        check(H, orc, v, cl, geo, True, True, bound=bound)
 
 
 @pytest.mark.parametrize("n", [LONG - 1, LONG, 13 * 256 + 1])

@@ -363,3 +363,20 @@ def test_expectations_of_cameras_on_both_sides_of_a_long_list():
     finally:
         dgr._expectations.clear()
         dgr._expectations.update(saved)
+
+
+def test_bound_that_leaves_no_tile_to_split():
+    # a quarter more than the longest list is below 3072: the view is launched without the way for longer lists
+    import diff_gaussian_rasterization as dgr
+    saved = dict(dgr._expectations)
+    dgr._expectations.clear()
+    try:
+        bounds = []
+        for longest in (0, 100, 1638, 1639, 2457, 2458, 3276, 4500, 2457, 1638):
+            dgr._remember("size", 1000, longest)
+            bounds.append(dgr._launch_bounds("size")[1])
+        assert bounds == [0, 256, 2048, 3071, 3071, 4096, 4096, 0, 0, 2048]
+        assert dgr._launch_bounds("no such size") == (0, 0)
+    finally:
+        dgr._expectations.clear()
+        dgr._expectations.update(saved)
