@@ -844,8 +844,12 @@ __device__ __forceinline__ void order_tiles(uint32_t T, const uint32_t* __restri
 // Workgroup 0 orders the tiles for the blend kernels, workgroup t + 1 sorts tile t.
 // Dynamic LDS: 8 bytes per record of the longest list the kernel takes, rounded up to a power of two (at least
 // 256 records).  Lists of more than max_n records are left to the radix sort's kernels.
+// MAX_E: the most keys a lane has.  Views without lists beyond 2048 have a kernel without the way for eight: in the other one
+// (64 registers to 40) the shorter lists take longer too.  1 M Gaussians, 1920x1080, lists up to 839: 27.2 us with it, 25.1
+// without; 160 k, 1709x858, 13.5 and 12.3; 300 k, 1237x822, 12.4 and 11.7.
 #define GS_SORT_CASE(EE, WW) register_sort_tile<EE, WW>(t, start, n, records, keys, emission, point_list, s_exchange)
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8)))
+template <int MAX_E>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MAX_E == 8 ? 8 : 2)))
 tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord* __restrict__ records,
                            uint64_t* __restrict__ keys, uint32_t* __restrict__ emission,
                            uint32_t* __restrict__ point_list, uint32_t max_n,
@@ -861,14 +865,14 @@ tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord
   const uint32_t t = blockIdx.x - 1;
   const uint32_t start = ranges[2 * t];
   const uint32_t n = ranges[2 * t + 1] - start;
-  if (n == 0 || n > (uint32_t)TILE_SORT_SMALL || n > max_n) return;
+  if (n == 0 || n > 512u * MAX_E || n > max_n) return;
   if (n <= 256) {
     if (threadIdx.x >= 256) return;  // (half the workgroup is enough; a wave that has left is not waited for)
     GS_SORT_CASE(1, 4);
   } else if (n <= 512) GS_SORT_CASE(1, 8);
   else if (n <= 1024) GS_SORT_CASE(2, 8);
-  else if (n <= 2048) GS_SORT_CASE(4, 8);
-  else GS_SORT_CASE(8, 8);
+  else if (MAX_E == 4 || n <= 2048) GS_SORT_CASE(4, 8);
+  else if constexpr (MAX_E == 8) GS_SORT_CASE(8, 8);
 }
 #undef GS_SORT_CASE
 
@@ -1000,9 +1004,9 @@ int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t sma
   const uint32_t whole = longest < small_limit ? longest : small_limit;  // the longest list sorted in registers
   uint32_t m = 256;
   while (m < whole) m <<= 1;
-  hipLaunchKernelGGL(tile_sort_registers_kernel, dim3(T + 1), dim3(512), (size_t)m * sizeof(uint64_t), stream, ranges,
-                     (const TileRecord*)records, keys, emission, point_list, small_limit, fits, tile_order,
-                     tile_order_word, n_consider, n_contrib);
+  hipLaunchKernelGGL(whole > 2048 ? tile_sort_registers_kernel<8> : tile_sort_registers_kernel<4>, dim3(T + 1), dim3(512),
+                     (size_t)m * sizeof(uint64_t), stream, ranges, (const TileRecord*)records, keys, emission, point_list,
+                     small_limit, fits, tile_order, tile_order_word, n_consider, n_contrib);
   if (longest > small_limit) {
     // (a launch with nothing to do takes 4.6 us of the device: a view whose longest list is bounded does without)
     const bool lng = (radix_tiles >> 16) != 0u && longest > radix_mid_limit(small_limit, block_limit);
