@@ -125,7 +125,8 @@ int launch_bucket_scatter(int P, int W, int H, const float* means2D, const float
 int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t small_limit, uint32_t block_limit,
                      const uint32_t* ranges, const void* table, const void* records, void* scratch, int64_t capacity,
                      uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
-                     uint32_t* tile_order_word, int* n_consider, int* n_contrib, bool ahead_of_host, hipStream_t stream);
+                     uint32_t* tile_order_word, uint32_t longest_split, int* n_consider, int* n_contrib,
+                     bool ahead_of_host, hipStream_t stream);
 int tile_radix_mid_records();    // records one workgroup of the radix sort's smaller kernel holds (4096)
 int tile_radix_block_records();  // ... and of its larger kernel (16384): longer lists are sorted in blocks
 int launch_tile_radix_sort(int T, bool mid, bool lng, const uint32_t* ranges, const uint32_t* tile_lists,
@@ -231,11 +232,22 @@ int launch_sort_pairs_u32(int64_t n, uint32_t* keys_a, uint32_t* keys_b, uint32_
 int64_t sort_clear_words(int64_t n, int end_bit);
 
 // ---- tile render ----
-// A list from which on a tile is blended by four workgroups (render_fwd.hip); a power of two or one and a half of one, since
-// the tiles are ordered by classes of these lengths.  A whole training view, us, with 2048, 3072, 4096, 6144 and without: 4 M
-// Gaussians from the air 1492, 1469, 1481, 1518, 1560; at street level, 10 M, 2848, 2842, 2820, 2813, 2937; rendering 20 M
-// from 600 m 2264, 2260, 2258, 2282, 2545.  Shorter lists pay for the instructions without ending a view.
+// Which tiles are blended by four workgroups (render_fwd.hip): those with GS_LONG_TILE entries or more, if no more than
+// GS_LONG_TILES have so many; else those with 4/3 of it, and with the geometry channels twice of it, at the most (the tiles
+// are ordered by classes of these lengths).  And none where the longest list is below two of GS_BLEND_SLOTS shares of the
+// view's entries: a tile takes 31 ns an entry, the full chip 42 ps, so the view does not end on a tile.  Split, a tile takes
+// 1.45 times the instructions: beyond a few hundred tiles, or where the chip is full to the end, that is all it does.  The
+// forward blend, us, unsplit, from 3072, 4096 and 6144 entries on, and as the rule has it:
+//   geometry channels: 4 M from the air 293, 194, 205, 241: 194; 5 M, 1500x900, 207, 227, 207, 206: 207; oblique, 3 M, 202,
+//   233, 206, 198: 202; 3 M, 800x600, 225, 262, 257, 212: 212; 2 M, 640x480, 202, 215, 180, 195: 180; 10 M at street level
+//   483, 375, 353, 343: 343; 8 M from 600 m 367, 305, 312, 312: 312
+//   colour only: 4 M from the air 221, 180, 192, 221: 180; oblique, 3 M, 171, 205, 178, 171: 171; 3 M, 500x400, 264, 234, 211,
+//   240: 211; 8 M and 20 M from 600 m 344, 264, 270, 282: 270 and 679, 415, 407, 428: 407
+// Over 45 such views the worst is 0.5 % slower than unsplit and the mean 1 % above the best of the columns.
 constexpr uint32_t GS_LONG_TILE = 3072;
+constexpr uint32_t GS_LONG_TILES = 340;
+constexpr uint32_t GS_BLEND_SLOTS = 1536;  // six workgroups of the forward blend on each of 256 CUs
+inline uint32_t longest_split_list(bool render_geo) { return render_geo ? GS_LONG_TILE * 2 : GS_LONG_TILE / 3 * 4; }
 
 struct RenderFwdArgs {
   int P, W, H;
@@ -265,7 +277,7 @@ struct RenderFwdArgs {
   // one 64-byte line instead of gathering them from means2D, conic_opacity, rgb, all_map (and depths)
   const float* packed = nullptr;
   const uint32_t* tile_order = nullptr;  // optional (T): the order in which the tiles are taken (launch_tile_sort)
-  // the word launch_tile_sort leaves beside it (1 + the number of tiles with GS_LONG_TILE entries or more), and a bound
+  // the word launch_tile_sort leaves beside it (1 + the number of tiles to split), and a bound
   // on the longest list
   const uint32_t* tile_order_word = nullptr;
   uint32_t longest = 0;

@@ -811,31 +811,57 @@ __device__ __forceinline__ void register_sort_tile(uint32_t t, uint32_t start, u
 // the image) ends with a few long tiles on an idle chip (backward blend 904 -> 716 us, forward 610 -> 564; views from
 // the air, whose lists differ less, take the same time either way).  The place inside a class is whatever the LDS counter
 // hands out (about ascending): no result depends on it.
-// order_word: 1 + the number of tiles with GS_LONG_TILE entries or more, which are the first of the order.  The two
-// per-tile sums that the forward blend's four workgroups of such a tile add up are cleared here.
+// order_word: 1 + the number of tiles that the forward blend splits, which are the first of the order (the rule: see
+// GS_LONG_TILE; longest_split is what it depends on).  The two per-tile sums that the four workgroups of such a tile add up
+// are cleared here.  s_count: CLASSES + 2 words.
 __device__ __forceinline__ void order_tiles(uint32_t T, const uint32_t* __restrict__ ranges, uint32_t* __restrict__ order,
-                                            uint32_t* __restrict__ order_word, int* __restrict__ n_consider,
-                                            int* __restrict__ n_contrib, uint32_t* s_count) {
+                                            uint32_t* __restrict__ order_word, uint32_t longest_split,
+                                            int* __restrict__ n_consider, int* __restrict__ n_contrib, uint32_t* s_count) {
   constexpr int CLASSES = 64;
   auto class_of_length = [](uint32_t n) {  // 0 = the longest lists
     if (n == 0) return CLASSES - 1;
     const int msb = 31 - __clz((int)n);
     return CLASSES - 2 - (2 * msb + (msb > 0 ? (int)((n >> (msb - 1)) & 1u) : 0));
   };
-  auto class_of = [&](uint32_t t) { return class_of_length(ranges[2 * t + 1] - ranges[2 * t]); };
-  if (threadIdx.x < CLASSES) s_count[threadIdx.x] = 0u;
+  auto length = [&](uint32_t t) { return ranges[2 * t + 1] - ranges[2 * t]; };
+  if (threadIdx.x < CLASSES + 2) s_count[threadIdx.x] = 0u;
   __syncthreads();
-  for (uint32_t t = threadIdx.x; t < T; t += blockDim.x) atomicAdd(&s_count[class_of(t)], 1u);
+  uint32_t entries = 0u, longest = 0u;
+  for (uint32_t t = threadIdx.x; t < T; t += blockDim.x) {
+    const uint32_t n = length(t);
+    entries += n;
+    longest = max(longest, n);
+    atomicAdd(&s_count[class_of_length(n)], 1u);
+  }
+#pragma unroll
+  for (int d = GS_WAVE / 2; d >= 1; d >>= 1) {
+    entries += __shfl_xor(entries, d, GS_WAVE);
+    longest = max(longest, __shfl_xor(longest, d, GS_WAVE));
+  }
+  if ((threadIdx.x & (GS_WAVE - 1)) == 0) {
+    atomicAdd(&s_count[CLASSES], entries);
+    atomicMax(&s_count[CLASSES + 1], longest);
+  }
   __syncthreads();
   if (threadIdx.x < CLASSES) {  // (one wave)
     const uint32_t c = s_count[threadIdx.x];
     s_count[threadIdx.x] = wave_inclusive_scan_u32(c, (int)threadIdx.x) - c;
   }
   __syncthreads();
-  if (threadIdx.x == 0) *order_word = 1u + s_count[class_of_length(GS_LONG_TILE) + 1];
+  if (threadIdx.x == 0) {
+    uint32_t split = 0u;
+    if ((uint64_t)s_count[CLASSES + 1] * (GS_BLEND_SLOTS / 2) >= s_count[CLASSES]) {
+#pragma unroll
+      for (uint32_t from : {GS_LONG_TILE, GS_LONG_TILE / 3 * 4, GS_LONG_TILE * 2}) {
+        split = s_count[class_of_length(from) + 1];
+        if (split <= GS_LONG_TILES || from >= longest_split) break;
+      }
+    }
+    *order_word = 1u + split;
+  }
   __syncthreads();
   for (uint32_t t = threadIdx.x; t < T; t += blockDim.x) {
-    order[atomicAdd(&s_count[class_of(t)], 1u)] = t;
+    order[atomicAdd(&s_count[class_of_length(length(t))], 1u)] = t;
     n_consider[t] = 0;
     n_contrib[t] = 0;
   }
@@ -854,12 +880,13 @@ tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord
                            uint64_t* __restrict__ keys, uint32_t* __restrict__ emission,
                            uint32_t* __restrict__ point_list, uint32_t max_n,
                            const uint32_t* __restrict__ fits_word, uint32_t* __restrict__ order,
-                           uint32_t* __restrict__ order_word, int* __restrict__ n_consider,
+                           uint32_t* __restrict__ order_word, uint32_t longest_split, int* __restrict__ n_consider,
                            int* __restrict__ n_contrib) {
   extern __shared__ uint64_t s_exchange[];
   if (fits_word != nullptr && *fits_word == 0u) return;  // launched ahead of the host's decision: see the scatter
   if (blockIdx.x == 0) {
-    order_tiles(gridDim.x - 1, ranges, order, order_word, n_consider, n_contrib, reinterpret_cast<uint32_t*>(s_exchange));
+    order_tiles(gridDim.x - 1, ranges, order, order_word, longest_split, n_consider, n_contrib,
+                reinterpret_cast<uint32_t*>(s_exchange));
     return;
   }
   const uint32_t t = blockIdx.x - 1;
@@ -997,7 +1024,8 @@ int launch_bucket_scatter(int P, int W, int H, const float* means2D, const float
 int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t small_limit, uint32_t block_limit,
                      const uint32_t* ranges, const void* table, const void* records, void* scratch, int64_t capacity,
                      uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
-                     uint32_t* tile_order_word, int* n_consider, int* n_contrib, bool ahead_of_host, hipStream_t stream) {
+                     uint32_t* tile_order_word, uint32_t longest_split, int* n_consider, int* n_contrib,
+                     bool ahead_of_host, hipStream_t stream) {
   if (T <= 0 || longest == 0) return 0;
   const uint32_t* fits = ahead_of_host ? bucket_fits_word(table, T) : nullptr;
   if (small_limit == 0 || small_limit > (uint32_t)TILE_SORT_SMALL) small_limit = TILE_SORT_SMALL;
@@ -1006,7 +1034,7 @@ int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t sma
   while (m < whole) m <<= 1;
   hipLaunchKernelGGL(whole > 2048 ? tile_sort_registers_kernel<8> : tile_sort_registers_kernel<4>, dim3(T + 1), dim3(512),
                      (size_t)m * sizeof(uint64_t), stream, ranges, (const TileRecord*)records, keys, emission, point_list,
-                     small_limit, fits, tile_order, tile_order_word, n_consider, n_contrib);
+                     small_limit, fits, tile_order, tile_order_word, longest_split, n_consider, n_contrib);
   if (longest > small_limit) {
     // (a launch with nothing to do takes 4.6 us of the device: a view whose longest list is bounded does without)
     const bool lng = (radix_tiles >> 16) != 0u && longest > radix_mid_limit(small_limit, block_limit);

@@ -144,3 +144,61 @@ def test_channels_that_are_not_finite(H, orc, value):
     cl = torch.ones(3, 5, dtype=torch.bool)
     for geo, records in ((True, True), (False, True), (True, False)):
         check(H, orc, v, cl, geo, False, records, gradients=False)
+
+
+def tiles_split(lengths, geo):
+    """How many tiles the forward blend splits, from the rule's statement."""
+    if 2 * lengths.sum() > 1536 * lengths.max():
+        return 0
+    for least in (3072, 4096, 6144) if geo else (3072, 4096):
+        count = int((lengths >= least).sum())
+        if count <= 340:
+            break
+    return count
+
+
+# (tiles in x and y, entries of every tile, further entries of the first)
+@pytest.mark.parametrize("gx,gy,n,first", [
+    (17, 1, 3072, 0),      # three groups of eight, the last one filled up with what there is
+    (34, 10, 3072, 0),     # as many as are split at this length
+    (31, 11, 3072, 2000),  # one more: the next length
+    (31, 11, 4096, 0),     # one more at the next length too: the third, or all of them where there is none
+    (31, 11, 6143, 1), (31, 11, 6144, 0),
+    (32, 24, 4100, 0),     # two shares of the entries, just
+    (769, 1, 4100, 0),     # one tile more, and the longest list is below two shares
+    (103, 10, 6144, 2300)  # more tiles to split than are
+])
+@pytest.mark.parametrize("geo", [True, False])
+def test_which_tiles_are_split(H, gx, gy, n, first, geo):
+    """The number of tiles to split, which the blend finds behind the word for packed records, and every output against
+    the lists built the other way, whose tiles are never split."""
+    import ctypes as C
+    import gsrast_native as gn
+    from diff_gaussian_rasterization import _C
+    W, Hh, P = 16 * gx - 3, 16 * gy - 5, n + first
+    gen = torch.Generator().manual_seed(n)
+    r = lambda *s: torch.rand(*s, generator=gen)
+    means2D = r(P, 2) * torch.tensor([float(W), float(Hh)])
+    means2D[n:] = torch.tensor([8.0, 8.0])
+    radii = torch.full((P,), 20000, dtype=torch.int32)
+    radii[n:] = 1
+    size = 1.0 + 12.0 * r(P)
+    co = torch.stack([1 / size ** 2, torch.zeros(P), 1 / size ** 2, 0.02 + 0.3 * r(P)], 1)
+    am = torch.randn(P, 5, generator=gen)
+    am[:, 2] = am[:, 2].abs() + 2.0
+    d = [t.to(DEV) for t in (means2D, r(P) * 10 + 1, radii, co, r(P, 3))]
+    cl = torch.ones(gy, gx, dtype=torch.bool, device=DEV)
+    outs = []
+    for limits in ((-1, -1), (0, 0)):
+        outs.append(_C.render_gaussians(torch.tensor([0.3, 0.6, 0.1], device=DEV), Hh, W, *d, cl, torch.eye(4, device=DEV),
+                                        torch.zeros(3, device=DEV), 0.5, 0.5, am.to(DEV), geo, False,
+                                        {"stats_collector": {}, "tile_sort_limits": limits}))
+    for a, b in zip(outs[0][1:8], outs[1][1:8]):
+        assert torch.equal(a, b)
+    lengths = outs[0][2].flatten().cpu().numpy().astype(np.int64)
+    assert (np.sort(lengths) == np.sort(np.array([n + first] + [n] * (gx * gy - 1)))).all()
+    total = C.c_size_t()
+    gn.check(gn.lib.gs_geometry_state_layout(P, None, None, C.byref(total)), "layout")
+    geom = outs[0][8]
+    at = -geom.data_ptr() % 256 + total.value - 512 + 4  # (the last two words but the alignment's reserve)
+    assert int(geom[at:at + 4].view(torch.int32)) == 1 + tiles_split(lengths, geo)
