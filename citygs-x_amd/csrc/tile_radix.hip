@@ -41,7 +41,8 @@ typedef __attribute__((address_space(3))) unsigned long long lds_mask;
 
 // The thread's number, opaque to the optimizer: what is computed from it is computed where it is used, not once for all
 // lists (some sixty registers of addresses, which the larger kernel has not and kept in scratch memory: its lists of 20 M
-// Gaussians from 600 m took 460 us, 422 so, those of 4 M 40 and 35).
+// Gaussians from 600 m took 460 us, 422 so, those of 4 M 40 and 35).  It still keeps some there: 58 registers, 84 bytes a
+// lane, where it had 99 and 232.
 __device__ __forceinline__ int thread_here() {
   int t = (int)threadIdx.x;
   asm volatile("" : "+v"(t));

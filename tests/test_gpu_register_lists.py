@@ -1,5 +1,6 @@
 """The register sort with eight keys a lane: lists of 2049 to 4096 entries, filled exactly, one short and one over; and views
-whose lists take every number of keys a lane at once, with and without such long ones."""
+whose lists take every number of keys a lane at once, with and without such long ones.  The same views with the register
+sort's limit lowered, where the smaller kernel of the per-tile radix sort has what lies between the limit and 4096."""
 import ctypes as C
 
 import numpy as np
@@ -29,8 +30,9 @@ def test_depths_that_agree_in_their_leading_bits(orc, H, P):
 
 
 @pytest.mark.parametrize("longest", [2048, 2049, 4096, 4097])
-@pytest.mark.parametrize("bound", [None, 2048, 4096, 0])
-def test_lists_of_every_class_in_one_view(orc, H, longest, bound):
+@pytest.mark.parametrize("bound,limits", [(None, None), (2048, None), (4096, None), (0, None), (None, (2048, 0)),
+                                          (None, (256, 0)), (None, (1500, 0)), (0, (2048, 0))])
+def test_lists_of_every_class_in_one_view(orc, H, longest, bound, limits):
     import gsrast_native as gn
     from diff_gaussian_rasterization import _C
     lengths = [1, 64, 256, 257, 512, 0, 513, 1024, 1025, longest - 1, longest, 3]
@@ -51,7 +53,7 @@ def test_lists_of_every_class_in_one_view(orc, H, longest, bound):
     out, info = _C.render_gaussians_ex(
         torch.zeros(3, device=lists.DEV), Hh, W, dev(means2D), dev(depths), dev(radii), co,
         torch.zeros(P, 3, device=lists.DEV), dev(cl), torch.eye(4, device=lists.DEV), torch.zeros(3, device=lists.DEV), 1.0,
-        1.0, torch.zeros(P, 5, device=lists.DEV), False, False, {"stats_collector": {}},
+        1.0, torch.zeros(P, 5, device=lists.DEV), False, False, {"stats_collector": {}, "tile_sort_limits": limits},
         expected_instances=0 if bound is None else P + 100, expected_longest_list=bound or 0)
     assert out[0] == P and info["launched_ahead"] == (bound is not None and (bound == 0 or longest <= bound))
     binB = out[9]

@@ -134,8 +134,9 @@ def test_equal_depths_keep_emission_order(orc, H):
                                       (110_000, "radix"), (230_000, "blocks"), (230_000, "blocks4k")])
 def test_long_lists(orc, H, P, expect):
     """A small image under many large Gaussians: lists of several thousand records per tile.  Up to 4096 the
-    smaller kernel of the per-tile radix sort takes them, up to 16384 the larger one, both inside the CU; beyond
-    that (or beyond the block size the call asks for) the larger kernel sorts block by block through memory."""
+    smaller kernel of the per-tile radix sort takes them where the call lowers the register sort's limit (as "mid" does),
+    up to 16384 the larger one, both inside the CU; beyond that (or beyond the block size the call asks for) the larger
+    kernel sorts block by block through memory."""
     import gs_scenes
     import gsrast_native as gn
     from diff_gaussian_rasterization import _C
@@ -155,7 +156,9 @@ def test_long_lists(orc, H, P, expect):
               "blocks": (16384, 65536), "blocks4k": (16384, 65536)}[expect]
     assert lo < longest <= hi, longest
     limits = None
-    if expect == "radix":
+    if expect == "mid":
+        limits = (2048, 0)
+    elif expect == "radix":
         limits = (0, 0)
     elif expect == "blocks4k":
         limits = (-1, 5000)
@@ -370,8 +373,8 @@ def test_list_lengths_at_the_edges_of_the_register_sort(orc, H, P, order):
 @pytest.mark.parametrize("longest,bound,ahead", [(2048, 4096, True), (2049, 4096, True), (4096, 4096, True),
                                                  (4097, 4096, False), (4097, 4097, True), (4097, 0, True)])
 def test_launching_ahead_with_a_bound_on_the_longest_list(orc, H, longest, bound, ahead):
-    """A view launched ahead with a bound that the radix sort's smaller kernel covers does without the larger one; where
-    a list is longer than the bound after all, the lists are built again.  One tile, whose list is the longest."""
+    """A view launched ahead with a bound that the register sort covers does without the radix sort; where a list is
+    longer than the bound after all, the lists are built again.  One tile, whose list is the longest."""
     import gsrast_native as gn
     from diff_gaussian_rasterization import _C
     gen = torch.Generator().manual_seed(longest)
