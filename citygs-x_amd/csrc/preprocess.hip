@@ -680,7 +680,12 @@ mark_visible_kernel(int P, const float* __restrict__ means, const float* __restr
 // Gaussians, a quarter of them visible, 639 us (3.6 GB) against 677 with each load where its value is used and each lane
 // storing its own rows; 4 M 276 against 291, 1 M 73 against 77.  (Fetching the rows through LDS as well costs what it
 // gains, with and without non-temporal loads.)
-template <bool SAVED, bool MAP>
+// FIRST: the screen gradient is among those loads and nothing is stored before them, instead of being asked for where it is
+// used, with the opacities' gradients stored at the start.  Better where the arrays are small or no coefficients' gradients
+// are written (6 M, colours given: 140 us, 172 without), worse beyond: 1 M 64.3 against 65.7 (with the channels' gradient
+// 66.6, 69.2), 2 M 120 and 120 (125, 128), 3 M 178 and 176 (188, 189), 4 M 238 and 232 (249, 248), 10 M at street level 608
+// and 586 (629, 618).
+template <bool SAVED, bool MAP, bool FIRST>
 __global__ void __launch_bounds__(GS_BLOCK_1D)
 preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, const int* __restrict__ radii,
                       const float* __restrict__ shs, const uint8_t* __restrict__ clamped,
@@ -703,6 +708,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   const bool sh_mode = (SAVED || shs != nullptr) && M > 0 && (dL_dsh != nullptr);
   const bool sh_staged = sh_mode && M == 16;  // coefficient rows and their gradients go through LDS
   const float4 gco = dL_dconic_opacity[i];
+  if (!FIRST && dL_dopacity && in_range) dL_dopacity[i] = gco.w;  // passthrough, rasterize_points.cu:191-194
   float gm[3] = {0.f, 0.f, 0.f}, gs_[3] = {0.f, 0.f, 0.f}, gq[4] = {0.f, 0.f, 0.f, 0.f};
   float gc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const bool live = in_range && radii[i] > 0;
@@ -716,7 +722,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   // (zero for a Gaussian no pixel blended, culled ones first of all)
   const bool map_live = MAP && !(map_g[0] == 0.f && map_g[1] == 0.f && map_g[2] == 0.f && map_g[3] == 0.f);
   // Everything the two parts below take of a Gaussian is asked for at once: one latency for all of it, and a line that
-  // several loads share is still there.  Nothing is stored before: a load behind a store waits for the store as well.
+  // several loads share is still there.  (A load behind a store waits for the store as well.)
   float mean[3] = {0.f, 0.f, 0.f}, sc[3] = {0.f, 0.f, 0.f}, gcol[3] = {0.f, 0.f, 0.f}, dd[9], g2x = 0.f, g2y = 0.f;
   uint8_t was_clamped[3] = {0, 0, 0};
   float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -729,7 +735,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
       q4 = reinterpret_cast<const float4*>(rots)[i];
     }
   }
-  if (live) {
+  if (FIRST && live) {
     g2x = dL_dmean2D[(size_t)mean2D_stride * i];
     g2y = dL_dmean2D[(size_t)mean2D_stride * i + 1];
   }
@@ -866,6 +872,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
     const float m_w = 1.0f / (mh[3] + 0.0000001f);
     const float mul1 = (((PM[0] * mean[0] + PM[4] * mean[1]) + PM[8] * mean[2]) + PM[12]) * m_w * m_w;
     const float mul2 = (((PM[1] * mean[0] + PM[5] * mean[1]) + PM[9] * mean[2]) + PM[13]) * m_w * m_w;
+    if (!FIRST) g2x = dL_dmean2D[(size_t)mean2D_stride * i], g2y = dL_dmean2D[(size_t)mean2D_stride * i + 1];
     gm[0] += (PM[0] * m_w - PM[3] * mul1) * g2x + (PM[1] * m_w - PM[3] * mul2) * g2y;
     gm[1] += (PM[4] * m_w - PM[7] * mul1) * g2x + (PM[5] * m_w - PM[7] * mul2) * g2y;
     gm[2] += (PM[8] * m_w - PM[11] * mul1) * g2x + (PM[9] * m_w - PM[11] * mul2) * g2y;
@@ -988,7 +995,7 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   wave_rows_turn_store<3>(dL_dmean3D + 3 * wave_first, rows, gm, lds, lane);
   if (dL_dscale) wave_rows_turn_store<3>(dL_dscale + 3 * wave_first, rows, gs_, lds, lane);
   if (!in_range) return;
-  if (dL_dopacity) dL_dopacity[i] = gco.w;  // passthrough, rasterize_points.cu:191-194
+  if (FIRST && dL_dopacity) dL_dopacity[i] = gco.w;  // passthrough, rasterize_points.cu:191-194
   if (dL_drot) reinterpret_cast<float4*>(dL_drot)[i] = make_float4(gq[0], gq[1], gq[2], gq[3]);
   if (dL_dcov3D_out) {
 #pragma unroll
@@ -1061,12 +1068,15 @@ int launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t stream) {
                        (const float4*)a.dL_dconic_opacity, a.dL_dcolor, a.dL_dmean3D, a.dL_dcov3D, a.dL_dsh,
                        a.dL_dscale, a.dL_drot, a.dL_dopacity, a.dcolor_ddir, a.dL_dall_map);
   };
+  // (see FIRST at the kernel)
   if (a.dL_dall_map != nullptr) {
-    if (a.dcolor_ddir != nullptr) go(preprocess_bwd_kernel<true, true>);
-    else go(preprocess_bwd_kernel<false, true>);
+    if (a.dcolor_ddir == nullptr) go(preprocess_bwd_kernel<false, true, true>);
+    else if (a.P <= 4 << 20) go(preprocess_bwd_kernel<true, true, true>);
+    else go(preprocess_bwd_kernel<true, true, false>);
   } else {
-    if (a.dcolor_ddir != nullptr) go(preprocess_bwd_kernel<true, false>);
-    else go(preprocess_bwd_kernel<false, false>);
+    if (a.dcolor_ddir == nullptr) go(preprocess_bwd_kernel<false, false, true>);
+    else if (a.P <= 2 << 20) go(preprocess_bwd_kernel<true, false, true>);
+    else go(preprocess_bwd_kernel<true, false, false>);
   }
   return 0;
 }

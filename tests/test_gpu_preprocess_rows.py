@@ -44,3 +44,40 @@ def test_colours_and_flags(orc, P, shift, records):
         r = n(rec)[ok]
         assert np.array_equal(r[:, :2], want["means2D"][ok]) and np.array_equal(r[:, 2:6], want["conic_opacity"][ok])
         assert np.array_equal(r[:, 6:9], want["rgb"][ok]) and np.array_equal(r[:, 14], want["depths"][ok])
+
+
+@pytest.mark.parametrize("P,channels", [((2 << 20) + 77, False), ((4 << 20) + 77, True)])
+def test_backward_of_many_gaussians(P, channels):
+    """The backward kernel for large steps against the one for small ones, bit for bit: a Gaussian's gradients do not depend
+    on the others, so the step in parts gives the same."""
+    import gs_scenes
+    from diff_gaussian_rasterization import _C
+    _, cams = gs_scenes.make_scene(0, P=8, n_views=1)
+    cam = cams[0]
+    W, Hh = cam.image_width, cam.image_height
+    gen = torch.Generator(device=DEV).manual_seed(P)
+    n = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    means, scales, rots = n(P, 3) * 6, torch.exp(n(P, 3) * 0.5 - 4), torch.nn.functional.normalize(n(P, 4))
+    sh, op = n(P, 16, 3) * 0.3, torch.sigmoid(n(P, 1))
+    view = [t.to(DEV) for t in (cam.world_view_transform, cam.full_proj_transform, cam.camera_center)]
+    args = {"stats_collector": {}}
+    (_, _, _, radii, _, _, _, clamped), ddir = _C.preprocess_gaussians_ex(
+        means, scales, rots, sh, op, 1.0, view[0], view[1], cam.tanfovx, cam.tanfovy, Hh, W, 3, view[2], False, False, args,
+        want_direction_derivative=True, want_cov3D=False)
+    live = int((radii > 0).sum())
+    assert 0 < live < P and bool(clamped.bool().any())
+    up = [n(P, 2), n(P, 4), n(P, 3)]
+    am = n(P, 5) if channels else None
+    if channels:
+        am[::3] = 0.0
+
+    def backward(a, b):
+        return _C.preprocess_gaussians_backward(
+            radii[a:b].contiguous(), None, clamped[a:b].contiguous(), means[a:b], scales[a:b], rots[a:b], sh[a:b], 1.0,
+            view[0], view[1], cam.tanfovx, cam.tanfovy, Hh, W, 3, view[2], up[0][a:b], up[1][a:b], up[2][a:b], live, False,
+            args, dcolor_ddir=ddir[a:b].contiguous(), dL_dall_map=None if am is None else am[a:b])
+
+    whole = backward(0, P)
+    for a, b in ((0, P // 2 + 3), (P // 2 + 3, P)):
+        for k, (w, part) in enumerate(zip(whole, backward(a, b))):
+            assert torch.equal(w[a:b], part), k
