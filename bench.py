@@ -62,7 +62,7 @@ BINNING_STAGES = ("tile_count", "inclusive_sum", "bucket_scatter", "tile_sort", 
                   "identify_tile_ranges")
 BINNING_KERNELS = ("bucket_count_kernel", "bucket_columns_kernel", "bucket_ranges_kernel",
                    "bucket_scatter_staged_kernel",  # (bucket_scatter_kernel beyond one round per workgroup)
-                   "tile_sort_registers_kernel")  # (views with lists above 2048 records: + tile_radix_sort_kernel)
+                   "tile_sort_registers_kernel")  # (views with lists above 4096 records: + tile_radix_sort_kernel)
 FP32_MATRIX_PEAK_TFLOPS = 157.3
 # Neural-Gaussian generation with 10 offsets: (bytes per anchor, bytes per selected Gaussian, flops per anchor).
 #   opacity:   feat 128 + anchor 12 in; 10 opacities, 10 mask bytes, 1 count out;      2 (35*32 + 32*10) flops

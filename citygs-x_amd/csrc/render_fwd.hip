@@ -32,10 +32,10 @@
 //
 // A tile's workgroup takes some 31 ns an entry whatever else the chip does: the chain of its waves' own instructions.  A
 // view whose lists differ much in length ended on a few such chains (4 M Gaussians from the air, lists up to 9600: 293 us,
-// in the last 150 of which less than a quarter of the chip had work; wave priorities change nothing).  Long tiles therefore
-// go to four workgroups, one per quadrant, whose waves have 16 pixels instead of 64 and four lanes for each
+// in the last 150 of which less than a quarter of the chip had work; wave priorities change nothing).  Long tiles (which:
+// GS_LONG_TILE) therefore go to four workgroups, one per quadrant, whose waves have 16 pixels instead of 64 and four lanes for each
 // (blend_quadrant): 4.4 us per 256 entries instead of 8, for about 1.45 times the instructions of a tile.
-// 4 M, 1152x864: 263 -> 201 us; 20 M from 600 m, lists up to 69 000, of which 0.4 is walked: 648 -> 415.
+// 4 M, 1152x864: 263 -> 196 us; 20 M from 600 m, lists up to 69 000, of which 0.4 is walked: 643 -> 408.
 //
 // The per-pixel arithmetic keeps a fixed operation order, so contributor
 // counts and images match a CPU evaluation bit for bit; exp() is gs_expf.

@@ -581,8 +581,9 @@ bucket_scatter_staged_kernel(int P, int per_block, int nblocks, uint32_t gx, uin
 // lane for 2048 records, not four with eight).  Lists of 2049 to 4096 records take eight, so that a view without longer
 // ones needs no further launch and the others have these lists under way beside the shorter: with a radix sort in a
 // launch of its own for them (tile_radix.hip, which is left with what a caller's options put between the limits) the two
-// kernels took 25.0 + 27.8 us for 20 M Gaussians from 600 m, 22.8 + 25.8 for 4 M from the air, 18.7 + 22.0 at street level
-// and, with hardly such a list, 22.6 + 4.7 for 1 M; this one takes 42.2, 44.4, 39.9 and 23.9.
+// kernels took 25.0 + 27.8 us for 20 M Gaussians from 600 m, 22.8 + 25.8 for 4 M from the air, 21.2 + 30.6 and 28.5 + 30.5 in
+// two views at street level and, with hardly such a list, 22.6 + 4.7 for 1 M; this one takes 43.2, 45.3, 56.8 and 56.8, and
+// 24.1.
 //
 // The key is one 32-bit word: (depth bits - smallest depth bits of the list) >> shift in the high bits, the
 // record's place in the unsorted segment in the low log2(64 E W) bits; shift is what it takes to fit the list's
