@@ -601,14 +601,18 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   }
   if (check_launch("inclusive_sum", stream, dbg)) return 1;
   // The blend kernels (this call's and the backward call's) can fetch a Gaussian's operands as one 64-byte record
-  // instead of gathering parts of five lines of memory.  Packing the records costs about 20 us per million
-  // Gaussians and saves about 25 us per million instances: done for a view with enough instances per Gaussian.
-  // The library's own records live at the end of the binning buffer, which is sized once the decision is made.
-  bool use_packed = false, pack_decided = false;
-  auto decide_packing = [&](int64_t instances) {
-    if (pack_decided) return;
-    pack_decided = true;
-    use_packed = caller_records != nullptr || instances * 5 > (int64_t)P * 4;
+  // instead of gathering parts of five lines of memory.  Packing the records costs 4 to 8 us per million Gaussians and
+  // about 15 more per million of them that are in view; what it saves depends on the lists.  Over 36 views (forward and
+  // backward, us, packed less gathered): with lists beyond the register sort's, whose tiles end the view and are split only
+  // with records, 0.62 instances per Gaussian 220 saved of 2056, 0.74 298 of 2420, 0.75 215 of 1553 and, at 320x240, 499 of
+  // 2667, but 0.28 instances 20 lost of 1056; without such lists 1.5 to 2.4 instances 13 saved of 260, 0.98 14 of 501, 0.33
+  // 7 lost of 402.  The library's own records live at the end of the binning buffer, which is sized once the decision is
+  // made.  A view that was launched ahead without records and did not fit is looked at again with its own figures (its
+  // buffer is another one); one that was launched with them keeps them, since the word that says so is set.
+  bool use_packed = caller_records != nullptr;
+  auto decide_packing = [&](int64_t instances, uint32_t longest_list) {
+    const bool long_lists = bucketed && longest_list > (uint32_t)TILE_SORT_SMALL;
+    if (instances * 5 > (int64_t)P * (long_lists ? 2 : 4)) use_packed = true;
   };
 
   EventTimer timer;
@@ -696,7 +700,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   Arrays A;
   if (ahead) {
     // (on the expected count less a fifth: the caller's expectation carries a margin of a quarter)
-    decide_packing(cap_n - cap_n / 5);
+    decide_packing(cap_n - cap_n / 5, cap_longest);
     if (carve(cap_n, A)) return 1;
     if (timer.begin(elapsed_ms != nullptr, stream)) return 1;
     if (pack_records(A)) return 1;
@@ -743,7 +747,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
 
   // The ordinary way (also after kernels launched ahead found that the view does not fit and did nothing).
   // (after kernels launched ahead: the records are packed again, the buffer may be another one)
-  decide_packing(R);
+  decide_packing(R, longest);
   if (carve(R, A)) return 1;
   if (!ahead && timer.begin(elapsed_ms != nullptr, stream)) return 1;
   if (pack_records(A)) return 1;

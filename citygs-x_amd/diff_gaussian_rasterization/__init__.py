@@ -151,12 +151,12 @@ def _have_versions(sources):
 
 
 def _records_wanted(rs, P, device):
-    """Whether preprocess should write the records: the last view of this image size had enough instances per
+    """Whether preprocess should write the records: one of the last views of this image size had enough instances per
     Gaussian for records to pay (written on the way they cost about a third of the library's packing pass, which
     pays from 0.8 instances per Gaussian), and render_gaussians will be able to use them (no geometry channels to
     render, or the caller builds them through build_all_map(..., blend_records_of=means2D))."""
     seen = _expectations.get((rs.image_height, rs.image_width, device))
-    if seen is None or seen[0] * 10 <= P * 3:
+    if seen is None or _most_instances(seen) * 10 <= P * 3:
         return False
     return (not rs.render_geo) or _linked_all_map_seen[0]
 
@@ -233,25 +233,34 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_setti
 
 # ------------------------------------------------------------------- render --
 
-# What the last view of a given image size needed, (instances, longest list, whether any view of the size had a list
-# beyond _LONG_LIST) keyed by (height, width, device): the
-# next view of that size is launched without waiting for its instance count, on buffers sized for these figures plus
+# What the last views of a given image size needed, (instances, longest list, whether any view of the size had a list
+# beyond _LONG_LIST, the instances of the _RECENT_VIEWS last ones) keyed by (height, width, device): the
+# next view of that size is launched without waiting for its instance count, on buffers sized for the most instances of
+# those views and the longest list of the last one plus
 # a margin (a training loop renders thousands of similar views; the number of Gaussians changes at every
-# densification, so it is not part of the key).  Only the time depends on it, never a result; a stale or missing
+# densification, so it is not part of the key).  A scene's cameras differ by more than the margin: in a loop over views of
+# 6.2 M and 2.7 M instances every view of the larger kind missed an expectation taken from the view before it.
+# Only the time depends on it, never a result; a stale or missing
 # entry costs one ordinary call.  A handful of image sizes at most are alive in a run: the oldest entry goes
 # when there are more than _MAX_EXPECTATIONS.
 _expectations = {}
 _MARGIN = 1.25
 _MAX_EXPECTATIONS = 16
+_RECENT_VIEWS = 8
 _LONG_LIST = 4096  # the longest list that is sorted in registers
 _LONG_TILE = 3072  # a list from which on the forward blend splits its tile
+
+
+def _most_instances(seen):
+    """Of the last views that an entry of _expectations tells of."""
+    return max(seen[0], *seen[3]) if len(seen) > 3 else seen[0]
 
 
 def _expectation(key):
     seen = _expectations.get(key)
     if seen is None:
         return 0, 0
-    instances, longest, *long = seen
+    longest, long = seen[1], seen[2:3]
     if longest <= 0:
         return 0, 0  # a view without per-tile lists (a tile grid too large for them): nothing to gain
     # whole variants of the register sort (256 ... 4096 records per list), so that a slightly longer list still fits; beyond
@@ -261,7 +270,7 @@ def _expectation(key):
     cap = 256
     while cap < longest * _MARGIN:
         cap *= 2
-    return int(instances * _MARGIN) + 65536, (0 if cap > _LONG_LIST or (cap == _LONG_LIST and any(long)) else cap)
+    return int(_most_instances(seen) * _MARGIN) + 65536, (0 if cap > _LONG_LIST or (cap == _LONG_LIST and any(long)) else cap)
 
 
 def _launch_bounds(key):
@@ -276,7 +285,8 @@ def _launch_bounds(key):
 
 def _remember(key, instances, longest):
     seen = _expectations.pop(key, ())  # (re-inserted at the end: the dict keeps insertion order)
-    _expectations[key] = (instances, longest, longest > _LONG_LIST or any(seen[2:]))
+    recent = (instances, *(seen[3] if len(seen) > 3 else seen[:1]))[:_RECENT_VIEWS]
+    _expectations[key] = (instances, longest, longest > _LONG_LIST or any(seen[2:3]), recent)
     while len(_expectations) > _MAX_EXPECTATIONS:
         # (a copy to look at: another thread may be adding entries, or have removed this one)
         _expectations.pop(list(_expectations)[0], None)

@@ -380,3 +380,22 @@ def test_bound_that_leaves_no_tile_to_split():
     finally:
         dgr._expectations.clear()
         dgr._expectations.update(saved)
+
+
+def test_expected_instances_are_those_of_the_fullest_of_the_last_views():
+    import diff_gaussian_rasterization as dgr
+    saved = dict(dgr._expectations)
+    dgr._expectations.clear()
+    try:
+        room = lambda n: int(n * dgr._MARGIN) + 65536
+        for n, most in ((1000, 1000), (500, 1000), (3000, 3000), *[(700, 3000)] * 7, (700, 700), (0, 700)):
+            dgr._remember("size", n, 100)
+            assert dgr._expectation("size") == (room(most), 256)
+            assert dgr._expectations["size"][:3] == (n, 100, False)
+        dgr._expectations["size"] = (2000, 100, False)  # (an entry without the views before)
+        assert dgr._expectation("size")[0] == room(2000)
+        dgr._remember("size", 900, 100)
+        assert dgr._expectation("size")[0] == room(2000)
+    finally:
+        dgr._expectations.clear()
+        dgr._expectations.update(saved)
