@@ -55,12 +55,18 @@ train_stats_kernel(IDX slots, int k, IDX Vk, IDX M, const uint8_t* __restrict__ 
 
 // ---- n_offsets <= STATS_MAX_OFFSETS
 
-constexpr int STATS_ROWS = 256;         // anchors per workgroup, one thread each for the visibility mask
-constexpr int STATS_SEL_CHUNK = 1024;   // candidates per prefix of the selection mask
-constexpr int STATS_ITEMS = 4;          // candidates per thread and round
-constexpr int STATS_ROUND = GS_BLOCK_1D * STATS_ITEMS;
+constexpr uint32_t STATS_ROWS = 256;          // anchors per workgroup, one thread each for the visibility mask
+constexpr uint32_t STATS_SEL_CHUNK = 1024;    // candidates per prefix of the selection mask
+constexpr uint32_t STATS_ITEMS = 5;           // candidates per thread and round
+constexpr uint32_t STATS_ROUND = GS_BLOCK_1D * STATS_ITEMS;
 constexpr int STATS_MAX_OFFSETS = 256;
-static_assert(STATS_ROWS == GS_BLOCK_1D && STATS_SEL_CHUNK == 16 * GS_WAVE, "a wave counts 1024 entries, 16 a lane");
+constexpr uint32_t STATS_COUNT_THREADS = 1024;
+constexpr uint32_t STATS_SPAN = STATS_COUNT_THREADS * 16;  // mask entries per counting workgroup, 16 a thread
+// Spans, of either mask, beyond which their totals are turned into prefixes by a launch of their own (4 us and its gap):
+// up to here a thread adds up two of them at the most.
+constexpr uint32_t STATS_SPANS = 512;
+static_assert(STATS_ROWS == GS_BLOCK_1D && STATS_MAX_OFFSETS <= STATS_ROUND, "a round holds whole anchors");
+static_assert(STATS_SPAN % STATS_ROWS == 0 && STATS_SPAN % STATS_SEL_CHUNK == 0, "whole chunks");
 
 __device__ __forceinline__ uint32_t nonzero_bytes(uint32_t x) {
   return (uint32_t)__popc((x | ((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu)) & 0x80808080u);
@@ -77,35 +83,45 @@ __device__ __forceinline__ uint32_t count16(const uint8_t* __restrict__ mask, ui
   return c;
 }
 
-// Set entries per STATS_ROWS anchors of the visibility mask and per STATS_SEL_CHUNK candidates of the selection mask;
-// a wave looks at 1024 entries of one of them.
-__global__ void __launch_bounds__(GS_BLOCK_1D)
-train_stats_count_kernel(uint32_t A, uint32_t Vk, uint32_t vis_waves, uint32_t waves, const uint8_t* __restrict__ visible,
-                         const uint8_t* __restrict__ selected, uint32_t* __restrict__ vis_counts,
-                         uint32_t* __restrict__ sel_counts) {
-  const uint32_t w = blockIdx.x * (GS_BLOCK_1D / GS_WAVE) + threadIdx.x / GS_WAVE;
-  if (w >= waves) return;
-  const uint32_t lane = threadIdx.x & (GS_WAVE - 1);
-  const bool first_mask = w < vis_waves;
-  const uint32_t start = (first_mask ? w : w - vis_waves) * 1024u, n = first_mask ? A : Vk;
-  uint32_t c = count16(first_mask ? visible : selected, start + 16 * lane, n);
-#pragma unroll
-  for (int d = 1; d < 16; d <<= 1) c += __shfl_xor(c, d, GS_WAVE);
-  if (first_mask) {
-    const uint32_t chunk = start / STATS_ROWS + lane / 16;
-    if (lane % 16 == 0 && start + 16 * lane < A) vis_counts[chunk] = c;
-  } else {
-    c += __shfl_xor(c, 16, GS_WAVE);
-    c += __shfl_xor(c, 32, GS_WAVE);
-    if (lane == 0) sel_counts[start / STATS_SEL_CHUNK] = c;
-  }
+// The set entries of a span of one of the masks (the first vis_spans workgroups: visibility): the total of the span, and
+// before every STATS_ROWS anchors or STATS_SEL_CHUNK candidates of it those that the span has before them.
+__global__ void __launch_bounds__(STATS_COUNT_THREADS)
+train_stats_count_kernel(uint32_t A, uint32_t Vk, uint32_t vis_spans, const uint8_t* __restrict__ visible,
+                         const uint8_t* __restrict__ selected, uint32_t* __restrict__ vis_prefix,
+                         uint32_t* __restrict__ sel_prefix, uint32_t* __restrict__ vis_totals,
+                         uint32_t* __restrict__ sel_totals) {
+  __shared__ uint32_t s_wave[STATS_COUNT_THREADS / GS_WAVE];
+  const bool first_mask = blockIdx.x < vis_spans;
+  const uint32_t span = first_mask ? blockIdx.x : blockIdx.x - vis_spans, n = first_mask ? A : Vk;
+  const uint32_t at = span * STATS_SPAN + 16 * threadIdx.x;
+  const uint32_t c = count16(first_mask ? visible : selected, at, n);
+  uint32_t total;
+  const uint32_t before = block_exclusive_scan<STATS_COUNT_THREADS>(c, s_wave, total);
+  const uint32_t chunk = first_mask ? STATS_ROWS : STATS_SEL_CHUNK;
+  if (at % chunk == 0 && at < n) (first_mask ? vis_prefix : sel_prefix)[at / chunk] = before;
+  if (threadIdx.x == 0) (first_mask ? vis_totals : sel_totals)[span] = total;
 }
 
+// The totals of the spans as prefixes, where a wave would have to add up too many of them.
 __global__ void __launch_bounds__(1024)
-train_stats_spine_kernel(uint32_t vis_chunks, uint32_t sel_chunks, uint32_t* vis_counts, uint32_t* sel_counts) {
+train_stats_spine_kernel(uint32_t vis_spans, uint32_t sel_spans, uint32_t* vis_totals, uint32_t* sel_totals) {
   __shared__ uint32_t s_wave[1024 / GS_WAVE];
-  if (blockIdx.x == 0) exclusive_prefix_in_place(vis_chunks, vis_counts, s_wave);
-  else exclusive_prefix_in_place(sel_chunks, sel_counts, s_wave);
+  if (blockIdx.x == 0) exclusive_prefix_in_place(vis_spans, vis_totals, s_wave);
+  else exclusive_prefix_in_place(sel_spans, sel_totals, s_wave);
+}
+
+// A thread's share of the set entries in the spans before this one.
+__device__ __forceinline__ uint32_t before_span(const uint32_t* __restrict__ totals, uint32_t span, bool prefixes) {
+  if (prefixes) return threadIdx.x == 0 ? totals[span] : 0u;
+  uint32_t sum = 0;
+  for (uint32_t s = threadIdx.x; s < span; s += GS_BLOCK_1D) sum += totals[s];
+  return sum;
+}
+
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+#pragma unroll
+  for (int d = 1; d < GS_WAVE; d <<= 1) v += __shfl_xor(v, d, GS_WAVE);
+  return v;
 }
 
 // A workgroup owns STATS_ROWS consecutive anchors.  Its visible ones are listed in LDS; their candidates are one run
@@ -114,29 +130,41 @@ train_stats_spine_kernel(uint32_t vis_chunks, uint32_t sel_chunks, uint32_t* vis
 // all of a thread's loads in flight at once.  The anchor's opacities are added from LDS in candidate order.
 // Bound by memory, most of it the lines of the two slot accumulators.  With the ranks written out by two scans and
 // one slot per thread, each waiting for six loads one after the other, the call took 139 us at 1 M anchors of 10
-// offsets (40 % visible, 60 % of those selected), 59 us now (33 with 5 offsets).  Eight candidates a thread, whose
-// registers leave five waves a SIMD, take 70 (42), six 68 (39), five 63 (36), three and two the same as four.  (The
-// accumulators asked for with the masks, before it is known which slots are hit: 60.)
-__global__ void __launch_bounds__(GS_BLOCK_1D)
-train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, uint32_t M,
+// offsets (40 % visible, 60 % of those selected).  Six sets of inputs in turn, with the spans' totals turned into prefixes
+// by a launch of its own and four candidates a thread -> now: 62 -> 59 us, 5 offsets 42 -> 40, 2 M anchors 111 -> 108,
+// 200 k 27 -> 24.  Five candidates are what eight waves a SIMD have registers for (slots in 32 bits): with six and five
+// waves 53 us where five take 48 and four 50.  Not kept: a wave for every 64 anchors, without barriers (50 us for this
+// kernel's 44); the accumulators asked for with the masks, before it is known which slots are hit (59 -> 63); gradients
+// and opacities past the caches (60); the workgroups of one XCD on neighbouring anchors (60).
+__global__ void __launch_bounds__(GS_BLOCK_1D) __attribute__((amdgpu_waves_per_eu(8)))
+train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, uint32_t M, bool prefixes,
                          const uint8_t* __restrict__ visible, const uint32_t* __restrict__ vis_prefix,
-                         const uint8_t* __restrict__ selected, const uint32_t* __restrict__ sel_prefix,
+                         const uint32_t* __restrict__ vis_totals, const uint8_t* __restrict__ selected,
+                         const uint32_t* __restrict__ sel_prefix, const uint32_t* __restrict__ sel_totals,
                          const uint8_t* __restrict__ update_filter, const float* __restrict__ grad, int grad_stride,
                          const float* __restrict__ opacity, float* __restrict__ opacity_accum,
                          float* __restrict__ anchor_demon, float* __restrict__ grad_accum, float* __restrict__ denom) {
   constexpr int WAVES = GS_BLOCK_1D / GS_WAVE;
   __shared__ float s_op[STATS_ROUND];
   __shared__ uint32_t s_row[STATS_ROWS];
-  __shared__ uint32_t s_count[WAVES];
+  __shared__ uint32_t s_count[WAVES], s_before[WAVES];
   __shared__ uint32_t s_sel[STATS_ITEMS][WAVES];
   const uint32_t tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   const uint64_t below = (1ull << lane) - 1ull;
   const uint32_t row0 = blockIdx.x * STATS_ROWS;
-  const uint32_t vis0 = vis_prefix[blockIdx.x];
+  const uint32_t vis_before = wave_sum(before_span(vis_totals, row0 / STATS_SPAN, prefixes));
+  uint32_t vis0 = vis_prefix[blockIdx.x];
   const bool set = row0 + tid < A && visible[row0 + tid] != 0;
   const uint64_t vm = gs_ballot(set);
-  if (lane == 0) s_count[wave] = (uint32_t)__popcll(vm);
-  // the rank of the chunk's first candidate: the prefix of its selection chunk and what is set before it there
+  if (lane == 0) {
+    s_count[wave] = (uint32_t)__popcll(vm);
+    s_before[wave] = vis_before;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t w = 0; w < WAVES; w++) vis0 += s_before[w];
+  // the rank of the chunk's first candidate: what is set in the spans before, in
+  // the chunks of its span before, and before it in its chunk
   const uint64_t first64 = (uint64_t)vis0 * k;
   const uint32_t first = first64 < Vk ? (uint32_t)first64 : Vk;
   const uint32_t sel_chunk = first / STATS_SEL_CHUNK;
@@ -146,6 +174,7 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
     const uint32_t e = sel_chunk * STATS_SEL_CHUNK + q * GS_BLOCK_1D + tid;
     head += (uint32_t)__popcll(gs_ballot(e < first && selected[e] != 0));
   }
+  if (first < Vk) head += wave_sum(before_span(sel_totals, first / STATS_SPAN, prefixes));
   if (lane == 0) s_sel[0][wave] = head;
   __syncthreads();
   uint32_t rank0 = first < Vk ? sel_prefix[sel_chunk] : 0u;  // (no candidates left: never used)
@@ -162,13 +191,15 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
   const uint32_t rows_per_round = STATS_ROUND / k;  // (at least 4)
   for (uint32_t r0 = 0; r0 < rows; r0 += rows_per_round) {
     const uint32_t nr = min(rows_per_round, rows - r0), n = nr * k;
-    const uint64_t c0 = ((uint64_t)vis0 + r0) * k;  // the round's first candidate
+    // the round's first candidate, and how many of the round's there are
+    const uint64_t c64 = ((uint64_t)vis0 + r0) * k;
+    const uint32_t c0 = c64 < Vk ? (uint32_t)c64 : Vk, have_n = min(n, Vk - c0);
     bool sel[STATS_ITEMS];
     float op[STATS_ITEMS];
 #pragma unroll
     for (uint32_t q = 0; q < STATS_ITEMS; q++) {
       const uint32_t c = q * GS_BLOCK_1D + tid;
-      const bool have = c < n && c0 + c < Vk;
+      const bool have = c < have_n;
       sel[q] = have && selected[c0 + c] != 0;
       op[q] = have ? opacity[c0 + c] : 0.f;
     }
@@ -191,7 +222,7 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
     }
     bool hit[STATS_ITEMS];
     float gx[STATS_ITEMS], gy[STATS_ITEMS], acc[STATS_ITEMS], den[STATS_ITEMS];
-    size_t slot[STATS_ITEMS];
+    uint32_t slot[STATS_ITEMS];
 #pragma unroll
     for (uint32_t q = 0; q < STATS_ITEMS; q++) {
       hit[q] = sel[q] && rank[q] < M;
@@ -209,7 +240,7 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
       acc[q] = den[q] = 0.f;
       slot[q] = 0;
       if (hit[q]) {
-        slot[q] = (size_t)s_row[r0 + r] * k + (c - r * k);
+        slot[q] = s_row[r0 + r] * k + (c - r * k);
         acc[q] = grad_accum[slot[q]];
         den[q] = denom[slot[q]];
       }
@@ -265,20 +296,25 @@ int launch_train_stats(long long A, int k, long long Vk, long long M, const uint
   const long long slots = A * k;
   if (k <= STATS_MAX_OFFSETS && slots < 0x7FFFFFFFll && Vk < 0x7FFFFFFFll && M < 0x7FFFFFFFll) {
     const uint32_t vis_chunks = (uint32_t)((A + STATS_ROWS - 1) / STATS_ROWS);
-    const uint32_t sel_chunks = (uint32_t)((Vk + STATS_SEL_CHUNK - 1) / STATS_SEL_CHUNK);
-    const uint32_t vis_waves = (uint32_t)((A + 1023) / 1024), waves = vis_waves + sel_chunks;
-    const uint32_t per_block = GS_BLOCK_1D / GS_WAVE;
-    // (prefixes a chunk: less than the ranks, an entry each, that the space is sized for)
-    uint32_t* vis_counts = (uint32_t*)temp;
-    uint32_t* sel_counts = (uint32_t*)((char*)temp + align_up((size_t)A * 4, 256));
-    hipLaunchKernelGGL(train_stats_count_kernel, dim3((waves + per_block - 1) / per_block), dim3(GS_BLOCK_1D), 0, stream,
-                       (uint32_t)A, (uint32_t)Vk, vis_waves, waves, visible, selected, vis_counts, sel_counts);
-    hipLaunchKernelGGL(train_stats_spine_kernel, dim3(2), dim3(1024), 0, stream, vis_chunks, sel_chunks, vis_counts,
-                       sel_counts);
-    hipLaunchKernelGGL(train_stats_chunk_kernel, dim3(vis_chunks), dim3(GS_BLOCK_1D), 0, stream, (uint32_t)A,
-                       (uint32_t)k, (uint32_t)(((1ull << 32) + k - 1) / k), (uint32_t)Vk, (uint32_t)M, visible,
-                       vis_counts, selected, sel_counts, update_filter, grad, grad_stride, opacity, opacity_accum,
-                       anchor_demon, grad_accum, denom);
+    const uint32_t vis_spans = (uint32_t)((A + STATS_SPAN - 1) / STATS_SPAN);
+    const uint32_t sel_spans = (uint32_t)((Vk + STATS_SPAN - 1) / STATS_SPAN);
+    // (a prefix per chunk and a total per span: less than the ranks, an entry each, that the space is sized for, a total
+    // beside fewer prefixes than there are entries at least)
+    uint32_t* vis_prefix = (uint32_t*)temp;
+    uint32_t* vis_totals = vis_prefix + vis_chunks;
+    uint32_t* sel_prefix = (uint32_t*)((char*)temp + align_up((size_t)A * 4, 256));
+    uint32_t* sel_totals = sel_prefix + (Vk + STATS_SEL_CHUNK - 1) / STATS_SEL_CHUNK;
+    const bool prefixes = vis_spans > STATS_SPANS || sel_spans > STATS_SPANS;
+    hipLaunchKernelGGL(train_stats_count_kernel, dim3(vis_spans + sel_spans), dim3(STATS_COUNT_THREADS), 0, stream,
+                       (uint32_t)A, (uint32_t)Vk, vis_spans, visible, selected, vis_prefix, sel_prefix, vis_totals,
+                       sel_totals);
+    if (prefixes)
+      hipLaunchKernelGGL(train_stats_spine_kernel, dim3(2), dim3(1024), 0, stream, vis_spans, sel_spans, vis_totals,
+                         sel_totals);
+    hipLaunchKernelGGL(train_stats_chunk_kernel, dim3(vis_chunks), dim3(GS_BLOCK_1D), 0, stream, (uint32_t)A, (uint32_t)k,
+                       (uint32_t)(((1ull << 32) + k - 1) / k), (uint32_t)Vk, (uint32_t)M, prefixes, visible, vis_prefix,
+                       vis_totals, selected, sel_prefix, sel_totals, update_filter, grad, grad_stride, opacity,
+                       opacity_accum, anchor_demon, grad_accum, denom);
     return 0;
   }
   char* base = (char*)temp;

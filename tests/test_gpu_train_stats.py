@@ -118,3 +118,19 @@ def test_training_stats_chunk_edges(orc, A, k, p, offset):
                                shifted(vis))
     for got, want in zip(d, ref):
         assert np.abs(got.cpu().numpy().ravel() - want).max() <= 1e-6 * max(1.0, np.abs(want).max())
+
+
+# spans of 16384 mask entries: on either side of one, of their number that a thread adds up by itself, and beyond
+@pytest.mark.parametrize("A,k,p", [(16384, 1, (1.0, 0.5, 0.9)), (16385, 3, (1.0, 1.0, 0.9)), (33_000, 10, (0.99, 0.6, 0.9)),
+                                   (512 * 16384, 1, (1.0, 0.6, 0.9)), (512 * 16384 + 1, 1, (0.5, 0.6, 0.9)),
+                                   (900_000, 10, (0.95, 0.6, 0.9))])
+def test_training_stats_span_edges(orc, A, k, p):
+    import gs_densify
+    vis, sel, flt, grad, opacity, acc = _case(A, k, A + k, *p)
+    ref = orc.training_stats(acc[0].numpy(), acc[1].numpy(), acc[2].numpy(), acc[3].numpy(), k, grad.numpy(),
+                             opacity.numpy(), flt.numpy(), sel.numpy(), vis.numpy())
+    d = [t.to(DEV) for t in acc]
+    gs_densify.training_statis(d[0], d[1], d[2], d[3], k, grad.to(DEV), opacity.to(DEV), flt.to(DEV), sel.to(DEV),
+                               vis.to(DEV))
+    for got, want in zip(d, ref):
+        assert np.abs(got.cpu().numpy().ravel() - want).max() <= 1e-6 * max(1.0, np.abs(want).max())
