@@ -55,7 +55,8 @@ train_stats_kernel(IDX slots, int k, IDX Vk, IDX M, const uint8_t* __restrict__ 
 
 // ---- n_offsets <= STATS_MAX_OFFSETS
 
-constexpr uint32_t STATS_ROWS = 256;          // anchors per workgroup, one thread each for the visibility mask
+constexpr uint32_t STATS_ROWS = 256;          // anchors per workgroup at the most, one thread each for the visibility mask
+constexpr uint32_t STATS_SLOTS = 4096;        // ... and slots, which LDS has to hold
 constexpr uint32_t STATS_SEL_CHUNK = 1024;    // candidates per prefix of the selection mask
 constexpr uint32_t STATS_ITEMS = 5;           // candidates per thread and round
 constexpr uint32_t STATS_ROUND = GS_BLOCK_1D * STATS_ITEMS;
@@ -84,9 +85,9 @@ __device__ __forceinline__ uint32_t count16(const uint8_t* __restrict__ mask, ui
 }
 
 // The set entries of a span of one of the masks (the first vis_spans workgroups: visibility): the total of the span, and
-// before every STATS_ROWS anchors or STATS_SEL_CHUNK candidates of it those that the span has before them.
+// before every `rows` anchors or STATS_SEL_CHUNK candidates of it those that the span has before them.
 __global__ void __launch_bounds__(STATS_COUNT_THREADS)
-train_stats_count_kernel(uint32_t A, uint32_t Vk, uint32_t vis_spans, const uint8_t* __restrict__ visible,
+train_stats_count_kernel(uint32_t A, uint32_t Vk, uint32_t vis_spans, uint32_t rows, const uint8_t* __restrict__ visible,
                          const uint8_t* __restrict__ selected, uint32_t* __restrict__ vis_prefix,
                          uint32_t* __restrict__ sel_prefix, uint32_t* __restrict__ vis_totals,
                          uint32_t* __restrict__ sel_totals) {
@@ -97,7 +98,7 @@ train_stats_count_kernel(uint32_t A, uint32_t Vk, uint32_t vis_spans, const uint
   const uint32_t c = count16(first_mask ? visible : selected, at, n);
   uint32_t total;
   const uint32_t before = block_exclusive_scan<STATS_COUNT_THREADS>(c, s_wave, total);
-  const uint32_t chunk = first_mask ? STATS_ROWS : STATS_SEL_CHUNK;
+  const uint32_t chunk = first_mask ? rows : STATS_SEL_CHUNK;
   if (at % chunk == 0 && at < n) (first_mask ? vis_prefix : sel_prefix)[at / chunk] = before;
   if (threadIdx.x == 0) (first_mask ? vis_totals : sel_totals)[span] = total;
 }
@@ -124,50 +125,77 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
   return v;
 }
 
-// A workgroup owns STATS_ROWS consecutive anchors.  Its visible ones are listed in LDS; their candidates are one run
-// of the candidate arrays, taken STATS_ITEMS per thread and round (whole anchors a round), so that mask bytes,
-// opacities and gradients are read in order and every step of the chain mask -> rank -> filter -> accumulator has
-// all of a thread's loads in flight at once.  The anchor's opacities are added from LDS in candidate order.
-// Bound by memory, most of it the lines of the two slot accumulators.  With the ranks written out by two scans and
-// one slot per thread, each waiting for six loads one after the other, the call took 139 us at 1 M anchors of 10
-// offsets (40 % visible, 60 % of those selected).  Six sets of inputs in turn, with the spans' totals turned into prefixes
-// by a launch of its own and four candidates a thread -> now: 62 -> 59 us, 5 offsets 42 -> 40, 2 M anchors 111 -> 108,
-// 200 k 27 -> 24.  Five candidates are what eight waves a SIMD have registers for (slots in 32 bits): with six and five
-// waves 53 us where five take 48 and four 50.  Not kept: a wave for every 64 anchors, without barriers (50 us for this
-// kernel's 44); the accumulators asked for with the masks, before it is known which slots are hit (59 -> 63); gradients
-// and opacities past the caches (60); the workgroups of one XCD on neighbouring anchors (60).
+// A workgroup owns `rows` consecutive anchors (a power of two that divides STATS_SPAN).  Its visible ones are listed in
+// LDS; their candidates are one run of the candidate arrays, taken STATS_ITEMS per thread and round (whole anchors a
+// round), so that mask bytes, opacities and gradients are read in order and every step of the chain mask -> rank ->
+// filter has all of a thread's loads in flight at once.  What a candidate adds to its slot waits in LDS; the slots'
+// accumulators follow in their own order, four a thread.
+// Bound by memory, most of it the two slot accumulators, 80 MB of which a view touches three quarters of the sectors at
+// 1 M anchors of 10 offsets (40 % visible, 60 % of those selected).  Where a lane loaded and stored the accumulators of its
+// own candidates, sectors went back in part: reading and writing such a pattern alone takes 39.5 us, with whole sectors
+// 30.0.  With the ranks written out by two scans and one slot per thread, each waiting for six loads one after the other,
+// the call took 139 us.  Six sets of inputs in turn, slot by slot -> sectors, the next round's masks asked for ahead:
+// 59 -> 56 us (the spans' totals turned into prefixes by a launch of its own: 62), 2 M anchors 108 -> 100.5, 5 offsets
+// 40 -> 39.  Five candidates are what eight waves a SIMD have registers for: with six and five waves 53 us where five took
+// 48 and four 50.  Not kept: a wave for every 64 anchors, without barriers (50 us for this kernel where it took 44); the
+// accumulators asked for with the masks, before it is known which slots gain (59 -> 63); gradients and opacities past the
+// caches (60); the workgroups of one XCD on neighbouring anchors (60).
 __global__ void __launch_bounds__(GS_BLOCK_1D) __attribute__((amdgpu_waves_per_eu(8)))
-train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, uint32_t M, bool prefixes,
-                         const uint8_t* __restrict__ visible, const uint32_t* __restrict__ vis_prefix,
+train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t rows_log2, uint32_t Vk, uint32_t M,
+                         bool prefixes, bool whole, const uint8_t* __restrict__ visible, const uint32_t* __restrict__ vis_prefix,
                          const uint32_t* __restrict__ vis_totals, const uint8_t* __restrict__ selected,
                          const uint32_t* __restrict__ sel_prefix, const uint32_t* __restrict__ sel_totals,
                          const uint8_t* __restrict__ update_filter, const float* __restrict__ grad, int grad_stride,
                          const float* __restrict__ opacity, float* __restrict__ opacity_accum,
                          float* __restrict__ anchor_demon, float* __restrict__ grad_accum, float* __restrict__ denom) {
   constexpr int WAVES = GS_BLOCK_1D / GS_WAVE;
+  constexpr uint32_t NONE = 0xFFFFFFFFu;
+  extern __shared__ float s_add[];  // of every candidate of the workgroup: what its slot gains, -1 where it gains nothing
   __shared__ float s_op[STATS_ROUND];
-  __shared__ uint32_t s_row[STATS_ROWS];
-  __shared__ uint32_t s_count[WAVES], s_before[WAVES];
+  __shared__ uint32_t s_row[STATS_ROWS];    // the visible anchors
+  __shared__ uint32_t s_first[STATS_ROWS];  // an anchor's first candidate among the workgroup's, NONE where it is not visible
+  __shared__ uint32_t s_count[WAVES], s_before[WAVES], s_head[WAVES];
   __shared__ uint32_t s_sel[STATS_ITEMS][WAVES];
   const uint32_t tid = threadIdx.x, lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
   const uint64_t below = (1ull << lane) - 1ull;
-  const uint32_t row0 = blockIdx.x * STATS_ROWS;
+  const uint32_t row0 = blockIdx.x << rows_log2;
   const uint32_t vis_before = wave_sum(before_span(vis_totals, row0 / STATS_SPAN, prefixes));
   uint32_t vis0 = vis_prefix[blockIdx.x];
-  const bool set = row0 + tid < A && visible[row0 + tid] != 0;
+  const bool set = (tid >> rows_log2) == 0u && row0 + tid < A && visible[row0 + tid] != 0;
   const uint64_t vm = gs_ballot(set);
   if (lane == 0) {
     s_count[wave] = (uint32_t)__popcll(vm);
     s_before[wave] = vis_before;
   }
   __syncthreads();
+  uint32_t place = (uint32_t)__popcll(vm & below), rows = 0;
 #pragma unroll
-  for (uint32_t w = 0; w < WAVES; w++) vis0 += s_before[w];
-  // the rank of the chunk's first candidate: what is set in the spans before, in
-  // the chunks of its span before, and before it in its chunk
+  for (uint32_t w = 0; w < WAVES; w++) {
+    vis0 += s_before[w];
+    if (w < wave) place += s_count[w];
+    rows += s_count[w];
+  }
   const uint64_t first64 = (uint64_t)vis0 * k;
   const uint32_t first = first64 < Vk ? (uint32_t)first64 : Vk;
+  const uint32_t candidates = min(rows * k, Vk - first);
+  // a round's masks and opacities are asked for one round ahead
+  const uint32_t rows_per_round = STATS_ROUND / k, round = rows_per_round * k;  // (at least 5 anchors)
+  uint8_t sel_next[STATS_ITEMS];
+  float op_next[STATS_ITEMS];
+  auto ask = [&](uint32_t at) {
+#pragma unroll
+    for (uint32_t q = 0; q < STATS_ITEMS; q++) {
+      const uint32_t c = q * GS_BLOCK_1D + tid;
+      const bool have = c < round && at + c < candidates;
+      sel_next[q] = have ? selected[first + at + c] : (uint8_t)0;
+      op_next[q] = have ? opacity[first + at + c] : 0.f;
+    }
+  };
+  ask(0);
+  // the rank of the chunk's first candidate: what is set in the spans before, in the chunks of its span before, and
+  // before it in its chunk
   const uint32_t sel_chunk = first / STATS_SEL_CHUNK;
+  uint32_t rank0 = first < Vk ? sel_prefix[sel_chunk] : 0u;  // (no candidates left: never used)
   uint32_t head = 0;
 #pragma unroll
   for (uint32_t q = 0; q < STATS_SEL_CHUNK / GS_BLOCK_1D; q++) {
@@ -175,34 +203,23 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
     head += (uint32_t)__popcll(gs_ballot(e < first && selected[e] != 0));
   }
   if (first < Vk) head += wave_sum(before_span(sel_totals, first / STATS_SPAN, prefixes));
-  if (lane == 0) s_sel[0][wave] = head;
-  __syncthreads();
-  uint32_t rank0 = first < Vk ? sel_prefix[sel_chunk] : 0u;  // (no candidates left: never used)
-  uint32_t place = (uint32_t)__popcll(vm & below), rows = 0;
-#pragma unroll
-  for (uint32_t w = 0; w < WAVES; w++) {
-    if (w < wave) place += s_count[w];
-    rows += s_count[w];
-    rank0 += s_sel[0][w];
-  }
+  if (lane == 0) s_head[wave] = head;
   if (set) s_row[place] = row0 + tid;
+  s_first[tid] = set ? place * k : NONE;
   __syncthreads();
+#pragma unroll
+  for (uint32_t w = 0; w < WAVES; w++) rank0 += s_head[w];
 
-  const uint32_t rows_per_round = STATS_ROUND / k;  // (at least 4)
   for (uint32_t r0 = 0; r0 < rows; r0 += rows_per_round) {
     const uint32_t nr = min(rows_per_round, rows - r0), n = nr * k;
-    // the round's first candidate, and how many of the round's there are
-    const uint64_t c64 = ((uint64_t)vis0 + r0) * k;
-    const uint32_t c0 = c64 < Vk ? (uint32_t)c64 : Vk, have_n = min(n, Vk - c0);
     bool sel[STATS_ITEMS];
     float op[STATS_ITEMS];
 #pragma unroll
     for (uint32_t q = 0; q < STATS_ITEMS; q++) {
-      const uint32_t c = q * GS_BLOCK_1D + tid;
-      const bool have = c < have_n;
-      sel[q] = have && selected[c0 + c] != 0;
-      op[q] = have ? opacity[c0 + c] : 0.f;
+      sel[q] = sel_next[q] != 0;
+      op[q] = op_next[q];
     }
+    if (r0 + rows_per_round < rows) ask((r0 + rows_per_round) * k);
     uint32_t rank[STATS_ITEMS];
 #pragma unroll
     for (uint32_t q = 0; q < STATS_ITEMS; q++) {
@@ -221,8 +238,7 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
       }
     }
     bool hit[STATS_ITEMS];
-    float gx[STATS_ITEMS], gy[STATS_ITEMS], acc[STATS_ITEMS], den[STATS_ITEMS];
-    uint32_t slot[STATS_ITEMS];
+    float gx[STATS_ITEMS], gy[STATS_ITEMS];
 #pragma unroll
     for (uint32_t q = 0; q < STATS_ITEMS; q++) {
       hit[q] = sel[q] && rank[q] < M;
@@ -236,21 +252,7 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
 #pragma unroll
     for (uint32_t q = 0; q < STATS_ITEMS; q++) {
       const uint32_t c = q * GS_BLOCK_1D + tid;
-      const uint32_t r = k == 1 ? c : __umulhi(c, k_magic);
-      acc[q] = den[q] = 0.f;
-      slot[q] = 0;
-      if (hit[q]) {
-        slot[q] = s_row[r0 + r] * k + (c - r * k);
-        acc[q] = grad_accum[slot[q]];
-        den[q] = denom[slot[q]];
-      }
-    }
-#pragma unroll
-    for (uint32_t q = 0; q < STATS_ITEMS; q++) {
-      if (hit[q]) {
-        grad_accum[slot[q]] = acc[q] + sqrtf(gx[q] * gx[q] + gy[q] * gy[q]);
-        denom[slot[q]] = den[q] + 1.0f;
-      }
+      if (c < n) s_add[r0 * k + c] = hit[q] ? sqrtf(gx[q] * gx[q] + gy[q] * gy[q]) : -1.0f;
     }
     if (tid < nr) {
       float sum = 0.f;
@@ -259,7 +261,50 @@ train_stats_chunk_kernel(uint32_t A, uint32_t k, uint32_t k_magic, uint32_t Vk, 
       opacity_accum[a] += sum;
       anchor_demon[a] += 1.0f;
     }
-    __syncthreads();  // (the next round's lists)
+    __syncthreads();  // (the next round's lists, the slots' gains)
+  }
+
+  // Sixteen slots, a sector of memory of either accumulator, are loaded and stored as a whole where one of them gains.
+  const uint32_t slots = min(1u << rows_log2, A - row0) * k;
+  float* const ga = grad_accum + (size_t)row0 * k;
+  float* const de = denom + (size_t)row0 * k;
+  for (uint32_t s0 = 4 * (tid & ~3u); s0 < slots; s0 += 4 * GS_BLOCK_1D) {
+    const uint32_t s = s0 + 4 * (tid & 3u);
+    float add[4];
+    bool any = false;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+      add[i] = -1.0f;
+      if (s + i < slots) {
+        const uint32_t a = k == 1 ? s + i : __umulhi(s + i, k_magic), f = s_first[a];
+        if (f != NONE) add[i] = s_add[f + (s + i - a * k)];
+      }
+      any |= !(add[i] < 0.f);
+    }
+    // (a quad takes part as a whole)
+    const uint64_t gains = gs_ballot(any);
+    if (((gains >> (lane & ~3u)) & 0xFull) == 0ull) continue;
+    if (whole && s + 4 <= slots) {
+      float4 g = *(const float4*)(ga + s), d = *(const float4*)(de + s);
+      g.x = add[0] < 0.f ? g.x : g.x + add[0];
+      g.y = add[1] < 0.f ? g.y : g.y + add[1];
+      g.z = add[2] < 0.f ? g.z : g.z + add[2];
+      g.w = add[3] < 0.f ? g.w : g.w + add[3];
+      d.x = add[0] < 0.f ? d.x : d.x + 1.0f;
+      d.y = add[1] < 0.f ? d.y : d.y + 1.0f;
+      d.z = add[2] < 0.f ? d.z : d.z + 1.0f;
+      d.w = add[3] < 0.f ? d.w : d.w + 1.0f;
+      *(float4*)(ga + s) = g;
+      *(float4*)(de + s) = d;
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) {
+        if (!(add[i] < 0.f)) {
+          ga[s + i] += add[i];
+          de[s + i] += 1.0f;
+        }
+      }
+    }
   }
 }
 
@@ -295,7 +340,10 @@ int launch_train_stats(long long A, int k, long long Vk, long long M, const uint
   if (A <= 0 || k <= 0) return 0;
   const long long slots = A * k;
   if (k <= STATS_MAX_OFFSETS && slots < 0x7FFFFFFFll && Vk < 0x7FFFFFFFll && M < 0x7FFFFFFFll) {
-    const uint32_t vis_chunks = (uint32_t)((A + STATS_ROWS - 1) / STATS_ROWS);
+    uint32_t rows_log2 = 8;  // (16 anchors of STATS_MAX_OFFSETS at the least: whole sectors of slots whatever k)
+    while ((uint32_t)k << rows_log2 > STATS_SLOTS) rows_log2--;
+    static_assert(STATS_ROWS == 1u << 8 && STATS_SLOTS == STATS_MAX_OFFSETS << 4, "between 16 and 256 anchors");
+    const uint32_t vis_chunks = (uint32_t)((A + (1ll << rows_log2) - 1) >> rows_log2);
     const uint32_t vis_spans = (uint32_t)((A + STATS_SPAN - 1) / STATS_SPAN);
     const uint32_t sel_spans = (uint32_t)((Vk + STATS_SPAN - 1) / STATS_SPAN);
     // (a prefix per chunk and a total per span: less than the ranks, an entry each, that the space is sized for, a total
@@ -306,13 +354,15 @@ int launch_train_stats(long long A, int k, long long Vk, long long M, const uint
     uint32_t* sel_totals = sel_prefix + (Vk + STATS_SEL_CHUNK - 1) / STATS_SEL_CHUNK;
     const bool prefixes = vis_spans > STATS_SPANS || sel_spans > STATS_SPANS;
     hipLaunchKernelGGL(train_stats_count_kernel, dim3(vis_spans + sel_spans), dim3(STATS_COUNT_THREADS), 0, stream,
-                       (uint32_t)A, (uint32_t)Vk, vis_spans, visible, selected, vis_prefix, sel_prefix, vis_totals,
-                       sel_totals);
+                       (uint32_t)A, (uint32_t)Vk, vis_spans, 1u << rows_log2, visible, selected, vis_prefix, sel_prefix,
+                       vis_totals, sel_totals);
     if (prefixes)
       hipLaunchKernelGGL(train_stats_spine_kernel, dim3(2), dim3(1024), 0, stream, vis_spans, sel_spans, vis_totals,
                          sel_totals);
-    hipLaunchKernelGGL(train_stats_chunk_kernel, dim3(vis_chunks), dim3(GS_BLOCK_1D), 0, stream, (uint32_t)A, (uint32_t)k,
-                       (uint32_t)(((1ull << 32) + k - 1) / k), (uint32_t)Vk, (uint32_t)M, prefixes, visible, vis_prefix,
+    hipLaunchKernelGGL(train_stats_chunk_kernel, dim3(vis_chunks), dim3(GS_BLOCK_1D),
+                       sizeof(float) * (size_t)k << rows_log2, stream, (uint32_t)A, (uint32_t)k,
+                       (uint32_t)(((1ull << 32) + k - 1) / k), rows_log2, (uint32_t)Vk, (uint32_t)M, prefixes,
+                       ((uintptr_t)grad_accum & 15) == 0 && ((uintptr_t)denom & 15) == 0, visible, vis_prefix,
                        vis_totals, selected, sel_prefix, sel_totals, update_filter, grad, grad_stride, opacity,
                        opacity_accum, anchor_demon, grad_accum, denom);
     return 0;

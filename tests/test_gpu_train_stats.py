@@ -134,3 +134,38 @@ def test_training_stats_span_edges(orc, A, k, p):
                                vis.to(DEV))
     for got, want in zip(d, ref):
         assert np.abs(got.cpu().numpy().ravel() - want).max() <= 1e-6 * max(1.0, np.abs(want).max())
+
+
+# whole sectors of 16 slots and what is left of them, accumulators that do not start at a multiple of 16 bytes, every
+# number of anchors a workgroup takes; gains of 0, infinite and NaN ones, and slots without a gain, which keep their bits
+@pytest.mark.parametrize("A,k", [(1003, 1), (513, 10), (300, 16), (301, 17), (130, 33), (67, 65), (35, 129), (17, 256)])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_training_stats_sectors(orc, A, k, shift):
+    import gs_densify
+    vis, sel, flt, grad, opacity, acc = _case(A, k, A + k, 0.4, 0.5, 0.7)
+    S = grad.shape[0]
+    grad[:: 7] = 0.0
+    grad[min(3, S - 1)] = float("inf")
+    grad[min(5, S - 1)] = float("nan")
+    acc[2][::3] = -0.0
+    acc[2][1::5] = float("nan")
+    ref = orc.training_stats(acc[0].numpy(), acc[1].numpy(), acc[2].numpy(), acc[3].numpy(), k, grad.numpy(),
+                             opacity.numpy(), flt.numpy(), sel.numpy(), vis.numpy())
+    place = lambda a: torch.cat([torch.full((shift, 1), 7.0), a, torch.full((3, 1), 7.0)]).to(DEV)
+    whole = [place(a) for a in acc]
+    d = [w[shift:shift + a.shape[0]] for w, a in zip(whole, acc)]
+    gs_densify.training_statis(d[0], d[1], d[2], d[3], k, grad.to(DEV), opacity.to(DEV), flt.to(DEV), sel.to(DEV),
+                               vis.to(DEV))
+    for w, a in zip(whole, acc):
+        assert bool((w[:shift] == 7.0).all()) and bool((w[shift + a.shape[0]:] == 7.0).all())
+    for got, want in zip(d, ref):
+        got, want = got.cpu().numpy().ravel(), want.ravel()
+        assert np.array_equal(np.isfinite(got), np.isfinite(want))
+        ok = np.isfinite(want)
+        assert np.abs(got[ok] - want[ok]).max() <= 1e-6 * max(1.0, np.abs(want[ok]).max())
+    hit = torch.zeros(A * k, dtype=torch.bool)
+    cand = hit.clone()
+    cand[vis.repeat_interleave(k)] = sel
+    hit[cand] = flt
+    bits = lambda x: x.cpu().contiguous().view(torch.int32).ravel()
+    assert torch.equal(bits(d[2])[~hit], bits(acc[2])[~hit]) and torch.equal(bits(d[3])[~hit], bits(acc[3])[~hit])
