@@ -844,6 +844,8 @@ int gs_render_backward(int P, int R, const float* background, int width, int hei
   a.packed = blend_records != nullptr ? blend_records : (const float*)(bbase + BL.packed);
   a.packed_valid = blend_records != nullptr ? nullptr : (const uint32_t*)(gbase + GL.packed_valid);
   a.instance_grads = (float*)align_ptr((const char*)instance_grads, 256);
+  a.R = R;
+  if (instance_grads_bytes >= gs_render_backward_sparse_workspace_bytes(R)) a.written = (uint8_t*)(a.instance_grads + 16 * (size_t)R);
   a.P = P; a.W = width; a.H = height;
   a.fy = height / (2.0f * tan_fovy);  // cuda_rasterizer/rasterizer_impl.cu:885-886
   a.fx = width / (2.0f * tan_fovx);
@@ -879,6 +881,10 @@ int gs_render_backward(int P, int R, const float* background, int width, int hei
 }
 
 size_t gs_render_backward_workspace_bytes(int R) { return (size_t)(R > 0 ? R : 1) * 16 * sizeof(float) + 256; }
+
+size_t gs_render_backward_sparse_workspace_bytes(int R) {
+  return gs_render_backward_workspace_bytes(R) + ((size_t)(R > 0 ? R : 1) + 3) / 4 * 4;
+}
 
 size_t gs_knn_workspace_bytes(int P) { return knn_temp_bytes(P) + 256; }
 

@@ -299,7 +299,11 @@ struct RenderBwdArgs {
   // prefix sum of tiles touched, i.e. Gaussian i owns emission indices [point_offsets[i-1], point_offsets[i]).
   const uint32_t* emission_sorted;
   const uint32_t* point_offsets;
-  float* instance_grads;  // (R,16) scratch, fully written by the blend kernel
+  float* instance_grads;  // (R,16) scratch, fully written by the blend kernel unless `written` says which are
+  // optional, whole words of 4 for R instances (cleared here): one byte per instance, 1 where the blend kernel has
+  // written a record; the others are zeros that are neither stored nor read
+  uint8_t* written = nullptr;
+  int R = 0;
   const uint32_t* block_hits = nullptr;  // optional (R): left by the forward blend (RenderFwdArgs::block_hits)
   const float* packed = nullptr;         // optional (P,4) 16-byte words: see RenderFwdArgs::packed
   // optional device word beside `packed`: non-zero if the forward call did pack the records (it decides per view)

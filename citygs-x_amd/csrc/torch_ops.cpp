@@ -276,7 +276,7 @@ py::tuple render_backward(const Tensor& background, float tan_fovx, float tan_fo
   const int H = (int)dL_dout_color.size(1), W = (int)dL_dout_color.size(2);
   Tensor d2 = at::empty({P, 2}, o.f32), dabs = at::empty({P, 3}, o.f32), dco = at::empty({P, 4}, o.f32),
          dcol = at::empty({P, CHANNELS}, o.f32), dmap = at::empty({P, MAP_CHANNELS}, o.f32);
-  const size_t ws_bytes = gs_render_backward_workspace_bytes(R);
+  const size_t ws_bytes = gs_render_backward_sparse_workspace_bytes(R);
   const Tensor workspace = at::empty({(int64_t)ws_bytes}, o.u8);
   const Tensor bg = f32c(background, "background"), gpix = f32c(dL_dout_color, "dL_dout_color");
   TORCH_CHECK_TYPE(!geo || (dL_dout_all_map && dL_dout_plane_depth && all_map_pixels && all_maps),

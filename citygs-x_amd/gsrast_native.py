@@ -72,6 +72,7 @@ _SIGNATURES = {
     "gs_render_forward": (_i, [RESIZE_FN, _vp, RESIZE_FN, _vp, RESIZE_FN, _vp, _i, _vp, _i, _i, _f, _f, _f, _f] +
                           [_vp] * 17 + [_i, _i, C.POINTER(_i), C.POINTER(_f), _vp, _vp, _vp]),
     "gs_render_backward_workspace_bytes": (_sz, [_i]),
+    "gs_render_backward_sparse_workspace_bytes": (_sz, [_i]),
     "gs_render_backward": (_i, [_i, _i, _vp, _i, _i, _f, _f] + [_vp] * 17 + [_i, _i, _vp, _sz, C.POINTER(_f), _i64,
                                 _vp, _vp]),
     "gs_ssim_l1_forward": (_i, [_i, _i, _i] + [_vp] * 9),

@@ -246,6 +246,9 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
  * binning_capacity: gs_render_result.binning_capacity of the forward call (0 or R if it did not run ahead).
  * blend_records: gs_render_options.blend_records of the forward call (NULL if that call was given none). */
 size_t gs_render_backward_workspace_bytes(int R);
+/* As much scratch lets gs_render_backward leave out the records of instances that no pixel blends, which are zeros, where
+ * that pays: a byte per instance says which records there are.  The results are the same. */
+size_t gs_render_backward_sparse_workspace_bytes(int R);
 int gs_render_backward(int P, int R, const float* background, int width, int height, float tan_fovx,
                        float tan_fovy, const char* geom_buffer, const char* binning_buffer,
                        const char* img_buffer, const uint8_t* compute_locally, const float* dL_dpix,
