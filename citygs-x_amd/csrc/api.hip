@@ -689,7 +689,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     {
       StageScope _t("tile_sort", stream);
       if (launch_tile_sort(T, longest_for_launch, radix_tiles, sort_limit, (uint32_t)limits.block, ranges,
-                           bucket_table, A.keys_other, A.radix_scratch, A.capacity, A.keys, A.emission,
+                           bucket_table, A.keys_other, A.radix_scratch, A.block_hits, A.capacity, A.keys, A.emission,
                            A.point_list, tile_order, packed_valid + 1, longest_split_list(render_geo != 0), n_consider,
                            n_contrib, ahead_of_host, stream))
         return 1;

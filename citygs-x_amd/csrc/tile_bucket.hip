@@ -165,8 +165,8 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_u32(uint32_t v, int lane
 // lists for the radix sort's kernels: lists of more than small_limit and at most mid_limit records ascending from
 // tile_lists[0], longer ones descending from tile_lists[T - 1]; tile_lists[T] = (number of the longer ones << 16
 // | number of the others) (T is at most 30000).  The lists beyond block_limit records, which are split before they
-// are sorted and take several times as long, are entered a second time in a list of their own, so that the larger
-// kernel can start with them: their number in tile_lists[T + 1], the tiles ascending from tile_lists[T + 2].  The longest list, that word and then the number of instances are
+// are sorted, are entered a second time in a list of their own: their number in tile_lists[T + 1], the tiles ascending from
+// tile_lists[T + 3] (tile_lists[T + 2]: see split_list).  The longest list, tile_lists[T] and then the number of instances are
 // stored where the host can read them (host_words[1], [2] and [0]; the host polls word 0, so it is written last).
 __global__ void __launch_bounds__(1024)
 bucket_ranges_kernel(uint32_t T, uint32_t small_limit, uint32_t mid_limit, uint32_t block_limit,
@@ -242,7 +242,7 @@ bucket_ranges_kernel(uint32_t T, uint32_t small_limit, uint32_t mid_limit, uint3
         ranges[2 * (t0 + q) + 1] = v[q] ? begin + v[q] : 0u;
         if (c[q] == 1u) tile_lists[begin_class & 0xFFFFu] = t0 + q;
         if (c[q] == 0x10000u) tile_lists[T - 1u - (begin_class >> 16)] = t0 + q;
-        if (v[q] > block_limit) tile_lists[T + 2u + begin_split] = t0 + q;
+        if (v[q] > block_limit) tile_lists[T + 3u + begin_split] = t0 + q;
       }
       begin += v[q];
       begin_class += c[q];
@@ -273,6 +273,7 @@ bucket_ranges_kernel(uint32_t T, uint32_t small_limit, uint32_t mid_limit, uint3
     }
     tile_lists[T] = carry_class;
     tile_lists[T + 1u] = carry_split;
+    tile_lists[T + 2u] = 0u;
     if (clear_word != nullptr) clear_word[0] = clear_word[1] = 0u;  // (two words the caller wants cleared: saves a launch)
     // more instances than 32-bit positions can address: the host must not go on with the wrapped count
     const uint32_t reported = all > (double)GS_MAX_INSTANCES ? GS_TOO_MANY_INSTANCES : carry;
@@ -868,7 +869,169 @@ __device__ __forceinline__ void order_tiles(uint32_t T, const uint32_t* __restri
   }
 }
 
-// Workgroup 0 orders the tiles for the blend kernels, workgroup t + 1 sorts tile t.
+// A list of more than `blk` records is split for the radix sort, by depth, into groups that it takes like short lists.  A
+// sample of the list gives the groups' bounds, in 256ths of the sample's range of depths, so that a group holds some four
+// fifths of blk; what lies outside that range goes to the first and the last group, equal depth bits into one group (the
+// sorts' last step sees runs of them whole), and a group beyond blk (many instances within 1/256 of the range) goes block by
+// block through memory.  Every wave counts the groups in its part of the list and then moves the part to `parted`.  The
+// groups' first places are left in list_words, from `start` on (an array that the blend kernel fills later), their number
+// beside the tile in `entry`, the largest of all lists in *most.
+// Here, beside the register sort, and not in the radix sort's own workgroups, each of which holds a CU for as long as its
+// list is: 20 M Gaussians from 600 m, two views whose longest lists have 69 000 and 43 000 entries, 43 + 491 and 43 + 349 us
+// (this kernel and the radix sort) -> 140 + 265 and 133 + 250.  Bound by the memory's traffic, 48 bytes a record.  With 256
+// bins, counted and filled by LDS atomics, 177 us of this kernel instead of 137; the moved records through the caches 152,
+// four of them in flight a lane instead of eight 165; three workgroups a list, each counting all of it, 198.  Without the
+// move, every group's workgroup looking for its entries in the whole list: 43 + 380 us.
+// s_words: SPLIT_WORDS words.
+constexpr uint32_t SPLIT_BINS = 256, SPLIT_GROUPS = GS_WAVE;  // (a lane for every group)
+constexpr uint32_t SPLIT_WAVES = 8;
+constexpr uint32_t SPLIT_WORDS = SPLIT_BINS + SPLIT_BINS / 4 + SPLIT_WAVES * SPLIT_GROUPS + 2 * SPLIT_WAVES;
+__device__ __forceinline__ void split_list(uint32_t t, uint32_t start, uint32_t n, uint32_t blk,
+                                           const TileRecord* __restrict__ records, TileRecord* __restrict__ parted,
+                                           uint32_t* __restrict__ list_words, uint32_t* __restrict__ entry,
+                                           uint32_t* __restrict__ most, uint32_t* s_words) {
+  constexpr uint32_t WAVES = SPLIT_WAVES, THREADS = WAVES * GS_WAVE, SAMPLED = 8, QUARTERS = SPLIT_BINS / GS_WAVE;
+  constexpr uint32_t COUNTED = 16, MOVED = 8;  // loads a lane keeps in flight
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  uint32_t* const s_bins = s_words;
+  uint8_t* const s_group = reinterpret_cast<uint8_t*>(s_words + SPLIT_BINS);  // a bin's group
+  uint32_t* const s_count = s_words + SPLIT_BINS + SPLIT_BINS / 4;            // [WAVES][SPLIT_GROUPS]
+  uint32_t* const s_scan = s_count + WAVES * SPLIT_GROUPS;
+  const TileRecord* const list = records + start;
+  const uint32_t step = n / (SAMPLED * THREADS) + 1u, in_all = (n + step - 1u) / step;
+  const uint32_t samples = min(SAMPLED * THREADS, in_all);
+  uint32_t z[SAMPLED], lo = 0xFFFFFFFFu, hi = 0u;
+#pragma unroll
+  for (uint32_t u = 0; u < SAMPLED; u++) z[u] = list[min(u * THREADS + tid, samples - 1u) * step].z;
+#pragma unroll
+  for (uint32_t u = 0; u < SAMPLED; u++) {
+    lo = min(lo, z[u]);
+    hi = max(hi, z[u]);
+  }
+  lo = ~(uint32_t)__builtin_amdgcn_readlane((int)wave_scan_max(~lo), GS_WAVE - 1);
+  hi = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_max(hi), GS_WAVE - 1);
+  if (lane == 0u) {
+    s_scan[wave] = lo;
+    s_scan[WAVES + wave] = hi;
+  }
+  if (tid < SPLIT_BINS) s_bins[tid] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t w = 0; w < WAVES; w++) {
+    lo = min(lo, s_scan[w]);
+    hi = max(hi, s_scan[WAVES + w]);
+  }
+  const uint32_t range = hi - lo;
+  const int bits = range != 0u ? 32 - __builtin_clz(range) : 0, shift = bits > 8 ? bits - 8 : 0;
+  auto bin_of = [&](uint32_t depth) { return (min(max(depth, lo), hi) - lo) >> shift; };
+#pragma unroll
+  for (uint32_t u = 0; u < SAMPLED; u++)
+    if (u * THREADS + tid < samples) atomicAdd(&s_bins[bin_of(z[u])], 1u);
+  __syncthreads();
+  if (wave == 0u) {
+    // ends[k] of lane l: the samples in the bins up to 64 k + l
+    uint32_t ends[QUARTERS], carry = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < QUARTERS; k++) {
+      ends[k] = carry + wave_inclusive_scan_u32(s_bins[k * GS_WAVE + lane], (int)lane);
+      carry = (uint32_t)__builtin_amdgcn_readlane((int)ends[k], GS_WAVE - 1);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < QUARTERS; k++) s_bins[k * GS_WAVE + lane] = ends[k];
+    auto bins_up_to = [&](uint32_t place) {
+      uint32_t c = 0u;
+#pragma unroll
+      for (uint32_t k = 0; k < QUARTERS; k++) c += (uint32_t)__popcll(gs_ballot(ends[k] <= place));
+      return c;
+    };
+    const uint32_t share = (uint32_t)((uint64_t)samples * blk / 5u * 4u / n), least = samples / (SPLIT_GROUPS - 16u) + 1u;
+    const uint32_t wanted = max(share, least);
+    uint32_t groups = 0u, first = 0u, bin = 0u;
+    while (bin < SPLIT_BINS) {
+      const uint32_t before = bins_up_to(first), whole = bins_up_to(first + wanted);
+      const uint32_t end =
+          groups + 1u == min(SPLIT_GROUPS, n) ? SPLIT_BINS : min(whole > before ? whole : before + 1u, SPLIT_BINS);
+#pragma unroll
+      for (uint32_t k = 0; k < QUARTERS; k++) {
+        const uint32_t b = k * GS_WAVE + lane;
+        if (b >= bin && b < end) s_group[b] = (uint8_t)groups;
+      }
+      first = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bins[end - 1u]);
+      bin = end;
+      groups++;
+    }
+    if (lane == 0u) s_scan[0] = groups;
+  }
+  __syncthreads();
+  const uint32_t groups = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_scan[0]);
+  const int group_bits = 32 - __builtin_clz(groups | 1u);  // (so that no group has all of them set: that is nobody's)
+  const uint32_t nobody = (1u << group_bits) - 1u;  // (a lane without a record; at least `groups`)
+  // The lanes whose g equals the lane's own `a`, and those with its `b`.
+  auto lanes_with = [&](uint32_t g, uint32_t a, uint32_t b, uint64_t& with_a, uint64_t& with_b) {
+    with_a = with_b = ~0ull;
+    for (int k = 0; k < group_bits; k++) {
+      const uint64_t set = gs_ballot((g >> k & 1u) != 0u);
+      with_a &= (a >> k & 1u) != 0u ? set : ~set;
+      with_b &= (b >> k & 1u) != 0u ? set : ~set;
+    }
+  };
+  const uint32_t part = (n + THREADS - 1u) / THREADS * GS_WAVE;  // a wave's records
+  const uint32_t from = min(wave * part, n), to = min(from + part, n);
+  uint32_t found = 0u;  // lane g: the wave's records of group g (lanes from `groups` on: anything)
+  for (uint32_t i0 = from; i0 < to; i0 += GS_WAVE * COUNTED) {
+    uint32_t d[COUNTED];
+#pragma unroll
+    for (uint32_t u = 0; u < COUNTED; u++) d[u] = list[min(i0 + u * GS_WAVE + lane, to - 1u)].z;
+#pragma unroll
+    for (uint32_t u = 0; u < COUNTED; u++) {
+      const uint32_t g = i0 + u * GS_WAVE + lane < to ? (uint32_t)s_group[bin_of(d[u])] : nobody;
+      uint64_t mine, unused;
+      lanes_with(g, lane, lane, mine, unused);
+      found += (uint32_t)__popcll(mine);
+    }
+  }
+  s_count[wave * SPLIT_GROUPS + lane] = found;
+  __syncthreads();
+  uint32_t total = 0u, place = 0u;  // lane g: all records of group g, and those of the waves before this one
+#pragma unroll
+  for (uint32_t w = 0; w < WAVES; w++) {
+    const uint32_t c = s_count[w * SPLIT_GROUPS + lane];
+    place += w < wave ? c : 0u;
+    total += c;
+  }
+  if (lane >= groups) total = 0u;
+  const uint32_t group_first = wave_inclusive_scan_u32(total, (int)lane) - total;
+  place += group_first;  // where the wave's next record of group g goes
+  for (uint32_t i0 = from; i0 < to; i0 += GS_WAVE * MOVED) {
+    TileRecord r[MOVED];
+#pragma unroll
+    for (uint32_t u = 0; u < MOVED; u++) r[u] = list[min(i0 + u * GS_WAVE + lane, to - 1u)];
+#pragma unroll
+    for (uint32_t u = 0; u < MOVED; u++) {
+      const uint32_t g = i0 + u * GS_WAVE + lane < to ? (uint32_t)s_group[bin_of(r[u].z)] : nobody;
+      uint64_t same, mine;
+      lanes_with(g, g, lane, same, mine);
+      const uint32_t next = (uint32_t)__shfl((int)place, (int)(g & 63u), GS_WAVE);
+      const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, next));
+      if (g != nobody)
+        store_streaming(reinterpret_cast<float4*>(parted + start + at),
+                        make_float4(__uint_as_float(r[u].x), __uint_as_float(r[u].y), __uint_as_float(r[u].z), 0.f));
+      place += (uint32_t)__popcll(mine);
+    }
+  }
+  if (wave == 0u) {
+    if (lane < groups) list_words[start + lane] = group_first;
+    if (lane == 0u) {
+      *entry = t | groups << 16;
+      atomicMax(most, groups);
+    }
+  }
+  __syncthreads();  // (the words are the next sort's)
+}
+
+// Workgroup 0 orders the tiles for the blend kernels, workgroup t + 1 sorts tile t; before that, the first workgroups split
+// the lists that are too long for one workgroup of the radix sort (split_lists: the number of them, see split_list, the tiles;
+// the kernel with MAX_E = 8 only).
 // Dynamic LDS: 8 bytes per record of the longest list the kernel takes, rounded up to a power of two (at least
 // 256 records).  Lists of more than max_n records are left to the radix sort's kernels.
 // MAX_E: the most keys a lane has.  Views without lists beyond 2048 have a kernel without the way for eight: in the other one
@@ -882,7 +1045,8 @@ tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord
                            uint32_t* __restrict__ point_list, uint32_t max_n,
                            const uint32_t* __restrict__ fits_word, uint32_t* __restrict__ order,
                            uint32_t* __restrict__ order_word, uint32_t longest_split, int* __restrict__ n_consider,
-                           int* __restrict__ n_contrib) {
+                           int* __restrict__ n_contrib, uint32_t* __restrict__ split_lists, uint32_t block_limit,
+                           TileRecord* __restrict__ parted, uint32_t* __restrict__ list_words) {
   extern __shared__ uint64_t s_exchange[];
   if (fits_word != nullptr && *fits_word == 0u) return;  // launched ahead of the host's decision: see the scatter
   if (blockIdx.x == 0) {
@@ -891,6 +1055,13 @@ tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord
     return;
   }
   const uint32_t t = blockIdx.x - 1;
+  if constexpr (MAX_E == 8) {
+    if (t < split_lists[0]) {
+      const uint32_t long_tile = split_lists[2u + t], first = ranges[2 * long_tile];
+      split_list(long_tile, first, ranges[2 * long_tile + 1] - first, block_limit, records, parted, list_words,
+                 split_lists + 2u + t, split_lists + 1, reinterpret_cast<uint32_t*>(s_exchange));
+    }
+  }
   const uint32_t start = ranges[2 * t];
   const uint32_t n = ranges[2 * t + 1] - start;
   if (n == 0 || n > 512u * MAX_E || n > max_n) return;
@@ -909,17 +1080,17 @@ tile_sort_registers_kernel(const uint32_t* __restrict__ ranges, const TileRecord
 // Tiles the LDS histograms of the counting kernels can hold.
 int bucket_max_tiles() { return 30000; }
 
-// workgroup-by-tile counts, then the tile totals, then the tile lists of the radix sort's kernels (2 T + 2 words), then
+// workgroup-by-tile counts, then the tile totals, then the tile lists of the radix sort's kernels (2 T + 3 words), then
 // the workgroups' sums of tiles touched and the word that says whether the view fits the buffers of kernels
 // launched ahead of the host
 size_t bucket_table_bytes(int T) {
-  return (((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 2 + BK_MAX_BLOCKS + 1) * sizeof(uint32_t);
+  return (((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 3 + BK_MAX_BLOCKS + 1) * sizeof(uint32_t);
 }
 static uint32_t* bucket_block_sums(void* table, uint32_t T) {
-  return (uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 2;
+  return (uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 3;
 }
 const uint32_t* bucket_fits_word(const void* table, int T) {
-  return (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 2 + BK_MAX_BLOCKS;
+  return (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 3) * (size_t)T + 3 + BK_MAX_BLOCKS;
 }
 
 // The longest list that the radix sort's smaller kernel takes (what one of its workgroups holds); longer ones go to the
@@ -1023,29 +1194,34 @@ int launch_bucket_scatter(int P, int W, int H, const float* means2D, const float
 // holds 24 bytes for each of the `capacity` instances the binning arrays are laid out for.  tile_order (T words) and
 // the word that says it is there: see order_tiles (neither is written where there is no list at all).
 int launch_tile_sort(int T, uint32_t longest, uint32_t radix_tiles, uint32_t small_limit, uint32_t block_limit,
-                     const uint32_t* ranges, const void* table, const void* records, void* scratch, int64_t capacity,
-                     uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
+                     const uint32_t* ranges, void* table, const void* records, void* scratch, uint32_t* list_words,
+                     int64_t capacity, uint64_t* keys, uint32_t* emission, uint32_t* point_list, uint32_t* tile_order,
                      uint32_t* tile_order_word, uint32_t longest_split, int* n_consider, int* n_contrib,
                      bool ahead_of_host, hipStream_t stream) {
   if (T <= 0 || longest == 0) return 0;
   const uint32_t* fits = ahead_of_host ? bucket_fits_word(table, T) : nullptr;
   if (small_limit == 0 || small_limit > (uint32_t)TILE_SORT_SMALL) small_limit = TILE_SORT_SMALL;
   const uint32_t whole = longest < small_limit ? longest : small_limit;  // the longest list sorted in registers
-  uint32_t m = 256;
+  const uint32_t block = (uint32_t)tile_radix_block_records();
+  if (block_limit == 0 || block_limit > block) block_limit = block;
+  const bool split = longest > block_limit;  // (there may be lists that the radix sort wants split)
+  uint32_t m = split ? 512 : 256;
+  static_assert(SPLIT_WORDS * sizeof(uint32_t) <= 512 * sizeof(uint64_t), "the split's words fit");
   while (m < whole) m <<= 1;
-  hipLaunchKernelGGL(whole > 2048 ? tile_sort_registers_kernel<8> : tile_sort_registers_kernel<4>, dim3(T + 1), dim3(512),
-                     (size_t)m * sizeof(uint64_t), stream, ranges, (const TileRecord*)records, keys, emission, point_list,
-                     small_limit, fits, tile_order, tile_order_word, longest_split, n_consider, n_contrib);
+  uint32_t* const tile_lists = (uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 1) * (size_t)T;
+  hipLaunchKernelGGL(whole > 2048 || split ? tile_sort_registers_kernel<8> : tile_sort_registers_kernel<4>, dim3(T + 1),
+                     dim3(512), (size_t)m * sizeof(uint64_t), stream, ranges, (const TileRecord*)records, keys, emission,
+                     point_list, small_limit, fits, tile_order, tile_order_word, longest_split, n_consider, n_contrib,
+                     tile_lists + T + 1, block_limit, (TileRecord*)scratch, list_words);
   if (longest > small_limit) {
     // (a launch with nothing to do takes 4.6 us of the device: a view whose longest list is bounded does without)
     const bool lng = (radix_tiles >> 16) != 0u && longest > radix_mid_limit(small_limit, block_limit);
-    const uint32_t* tile_lists = (const uint32_t*)table + ((size_t)BK_MAX_BLOCKS + 1) * (size_t)T;
     // scratch: `capacity` 16-byte records for the lists that are split first, then as many 8-byte words
     uint64_t* pong = (uint64_t*)((char*)scratch + (size_t)capacity * 16);
     // (the smaller kernel has lists only where the caller's options leave some between the two limits)
     const bool mid = (radix_tiles & 0xFFFFu) != 0u && radix_mid_limit(small_limit, block_limit) > small_limit;
     if (launch_tile_radix_sort(T, mid, lng, ranges, tile_lists,
-                               tile_lists + T, block_limit, records, scratch, keys, pong, keys, emission, point_list,
+                               tile_lists + T, block_limit, records, scratch, list_words, keys, pong, keys, emission, point_list,
                                fits, stream))
       return 1;
   }

@@ -9,7 +9,7 @@
 // ranks the keys of a pass per wave (lanes that hold the same digit find each other through a 64-bit lane mask per
 // digit in LDS, a running count per wave and digit makes the rank stable), turns the waves' digit counts into
 // places by one scan, moves every key to its place through LDS and reads its next batch back: two passes on 9-bit
-// digits.  A longer list is first split by its leading depth bits into parts that fit; a part that still does not
+// digits.  A longer list arrives split by depth into groups that fit (split_list, tile_bucket.hip); a group that does not
 // is sorted block by block on 64-bit records (depth bits << 32 | place) with 8-bit digits against running digit
 // bases, ping-ponging between two arrays in memory.  The last step looks Gaussian, emission index and depth bits of
 // every sorted entry up in the segment (a gather inside the tile's own records, through LDS) and writes the three
@@ -93,7 +93,6 @@ struct TileRadixLds {
   lds_u32* first;      // [256]
   lds_u32* base;       // [4][256] blocked sort: where the next record of a digit goes in the segment, per pass
   lds_u32* scan;       // [16]
-  lds_u32* bins;       // [257] partitioned sort: first place of every leading-digit bin in the list, then its length
   __device__ explicit TileRadixLds(lds_u64* p) {
     rec = p;
     key = (lds_u32*)p;
@@ -103,11 +102,10 @@ struct TileRadixLds {
     first = total + TR_DIGITS;
     base = first + TR_DIGITS;
     scan = base + TR_PASSES * TR_DIGITS;
-    bins = scan + 16;
   }
   static constexpr size_t bytes() {
     return LEAD_BYTES +
-           (size_t)(WAVES * TR_DIGITS + 2 * TR_DIGITS + TR_PASSES * TR_DIGITS + 16 + TR_DIGITS + 4) * 4;
+           (size_t)(WAVES * TR_DIGITS + 2 * TR_DIGITS + TR_PASSES * TR_DIGITS + 16) * 4;
   }
   __device__ PassLds<lds_u64*> wide() const { return {rec, (lds_mask*)rec, count, total, first, scan}; }
   __device__ PassLds<lds_u32*> narrow() const { return {key, (lds_mask*)rec, key_count, total, first, scan}; }
@@ -551,146 +549,52 @@ __device__ __forceinline__ void sort_blocked(uint32_t tile, uint32_t start, uint
   }
 }
 
-// A list of more than `blk` records: split by the leading eight bits of (depth bits - smallest) into bins, moved
-// bin by bin into `parted` (any order inside a bin), and runs of consecutive bins that hold at most blk records
-// together are sorted like short lists, inside the CU.  A single bin beyond blk records (many instances within
-// 1/256 of the list's depth range) goes block by block through memory.  Runs of equal depth bits never straddle
-// two bins, so the last step of the sorts still sees them whole.
-template <int WAVES, int ITEMS>
-__device__ __forceinline__ void sort_partitioned(uint32_t tile, uint32_t start, uint32_t n, uint32_t blk,
-                                                 const TileRecord* __restrict__ records, TileRecord* parted,
-                                                 uint64_t* ping, uint64_t* pong, uint64_t* keys, uint32_t* emission,
-                                                 uint32_t* point_list, const TileRadixLds<WAVES, ITEMS>& L) {
-  constexpr int THREADS = WAVES * GS_WAVE;
-  constexpr int SWEEP = 8;  // loads a thread keeps in flight in every sweep over the list
-  const int tid = thread_here(), lane = tid & (GS_WAVE - 1), wave = tid / GS_WAVE;
-  uint32_t dmin = 0xFFFFFFFFu, dmax = 0u;
-  for (uint32_t i0 = 0; i0 < n; i0 += THREADS * SWEEP) {
-    uint32_t depth_bits[SWEEP];
-#pragma unroll
-    for (int u = 0; u < SWEEP; u++) {
-      const uint32_t i = i0 + (uint32_t)u * THREADS + (uint32_t)tid;
-      depth_bits[u] = i < n ? records[start + i].z : dmax;
-    }
-#pragma unroll
-    for (int u = 0; u < SWEEP; u++) {
-      const uint32_t i = i0 + (uint32_t)u * THREADS + (uint32_t)tid;
-      if (i < n) {
-        dmin = depth_bits[u] < dmin ? depth_bits[u] : dmin;
-        dmax = depth_bits[u] > dmax ? depth_bits[u] : dmax;
-      }
-    }
-  }
-  workgroup_min_max<WAVES>(dmin, dmax, L.scan, L.total);
-  const uint32_t range = dmax - dmin;
-  const int bits = range != 0u ? 32 - __builtin_clz(range) : 0;
-  const int shift = bits > 8 ? bits - 8 : 0;
-  for (int i = tid; i <= TR_DIGITS; i += THREADS) L.bins[i] = 0u;
-  __syncthreads();
-  for (uint32_t i0 = 0; i0 < n; i0 += THREADS * SWEEP) {
-    uint32_t depth_bits[SWEEP];
-#pragma unroll
-    for (int u = 0; u < SWEEP; u++) {
-      const uint32_t i = i0 + (uint32_t)u * THREADS + (uint32_t)tid;
-      depth_bits[u] = i < n ? records[start + i].z : dmin;
-    }
-#pragma unroll
-    for (int u = 0; u < SWEEP; u++) {
-      const bool valid = i0 + (uint32_t)u * THREADS + (uint32_t)tid < n;
-      const uint32_t d = (depth_bits[u] - dmin) >> shift;
-      // a digit shared by the whole wave would serialise the LDS atomic 64 ways: one lane adds
-      const uint64_t vm = gs_ballot(valid);
-      const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
-      if (vm != 0ull && gs_ballot(valid && d == d0) == vm && (vm & 1ull)) {
-        if (lane == 0) atomicAdd((uint32_t*)&L.bins[d0], (uint32_t)__popcll(vm));
-      } else if (valid) {
-        atomicAdd((uint32_t*)&L.bins[d], 1u);
-      }
-    }
-  }
-  __syncthreads();
-  {
-    uint32_t v = 0, inc = 0;
-    if (tid < TR_DIGITS) {
-      v = L.bins[tid];
-      inc = tr_wave_inclusive_scan(v, lane);
-      if (lane == GS_WAVE - 1) L.scan[wave] = inc;
-    }
-    __syncthreads();
-    if (tid < TR_DIGITS) {
-      uint32_t before = 0;
-#pragma unroll
-      for (int w = 0; w < TR_DIGITS / GS_WAVE; w++)
-        if (w < wave) before += L.scan[w];
-      L.bins[tid] = before + inc - v;
-      L.first[tid] = before + inc - v;  // where the bin's next record goes
-      if (tid == TR_DIGITS - 1) L.bins[TR_DIGITS] = before + inc;
-    }
-    __syncthreads();
-  }
-  for (uint32_t i0 = 0; i0 < n; i0 += THREADS * SWEEP) {
-    TileRecord r[SWEEP];
-#pragma unroll
-    for (int u = 0; u < SWEEP; u++) {
-      const uint32_t i = i0 + (uint32_t)u * THREADS + (uint32_t)tid;
-      r[u] = i < n ? records[start + i] : make_uint4(0u, 0u, dmin, 0u);
-    }
-#pragma unroll
-    for (int u = 0; u < SWEEP; u++) {
-      const uint32_t i = i0 + (uint32_t)u * THREADS + (uint32_t)tid;
-      if (i < n) parted[start + atomicAdd((uint32_t*)&L.first[(r[u].z - dmin) >> shift], 1u)] = r[u];
-    }
-  }
-  __syncthreads();  // (the moved records are read back by this workgroup only: see sort_blocked)
-  uint32_t g0 = 0;
-  while (g0 < (uint32_t)TR_DIGITS) {
-    const uint32_t first = L.bins[g0];
-    uint32_t g1 = g0 + 1u;
-    while (g1 < (uint32_t)TR_DIGITS && L.bins[g1 + 1u] - first <= blk) g1++;
-    const uint32_t cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)(L.bins[g1] - first));
-    g0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)g1);
-    if (cnt == 0u) continue;
-    if (cnt <= blk)
-      sort_resident<WAVES, ITEMS>(tile, start + first, cnt, parted, keys, emission, point_list, L);
-    else
-      sort_blocked<WAVES, ITEMS>(tile, start + first, cnt, blk, parted, ping, pong, keys, emission, point_list, L);
-    __syncthreads();
-  }
-}
-
-// tile_list[0 .. *list_count) (walked with `step` = +1 or -1 from `tile_list`): the tiles this kernel sorts.  The
-// lists that are split before they are sorted (more than block_limit records; the larger kernel only) are also
-// entered in a list of their own, list_count[1] tiles from list_count + 2.  Such a list takes several times as long
-// as the others, a CU holds one workgroup, and workgroups start in the order of their numbers: while there are
-// fewer of them than CUs, they are taken first, so that the long jobs start at once and the short ones fill the
-// gaps behind them (a view with 54 such lists among 900: 292 -> 250 us).  With more of them than CUs the tiles'
-// own order, a mix of both kinds, is kept: all long jobs first then sweep their lists at the same time, bound by
-// memory in that phase and idle in the next (3 % slower), and any order that starts some of them late is worse.
+// tile_list[0 .. *list_count) (walked with `step` = +1 or -1 from `tile_list`): the tiles this kernel sorts.  The lists of
+// more than block_limit records (the larger kernel's only) are split already (split_list): list_count[1] of them, with at
+// most list_count[2] groups, and from list_count + 3 on (tile | groups << 16), the groups' first places in the list's
+// list_words.  Their groups are jobs like the unsplit lists, and come first: the first group of every
+// list, then the second ones, ..., whatever list is the longest.
 template <int WAVES, int ITEMS>
 __global__ void __launch_bounds__(WAVES * GS_WAVE) __attribute__((amdgpu_waves_per_eu(4)))
 tile_radix_sort_kernel(const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ tile_list, int step,
                        const uint32_t* __restrict__ list_count, uint32_t count_shift, uint32_t block_limit,
-                       const TileRecord* __restrict__ records, TileRecord* parted, uint64_t* ping, uint64_t* pong,
-                       uint64_t* keys, uint32_t* emission, uint32_t* point_list,
+                       const TileRecord* __restrict__ records, const TileRecord* __restrict__ parted,
+                       const uint32_t* __restrict__ list_words, uint64_t* ping, uint64_t* pong, uint64_t* keys, uint32_t* emission, uint32_t* point_list,
                        const uint32_t* __restrict__ fits_word) {
   extern __shared__ uint64_t s_tile_radix[];
   if (fits_word != nullptr && *fits_word == 0u) return;  // launched ahead of the host's decision: see the scatter
   const TileRadixLds<WAVES, ITEMS> L((lds_u64*)s_tile_radix);
-  const uint32_t split = (WAVES == 16 && list_count[1] <= 256u) ? list_count[1] : 0u;  // taken first
-  const uint32_t count = ((*list_count >> count_shift) & 0xFFFFu) + split;
+  const uint32_t split = WAVES == 16 ? list_count[1] : 0u;
+  const uint32_t groups = split != 0u ? split * list_count[2] : 0u;
+  const uint32_t count = ((*list_count >> count_shift) & 0xFFFFu) + groups;
   uint32_t blk = block_limit < (uint32_t)TileRadixLds<WAVES, ITEMS>::BLOCK ? block_limit
                                                                            : (uint32_t)TileRadixLds<WAVES, ITEMS>::BLOCK;
   if (blk == 0u) blk = 1u;
   for (uint32_t li = blockIdx.x; li < count; li += gridDim.x) {
-    const uint32_t t = li < split ? list_count[2u + li] : tile_list[(int)(li - split) * step];
-    const uint32_t start = ranges[2 * t];
-    const uint32_t n = ranges[2 * t + 1] - start;
-    if (n == 0u || (li >= split && split != 0u && n > blk)) continue;  // (the latter: done as one of the first)
+    uint32_t t, start, n;
+    const TileRecord* from = records;
+    if (WAVES == 16 && li < groups) {
+      const uint32_t g = li / split, entry = list_count[3u + (li - g * split)];
+      if (g >= entry >> 16) continue;
+      t = entry & 0xFFFFu;
+      const uint32_t* const firsts = list_words + ranges[2 * t];
+      const uint32_t size = ranges[2 * t + 1] - ranges[2 * t];
+      start = firsts[g];
+      n = (g + 1u < entry >> 16 ? firsts[g + 1u] : size) - start;
+      if (n == 0u) continue;
+      start += ranges[2 * t];
+      from = parted;
+    } else {
+      t = tile_list[(int)(li - groups) * step];
+      start = ranges[2 * t];
+      n = ranges[2 * t + 1] - start;
+      if (n == 0u || n > blk) continue;  // (the latter: sorted as its groups)
+    }
     if (n <= blk)
-      sort_resident<WAVES, ITEMS>(t, start, n, records, keys, emission, point_list, L);
+      sort_resident<WAVES, ITEMS>(t, start, n, from, keys, emission, point_list, L);
     else if constexpr (WAVES == 16)
-      sort_partitioned<WAVES, ITEMS>(t, start, n, blk, records, parted, ping, pong, keys, emission, point_list, L);
-    __syncthreads();  // the next tile overwrites the LDS the last step has been reading
+      sort_blocked<WAVES, ITEMS>(t, start, n, blk, from, ping, pong, keys, emission, point_list, L);
+    __syncthreads();  // the next job overwrites the LDS the last step has been reading
   }
 }
 
@@ -702,12 +606,12 @@ int tile_radix_block_records() { return TileRadixLds<16, 16>::BLOCK; }
 // Sorts the tiles of the two lists the ranges kernel of the counting sort made: `mid` lists (ascending from
 // tile_lists[0], their number in the low half of *counts) by workgroups of 8 waves that hold up to 4096 records,
 // `long` lists (descending from tile_lists[T - 1], their number in the high half) by workgroups of 16 waves that
-// hold up to 16384 records; a longer list (or one beyond block_limit records, at most 16384) is first split by its
-// leading depth bits into `parted` (16 bytes per instance), and a part that is still too long goes block by block
+// hold up to 16384 records; a longer list (or one beyond block_limit records, at most 16384) lies in `parted` (16
+// bytes per instance) in groups (list_words), and a group that is still too long goes block by block
 // through `ping` (which may be `keys`) and `pong` (8 bytes per instance each).
 int launch_tile_radix_sort(int T, bool mid, bool lng, const uint32_t* ranges, const uint32_t* tile_lists,
-                           const uint32_t* counts, uint32_t block_limit, const void* records, void* parted,
-                           uint64_t* ping, uint64_t* pong, uint64_t* keys, uint32_t* emission, uint32_t* point_list,
+                           const uint32_t* counts, uint32_t block_limit, const void* records, const void* parted,
+                           const uint32_t* list_words, uint64_t* ping, uint64_t* pong, uint64_t* keys, uint32_t* emission, uint32_t* point_list,
                            const uint32_t* fits_word, hipStream_t stream) {
   if (T <= 0) return 0;
   // more than 64 KB of dynamic LDS has to be asked for, once per device
@@ -730,12 +634,12 @@ int launch_tile_radix_sort(int T, bool mid, bool lng, const uint32_t* ranges, co
   const uint32_t mid_block = Mid::BLOCK;
   if (mid)
     hipLaunchKernelGGL((tile_radix_sort_kernel<8, 8>), dim3(T < 2048 ? T : 2048), dim3(8 * GS_WAVE), mid_lds, stream,
-                       ranges, tile_lists, 1, counts, 0u, mid_block, (const TileRecord*)records, (TileRecord*)parted,
-                       ping, pong, keys, emission, point_list, fits_word);
+                       ranges, tile_lists, 1, counts, 0u, mid_block, (const TileRecord*)records, (const TileRecord*)parted,
+                       list_words, ping, pong, keys, emission, point_list, fits_word);
   if (lng)
     hipLaunchKernelGGL((tile_radix_sort_kernel<16, 16>), dim3(T < 1024 ? T : 1024), dim3(16 * GS_WAVE), long_lds,
                        stream, ranges, tile_lists + (T - 1), -1, counts, 16u, block_limit, (const TileRecord*)records,
-                       (TileRecord*)parted, ping, pong, keys, emission, point_list, fits_word);
+                       (const TileRecord*)parted, list_words, ping, pong, keys, emission, point_list, fits_word);
   return 0;
 }
 
