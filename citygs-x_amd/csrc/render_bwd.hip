@@ -61,7 +61,10 @@
 // us for 300 k without geometry channels.  Four workgroups a CU with 64 slots, or
 // five with 48: 464 and 522 us at 4 M with geometry channels, whose 118 registers
 // do not fit five; without them 56 slots and five (96 us against 106).  The
-// accumulators' reads a pass ahead of their use gain nothing.
+// accumulators' reads a pass ahead of their use gain nothing.  The list words a pass
+// ahead and the Gaussians' numbers in the ring (at 60 slots): 463 -> 450 us at 4 M,
+// 467 -> 457 at street level, where the longest tiles' chains decide; at 1 M the same.
+// The records' places asked for before the walk: 473.
 // The matrix cores take what contracts an operand that all
 // entries or all pixels share; the recurrence itself is a serial chain per
 // pixel.
@@ -123,8 +126,12 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   const float4* packed = (packed_records != nullptr && (packed_valid == nullptr || *packed_valid != 0u))
                              ? packed_records : nullptr;
   constexpr bool render_geo = RENDER_GEO;
+  // Which Gaussian a position holds is fetched with the position's hit word and waits beside it: a window's staging then has
+  // one trip to memory in its chain, not two.  It takes the LDS of four slots a wave.  (Without channels, five workgroups a
+  // CU, it costs more than it saves: 300 k 101 us, 108 so.)
+  constexpr bool GAUSSIANS_WAIT = RENDER_GEO;
   // The Gaussians a wave can stage at a time: as many as the LDS holds with four or five workgroups.
-  constexpr int SLOTS = RENDER_GEO ? 64 : 56;
+  constexpr int SLOTS = RENDER_GEO ? 60 : 56;
   constexpr int LIST_BYTES = SLOTS + RUN;  // a row's list: its entries, and what keeps the places of a run that began earlier
   static_assert(SLOTS <= GS_WAVE && SLOTS % GROUP == 0 && LIST_BYTES % GROUP == 0, "a lane per slot, whole words of lists");
   static_assert(LIST_BYTES <= 2 * GS_WAVE, "a wave clears its four lists in two rounds");
@@ -142,6 +149,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   // the Gaussians that wait to be staged: position in the list, blocks touched
   __shared__ int s_pend[PENDING];
   __shared__ uint16_t s_pend_hits[PENDING];
+  __shared__ uint32_t s_pend_gaussian[GAUSSIANS_WAIT ? PENDING : 1];
   __shared__ int s_found[2][WAVES];
   // which slot each wave has given a Gaussian of the window (byte w of a word: wave w's, or NO_SLOT); a wave's own slots:
   // place in the window, rows touched << 8; how much of the window the wave has slots for
@@ -297,6 +305,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
   // 0.45 us of a chain that decides how long the kernel takes.  10 M Gaussians at street level, lists up to 22 k entries, two
   // pairs of views: 569 and 867 us a launch so, 551 and 829 now)
   uint32_t hits_next = HITS ? hits_at(unscanned - 1 - tid) : 0u;
+  auto gaussian_at = [&](int pos) { return GAUSSIANS_WAIT && pos >= 0 ? point_list[range.x + (uint32_t)pos] : 0u; };
+  uint32_t gaussian_next = gaussian_at(unscanned - 1 - tid);
   uint32_t carried[4] = {0u, 0u, 0u, 0u}, carried_run = 0xFFFFFFFFu;  // see `aligned` below
   for (;;) {
     while (tail - head < (uint32_t)WINDOW && unscanned > 0) {
@@ -304,6 +314,8 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
       uint32_t hits = HITS ? hits_from_bytes(hits_next) : hits_by_test(pos);
       unscanned = max(unscanned - GS_TILE_PIX, 0);
       if (HITS) hits_next = hits_at(unscanned - 1 - tid);
+      const uint32_t gaussian = gaussian_next;
+      gaussian_next = gaussian_at(unscanned - 1 - tid);
 #pragma unroll
       for (int w = 0; w < WAVES; w++) {
         const int4 last = s_row_last[w];
@@ -327,6 +339,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)take_m, 0u))) &
                             (PENDING - 1);
         s_pend[at] = pos;
+        if (GAUSSIANS_WAIT) s_pend_gaussian[at] = gaussian;
         s_pend_hits[at] = (uint16_t)hits;
       }
       parity ^= 1u;  // (the counts are rewritten two barriers later)
@@ -368,7 +381,7 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
       const uint32_t nibble = have ? own >> 8 : 0u;
       bool is_thin = false;
       if (have) {
-        const uint32_t g = point_list[range.x + (uint32_t)pos];
+        const uint32_t g = GAUSSIANS_WAIT ? s_pend_gaussian[(head + (own & 255u)) & (PENDING - 1)] : point_list[range.x + (uint32_t)pos];
         // A Gaussian's operands: one 64-byte record where the forward call packed them (a single line of memory,
         // every byte of it used), else gathered from the four arrays.  (Each route loads and then stages by itself:
         // with the loaded values merged across the two routes the compiler splits the gathers into single words.)
@@ -468,9 +481,11 @@ render_bwd_kernel(const uint2* __restrict__ ranges, const uint32_t* __restrict__
         carried_run = last_run;
       }
       sync_wave();
+      uint32_t word_next = s_idx[wave][row][0];  // (read a pass ahead: the head of a pass is a chain of LDS reads)
       for (uint32_t n = 0; n < passes; n += GROUP) {
         // Four entries of every row's list.  Lane e of each of the row's quads fetches entry e.
-        const uint32_t word = s_idx[wave][row][n / GROUP];
+        const uint32_t word = word_next;
+        word_next = s_idx[wave][row][min(n / GROUP + 1u, (uint32_t)LIST_BYTES / 4u - 1u)];
         const uint32_t j_own = __builtin_amdgcn_ubfe(word, quad_shift, 8u);
         const float4 xyp = s_xyp[wave][j_own];
         const float4 co = s_co[wave][j_own];

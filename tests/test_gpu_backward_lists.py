@@ -185,3 +185,21 @@ def test_results_of_a_large_view_are_streamed(H, orc, P, geo):
         assert large[k].shape[0] == P
         assert torch.equal(large[k][index], small[k]), k
         assert not large[k][half:P - (n - half)].any(), k
+
+
+# With the geometry channels a wave has 60 slots: windows that hold one Gaussian less, as many and one more.  (With three in
+# ten of them small, 59 and 61 are not the view that _covering_view wants.)
+@pytest.mark.parametrize("n,small", [(59, 0.0), (60, 0.0), (61, 0.0), (58, 0.3), (60, 0.3), (62, 0.3), (119, 0.3), (120, 0.0),
+                                     (120, 0.3), (121, 0.3), (181, 0.3)])
+def test_sixty_slots(H, orc, n, small):
+    run, reference, is_thin = _covering_view(H, orc, n, small)
+    got, ref = run(True), reference(True)
+    # the bound of test_list_lengths (561 pixels here)
+    for k, want in (("dL_dmeans2D", ref["dL_dmeans2D"][:, :2]), ("dL_dmeans2D_abs", ref["dL_dmeans2D_abs"]),
+                    ("dL_dconic_opacity", ref["dL_dconic_opacity"]), ("dL_dcolors", ref["dL_dcolors"]),
+                    ("dL_dall_map", ref["dL_dall_map"])):
+        assert H.rel_l2(got[k].cpu().numpy(), want) <= 1e-4, (k, H.rel_l2(got[k].cpu().numpy(), want))
+    a, b = run(True, 0.0), run(False, 0.0)
+    thin = torch.from_numpy(is_thin).to(H.DEV)
+    for k in ("dL_dmeans2D", "dL_dmeans2D_abs", "dL_dconic_opacity"):
+        assert torch.equal(a[k][thin], b[k][thin]), k
