@@ -343,14 +343,14 @@ int gs_preprocess_forward(float* means2D, float* depths, int* radii, float* cov3
                                         dcolor_ddir, blend_records, nullptr, stream);
 }
 
-int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
-                                    int width, int height, const float* means3D, const float* scales, const float* rotations,
-                                    const float* shs, float scale_modifier, const float* viewmatrix, const float* projmatrix,
-                                    const float* campos, float tan_fovx, float tan_fovy, const float* dL_dmean2D,
-                                    int mean2D_stride, const float* dL_dconic_opacity, const float* dL_dcolor,
-                                    float* dL_dmean3D, float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
-                                    float* dL_dopacity, int debug, const float* dcolor_ddir, const float* dL_dall_map,
-                                    gs_stream_t stream) {
+int gs_preprocess_rows_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
+                                int width, int height, const float* means3D, const float* scales, const float* rotations,
+                                const float* shs, float scale_modifier, const float* viewmatrix, const float* projmatrix,
+                                const float* campos, float tan_fovx, float tan_fovy, const float* dL_dmean2D,
+                                int mean2D_stride, const float* dL_dconic_opacity, const float* dL_dcolor,
+                                float* dL_dmean3D, float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
+                                float* dL_dopacity, int debug, const float* dcolor_ddir, const float* dL_dall_map,
+                                float* zero_rows, gs_stream_t stream) {
   GS_REQUIRE(P >= 0 && width > 0 && height > 0, "gs_preprocess_backward: bad sizes");
   if (P == 0) return 0;
   GS_REQUIRE(radii && means3D && viewmatrix && projmatrix && dL_dmean2D && dL_dconic_opacity && dL_dmean3D,
@@ -365,6 +365,7 @@ int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const 
   GS_REQUIRE(dL_dall_map == nullptr || (scales && rotations && campos),
              "gs_preprocess_backward: dL_dall_map needs scales, rotations and campos");
   PreprocessBwdArgs a;
+  a.zero_rows = zero_rows;
   a.P = P; a.D = D; a.M = sh_mode ? M : 0; a.W = width; a.H = height;
   a.means3D = means3D; a.radii = radii; a.shs = sh_mode ? shs : nullptr; a.clamped = clamped;
   a.dcolor_ddir = sh_mode ? dcolor_ddir : nullptr;
@@ -381,6 +382,20 @@ int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const 
     launch_preprocess_bwd(a, (hipStream_t)stream);
   }
   return check_launch("preprocess_backward", (hipStream_t)stream, debug != 0);
+}
+
+int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
+                                    int width, int height, const float* means3D, const float* scales, const float* rotations,
+                                    const float* shs, float scale_modifier, const float* viewmatrix, const float* projmatrix,
+                                    const float* campos, float tan_fovx, float tan_fovy, const float* dL_dmean2D,
+                                    int mean2D_stride, const float* dL_dconic_opacity, const float* dL_dcolor,
+                                    float* dL_dmean3D, float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh,
+                                    float* dL_dopacity, int debug, const float* dcolor_ddir, const float* dL_dall_map,
+                                    gs_stream_t stream) {
+  return gs_preprocess_rows_backward(radii, cov3D, clamped, P, D, M, width, height, means3D, scales, rotations, shs,
+                                     scale_modifier, viewmatrix, projmatrix, campos, tan_fovx, tan_fovy, dL_dmean2D,
+                                     mean2D_stride, dL_dconic_opacity, dL_dcolor, dL_dmean3D, dL_dcov3D, dL_dscale, dL_drot,
+                                     dL_dsh, dL_dopacity, debug, dcolor_ddir, dL_dall_map, nullptr, stream);
 }
 
 int gs_preprocess_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
@@ -489,6 +504,8 @@ int pending_fault(const char* who) {
 struct TileSortLimits {
   int small, block;
 };
+// The size of gs_render_options without clear_geo_images.
+constexpr size_t OPTIONS_WITH_RECORDS = offsetof(gs_render_options, clear_geo_images);
 // The defaults, or what the caller's options ask for: the list length up to which a list is sorted in registers
 // (0: the view takes the radix sort over all its keys), and the number of records the per-tile radix sort holds
 // in one block (longer lists are sorted block by block through memory).
@@ -533,7 +550,12 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   // The blend kernels' operand records: the caller's (complete: gs_preprocess_forward and gs_all_map_forward wrote
   // their parts), or packed here for a view with enough instances per Gaussian.
   const float* caller_records =
-      (options != nullptr && options->struct_bytes >= sizeof(gs_render_options)) ? options->blend_records : nullptr;
+      (options != nullptr && options->struct_bytes >= OPTIONS_WITH_RECORDS) ? options->blend_records : nullptr;
+  const bool clear_geo = render_geo == 0 && options != nullptr && options->struct_bytes >= sizeof(gs_render_options) &&
+                         options->clear_geo_images != 0;
+  GS_REQUIRE(!clear_geo || (out_all_map && out_plane_depth), "gs_render_forward: no images to clear");
+  GS_REQUIRE(!clear_geo || (((uintptr_t)out_all_map | (uintptr_t)out_plane_depth) & 15u) == 0u,
+             "gs_render_forward: the images to clear must be 16-byte aligned");
   GS_REQUIRE(((uintptr_t)caller_records & 15u) == 0u, "gs_render_forward: blend_records must be 16-byte aligned");
   const GeometryLayout GL = geometry_layout(P);
   char* gbase = geometryBuffer(GL.total, geometry_user);
@@ -571,23 +593,27 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   int64_t cap_n = 0;
   uint32_t cap_longest = 0;
   if (bucketed && !dbg && result != nullptr && result->struct_bytes >= sizeof(gs_render_result) &&
-      options != nullptr && options->struct_bytes >= sizeof(gs_render_options) && options->expected_instances > 0) {
+      options != nullptr && options->struct_bytes >= OPTIONS_WITH_RECORDS && options->expected_instances > 0) {
     cap_n = options->expected_instances < (int64_t)GS_MAX_INSTANCES ? options->expected_instances
                                                                      : (int64_t)GS_MAX_INSTANCES;
     // (0: any length; the sort kernels launched and their LDS depend on it)
     cap_longest = options->expected_longest_list > 0 ? (uint32_t)options->expected_longest_list : GS_MAX_INSTANCES;
   }
   const bool ahead = cap_n > 0;
+  const uint64_t image = clear_geo ? (uint64_t)width * height : 0u;
+  const ClearedArrays cleared = {{out_all_map, out_plane_depth}, {GS_N_MAP * image, image}};
 
   if (bucketed) {
     StageScope _t("tile_count", stream);
     // the histogram's grand total is the instance count: the host gets it from here
     if (launch_bucket_count(P, width, height, radii, means2D, compute_locally, tiles_touched, bucket_table, ranges,
                             sort_limit, (uint32_t)limits.block, total_slot, out_observe, (uint32_t)cap_n, cap_longest,
-                            packed_valid, stream))
+                            packed_valid, cleared, stream))
       return 1;
   } else {
     StageScope _t("tile_count", stream);
+    for (int k = 0; k < 2; k++)
+      launch_fill_u32((int64_t)cleared.floats[k], 0u, reinterpret_cast<uint32_t*>(cleared.data[k]), stream);
     // also clears the tile ranges (cudaMemset of CR/rasterizer_impl.cu:687), which nothing reads before
     // identify_tile_ranges fills them
     launch_fill_u32(2, 0u, packed_valid, stream);
@@ -660,8 +686,8 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     a.means2D = means2D; a.rgb = rgb; a.all_map = all_map; a.conic_opacity = conic_opacity;
     a.compute_locally = compute_locally; a.bg = background; a.render_geo = render_geo;
     a.final_T = accum_alpha; a.n_contrib_px = n_contrib_px; a.n_contrib2loss_px = n_contrib2loss_px;
-    a.out_color = out_color; a.out_observe = out_observe; a.out_all_map = out_all_map;
-    a.out_plane_depth = out_plane_depth;
+    a.out_color = out_color; a.out_observe = out_observe;
+    a.out_all_map = out_all_map; a.out_plane_depth = out_plane_depth;
     a.depths = depths; a.out_max_weight_depth = out_max_weight_depth;
     a.n_render = n_render; a.n_consider = n_consider; a.n_contrib_tile = n_contrib;
     a.fits_word = ahead_of_host ? bucket_fits_word(bucket_table, T) : nullptr;
@@ -1402,8 +1428,8 @@ int gs_render_tiles_forward(int P, int width, int height, float focal_x, float f
   a.means2D = means2D; a.rgb = rgb; a.all_map = all_map; a.conic_opacity = conic_opacity;
   a.compute_locally = compute_locally; a.bg = background; a.render_geo = render_geo;
   a.final_T = final_T; a.n_contrib_px = n_contrib_px; a.n_contrib2loss_px = n_contrib2loss_px;
-  a.out_color = out_color; a.out_observe = out_observe; a.out_all_map = out_all_map;
-  a.out_plane_depth = out_plane_depth;
+  a.out_color = out_color; a.out_observe = out_observe;
+  a.out_all_map = out_all_map; a.out_plane_depth = out_plane_depth;
   a.n_render = n_render; a.n_consider = n_consider; a.n_contrib_tile = n_contrib;
   launch_render_fwd(a, (hipStream_t)stream);
   return check_launch("render_tiles_forward", (hipStream_t)stream, false);

@@ -46,6 +46,7 @@ struct PreprocessBwdArgs {
   float *dL_dmean3D, *dL_dcov3D /*optional*/, *dL_dsh /*optional*/, *dL_dscale, *dL_drot, *dL_dopacity /*optional*/;
   const float* dcolor_ddir = nullptr;  // optional: what the forward kernel left (PreprocessFwdArgs::dcolor_ddir)
   const float* dL_dall_map = nullptr;  // optional (P,5): gradient of the channels (PreprocessFwdArgs::all_map)
+  float* zero_rows = nullptr;          // optional (P,3): receives zeros
 };
 
 // Brackets a stage with an event pair on its stream while stage timing is enabled (gs_stage_timing_enable; the
@@ -107,11 +108,15 @@ size_t bucket_table_bytes(int T);
 // holds in one block, see launch_tile_sort.
 // cap_instances / cap_longest: what kernels launched ahead of the host's decision were sized for; the ranges kernel
 // leaves 1 in bucket_fits_word(table) if the view has at most that many instances and no longer list, else 0.
-// clear_word: two words the ranges kernel clears
+// clear_word: two words the ranges kernel clears; cleared: two arrays, on 16-byte boundaries, that are cleared beside it
+struct ClearedArrays {
+  float* data[2];
+  uint64_t floats[2];
+};
 int launch_bucket_count(int P, int W, int H, const int* radii, const float* means2D, const uint8_t* compute_locally,
                         uint32_t* tiles_touched, void* table, uint32_t* ranges, uint32_t small_limit,
                         uint32_t block_limit, uint32_t* host_words, int* zero_per_gaussian, uint32_t cap_instances,
-                        uint32_t cap_longest, uint32_t* clear_word, hipStream_t stream);
+                        uint32_t cap_longest, uint32_t* clear_word, const ClearedArrays& cleared, hipStream_t stream);
 const uint32_t* bucket_fits_word(const void* table, int T);
 // records: one 16-byte record (Gaussian, emission index, depth bits, 0) per instance, grouped by tile in any
 // order.  Also writes point_offsets (the inclusive prefix sum of tiles_touched).

@@ -696,7 +696,8 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
                       const float4* __restrict__ dL_dconic_opacity, const float* __restrict__ dL_dcolor,
                       float* __restrict__ dL_dmean3D, float* __restrict__ dL_dcov3D_out, float* __restrict__ dL_dsh,
                       float* __restrict__ dL_dscale, float* __restrict__ dL_drot, float* __restrict__ dL_dopacity,
-                      const float* __restrict__ dcolor_ddir, const float* __restrict__ dL_dall_map) {
+                      const float* __restrict__ dcolor_ddir, const float* __restrict__ dL_dall_map,
+                      float* __restrict__ zero_rows) {
   // (SAVED stages sixteen rows at a time: all rows of a wave would take 53 KB and leave three waves per SIMD, which cost
   // 10 us of 87 at 1 M Gaussians and 85 of 765 at 10 M)
   constexpr int STORE_ROWS = SAVED ? GS_WAVE / 4 : GS_WAVE;
@@ -994,6 +995,11 @@ preprocess_bwd_kernel(int P, int D, int M, const float* __restrict__ means, cons
   float* const lds = reinterpret_cast<float*>(s_rows[wave]);
   wave_rows_turn_store<3>(dL_dmean3D + 3 * wave_first, rows, gm, lds, lane);
   if (dL_dscale) wave_rows_turn_store<3>(dL_dscale + 3 * wave_first, rows, gs_, lds, lane);
+  if (zero_rows != nullptr) {
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      if (j * GS_WAVE + lane < 3 * rows) zero_rows[3 * wave_first + j * GS_WAVE + lane] = 0.f;
+  }
   if (!in_range) return;
   if (FIRST && dL_dopacity) dL_dopacity[i] = gco.w;  // passthrough, rasterize_points.cu:191-194
   if (dL_drot) reinterpret_cast<float4*>(dL_drot)[i] = make_float4(gq[0], gq[1], gq[2], gq[3]);
@@ -1066,7 +1072,7 @@ int launch_preprocess_bwd(const PreprocessBwdArgs& a, hipStream_t stream) {
                        a.clamped, a.scales, a.rotations, a.scale_modifier, a.cov3D, a.viewmatrix, a.projmatrix,
                        a.campos, h_x, h_y, a.tanx, a.tany, a.dL_dmean2D, a.mean2D_stride,
                        (const float4*)a.dL_dconic_opacity, a.dL_dcolor, a.dL_dmean3D, a.dL_dcov3D, a.dL_dsh,
-                       a.dL_dscale, a.dL_drot, a.dL_dopacity, a.dcolor_ddir, a.dL_dall_map);
+                       a.dL_dscale, a.dL_drot, a.dL_dopacity, a.dcolor_ddir, a.dL_dall_map, a.zero_rows);
   };
   // (see FIRST at the kernel)
   if (a.dL_dall_map != nullptr) {

@@ -142,7 +142,7 @@ py::tuple preprocess_backward(const Tensor& radii, const OptTensor& cov3D_, cons
   const Options o(means3D.device());
   const c10::DeviceGuard guard(means3D.device());
   const int64_t M = sh_mode ? sh->size(1) : 0;
-  Tensor dL_dsh = sh_mode ? at::empty({P, M, 3}, o.f32) : at::zeros({P, 3}, o.f32);
+  Tensor dL_dsh = sh_mode ? at::empty({P, M, 3}, o.f32) : at::empty({P, 3}, o.f32);  // (the latter: zeros)
   Tensor dmeans = at::empty({P, 3}, o.f32), dscales = at::empty({P, 3}, o.f32), drot = at::empty({P, 4}, o.f32),
          dopacity = at::empty({P, 1}, o.f32);
   const Tensor g2 = f32c(dL_dmeans2D, "dL_dmeans2D"), gco = f32c(dL_dconic_opacity, "dL_dconic_opacity");
@@ -156,12 +156,13 @@ py::tuple preprocess_backward(const Tensor& radii, const OptTensor& cov3D_, cons
   int status;
   {
     py::gil_scoped_release nogil;
-    status = gs_preprocess_channels_backward(
+    status = gs_preprocess_rows_backward(
         ptr<int>(rad), ptr(cov3D), ptr<uint8_t>(cl), (int)P, degree, (int)M, width, height, ptr(means3D), ptr(scales),
         ptr(rotations), ptr(shc), scale_modifier, ptr(vm), ptr(pm), ptr(cp), tan_fovx, tan_fovy, ptr(g2),
         (int)g2.size(1), ptr(gco), ptr(gcol), ptr(dmeans), nullptr, ptr(dscales), ptr(drot),
         sh_mode ? ptr(dL_dsh) : nullptr, ptr(dopacity), debug,
-        sh_mode && dcolor_ddir.has_value() ? ptr(*dcolor_ddir) : nullptr, ptr(gmap), stream_of(stream));
+        sh_mode && dcolor_ddir.has_value() ? ptr(*dcolor_ddir) : nullptr, ptr(gmap),
+        sh_mode ? nullptr : ptr(dL_dsh), stream_of(stream));
   }
   check(status, "preprocess_gaussians_backward");
   return py::make_tuple(dmeans, dscales, drot, dL_dsh, dopacity);
@@ -226,8 +227,8 @@ py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& m
   const Tensor am = geo ? f32c(*all_map, "all_map") : Tensor();
   check_rows(blend_records, "blend_records", means2D, {P, 16});
   Tensor color = at::empty({CHANNELS, H, W}, o.f32), observe = at::empty({P}, o.i32);
-  Tensor map = geo ? at::empty({MAP_CHANNELS, H, W}, o.f32) : at::zeros({MAP_CHANNELS, H, W}, o.f32);
-  Tensor depth = geo ? at::empty({1, H, W}, o.f32) : at::zeros({1, H, W}, o.f32);
+  // (zeros without geometry channels, cleared in the call)
+  Tensor map = at::empty({MAP_CHANNELS, H, W}, o.f32), depth = at::empty({1, H, W}, o.f32);
   Tensor n_render = at::empty({tiles}, o.i32), n_consider = at::empty({tiles}, o.i32),
          n_contrib = at::empty({tiles}, o.i32);
   Tensor mwd = want_max_weight_depth ? at::empty({1, H, W}, o.f32) : Tensor();
@@ -239,6 +240,7 @@ py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& m
   options.expected_longest_list = expected_longest_list;
   options.expected_instances = expected_instances;
   options.blend_records = blend_records.has_value() ? ptr(*blend_records) : nullptr;
+  options.clear_geo_images = 1;
   gs_render_result result = {};
   result.struct_bytes = sizeof(result);
   // fp32 arithmetic, as `H / (2.0f * tan_fovy)` at rasterize_points.cu:328-329

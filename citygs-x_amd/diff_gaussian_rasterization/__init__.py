@@ -206,8 +206,6 @@ class _PreprocessGaussians(torch.autograd.Function):
         P = means3D.shape[0]
         if grad_means2D is None:
             grad_means2D = means3D.new_zeros(P, 2)
-        if grad_rgb is None:
-            grad_rgb = means3D.new_zeros(P, 3)
         if grad_conic_opacity is None:
             grad_conic_opacity = means3D.new_zeros(P, 4)
         dL_dmeans3D, dL_dscales, dL_drotations, dL_dsh, dL_dopacity = _C.preprocess_gaussians_backward(

@@ -69,6 +69,8 @@ _SIGNATURES = {
                                        [_vp] * 4),
     "gs_preprocess_channels_backward": (_i, [_vp] * 3 + [_i] * 5 + [_vp] * 4 + [_f] + [_vp] * 3 + [_f, _f] +
                                         [_vp, _i] + [_vp] * 8 + [_i] + [_vp] * 3),
+    "gs_preprocess_rows_backward": (_i, [_vp] * 3 + [_i] * 5 + [_vp] * 4 + [_f] + [_vp] * 3 + [_f, _f] +
+                                    [_vp, _i] + [_vp] * 8 + [_i] + [_vp] * 4),
     "gs_render_forward": (_i, [RESIZE_FN, _vp, RESIZE_FN, _vp, RESIZE_FN, _vp, _i, _vp, _i, _i, _f, _f, _f, _f] +
                           [_vp] * 17 + [_i, _i, C.POINTER(_i), C.POINTER(_f), _vp, _vp, _vp]),
     "gs_render_backward_workspace_bytes": (_sz, [_i]),
@@ -136,7 +138,8 @@ class RenderOptions(C.Structure):
     means none."""
     _fields_ = [("struct_bytes", C.c_uint32), ("tile_sort_small_limit", C.c_int32),
                 ("tile_sort_block_records", C.c_int32), ("expected_longest_list", C.c_int32),
-                ("expected_instances", C.c_int64), ("blend_records", C.c_void_p)]
+                ("expected_instances", C.c_int64), ("blend_records", C.c_void_p), ("clear_geo_images", C.c_int32),
+                ("reserved", C.c_int32)]
 
     def __init__(self, tile_sort_small_limit=-1, tile_sort_block_records=-1, expected_instances=0,
                  expected_longest_list=0, blend_records=None):

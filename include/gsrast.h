@@ -142,6 +142,18 @@ int gs_preprocess_channels_backward(const int* radii, const float* cov3D, const 
                                     float* dL_dopacity, int debug, const float* dcolor_ddir,
                                     const float* dL_dall_map, gs_stream_t stream);
 
+/* gs_preprocess_channels_backward that also writes zeros to zero_rows (P,3), if not NULL: the gradient of colours that
+ * are not spherical-harmonics coefficients, which the reference returns as zeros. */
+int gs_preprocess_rows_backward(const int* radii, const float* cov3D, const uint8_t* clamped, int P, int D, int M,
+                                int width, int height, const float* means3D, const float* scales,
+                                const float* rotations, const float* shs, float scale_modifier,
+                                const float* viewmatrix, const float* projmatrix, const float* campos, float tan_fovx,
+                                float tan_fovy, const float* dL_dmean2D, int mean2D_stride,
+                                const float* dL_dconic_opacity, const float* dL_dcolor, float* dL_dmean3D,
+                                float* dL_dcov3D, float* dL_dscale, float* dL_drot, float* dL_dsh, float* dL_dopacity,
+                                int debug, const float* dcolor_ddir, const float* dL_dall_map, float* zero_rows,
+                                gs_stream_t stream);
+
 /* No counterpart in the reference: per-call options of gs_render_forward (NULL = all defaults).  A field below
  * zero keeps its default; struct_bytes is sizeof(gs_render_options) as the caller compiled it.
  * gs_render_forward builds the per-tile lists by bucketing the instances by tile (a counting sort) and sorting
@@ -174,6 +186,9 @@ typedef struct gs_render_options {
    * them itself when the view has more than 0.8 instances per Gaussian.  The same pointer goes to
    * gs_render_backward; the records must stay as they are until that call has run. */
   const float* blend_records;
+  /* With render_geo == 0: non-zero has out_all_map and out_plane_depth written as zeros (otherwise they are not touched). */
+  int32_t clear_geo_images;
+  int32_t reserved;
 } gs_render_options;
 
 /* What gs_render_forward reports besides the instance count (optional, NULL to skip; struct_bytes as above):
@@ -195,8 +210,8 @@ typedef struct gs_render_result {
  * -> tile ranges -> blend -> per-tile statistics.
  * out_color (3,H,W) is written in full: pixels of tiles with compute_locally == 0 read 0, as in the reference,
  * whose binding allocates the images zero-filled (rasterize_points.cu:303-307); so are out_all_map (5,H,W) and
- * out_plane_depth (1,H,W) when render_geo != 0 (they are not touched otherwise: pass them zero-filled, as the
- * reference leaves them) and out_max_weight_depth when given.  A Gaussian whose colour or geometry channels are
+ * out_plane_depth (1,H,W) when render_geo != 0 (otherwise they are zeros with gs_render_options.clear_geo_images and not
+ * touched without: pass them zero-filled then, as the reference leaves them) and out_max_weight_depth when given.  A Gaussian whose colour or geometry channels are
  * not finite reaches exactly the pixels that blend it (CR/forward.cu:381-407).
  * out_observe (P) int32 is cleared by the call
  * (the reference's binding allocates it zeroed, rasterize_points.cu:305) and then counted;
