@@ -14,6 +14,8 @@
 //
 // The weights are rearranged once per call into those per-step operand orders ("packed" buffer); the kernels
 // then read them with index step * 64 + lane.
+#include <type_traits>
+
 #include "gs_common.h"
 #include "gs_kernels.h"
 
@@ -33,6 +35,7 @@ constexpr int SG_STRIDE = 33;
 constexpr int NG_SLOT_GRADS = 11;    // pre-activation gradients per offset: 1 opacity, 3 color, 7 cov
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 __host__ __device__ constexpr int even_up(int v) { return (v + 1) & ~1; }
 __host__ __device__ constexpr int hrow(int half, int i) { return 8 * (i >> 2) + 4 * half + (i & 3); }
@@ -52,10 +55,12 @@ struct Shape {
   // row numbering shared by the output-layer weights and the output-gradient matrix: the three MLPs' output
   // units one after the other, each block padded to an even count
   static constexpr int G0 = 0, G1 = even_up(OUT0), G2 = G1 + even_up(OUT1), GROWS = G2 + even_up(OUT2);
-  static constexpr int BWD_WAVES = GROWS <= 110 ? 4 : 2;   // waves per block of the backward kernel (LDS)
+  static constexpr int BWD_PAIRS = GROWS <= 110 ? 4 : 2;   // pairs of waves per block of the backward kernel (LDS)
   __host__ __device__ static constexpr int out(int m) { return m == 0 ? OUT0 : m == 1 ? OUT1 : OUT2; }
   __host__ __device__ static constexpr int tiles(int m) { return m == 0 ? T0 : m == 1 ? T1 : T2; }
   __host__ __device__ static constexpr int first_tile(int m) { return m == 0 ? 0 : m == 1 ? T0 : T0 + T1; }
+  // whole tiles of 32 output rows; up to 16 rows past them make half a tile of their own in the weight gradients
+  __host__ __device__ static constexpr int whole_tiles(int m) { return (out(m) + 15) / 32; }
   __host__ __device__ static constexpr int grow(int m) { return m == 0 ? G0 : m == 1 ? G1 : G2; }
 };
 
@@ -170,18 +175,26 @@ __device__ __forceinline__ void unpack_x(float (&xb)[NG_W1_STEPS], float (&nv)[3
 }
 
 // relu(W1 x + b1) for the wave's 32 anchors; w1t = this MLP's [slot][WS] array
-__device__ __forceinline__ v16f hidden_layer(const float* w1t, const float (&xb)[NG_W1_STEPS], int al, int half) {
-  v16f acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+__device__ __forceinline__ void hidden_weights(float (&w)[NG_W1_STEPS], const float* w1t, int al, int half) {
   const float* lo = w1t + half * 16 * WS + al;  // slots 16 half + s
-  const float* hi = w1t + (32 + half) * WS + al;  // slots 32 + half, 34 + half
+  const float* hi = w1t + (32 + half) * WS + al;  // slots 32 + half, 34 + half, 36 + half
 #pragma unroll
-  for (int s = 0; s < 16; s++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(lo[s * WS], xb[s], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(hi[0], xb[16], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(hi[2 * WS], xb[17], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(hi[4 * WS], xb[18], acc, 0, 0, 0);
+  for (int s = 0; s < 16; s++) w[s] = lo[s * WS];
+#pragma unroll
+  for (int s = 0; s < 3; s++) w[16 + s] = hi[2 * s * WS];
+}
+__device__ __forceinline__ v16f hidden_products(const float (&w)[NG_W1_STEPS], const float (&xb)[NG_W1_STEPS]) {
+  v16f acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < NG_W1_STEPS; s++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w[s], xb[s], acc, 0, 0, 0);
 #pragma unroll
   for (int i = 0; i < 16; i++) acc[i] = acc[i] > 0.0f ? acc[i] : 0.0f;
   return acc;
+}
+__device__ __forceinline__ v16f hidden_layer(const float* w1t, const float (&xb)[NG_W1_STEPS], int al, int half) {
+  float w[NG_W1_STEPS];
+  hidden_weights(w, w1t, al, half);
+  return hidden_products(w, xb);
 }
 
 // rows [32 lt, 32 lt + 32) of W2 h + b2 of an MLP with `out` output units; w2, b2 = the MLP's first row
@@ -503,14 +516,23 @@ neural_offset_backward_kernel(int64_t N, const float* __restrict__ offsets,
 // pre-activation output gradients, and per MLP
 //   H = relu(W1 x + b1) (recomputed), dH = W2^T G, dHpre = dH where H > 0, dX += W1^T dHpre,
 //   dW2 += G H^T, [dW1 | db1] += dHpre [x | 1]^T, db2 += row sums of G,
-// the weight gradients staying in matrix-core accumulators over all tiles of the wave; they are reduced over the
-// block at the end (one partial set per block; a last kernel adds the blocks in a fixed order).  The next tile's
-// features and gradient records are requested before the current tile's products start.
+// the weight gradients staying in matrix-core accumulators over all tiles of a pair of waves; they are reduced over
+// the block at the end (one partial set per block; a last kernel adds the blocks in a fixed order).
+//
+// LDS holds the matrices of four tiles (two from 11 offsets on) beside the weights and bounds the tiles in flight, one
+// on each SIMD.  Two waves share a tile: the first makes H, dHpre, dX and the anchors' gradients, the second brings G to
+// LDS and adds to the weights' gradients, one MLP behind the first, so that each runs its products while the other
+// waits for LDS, stores or reads.  The next tile's features and records are asked for a tile ahead.  One wave for both
+// held 336 accumulator and prefetch registers and waited for each of these by itself, 48 k cycles a tile where its
+// products take 21 k; together they take 30 k, of which the products, fewer by those of half tiles, 19 k: 175 k visible
+// anchors of ten offsets 124 -> 92 us.  Of that, two waves as such 124 -> 104 (119 as long as the second one's read
+// addresses were kept in registers and spilled), half tiles 104 -> 92; operands asked for a dozen products ahead in
+// the first wave are worth 4 of these (without half tiles nothing: the second wave is the longer one there).
 template <int K>
 struct BwdLds {
   using S = Shape<K>;
   float g[S::GROWS * SG_STRIDE];
-  float hd[2 * 32 * SG_STRIDE];  // H, then dHpre; also the staging area of the final block reduction
+  float hd[2 * 32 * SG_STRIDE];  // H and dHpre of one MLP; also the staging area of the final block reduction
   float x[NG_ANCHORS * SX_STRIDE];
 };
 
@@ -521,18 +543,20 @@ __host__ __device__ constexpr int partial_floats() {
 }
 
 template <int K>
-__global__ void __launch_bounds__(64 * Shape<K>::BWD_WAVES)
+__global__ void __launch_bounds__(128 * Shape<K>::BWD_PAIRS)
 neural_mlp_backward_kernel(int64_t N, int ntiles, const float* __restrict__ anchor, const float* __restrict__ feat,
                            const float* __restrict__ level, const float* __restrict__ campos, const float* __restrict__ packed,
                            const float* __restrict__ slot_grads, float* __restrict__ d_anchor,
                            float* __restrict__ d_feat, float* __restrict__ partials) {
   using S = Shape<K>;
   constexpr PackLayout L = pack_layout(S::GROWS);
-  constexpr int NW = S::BWD_WAVES, NT = 64 * NW;
+  constexpr int NP = S::BWD_PAIRS, NT = 128 * NP;
   constexpr int B2N = (S::GROWS + 63) / 64;
   constexpr int TILE_FLOATS = NG_ANCHORS * K * NG_SLOT_GRADS;
   constexpr int NQ = (TILE_FLOATS / 4 + 63) / 64;  // float4 loads per lane and tile
-  __shared__ BwdLds<K> lds[NW];
+  constexpr int NACC = S::TILES + 4;
+  constexpr int DH_STEPS = 12;  // products whose operands are asked for together
+  __shared__ BwdLds<K> lds[NP];
   __shared__ float sW1[3 * NG_SLOTS * WS];
   __shared__ float sW2[S::GROWS * WS];
   // W1's view-direction columns (c = 0..2) and distance column (c = 3) as [m][c][h]
@@ -549,208 +573,18 @@ neural_mlp_backward_kernel(int64_t N, int ntiles, const float* __restrict__ anch
     const int row = comp == 0 ? S::G0 + j : comp < 4 ? S::G1 + 3 * j + (comp - 1) : S::G2 + 7 * j + (comp - 4);
     sWhere[e] = (unsigned short)(row * SG_STRIDE + ax);
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, al = lane & 31;
-  const float cam[3] = {campos[0], campos[1], campos[2]};
-  BwdLds<K>& W = lds[wave];
-  // rows that pad a block of G to an even count are read by the dH products and never written below
-  for (int e = lane; e < S::GROWS * SG_STRIDE; e += 64) W.g[e] = 0.0f;
-  __syncthreads();
-
-  // weight-gradient accumulators: the W2 tiles, the 32 feature columns of W1 per MLP, and one tile that holds the
-  // six remaining columns of W1 (view direction, bias, distance, level) of all three MLPs as its rows 6 m + c
-  v16f accW2[S::TILES], accW1[3], accWx;
-  float accB2[B2N];
-#pragma unroll
-  for (int t = 0; t < S::TILES; t++)
-#pragma unroll
-    for (int i = 0; i < 16; i++) accW2[t][i] = 0.0f;
-#pragma unroll
-  for (int m = 0; m < 3; m++) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) accW1[m][i] = 0.0f;
-  }
-#pragma unroll
-  for (int i = 0; i < 16; i++) accWx[i] = 0.0f;
-#pragma unroll
-  for (int q = 0; q < B2N; q++) accB2[q] = 0.0f;
-
-  const int64_t total_floats = N * K * NG_SLOT_GRADS;
-  const int stride = gridDim.x * NW;
-  int tile = blockIdx.x * NW + wave;
-  XOperand xo;
-  float4 gq[NQ];
-  float da[3] = {0.0f, 0.0f, 0.0f};  // the anchor's direct gradient, as the first kernel left it
-  auto fetch_tile = [&](int t) {
-    const int64_t a = (int64_t)t * NG_ANCHORS + al;
-    xo = fetch_x(a < N, a, half, anchor, feat, level);
-    if (a < N && half == 0) {
-#pragma unroll
-      for (int c = 0; c < 3; c++) da[c] = d_anchor[a * 3 + c];
-    }
-    const int64_t base = (int64_t)t * TILE_FLOATS;
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int e = (q * 64 + lane) * 4;
-      // the buffer is padded, so a float4 that straddles the end is readable; its tail is dropped below
-      gq[q] = (e < TILE_FLOATS && base + e < total_floats) ? *(const float4*)(slot_grads + base + e)
-                                                           : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-  };
-  if (tile < ntiles) fetch_tile(tile);
-  for (; tile < ntiles; tile += stride) {
-    const int64_t a = (int64_t)tile * NG_ANCHORS + al;
-    const bool valid = a < N;
-    float nv[3], dist;
-    const float da_now[3] = {da[0], da[1], da[2]};
-    {
-      float xb[NG_W1_STEPS];
-      unpack_x(xb, nv, dist, xo, valid, half, cam);
-#pragma unroll
-      for (int s = 0; s < NG_W1_STEPS; s++) W.x[al * SX_STRIDE + xslot(half, s)] = xb[s];
-      const int64_t left = total_floats - (int64_t)tile * TILE_FLOATS;
-      const int nvalid = left < TILE_FLOATS ? (int)left : TILE_FLOATS;  // floats of this tile that exist
-#pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const int e = (q * 64 + lane) * 4;
-        if (e < TILE_FLOATS) {
-          const float v[4] = {gq[q].x, gq[q].y, gq[q].z, gq[q].w};
-#pragma unroll
-          for (int c = 0; c < 4; c++) W.g[sWhere[e + c]] = e + c < nvalid ? v[c] : 0.0f;
-        }
-      }
-    }
-    wave_sync();
-
-    v16f dxf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // this half's share of the gradient of the view direction (0..2) and of the distance (3)
-    float dv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const float* xrow = W.x + al * SX_STRIDE;
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-      // the next tile's loads go out before the last and longest MLP, late enough to keep their registers
-      // free until then and early enough to land behind its products
-      if (m == 2 && tile + stride < ntiles) fetch_tile(tile + stride);
-      const float* w1t = sW1 + m * NG_SLOTS * WS;
-      v16f h = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-      {
-        const float* lo = w1t + half * 16 * WS + al;
-        const float* hi = w1t + (32 + half) * WS + al;
-#pragma unroll
-        for (int s = 0; s < 16; s++) h = __builtin_amdgcn_mfma_f32_32x32x2f32(lo[s * WS], xrow[16 * half + s], h, 0, 0, 0);
-        h = __builtin_amdgcn_mfma_f32_32x32x2f32(hi[0], xrow[32 + half], h, 0, 0, 0);
-        h = __builtin_amdgcn_mfma_f32_32x32x2f32(hi[2 * WS], xrow[34 + half], h, 0, 0, 0);
-        h = __builtin_amdgcn_mfma_f32_32x32x2f32(hi[4 * WS], xrow[36 + half], h, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; i++) h[i] = h[i] > 0.0f ? h[i] : 0.0f;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      v16f dh = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-      {
-        // dH = W2^T G over this MLP's rows (pad row included: zero on both sides)
-        const float* w2r = sW2 + (S::grow(m) + half) * WS + al;
-        const float* gr = W.g + (S::grow(m) + half) * SG_STRIDE + al;
-#pragma unroll
-        for (int s = 0; s < even_up(S::out(m)) / 2; s++)
-          dh = __builtin_amdgcn_mfma_f32_32x32x2f32(w2r[2 * s * WS], gr[2 * s * SG_STRIDE], dh, 0, 0, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 16; i++) dh[i] = h[i] > 0.0f ? dh[i] : 0.0f;
-      __builtin_amdgcn_sched_barrier(0);
-      {
-        // dX += W1^T dHpre: the 32 feature rows on the matrix cores, the 3 view rows and the distance row as plain
-        // sums over the 16 hidden units this lane holds (the other 16 sit in the lane of the other half)
-        const float* wf = w1t + al * WS + 4 * half;
-#pragma unroll
-        for (int s = 0; s < 16; s++)
-          dxf = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[8 * (s >> 2) + (s & 3)], dh[s], dxf, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const float4 w = *(const float4*)(sWview + (m * 4 + c) * 32 + 8 * q + 4 * half);
-            dv[c] = __builtin_fmaf(w.x, dh[4 * q], dv[c]);
-            dv[c] = __builtin_fmaf(w.y, dh[4 * q + 1], dv[c]);
-            dv[c] = __builtin_fmaf(w.z, dh[4 * q + 2], dv[c]);
-            dv[c] = __builtin_fmaf(w.w, dh[4 * q + 3], dv[c]);
-          }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        W.hd[hrow(half, i) * SG_STRIDE + al] = h[i];
-        W.hd[(32 + hrow(half, i)) * SG_STRIDE + al] = dh[i];
-      }
-      wave_sync();
-      // weight gradients: the inner dimension is the 32 anchors of the tile
-#pragma unroll
-      for (int lt = 0; lt < S::tiles(m); lt++) {
-        const int last = S::out(m) - 32 * lt - 1;  // rows past the last one repeat it; their results are dropped
-        const float* gt = W.g + (S::grow(m) + 32 * lt + (al < last ? al : last)) * SG_STRIDE;
-#pragma unroll
-        for (int s = 0; s < 16; s++)
-          accW2[S::first_tile(m) + lt] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-              gt[2 * s + half], W.hd[al * SG_STRIDE + 2 * s + half], accW2[S::first_tile(m) + lt], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      const float* dhrow = W.hd + (32 + al) * SG_STRIDE;
-#pragma unroll 4
-      for (int s = 0; s < 16; s++) {
-        const float dhv = dhrow[2 * s + half];
-        const float* xr = W.x + (2 * s + half) * SX_STRIDE;
-        accW1[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(dhv, xr[al], accW1[m], 0, 0, 0);
-        // rows 6 m .. 6 m + 5 of the shared tile take this MLP's view, bias, distance and level columns, the
-        // other rows add zero
-        const float xv = xr[32 + (al % 6)];
-        accWx = __builtin_amdgcn_mfma_f32_32x32x2f32((al / 6) == m ? xv : 0.0f, dhv, accWx, 0, 0, 0);
-      }
-      wave_sync();
-    }
-#pragma unroll
-    for (int q = 0; q < B2N; q++) {
-      const int row = q * 64 + lane;
-      if (row < S::GROWS) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int c = 0; c < NG_ANCHORS; c++) sum += W.g[row * SG_STRIDE + c];
-        accB2[q] += sum;
-      }
-    }
-
-    // ---- per anchor results
-#pragma unroll
-    for (int c = 0; c < 4; c++) dv[c] += __shfl_xor(dv[c], 32);
-    if (valid) {
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        *(float4*)(d_feat + a * 32 + 8 * q + 4 * half) = make_float4(dxf[4 * q], dxf[4 * q + 1], dxf[4 * q + 2], dxf[4 * q + 3]);
-      if (half == 0) {
-        // the view direction n = v / |v| adds (g - n (n.g)) / |v| to the anchor's direct gradient, the distance
-        // |v| adds n g
-        const float ng = (nv[0] * dv[0] + nv[1] * dv[1]) + nv[2] * dv[2];
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-          d_anchor[a * 3 + c] = (da_now[c] + (dv[c] - nv[c] * ng) / dist) + nv[c] * dv[3];
-      }
-    }
-    wave_sync();
-  }
-
-  // ---- reduce the waves' accumulators, one 32x32 tile at a time, through each wave's staging area
-  float* out = partials + (size_t)blockIdx.x * partial_floats<K>();
-  constexpr int NACC = S::TILES + 4;
-#pragma unroll
-  for (int t = 0; t < NACC; t++) {
-    const v16f& acc = t < S::TILES ? accW2[t] : t < S::TILES + 3 ? accW1[t - S::TILES] : accWx;
+  const int lane = threadIdx.x & 63, half = lane >> 5, al = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), pair = wave % NP;
+  BwdLds<K>& W = lds[pair];
+  const int stride = gridDim.x * NP;
+  float* const out = partials + (size_t)blockIdx.x * partial_floats<K>();
+  // one 32x32 accumulator of all pairs, staged in their hd arrays, to the block's partial set
+  auto add_pairs = [&](int t) {
     float* dst = out + (t < S::TILES ? t : S::TILES + 2 * (t - S::TILES)) * NG_TILE;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 16; i++) W.hd[hrow(half, i) * 32 + al] = acc[i];
-    __syncthreads();
     for (int e = threadIdx.x; e < NG_TILE; e += NT) {
       float sum = lds[0].hd[e];
 #pragma unroll
-      for (int w = 1; w < NW; w++) sum += lds[w].hd[e];
+      for (int w = 1; w < NP; w++) sum += lds[w].hd[e];
       if (t < S::TILES + 3) {
         dst[e] = sum;
       } else if (e < 18 * 32) {
@@ -760,15 +594,342 @@ neural_mlp_backward_kernel(int64_t N, int ntiles, const float* __restrict__ anch
         out[(S::TILES + 2 * (row / 6) + 1) * NG_TILE + h * 32 + (row % 6)] = sum;
       }
     }
-  }
+  };
   __syncthreads();
+
+  // Both branches meet the same barriers: seven for each tile of the block's pairs, whether a pair has one or not,
+  // and two for each array of the reduction.
+  if (wave < NP) {
+    // ---- first wave: activations, and what goes to the anchors
+    const float cam[3] = {campos[0], campos[1], campos[2]};
+    XOperand xo;
+    float da[3] = {0.0f, 0.0f, 0.0f};  // the anchor's direct gradient, as the first kernel left it
+    auto fetch_tile = [&](int t) {
+      const int64_t a = (int64_t)t * NG_ANCHORS + al;
+      xo = fetch_x(a < N, a, half, anchor, feat, level);
+      if (a < N && half == 0) {
 #pragma unroll
-  for (int q = 0; q < B2N; q++) W.hd[q * 64 + lane] = accB2[q];
+        for (int c = 0; c < 3; c++) da[c] = d_anchor[a * 3 + c];
+      }
+    };
+    int tile = blockIdx.x * NP + pair;
+    if (tile < ntiles) fetch_tile(tile);
+    for (int first = blockIdx.x * NP; first < ntiles; first += stride, tile += stride) {
+      const bool live = tile < ntiles;  // uniform
+      const int64_t a = (int64_t)tile * NG_ANCHORS + al;
+      const bool valid = a < N;
+      float xb[NG_W1_STEPS], wh[NG_W1_STEPS], nv[3], dist;
+      const float da_now[3] = {da[0], da[1], da[2]};
+      v16f h, dxf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+      // this half's share of the gradient of the view direction (0..2) and of the distance (3)
+      float dv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (live) {
+        hidden_weights(wh, sW1, al, half);
+        __builtin_amdgcn_sched_barrier(0);
+        unpack_x(xb, nv, dist, xo, valid, half, cam);
+        h = hidden_products(wh, xb);
+      }
+      __syncthreads();  // the other wave is through with the tile before
+      if (live) {
+#pragma unroll
+        for (int s = 0; s < NG_W1_STEPS; s++) W.x[al * SX_STRIDE + xslot(half, s)] = xb[s];
+      }
+      __syncthreads();  // x and G are there
+      // dX += W1^T dHpre: the 32 feature rows on the matrix cores, the 3 view rows and the distance row as plain sums
+      // over the 16 hidden units this lane holds (the other 16 sit in the lane of the other half)
+      float wx[16];
+      float4 wv[2][4];
+      auto ask_view = [&](int m, int c0) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) wv[c][q] = *(const float4*)(sWview + (m * 4 + c0 + c) * 32 + 8 * q + 4 * half);
+      };
+      auto add_view = [&](const v16f& d, int c0) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            dv[c0 + c] = __builtin_fmaf(wv[c][q].x, d[4 * q], dv[c0 + c]);
+            dv[c0 + c] = __builtin_fmaf(wv[c][q].y, d[4 * q + 1], dv[c0 + c]);
+            dv[c0 + c] = __builtin_fmaf(wv[c][q].z, d[4 * q + 2], dv[c0 + c]);
+            dv[c0 + c] = __builtin_fmaf(wv[c][q].w, d[4 * q + 3], dv[c0 + c]);
+          }
+      };
+      auto ask_dx = [&](int m) {
+        const float* wf = sW1 + m * NG_SLOTS * WS + al * WS + 4 * half;
+#pragma unroll
+        for (int s = 0; s < 16; s++) wx[s] = wf[8 * (s >> 2) + (s & 3)];
+        ask_view(m, 0);
+      };
+      auto add_dx = [&](const v16f& d) {
+#pragma unroll
+        for (int s = 0; s < 16; s++) dxf = __builtin_amdgcn_mfma_f32_32x32x2f32(wx[s], d[s], dxf, 0, 0, 0);
+        add_view(d, 0);
+      };
+      v16f dh;
+#pragma unroll
+      for (int m = 0; m < 3; m++) {
+        if (live) {
+          // dH = W2^T G over this MLP's rows (pad row included: zero on both sides)
+          const int steps = even_up(S::out(m)) / 2;
+          const float* w2r = sW2 + (S::grow(m) + half) * WS + al;
+          const float* gr = W.g + (S::grow(m) + half) * SG_STRIDE + al;
+          float wq[2][DH_STEPS], gq[2][DH_STEPS];
+          auto ask_dh = [&](int c) {
+#pragma unroll
+            for (int s = 0; s < DH_STEPS; s++)
+              if (c * DH_STEPS + s < steps) {
+                wq[c & 1][s] = w2r[2 * (c * DH_STEPS + s) * WS];
+                gq[c & 1][s] = gr[2 * (c * DH_STEPS + s) * SG_STRIDE];
+              }
+          };
+          if (m > 0) {
+            ask_dx(m - 1);
+            hidden_weights(wh, sW1 + m * NG_SLOTS * WS, al, half);
+            __builtin_amdgcn_sched_barrier(0);
+            add_dx(dh);
+            __builtin_amdgcn_sched_barrier(0);
+            ask_view(m - 1, 2);
+            ask_dh(0);
+            __builtin_amdgcn_sched_barrier(0);
+            h = hidden_products(wh, xb);
+            add_view(dh, 2);
+            if (m == 1 && tile + stride < ntiles) fetch_tile(tile + stride);
+          } else {
+            ask_dh(0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          dh = v16f{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+          for (int c = 0; c * DH_STEPS < steps; c++) {
+            ask_dh(c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < DH_STEPS; s++)
+              if (c * DH_STEPS + s < steps)
+                dh = __builtin_amdgcn_mfma_f32_32x32x2f32(wq[c & 1][s], gq[c & 1][s], dh, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int i = 0; i < 16; i++) dh[i] = h[i] > 0.0f ? dh[i] : 0.0f;
+        }
+        if (m > 0) __syncthreads();  // the other wave has read H and dHpre of the MLP before
+        if (live) {
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            W.hd[hrow(half, i) * SG_STRIDE + al] = h[i];
+            W.hd[(32 + hrow(half, i)) * SG_STRIDE + al] = dh[i];
+          }
+        }
+        __syncthreads();  // H and dHpre are there
+      }
+      if (live) {
+        ask_dx(2);
+        __builtin_amdgcn_sched_barrier(0);
+        add_dx(dh);
+        ask_view(2, 2);
+        add_view(dh, 2);
+      }
+      if (live) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) dv[c] += __shfl_xor(dv[c], 32);
+        if (valid) {
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            *(float4*)(d_feat + a * 32 + 8 * q + 4 * half) = make_float4(dxf[4 * q], dxf[4 * q + 1], dxf[4 * q + 2], dxf[4 * q + 3]);
+          if (half == 0) {
+            // the view direction n = v / |v| adds (g - n (n.g)) / |v| to the anchor's direct gradient, the distance
+            // |v| adds n g
+            const float ng = (nv[0] * dv[0] + nv[1] * dv[1]) + nv[2] * dv[2];
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+              d_anchor[a * 3 + c] = (da_now[c] + (dv[c] - nv[c] * ng) / dist) + nv[c] * dv[3];
+          }
+        }
+      }
+    }
+    for (int t = 0; t < NACC; t++) {
+      __syncthreads();
+      __syncthreads();
+      add_pairs(t);
+    }
+    __syncthreads();
+  } else {
+    // ---- second wave: G, and the weights' gradients.  Accumulators: the W2 tiles, the 32 feature columns of W1 per
+    // MLP, and the six remaining columns of W1 (view direction, bias, distance, level) as rows 6 m + c of a tile of the
+    // first two MLPs and rows c of one of the third.  What has at most 16 rows goes through the 16x16x4 form, half the
+    // cycles of a 32x32 tile: operand layout A lane l -> A[l % 16][l / 16], B lane l -> B[l / 16][l % 16], result
+    // register i of lane l -> D[4 * (l / 16) + i][l % 16], two of them for the 32 hidden units.
+    const int l16 = lane & 15, k4 = lane >> 4;
+    v16f accW2[S::TILES], accW1[3];
+    v4f accRest[3][2], accWx[2][2];
+    float accB2[B2N];
+#pragma unroll
+    for (int t = 0; t < S::TILES; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) accW2[t][i] = 0.0f;
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) accW1[m][i] = 0.0f;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+#pragma unroll
+      for (int m = 0; m < 3; m++) accRest[m][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int i = 0; i < 2; i++) accWx[i][t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int q = 0; q < B2N; q++) accB2[q] = 0.0f;
+    // rows that pad a block of G to an even count are read by the dH products and never written below
+    for (int e = lane; e < S::GROWS * SG_STRIDE; e += 64) W.g[e] = 0.0f;
+
+    const int64_t total_floats = N * K * NG_SLOT_GRADS;
+    float4 gq[NQ];
+    // A wave's place in the records, hidden from the compiler: it would hold the addresses of the fourteen reads and of
+    // their places in G from one tile to the next, more registers than there are
+    auto first_float = [&]() {
+      int e = lane * 4;
+      asm volatile("" : "+v"(e));
+      return e;
+    };
+    auto floats_of = [&](int t) {  // floats of tile t that exist
+      const int64_t left = total_floats - (int64_t)t * TILE_FLOATS;
+      return left < TILE_FLOATS ? (int)left : TILE_FLOATS;
+    };
+    auto fetch_tile = [&](int t) {
+      // reads past a tile's end repeat its last float4 and are dropped below; the buffer is padded, so a float4 that
+      // straddles the end of the last tile is readable
+      const float* base = slot_grads + (int64_t)t * TILE_FLOATS;
+      const int last = (floats_of(t) - 1) & ~3, e0 = first_float();
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        const int e = e0 + q * 256;
+        gq[q] = *(const float4*)(base + (e < last ? e : last));
+      }
+    };
+    int tile = blockIdx.x * NP + pair;
+    if (tile < ntiles) fetch_tile(tile);
+    for (int first = blockIdx.x * NP; first < ntiles; first += stride, tile += stride) {
+      const bool live = tile < ntiles;  // uniform
+      __syncthreads();  // the first wave is through with the tile before
+      if (live) {
+        const int nvalid = floats_of(tile), e0 = first_float();
+        auto place = [&](auto whole) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) {
+            const int e = e0 + q * 256;
+            if ((q + 1) * 256 <= TILE_FLOATS || e < TILE_FLOATS) {
+              const float v[4] = {gq[q].x, gq[q].y, gq[q].z, gq[q].w};
+#pragma unroll
+              for (int c = 0; c < 4; c++) W.g[sWhere[e + c]] = whole.value || e + c < nvalid ? v[c] : 0.0f;
+            }
+          }
+        };
+        if (nvalid == TILE_FLOATS) place(std::true_type());
+        else place(std::false_type());
+      }
+      __syncthreads();  // x and G are there
+      if (tile + stride < ntiles) fetch_tile(tile + stride);
+#pragma unroll
+      for (int m = 0; m < 3; m++) {
+        if (m > 0) __syncthreads();  // H and dHpre of the MLP before have been read
+        __syncthreads();  // H and dHpre are there
+        if (!live) continue;
+        // weight gradients: the inner dimension is the 32 anchors of the tile
+        const float* hrow16 = W.hd + l16 * SG_STRIDE + k4;
+#pragma unroll
+        for (int lt = 0; lt < S::whole_tiles(m); lt++) {
+          const int last = S::out(m) - 32 * lt - 1;  // rows past the last one repeat it; their results are dropped
+          const float* gt = W.g + (S::grow(m) + 32 * lt + (al < last ? al : last)) * SG_STRIDE;
+#pragma unroll
+          for (int s = 0; s < 16; s++)
+            accW2[S::first_tile(m) + lt] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                gt[2 * s + half], W.hd[al * SG_STRIDE + 2 * s + half], accW2[S::first_tile(m) + lt], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (S::whole_tiles(m) < S::tiles(m)) {
+          const int last = S::out(m) - 32 * S::whole_tiles(m) - 1;
+          const float* gt = W.g + (S::grow(m) + 32 * S::whole_tiles(m) + (l16 < last ? l16 : last)) * SG_STRIDE + k4;
+#pragma unroll
+          for (int s = 0; s < 8; s++) {
+            const float g = gt[4 * s];
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+              accRest[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(g, hrow16[16 * t * SG_STRIDE + 4 * s], accRest[m][t], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const float* dhrow = W.hd + (32 + al) * SG_STRIDE;
+#pragma unroll 4
+        for (int s = 0; s < 16; s++)
+          accW1[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(dhrow[2 * s + half], W.x[(2 * s + half) * SX_STRIDE + al],
+                                                          accW1[m], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        {
+          // the other MLP's rows of the shared tile, and those past the last one, add zero
+          const bool mine = m < 2 ? l16 / 6 == m : l16 < 6;
+          const float* xr = W.x + k4 * SX_STRIDE + 32 + l16 % 6;
+#pragma unroll
+          for (int s = 0; s < 8; s++) {
+            const float x = xr[4 * s * SX_STRIDE];
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+              accWx[m >> 1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                  mine ? x : 0.0f, hrow16[(32 + 16 * t) * SG_STRIDE + 4 * s], accWx[m >> 1][t], 0, 0, 0);
+          }
+        }
+        if (m > 0) {
+#pragma unroll
+          for (int q = m - 1; q < B2N; q += 2) {
+            const int row = q * 64 + lane;
+            if (row < S::GROWS) {
+              float sum = 0.0f;
+#pragma unroll
+              for (int c = 0; c < NG_ANCHORS; c++) sum += W.g[row * SG_STRIDE + c];
+              accB2[q] += sum;
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NACC; t++) {
+      const int m = t < S::T0 ? 0 : t < S::T0 + S::T1 ? 1 : 2;  // of a W2 tile
+      __syncthreads();
+      if (t == S::TILES + 3) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int row = 4 * k4 + i;
+            if (row < 12) W.hd[row * 32 + 16 * c + l16] = accWx[0][c][i];
+            if (row < 6) W.hd[(12 + row) * 32 + 16 * c + l16] = accWx[1][c][i];
+          }
+      } else if (t < S::TILES && t - S::first_tile(m) == S::whole_tiles(m)) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) W.hd[(4 * k4 + i) * 32 + 16 * c + l16] = accRest[m][c][i];
+      } else {
+        const v16f& acc = t < S::TILES ? accW2[t] : accW1[t - S::TILES];
+#pragma unroll
+        for (int i = 0; i < 16; i++) W.hd[hrow(half, i) * 32 + al] = acc[i];
+      }
+      __syncthreads();
+      add_pairs(t);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < B2N; q++) W.hd[q * 64 + lane] = accB2[q];
+  }
   __syncthreads();
   for (int e = threadIdx.x; e < B2N * 64; e += NT) {
     float sum = lds[0].hd[e];
 #pragma unroll
-    for (int w = 1; w < NW; w++) sum += lds[w].hd[e];
+    for (int w = 1; w < NP; w++) sum += lds[w].hd[e];
     out[(S::TILES + 6) * NG_TILE + e] = sum;
   }
 }
@@ -873,7 +1034,7 @@ struct Launcher {
                        color, opacity, scal, rot, aux);
   }
   static int backward_blocks(int64_t N) {
-    return blocks_for((int)((N + NG_ANCHORS - 1) / NG_ANCHORS), S::BWD_WAVES, 1);
+    return blocks_for((int)((N + NG_ANCHORS - 1) / NG_ANCHORS), S::BWD_PAIRS, 1);
   }
   static void backward(int64_t N, const float* anchor, const float* feat, const float* level, int input_flags,
                        const float* offsets, const float* scaling, const float* campos, const float* packed, const float* neural_opacity,
@@ -889,7 +1050,7 @@ struct Launcher {
                        first, color_out, rot_out, aux, g_xyz, g_color, g_opacity, g_scal, g_rot, slot_grads, d_anchor,
                        d_offsets, d_scaling);
     const int nblocks = backward_blocks(N);
-    hipLaunchKernelGGL(neural_mlp_backward_kernel<K>, dim3(nblocks), dim3(64 * S::BWD_WAVES), 0, stream, N, ntiles,
+    hipLaunchKernelGGL(neural_mlp_backward_kernel<K>, dim3(nblocks), dim3(128 * S::BWD_PAIRS), 0, stream, N, ntiles,
                        anchor, feat, level, campos, packed, slot_grads, d_anchor, d_feat, partials);
     MlpGrads d;
     for (int i = 0; i < 12; i++) d.p[i] = d_params[i];

@@ -421,3 +421,31 @@ def test_drop_in_with_appearance_embedding_and_feature_bank():
         grads.append([p.grad.clone() for p in params])
     for i, (a, b) in enumerate(zip(*grads)):
         assert float((a - b).norm()) <= 2e-4 * float(b.norm()) + 1e-12, i
+
+
+@pytest.mark.parametrize("k,pairs", [(1, 4), (10, 4), (11, 2), (16, 2)])
+def test_gradients_of_more_tiles_than_a_pass_holds(k, pairs):
+    """The backward's blocks take `pairs` tiles of 32 anchors at a time: one tile and one anchor more than 256 blocks
+    take at once, so that a block comes back with pairs that have no tile and with one that is nearly empty.  An
+    anchor's gradients do not depend on where its tile lies; the weights' are sums of the same terms in another order
+    (float32 sums of n terms in two orders: relative difference of the order of 2^-24 sqrt(n), 1e-5 at 33,000)."""
+    from gs_neural import neural_gaussians
+    N = 32 * pairs * 256 + 33
+    s = gs_scenes.make_anchor_scene(N, k, 40 + k)
+    ups = torch.randn(N * k, 14, generator=torch.Generator().manual_seed(k)).to(DEV)  # by slot
+
+    def grads(lo, hi):
+        part = dict(s)
+        for name in ("anchor", "feat", "offsets", "scaling"):
+            part[name] = s[name][lo:hi].clone()
+        anchor, feat, offsets, scaling, campos, mlps = _to_dev(part, grad=True)
+        out = neural_gaussians(anchor, feat, offsets, scaling, campos, *mlps)
+        torch.cat(out[:5], 1).backward(ups[lo * k:hi * k][out[6]])
+        return [t.grad.cpu() for t in (anchor, feat)], [x.grad.cpu().double() for m in mlps for x in m]
+
+    rows, weights = grads(0, N)
+    parts = [grads(lo, min(lo + 8192, N)) for lo in range(0, N, 8192)]
+    for i in range(2):
+        assert torch.equal(rows[i], torch.cat([p[0][i] for p in parts]))
+    for i, w in enumerate(weights):
+        assert _rel(w, sum(p[1][i] for p in parts)) <= 2e-5, i
