@@ -3,14 +3,14 @@
 // direction] and, where the model asks for them, the distance and the anchor's level,
 // scene/gaussian_model.py:118-149), forward and backward.
 //
-// One wave owns 32 anchors.  Both layers run on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) in the
-// transposed form D[unit][anchor] = W[unit][:] . X[:][anchor]: the anchors sit on the 32 columns, so the
-// hidden layer comes out of layer 1 with lane = anchor, register = hidden unit, which is exactly the B
-// operand layer 2 wants.  Nothing of the hidden layer ever leaves the registers.  Operand layout of the
-// instruction, with l the lane, half = l / 32:  A lane l -> A[l % 32][half], B lane l -> B[half][l % 32],
-// result register i of lane l -> D[8 * (i / 4) + 4 * half + i % 4][l % 32].  The order in which the inner
-// dimension is walked is free as long as both operands agree, so every inner index below is permuted to
-// whatever the lanes already hold.
+// One wave (in the backward through the MLPs, two) owns 32 anchors.  Both layers run on the fp32 matrix cores
+// (v_mfma_f32_32x32x2_f32) in the transposed form D[unit][anchor] = W[unit][:] . X[:][anchor]: the anchors sit
+// on the 32 columns, so the hidden layer comes out of layer 1 with lane = anchor, register = hidden unit, which
+// is exactly the B operand layer 2 wants.  Nothing of the hidden layer ever leaves the registers in the forward
+// kernels.  Operand layout of the instruction, with l the lane, half = l / 32:  A lane l -> A[l % 32][half],
+// B lane l -> B[half][l % 32], result register i of lane l -> D[8 * (i / 4) + 4 * half + i % 4][l % 32].  The
+// order in which the inner dimension is walked is free as long as both operands agree, so every inner index
+// below is permuted to whatever the lanes already hold.
 //
 // The weights are rearranged once per call into those per-step operand orders ("packed" buffer); the kernels
 // then read them with index step * 64 + lane.
@@ -545,8 +545,8 @@ neural_offset_backward_kernel(int64_t N, const float* __restrict__ offsets,
 // held 336 accumulator and prefetch registers and waited for each of these by itself, 48 k cycles a tile where its
 // products take 21 k; together they take 30 k, of which the products, fewer by those of half tiles, 19 k: 175 k visible
 // anchors of ten offsets 124 -> 92 us.  Of that, two waves as such 124 -> 104 (119 as long as the second one's read
-// addresses were kept in registers and spilled), half tiles 104 -> 92; operands asked for a dozen products ahead in
-// the first wave are worth 4 of these (without half tiles nothing: the second wave is the longer one there).
+// addresses were kept in registers and spilled), half tiles 104 -> 92; without these, operands asked for a dozen products
+// ahead in the first wave changed nothing, the second one being the longer.
 template <int K>
 struct BwdLds {
   using S = Shape<K>;
