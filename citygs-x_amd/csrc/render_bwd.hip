@@ -718,7 +718,9 @@ constexpr int REDUCE_STREAM_GAUSSIANS = 1'500'000;
 // follows otherwise runs beside the write-back of the lines they left dirty: 4 M Gaussians, 1152 x 864, 79.3 + 277 us ->
 // 79.5 + 248 (this kernel + that one), 10 M, 1920 x 1080, 175 + 633 -> 175 + 595.  That wants whole lines per store, so
 // the rows of 3 and 5 floats are turned in LDS (stored from the lanes that hold them, 80.5 and 180).
-template <bool STREAM>
+// SPARSE: only the records that `written` tells of are there.  Kernels of their own: as a test of the pointer it cost the
+// views with every record 3 to 11 % here (3 M at 1920 x 1080 89.0 -> 94.5 us, 1 M 33.4 -> 34.3, 300 k 15.3 -> 17.0).
+template <bool STREAM, bool SPARSE>
 __global__ void __launch_bounds__(GS_BLOCK_1D)
 reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const float4* __restrict__ instance_grads,
                         const uint8_t* __restrict__ written, float ddelx_dx, float ddely_dy, int render_geo,
@@ -745,20 +747,22 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
     many &= many - 1ull;
     const uint32_t ob = __shfl(b, owner, GS_WAVE), on = __shfl(n, owner, GS_WAVE);
     float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0, p2 = p0, p3 = p0;
-    // (four rounds' bytes are asked for together)
-    for (uint32_t k = (uint32_t)lane; k < on; k += 4 * GS_WAVE) {
-      bool have[4];
+    auto add_record = [&](uint32_t k) {
+      const float4* rec = instance_grads + 4 * (size_t)(ob + k);
+      add(p0, rec[0]); add(p1, rec[1]); add(p2, rec[2]); add(p3, rec[3]);
+    };
+    if constexpr (SPARSE) {
+      // (two rounds' bytes are asked for together: for four there are no registers at seven waves a SIMD)
+      for (uint32_t k = (uint32_t)lane; k < on; k += 2 * GS_WAVE) {
+        bool have[2];
 #pragma unroll
-      for (uint32_t j = 0; j < 4; j++) {
-        const uint32_t at = k + j * GS_WAVE;
-        have[j] = at < on && (written == nullptr || written[ob + at] != 0);
-      }
+        for (uint32_t j = 0; j < 2; j++) have[j] = k + j * GS_WAVE < on && written[ob + k + j * GS_WAVE] != 0;
 #pragma unroll
-      for (uint32_t j = 0; j < 4; j++) {
-        if (!have[j]) continue;
-        const float4* rec = instance_grads + 4 * (size_t)(ob + k + j * GS_WAVE);
-        add(p0, rec[0]); add(p1, rec[1]); add(p2, rec[2]); add(p3, rec[3]);
+        for (uint32_t j = 0; j < 2; j++)
+          if (have[j]) add_record(k + j * GS_WAVE);
       }
+    } else {
+      for (uint32_t k = (uint32_t)lane; k < on; k += GS_WAVE) add_record(k);
     }
 #pragma unroll
     for (int d = GS_WAVE / 2; d >= 1; d >>= 1) {
@@ -777,7 +781,7 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
     // (a wave that holds such a Gaussian reads the others' records directly: rare)
     if (live && n <= MANY) {
       for (uint32_t k = b; k < e; k++) {
-        if (written != nullptr && written[k] == 0) continue;
+        if (SPARSE && written[k] == 0) continue;
         const float4* rec = instance_grads + 4 * (size_t)k;
         add(a0, rec[0]); add(a1, rec[1]); add(a2, rec[2]); add(a3, rec[3]);
       }
@@ -796,7 +800,7 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
     run_end = (uint32_t)__builtin_amdgcn_readfirstlane((int)run_end);
     for (uint32_t c = run_begin; c < run_end; c += REC_CHUNK) {
       uint64_t have_m = ~0ull;
-      if (written != nullptr) {
+      if constexpr (SPARSE) {
         have_m = gs_ballot(c + (uint32_t)lane < run_end && written[c + (uint32_t)lane] != 0);
         if (have_m == 0ull) continue;
       }
@@ -805,10 +809,11 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
       for (int j = 0; j < 4; j++) {
         const uint32_t idx = (uint32_t)(j * GS_WAVE + lane), r = c + (idx >> 2);
         const float4* part = instance_grads + 4 * (size_t)r + (idx & 3u);
+        const bool there = r < run_end && (!SPARSE || (have_m >> (idx >> 2) & 1u));
         if constexpr (STREAM)
-          v[j] = r < run_end && (have_m >> (idx >> 2) & 1u) ? load_streaming(part) : make_float4(0.f, 0.f, 0.f, 0.f);
+          v[j] = there ? load_streaming(part) : make_float4(0.f, 0.f, 0.f, 0.f);
         else
-          v[j] = r < run_end && (have_m >> (idx >> 2) & 1u) ? *part : make_float4(0.f, 0.f, 0.f, 0.f);
+          v[j] = there ? *part : make_float4(0.f, 0.f, 0.f, 0.f);
       }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
@@ -820,7 +825,7 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       const uint32_t lo = max(b, c), hi = min(e, c + REC_CHUNK);
       for (uint32_t k = lo; k < hi; k++) {
-        if (!((have_m >> (k - c)) & 1u)) continue;
+        if (SPARSE && !((have_m >> (k - c)) & 1u)) continue;
         const float4* rec = mine + (k - c) * REC_STRIDE4;
         add(a0, rec[0]); add(a1, rec[1]); add(a2, rec[2]); add(a3, rec[3]);
       }
@@ -901,8 +906,13 @@ int launch_render_bwd(const RenderBwdArgs& a, hipStream_t stream) {
                        a.render_geo, (float2*)a.dL_dmean2D, a.dL_dmean2D_abs, (float4*)a.dL_dconic_opacity,
                        a.dL_dcolors, a.dL_dall_map);
   };
-  if (a.P >= REDUCE_STREAM_GAUSSIANS) reduce(reduce_instances_kernel<true>);
-  else reduce(reduce_instances_kernel<false>);
+  if (a.P >= REDUCE_STREAM_GAUSSIANS) {
+    if (written != nullptr) reduce(reduce_instances_kernel<true, true>);
+    else reduce(reduce_instances_kernel<true, false>);
+  } else {
+    if (written != nullptr) reduce(reduce_instances_kernel<false, true>);
+    else reduce(reduce_instances_kernel<false, false>);
+  }
   return 0;
 }
 
