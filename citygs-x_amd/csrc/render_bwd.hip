@@ -34,7 +34,7 @@
 //     them: all instances of a Gaussian are consecutive there).  No global
 //     atomics either.
 //   * Instances that no pixel blends have records of zeros.  In views with many
-//     Gaussians per pixel, where those are nearly all, they are left out: a byte
+//     instances per pixel, where those are nearly all, they are left out: a byte
 //     per instance (`written`, cleared first) says which records there are.  The
 //     zeros' stores were in the chain of the longest tiles, too (a load behind
 //     them waits for them): 10 M Gaussians at street level, two views of 2.7 M and
@@ -874,17 +874,20 @@ reduce_instances_kernel(int P, const uint32_t* __restrict__ point_offsets, const
 
 }  // namespace
 
-// Gaussians per pixel, in halves, from which on records of zeros are left out.  A pixel blends some twenty, so it is their
-// number per pixel that says how many have none.  The bytes cost a launch that clears them (5 us) and the reduction a round
-// trip (1 M 33 -> 36 us).  A training view with every record and without zeros: 3 M obliquely and from the air at 1152 x 864
-// (3 a pixel) 1333 and 1339 us, 1 M 547 and 553; 4 M from the air (4 a pixel) 1399 and 1394; at street level 3 M at
-// 1920 x 1080 (1.4) 974 and 982, 8 M (3.9) 1965 and 1930, 3 M at 800 x 600 (6.3) 1318 and 1289; 2 M obliquely at 640 x 480
-// (6.5) 1023 and 1000; 3 M from the air at 400 x 300 (25) 1710 and 1661.
-constexpr int64_t SPARSE_HALVES = 7;
+// Instances per pixel from which on records of zeros are left out.  A pixel blends some twenty Gaussians, whatever its tile's
+// list holds, so it is the lists' length per pixel that says how many instances have no record.  The bytes cost a launch that
+// clears them (5 us) and the sums a round trip for every 64 instances of a wave.  119 training views (23 thousand to 10 M
+// Gaussians, 320 x 240 to 1920 x 1080, 0.05 to 18 instances a Gaussian), us with the zeros left out less us with them: up to 1
+// instance a pixel 2 to 21 lost; 1 to 1.5 18 lost to 3 gained; 1.5 to 2 8 lost to 38 gained; 2 to 2.5 7 lost to 42 gained (two of
+// 14 above 10, street level); 2.5 to 4 8 to 126 gained in 26 views, 5 to 14 lost in four (of 614 to 1932), the others within
+// 3; from 4 on 5 to 112 gained in 25, 8 lost in one (of 1337), the others within 2.  (Gaussians per pixel, those out of view
+// included, are no measure: a view of a tenth of 10 M Gaussians, 10 of them a pixel, lost 21 of 1477, one of 200 thousand large
+// ones, 0.2 a pixel, gains 44 of 698.)
+constexpr int64_t SPARSE_INSTANCES = 2;
 
 int launch_render_bwd(const RenderBwdArgs& a, hipStream_t stream) {
   const uint32_t gx = (a.W + GS_TILE_X - 1) / GS_TILE_X, gy = (a.H + GS_TILE_Y - 1) / GS_TILE_Y;
-  uint8_t* const written = 2 * (int64_t)a.P >= SPARSE_HALVES * (int64_t)a.W * a.H ? a.written : nullptr;
+  uint8_t* const written = a.R >= SPARSE_INSTANCES * (int64_t)a.W * a.H ? a.written : nullptr;
   if (written != nullptr) launch_fill_u32(((int64_t)a.R + 3) / 4, 0u, reinterpret_cast<uint32_t*>(written), stream);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(gx * gy), dim3(GS_TILE_PIX), 0, stream, (const uint2*)a.ranges, a.point_list, a.W, a.H,
