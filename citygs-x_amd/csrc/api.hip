@@ -628,11 +628,14 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   if (check_launch("inclusive_sum", stream, dbg)) return 1;
   // The blend kernels (this call's and the backward call's) can fetch a Gaussian's operands as one 64-byte record
   // instead of gathering parts of five lines of memory.  Packing the records costs 4 to 8 us per million Gaussians and
-  // about 15 more per million of them that are in view; what it saves depends on the lists.  Over 36 views (forward and
-  // backward, us, packed less gathered): with lists beyond the register sort's, whose tiles end the view and are split only
-  // with records, 0.62 instances per Gaussian 220 saved of 2056, 0.74 298 of 2420, 0.75 215 of 1553 and, at 320x240, 499 of
-  // 2667, but 0.28 instances 20 lost of 1056; without such lists 1.5 to 2.4 instances 13 saved of 260, 0.98 14 of 501, 0.33
-  // 7 lost of 402.  The library's own records live at the end of the binning buffer, which is sized once the decision is
+  // about 15 more per million of them that are in view; what it saves depends on the lists, and with lists beyond the
+  // register sort's, whose tiles end the view and are split only with records, on how far into them the pixels see.  Packed
+  // less gathered, forward and backward, 118 views of 200 thousand to 10 M Gaussians, by instances per Gaussian:
+  //   with such lists: 0.2 to 0.3 60 us saved to 23 lost (2 of 8 save), 0.3 to 0.4 222 saved to 80 lost (2 of 10), 0.4 to 0.6
+  //   371 saved to 96 lost (16 of 23; what loses are views of 8 M at street level through a lens of 40 to 75 degrees), 0.6 to
+  //   0.8 15 to 434 saved (21 of 22, one 1.5 lost), more 8 to 150 saved
+  //   without: to 0.4 4 to 44 lost, 0.4 to 0.8 29 saved to 9 lost (colour only 4 saved to 19 lost), more 36 saved to 8 lost
+  // The library's own records live at the end of the binning buffer, which is sized once the decision is
   // made.  A view that was launched ahead without records and did not fit is looked at again with its own figures (its
   // buffer is another one); one that was launched with them keeps them, since the word that says so is set.
   bool use_packed = caller_records != nullptr;
@@ -725,8 +728,11 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
 
   Arrays A;
   if (ahead) {
-    // (on the expected count less a fifth: the caller's expectation carries a margin of a quarter)
-    decide_packing(cap_n - cap_n / 5, cap_longest);
+    // (on the expected count less a fifth: the caller's expectation carries a margin of a quarter.  The bound on the lists
+    // that the kernels are launched for says little about their length: "any" is also what a view of 3300 at the most, or
+    // any view of a size that once had a longer list, is launched with)
+    const int recent = options->struct_bytes >= sizeof(gs_render_options) ? options->recent_longest_list : 0;
+    decide_packing(cap_n - cap_n / 5, recent > 0 ? (uint32_t)recent : cap_longest);
     if (carve(cap_n, A)) return 1;
     if (timer.begin(elapsed_ms != nullptr, stream)) return 1;
     if (pack_records(A)) return 1;

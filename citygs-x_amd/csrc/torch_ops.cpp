@@ -209,8 +209,8 @@ py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& m
                          const Tensor& radii_, const Tensor& conic_opacity, const Tensor& rgb, const Tensor& locally,
                          float tan_fovx, float tan_fovy, const OptTensor& all_map, bool geo, bool debug,
                          bool want_max_weight_depth, bool timing, int small_limit, int block_records,
-                         int64_t expected_instances, int expected_longest_list, const OptTensor& blend_records,
-                         uintptr_t stream) {
+                         int64_t expected_instances, int expected_longest_list, int recent_longest_list,
+                         const OptTensor& blend_records, uintptr_t stream) {
   const Tensor means2D = f32c(means2D_, "means2D");
   const int64_t P = means2D.size(0);
   const Options o(means2D.device());
@@ -241,6 +241,7 @@ py::tuple render_forward(const Tensor& background, int H, int W, const Tensor& m
   options.expected_instances = expected_instances;
   options.blend_records = blend_records.has_value() ? ptr(*blend_records) : nullptr;
   options.clear_geo_images = 1;
+  options.recent_longest_list = recent_longest_list;
   gs_render_result result = {};
   result.struct_bytes = sizeof(result);
   // fp32 arithmetic, as `H / (2.0f * tan_fovy)` at rasterize_points.cu:328-329

@@ -199,12 +199,14 @@ def _write_tile_log(args, H, W, n_render, n_consider, n_contrib):
 
 def render_gaussians_ex(background, image_height, image_width, means2D, depths, radii, conic_opacity, rgb,
                         compute_locally, viewmatrix, campos, tan_fovx, tan_fovy, all_map, render_geo, debug, args,
-                        expected_instances=0, expected_longest_list=0, blend_records=None):
+                        expected_instances=0, expected_longest_list=0, blend_records=None,
+                        recent_longest_list=0):
     """render_gaussians plus what the reference's tuple has no slot for: returns (tuple, info) with info =
     {"longest_list", "binning_capacity", "launched_ahead"}.  With expected_instances > 0 the list kernels and the
     blend are launched without waiting for the instance count, on a binning buffer laid out for
     expected_instances; info["binning_capacity"] then has to be handed to render_gaussians_backward (and to
     gs_binning_state_layout) in place of the instance count.  Results do not depend on the expectation.
+    recent_longest_list: the longest list of the views that the expectation comes from (0: not known).
     blend_records: the (P,16) operand records that preprocess_gaussians_ex wrote for exactly these inputs, all_map
     being build_all_map of the same Gaussians and camera (the blend kernels then read them and nothing is
     packed); the same tensor goes to render_gaussians_backward."""
@@ -228,7 +230,8 @@ def render_gaussians_ex(background, image_height, image_width, means2D, depths, 
      img, longest_list, binning_capacity, launched_ahead, elapsed, mwd) = _ops.render_forward(
         background, H, W, means2D, depths, radii, conic_opacity, rgb, compute_locally, float(tan_fovx), float(tan_fovy),
         all_map if render_geo else None, bool(render_geo), bool(debug), want_mwd, _want_timing(args), int(small_limit),
-        int(block_records), int(expected_instances), int(expected_longest_list), blend_records, _n.stream_handle(dev))
+        int(block_records), int(expected_instances), int(expected_longest_list), int(recent_longest_list),
+        blend_records, _n.stream_handle(dev))
     _record_time(args, "forward_render_time", elapsed)
     if want_mwd:
         args.setdefault("stats_collector", {})["max_weight_depth"] = mwd

@@ -232,7 +232,7 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_setti
 # ------------------------------------------------------------------- render --
 
 # What the last views of a given image size needed, (instances, longest list, whether any view of the size had a list
-# beyond _LONG_LIST, the instances of the _RECENT_VIEWS last ones) keyed by (height, width, device): the
+# beyond _LONG_LIST, the first two of the _RECENT_VIEWS last ones) keyed by (height, width, device): the
 # next view of that size is launched without waiting for its instance count, on buffers sized for the most instances of
 # those views and the longest list of the last one plus
 # a margin (a training loop renders thousands of similar views; the number of Gaussians changes at every
@@ -251,7 +251,13 @@ _LONG_TILE = 3072  # a list from which on the forward blend splits its tile
 
 def _most_instances(seen):
     """Of the last views that an entry of _expectations tells of."""
-    return max(seen[0], *seen[3]) if len(seen) > 3 else seen[0]
+    return max(n for n, _ in seen[3]) if len(seen) > 3 else seen[0]
+
+
+def _recent_longest(key):
+    """The longest list of the views that the expectation of a size comes from."""
+    seen = _expectations.get(key, (0, 0))
+    return max(n for _, n in seen[3]) if len(seen) > 3 else seen[1]
 
 
 def _expectation(key):
@@ -283,7 +289,7 @@ def _launch_bounds(key):
 
 def _remember(key, instances, longest):
     seen = _expectations.pop(key, ())  # (re-inserted at the end: the dict keeps insertion order)
-    recent = (instances, *(seen[3] if len(seen) > 3 else seen[:1]))[:_RECENT_VIEWS]
+    recent = ((instances, longest), *(seen[3] if len(seen) > 3 else (seen[:2],) if seen else ()))[:_RECENT_VIEWS]
     _expectations[key] = (instances, longest, longest > _LONG_LIST or any(seen[2:3]), recent)
     while len(_expectations) > _MAX_EXPECTATIONS:
         # (a copy to look at: another thread may be adding entries, or have removed this one)
@@ -311,7 +317,8 @@ class _RenderGaussians(torch.autograd.Function):
           binningBuffer, imgBuffer), info) = _C.render_gaussians_ex(
             rs.bg, rs.image_height, rs.image_width, means2D, depths, radii, conic_opacity, rgb, mask, rs.viewmatrix,
             rs.campos, rs.tanfovx, rs.tanfovy, all_maps, rs.render_geo, rs.debug, cuda_args,
-            expected_instances=expected_instances, expected_longest_list=expected_longest, blend_records=records)
+            expected_instances=expected_instances, expected_longest_list=expected_longest, blend_records=records,
+            recent_longest_list=_recent_longest(key))
         ctx.blend_records = records
         if means2D.shape[0] > 0:
             _remember(key, num_rendered, info["longest_list"])

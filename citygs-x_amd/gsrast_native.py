@@ -139,7 +139,7 @@ class RenderOptions(C.Structure):
     _fields_ = [("struct_bytes", C.c_uint32), ("tile_sort_small_limit", C.c_int32),
                 ("tile_sort_block_records", C.c_int32), ("expected_longest_list", C.c_int32),
                 ("expected_instances", C.c_int64), ("blend_records", C.c_void_p), ("clear_geo_images", C.c_int32),
-                ("reserved", C.c_int32)]
+                ("recent_longest_list", C.c_int32)]
 
     def __init__(self, tile_sort_small_limit=-1, tile_sort_block_records=-1, expected_instances=0,
                  expected_longest_list=0, blend_records=None):

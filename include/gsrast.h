@@ -188,7 +188,9 @@ typedef struct gs_render_options {
   const float* blend_records;
   /* With render_geo == 0: non-zero has out_all_map and out_plane_depth written as zeros (otherwise they are not touched). */
   int32_t clear_geo_images;
-  int32_t reserved;
+  /* The longest list of the views that expected_instances comes from (0: not known, expected_longest_list is taken for it):
+   * whether a view launched ahead packs operand records depends on it. */
+  int32_t recent_longest_list;
 } gs_render_options;
 
 /* What gs_render_forward reports besides the instance count (optional, NULL to skip; struct_bytes as above):

@@ -28,7 +28,7 @@ def view(n, everywhere, unseen, seed):
         u1=torch.randn(1, H, W, generator=gen)).items()}
 
 
-def render(d, instances, longest):
+def render(d, instances, longest, recent=0):
     import gsrast_native as gn
     from diff_gaussian_rasterization import _C
     cl = torch.ones(3, 5, dtype=torch.bool, device=DEV)
@@ -36,7 +36,8 @@ def render(d, instances, longest):
     gn.stage_timing(True)
     out, info = _C.render_gaussians_ex(d["bg"], H, W, d["means2D"], d["depths"], d["radii"], d["co"], d["rgb"], cl,
                                        torch.eye(4, device=DEV), torch.zeros(3, device=DEV), 0.5, 0.5, d["am"], True,
-                                       False, args, expected_instances=instances, expected_longest_list=longest)
+                                       False, args, expected_instances=instances, expected_longest_list=longest,
+                                       recent_longest_list=recent)
     torch.cuda.synchronize()
     gn.stage_timing(False)
     packs = gn.stage_timing_collect().get("pack_operands", (0.0, 0))[1]
@@ -66,3 +67,16 @@ def test_by_the_views_own_figures(n, everywhere, unseen, packed):
         assert packs == (1 if ahead and expected else 0 if ahead else 2 if expected else 1 if packed else 0)
         for a, b in zip(want, got):
             assert np.array_equal(a.cpu().numpy(), b.cpu().numpy(), equal_nan=True)
+
+
+# launched for lists of any length: the views that the expectation comes from say how long they are
+@pytest.mark.parametrize("instances,recent,packed", [(0.7, 0, True), (0.7, -1, True), (0.7, 100, False), (0.7, 4096, False),
+                                                     (0.7, 4097, True), (0.39, 4097, False), (0.9, 100, True)])
+def test_by_the_lists_of_the_views_before(instances, recent, packed):
+    d = view(3000, 100, 2600, seed=3)
+    want = render(d, 0, 0)[3]
+    packs, info, _, got = render(d, int(instances * 5700 * 1.25), 0, recent)
+    assert info["launched_ahead"] == (instances * 5700 * 1.25 >= 4500)
+    assert packs == (1 if packed else 0)  # (the view's own figures, 4500 instances and a list of 300: none)
+    for a, b in zip(want, got):
+        assert np.array_equal(a.cpu().numpy(), b.cpu().numpy(), equal_nan=True)

@@ -399,3 +399,21 @@ def test_expected_instances_are_those_of_the_fullest_of_the_last_views():
     finally:
         dgr._expectations.clear()
         dgr._expectations.update(saved)
+
+
+def test_longest_list_of_the_last_views():
+    import diff_gaussian_rasterization as dgr
+    saved = dict(dgr._expectations)
+    dgr._expectations.clear()
+    try:
+        assert dgr._recent_longest("size") == 0
+        for longest, most in ((100, 100), (5000, 5000), *[(200, 5000)] * 7, (300, 300)):
+            dgr._remember("size", 1000, longest)
+            assert dgr._recent_longest("size") == most
+        dgr._expectations["size"] = (2000, 70, False)  # (an entry without the views before)
+        assert dgr._recent_longest("size") == 70
+        dgr._remember("size", 900, 50)
+        assert dgr._recent_longest("size") == 70 and dgr._expectation("size")[0] == int(2000 * dgr._MARGIN) + 65536
+    finally:
+        dgr._expectations.clear()
+        dgr._expectations.update(saved)
