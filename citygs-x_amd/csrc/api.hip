@@ -552,7 +552,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   const float* caller_records =
       (options != nullptr && options->struct_bytes >= OPTIONS_WITH_RECORDS) ? options->blend_records : nullptr;
   const bool clear_geo = render_geo == 0 && options != nullptr && options->struct_bytes >= sizeof(gs_render_options) &&
-                         options->clear_geo_images != 0;
+                         options->clear_geo_images > 0;
   GS_REQUIRE(!clear_geo || (out_all_map && out_plane_depth), "gs_render_forward: no images to clear");
   GS_REQUIRE(!clear_geo || (((uintptr_t)out_all_map | (uintptr_t)out_plane_depth) & 15u) == 0u,
              "gs_render_forward: the images to clear must be 16-byte aligned");

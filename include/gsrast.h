@@ -186,7 +186,8 @@ typedef struct gs_render_options {
    * them itself when the view has more than 0.8 instances per Gaussian.  The same pointer goes to
    * gs_render_backward; the records must stay as they are until that call has run. */
   const float* blend_records;
-  /* With render_geo == 0: non-zero has out_all_map and out_plane_depth written as zeros (otherwise they are not touched). */
+  /* With render_geo == 0: above zero has out_all_map and out_plane_depth, on 16-byte boundaries, written as zeros (otherwise
+   * they are not touched and may be NULL).  (struct_bytes may leave this field and the next one out.) */
   int32_t clear_geo_images;
   /* The longest list of the views that expected_instances comes from (0: not known, expected_longest_list is taken for it):
    * whether a view launched ahead packs operand records depends on it. */

@@ -61,3 +61,53 @@ def test_gradient_of_plain_colours(P):
         assert torch.equal(a, b) and torch.isfinite(a).all()
     assert got[3].shape == (P, 3) and not got[3].view(torch.int32).any()
     assert torch.equal(got[4], gco[:, 3:])
+
+
+# A caller that was compiled before the field, one that leaves it at its default (0, or below zero as in any field), and one
+# that asks for it.  The other fields hold either way: lists launched ahead, the caller's operand records.
+@pytest.mark.parametrize("older,clear,images", [(False, 1, True), (False, 0, True), (False, 0, False), (False, -1, True),
+                                                (False, -1, False), (True, 1, True), (True, 1, False)])
+def test_who_has_the_images_cleared(older, clear, images):
+    import ctypes as C
+    import gsrast_native as gn
+    n, W, H = 300, 41, 27
+    gen = torch.Generator().manual_seed(n)
+    r = lambda *s: torch.rand(*s, generator=gen).to(DEV)
+    m2, co = r(n, 2) * torch.tensor([W, H], device=DEV), torch.tensor([[0.5, 0.0, 0.5, 0.3]], device=DEV).repeat(n, 1)
+    depths, rgb, radii = r(n) + 1, r(n, 3), torch.ones(n, dtype=torch.int32, device=DEV)
+    records = torch.cat([m2, co, rgb, torch.zeros(n, 5, device=DEV), depths[:, None], torch.zeros(n, 1, device=DEV)], 1).contiguous()
+    cl, zero3 = torch.ones(2, 3, dtype=torch.bool, device=DEV), torch.zeros(3, device=DEV)
+    p = lambda t: None if t is None else C.c_void_p(t.data_ptr())
+
+    def run(options):
+        kept = []
+
+        def buffer(size, user):
+            kept.append(torch.zeros(size, dtype=torch.uint8, device=DEV))
+            return kept[-1].data_ptr()
+        fn, result, count = gn.RESIZE_FN(buffer), gn.RenderResult(), C.c_int()
+        color = torch.full((3, H, W), float("nan"), device=DEV)
+        stats = [torch.zeros(k, dtype=torch.int32, device=DEV) for k in (6, 6, 6, n)]
+        geo = [torch.full((k, H, W), 7.0, device=DEV) if images else None for k in (5, 1)]
+        gn.stage_timing(True)
+        status = gn.lib.gs_render_forward(fn, None, fn, None, fn, None, n, p(zero3), W, H, 41.0, 27.0, W / 2, H / 2, None, None,
+                                          None, p(m2), p(depths), p(radii), p(co), p(rgb), p(cl), p(color),
+                                          *[p(s) for s in stats], p(geo[0]), p(geo[1]), None, 0, 0, C.byref(count), None,
+                                          C.byref(options) if options else None, C.byref(result),
+                                          C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        gn.stage_timing(False)
+        gn.check(status, "gs_render_forward")
+        return color, geo, result, gn.stage_timing_collect().get("pack_operands", (0.0, 0))[1], count.value
+
+    options = gn.RenderOptions(expected_instances=20 * n, blend_records=records.data_ptr())
+    options.clear_geo_images = clear
+    if older:
+        options.struct_bytes = gn.RenderOptions.clear_geo_images.offset
+        options.recent_longest_list = -559038737
+    color, geo, result, packs, R = run(options)
+    assert result.launched_ahead == 1 and packs == 0 and R * 5 > n * 4
+    want, _, _, packs, _ = run(None)
+    assert packs == 1 and torch.equal(color.view(torch.int32), want.view(torch.int32))
+    for image in geo:
+        assert image is None or bool((image == (0.0 if clear > 0 and not older else 7.0)).all())
