@@ -61,3 +61,46 @@ def test_order_of_a_split_list(kind, n, limits):
     want = np.argsort(bits, kind="stable")
     assert np.array_equal(point_list, want)
     assert np.array_equal(keys, bits[want])  # (tile 0)
+
+
+# Several lists in one view, whose groups are jobs for the same workgroups: lists of one to a dozen groups (and of 64 with a
+# block of 300 records), beside lists that are sorted whole, in registers, or empty.  300 tiles: as many workgroups as tiles;
+# fewer than 256: up to 64 workgroups a tile.
+@pytest.mark.parametrize("gx,gy,sizes,limits", [
+    (3, 2, (20_000, 70_000, 17_000, 16_384, 4097, 100), None), (3, 2, (0, 16_385, 0, 140_000, 0, 33_000), None),
+    (2, 1, (17_000, 70_000), None), (3, 2, (4097, 33_000, 5000, 300, 301, 0), (-1, 300)),
+    (3, 2, (9, 8, 70, 500, 7, 64), (7, 7)), (20, 15, (17_000, 5000, 41_000) + (300,) * 297, None)])
+@pytest.mark.parametrize("ahead", [False, True])
+def test_order_of_several_split_lists(gx, gy, sizes, limits, ahead):
+    import gsrast_native as gn
+    from diff_gaussian_rasterization import _C
+    gen = torch.Generator().manual_seed(sum(sizes))
+    W, H, n = 16 * gx, 16 * gy, sum(sizes)
+    tile = torch.repeat_interleave(torch.arange(gx * gy), torch.tensor(sizes))
+    d = torch.cat([depths(("even", "heavy", "outliers")[i % 3], k, gen) if k > 8 else torch.rand(k, generator=gen) + 1
+                   for i, k in enumerate(sizes)])
+    mix = torch.randperm(n, generator=gen)  # (a list's Gaussians lie anywhere)
+    tile, d = tile[mix], d[mix]
+    m2 = torch.stack([(tile % gx) * 16.0, (tile // gx) * 16.0], 1) + 3 + torch.rand(n, 2, generator=gen) * 9
+    co = torch.tensor([[0.5, 0.0, 0.5, 0.3]]).repeat(n, 1).to(DEV)
+    args = {"stats_collector": {}}
+    if limits is not None:
+        args["tile_sort_limits"] = limits
+    out, info = _C.render_gaussians_ex(torch.zeros(3, device=DEV), H, W, m2.to(DEV), d.to(DEV),
+                                       torch.full((n,), 2, dtype=torch.int32, device=DEV), co,
+                                       torch.rand(n, 3, generator=gen).to(DEV),
+                                       torch.ones(gy, gx, dtype=torch.bool, device=DEV), torch.eye(4, device=DEV),
+                                       torch.zeros(3, device=DEV), 0.5, 0.5, None, False, False, args,
+                                       expected_instances=n + 5 if ahead else 0)
+    assert out[0] == n and info["launched_ahead"] == ahead and info["longest_list"] == max(sizes)
+    capacity = info["binning_capacity"]
+    off = [C.c_size_t() for _ in range(5)]
+    gn.check(gn.lib.gs_binning_state_layout(capacity, W, H, *[C.byref(x) for x in off]), "layout")
+    binning = out[9]
+    base = -binning.data_ptr() % 256
+    point_list = binning[base + off[0].value: base + off[0].value + 4 * n].view(torch.int32).cpu().numpy()
+    keys = binning[base + off[1].value: base + off[1].value + 8 * n].view(torch.int64).cpu().numpy()
+    key = tile.numpy().astype(np.int64) << 32 | d.numpy().view(np.uint32).astype(np.int64)
+    want = np.argsort(key, kind="stable")
+    assert np.array_equal(point_list, want)
+    assert np.array_equal(keys, key[want])
