@@ -980,11 +980,15 @@ __device__ __forceinline__ void split_list(uint32_t t, uint32_t start, uint32_t 
   const uint32_t groups = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_scan[0]);
   const int group_bits = 32 - __builtin_clz(groups | 1u);  // (so that no group has all of them set: that is nobody's)
   const uint32_t nobody = (1u << group_bits) - 1u;  // (a lane without a record; at least `groups`)
-  // The lanes whose g equals the lane's own `a`, and those with its `b`.
+  // The lanes whose g equals the lane's own `a`, and those with its `b`: from one ballot for every bit of g.  A ballot's result
+  // is hidden from the compiler before the lanes select on it.  Where it saw both (a ballot of g == k, selected by the lane
+  // with that k) it put the lane's own number into the ballot, as if it were one lane's comparison: the counts came out wrong
+  // and the records that are placed by them out of the list.
   auto lanes_with = [&](uint32_t g, uint32_t a, uint32_t b, uint64_t& with_a, uint64_t& with_b) {
     with_a = with_b = ~0ull;
     for (int k = 0; k < group_bits; k++) {
-      const uint64_t set = gs_ballot((g >> k & 1u) != 0u);
+      uint64_t set = gs_ballot((g >> k & 1u) != 0u);
+      asm("" : "+s"(set));
       with_a &= (a >> k & 1u) != 0u ? set : ~set;
       with_b &= (b >> k & 1u) != 0u ? set : ~set;
     }
