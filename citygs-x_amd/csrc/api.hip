@@ -637,7 +637,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   //   without: to 0.4 4 to 44 lost, 0.4 to 0.8 29 saved to 9 lost (colour only 4 saved to 19 lost), more 36 saved to 8 lost
   // The library's own records live at the end of the binning buffer, which is sized once the decision is
   // made.  A view that was launched ahead without records and did not fit is looked at again with its own figures (its
-  // buffer is another one); one that was launched with them keeps them, since the word that says so is set.
+  // buffer is another one); one that was launched with them is packed all the same, on its new buffer.
   bool use_packed = caller_records != nullptr;
   auto decide_packing = [&](int64_t instances, uint32_t longest_list) {
     const bool long_lists = bucketed && longest_list > (uint32_t)TILE_SORT_SMALL;
@@ -674,11 +674,11 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   // Packs the library's own records into the arrays just carved.  With the caller's records, or none, the word
   // beside them must say "none" (a backward call that is not handed the caller's records again then gathers the
   // operands from the arrays): the counting step has cleared it.
-  auto pack_records = [&](const Arrays& A) -> int {
+  auto pack_records = [&](const Arrays& A, bool ahead_of_host) -> int {
     if (caller_records != nullptr || !use_packed) return 0;
     StageScope _t("pack_operands", stream);
     launch_pack_blend_operands(P, radii, means2D, conic_opacity, rgb, render_geo ? all_map : nullptr, depths,
-                               A.packed, packed_valid, stream);
+                               A.packed, packed_valid, ahead_of_host ? bucket_fits_word(bucket_table, T) : nullptr, stream);
     return check_launch("pack_operands", stream, dbg);
   };
   auto blend = [&](const Arrays& A, bool ordered, uint32_t longest_for_launch, bool ahead_of_host) -> int {
@@ -735,7 +735,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
     decide_packing(cap_n - cap_n / 5, recent > 0 ? (uint32_t)recent : cap_longest);
     if (carve(cap_n, A)) return 1;
     if (timer.begin(elapsed_ms != nullptr, stream)) return 1;
-    if (pack_records(A)) return 1;
+    if (pack_records(A, true)) return 1;
     if (lists_by_tile(A, cap_longest, 0xFFFFFFFFu, true)) return 1;
     if (blend(A, cap_longest > 0, cap_longest, true)) return 1;
   }
@@ -778,11 +778,11 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
   }
 
   // The ordinary way (also after kernels launched ahead found that the view does not fit and did nothing).
-  // (after kernels launched ahead: the records are packed again, the buffer may be another one)
+  // (after kernels launched ahead: the records are packed now, the buffer may be another one)
   decide_packing(R, longest);
   if (carve(R, A)) return 1;
   if (!ahead && timer.begin(elapsed_ms != nullptr, stream)) return 1;
-  if (pack_records(A)) return 1;
+  if (pack_records(A, false)) return 1;
 
   if (bucketed) {
     if (lists_by_tile(A, longest, radix_tiles, false)) return 1;

@@ -170,7 +170,9 @@ __global__ void __launch_bounds__(GS_BLOCK_1D)
 pack_blend_operands_kernel(int P, const int* __restrict__ radii, const float2* __restrict__ means2D,
                            const float4* __restrict__ conic_opacity, const float* __restrict__ rgb,
                            const float* __restrict__ all_map, const float* __restrict__ depths,
-                           float4* __restrict__ packed, uint32_t* __restrict__ valid_word) {
+                           float4* __restrict__ packed, uint32_t* __restrict__ valid_word,
+                           const uint32_t* __restrict__ fits_word) {
+  if (fits_word != nullptr && *fits_word == 0u) return;  // launched ahead of the host's decision, for a view that does not fit
   if (valid_word != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *valid_word = 1u;
   constexpr int WORD_STRIDE = GS_WAVE + 1;  // in 16-byte units
   __shared__ float4 s_rec[GS_BLOCK_1D / GS_WAVE][4 * WORD_STRIDE];
@@ -373,11 +375,11 @@ int launch_duplicate_with_keys(int P, int W, int H, const float* means2D, const 
 
 int launch_pack_blend_operands(int P, const int* radii, const float* means2D, const float* conic_opacity,
                                const float* rgb, const float* all_map, const float* depths, float* packed,
-                               uint32_t* valid_word, hipStream_t stream) {
+                               uint32_t* valid_word, const uint32_t* fits_word, hipStream_t stream) {
   if (P <= 0) return 0;
   hipLaunchKernelGGL(pack_blend_operands_kernel, dim3((P + GS_BLOCK_1D - 1) / GS_BLOCK_1D), dim3(GS_BLOCK_1D), 0,
                      stream, P, radii, (const float2*)means2D, (const float4*)conic_opacity, rgb, all_map, depths,
-                     (float4*)packed, valid_word);
+                     (float4*)packed, valid_word, fits_word);
   return 0;
 }
 

@@ -141,10 +141,10 @@ int launch_tile_radix_sort(int T, bool mid, bool lng, const uint32_t* ranges, co
 // What the blend kernels read of a Gaussian, in one 64-byte record per Gaussian: (x, y, A, B), (C, opacity, r, g),
 // (b, map0, map1, map2), (map3, map4, depth, 0); all_map and depths may be null (zeros).  Records of Gaussians with
 // radius 0 are left as they are (no tile lists them).
-// valid_word (optional): set to 1 by the kernel.
+// valid_word (optional): set to 1 by the kernel.  fits_word (optional): the kernel does nothing if it is 0.
 int launch_pack_blend_operands(int P, const int* radii, const float* means2D, const float* conic_opacity,
                                const float* rgb, const float* all_map, const float* depths, float* packed,
-                               uint32_t* valid_word, hipStream_t stream);
+                               uint32_t* valid_word, const uint32_t* fits_word, hipStream_t stream);
 int launch_fill_u32(int64_t n, uint32_t value, uint32_t* p, hipStream_t stream);
 int launch_gather_u32(int64_t n, const uint32_t* index, const uint32_t* table, uint32_t* out, hipStream_t stream);
 int launch_ssim_l1_fwd(int C, int H, int W, const float* img1, const float* img2, const uint8_t* mask,

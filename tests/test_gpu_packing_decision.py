@@ -80,3 +80,36 @@ def test_by_the_lists_of_the_views_before(instances, recent, packed):
     assert packs == (1 if packed else 0)  # (the view's own figures, 4500 instances and a list of 300: none)
     for a, b in zip(want, got):
         assert np.array_equal(a.cpu().numpy(), b.cpu().numpy(), equal_nan=True)
+
+
+# launched ahead on a buffer that turns out too small, or on too short a bound: whatever was launched leaves it alone, the
+# operand records too
+@pytest.mark.parametrize("instances,longest", [(5000, 0), (100_000, 299)])
+def test_a_view_that_does_not_fit_leaves_the_buffer_it_was_launched_on(instances, longest):
+    import ctypes as C
+    import gsrast_native as gn
+    d = view(4500, 300, 100, seed=9)
+    P, R = 4900, 4500 + 15 * 300
+    want = render(d, 0, 0)[3]
+    p, kept = (lambda t: C.c_void_p(t.data_ptr())), []
+
+    def buffer(fill):
+        def resize(size, user):
+            kept.append(torch.full((size,), fill, dtype=torch.uint8, device=DEV))
+            return kept[-1].data_ptr()
+        return gn.RESIZE_FN(resize)
+    other, binning = buffer(0), buffer(0xAB)
+    color, omap, depth = (torch.full((k, H, W), float("nan"), device=DEV) for k in (3, 5, 1))
+    stats = [torch.zeros(k, dtype=torch.int32, device=DEV) for k in (15, 15, 15, P)]
+    cl, zero3 = torch.ones(3, 5, dtype=torch.bool, device=DEV), torch.zeros(3, device=DEV)
+    options, result, count = gn.RenderOptions(-1, -1, instances, longest), gn.RenderResult(), C.c_int()
+    gn.check(gn.lib.gs_render_forward(other, None, binning, None, other, None, P, p(d["bg"]), W, H, W / 1.0, H / 1.0, W / 2, H / 2,
+                                      None, None, p(d["am"]), p(d["means2D"]), p(d["depths"]),
+                                      p(d["radii"]), p(d["co"]), p(d["rgb"]), p(cl), p(color), *[p(s) for s in stats], p(omap),
+                                      p(depth), None, 1, 0, C.byref(count), None, C.byref(options), C.byref(result),
+                                      C.c_void_p(torch.cuda.current_stream().cuda_stream)), "gs_render_forward")
+    torch.cuda.synchronize()
+    assert count.value == R and result.launched_ahead == 0
+    first, second = [b for b in kept if bool((b[-1:] == 0xAB).all())]
+    assert first.numel() >= 64 * P and bool((first == 0xAB).all())
+    assert torch.equal(color.view(torch.int32), want[0].view(torch.int32))
