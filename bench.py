@@ -263,8 +263,8 @@ def interleaved(args, steppers, P):
             "never_ahead": {"ms_per_view_mean": round(wall_miss, 4), "launched_ahead_rate": round(rate_miss, 4),
                             "ms_per_view_by_camera": cam_miss},
             "miss_cost_ms_per_view": round(wall_miss - wall, 4) if rate > 0 else None,
-            "note": "a view whose expectation does not hold (more instances than the previous view's figure plus 25 % "
-                    "+ 65536, or a longer list than its sort variant takes) runs the launched-ahead kernels as "
+            "note": "a view whose expectation does not hold (more instances than the fullest of the last views had plus "
+                    "25 % + 65536, or a longer list than its sort variant takes) runs the launched-ahead kernels as "
                     "no-ops and then the ordinary route; never_ahead is that ordinary route for every view"}
 
 

@@ -586,7 +586,7 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
 
   // The instance count decides the size of the binning buffer, and the host learns it only after the counting
   // kernels have run: a round trip during which the GPU would idle.  A caller that says how many instances and
-  // how long a list it expects (the previous view's figures with a margin) gets the list kernels and the blend
+  // how long a list it expects (the last views' figures with a margin) gets the list kernels and the blend
   // launched right behind the counting kernels, on buffers of the expected size; a device word tells them whether
   // the view fits (they do nothing otherwise), and the host, which meanwhile has received the counts, either
   // returns or builds the lists again the ordinary way.

@@ -23,7 +23,7 @@
 namespace gs {
 namespace {
 
-constexpr int TR_DIGITS = 256;  // digit values of the passes that go through memory and of the split by leading bits
+constexpr int TR_DIGITS = 256;  // digit values of the passes that go through memory
 constexpr int TR_PASSES = 4;
 // Lists that one workgroup holds are sorted on one-word keys: a depth field of TR_FIELD_BITS bits over the
 // record's place in the unsorted list, in two passes (or one) on digits of TR_KEY_DIGIT_BITS bits.

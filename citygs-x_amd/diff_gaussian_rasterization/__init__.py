@@ -153,7 +153,7 @@ def _have_versions(sources):
 def _records_wanted(rs, P, device):
     """Whether preprocess should write the records: one of the last views of this image size had enough instances per
     Gaussian for records to pay (written on the way they cost about a third of the library's packing pass, which
-    pays from 0.8 instances per Gaussian), and render_gaussians will be able to use them (no geometry channels to
+    pays from 0.8 instances per Gaussian, 0.4 with long lists), and render_gaussians will be able to use them (no geometry channels to
     render, or the caller builds them through build_all_map(..., blend_records_of=means2D))."""
     seen = _expectations.get((rs.image_height, rs.image_width, device))
     if seen is None or _most_instances(seen) * 10 <= P * 3:
@@ -238,8 +238,15 @@ def preprocess_gaussians(means3D, scales, rotations, sh, opacities, raster_setti
 # a margin (a training loop renders thousands of similar views; the number of Gaussians changes at every
 # densification, so it is not part of the key).  A scene's cameras differ by more than the margin: in a loop over views of
 # 6.2 M and 2.7 M instances every view of the larger kind missed an expectation taken from the view before it.
-# Only the time depends on it, never a result; a stale or missing
-# entry costs one ordinary call.  A handful of image sizes at most are alive in a run: the oldest entry goes
+# Only the time and the memory depend on it, never a result; a stale or missing entry costs one ordinary call, and the
+# binning buffer of a view that fits has the expected size until its backward pass has run.
+# Behind a dense view the next seven of its size pack or write operand records for its sake, sparse ones too.  One dense
+# view in eight, us a training view with this expectation and with that of the last view alone (channels linked; built
+# apart; colour only): 1 M Gaussians obliquely and through a narrow lens 387 and 387; 425 and 436; 353 and 353; 4 M from the
+# air, 0.8 and 0.1 instances a Gaussian, 736 and 740; 902 and 888; 696 and 688; 10 M at street level, 0.6 and 0.02, 1371 and
+# 1373; 1753 and 1735; 1303 and 1288.  Peak memory 288 MB for 258 (1 M), else the same.  Against that stands a dense view of
+# 10 M that is launched on a buffer that fits but without its records: 350 us of that view.
+# A handful of image sizes at most are alive in a run: the oldest entry goes
 # when there are more than _MAX_EXPECTATIONS.
 _expectations = {}
 _MARGIN = 1.25

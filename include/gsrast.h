@@ -158,10 +158,10 @@ int gs_preprocess_rows_backward(const int* radii, const float* cov3D, const uint
  * zero keeps its default; struct_bytes is sizeof(gs_render_options) as the caller compiled it.
  * gs_render_forward builds the per-tile lists by bucketing the instances by tile (a counting sort) and sorting
  * each tile's list on its own: lists of up to 4096 records in registers, longer ones by a radix sort on the depth
- * bits that one workgroup runs inside its CU (up to 16384 records at once; a longer list is first split by its
- * leading depth bits into parts that fit).  A tile grid of more than 30000 tiles takes the reference's own route instead: (tile | depth) keys
- * (rasterizer_impl.cu:74-117), one radix sort over all of them (:675-684), identifyTileRanges (:122-144).  All
- * give the same lists bit for bit.
+ * bits that one workgroup runs inside its CU (up to 16384 records at once; a longer list is first split by depth, at
+ * bounds that a sample of it gives, into parts that fit).  A tile grid of more than 30000 tiles takes the reference's own
+ * route instead: (tile | depth) keys (rasterizer_impl.cu:74-117), one radix sort over all of them (:675-684),
+ * identifyTileRanges (:122-144).  All give the same lists bit for bit.
  * tile_sort_small_limit lowers the list length that is sorted in registers (default and maximum 4096; 0 = the
  * view takes the reference's route) and tile_sort_block_records the number of records the per-tile radix sort
  * holds at once (default and maximum 16384; 0 or below = default), so that small scenes can exercise every route.
@@ -171,20 +171,24 @@ typedef struct gs_render_options {
   int32_t tile_sort_small_limit;
   int32_t tile_sort_block_records;
   int32_t expected_longest_list;
-  /* What the caller expects of the view, typically the previous view's figures with a margin (0 = no idea).
+  /* What the caller expects of the view, typically the instances of the fullest of the last views and the longest list of
+   * the last one, with a margin of a quarter (0 = no idea).
    * With expected_instances > 0 (and a gs_render_result to report into) gs_render_forward does not wait for the
    * instance count before it goes on: it sizes the binning buffer for expected_instances, launches the list
    * kernels and the blend right behind the counting kernels, and lets a device-side check turn them into no-ops
    * if the view has more instances than that or a list longer than expected_longest_list (0 = any length; a
    * figure of at most 4096 spares the launch of the radix sort's kernels, one below 3072 a blend kernel that is
    * ready to split the tiles of longer lists); in that case the lists are built
-   * again the ordinary way, so the result never depends on the expectation, only the time does. */
+   * again the ordinary way, so the result never depends on the expectation, only the time does, and the memory: a
+   * view that fits keeps a binning buffer of the expected size until its backward call has run. */
   int64_t expected_instances;
   /* The blend kernels' operand records of this view's Gaussians as gs_preprocess_forward wrote them (their
    * geometry channels must be the all_map this call is given; with render_geo == 0 they are not read), or NULL:
-   * the call then packs
-   * them itself when the view has more than 0.8 instances per Gaussian.  The same pointer goes to
-   * gs_render_backward; the records must stay as they are until that call has run. */
+   * the call then packs them itself where that pays: when the view has more than 0.8 instances per Gaussian, or more
+   * than 0.4 and a tile list of more than 4096 entries.  A call that launches ahead decides by what is expected
+   * (expected_instances less a fifth, recent_longest_list); if the view does not fit and was not to be packed, its own
+   * figures decide.  The same pointer goes to gs_render_backward; the records must stay as they are until that call
+   * has run. */
   const float* blend_records;
   /* With render_geo == 0: above zero has out_all_map and out_plane_depth, on 16-byte boundaries, written as zeros (otherwise
    * they are not touched and may be NULL).  (struct_bytes may leave this field and the next one out.) */
@@ -232,8 +236,8 @@ typedef struct gs_render_result {
  * The geometry buffer is asked for 8 bytes per Gaussian (tile counts and their prefix sum) plus the prefix sum's
  * workspace (the reference's holds the preprocess outputs as well, CR/rasterizer_impl.cu:160-188; here those are
  * the caller's tensors).  The binning buffer is asked for 64 bytes per Gaussian beyond what
- * gs_binning_state_layout reports when this call packs the blend kernels' operand records itself (a view with
- * more than 0.8 instances per Gaussian and no blend_records from the caller). */
+ * gs_binning_state_layout reports when this call packs the blend kernels' operand records itself (see
+ * gs_render_options.blend_records). */
 int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resize_fn binningBuffer,
                       void* binning_user, gs_resize_fn imageBuffer, void* image_user, int P,
                       const float* background, int width, int height, float focal_x, float focal_y, float cx,
@@ -249,10 +253,10 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
  * CR/rasterizer_impl.cu:850-932) plus the repacking of
  * RenderGaussiansBackwardCUDA (DGR/rasterize_points.cu:428-440).  The three
  * buffers are the ones gs_render_forward filled (the geometry buffer is read
- * too: it holds the per-Gaussian instance offsets and, for a view with more than 0.8 instances per Gaussian, one
- * 64-byte record per visible Gaussian with the values of means2D, conic_opacity, rgb and all_maps that the forward
- * call was given, which the kernel then reads instead of those arrays: pass the forward call's arrays, as the
- * reference does).  Gradient outputs are
+ * too: it holds the per-Gaussian instance offsets and says whether the binning buffer holds, where the forward call
+ * packed them (see gs_render_options.blend_records), one 64-byte record per visible Gaussian with the values of
+ * means2D, conic_opacity, rgb and all_maps that that call was given, which the kernel then reads instead of those
+ * arrays: pass the forward call's arrays, as the reference does).  Gradient outputs are
  * fully written and need no initialisation: dL_dmean2D (P,2), dL_dmean2D_abs
  * (P,3), dL_dconic_opacity (P,4) packed [x, y, w, opacity], dL_dcolor (P,3),
  * dL_dall_map (P,5).  Where the reference adds every pixel's contribution
@@ -265,7 +269,8 @@ int gs_render_forward(gs_resize_fn geometryBuffer, void* geometry_user, gs_resiz
  * blend_records: gs_render_options.blend_records of the forward call (NULL if that call was given none). */
 size_t gs_render_backward_workspace_bytes(int R);
 /* As much scratch lets gs_render_backward leave out the records of instances that no pixel blends, which are zeros, where
- * that pays: a byte per instance says which records there are.  The results are the same. */
+ * that pays (two instances per pixel and more): a byte per instance says which records there are.  The results are the
+ * same. */
 size_t gs_render_backward_sparse_workspace_bytes(int R);
 int gs_render_backward(int P, int R, const float* background, int width, int height, float tan_fovx,
                        float tan_fovy, const char* geom_buffer, const char* binning_buffer,

@@ -495,7 +495,7 @@ def test_records_written_by_the_producers_give_the_same_results(geo):
 @pytest.mark.parametrize("poison", [False, True])
 def test_packed_and_gathered_operands_give_the_same_results(poison):
     """The forward call packs the blend kernels' operands into one record per Gaussian when the view has more than
-    0.8 instances per Gaussian, and lets both blend kernels gather them from the caller's arrays otherwise.  The
+    0.8 instances per Gaussian (no list here is beyond 4096 entries), and lets both blend kernels gather them from the caller's arrays otherwise.  The
     same Gaussians with and without a crowd of Gaussians behind the camera (which adds no instance and tips the
     decision) must render and differentiate to the same bits; so must a view in which some Gaussians carry NaN or
     infinite colours and geometry channels (NaNs in the same places, the same bits everywhere else)."""
